@@ -1017,7 +1017,7 @@ kvhip_status kvhip_cache_update(kvhip_cache *c, const void *keys, const void *va
 
 namespace {
 // host description -> device description; `H` heads per batch row of the rotated array
-kvhip_status rope_dev(const kvhip_rope *rope, int D, int H, int64_t pos0, const int32_t *batch_pos, RopeDev &r) {
+kvhip_status rope_dev(const kvhip_rope *rope, int D, int H, int dtype, int64_t pos0, const int32_t *batch_pos, RopeDev &r) {
     if (!rope) return fail(KVHIP_ERR_INVALID_ARG, "null rope description");
     if (rope->dims <= 0 || (rope->dims & 1) || rope->dims > D)
         return fail(KVHIP_ERR_INVALID_ARG, "rope dims must be even and at most the head dim");
@@ -1030,6 +1030,9 @@ kvhip_status rope_dev(const kvhip_rope *rope, int D, int H, int64_t pos0, const 
     r.pos0 = (int32_t)pos0;
     r.batch_pos = batch_pos;
     r.H = H;
+    // chunks of 8 (float32: 4) elements: whole rows, and both halves of the rotating range on chunk boundaries
+    const int v = dtype == KVHIP_F32 ? 4 : 8;
+    r.vec = D % v == 0 && (r.traditional ? r.dims : r.dims / 2) % v == 0;
     return KVHIP_OK;
 }
 }  // namespace
@@ -1042,7 +1045,7 @@ kvhip_status kvhip_rope_apply(const kvhip_rope *rope, const void *x, void *out, 
     if (dtype != KVHIP_F16 && dtype != KVHIP_BF16 && dtype != KVHIP_F32)
         return fail(KVHIP_ERR_INVALID_ARG, "rope needs a floating-point dtype");
     RopeDev r;
-    KV_TRY(rope_dev(rope, D, H, offset, batch_offsets, r));
+    KV_TRY(rope_dev(rope, D, H, dtype, offset, batch_offsets, r));
     KV_HIP(launch_rope_apply(r, x, out, B, H, L, D, dtype, S(stream)));
     return KVHIP_OK;
 }
@@ -1055,7 +1058,7 @@ kvhip_status kvhip_cache_update_rope(kvhip_cache *c, const kvhip_rope *rope, con
     // `ropeOffset` is read before the write (Llama.swift:58-62); the staged wrapper's offset
     // counts its staged rows (RotatingStagedKVCache.swift:33-37)
     const int64_t pos0 = c->offset + (c->staging ? (int64_t)c->staged.size() : 0);
-    KV_TRY(rope_dev(rope, Dk, Hkv, pos0, batch_offsets, r));
+    KV_TRY(rope_dev(rope, Dk, Hkv, dtype, pos0, batch_offsets, r));
     c->rope = &r;
     const kvhip_status st = kvhip_cache_update(c, keys, values, B, Hkv, L, Dk, Dv, dtype, stream);
     c->rope = nullptr;

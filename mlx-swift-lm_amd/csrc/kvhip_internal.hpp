@@ -220,6 +220,7 @@ struct RopeDev {
     int32_t pos0 = 0;
     const int32_t *batch_pos = nullptr;  // optional [B] (device)
     int32_t H = 1;             // heads per batch row of the array being rotated
+    int32_t vec = 0;           // 1: rows are whole 16-byte chunks and no pair's half cuts through one (chunk kernels)
 };
 
 // ---- kernel launchers (defined in the .hip files) ---------------------------

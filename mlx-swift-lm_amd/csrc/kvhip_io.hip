@@ -7,7 +7,16 @@ namespace kvhip {
 
 namespace {
 
-// grid (L, B*H): one row per workgroup
+// grid (L, B): the queries of one row position, every head of it (rope_rows_body).  512 rows of 32 heads x 128 in
+// bfloat16 (8.4 MB moved): 10.5 us with a workgroup per row and head and a sine, cosine and exponential per element,
+// 4.9 us so.
+template <int DT>
+__global__ void __launch_bounds__(256) rope_rows_kernel(RopeDev r, const char *x, char *out, int H, int L, int D) {
+    __shared__ float inv_s[512];
+    rope_rows_body<DT>(r, x, out, H, L, D, blockIdx.y, blockIdx.x, 0, H, inv_s);
+}
+
+// grid (L, B*H): one row per workgroup; arrays whose pairs cut through 16-byte chunks
 template <int DT>
 __global__ void rope_apply_kernel(RopeDev r, const char *x, char *out, int L, int D) {
     const int bh = blockIdx.y, l = blockIdx.x;
@@ -398,6 +407,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
     constexpr int TPRK = DK / 8, TPR = D / 8;
     constexpr int VPW = D / 2 + 1;  // dword pitch of a token's V row in LDS (odd: column reads spread over banks)
     __shared__ uint32_t vt[TILE * VPW];
+    __shared__ float inv_s[DK / 2];
     const int bh = blockIdx.y;
     const int slot_t = slot0 + blockIdx.x * TILE;
     const int l_t = src0 + blockIdx.x * TILE;
@@ -409,6 +419,10 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
     for (int e = 0; e < NCK; ++e) kraw[e] = *reinterpret_cast<const u4v *>(kbase + (size_t)(e * 256 + threadIdx.x) * 16);
 #pragma unroll
     for (int e = 0; e < NCV; ++e) vraw[e] = *reinterpret_cast<const u4v *>(vbase + (size_t)(e * 256 + threadIdx.x) * 16);
+    if (rope.dims > 0) {
+        rope_inv_table(rope, inv_s);
+        __syncthreads();
+    }
 #pragma unroll
     for (int e = 0; e < NCK; ++e) {
         const int c = e * 256 + threadIdx.x;
@@ -417,20 +431,14 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
         if (rope.dims > 0 && d0 < rope.dims) {
             const int pos = rope_pos(rope, bh, l_t + r);
             const char *row = kbase + (size_t)r * DK * 2;
-            uint32_t u[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                uint16_t lo, hi;
-                if (st.dtype == KVHIP_F16) {
-                    lo = __half_as_ushort(__float2half_rn(rope_elem<0>(rope, row, d0 + 2 * j, pos)));
-                    hi = __half_as_ushort(__float2half_rn(rope_elem<0>(rope, row, d0 + 2 * j + 1, pos)));
-                } else {
-                    lo = Elem<1>::bits(rope_elem<1>(rope, row, d0 + 2 * j, pos));
-                    hi = Elem<1>::bits(rope_elem<1>(rope, row, d0 + 2 * j + 1, pos));
-                }
-                u[j] = (uint32_t)lo | ((uint32_t)hi << 16);
+            float w[8];
+            if (st.dtype == KVHIP_F16) {
+                unpack8<0>(k, row, d0, rope, inv_s, pos, w);
+                k = chunk_pack<0>(w);
+            } else {
+                unpack8<1>(k, row, d0, rope, inv_s, pos, w);
+                k = chunk_pack<1>(w);
             }
-            k = u4v{u[0], u[1], u[2], u[3]};
         }
         *reinterpret_cast<u4v *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
     }
@@ -721,6 +729,14 @@ hipError_t launch_append_fp(const Store &st, const void *keys, const void *value
 hipError_t launch_rope_apply(const RopeDev &rope, const void *x, void *out, int B, int H, int L, int D,
                              int dtype, hipStream_t s) {
     if ((size_t)B * H * L == 0) return hipSuccess;
+    if (rope.vec) {
+#define ROPE_ROWS(DT) hipLaunchKernelGGL(rope_rows_kernel<DT>, dim3(L, B), dim3(256), 0, s, rope, (const char *)x, (char *)out, H, L, D)
+        if (dtype == KVHIP_F16) ROPE_ROWS(0);
+        else if (dtype == KVHIP_BF16) ROPE_ROWS(1);
+        else ROPE_ROWS(2);
+#undef ROPE_ROWS
+        return hipGetLastError();
+    }
     dim3 grid(L, B * H), block(D <= 64 ? 64 : (D <= 128 ? 128 : 256));  // at most 4 elements per thread up to D = 1024
     if (dtype == KVHIP_F16) hipLaunchKernelGGL(rope_apply_kernel<0>, grid, block, 0, s, rope, (const char *)x, (char *)out, L, D);
     else if (dtype == KVHIP_BF16) hipLaunchKernelGGL(rope_apply_kernel<1>, grid, block, 0, s, rope, (const char *)x, (char *)out, L, D);

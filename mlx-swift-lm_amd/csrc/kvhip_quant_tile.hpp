@@ -1,45 +1,11 @@
 // Quantize-on-append of whole 64-token tiles: the element functions, the tile body and its two kernels,
 // and the launchers of one code width (instantiated per width in kvhip_io.hip and kvhip_quant_tile_other.hip).
 #pragma once
-#include "kvhip_device.hpp"
+#include "kvhip_rope.hpp"
 
 namespace kvhip {
 
 namespace {
-
-// Element d of a row at position `pos` after the rotary embedding, rounded to the row's dtype
-// (what the reference hands to the cache: `applyRotaryPosition` runs before `update`,
-// Llama.swift:58-62).  The angle is the float32 product of position * scale and the inverse
-// frequency exp(-i * log(base) / half), or 1 / freqs[i].
-template <int DT>
-__device__ __forceinline__ float rope_elem(const RopeDev &r, const void *row, int d, int pos) {
-    const float x = Elem<DT>::load(row, d);
-    if (d >= r.dims) return x;
-    const int half = r.dims >> 1;
-    int i, partner;
-    bool first;
-    if (r.traditional) {
-        i = d >> 1;
-        partner = d ^ 1;
-        first = (d & 1) == 0;
-    } else {
-        first = d < half;
-        i = first ? d : d - half;
-        partner = first ? d + half : d - half;
-    }
-    // the inverse frequency is formed in double and rounded once, so that it does not depend on
-    // one exp implementation's last float32 bit (a position of 10^5 turns one such bit into 10^-2 rad)
-    const float inv = r.freqs ? 1.0f / r.freqs[i] : (float)exp(-(double)i * r.log_base_over_half);
-    const float theta = ((float)pos * r.scale) * inv;
-    float sn, cs;
-    sincosf(theta, &sn, &cs);
-    const float y = Elem<DT>::load(row, partner);
-    const float v = first ? x * cs - y * sn : y * sn + x * cs;
-    return round_dt<DT>(v);
-}
-__device__ __forceinline__ int rope_pos(const RopeDev &r, int bh, int l) {
-    return (r.batch_pos ? r.batch_pos[bh / r.H] : r.pos0) + l;
-}
 
 // ---- whole 64-token tiles (prompt-sized appends) -----------------------------------------
 // The per-row kernels above fetch one element per lane and wait for every row in turn; for
@@ -49,25 +15,20 @@ __device__ __forceinline__ int rope_pos(const RopeDev &r, int bh, int l) {
 // rotation are those of the per-row kernels (the same element functions).
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
+// Eight elements of a row from the 16-byte chunk `raw` at d0, rotated when the chunk lies inside the rotary range.
 template <int DT>
-__device__ __forceinline__ void unpack8(const u4v &raw, const void *row, int d0, const RopeDev &rope, int pos,
+__device__ __forceinline__ void unpack8(const u4v &raw, const char *row, int d0, const RopeDev &rope, const float *inv_s, int pos,
                                         float (&w)[8]) {
     if (rope.dims > 0 && d0 < rope.dims) {
+        if (rope.vec) {
+            rope_chunk<DT>(rope, inv_s, row, d0, pos, raw, w);
+        } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = rope_elem<DT>(rope, row, d0 + j, pos);
+            for (int j = 0; j < 8; ++j) w[j] = rope_elem<DT>(rope, row, d0 + j, pos);
+        }
         return;
     }
-    const uint32_t u[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (DT == 0) {
-            w[2 * j] = __half2float(__ushort_as_half((unsigned short)(u[j] & 0xffffu)));
-            w[2 * j + 1] = __half2float(__ushort_as_half((unsigned short)(u[j] >> 16)));
-        } else {
-            w[2 * j] = __uint_as_float(u[j] << 16);
-            w[2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u);
-        }
-    }
+    chunk_unpack<DT>(raw, w);
 }
 
 // Codes of the eight elements a thread holds, as integer-valued floats in [0, 2^BITS - 1], from
@@ -159,6 +120,7 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
     constexpr bool GEN = BITS != 4 && BITS != 8;  // 2, 3, 5, 6 bits: codes as a plain bit stream, K rows and V tile rows alike
     __shared__ __attribute__((aligned(8))) uint8_t vcodes[DO_V ? TILE * VP : 8];
     __shared__ __attribute__((aligned(16))) uint8_t kcodes[GEN && DO_K ? TILE * D * BITS / 8 : 16];  // the tile's K rows as stored
+    __shared__ float inv_s[ROPE ? D / 2 : 1];
     __shared__ __attribute__((aligned(16))) uint8_t vstage[PAGED && DO_V ? TILE * D * 2 : 16];  // the source V tile as stored
     const int bh = blockIdx.y;
     const int slot_t = slot0 + blockIdx.x * TILE;
@@ -195,7 +157,10 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
             if constexpr (DO_V) vraw[e] = *reinterpret_cast<const u4v *>(vbase + (size_t)c * 16);
         }
     }
-    const RopeDev no_rope;
+    if constexpr (ROPE) {
+        rope_inv_table(rope, inv_s);
+        __syncthreads();
+    }
     const float nb = (float)((1 << BITS) - 1);
     const int lane = threadIdx.x & 63;
     const int pos = lane & (GL - 1);            // place in the group
@@ -216,10 +181,10 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
             const int d0 = col_of(e);
             if (!is_v(i)) {
                 const int r = row_of(e);
-                if constexpr (ROPE) unpack8<DT>(kraw[e], kbase + (size_t)r * D * 2, d0, rope, rope_pos(rope, bh, l_t + r), w[i]);
-                else unpack8<DT>(kraw[e], nullptr, d0, no_rope, 0, w[i]);
+                if constexpr (ROPE) unpack8<DT>(kraw[e], kbase + (size_t)r * D * 2, d0, rope, inv_s, rope_pos(rope, bh, l_t + r), w[i]);
+                else chunk_unpack<DT>(kraw[e], w[i]);
             } else {
-                unpack8<DT>(vraw[e], nullptr, d0, no_rope, 0, w[i]);
+                chunk_unpack<DT>(vraw[e], w[i]);
             }
             float a = w[i][0], b = w[i][0];
 #pragma unroll

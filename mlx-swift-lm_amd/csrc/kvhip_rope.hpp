@@ -1,0 +1,202 @@
+// Rotary position embedding as the append kernels and the query pass apply it: the angle and its sine and
+// cosine, single elements (any shape), and 16-byte chunks (what the tuned kernels move).
+#pragma once
+#include "kvhip_device.hpp"
+
+namespace kvhip {
+
+// Sine and cosine of a float32 angle.  The angle is reduced by the nearest multiple of pi/2 in double (positions of
+// 10^5 leave an error below 10^-11), the remainder, at most pi/4, goes through the Taylor polynomials of degree 9 and
+// 10 (next terms below 2 10^-9 and 2 10^-10 there).  Some 30 instructions; the library's sincosf carries a
+// multi-word reduction for large angles that the appends spent most of their time in (512 rows of 8 heads x 128:
+// 22.7 us full precision and 18.8 us quantized with it and an exponential per element, 10.3 and 11.4 us so).
+__device__ __forceinline__ void rope_sincos(float theta, float &sn, float &cs) {
+    const double t = (double)theta;
+    const double k = rint(t * 0.63661977236758134308);
+    const float x = (float)fma(-k, 1.57079632679489661923, t);
+    const int quad = (int)(k - 4.0 * floor(k * 0.25));
+    const float z = x * x;
+    float s = __builtin_fmaf(z, 2.7557319223985893e-6f, -1.9841269841269841e-4f);
+    s = __builtin_fmaf(z, s, 8.3333333333333332e-3f);
+    s = __builtin_fmaf(z, s, -1.6666666666666667e-1f);
+    s = __builtin_fmaf(x * z, s, x);
+    float c = __builtin_fmaf(z, -2.7557319223985888e-7f, 2.4801587301587302e-5f);
+    c = __builtin_fmaf(z, c, -1.3888888888888889e-3f);
+    c = __builtin_fmaf(z, c, 4.1666666666666664e-2f);
+    c = __builtin_fmaf(z, c, -0.5f);
+    c = __builtin_fmaf(z, c, 1.0f);
+    const float a = (quad & 1) ? c : s, b = (quad & 1) ? s : c;
+    sn = (quad & 2) ? -a : a;
+    cs = ((quad + 1) & 2) ? -b : b;
+}
+
+// The inverse frequency of pair i is formed in double and rounded once, so that it does not depend on
+// one exp implementation's last float32 bit (a position of 10^5 turns one such bit into 10^-2 rad).
+__device__ __forceinline__ float rope_inv_freq(const RopeDev &r, int i) {
+    return r.freqs ? 1.0f / r.freqs[i] : (float)exp(-(double)i * r.log_base_over_half);
+}
+__device__ __forceinline__ float rope_angle(const RopeDev &r, int pos, float inv) { return ((float)pos * r.scale) * inv; }
+__device__ __forceinline__ int rope_pos(const RopeDev &r, int bh, int l) {
+    return (r.batch_pos ? r.batch_pos[bh / r.H] : r.pos0) + l;
+}
+// one element of a rotated pair (x: itself, y: its partner)
+__device__ __forceinline__ float rope_turn(float x, float y, bool first, float sn, float cs) {
+    return first ? x * cs - y * sn : y * sn + x * cs;
+}
+
+// Element d of a row at position `pos` after the rotary embedding, rounded to the row's dtype
+// (what the reference hands to the cache: `applyRotaryPosition` runs before `update`,
+// Llama.swift:58-62).  The angle is the float32 product of position * scale and the inverse
+// frequency exp(-i * log(base) / half), or 1 / freqs[i].
+template <int DT>
+__device__ __forceinline__ float rope_elem(const RopeDev &r, const void *row, int d, int pos) {
+    const float x = Elem<DT>::load(row, d);
+    if (d >= r.dims) return x;
+    const int half = r.dims >> 1;
+    int i, partner;
+    bool first;
+    if (r.traditional) {
+        i = d >> 1;
+        partner = d ^ 1;
+        first = (d & 1) == 0;
+    } else {
+        first = d < half;
+        i = first ? d : d - half;
+        partner = first ? d + half : d - half;
+    }
+    float sn, cs;
+    rope_sincos(rope_angle(r, pos, rope_inv_freq(r, i)), sn, cs);
+    return round_dt<DT>(rope_turn(x, Elem<DT>::load(row, partner), first, sn, cs));
+}
+
+// ---- 16-byte chunks: V = 8 elements of a 16-bit dtype, 4 floats ------------------------------------------------
+// (RopeDev::vec says that pairs never cut through a chunk)
+template <int DT> constexpr int rope_chunk_elems() { return DT == 2 ? 4 : 8; }
+template <int DT> __device__ __forceinline__ void chunk_unpack(const kv_u4 &raw, float (&w)[rope_chunk_elems<DT>()]) {
+    const uint32_t u[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if constexpr (DT == 2) {
+            w[j] = __uint_as_float(u[j]);
+        } else if constexpr (DT == 1) {
+            w[2 * j] = __uint_as_float(u[j] << 16);
+            w[2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u);
+        } else {
+            w[2 * j] = __half2float(__ushort_as_half((unsigned short)(u[j] & 0xffffu)));
+            w[2 * j + 1] = __half2float(__ushort_as_half((unsigned short)(u[j] >> 16)));
+        }
+    }
+}
+template <int DT> __device__ __forceinline__ kv_u4 chunk_pack(const float (&w)[rope_chunk_elems<DT>()]) {
+    uint32_t u[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if constexpr (DT == 2) u[j] = __float_as_uint(w[j]);
+        else if constexpr (DT == 1) u[j] = (uint32_t)Elem<1>::bits(w[2 * j]) | ((uint32_t)Elem<1>::bits(w[2 * j + 1]) << 16);
+        else u[j] = (uint32_t)__half_as_ushort(__float2half_rn(w[2 * j])) | ((uint32_t)__half_as_ushort(__float2half_rn(w[2 * j + 1])) << 16);
+    }
+    return kv_u4{u[0], u[1], u[2], u[3]};
+}
+// the inverse frequencies of all pairs, into LDS (the caller synchronises)
+__device__ __forceinline__ void rope_inv_table(const RopeDev &r, float *inv_s) {
+    for (int i = threadIdx.x; i < (r.dims >> 1); i += blockDim.x) inv_s[i] = rope_inv_freq(r, i);
+}
+// sines and cosines for the elements of the chunk at d0 < dims (one per pair: `traditional` chunks hold V / 2 pairs)
+template <int DT>
+__device__ __forceinline__ void rope_chunk_sincos(const RopeDev &r, const float *inv_s, int d0, int pos,
+                                                  float (&sn)[rope_chunk_elems<DT>()], float (&cs)[rope_chunk_elems<DT>()]) {
+    constexpr int V = rope_chunk_elems<DT>();
+    if (r.traditional) {
+#pragma unroll
+        for (int j = 0; j < V / 2; ++j) {
+            rope_sincos(rope_angle(r, pos, inv_s[d0 / 2 + j]), sn[2 * j], cs[2 * j]);
+            sn[2 * j + 1] = sn[2 * j];
+            cs[2 * j + 1] = cs[2 * j];
+        }
+    } else {
+        const int half = r.dims >> 1, i0 = d0 < half ? d0 : d0 - half;
+#pragma unroll
+        for (int j = 0; j < V; ++j) rope_sincos(rope_angle(r, pos, inv_s[i0 + j]), sn[j], cs[j]);
+    }
+}
+// The chunk at d0 < dims of a row, rotated and rounded to the dtype; `row` is the unrotated row.
+template <int DT>
+__device__ __forceinline__ void rope_chunk(const RopeDev &r, const float *inv_s, const char *row, int d0, int pos, const kv_u4 &raw,
+                                           float (&w)[rope_chunk_elems<DT>()]) {
+    constexpr int V = rope_chunk_elems<DT>();
+    const int half = r.dims >> 1;
+    const bool first = d0 < half;
+    float x[V], y[V], sn[V], cs[V];
+    chunk_unpack<DT>(raw, x);
+    if (!r.traditional)
+        chunk_unpack<DT>(*reinterpret_cast<const kv_u4 *>(row + (size_t)(first ? d0 + half : d0 - half) * (DT == 2 ? 4 : 2)), y);
+    rope_chunk_sincos<DT>(r, inv_s, d0, pos, sn, cs);
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+        w[j] = round_dt<DT>(r.traditional ? rope_turn(x[j], x[j ^ 1], (j & 1) == 0, sn[j], cs[j]) : rope_turn(x[j], y[j], first, sn[j], cs[j]));
+}
+
+// ---- the queries of a forward ----------------------------------------------------------------------------------
+// One row position (batch row b, row l of L) of `x` [B, H, L, D] into `out` (which may be x) for heads [h0, h1): a
+// thread owns one chunk pair (chunk, when the pairs are adjacent), works out its sines and cosines once and turns
+// that chunk pair of every head it takes.  `inv_s`: dims / 2 floats of LDS.  blockDim.x = 256.
+// Bound by the read and the write of the queries: 512 rows of 32 heads x 128 in bfloat16, 8.4 MB, see
+// rope_rows_kernel.
+template <int DT>
+__device__ __forceinline__ void rope_rows_body(const RopeDev &r, const char *x, char *out, int H, int L, int D, int b, int l,
+                                               int h0, int h1, float *inv_s) {
+    constexpr int V = rope_chunk_elems<DT>(), ES = DT == 2 ? 4 : 2;
+    const int half = r.dims >> 1;
+    const int np = r.traditional ? r.dims / V : half / V;  // rotating items of a head, then the chunks that pass through
+    const int items = np + (D - r.dims) / V;
+    const int item = threadIdx.x % items, slot = threadIdx.x / items, ns = 256 / items;
+    const bool live = slot < ns;
+    const bool turn = item < np;
+    const int d0 = turn ? item * V : r.dims + (item - np) * V;
+    const int d1 = turn && !r.traditional ? d0 + half : d0;
+    const size_t hs = (size_t)L * D * ES;
+    const size_t off = ((size_t)b * H * L + l) * D * ES;
+    int h = h0 + slot;
+    kv_u4 a{0u, 0u, 0u, 0u}, c{0u, 0u, 0u, 0u};
+    const bool some = live && h < h1;
+    if (some) {
+        a = *reinterpret_cast<const kv_u4 *>(x + off + h * hs + (size_t)d0 * ES);
+        c = *reinterpret_cast<const kv_u4 *>(x + off + h * hs + (size_t)d1 * ES);
+    }
+    rope_inv_table(r, inv_s);
+    __syncthreads();
+    if (!some) return;
+    float sn[V], cs[V];
+    if (turn) rope_chunk_sincos<DT>(r, inv_s, d0, (r.batch_pos ? r.batch_pos[b] : r.pos0) + l, sn, cs);
+    for (;;) {
+        const int hn = h + ns;
+        kv_u4 an = a, cn = c;
+        if (hn < h1) {
+            an = *reinterpret_cast<const kv_u4 *>(x + off + hn * hs + (size_t)d0 * ES);
+            cn = *reinterpret_cast<const kv_u4 *>(x + off + hn * hs + (size_t)d1 * ES);
+        }
+        if (turn) {
+            float xa[V], xc[V], ya[V], yc[V];
+            chunk_unpack<DT>(a, xa);
+            chunk_unpack<DT>(c, xc);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                if (r.traditional) {
+                    ya[j] = rope_turn(xa[j], xa[j ^ 1], (j & 1) == 0, sn[j], cs[j]);
+                } else {
+                    ya[j] = rope_turn(xa[j], xc[j], true, sn[j], cs[j]);
+                    yc[j] = rope_turn(xc[j], xa[j], false, sn[j], cs[j]);
+                }
+            }
+            a = chunk_pack<DT>(ya);
+            if (!r.traditional) *reinterpret_cast<kv_u4 *>(out + off + h * hs + (size_t)d1 * ES) = chunk_pack<DT>(yc);
+        }
+        *reinterpret_cast<kv_u4 *>(out + off + h * hs + (size_t)d0 * ES) = a;
+        if (hn >= h1) return;
+        h = hn;
+        a = an;
+        c = cn;
+    }
+}
+
+}  // namespace kvhip
