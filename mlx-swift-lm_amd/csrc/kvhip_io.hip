@@ -399,26 +399,36 @@ __global__ void __launch_bounds__(256) dequant_units_kernel(Store q, Store dst, 
     }
 }
 
-// grid (whole tiles, BH), 256 threads; 16-bit dtypes, Dk == 32 NCK, Dv == 32 NCV
+// grid (tiles touched, BH), 256 threads: rows src0 .. src0 + n - 1 to slots slot0 .. slot0 + n - 1, which may start and
+// end inside a tile; 16-bit dtypes, Dk == 32 NCK, Dv == 32 NCV
 template <int NCK, int NCV>
 __global__ void __launch_bounds__(256)
-append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, RopeDev rope) {
+append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, int n, RopeDev rope) {
     constexpr int DK = 32 * NCK, D = 32 * NCV;
     constexpr int TPRK = DK / 8, TPR = D / 8;
     constexpr int VPW = D / 2 + 1;  // dword pitch of a token's V row in LDS (odd: column reads spread over banks)
     __shared__ uint32_t vt[TILE * VPW];
     __shared__ float inv_s[DK / 2];
     const int bh = blockIdx.y;
-    const int slot_t = slot0 + blockIdx.x * TILE;
-    const int l_t = src0 + blockIdx.x * TILE;
-    const char *kbase = keys + ((size_t)bh * L + l_t) * DK * 2;
-    const char *vbase = values + ((size_t)bh * L + l_t) * D * 2;
+    const int slot_t = (slot0 & ~(TILE - 1)) + blockIdx.x * TILE;
+    const int l_t = src0 + slot_t - slot0;  // the row in the tile's first slot (before the first new row: t_lo > 0)
+    // tokens [t_lo, t_hi) of the tile are new; the threads of the others repeat the nearest new row and write nothing
+    const int t_lo = max(slot0 - slot_t, 0), t_hi = min(slot0 + n - slot_t, TILE);
+    const char *kbase = keys + ((ptrdiff_t)bh * L + l_t) * DK * 2;
+    const char *vbase = values + ((ptrdiff_t)bh * L + l_t) * D * 2;
+    auto new_row = [&](int r) { return min(max(r, t_lo), t_hi - 1); };
     char *kcell = st.pt[slot_t >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;  // a tile lies inside one page
     u4v kraw[NCK], vraw[NCV];
 #pragma unroll
-    for (int e = 0; e < NCK; ++e) kraw[e] = *reinterpret_cast<const u4v *>(kbase + (size_t)(e * 256 + threadIdx.x) * 16);
+    for (int e = 0; e < NCK; ++e) {
+        const int c = e * 256 + threadIdx.x, r = c / TPRK;
+        kraw[e] = *reinterpret_cast<const u4v *>(kbase + (ptrdiff_t)(c + (new_row(r) - r) * TPRK) * 16);
+    }
 #pragma unroll
-    for (int e = 0; e < NCV; ++e) vraw[e] = *reinterpret_cast<const u4v *>(vbase + (size_t)(e * 256 + threadIdx.x) * 16);
+    for (int e = 0; e < NCV; ++e) {
+        const int c = e * 256 + threadIdx.x, r = c / TPR;
+        vraw[e] = *reinterpret_cast<const u4v *>(vbase + (ptrdiff_t)(c + (new_row(r) - r) * TPR) * 16);
+    }
     if (rope.dims > 0) {
         rope_inv_table(rope, inv_s);
         __syncthreads();
@@ -429,8 +439,9 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
         const int r = c / TPRK, d0 = (c - r * TPRK) * 8;
         u4v k = kraw[e];
         if (rope.dims > 0 && d0 < rope.dims) {
-            const int pos = rope_pos(rope, bh, l_t + r);
-            const char *row = kbase + (size_t)r * DK * 2;
+            const int rn = new_row(r);
+            const int pos = rope_pos(rope, bh, l_t + rn);
+            const char *row = kbase + (ptrdiff_t)rn * DK * 2;
             float w[8];
             if (st.dtype == KVHIP_F16) {
                 unpack8<0>(k, row, d0, rope, inv_s, pos, w);
@@ -440,7 +451,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
                 k = chunk_pack<1>(w);
             }
         }
-        *reinterpret_cast<u4v *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
+        if (r >= t_lo && r < t_hi) *reinterpret_cast<u4v *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
     }
 #pragma unroll
     for (int e = 0; e < NCV; ++e) {
@@ -466,7 +477,14 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
             const uint32_t hi = vt16[(8 * c8 + 2 * j + 1) * (2 * VPW) + d];
             out[j] = lo | (hi << 16);
         }
-        *reinterpret_cast<u4v *>(cell + vfp_off(st, slot_t + 8 * c8, d)) = u4v{out[0], out[1], out[2], out[3]};
+        char *dst = cell + vfp_off(st, slot_t + 8 * c8, d);
+        if (8 * c8 >= t_lo && 8 * c8 + 8 <= t_hi) {
+            *reinterpret_cast<u4v *>(dst) = u4v{out[0], out[1], out[2], out[3]};
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (8 * c8 + j >= t_lo && 8 * c8 + j < t_hi) reinterpret_cast<uint16_t *>(dst)[j] = (uint16_t)(out[j >> 1] >> (16 * (j & 1)));
+        }
     }
 }
 
@@ -689,17 +707,6 @@ hipError_t launch_append_fp_rows(const Store &st, const void *keys, const void *
         hipLaunchKernelGGL(append_fp_kernel<4>, grid, block, 0, s, st, (const char *)keys, (const char *)values, L, src0, slot0, r);
     return hipGetLastError();
 }
-// slots [slot0, slot0 + n) as: rows up to the next tile boundary, whole tiles, remaining rows
-struct TileSplit {
-    int head, tiles, tail;
-};
-TileSplit tile_split(int slot0, int n) {
-    TileSplit t{0, 0, 0};
-    t.head = std::min(n, (TILE - (slot0 & (TILE - 1))) & (TILE - 1));
-    t.tiles = (n - t.head) / TILE;
-    t.tail = n - t.head - t.tiles * TILE;
-    return t;
-}
 }  // namespace
 
 hipError_t launch_append_fp(const Store &st, const void *keys, const void *values, int L, int src0,
@@ -708,22 +715,18 @@ hipError_t launch_append_fp(const Store &st, const void *keys, const void *value
     const RopeDev r = rope ? *rope : RopeDev();
     const bool mla = st.Dk == 192 && st.Dv == 128;  // keys of 192 with values of 128
     const bool tiled = st.es == 2 && ((st.Dk == st.Dv && (st.Dk == 64 || st.Dk == 96 || st.Dk == 128 || st.Dk == 256)) || mla);
-    const TileSplit t = tile_split(slot0, n);
-    if (!tiled || t.tiles == 0) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
-    hipError_t e = launch_append_fp_rows(st, keys, values, L, src0, slot0, t.head, s, r);
-    if (e != hipSuccess) return e;
-    dim3 grid(t.tiles, st.BH), block(256);
-    const int a0 = src0 + t.head, b0 = slot0 + t.head;
-#define FP_TILE(NCK, NCV) hipLaunchKernelGGL((append_fp_tile_kernel<NCK, NCV>), grid, block, 0, s, st, (const char *)keys, (const char *)values, L, a0, b0, r)
+    // One launch for whole tiles and the pieces of tiles at either end.  Fewer rows than a tile go one to a workgroup:
+    // that takes 5 us whatever their number, less than a tile's workgroup behind its barriers.
+    if (!tiled || n < TILE) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
+    dim3 grid(((slot0 & (TILE - 1)) + n + TILE - 1) / TILE, st.BH), block(256);
+#define FP_TILE(NCK, NCV) hipLaunchKernelGGL((append_fp_tile_kernel<NCK, NCV>), grid, block, 0, s, st, (const char *)keys, (const char *)values, L, src0, slot0, n, r)
     if (mla) FP_TILE(6, 4);
     else if (st.Dk == 64) FP_TILE(2, 2);
     else if (st.Dk == 96) FP_TILE(3, 3);
     else if (st.Dk == 128) FP_TILE(4, 4);
     else FP_TILE(8, 8);
 #undef FP_TILE
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_append_fp_rows(st, keys, values, L, a0 + t.tiles * TILE, b0 + t.tiles * TILE, t.tail, s, r);
+    return hipGetLastError();
 }
 
 hipError_t launch_rope_apply(const RopeDev &rope, const void *x, void *out, int B, int H, int L, int D,
@@ -767,21 +770,21 @@ hipError_t launch_append_quant_rows(const Store &st, const void *keys, const voi
 }
 }  // namespace
 
+// rows from which the whole-tile quantizer is the faster one
+constexpr int QUANT_TILE_ROWS = 9;
+
 hipError_t launch_append_quant(const Store &st, const void *keys, const void *values, int L, int src0,
                                int slot0, int n, hipStream_t s, const RopeDev *rope) {
     if (n <= 0) return hipSuccess;
     const RopeDev r = rope ? *rope : RopeDev();
     const bool tiled = quant_tiles_one_launch(st) || quant_tiles_two_sided(st);
-    const TileSplit t = tile_split(slot0, n);
-    if (!tiled || t.tiles == 0) return launch_append_quant_rows(st, keys, values, L, src0, slot0, n, s, r);
-    hipError_t e = launch_append_quant_rows(st, keys, values, L, src0, slot0, t.head, s, r);
-    if (e != hipSuccess) return e;
-    const int a0 = src0 + t.head, b0 = slot0 + t.head;
-    if (st.bits == 4) e = launch_quant_tiles_bits<4, true, false>(st, st, keys, values, L, a0, b0, t.tiles, s, r);
-    else if (st.bits == 8) e = launch_quant_tiles_bits<8, true, false>(st, st, keys, values, L, a0, b0, t.tiles, s, r);
-    else e = launch_quant_tiles_other(st, keys, values, L, a0, b0, t.tiles, s, r);
-    if (e != hipSuccess) return e;
-    return launch_append_quant_rows(st, keys, values, L, a0 + t.tiles * TILE, b0 + t.tiles * TILE, t.tail, s, r);
+    // The row kernel's wavefronts take their rows one after the other (about 2.6 us a row and wavefront: 33 us for 50
+    // rows of 128); one launch of the tile kernel takes every row of its tiles at once, 7 to 11 us whatever their number.
+    // A 501-row piece at an odd slot, rotated: 50 us as rows, whole tiles, rows (three launches), 11.5 us so.
+    if (!tiled || n < QUANT_TILE_ROWS) return launch_append_quant_rows(st, keys, values, L, src0, slot0, n, s, r);
+    if (st.bits == 4) return launch_quant_tiles_bits<4, true, false>(st, st, keys, values, L, src0, slot0, n, s, r);
+    if (st.bits == 8) return launch_quant_tiles_bits<8, true, false>(st, st, keys, values, L, src0, slot0, n, s, r);
+    return launch_quant_tiles_other(st, keys, values, L, src0, slot0, n, s, r);
 }
 
 hipError_t launch_requant_pages(const Store &src, const Store &st, int rows, hipStream_t s) {
@@ -798,9 +801,9 @@ hipError_t launch_requant_pages(const Store &src, const Store &st, int rows, hip
     // whole tiles, the last one included: its rows past `rows` hold zeros or rows trimmed earlier, and
     // what they quantize to lies past the new cache's offset, where the next append overwrites it
     const RopeDev none;
-    if (st.bits == 4) return launch_quant_tiles_bits<4, true, true>(st, src, nullptr, nullptr, 0, 0, 0, tiles, s, none);
-    if (st.bits == 8) return launch_quant_tiles_bits<8, true, true>(st, src, nullptr, nullptr, 0, 0, 0, tiles, s, none);
-    return launch_requant_tiles_other(src, st, tiles, s);
+    if (st.bits == 4) return launch_quant_tiles_bits<4, true, true>(st, src, nullptr, nullptr, 0, 0, 0, rows, s, none);
+    if (st.bits == 8) return launch_quant_tiles_bits<8, true, true>(st, src, nullptr, nullptr, 0, 0, 0, rows, s, none);
+    return launch_requant_tiles_other(src, st, rows, s);
 }
 
 hipError_t launch_dequant_pages(const Store &q, const Store &dst, int rows, hipStream_t s) {

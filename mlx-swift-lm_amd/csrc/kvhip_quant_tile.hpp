@@ -85,7 +85,8 @@ template <int DT> __device__ __forceinline__ uint32_t pack_scale_bias(float scal
     return (uint32_t)Elem<1>::bits(scale) | ((uint32_t)Elem<1>::bits(bias) << 16);
 }
 
-// grid (whole tiles, BH), 256 threads; slot0 is a multiple of 64; 16-bit dtypes, Dk == Dv == 32 NC;
+// grid (tiles touched, BH), 256 threads: rows src0 .. src0 + n - 1 go to slots slot0 .. slot0 + n - 1, which may start
+// and end inside a tile; 16-bit dtypes, Dk == Dv == 32 NC;
 // GL = group size / 8 lanes share a quantization group; ROPE = false carries no rotation code.
 // A thread holds 16-byte chunks of K and of V rows (a "chunk-instance" each), up to eight at a
 // time.  The extrema of every chunk-instance are reduced over the lanes of its group; then the
@@ -99,7 +100,7 @@ template <int DT> __device__ __forceinline__ uint32_t pack_scale_bias(float scal
 // values differ in head size take one launch for each, NC being that side's).
 template <int DT, int BITS, int NC, int GL, bool ROPE, bool PAGED, int SIDE = 0>
 __device__ __forceinline__ void append_quant_tile_body(const Store &st, const Store &src, const char *keys, const char *values,
-                                                       int L, int src0, int slot0, const RopeDev &rope) {
+                                                       int L, int src0, int slot0, int n, const RopeDev &rope) {
     constexpr int D = 32 * NC;
     constexpr int GS = 8 * GL;
     constexpr int TPR = D / 8;   // threads per row
@@ -123,10 +124,14 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
     __shared__ float inv_s[ROPE ? D / 2 : 1];
     __shared__ __attribute__((aligned(16))) uint8_t vstage[PAGED && DO_V ? TILE * D * 2 : 16];  // the source V tile as stored
     const int bh = blockIdx.y;
-    const int slot_t = slot0 + blockIdx.x * TILE;
-    const int l_t = src0 + blockIdx.x * TILE;
-    const char *kbase = PAGED ? nullptr : keys + ((size_t)bh * L + l_t) * D * 2;
-    const char *vbase = PAGED ? nullptr : values + ((size_t)bh * L + l_t) * D * 2;
+    const int slot_t = (slot0 & ~(TILE - 1)) + blockIdx.x * TILE;
+    const int l_t = src0 + slot_t - slot0;  // the row in the tile's first slot (before the first new row: t_lo > 0)
+    // tokens [t_lo, t_hi) of the tile are new.  The threads of the others repeat the nearest new row, which keeps their
+    // loads inside the arrays, and write nothing.
+    const int t_lo = PAGED ? 0 : max(slot0 - slot_t, 0), t_hi = PAGED ? TILE : min(slot0 + n - slot_t, TILE);
+    const bool whole = t_lo == 0 && t_hi == TILE;
+    const char *kbase = PAGED ? nullptr : keys + ((ptrdiff_t)bh * L + l_t) * D * 2;
+    const char *vbase = PAGED ? nullptr : values + ((ptrdiff_t)bh * L + l_t) * D * 2;
     u4v kraw[NC], vraw[NC];
     if constexpr (PAGED) {
         const char *kt = k_cell_ptr(src, bh, l_t) + kfp_off(src, l_t, 0);   // tile start: [chunk][token][16 B]
@@ -152,9 +157,10 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
     } else {
 #pragma unroll
         for (int e = 0; e < NC; ++e) {
-            const int c = e * 256 + threadIdx.x;
-            if constexpr (DO_K) kraw[e] = *reinterpret_cast<const u4v *>(kbase + (size_t)c * 16);
-            if constexpr (DO_V) vraw[e] = *reinterpret_cast<const u4v *>(vbase + (size_t)c * 16);
+            const int c = e * 256 + threadIdx.x, r = c / TPR;
+            const int cc = c + (min(max(r, t_lo), t_hi - 1) - r) * TPR;
+            if constexpr (DO_K) kraw[e] = *reinterpret_cast<const u4v *>(kbase + (ptrdiff_t)cc * 16);
+            if constexpr (DO_V) vraw[e] = *reinterpret_cast<const u4v *>(vbase + (ptrdiff_t)cc * 16);
         }
     }
     if constexpr (ROPE) {
@@ -180,7 +186,7 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
             const int e = e0 + chunk_of(i);
             const int d0 = col_of(e);
             if (!is_v(i)) {
-                const int r = row_of(e);
+                const int r = min(max(row_of(e), t_lo), t_hi - 1);
                 if constexpr (ROPE) unpack8<DT>(kraw[e], kbase + (size_t)r * D * 2, d0, rope, inv_s, rope_pos(rope, bh, l_t + r), w[i]);
                 else chunk_unpack<DT>(kraw[e], w[i]);
             } else {
@@ -208,9 +214,10 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
                 }
             affine_params(a, b, nb, sc[k], bi[k]);
             iv[k] = __builtin_amdgcn_rcpf(sc[k]);
-            if (pos < SH && psel + k * SH < NI) {
+            const int t_sb = row_of(e0 + chunk_of(psel + k * SH));
+            if (pos < SH && psel + k * SH < NI && t_sb >= t_lo && t_sb < t_hi) {
                 const int i = psel + k * SH;  // this lane's chunk-instance
-                const int row = page_off + row_of(e0 + chunk_of(i));
+                const int row = page_off + t_sb;
                 const int d0 = col_of(e0 + chunk_of(i));
                 char *sb = is_v(i) ? page.vsb + (size_t)bh * st.vsb_cell + (size_t)row * st.vsb_row
                                    : page.ksb + (size_t)bh * st.ksb_cell + (size_t)row * st.ksb_row;
@@ -230,6 +237,7 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
             if (!is_v(i)) {
                 // ---- K: packed words in natural order --------------------------------------------
                 uint32_t *kw = reinterpret_cast<uint32_t *>(page.k + (size_t)bh * st.k_cell + (size_t)(page_off + r) * st.k_row);
+                if (!GEN && (r < t_lo || r >= t_hi)) continue;
                 if constexpr (BITS == 4) {
                     kw[d0 / 8] = pack_nibbles(q[0], q[1], q[2], q[3]) | (pack_nibbles(q[4], q[5], q[6], q[7]) << 16);
                 } else if constexpr (BITS == 8) {
@@ -255,8 +263,14 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
     if constexpr (GEN && DO_K) {
         __syncthreads();
         char *kt = page.k + (size_t)bh * st.k_cell + (size_t)page_off * st.k_row;  // 64 rows of D BITS / 8 bytes, contiguous
-        for (int c = threadIdx.x; c < TILE * D * BITS / 8 / 16; c += 256)
-            *reinterpret_cast<u4v *>(kt + (size_t)c * 16) = *reinterpret_cast<const u4v *>(&kcodes[c * 16]);
+        if (whole) {
+            for (int c = threadIdx.x; c < TILE * D * BITS / 8 / 16; c += 256)
+                *reinterpret_cast<u4v *>(kt + (size_t)c * 16) = *reinterpret_cast<const u4v *>(&kcodes[c * 16]);
+        } else {  // (rows are whole words: D is a multiple of 32)
+            constexpr int RW = D * BITS / 32;
+            for (int c = t_lo * RW + threadIdx.x; c < t_hi * RW; c += 256)
+                reinterpret_cast<uint32_t *>(kt)[c] = reinterpret_cast<const uint32_t *>(kcodes)[c];
+        }
     }
     if constexpr (!DO_V) return;
     if constexpr (!(GEN && DO_K)) __syncthreads();
@@ -268,13 +282,18 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
         for (int c = threadIdx.x; c < D * WPR; c += 256) {
             const int d = c / WPR, w = c - d * WPR;
             const int t0 = (32 * w) / BITS;  // the first token with bits in word w
-            uint32_t word = 0;
+            uint32_t word = 0, mine = 0;  // (mine: the bits of new tokens)
 #pragma unroll
             for (int i = 0; i < 32 / BITS + 2; ++i) {
                 const int t = t0 + i;
-                if (t < TILE && t * BITS < 32 * w + 32) word |= stream_bits(vcodes[t * VP + d], t * BITS, w);
+                if (t < TILE && t * BITS < 32 * w + 32 && t >= t_lo && t < t_hi) {
+                    word |= stream_bits(vcodes[t * VP + d], t * BITS, w);
+                    mine |= stream_bits((1u << BITS) - 1u, t * BITS, w);
+                }
             }
-            reinterpret_cast<uint32_t *>(cell + (size_t)d * (TILE * BITS / 8))[w] = word;
+            uint32_t *p = reinterpret_cast<uint32_t *>(cell + (size_t)d * (TILE * BITS / 8)) + w;
+            if (mine == 0xffffffffu) *p = word;
+            else if (mine != 0) *p = (*p & ~mine) | word;
         }
         return;
     }
@@ -295,20 +314,36 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
             }
             out[wi] = word;
         }
-        *reinterpret_cast<u4v *>(cell + (size_t)d * (TILE * BITS / 8) + 16 * q) = u4v{out[0], out[1], out[2], out[3]};
+        char *dst = cell + (size_t)d * (TILE * BITS / 8) + 16 * q;
+        if (whole) {
+            *reinterpret_cast<u4v *>(dst) = u4v{out[0], out[1], out[2], out[3]};
+        } else {
+#pragma unroll
+            for (int wi = 0; wi < 4; ++wi) {
+                uint32_t mine = 0;  // the bits of new tokens in this word
+#pragma unroll
+                for (int tt = 0; tt < TPW; ++tt) {
+                    const int t = (4 * q + wi) * TPW + tt;
+                    if (t >= t_lo && t < t_hi) mine |= ((1u << BITS) - 1u) << (v_bitpos<BITS>(t) & 31);
+                }
+                uint32_t *p = reinterpret_cast<uint32_t *>(dst) + wi;
+                if (mine == 0xffffffffu) *p = out[wi];
+                else if (mine != 0) *p = (*p & ~mine) | (out[wi] & mine);
+            }
+        }
     }
 }
 
 template <int DT, int BITS, int NC, int GL, bool ROPE, int SIDE = 0>
 __global__ void __launch_bounds__(256)
-append_quant_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, RopeDev rope) {
-    append_quant_tile_body<DT, BITS, NC, GL, ROPE, false, SIDE>(st, st, keys, values, L, src0, slot0, rope);
+append_quant_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, int n, RopeDev rope) {
+    append_quant_tile_body<DT, BITS, NC, GL, ROPE, false, SIDE>(st, st, keys, values, L, src0, slot0, n, rope);
 }
 
 // grid (tiles, BH): tiles [0, gridDim.x) of the full-precision store `src` into the same slots of `st`
 template <int DT, int BITS, int NC, int GL, int SIDE = 0>
 __global__ void __launch_bounds__(256) requant_tile_kernel(Store st, Store src) {
-    append_quant_tile_body<DT, BITS, NC, GL, false, true, SIDE>(st, src, nullptr, nullptr, 0, 0, 0, RopeDev());
+    append_quant_tile_body<DT, BITS, NC, GL, false, true, SIDE>(st, src, nullptr, nullptr, 0, 0, 0, 0, RopeDev());
 }
 
 // Which stores the tile kernels take: 16-bit dtypes, group size 32 / 64 / 128 dividing the head size; keys and
@@ -322,29 +357,29 @@ inline bool quant_tiles_two_sided(const Store &st) {
     return st.es == 2 && st.Dk == 192 && st.Dv == 128 && (st.bits == 4 || st.bits == 8) && (st.gs == 32 || st.gs == 64);
 }
 
-// The launches of one code width.  PAGED = false: `tiles` whole tiles of the dense rows from row a0 on into the slots
-// from b0 on (a multiple of 64); PAGED = true: tiles [0, tiles) of the full-precision store `src` into the same slots.
+// The launches of one code width.  PAGED = false: `n` dense rows from row a0 on into the slots from b0 on; PAGED = true:
+// the tiles that hold rows [0, n) of the full-precision store `src` into the same slots.
 // TWO_SIDED: also the instances for keys of 192 with values of 128.
 template <int DT, int BITS, int NC, int GL, int SIDE, bool PAGED>
 void launch_quant_tile_instance(const Store &st, const Store &src, const void *keys, const void *values, int L, int a0,
-                                int b0, int tiles, hipStream_t s, const RopeDev &r) {
-    dim3 grid(tiles, st.BH), block(256);
+                                int b0, int n, hipStream_t s, const RopeDev &r) {
+    dim3 grid((PAGED ? (n + TILE - 1) : ((b0 & (TILE - 1)) + n + TILE - 1)) / TILE, st.BH), block(256);
     if constexpr (PAGED) {
         hipLaunchKernelGGL((requant_tile_kernel<DT, BITS, NC, GL, SIDE>), grid, block, 0, s, st, src);
     } else {
         if (r.dims > 0 && SIDE != 2)
             hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, true, SIDE>), grid, block, 0, s, st,
-                               (const char *)keys, (const char *)values, L, a0, b0, r);
+                               (const char *)keys, (const char *)values, L, a0, b0, n, r);
         else
             hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, false, SIDE>), grid, block, 0, s, st,
-                               (const char *)keys, (const char *)values, L, a0, b0, r);
+                               (const char *)keys, (const char *)values, L, a0, b0, n, r);
     }
 }
 
 template <int DT, int BITS, bool TWO_SIDED, bool PAGED>
 hipError_t launch_quant_tiles_dt(const Store &st, const Store &src, const void *keys, const void *values, int L, int a0,
-                                 int b0, int tiles, hipStream_t s, const RopeDev &r) {
-#define KV_TILE(NC, GL, SIDE) launch_quant_tile_instance<DT, BITS, NC, GL, SIDE, PAGED>(st, src, keys, values, L, a0, b0, tiles, s, r)
+                                 int b0, int n, hipStream_t s, const RopeDev &r) {
+#define KV_TILE(NC, GL, SIDE) launch_quant_tile_instance<DT, BITS, NC, GL, SIDE, PAGED>(st, src, keys, values, L, a0, b0, n, s, r)
 #define KV_TILE_GL(NC)                        \
     do {                                      \
         if (st.gs == 32) KV_TILE(NC, 4, 0);   \
@@ -377,10 +412,10 @@ hipError_t launch_quant_tiles_dt(const Store &st, const Store &src, const void *
 
 template <int BITS, bool TWO_SIDED, bool PAGED>
 hipError_t launch_quant_tiles_bits(const Store &st, const Store &src, const void *keys, const void *values, int L, int a0,
-                                   int b0, int tiles, hipStream_t s, const RopeDev &r) {
-    if (tiles <= 0) return hipSuccess;
-    if (st.dtype == KVHIP_F16) return launch_quant_tiles_dt<0, BITS, TWO_SIDED, PAGED>(st, src, keys, values, L, a0, b0, tiles, s, r);
-    if (st.dtype == KVHIP_BF16) return launch_quant_tiles_dt<1, BITS, TWO_SIDED, PAGED>(st, src, keys, values, L, a0, b0, tiles, s, r);
+                                   int b0, int n, hipStream_t s, const RopeDev &r) {
+    if (n <= 0) return hipSuccess;
+    if (st.dtype == KVHIP_F16) return launch_quant_tiles_dt<0, BITS, TWO_SIDED, PAGED>(st, src, keys, values, L, a0, b0, n, s, r);
+    if (st.dtype == KVHIP_BF16) return launch_quant_tiles_dt<1, BITS, TWO_SIDED, PAGED>(st, src, keys, values, L, a0, b0, n, s, r);
     return hipErrorInvalidValue;
 }
 
