@@ -305,6 +305,9 @@ int32_t kvhip_cache_state_count(const kvhip_cache *cache);
 kvhip_status kvhip_cache_state_desc(const kvhip_cache *cache, int32_t index, int64_t shape[4],
                                     int32_t *dtype);
 kvhip_status kvhip_cache_state_export(const kvhip_cache *cache, int32_t index, void *dst, void *stream);
+/* Every state array in one call (quantized caches: one launch); `count` is kvhip_cache_state_count, dsts[i] what
+   kvhip_cache_state_export would take for array i. */
+kvhip_status kvhip_cache_state_export_all(const kvhip_cache *cache, int32_t count, void *const *dsts, void *stream);
 /*
  * `state` setter (KVCache.swift:461-468, :764-773, :1131-1146): `count` arrays in
  * the getter's order, shapes[i] = 4 extents, dtypes[i] a kvhip_dtype.  Simple

@@ -1419,7 +1419,9 @@ kvhip_status kvhip_cache_state_export(const kvhip_cache *c, int32_t i, void *dst
     if (!dst) return fail(KVHIP_ERR_INVALID_ARG, "null argument");
     if (c->kind == KVHIP_KIND_QUANTIZED) {
         if (!c->padded()) {
-            KV_HIP(launch_export_quant(c->st, i, (int)n, dst, S(c, stream)));
+            QuantArrays one;
+            one.a[i] = dst;
+            KV_HIP(launch_export_quant(c->st, one, (int)n, S(c, stream)));
             return KVHIP_OK;
         }
         // the array of the stored width first, then its leading columns (codes are a bit stream from column 0 on,
@@ -1432,7 +1434,9 @@ kvhip_status kvhip_cache_state_export(const kvhip_cache *c, int32_t i, void *dst
         void *tmp = nullptr;
         size_t got = 0;
         KV_HIP(pool_alloc(&tmp, rows * wide, &got));
-        hipError_t e = launch_export_quant(st, i, (int)n, tmp, S(c, stream));
+        QuantArrays one;
+        one.a[i] = tmp;
+        hipError_t e = launch_export_quant(st, one, (int)n, S(c, stream));
         if (e == hipSuccess) e = launch_repitch_rows(dst, narrow, tmp, wide, rows, S(c, stream));
         std::vector<std::pair<void *, size_t>> t{{tmp, got}};
         retire(std::move(t), S(c, stream));
@@ -1447,6 +1451,24 @@ kvhip_status kvhip_cache_state_export(const kvhip_cache *c, int32_t i, void *dst
         slots = ident.data();
     }
     return export_slots(c, slots, n, i == 0 ? dst : nullptr, i == 1 ? dst : nullptr, S(c, stream));
+}
+
+kvhip_status kvhip_cache_state_export_all(const kvhip_cache *c, int32_t count, void *const *dsts, void *stream) {
+    if (!c || !dsts) return fail(KVHIP_ERR_INVALID_ARG, "null argument");
+    if (count != kvhip_cache_state_count(c)) return fail(KVHIP_ERR_INVALID_ARG, "one destination per state array");
+    if (c->kind != KVHIP_KIND_QUANTIZED || c->padded()) {
+        for (int32_t i = 0; i < count; ++i) KV_TRY(kvhip_cache_state_export(c, i, dsts[i], stream));
+        return KVHIP_OK;
+    }
+    const int64_t n = state_rows(c);
+    if (count == 0 || n == 0) return KVHIP_OK;
+    QuantArrays all;
+    for (int i = 0; i < 6; ++i) {
+        if (!dsts[i]) return fail(KVHIP_ERR_INVALID_ARG, "null argument");
+        all.a[i] = dsts[i];
+    }
+    KV_HIP(launch_export_quant(c->st, all, (int)n, S(c, stream)));
+    return KVHIP_OK;
 }
 
 kvhip_status kvhip_cache_state_import(kvhip_cache *c, int32_t count, const void *const *srcs,

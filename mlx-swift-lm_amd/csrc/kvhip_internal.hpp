@@ -237,8 +237,12 @@ hipError_t launch_rope_apply(const RopeDev &rope, const void *x, void *out, int 
 // row 0 corresponds to row dst_row0 of `runs`.  Either destination may be NULL.
 hipError_t launch_export_fp(const Store &st, const Runs &runs, int row_begin, int count, int dst_row0,
                             int dst_rows, void *dst_k, void *dst_v, hipStream_t s);
-// which: 0 k.wq 1 k.scales 2 k.biases 3 v.wq 4 v.scales 5 v.biases
-hipError_t launch_export_quant(const Store &st, int which, int nrows, void *dst, hipStream_t s);
+// The six dense arrays of a quantized state: 0 k.wq 1 k.scales 2 k.biases 3 v.wq 4 v.scales 5 v.biases
+struct QuantArrays {
+    void *a[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+};
+// rows [0, nrows) into the arrays that are not null
+hipError_t launch_export_quant(const Store &st, const QuantArrays &out, int nrows, hipStream_t s);
 // Dense [BH, nrows, D] arrays into slots [0, nrows).
 hipError_t launch_import_fp(const Store &st, const void *src_k, const void *src_v, int nrows, hipStream_t s);
 hipError_t launch_import_quant(const Store &st, const void *const srcs[6], int nrows, hipStream_t s);

@@ -538,49 +538,84 @@ __global__ void compact_fp_kernel(Store src, Runs runs, Store dst, int nrows) {
         *reinterpret_cast<E *>(vd + vfp_off(dst, i, d)) = *reinterpret_cast<const E *>(vs + vfp_off(src, slot, d));
 }
 
-// which: 0 k.wq 1 k.scales 2 k.biases 3 v.wq 4 v.scales 5 v.biases; grid (nrows, BH)
-template <int BITS>
-__global__ void export_quant_kernel(Store st, int which, int nrows, char *dst) {
-    const int bh = blockIdx.y;
-    const int slot = blockIdx.x;
-    const int es = st.es;
-    if (which == 0) {
-        const int W = st.Dk * BITS / 32;
-        const uint32_t *s = reinterpret_cast<const uint32_t *>(k_row_ptr(st, bh, slot));
-        uint32_t *d = reinterpret_cast<uint32_t *>(dst) + ((size_t)bh * nrows + slot) * W;
-        for (int w = threadIdx.x; w < W; w += blockDim.x) d[w] = s[w];
-    } else if (which == 3) {
-        constexpr int per = 32 / BITS;
-        const int W = st.Dv * BITS / 32;
-        const char *cell = v_cell_ptr(st, bh, slot);
-        const int t = slot & (TILE - 1);
-        uint32_t *d = reinterpret_cast<uint32_t *>(dst) + ((size_t)bh * nrows + slot) * W;
-        for (int w = threadIdx.x; w < W; w += blockDim.x) {
+// The arrays of a quantized state, any of the six (null: not asked for).  grid (64-token tiles, BH), 256 threads: K rows
+// are contiguous in page and array alike and are copied (VEC: as 16-byte pieces); V rows are put together from the
+// transposed tile, 128 columns at a time through LDS, lanes taking the tokens of a column (their codes lie in adjacent
+// dwords: no bank conflicts); pairs are split into scales and biases.  A row to a workgroup and an array to a launch,
+// as it was, takes 19 us an array for 5000 rows of 16 (batch, head) pairs x 128 at 4 bits; four such caches converted
+// and read out: 630 us then, 188 us in one launch a cache.
+template <int BITS, bool VEC>
+__global__ void __launch_bounds__(256) export_quant_kernel(Store st, QuantArrays out, int nrows) {
+    constexpr int CB = 128;  // columns per round
+    __shared__ __attribute__((aligned(16))) uint32_t vs[CB * 2 * BITS];
+    const int bh = blockIdx.y, lo = blockIdx.x * TILE, n = min(TILE, nrows - lo);
+    const int tid = threadIdx.x;
+    const size_t row0 = (size_t)bh * nrows + lo;
+    if (out.a[0]) {
+        const char *src = k_row_ptr(st, bh, lo);
+        char *dst = static_cast<char *>(out.a[0]) + row0 * st.k_row;
+        if (VEC) {
+            for (int i = tid; i < n * (int)(st.k_row / 16); i += 256)
+                reinterpret_cast<u4v *>(dst)[i] = reinterpret_cast<const u4v *>(src)[i];
+        } else {
+            for (int i = tid; i < n * (int)(st.k_row / 4); i += 256)
+                reinterpret_cast<uint32_t *>(dst)[i] = reinterpret_cast<const uint32_t *>(src)[i];
+        }
+    }
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        void *sc = out.a[1 + 3 * side], *bi = out.a[2 + 3 * side];
+        if (!sc && !bi) continue;
+        const char *src = side == 0 ? ksb_row_ptr(st, bh, lo) : vsb_row_ptr(st, bh, lo);
+        const int G = (side == 0 ? st.Dk : st.Dv) / st.gs;
+        for (int i = tid; i < n * G; i += 256) {
+            if (st.es == 2) {
+                const uint32_t pair = reinterpret_cast<const uint32_t *>(src)[i];
+                if (sc) reinterpret_cast<uint16_t *>(sc)[row0 * G + i] = (uint16_t)pair;
+                if (bi) reinterpret_cast<uint16_t *>(bi)[row0 * G + i] = (uint16_t)(pair >> 16);
+            } else {
+                const uint2 pair = reinterpret_cast<const uint2 *>(src)[i];
+                if (sc) reinterpret_cast<uint32_t *>(sc)[row0 * G + i] = pair.x;
+                if (bi) reinterpret_cast<uint32_t *>(bi)[row0 * G + i] = pair.y;
+            }
+        }
+    }
+    if (!out.a[3]) return;
+    const int W = st.Dv * BITS / 32;
+    const char *cell = v_cell_ptr(st, bh, lo) + v_row_off(st, lo, 0);
+    uint32_t *dst = static_cast<uint32_t *>(out.a[3]) + row0 * W;
+    for (int c0 = 0; c0 < st.Dv; c0 += CB) {
+        const int cols = min(CB, st.Dv - c0), words = cols * BITS / 32;  // (head sizes are multiples of 32 columns)
+        __syncthreads();
+        for (int i = tid; i < cols * BITS / 2; i += 256)
+            reinterpret_cast<u4v *>(vs)[i] = reinterpret_cast<const u4v *>(cell + (size_t)c0 * (8 * BITS))[i];
+        __syncthreads();
+        auto word_of = [&](int t, int w) -> uint32_t {
             uint32_t word = 0;
             if constexpr ((32 % BITS) == 0) {
+                constexpr int per = 32 / BITS;
+#pragma unroll
                 for (int i = 0; i < per; ++i)
-                    word |= v_code_load<BITS>(cell + v_row_off(st, slot, w * per + i), t) << (i * BITS);
+                    word |= v_code_load<BITS>(reinterpret_cast<const char *>(vs + (w * per + i) * 2 * BITS), t) << (i * BITS);
             } else {
                 const int j0 = (32 * w) / BITS;  // the first column with bits in word w of the row's bit stream
-                for (int i = 0; i < per + 2; ++i) {
+#pragma unroll
+                for (int i = 0; i < 32 / BITS + 2; ++i) {
                     const int j = j0 + i;
-                    if (j < st.Dv && j * BITS < 32 * w + 32)
-                        word |= stream_bits(v_code_load<BITS>(cell + v_row_off(st, slot, j), t), j * BITS, w);
+                    if (j < cols && j * BITS < 32 * w + 32)
+                        word |= stream_bits(v_code_load<BITS>(reinterpret_cast<const char *>(vs + j * 2 * BITS), t), j * BITS, w);
                 }
             }
-            d[w] = word;
-        }
-    } else {
-        const bool isk = which < 3;
-        const int G = (isk ? st.Dk : st.Dv) / st.gs;
-        const int comp = (which == 1 || which == 4) ? 0 : 1;
-        const char *s = isk ? ksb_row_ptr(st, bh, slot) : vsb_row_ptr(st, bh, slot);
-        char *d = dst + ((size_t)bh * nrows + slot) * G * es;
-        for (int g = threadIdx.x; g < G; g += blockDim.x) {
-            if (es == 2)
-                reinterpret_cast<uint16_t *>(d)[g] = reinterpret_cast<const uint16_t *>(s)[2 * g + comp];
-            else
-                reinterpret_cast<uint32_t *>(d)[g] = reinterpret_cast<const uint32_t *>(s)[2 * g + comp];
+            return word;
+        };
+        const int t = tid & (TILE - 1);
+        if (t >= n) continue;
+        uint32_t *row = dst + (size_t)t * W + c0 * BITS / 32;
+        if (VEC && words % 4 == 0) {
+            for (int w = (tid >> 6) * 4; w < words; w += 16)
+                *reinterpret_cast<u4v *>(row + w) = u4v{word_of(t, w), word_of(t, w + 1), word_of(t, w + 2), word_of(t, w + 3)};
+        } else {
+            for (int w = tid >> 6; w < words; w += 4) row[w] = word_of(t, w);
         }
     }
 }
@@ -883,10 +918,17 @@ hipError_t launch_compact_fp(const Store &src, const Runs &runs, const Store &ds
     return hipGetLastError();
 }
 
-hipError_t launch_export_quant(const Store &st, int which, int nrows, void *dst, hipStream_t s) {
+hipError_t launch_export_quant(const Store &st, const QuantArrays &out, int nrows, hipStream_t s) {
     if (nrows <= 0) return hipSuccess;
-    dim3 grid(nrows, st.BH), block(64);
-#define EXP(BITS) hipLaunchKernelGGL(export_quant_kernel<BITS>, grid, block, 0, s, st, which, nrows, (char *)dst)
+    dim3 grid((nrows + TILE - 1) / TILE, st.BH), block(256);
+    // 16-byte pieces where every row of both code arrays starts on a 16-byte boundary
+    const bool vec = st.k_row % 16 == 0 && (st.Dv * st.bits / 8) % 16 == 0 &&
+                     ((reinterpret_cast<uintptr_t>(out.a[0]) | reinterpret_cast<uintptr_t>(out.a[3])) & 15) == 0;
+#define EXP(BITS)                                                                                        \
+    do {                                                                                                 \
+        if (vec) hipLaunchKernelGGL((export_quant_kernel<BITS, true>), grid, block, 0, s, st, out, nrows); \
+        else hipLaunchKernelGGL((export_quant_kernel<BITS, false>), grid, block, 0, s, st, out, nrows);    \
+    } while (0)
     switch (st.bits) {
         case 4: EXP(4); break;
         case 8: EXP(8); break;

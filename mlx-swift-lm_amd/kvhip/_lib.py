@@ -86,6 +86,7 @@ SIGNATURES = {
     "kvhip_cache_state_count": (_I32, [_P]),
     "kvhip_cache_state_desc": (_I32, [_P, _I32, C.POINTER(_I64 * 4), C.POINTER(_I32)]),
     "kvhip_cache_state_export": (_I32, [_P, _I32, _P, _P]),
+    "kvhip_cache_state_export_all": (_I32, [_P, _I32, C.POINTER(_P), _P]),
     "kvhip_cache_state_import": (_I32, [_P, _I32, C.POINTER(_P), C.POINTER(_I64), C.POINTER(_I32), _P]),
     "kvhip_cache_meta_count": (_I32, [_P]),
     "kvhip_cache_meta_get": (_I32, [_P, _I32, C.c_char_p, _I32]),

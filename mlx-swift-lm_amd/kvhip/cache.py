@@ -276,9 +276,10 @@ class _Cache:
             shape = (C.c_int64 * 4)()
             dt = C.c_int32()
             L.check(self._lib.kvhip_cache_state_desc(self._h, i, C.byref(shape), C.byref(dt)))
-            t = torch.empty(tuple(shape), dtype=_TORCH[dt.value], device="cuda")
-            L.check(self._lib.kvhip_cache_state_export(self._h, i, _ptr(t), _stream()))
-            out.append(t)
+            out.append(torch.empty(tuple(shape), dtype=_TORCH[dt.value], device="cuda"))
+        if n:
+            dsts = (C.c_void_p * n)(*[t.data_ptr() for t in out])
+            L.check(self._lib.kvhip_cache_state_export_all(self._h, n, dsts, _stream()))
         return out
 
     @state.setter
