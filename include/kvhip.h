@@ -230,6 +230,15 @@ kvhip_status kvhip_cache_update_rope(kvhip_cache *cache, const kvhip_rope *rope,
                                      const void *keys, const void *values, int32_t B, int32_t Hkv,
                                      int32_t L, int32_t Dk, int32_t Dv, int32_t dtype, void *stream);
 
+/* An attention layer's call sequence (Llama.swift:58-70) in one: kvhip_rope_apply on the queries and
+ * kvhip_cache_update_rope at the cache's `ropeOffset` (or at batch_offsets), then kvhip_cache_attend.  The queries
+ * turn in the append's launch where their rows are whole 16-byte chunks.  `q_rotated`: device scratch of the
+ * queries' size that holds them in between (it may be `queries`); NULL: a buffer the cache keeps for it. */
+kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *cache, const kvhip_rope *rope, const int32_t *batch_offsets,
+                                            const void *queries, const void *keys, const void *values, int32_t B,
+                                            int32_t Hq, int32_t Hkv, int32_t L, int32_t Dk, int32_t Dv, int32_t dtype,
+                                            float scale, const kvhip_mask *mask, void *q_rotated, void *out, void *stream);
+
 /* The arrays the last `update` returned: dst_keys [B,Hkv,P,Dk], dst_values
  * [B,Hkv,P,Dv], P = kvhip_cache_presented_length.  Not for quantized caches. */
 kvhip_status kvhip_cache_fetch(const kvhip_cache *cache, void *dst_keys, void *dst_values, void *stream);

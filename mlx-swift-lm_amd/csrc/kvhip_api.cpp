@@ -98,8 +98,10 @@ struct kvhip_cache {
     // zero value columns give output columns nobody reads), arrays are widened on the way in and narrowed on the
     // way out, and everything between works on the stored sizes.
     int Dk_user = 0, Dv_user = 0;
-    void *pad_buf[4] = {nullptr, nullptr, nullptr, nullptr};  // widened keys, values, queries; outputs before narrowing
-    size_t pad_bytes[4] = {0, 0, 0, 0};
+    // widened keys, values, queries; outputs before narrowing; the rotated queries of a step
+    static constexpr int PAD_BUFS = 5;
+    void *pad_buf[PAD_BUFS] = {};
+    size_t pad_bytes[PAD_BUFS] = {};
     std::vector<Slab> slabs;   // the allocations behind the pages, in page order
     int64_t cap_pages = 0;     // pages allocated (= page-table entries in use)
     int64_t pt_cap = 0;        // entries the device page table has room for
@@ -115,7 +117,7 @@ struct kvhip_cache {
     int64_t presented_live = 0;       // `presented` of the live ring when the round opened
     void *stage_tmp_k = nullptr, *stage_tmp_v = nullptr;  // dense copy of the rows a commit keeps
     size_t stage_tmp_rows = 0;
-    const RopeDev *rope = nullptr;  // set for the duration of one update_rope call
+    RopeDev *rope = nullptr;  // set for the duration of one update_rope call
     // scratch for attention
     float *ws = nullptr;
     size_t ws_bytes = 0;
@@ -907,7 +909,7 @@ void kvhip_cache_free(kvhip_cache *c) {
     for (const Slab &sl : c->slabs) ptrs.push_back({sl.base, sl.bytes});
     if (c->st.pt) ptrs.push_back({const_cast<PageEntry *>(c->st.pt), (size_t)0});
     if (c->ws) ptrs.push_back({c->ws, c->ws_bytes});
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kvhip_cache::PAD_BUFS; ++i)
         if (c->pad_buf[i]) ptrs.push_back({c->pad_buf[i], c->pad_bytes[i]});
     if (c->stage_tmp_k) ptrs.push_back({c->stage_tmp_k, (size_t)0});
     if (c->stage_tmp_v) ptrs.push_back({c->stage_tmp_v, (size_t)0});
@@ -1321,6 +1323,45 @@ kvhip_status kvhip_cache_update_attend(kvhip_cache *c, const void *q, const void
     }
     KV_TRY(kvhip_cache_update(c, k, v, B, Hkv, L, Dk, Dv, dtype, stream));
     return kvhip_cache_attend(c, q, B, Hq, L, Dk, scale, mask, out, stream);
+}
+
+kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *rope, const int32_t *batch_offsets,
+                                            const void *q, const void *k, const void *v, int32_t B, int32_t Hq,
+                                            int32_t Hkv, int32_t L, int32_t Dk, int32_t Dv, int32_t dtype, float scale,
+                                            const kvhip_mask *mask, void *q_rotated, void *out, void *stream) {
+    if (!c || !q || !k || !v || !out) return fail(KVHIP_ERR_INVALID_ARG, "null argument");
+    if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || Dk <= 0 || Dk > 1024) return fail(KVHIP_ERR_INVALID_ARG, "shape out of range");
+    if (dtype != KVHIP_F16 && dtype != KVHIP_BF16 && dtype != KVHIP_F32)
+        return fail(KVHIP_ERR_INVALID_ARG, "rope needs a floating-point dtype");
+    RopeDev r;
+    const int64_t offset = c->offset;
+    KV_TRY(rope_dev(rope, Dk, Hkv, dtype, offset + (c->staging ? (int64_t)c->staged.size() : 0), batch_offsets, r));
+    if (!q_rotated) {
+        KV_TRY(ensure_pad_buf(c, 4, (size_t)B * Hq * L * Dk * (dtype == KVHIP_F32 ? 4 : 2)));
+        q_rotated = c->pad_buf[4];
+    }
+    // The queries turn in the append's launch when their rows are whole 16-byte chunks (a launch of their own costs
+    // 3 to 5 us on the device and as much on the host).
+    const size_t q_rows = (size_t)B * L;  // (at most so many grid rows of query workgroups: rope_ride_rows)
+    if (r.vec && !c->staging && (size_t)B * Hkv + (q_rows >= 256 ? q_rows : q_rows * Hq) <= 65535) {
+        r.qx = static_cast<const char *>(q);
+        r.qo = static_cast<char *>(q_rotated);
+        r.qB = B;
+        r.qH = Hq;
+        r.qL = L;
+        r.qD = Dk;
+    }
+    const bool ride = r.qx != nullptr;
+    c->rope = &r;
+    const kvhip_status st = kvhip_cache_update(c, k, v, B, Hkv, L, Dk, Dv, dtype, stream);
+    c->rope = nullptr;
+    if (st != KVHIP_OK) return st;
+    if (!ride || r.qx != nullptr) {
+        RopeDev own;
+        KV_TRY(rope_dev(rope, Dk, Hq, dtype, offset, batch_offsets, own));
+        KV_HIP(launch_rope_apply(own, q, q_rotated, B, Hq, L, Dk, dtype, S(c, stream)));
+    }
+    return kvhip_cache_attend(c, q_rotated, B, Hq, L, Dk, scale, mask, out, stream);
 }
 
 kvhip_status kvhip_cache_mask_plan(const kvhip_cache *c, int32_t n, int32_t window, int32_t return_array,

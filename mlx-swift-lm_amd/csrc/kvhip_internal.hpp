@@ -221,15 +221,20 @@ struct RopeDev {
     const int32_t *batch_pos = nullptr;  // optional [B] (device)
     int32_t H = 1;             // heads per batch row of the array being rotated
     int32_t vec = 0;           // 1: rows are whole 16-byte chunks and no pair's half cuts through one (chunk kernels)
+    // Queries [qB, qH, qL, qD] of the same forward, turned at the same positions into `qo` by further workgroups of the
+    // append's launch (rope_queries_ride).  The launcher that takes them along clears `qx`.  Needs `vec`.
+    const char *qx = nullptr;
+    char *qo = nullptr;
+    int32_t qB = 0, qH = 0, qL = 0, qD = 0;
 };
 
 // ---- kernel launchers (defined in the .hip files) ---------------------------
 // New rows src[l] for l in [src0, src0+n) go to physical slots [slot0, slot0+n); with `rope`
 // the K rows are rotated (and rounded to the cache dtype) on the way in.
 hipError_t launch_append_fp(const Store &st, const void *keys, const void *values, int L, int src0,
-                            int slot0, int n, hipStream_t s, const RopeDev *rope = nullptr);
+                            int slot0, int n, hipStream_t s, RopeDev *rope = nullptr);
 hipError_t launch_append_quant(const Store &st, const void *keys, const void *values, int L, int src0,
-                               int slot0, int n, hipStream_t s, const RopeDev *rope = nullptr);
+                               int slot0, int n, hipStream_t s, RopeDev *rope = nullptr);
 // out = rope(x) for x [B, H, L, D] of `dtype` (out may alias x)
 hipError_t launch_rope_apply(const RopeDev &rope, const void *x, void *out, int B, int H, int L, int D,
                              int dtype, hipStream_t s);

@@ -7,13 +7,14 @@ namespace kvhip {
 
 namespace {
 
-// grid (L, B): the queries of one row position, every head of it (rope_rows_body).  512 rows of 32 heads x 128 in
+// grid (L, B, head groups): the queries of one row position (rope_rows_body).  512 rows of 32 heads x 128 in
 // bfloat16 (8.4 MB moved): 10.5 us with a workgroup per row and head and a sine, cosine and exponential per element,
 // 4.9 us so.
 template <int DT>
 __global__ void __launch_bounds__(256) rope_rows_kernel(RopeDev r, const char *x, char *out, int H, int L, int D) {
     __shared__ float inv_s[512];
-    rope_rows_body<DT>(r, x, out, H, L, D, blockIdx.y, blockIdx.x, 0, H, inv_s);
+    const int hg = rope_heads_per_group(gridDim.x * gridDim.y, H, D, DT == 2 ? 4 : 2), h0 = blockIdx.z * hg;
+    rope_rows_body<DT>(r, x, out, H, L, D, blockIdx.y, blockIdx.x, h0, min(H, h0 + hg), inv_s);
 }
 
 // grid (L, B*H): one row per workgroup; arrays whose pairs cut through 16-byte chunks
@@ -46,11 +47,19 @@ __device__ __forceinline__ void quantize_row_wave(const void *src, int D, int gs
         [&](int d, uint32_t code) { if (code_out) code_out[d] = (uint8_t)code; }, sb_row, scales, biases);
 }
 
-// grid (rows, BH): one new row per workgroup, scattered into the chunk-interleaved tile.
+// grid (rows, BH + query rows): one new row per workgroup, scattered into the chunk-interleaved tile; with queries of
+// the same forward behind them (RopeDev::qx; 256 threads then).
 template <int ES>
 __global__ void append_fp_kernel(Store st, const char *keys, const char *values, int L, int src0,
                                  int slot0, RopeDev rope) {
     const int bh = blockIdx.y;
+    if (bh >= st.BH) {
+        __shared__ float inv_s[512];
+        if (ES == 4) rope_queries_ride<2>(rope, st.BH, inv_s);
+        else if (st.dtype == KVHIP_F16) rope_queries_ride<0>(rope, st.BH, inv_s);
+        else rope_queries_ride<1>(rope, st.BH, inv_s);
+        return;
+    }
     const int i = blockIdx.x;
     const int slot = slot0 + i;
     const int l = src0 + i;
@@ -82,7 +91,7 @@ __global__ void append_fp_kernel(Store st, const char *keys, const char *values,
 template <int DT, int BITS, bool ROPE, bool PAGED>
 __device__ __forceinline__ void append_quant_body(const Store &st, const Store &src, const char *keys, const char *values,
                                                   int L, int src0, int slot0, int n, const RopeDev &rope) {
-    extern __shared__ uint8_t vcodes[];  // [64][Dv]
+    extern __shared__ __attribute__((aligned(16))) uint8_t vcodes[];  // [64][Dv]
     const int bh = blockIdx.y;
     const int tile = (slot0 >> 6) + blockIdx.x;
     const int lo = max(slot0, tile * TILE);
@@ -175,6 +184,13 @@ template <int DT, int BITS, bool ROPE>
 __global__ void __launch_bounds__(512)
 append_quant_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, int n,
                     RopeDev rope) {
+    if constexpr (ROPE) {
+        if ((int)blockIdx.y >= st.BH) {  // queries of the same forward (64 Dv bytes of LDS hold dims / 2 floats)
+            extern __shared__ __attribute__((aligned(16))) uint8_t vcodes[];
+            rope_queries_ride<DT>(rope, st.BH, reinterpret_cast<float *>(vcodes));
+            return;
+        }
+    }
     append_quant_body<DT, BITS, ROPE, false>(st, st, keys, values, L, src0, slot0, n, rope);
 }
 
@@ -410,6 +426,11 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
     __shared__ uint32_t vt[TILE * VPW];
     __shared__ float inv_s[DK / 2];
     const int bh = blockIdx.y;
+    if (bh >= st.BH) {  // queries of the same forward
+        if (st.dtype == KVHIP_F16) rope_queries_ride<0>(rope, st.BH, inv_s);
+        else rope_queries_ride<1>(rope, st.BH, inv_s);
+        return;
+    }
     const int slot_t = (slot0 & ~(TILE - 1)) + blockIdx.x * TILE;
     const int l_t = src0 + slot_t - slot0;  // the row in the tile's first slot (before the first new row: t_lo > 0)
     // tokens [t_lo, t_hi) of the tile are new; the threads of the others repeat the nearest new row and write nothing
@@ -732,10 +753,18 @@ __global__ void mask_materialize_kernel(kvhip_mask_plan_t p, uint8_t *dst) {
     } while (0)
 
 namespace {
+// The caller's rotation as this launch takes it: queries that ride along ride once.
+RopeDev take_rope(RopeDev *rope) {
+    if (!rope) return RopeDev();
+    const RopeDev r = *rope;
+    rope->qx = nullptr;
+    return r;
+}
+
 hipError_t launch_append_fp_rows(const Store &st, const void *keys, const void *values, int L, int src0,
                                  int slot0, int n, hipStream_t s, const RopeDev &r) {
     if (n <= 0) return hipSuccess;
-    dim3 grid(n, st.BH), block(128);
+    dim3 grid(n, st.BH + rope_ride_rows(r, n, st.es)), block(r.qx ? 256 : 128);
     if (st.es == 2)
         hipLaunchKernelGGL(append_fp_kernel<2>, grid, block, 0, s, st, (const char *)keys, (const char *)values, L, src0, slot0, r);
     else
@@ -745,15 +774,16 @@ hipError_t launch_append_fp_rows(const Store &st, const void *keys, const void *
 }  // namespace
 
 hipError_t launch_append_fp(const Store &st, const void *keys, const void *values, int L, int src0,
-                            int slot0, int n, hipStream_t s, const RopeDev *rope) {
+                            int slot0, int n, hipStream_t s, RopeDev *rope) {
     if (n <= 0) return hipSuccess;
-    const RopeDev r = rope ? *rope : RopeDev();
+    const RopeDev r = take_rope(rope);
     const bool mla = st.Dk == 192 && st.Dv == 128;  // keys of 192 with values of 128
     const bool tiled = st.es == 2 && ((st.Dk == st.Dv && (st.Dk == 64 || st.Dk == 96 || st.Dk == 128 || st.Dk == 256)) || mla);
     // One launch for whole tiles and the pieces of tiles at either end.  Fewer rows than a tile go one to a workgroup:
     // that takes 5 us whatever their number, less than a tile's workgroup behind its barriers.
     if (!tiled || n < TILE) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
-    dim3 grid(((slot0 & (TILE - 1)) + n + TILE - 1) / TILE, st.BH), block(256);
+    const int tiles = ((slot0 & (TILE - 1)) + n + TILE - 1) / TILE;
+    dim3 grid(tiles, st.BH + rope_ride_rows(r, tiles, st.es)), block(256);
 #define FP_TILE(NCK, NCV) hipLaunchKernelGGL((append_fp_tile_kernel<NCK, NCV>), grid, block, 0, s, st, (const char *)keys, (const char *)values, L, src0, slot0, n, r)
     if (mla) FP_TILE(6, 4);
     else if (st.Dk == 64) FP_TILE(2, 2);
@@ -768,7 +798,8 @@ hipError_t launch_rope_apply(const RopeDev &rope, const void *x, void *out, int 
                              int dtype, hipStream_t s) {
     if ((size_t)B * H * L == 0) return hipSuccess;
     if (rope.vec) {
-#define ROPE_ROWS(DT) hipLaunchKernelGGL(rope_rows_kernel<DT>, dim3(L, B), dim3(256), 0, s, rope, (const char *)x, (char *)out, H, L, D)
+        const int hg = rope_heads_per_group(L * B, H, D, dtype == KVHIP_F32 ? 4 : 2);
+#define ROPE_ROWS(DT) hipLaunchKernelGGL(rope_rows_kernel<DT>, dim3(L, B, (H + hg - 1) / hg), dim3(256), 0, s, rope, (const char *)x, (char *)out, H, L, D)
         if (dtype == KVHIP_F16) ROPE_ROWS(0);
         else if (dtype == KVHIP_BF16) ROPE_ROWS(1);
         else ROPE_ROWS(2);
@@ -788,7 +819,7 @@ hipError_t launch_append_quant_rows(const Store &st, const void *keys, const voi
     if (n <= 0) return hipSuccess;
     const int ntile = ((slot0 + n - 1) >> 6) - (slot0 >> 6) + 1;
     // (a speculative-verify step appends 4 rows: 8 (row, K or V) items, one per wavefront)
-    dim3 grid(ntile, st.BH), block(n >= 3 ? 512 : 256);
+    dim3 grid(ntile, st.BH + rope_ride_rows(r, ntile, st.es)), block(n >= 3 ? 512 : 256);
     const size_t lds = (size_t)TILE * st.Dv;
 #define CALL(DT, BITS)                                                                                      \
     do {                                                                                                    \
@@ -809,9 +840,9 @@ hipError_t launch_append_quant_rows(const Store &st, const void *keys, const voi
 constexpr int QUANT_TILE_ROWS = 9;
 
 hipError_t launch_append_quant(const Store &st, const void *keys, const void *values, int L, int src0,
-                               int slot0, int n, hipStream_t s, const RopeDev *rope) {
+                               int slot0, int n, hipStream_t s, RopeDev *rope) {
     if (n <= 0) return hipSuccess;
-    const RopeDev r = rope ? *rope : RopeDev();
+    const RopeDev r = take_rope(rope);
     const bool tiled = quant_tiles_one_launch(st) || quant_tiles_two_sided(st);
     // The row kernel's wavefronts take their rows one after the other (about 2.6 us a row and wavefront: 33 us for 50
     // rows of 128); one launch of the tile kernel takes every row of its tiles at once, 7 to 11 us whatever their number.

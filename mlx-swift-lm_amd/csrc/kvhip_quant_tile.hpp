@@ -337,6 +337,13 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
 template <int DT, int BITS, int NC, int GL, bool ROPE, int SIDE = 0>
 __global__ void __launch_bounds__(256)
 append_quant_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, int n, RopeDev rope) {
+    if constexpr (ROPE) {
+        if ((int)blockIdx.y >= st.BH) {  // queries of the same forward
+            __shared__ float q_inv_s[NC * 16];
+            rope_queries_ride<DT>(rope, st.BH, q_inv_s);
+            return;
+        }
+    }
     append_quant_tile_body<DT, BITS, NC, GL, ROPE, false, SIDE>(st, st, keys, values, L, src0, slot0, n, rope);
 }
 
@@ -367,6 +374,7 @@ void launch_quant_tile_instance(const Store &st, const Store &src, const void *k
     if constexpr (PAGED) {
         hipLaunchKernelGGL((requant_tile_kernel<DT, BITS, NC, GL, SIDE>), grid, block, 0, s, st, src);
     } else {
+        if (SIDE != 2) grid.y += rope_ride_rows(r, grid.x, st.es);
         if (r.dims > 0 && SIDE != 2)
             hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, true, SIDE>), grid, block, 0, s, st,
                                (const char *)keys, (const char *)values, L, a0, b0, n, r);

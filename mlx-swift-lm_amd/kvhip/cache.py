@@ -20,11 +20,12 @@ _TORCH = {L.F16: torch.float16, L.BF16: torch.bfloat16, L.F32: torch.float32, L.
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current device's current stream as an address (`torch.cuda.current_stream()` without its Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 class MaskMode:
@@ -63,6 +64,8 @@ class MaskMode:
         return MaskMode(L.MASK_WINDOW, offset=offset, window=window, lengths=lengths, left_pad=left_pad)
 
     def to_c(self, B, Hq, Lq):
+        if self.mode == L.MASK_NONE or self.mode == L.MASK_CAUSAL:
+            return _PLAIN[self.mode], None
         m = L.Mask()
         m.mode = self.mode
         keep = []
@@ -94,6 +97,12 @@ class MaskMode:
                     setattr(m, name, t.data_ptr())
                     keep.append(t)
         return m, keep
+
+
+# masks that are nothing but their mode, read by the library and never written
+_PLAIN = {L.MASK_NONE: L.Mask(mode=L.MASK_NONE), L.MASK_CAUSAL: L.Mask(mode=L.MASK_CAUSAL)}
+# rotated queries up to this size stay in a buffer of the cache's; larger ones are allocated for the call
+_Q_ROTATED_KEPT = 1 << 18
 
 
 class _Cache:
@@ -248,6 +257,24 @@ class _Cache:
                                                     _ptr(out), _stream()))
         self._note_shape(k, v)
         del keep
+        return out
+
+    def update_attend_rope(self, rope, queries, keys, values, scale, mask=None, batch_offsets=None):
+        """Queries and keys rotated at this cache's `ropeOffset` (or at `batch_offsets`), update, attention."""
+        q, k, v = queries.contiguous(), keys.contiguous(), values.contiguous()
+        assert k.is_cuda and v.is_cuda and k.dtype == v.dtype
+        B, Hq, Lq, D = q.shape
+        Dv = v.shape[3]
+        out = torch.empty((B, Hq, Lq, Dv), dtype=q.dtype, device=q.device)
+        q_rot = torch.empty_like(q) if q.numel() * q.element_size() > _Q_ROTATED_KEPT else None
+        m, keep = (mask or MaskMode.none()).to_c(B, Hq, Lq)
+        r, freqs = rope.to_c()
+        bo = None if batch_offsets is None else batch_offsets.to(device="cuda", dtype=torch.int32).contiguous()
+        L.check(self._lib.kvhip_cache_update_attend_rope(
+            self._h, C.byref(r), _ptr(bo) if bo is not None else None, _ptr(q), _ptr(k), _ptr(v), B, Hq, k.shape[1], Lq, D, Dv,
+            _DT[k.dtype], float(scale), C.byref(m), _ptr(q_rot) if q_rot is not None else None, _ptr(out), _stream()))
+        self._note_shape(k, v)
+        del keep, freqs
         return out
 
     def make_mask(self, n, window_size=None, return_array=False):

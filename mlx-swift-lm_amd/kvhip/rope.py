@@ -14,7 +14,7 @@ import ctypes as C
 import torch
 
 from . import _lib as L
-from .cache import MaskMode, _DT, _ptr, _stream
+from .cache import MaskMode, _Cache, _DT, _ptr, _stream
 
 
 class RoPE:
@@ -58,8 +58,13 @@ def apply_rotary_position(rope, x, offset=None):
 
 def attention_with_rope_and_cache_update(rope, queries, keys, values, cache, scale, mask=None, batch_offsets=None):
     """Rotate queries and keys at the cache's `ropeOffset`, write the cache, attend
-    (Llama.swift:58-70 + AttentionUtils.swift:37-95): one launch for the queries, one fused
-    rotate-and-append (or rotate-quantize-append) for the keys and values, one for attention."""
+    (Llama.swift:58-70 + AttentionUtils.swift:37-95): one launch rotates the queries and rotates and appends
+    (or rotates, quantizes and appends) the keys and values, then attention.  Queries that do not go with the
+    keys row by row are taken in separate calls."""
+    if (isinstance(cache, _Cache) and queries.dtype == keys.dtype and queries.dim() == 4 and keys.dim() == 4
+            and (cache._shape is None or cache._shape[4] == keys.dtype)
+            and queries.shape[0] == keys.shape[0] and queries.shape[2:] == keys.shape[2:]):
+        return cache.update_attend_rope(rope, queries, keys, values, scale, mask, batch_offsets)
     offset = batch_offsets if batch_offsets is not None else cache.rope_offset
     q = apply_rotary_position(rope, queries, offset)
     cache.update_rope(rope, keys, values, batch_offsets)
