@@ -1,5 +1,5 @@
 // Attention on the vector ALUs, for the full-precision caches the matrix-core kernels are not built for: float32
-// caches, and 16-bit caches of head sizes above 256 (Gemma 4's full-attention layers: 512).  The fused op
+// caches, and 16-bit caches of head sizes above 256 other than 512 (kvhip_attend_wide.hip).  The fused op
 // (AttentionUtils.swift:86-93) computes in float32, excluded keys contribute nothing, one rounding at the output.
 //
 // 2 * rows FMAs per cached element is below what the memory system delivers them at up to 8 query rows per kv head,
@@ -365,8 +365,7 @@ hipError_t launch_dt(const AttendArgs &a, const PlanValu &p, hipStream_t s) {
     profile_mark(s, false);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.nparts == 1) return e;
-    hipLaunchKernelGGL(merge_valu_kernel<DT>, dim3((a.Hq / a.Hkv) * a.L, a.st.BH), dim3(FT), 0, s, a, p.nparts);
-    return hipGetLastError();
+    return launch_merge_valu(a, p.nparts, s);
 }
 
 }  // namespace
@@ -386,12 +385,22 @@ bool attend_valu_dequant_first(const AttendArgs &a) {
     return attend_valu_supported(fp);
 }
 
+hipError_t launch_merge_valu(const AttendArgs &a, int nparts, hipStream_t s) {
+    const dim3 grid((a.Hq / a.Hkv) * a.L, a.st.BH), block(FT);
+    if (a.st.dtype == KVHIP_F16) hipLaunchKernelGGL(merge_valu_kernel<0>, grid, block, 0, s, a, nparts);
+    else if (a.st.dtype == KVHIP_BF16) hipLaunchKernelGGL(merge_valu_kernel<1>, grid, block, 0, s, a, nparts);
+    else hipLaunchKernelGGL(merge_valu_kernel<2>, grid, block, 0, s, a, nparts);
+    return hipGetLastError();
+}
+
 size_t attend_valu_workspace(const AttendArgs &a) {
+    if (attend_wide_supported(a)) return attend_wide_workspace(a);
     const PlanValu p = plan_valu(a);
     return p.nparts == 1 ? 0 : (size_t)a.st.BH * p.nparts * (a.Hq / a.Hkv) * a.L * (a.st.Dv + 2) * sizeof(float);
 }
 
 hipError_t launch_attend_valu(const AttendArgs &a, hipStream_t s) {
+    if (attend_wide_supported(a)) return launch_attend_wide(a, s);
     const PlanValu p = plan_valu(a);
     if (a.st.dtype == KVHIP_F16) return launch_dt<0>(a, p, s);
     if (a.st.dtype == KVHIP_BF16) return launch_dt<1>(a, p, s);

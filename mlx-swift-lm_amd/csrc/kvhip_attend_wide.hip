@@ -1,0 +1,340 @@
+// Attention over 16-bit full-precision caches of head size 512 (Gemma 4's full-attention layers) on the matrix cores.
+// The fused op (AttentionUtils.swift:86-93) computes in float32, excluded keys contribute nothing, one rounding at the
+// output.
+//
+// A row of 512 is too wide for one wavefront's registers to hold queries, keys and outputs, so the four wavefronts of
+// a workgroup divide the head dimension: wavefront w contracts elements 128 w .. 128 w + 127 of the scores and owns
+// those columns of the output, and every cached element is loaded once per workgroup, from the page straight into the
+// operand registers (the interleaved pages hold 8 elements of a token, or 8 tokens of a column, as one 16-byte chunk).
+// Per tile of 32 tokens and 16 QT query rows:
+//   S^T partials  K (32 tokens x 128) . Q^T on v_mfma_f32_16x16x32, into LDS, added up behind a barrier;
+//   softmax       QT = 2: wavefronts 0 and 1 for sixteen query rows each, probabilities handed round through LDS;
+//                 QT = 1: every wavefront for all sixteen rows (no second barrier);
+//   out^T         V^T (128 columns x 32 tokens) . P^T, the probabilities as the sum of two 16-bit operands, high part
+//                 and remainder: 22 bits of a float32 probability in float16 (scaled by 2^10, so that the remainder
+//                 stays above the subnormals), 16 in bfloat16, where the output keeps 8.
+// Two rows of query tiles at most: the accumulators of four leave one wavefront per SIMD and are copied between the two
+// register files every tile (512 rows x 2048 keys, 8 query and 2 kv heads, bfloat16: 69 us the call, against 57 us).
+// Decode is bound by HBM where the batch fills the chip (B8, 4096 keys, one token: 26.5 us, 5.1 TB/s)
+// and by launch, one pass of loads and the merge below that (one sequence of 2048 keys 12 us, 63 us
+// before); a prompt chunk by the latency of the two barriers per tile (512 x 2048, 44 us and 14 us for the merge; 263 us
+// before).
+// K rows are loaded in the token order that leaves lane group g of the scores with tokens 8 g .. 8 g + 7, which is the
+// order the probabilities are read in as an operand: they never cross lanes.
+#include <algorithm>
+
+#include "kvhip_mask.hpp"
+
+namespace kvhip {
+
+namespace {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+constexpr int WD = 512;        // head size
+constexpr int WW = 4;          // wavefronts
+constexpr int WT = 32;         // tokens per tile
+constexpr int NS = WD / WW / 32;  // contraction steps of a wavefront
+constexpr int NCT = WD / WW / 16; // 16-column output tiles of a wavefront
+constexpr float WLOG2E = 1.4426950408889634f;
+
+template <int DT> __device__ __forceinline__ f4 mfma(const kv_u4 &a, const kv_u4 &b, f4 c) {
+    if constexpr (DT == 0) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
+}
+template <int DT> __device__ __forceinline__ uint32_t pack2(float x, float y) { return DT == 0 ? pk_h2(x, y) : pk_bf2(x, y); }
+template <int DT> __device__ __forceinline__ float low_of(uint32_t w) {
+    return DT == 0 ? (float)__builtin_bit_cast(_Float16, (uint16_t)w) : __uint_as_float(w << 16);
+}
+template <int DT> __device__ __forceinline__ float high_of(uint32_t w) {
+    return DT == 0 ? (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)) : __uint_as_float(w & 0xffff0000u);
+}
+
+// grid (row blocks of 16 QT, BH, parts), four wavefronts.  Parts divide the key tiles the row block sees.
+template <int DT, int QT>
+__global__ void __launch_bounds__(256, 2)
+attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
+    constexpr int NB = QT == 1 ? 2 : 1;           // score buffers (QT = 1 has one barrier per tile)
+    __shared__ f4 part_s[NB][WW][QT][2][64];      // partial scores of the wavefronts
+    __shared__ kv_u4 prob_s[QT == 1 ? 1 : QT][2][64];
+    __shared__ float stat_s[QT][16], sum_s[QT][16], max_s[QT][16];
+    const Store &st = a.st;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, g = lane >> 4;
+    // (the row blocks of one kv head and part run on one XCD and share its L2: see attend_valu_kernel)
+    int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int total = gridDim.x * gridDim.y * gridDim.z;
+    if (gridDim.x > 1 && (total & 7) == 0) lin = (lin & 7) * (total >> 3) + (lin >> 3);
+    const int bh = (lin / gridDim.x) % gridDim.y, part = lin / (gridDim.x * gridDim.y);
+    const int b = bh / a.Hkv, h = bh % a.Hkv;
+    const int r = a.Hq / a.Hkv, R = r * a.L;
+    const int row0 = (lin % gridDim.x) * 16 * QT, row1 = min(row0 + 16 * QT, R) - 1;
+
+    // ---- the keys this row block sees (vis) and those all of its rows see (full) --------------------
+    const bool one_head = row0 / a.L == row1 / a.L;
+    const int l0 = one_head ? row0 % a.L : 0, l1 = one_head ? row1 % a.L : a.L - 1;
+    int vis_lo = 0, vis_hi = a.T - 1, full_lo = 0, full_hi = a.T - 1;
+    if (a.mask.mode == KVHIP_MASK_CAUSAL) {
+        vis_hi = min(vis_hi, a.T - a.L + l1);
+        full_hi = min(full_hi, a.T - a.L + l0);
+    } else if (a.mask.mode == KVHIP_MASK_WINDOW) {
+        const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
+        vis_lo = max(0, sym.pad_b);
+        full_lo = vis_lo;
+        if (sym.window > 0) {
+            vis_lo = max(vis_lo, sym.offset + l0 - sym.window + 1);
+            full_lo = max(full_lo, sym.offset + l1 - sym.window + 1);
+        }
+        vis_hi = min(vis_hi, min(sym.offset + l1, sym.len_b - 1));
+        full_hi = min(full_hi, min(sym.offset + l0, sym.len_b - 1));
+    } else if (a.mask.mode == KVHIP_MASK_ARRAY) {
+        full_hi = -1;
+    }
+    const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
+    int t_lo = 0, t_hi = tiles_total;
+    if (ident) {
+        t_lo = min(vis_lo / WT, tiles_total);
+        t_hi = vis_hi < vis_lo ? t_lo : min(tiles_total, vis_hi / WT + 1);
+    }
+    const int per = (max(t_hi - t_lo, 1) + nparts - 1) / nparts;
+    const int tb = min(t_lo + part * per, t_hi), te = min(tb + per, t_hi);
+
+    // ---- query operands: lane (col, g) holds elements 8 g .. 8 g + 7 of step s of row 16 qt + col ----
+    kv_u4 qop[QT][NS];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        const int rr = min(row0 + 16 * qt + col, R - 1);  // rows beyond the last: the last again, which nobody keeps
+        gptr qp = as_global(a.q) + (((size_t)(b * a.Hq + h * r + rr / a.L) * a.L + rr % a.L) * WD + wave * (WD / WW) + 8 * g) * 2;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) qop[qt][s] = ld_global<kv_u4>(qp + s * 64);
+    }
+
+    kv_u4 kreg[NS][2], vreg[NCT];
+    const uint32_t k_lane = ((uint32_t)(16 * wave + g) * TILE + 8 * (col >> 2) + (col & 3)) * 16;
+    const uint32_t v_lane = ((uint32_t)g * WD + wave * (WD / WW) + col) * 16;
+    PageCursor kpage(st, tb < te ? tb * WT : 0), vpage = kpage;
+    auto load_k = [&](int t) __attribute__((always_inline)) {
+        const int slot0 = t * WT;
+        gptr p = as_global(kpage.at(st, slot0).k) + (size_t)bh * st.k_cell + (size_t)((slot0 & (PAGE - 1)) >> 6) * ((size_t)TILE * st.k_row) +
+                 (slot0 & 32) * 16 + k_lane;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) kreg[s][x] = ld_global<kv_u4>(p + s * (4 * TILE * 16) + x * 64);
+    };
+    auto load_v = [&](int t) __attribute__((always_inline)) {
+        const int slot0 = t * WT;
+        gptr p = as_global(vpage.at(st, slot0).v) + (size_t)bh * st.v_cell + (size_t)((slot0 & (PAGE - 1)) >> 6) * ((size_t)TILE * WD * 2) +
+                 (size_t)((slot0 & 32) >> 3) * (WD * 16) + v_lane;
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) vreg[c] = ld_global<kv_u4>(p + c * 256);
+    };
+
+    f4 acc[QT][NCT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) acc[qt][c] = f4{0.f, 0.f, 0.f, 0.f};
+    const int own = QT == 1 ? 0 : wave & 1;  // the query rows whose softmax this wavefront works out
+    const int my = row0 + 16 * own + col;
+    const int my_hq = h * r + min(my, R - 1) / a.L, my_l = min(my, R - 1) % a.L;
+    float m_run = -INFINITY, l_run = 0.f;
+    constexpr float P_UP = DT == 0 ? 10.f : 0.f;  // (float16 probabilities are carried times 2^10)
+
+    // the probabilities of row `my` for tokens 8 g .. 8 g + 7 of tile t, high parts and remainders, and the factor its
+    // sums so far take
+    auto softmax = [&](int t, int buf, kv_u4 &ph, kv_u4 &pl, float &alpha) __attribute__((always_inline)) {
+        f4 sum[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            sum[x] = part_s[buf][0][own][x][lane];
+#pragma unroll
+            for (int w = 1; w < WW; ++w) sum[x] += part_s[buf][w][own][x][lane];
+        }
+        float sc[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sc[j] = sum[j >> 2][j & 3] * a.scale;
+        const int slot0 = t * WT;
+        if (!ident || slot0 < full_lo || slot0 + WT - 1 > full_hi) {  // workgroup-uniform
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int slot = slot0 + 8 * g + j;
+                const int row = ident ? slot : slot < a.slots ? slot_to_row(a.runs, slot) : -1;
+                float add = 0.f;
+                const bool keep = row >= 0 && row < a.T && mask_keep(a.mask, b, my_hq, my_l, row, a.L, a.T, add);
+                sc[j] = keep ? sc[j] + add : -INFINITY;
+            }
+        }
+        float mx = sc[0];
+#pragma unroll
+        for (int j = 1; j < 8; ++j) mx = fmaxf(mx, sc[j]);
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        // The reference of the exponentials is raised only when a score exceeds it by more than 2^5, so that the
+        // accumulators are rarely touched after the first tiles (probabilities stay below 2^5, 2^15 in float16).
+        const float m_new = (mx - m_run) * WLOG2E > 5.f || m_run == -INFINITY ? fmaxf(m_run, mx) : m_run;
+        const float m_use = m_new > -INFINITY ? m_new : 0.f;
+        alpha = m_new > m_run ? __builtin_amdgcn_exp2f((m_run - m_new) * WLOG2E) : 1.f;
+        float p[8], ps = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j] - m_use, WLOG2E, P_UP));
+            ps += p[j];
+        }
+        l_run = l_run * alpha + ps;
+        m_run = m_new;
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            hi[j] = pack2<DT>(p[2 * j], p[2 * j + 1]);
+            lo[j] = pack2<DT>(p[2 * j] - low_of<DT>(hi[j]), p[2 * j + 1] - high_of<DT>(hi[j]));
+        }
+        ph = kv_u4{hi[0], hi[1], hi[2], hi[3]};
+        pl = kv_u4{lo[0], lo[1], lo[2], lo[3]};
+    };
+
+    if (tb < te) {  // workgroup-uniform
+        load_k(tb);
+        load_v(tb);
+    }
+    for (int t = tb; t < te; ++t) {
+        f4 sacc[QT][2];
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) sacc[qt][0] = sacc[qt][1] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) sacc[qt][x] = mfma<DT>(kreg[s][x], qop[qt][s], sacc[qt][x]);
+        load_k(min(t + 1, te - 1));
+        const int buf = NB == 1 ? 0 : (t & 1);
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) part_s[buf][wave][qt][x][lane] = sacc[qt][x];
+        __syncthreads();
+        kv_u4 ph, pl;
+        float alpha = 1.f;
+        if (QT == 1 || wave < QT) softmax(t, buf, ph, pl, alpha);  // wave-uniform
+        if constexpr (QT > 1) {
+            if (wave < QT) {
+                prob_s[own][0][lane] = ph;
+                prob_s[own][1][lane] = pl;
+                if (g == 0) stat_s[own][col] = alpha;
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            const float al = QT == 1 ? alpha : stat_s[qt][col];
+            if (__any(al != 1.f)) {  // (a raised maximum: rare after the first tiles)
+#pragma unroll
+                for (int c = 0; c < NCT; ++c) acc[qt][c] *= al;
+            }
+            if constexpr (QT > 1) {
+                ph = prob_s[qt][0][lane];
+                pl = prob_s[qt][1][lane];
+            }
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(vreg[c], ph, acc[qt][c]);
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(vreg[c], pl, acc[qt][c]);
+        }
+        load_v(min(t + 1, te - 1));
+    }
+
+    // ---- the rows' maxima and sums to every wavefront, then the output ------------------------------
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+    if (g == 0 && wave < QT) {
+        max_s[own][col] = m_run;
+        sum_s[own][col] = l_run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        const int rr = row0 + 16 * qt + col;
+        if (rr >= R) continue;
+        const float l = sum_s[qt][col];
+        if (nparts == 1) {
+            const float inv = l > 0.f ? 1.f / l : 0.f;
+            uint16_t *dst = reinterpret_cast<uint16_t *>(a.out) + ((size_t)(b * a.Hq + h * r + rr / a.L) * a.L + rr % a.L) * WD + wave * (WD / WW) + 4 * g;
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) {
+                const f4 v = acc[qt][c] * inv;
+                *reinterpret_cast<kv_u2 *>(dst + 16 * c) = kv_u2{pack2<DT>(v.x, v.y), pack2<DT>(v.z, v.w)};
+            }
+        } else {
+            float *dst = a.workspace + ((size_t)(bh * nparts + part) * R + rr) * (WD + 2);
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) {
+                float *d = dst + wave * (WD / WW) + 16 * c + 4 * g;  // (rows of 514 floats: 8-byte aligned)
+                *reinterpret_cast<kv_f2 *>(d) = kv_f2{acc[qt][c].x, acc[qt][c].y};
+                *reinterpret_cast<kv_f2 *>(d + 2) = kv_f2{acc[qt][c].z, acc[qt][c].w};
+            }
+            if (wave == 0 && g == 0) {
+                dst[WD] = max_s[qt][col];
+                dst[WD + 1] = l;
+            }
+        }
+    }
+}
+
+struct PlanWide {
+    int qt, row_blocks, tiles, nparts;
+};
+
+PlanWide plan_wide(const AttendArgs &a) {
+    PlanWide p;
+    const int R = (a.Hq / a.Hkv) * a.L;
+    p.qt = R <= 16 ? 1 : 2;
+    p.row_blocks = (R + 16 * p.qt - 1) / (16 * p.qt);
+    p.tiles = (a.slots + WT - 1) / WT;
+    // One token: a workgroup per CU (two: B8 over 4096 keys 29.4 us against 26.8), parts of at least two tiles (one: 14.1 us
+    // against 12.1 for a sequence of 2048 keys, whose merge then reads twice the partials).  Chunks: two per CU (one: 76 us
+    // against 57 for 512 x 2048; three, which need a second round: 72 us).
+    static const int target = measure_knob("KVHIP_WIDE_TARGET", 256), target2 = measure_knob("KVHIP_WIDE_TARGET2", 512), least = measure_knob("KVHIP_WIDE_LEAST", 2);  // (timing builds only)
+    const long wgs = (long)p.row_blocks * a.st.BH;
+    int n = (int)std::max(1L, std::min<long>((p.qt == 1 ? target : target2) / std::max(1L, wgs), p.tiles / (p.qt == 1 ? least : 4)));
+    n = std::min(n, 64);
+    const size_t per_part = (size_t)a.st.BH * R * (a.st.Dv + 2) * sizeof(float);
+    while (n > 1 && a.workspace_cap && per_part * n > a.workspace_cap) --n;
+    p.nparts = n;
+    return p;
+}
+
+}  // namespace
+
+bool attend_wide_supported(const AttendArgs &a) {
+    const Store &s = a.st;
+    return s.bits == 0 && s.es == 2 && s.Dk == WD && s.Dv == WD && s.BH <= 65535;
+}
+
+size_t attend_wide_workspace(const AttendArgs &a) {
+    const PlanWide p = plan_wide(a);
+    return p.nparts == 1 ? 0 : (size_t)a.st.BH * p.nparts * (a.Hq / a.Hkv) * a.L * (a.st.Dv + 2) * sizeof(float);
+}
+
+hipError_t launch_attend_wide(const AttendArgs &a, hipStream_t s) {
+    const PlanWide p = plan_wide(a);
+    const dim3 grid(p.row_blocks, a.st.BH, p.nparts), block(256);
+    profile_mark(s, true);
+#define WIDE(DT, QT) hipLaunchKernelGGL((attend_wide_kernel<DT, QT>), grid, block, 0, s, a, p.tiles, p.nparts)
+    if (a.st.dtype == KVHIP_F16) {
+        if (p.qt == 1) WIDE(0, 1);
+        else WIDE(0, 2);
+    } else {
+        if (p.qt == 1) WIDE(1, 1);
+        else WIDE(1, 2);
+    }
+#undef WIDE
+    profile_mark(s, false);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || p.nparts == 1) return e;
+    return launch_merge_valu(a, p.nparts, s);
+}
+
+}  // namespace kvhip

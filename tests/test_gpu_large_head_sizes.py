@@ -1,5 +1,6 @@
 """16-bit caches of head sizes above 256 (Gemma 4's full-attention layers use 512: Gemma4Text.swift:53, :243-245), which
-the matrix-core kernels are not built for: the vector-ALU kernel (family 5) against the oracle, through the
+the matrix-core tiles of smaller head sizes are not built for: the kernels of family 5 (the vector ALUs; the matrix
+cores at head size 512) against the oracle, through the
 allocation-free entry point, and against the plain kernel over drawn shapes and masks."""
 import numpy as np
 import pytest
@@ -186,3 +187,31 @@ def test_quantized_cache_is_dequantized_for_the_vector_alu_kernel(dtype, bits, g
         check_attention(out, ref, dtype, f"L={Lq} {mode}", exact)
     for i, (a, b) in enumerate(zip(c.state, o.get_state())):
         assert np.array_equal(np32(a), b) if i % 3 == 0 else np.array_equal(np32(a), b.astype(np.float32)), i
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,n,mode", [(1, 1, "none"), (31, 1, "none"), (32, 4, "causal"), (33, 5, "causal"), (64, 16, "window"), (65, 8, "causal"),
+                                      (257, 9, "window"), (700, 33, "causal"), (1025, 130, "window"), (511, 511, "causal"), (9000, 2, "window")])
+def test_head_size_512_at_the_edges_of_its_tiles(dtype, T, n, mode):
+    """Keys around multiples of the 32-token tile, rows per kv head around 16 and 32, masks that leave tiles out.  Against
+    float64: half an ulp of the output, plus 2^-14 of the weighted values (a bfloat16 probability is kept to 2^-17)."""
+    B, Hkv, r, D = 2, 2, 4, 512
+    gen = torch.Generator(device="cuda").manual_seed(T + n)
+    q, k, v = (torch.randn(B, h, m, D, generator=gen, device="cuda").to(dtype) for h, m in ((Hkv * r, n), (Hkv, T), (Hkv, T)))
+    c = kvhip.KVCacheSimple()
+    c.update(k, v, fetch=False)
+    i, j = torch.arange(n, device="cuda")[:, None] + T - n, torch.arange(T, device="cuda")[None]
+    hidden = (j > i).expand(B, 1, n, T)
+    mask = {"none": kvhip.MaskMode.none(), "causal": kvhip.MaskMode.causal()}.get(mode)
+    if mode == "window":
+        pad = torch.tensor([0, T // 3], dtype=torch.int32, device="cuda")
+        mask = kvhip.MaskMode.window_mask(T - n, T // 2, left_pad=pad)
+        hidden = hidden | (i >= j + T // 2) | (j[None, None] < pad[:, None, None, None])
+    out = c.attend(q, D ** -0.5, mask).double()
+    kk, vv = (x.double().repeat_interleave(r, 1).contiguous() for x in (k, v))
+    s = torch.matmul(q.double(), kk.transpose(-1, -2).contiguous()) * D ** -0.5
+    p = torch.nan_to_num(torch.softmax(s.masked_fill(hidden, float("-inf")), -1))  # (a row without keys gives zeros)
+    want, weighted = torch.matmul(p, vv), torch.matmul(p, vv.abs())
+    half_ulp = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8  # of the value at most: 11 and 8 significant bits
+    assert family() == 5
+    assert bool(((out - want).abs() <= half_ulp * want.abs() + 2.0 ** -14 * weighted + 1e-7).all())
