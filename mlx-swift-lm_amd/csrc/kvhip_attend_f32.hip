@@ -1,0 +1,320 @@
+// Attention over float32 caches on the float32 matrix instruction (v_mfma_f32_16x16x4_f32: products and sums in
+// float32, twice the rate of the vector ALUs).  The fused op (AttentionUtils.swift:86-93): excluded keys contribute
+// nothing, no rounding but float32's.
+//
+// A workgroup takes 16 QT query rows of one kv head and one range of keys; its four wavefronts walk alternate tiles of
+// 16 TB tokens with their own maxima, sums and accumulators and meet once, through LDS, at the end.  Nothing crosses
+// lanes in the loop but the row maxima, because the interleaved pages hold what each operand wants:
+//   S^T = K Q^T    lane (i, g) loads 16 bytes, elements 16 s + 4 g .. + 3 of token i: its operand of four instructions
+//                  (instruction j contracts elements 16 s + 4 g + j, g = 0..3), the queries likewise from their rows;
+//   out^T = V^T P^T  lane (i, g) loads tokens 4 g .. 4 g + 3 of column i, and the scores leave the first product with
+//                  tokens 4 g .. 4 g + 3 of query i in lane (i, g): the probabilities are the operand as they are.
+// Measured against the vector-ALU kernel, whole calls: 512 x 4096, B4, 32q/8kv 1626 -> 654 us (D 64), 2644 -> 1215
+// (D 128: 106 TFLOP/s of the 157 that the instruction has), 6755 -> 2524 (D 256); one token of one sequence, 16q/4kv, 1500
+// keys 17.3 -> 12.4 us (D 64: one pass of loads and the merge); 8192 keys of B8, 8 kv heads, HBM: 102 -> 101 us (D 128).
+#include <algorithm>
+
+#include "kvhip_mask.hpp"
+
+namespace kvhip {
+
+namespace {
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+constexpr int MW = 4;  // wavefronts
+
+__device__ __forceinline__ f4 mfma4(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// token blocks of 16 per tile: as many as the registers of two wavefronts per SIMD hold
+constexpr int token_blocks(int dk, int qt) { return dk <= 64 ? 4 / qt : dk <= 128 ? 2 / qt : 1; }
+constexpr int query_tiles(int dk) { return dk <= 128 ? 2 : 1; }
+
+// grid (row blocks of 16 QT, BH, parts).  Parts divide the key tiles the row block sees.
+template <int DK, int DV, int QT>
+__global__ void __launch_bounds__(256, 2)
+attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
+    constexpr int TB = token_blocks(DK, QT), WT = 16 * TB;
+    constexpr int NS = DK / 16, NCT = DV / 16;
+    extern __shared__ __align__(16) float smem[];
+    f4 *acc_s = reinterpret_cast<f4 *>(smem);         // [MW][QT][NCT][64]
+    constexpr bool QL = DK > 128;                     // query operands in LDS: no registers are left for them
+    __shared__ f4 q_s[QL ? QT * NS * 64 : 1];
+    __shared__ float max_s[MW][QT][16], sum_s[MW][QT][16];
+    const Store &st = a.st;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, g = lane >> 4;
+    // (the row blocks of one kv head and part run on one XCD and share its L2: see attend_valu_kernel)
+    int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int total = gridDim.x * gridDim.y * gridDim.z;
+    if (gridDim.x > 1 && (total & 7) == 0) lin = (lin & 7) * (total >> 3) + (lin >> 3);
+    const int bh = (lin / gridDim.x) % gridDim.y, part = lin / (gridDim.x * gridDim.y);
+    const int b = bh / a.Hkv, h = bh % a.Hkv;
+    const int r = a.Hq / a.Hkv, R = r * a.L;
+    const int row0 = (lin % gridDim.x) * 16 * QT, row1 = min(row0 + 16 * QT, R) - 1;
+
+    const bool one_head = row0 / a.L == row1 / a.L;
+    const KeyRange keys = visible_keys(a.mask, b, a.L, a.T, one_head ? row0 % a.L : 0, one_head ? row1 % a.L : a.L - 1);
+    const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
+    int t_lo = 0, t_hi = tiles_total;
+    if (ident) {
+        t_lo = min(keys.lo / WT, tiles_total);
+        t_hi = keys.hi < keys.lo ? t_lo : min(tiles_total, keys.hi / WT + 1);
+    }
+    const int per = (max(t_hi - t_lo, 1) + nparts - 1) / nparts;
+    const int tb = min(t_lo + part * per, t_hi), te = min(tb + per, t_hi);
+
+    // rows beyond the last: the last again, which nobody keeps
+    f4 qop[QT][QL ? 1 : NS];
+    int my_hq[QT], my_l[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        const int rr = min(row0 + 16 * qt + col, R - 1);
+        my_hq[qt] = h * r + rr / a.L;
+        my_l[qt] = rr % a.L;
+        gptr qp = as_global(a.q) + (((size_t)(b * a.Hq + my_hq[qt]) * a.L + my_l[qt]) * DK + 4 * g) * 4;
+#pragma unroll
+        for (int s = 0; s < (QL ? 0 : NS); ++s) qop[qt][s] = ld_global<f4>(qp + s * 64);
+        if constexpr (QL) {
+            for (int s = wave; s < NS; s += MW) q_s[(qt * NS + s) * 64 + lane] = ld_global<f4>(qp + s * 64);
+        }
+    }
+    if constexpr (QL) __syncthreads();
+
+    f4 kreg[TB][NS], vreg[TB][NCT];
+    const uint32_t k_lane = ((uint32_t)g * TILE + col) * 16, v_lane = ((uint32_t)g * DV + col) * 16;
+    const int first = tb + wave;
+    PageCursor kpage(st, first < te ? first * WT : 0), vpage = kpage;
+    auto load_k = [&](int t) __attribute__((always_inline)) {
+        const int slot0 = t * WT;
+        gptr p = as_global(kpage.at(st, slot0).k) + (size_t)bh * st.k_cell + (size_t)((slot0 & (PAGE - 1)) >> 6) * (TILE * DK * 4) +
+                 (slot0 & 63) * 16 + k_lane;
+#pragma unroll
+        for (int x = 0; x < TB; ++x)
+#pragma unroll
+            for (int s = 0; s < NS; ++s) kreg[x][s] = ld_global<f4>(p + s * (4 * TILE * 16) + x * 256);
+    };
+    auto load_v = [&](int t) __attribute__((always_inline)) {
+        const int slot0 = t * WT;
+        gptr p = as_global(vpage.at(st, slot0).v) + (size_t)bh * st.v_cell + (size_t)((slot0 & (PAGE - 1)) >> 2) * (DV * 16) + v_lane;
+#pragma unroll
+        for (int x = 0; x < TB; ++x)
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) vreg[x][c] = ld_global<f4>(p + x * (4 * DV * 16) + c * 256);
+    };
+
+    f4 acc[QT][NCT];
+    float m_run[QT], l_run[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        m_run[qt] = -INFINITY;
+        l_run[qt] = 0.f;
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) acc[qt][c] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (first < te) {  // wave-uniform
+        load_k(first);
+        load_v(first);
+    }
+    for (int t = first; t < te; t += MW) {
+        const int next = t + MW < te ? t + MW : t;
+        f4 s[QT][TB];
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+            for (int x = 0; x < TB; ++x) s[qt][x] = f4{0.f, 0.f, 0.f, 0.f};
+        f4 q[QT], qn[QT];
+#pragma unroll
+        for (int qt = 0; qt < (QL ? QT : 0); ++qt) qn[qt] = q_s[qt * NS * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < NS; ++e) {
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) {
+                if constexpr (QL) {
+                    q[qt] = qn[qt];
+                    qn[qt] = q_s[(qt * NS + min(e + 1, NS - 1)) * 64 + lane];
+                } else {
+                    q[qt] = qop[qt][e];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int x = 0; x < TB; ++x)
+#pragma unroll
+                    for (int qt = 0; qt < QT; ++qt) s[qt][x] = mfma4(kreg[x][e][j], q[qt][j], s[qt][x]);
+            if constexpr (QL) __builtin_amdgcn_sched_barrier(0);  // (one step's queries ahead, not all of them: registers)
+        }
+        load_k(next);
+        const int slot0 = t * WT;
+        const bool full = ident && slot0 >= keys.full_lo && slot0 + WT - 1 <= keys.full_hi;  // wave-uniform
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+            for (int x = 0; x < TB; ++x) s[qt][x] *= a.scale;
+            if (!full) {
+#pragma unroll
+                for (int x = 0; x < TB; ++x)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int slot = slot0 + 16 * x + 4 * g + j;
+                        const int row = ident ? slot : slot < a.slots ? slot_to_row(a.runs, slot) : -1;
+                        float add = 0.f;
+                        const bool keep = row >= 0 && row < a.T && mask_keep(a.mask, b, my_hq[qt], my_l[qt], row, a.L, a.T, add);
+                        s[qt][x][j] = keep ? s[qt][x][j] + add : -INFINITY;
+                    }
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int x = 0; x < TB; ++x)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[qt][x][j]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            // (the reference is raised only by more than 3, so that the accumulators are rarely touched after the first tiles)
+            const bool raise = mx - m_run[qt] > 3.f || (m_run[qt] == -INFINITY && mx > -INFINITY);
+            if (__any(raise)) {
+                const float m_new = raise ? mx : m_run[qt];
+                const float alpha = raise ? expf(m_run[qt] - m_new) : 1.f;
+                l_run[qt] *= alpha;
+#pragma unroll
+                for (int c = 0; c < NCT; ++c) acc[qt][c] *= alpha;
+                m_run[qt] = m_new;
+            }
+            const float m_use = m_run[qt] > -INFINITY ? m_run[qt] : 0.f;
+#pragma unroll
+            for (int x = 0; x < TB; ++x)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float p = expf(s[qt][x][j] - m_use);
+                    s[qt][x][j] = p;
+                    l_run[qt] += p;
+                }
+        }
+#pragma unroll
+        for (int x = 0; x < TB; ++x)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                    for (int qt = 0; qt < QT; ++qt) acc[qt][c] = mfma4(vreg[x][c][j], s[qt][x][j], acc[qt][c]);
+        load_v(next);
+    }
+
+    // ---- the four wavefronts' states: each scales its own to the common maximum, then adds up a quarter of the columns ----
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        l_run[qt] += __shfl_xor(l_run[qt], 16);
+        l_run[qt] += __shfl_xor(l_run[qt], 32);
+        if (g == 0) {
+            max_s[wave][qt][col] = m_run[qt];
+            sum_s[wave][qt][col] = l_run[qt];
+        }
+    }
+    __syncthreads();
+    float M[QT], L[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        M[qt] = max_s[0][qt][col];
+#pragma unroll
+        for (int w = 1; w < MW; ++w) M[qt] = fmaxf(M[qt], max_s[w][qt][col]);
+        L[qt] = 0.f;
+#pragma unroll
+        for (int w = 0; w < MW; ++w) {
+            const float mw = max_s[w][qt][col];
+            if (mw > -INFINITY) L[qt] += sum_s[w][qt][col] * expf(mw - M[qt]);
+        }
+        const float f = m_run[qt] > -INFINITY ? expf(m_run[qt] - M[qt]) : 0.f;
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) acc_s[((wave * QT + qt) * NCT + c) * 64 + lane] = acc[qt][c] * f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        const int rr = row0 + 16 * qt + col;
+        if (rr >= R) continue;
+        float *dst = nparts == 1 ? reinterpret_cast<float *>(a.out) + ((size_t)(b * a.Hq + my_hq[qt]) * a.L + my_l[qt]) * DV
+                                 : a.workspace + ((size_t)(bh * nparts + part) * R + rr) * (DV + 2);
+        for (int c = wave; c < NCT; c += MW) {
+            f4 v = acc_s[(qt * NCT + c) * 64 + lane];
+#pragma unroll
+            for (int w = 1; w < MW; ++w) v += acc_s[((w * QT + qt) * NCT + c) * 64 + lane];
+            if (nparts == 1) v = L[qt] > 0.f ? v / L[qt] : f4{0.f, 0.f, 0.f, 0.f};
+            float *d = dst + 16 * c + 4 * g;  // (partials: rows of DV + 2 floats, 8-byte aligned)
+            *reinterpret_cast<kv_f2 *>(d) = kv_f2{v.x, v.y};
+            *reinterpret_cast<kv_f2 *>(d + 2) = kv_f2{v.z, v.w};
+        }
+        if (nparts > 1 && wave == 0 && g == 0) {
+            dst[DV] = M[qt];
+            dst[DV + 1] = L[qt];
+        }
+    }
+}
+
+struct PlanF32 {
+    int qt, row_blocks, tiles, nparts;
+};
+
+PlanF32 plan_f32(const AttendArgs &a) {
+    PlanF32 p;
+    const int R = (a.Hq / a.Hkv) * a.L;
+    p.qt = R <= 16 ? 1 : query_tiles(a.st.Dk);
+    const int wt = 16 * token_blocks(a.st.Dk, p.qt);
+    p.row_blocks = (R + 16 * p.qt - 1) / (16 * p.qt);
+    p.tiles = (a.slots + wt - 1) / wt;
+    static const int target = measure_knob("KVHIP_F32_TARGET", 512), least = measure_knob("KVHIP_F32_LEAST", 2);  // (timing builds only)
+    const long wgs = (long)p.row_blocks * a.st.BH;
+    int n = (int)std::max(1L, std::min<long>(target / std::max(1L, wgs), p.tiles / least));
+    n = std::min(n, 32);  // (a merge of 64 parts takes as long as the halves save: 8192 keys, 8 kv heads of 128: 27.6 against 20.7 us)
+    const size_t per_part = (size_t)a.st.BH * R * (a.st.Dv + 2) * sizeof(float);
+    while (n > 1 && a.workspace_cap && per_part * n > a.workspace_cap) --n;
+    p.nparts = n;
+    return p;
+}
+
+template <int DK, int DV, int QT>
+hipError_t launch_instance(const AttendArgs &a, const PlanF32 &p, hipStream_t s) {
+    hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT>), dim3(p.row_blocks, a.st.BH, p.nparts), dim3(256), MW * QT * (DV / 16) * 64 * sizeof(f4), s,
+                       a, p.tiles, p.nparts);
+    return hipGetLastError();
+}
+
+template <int DK, int DV>
+hipError_t launch_sizes(const AttendArgs &a, const PlanF32 &p, hipStream_t s) {
+    if (p.qt == 1) return launch_instance<DK, DV, 1>(a, p, s);
+    return launch_instance<DK, DV, query_tiles(DK)>(a, p, s);
+}
+
+}  // namespace
+
+bool attend_f32_supported(const AttendArgs &a) {
+    const Store &s = a.st;
+    if (s.bits != 0 || s.dtype != KVHIP_F32 || s.BH > 65535) return false;
+    // Few query rows over many pairs of head size 256 and enough keys are bound by HBM, where the vector-ALU kernel's 1 KB
+    // loads are the better ones (B8, 8 kv heads, 8192 keys, one token: 185 us against 201; B4, 4 kv heads, 4096 keys: 36.2
+    // against 37.0; but one sequence, 8 kv heads, 8192 keys: 40.6 against 31).
+    if (s.Dk == 256 && s.BH >= 16 && (size_t)s.BH * a.T >= 65536 && (a.Hq / a.Hkv) * a.L <= 8) return false;
+    return (s.Dk == 192 && s.Dv == 128) || (s.Dk == s.Dv && (s.Dk == 64 || s.Dk == 96 || s.Dk == 128 || s.Dk == 256));
+}
+
+size_t attend_f32_workspace(const AttendArgs &a) {
+    const PlanF32 p = plan_f32(a);
+    return p.nparts == 1 ? 0 : (size_t)a.st.BH * p.nparts * (a.Hq / a.Hkv) * a.L * (a.st.Dv + 2) * sizeof(float);
+}
+
+hipError_t launch_attend_f32(const AttendArgs &a, hipStream_t s) {
+    const PlanF32 p = plan_f32(a);
+    profile_mark(s, true);
+    hipError_t e;
+    if (a.st.Dk == 192) e = launch_sizes<192, 128>(a, p, s);
+    else if (a.st.Dk == 64) e = launch_sizes<64, 64>(a, p, s);
+    else if (a.st.Dk == 96) e = launch_sizes<96, 96>(a, p, s);
+    else if (a.st.Dk == 128) e = launch_sizes<128, 128>(a, p, s);
+    else e = launch_sizes<256, 256>(a, p, s);
+    profile_mark(s, false);
+    if (e != hipSuccess || p.nparts == 1) return e;
+    return launch_merge_valu(a, p.nparts, s);
+}
+
+}  // namespace kvhip

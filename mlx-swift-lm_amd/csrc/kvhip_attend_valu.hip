@@ -1,5 +1,5 @@
 // Attention on the vector ALUs, for the full-precision caches the matrix-core kernels are not built for: float32
-// caches, and 16-bit caches of head sizes above 256 other than 512 (kvhip_attend_wide.hip).  The fused op
+// caches of unusual head sizes (the others: kvhip_attend_f32.hip), and 16-bit caches of head sizes above 256 other than 512 (kvhip_attend_wide.hip).  The fused op
 // (AttentionUtils.swift:86-93) computes in float32, excluded keys contribute nothing, one rounding at the output.
 //
 // 2 * rows FMAs per cached element is below what the memory system delivers them at up to 8 query rows per kv head,
@@ -395,12 +395,14 @@ hipError_t launch_merge_valu(const AttendArgs &a, int nparts, hipStream_t s) {
 
 size_t attend_valu_workspace(const AttendArgs &a) {
     if (attend_wide_supported(a)) return attend_wide_workspace(a);
+    if (attend_f32_supported(a)) return attend_f32_workspace(a);
     const PlanValu p = plan_valu(a);
     return p.nparts == 1 ? 0 : (size_t)a.st.BH * p.nparts * (a.Hq / a.Hkv) * a.L * (a.st.Dv + 2) * sizeof(float);
 }
 
 hipError_t launch_attend_valu(const AttendArgs &a, hipStream_t s) {
     if (attend_wide_supported(a)) return launch_attend_wide(a, s);
+    if (attend_f32_supported(a)) return launch_attend_f32(a, s);
     const PlanValu p = plan_valu(a);
     if (a.st.dtype == KVHIP_F16) return launch_dt<0>(a, p, s);
     if (a.st.dtype == KVHIP_BF16) return launch_dt<1>(a, p, s);

@@ -72,31 +72,14 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
     const int r = a.Hq / a.Hkv, R = r * a.L;
     const int row0 = (lin % gridDim.x) * 16 * QT, row1 = min(row0 + 16 * QT, R) - 1;
 
-    // ---- the keys this row block sees (vis) and those all of its rows see (full) --------------------
+    // ---- the keys this row block sees ---------------------------------------------------------------
     const bool one_head = row0 / a.L == row1 / a.L;
-    const int l0 = one_head ? row0 % a.L : 0, l1 = one_head ? row1 % a.L : a.L - 1;
-    int vis_lo = 0, vis_hi = a.T - 1, full_lo = 0, full_hi = a.T - 1;
-    if (a.mask.mode == KVHIP_MASK_CAUSAL) {
-        vis_hi = min(vis_hi, a.T - a.L + l1);
-        full_hi = min(full_hi, a.T - a.L + l0);
-    } else if (a.mask.mode == KVHIP_MASK_WINDOW) {
-        const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
-        vis_lo = max(0, sym.pad_b);
-        full_lo = vis_lo;
-        if (sym.window > 0) {
-            vis_lo = max(vis_lo, sym.offset + l0 - sym.window + 1);
-            full_lo = max(full_lo, sym.offset + l1 - sym.window + 1);
-        }
-        vis_hi = min(vis_hi, min(sym.offset + l1, sym.len_b - 1));
-        full_hi = min(full_hi, min(sym.offset + l0, sym.len_b - 1));
-    } else if (a.mask.mode == KVHIP_MASK_ARRAY) {
-        full_hi = -1;
-    }
+    const KeyRange keys = visible_keys(a.mask, b, a.L, a.T, one_head ? row0 % a.L : 0, one_head ? row1 % a.L : a.L - 1);
     const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
     int t_lo = 0, t_hi = tiles_total;
     if (ident) {
-        t_lo = min(vis_lo / WT, tiles_total);
-        t_hi = vis_hi < vis_lo ? t_lo : min(tiles_total, vis_hi / WT + 1);
+        t_lo = min(keys.lo / WT, tiles_total);
+        t_hi = keys.hi < keys.lo ? t_lo : min(tiles_total, keys.hi / WT + 1);
     }
     const int per = (max(t_hi - t_lo, 1) + nparts - 1) / nparts;
     const int tb = min(t_lo + part * per, t_hi), te = min(tb + per, t_hi);
@@ -157,7 +140,7 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) sc[j] = sum[j >> 2][j & 3] * a.scale;
         const int slot0 = t * WT;
-        if (!ident || slot0 < full_lo || slot0 + WT - 1 > full_hi) {  // workgroup-uniform
+        if (!ident || slot0 < keys.full_lo || slot0 + WT - 1 > keys.full_hi) {  // workgroup-uniform
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int slot = slot0 + 8 * g + j;

@@ -319,11 +319,14 @@ bool attend_valu_supported(const AttendArgs &a);
 bool attend_valu_dequant_first(const AttendArgs &a);
 size_t attend_valu_workspace(const AttendArgs &a);
 hipError_t launch_attend_valu(const AttendArgs &a, hipStream_t s);
-// The same calls where the matrix cores serve them (kvhip_attend_wide.hip: 16-bit caches of head size 512); the merge
+// The same calls where the matrix cores serve them (kvhip_attend_wide.hip: 16-bit caches of head size 512), and the merge
 // of their key-range partials [bh][part][row][Dv + 2] (output row, maximum, sum).
 bool attend_wide_supported(const AttendArgs &a);
 size_t attend_wide_workspace(const AttendArgs &a);
 hipError_t launch_attend_wide(const AttendArgs &a, hipStream_t s);
+bool attend_f32_supported(const AttendArgs &a);  // kvhip_attend_f32.hip: float32 caches of the usual head sizes
+size_t attend_f32_workspace(const AttendArgs &a);
+hipError_t launch_attend_f32(const AttendArgs &a, hipStream_t s);
 hipError_t launch_merge_valu(const AttendArgs &a, int nparts, hipStream_t s);
 // Fast split-sequence decode kernels; `supported` says whether the shape is covered.
 bool attend_decode_supported(const AttendArgs &a);

@@ -112,6 +112,31 @@ __device__ __forceinline__ void sym_mask_full_range(const SymMask &s, int &lo, i
     if (s.window > 0) lo = max(lo, s.offset + s.L - s.window);
 }
 
+// Key rows some (lo .. hi) and all (full_lo .. full_hi) of the query positions l0 .. l1 of batch row b see, both
+// inclusive, empty if low > high; array masks: every key, and none for certain.
+struct KeyRange {
+    int lo, hi, full_lo, full_hi;
+};
+__device__ __forceinline__ KeyRange visible_keys(const MaskDev &m, int b, int L, int T, int l0, int l1) {
+    KeyRange k{0, T - 1, 0, T - 1};
+    if (m.mode == KVHIP_MASK_CAUSAL) {
+        k.hi = min(k.hi, T - L + l1);
+        k.full_hi = min(k.full_hi, T - L + l0);
+    } else if (m.mode == KVHIP_MASK_WINDOW) {
+        const SymMask s = sym_mask_init(m, b, L, T);
+        k.lo = k.full_lo = max(0, s.pad_b);
+        if (s.window > 0) {
+            k.lo = max(k.lo, s.offset + l0 - s.window + 1);
+            k.full_lo = max(k.full_lo, s.offset + l1 - s.window + 1);
+        }
+        k.hi = min(k.hi, min(s.offset + l1, s.len_b - 1));
+        k.full_hi = min(k.full_hi, min(s.offset + l0, s.len_b - 1));
+    } else if (m.mode == KVHIP_MASK_ARRAY) {
+        k.full_hi = -1;
+    }
+    return k;
+}
+
 // ---- which batch row a workgroup row takes, for ragged batches ------------------------------------
 // Workgroups are started in id order, one per CU and then a second one per CU, so rows v and v + B/2 of a
 // launch of 512 workgroups share CUs.  Taking the batch rows in order of their visible length -- the first

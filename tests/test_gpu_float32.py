@@ -200,3 +200,27 @@ def test_quantized_cache_with_float32_scales(bits, gs, Dk, Dv):
         close(out, ref.astype(np.float64), f"L={Lq} {mode}")
     for i, (a, b) in enumerate(zip(c.state, o.get_state())):
         assert np.array_equal(np32(a), b.astype(np.float32) if i % 3 else b), i
+
+
+@pytest.mark.parametrize("Dk,Dv", [(64, 64), (96, 96), (128, 128), (256, 256), (192, 128)])
+@pytest.mark.parametrize("T,n", [(1, 1), (15, 1), (17, 4), (33, 5), (63, 8), (65, 9), (256, 2), (300, 70), (1030, 17), (5000, 1)])
+def test_edges_of_the_matrix_core_tiles(Dk, Dv, T, n):
+    """Keys around multiples of the 16-, 32- and 64-token tiles, rows per kv head around 16 and 32, a window and padding that
+    leave tiles out; float64 at the tolerance above (a float32 sum of 256 products and one of T probabilities)."""
+    B, Hkv, r = 2, 2, 4
+    gen = torch.Generator(device="cuda").manual_seed(T + n + Dk)
+    q, k, v = (torch.randn(B, h, m, d, generator=gen, device="cuda") for h, m, d in ((Hkv * r, n, Dk), (Hkv, T, Dk), (Hkv, T, Dv)))
+    c = kvhip.KVCacheSimple()
+    c.update(k, v, fetch=False)
+    i, j = torch.arange(n, device="cuda")[:, None] + T - n, torch.arange(T, device="cuda")[None]
+    pad = torch.tensor([0, T // 3], dtype=torch.int32, device="cuda")
+    window = T // 2 + 1
+    for mask, hidden in [(kvhip.MaskMode.causal(), (j > i).expand(B, 1, n, T)),
+                         (kvhip.MaskMode.window_mask(T - n, window, left_pad=pad),
+                          (j > i) | (i >= j + window) | (j[None, None] < pad[:, None, None, None]))]:
+        out = c.attend(q, Dk ** -0.5, mask)
+        assert family() == 5
+        kk, vv = (x.double().repeat_interleave(r, 1).contiguous() for x in (k, v))
+        s = torch.matmul(q.double(), kk.transpose(-1, -2).contiguous()) * Dk ** -0.5
+        p = torch.nan_to_num(torch.softmax(s.masked_fill(hidden, float("-inf")), -1))  # (a row without keys gives zeros)
+        close(out, torch.matmul(p, vv).cpu().numpy(), f"{mask.mode}")
