@@ -1155,12 +1155,23 @@ kvhip_status attend_dequant_first(kvhip_cache *c, const AttendArgs &a, hipStream
     return KVHIP_OK;
 }
 
+// the queries [B, Hq, L, D] go along with the next append of this rotation
+void queries_ride(RopeDev &r, const void *q, void *q_rotated, int B, int Hq, int L, int D) {
+    r.qx = static_cast<const char *>(q);
+    r.qo = static_cast<char *>(q_rotated);
+    r.qB = B;
+    r.qH = Hq;
+    r.qL = L;
+    r.qD = D;
+}
+
 // new_k / new_v: the rows of a single-token step whose bookkeeping is done but whose write into physical
 // slot `new_slot` is still owed; the decode kernel takes them along when it can, else they are
-// appended by a launch of their own first.
+// appended by a launch of their own first.  `rope`: the queries and the new key row are still to be rotated (its H:
+// kv heads), by whichever of the two launches takes the row.
 kvhip_status attend_impl(kvhip_cache *c, const void *q, int32_t B, int32_t Hq, int32_t L, int32_t D, float scale,
                          const kvhip_mask *mask, void *out, void *stream, float *fixed, size_t fixed_bytes,
-                         const void *new_k = nullptr, const void *new_v = nullptr, int32_t new_slot = -1) {
+                         const void *new_k = nullptr, const void *new_v = nullptr, int32_t new_slot = -1, RopeDev *rope = nullptr) {
     if (!c || !q || !out) return fail(KVHIP_ERR_INVALID_ARG, "null argument");
     const bool staged_view = c->staging && !c->stage_view.empty();
     if (!c->has_geom || (!c->has_buffers && !staged_view) || c->presented <= 0)
@@ -1233,10 +1244,20 @@ kvhip_status attend_impl(kvhip_cache *c, const void *q, int32_t B, int32_t Hq, i
             a.new_k = new_k;
             a.new_v = new_v;
             a.new_slot = new_slot;
-        } else if (c->st.bits != 0) {
-            KV_HIP(launch_append_quant(c->st, new_k, new_v, 1, 0, new_slot, 1, s, nullptr));
+            a.rope = rope;
         } else {
-            KV_HIP(launch_append_fp(c->st, new_k, new_v, 1, 0, new_slot, 1, s, nullptr));
+            if (rope) {
+                KV_TRY(ensure_pad_buf(c, 4, (size_t)B * Hq * D * c->st.es));
+                a.q = c->pad_buf[4];
+                if (rope->vec) queries_ride(*rope, q, c->pad_buf[4], B, Hq, 1, D);
+                else {
+                    RopeDev own = *rope;
+                    own.H = Hq;
+                    KV_HIP(launch_rope_apply(own, q, c->pad_buf[4], B, Hq, 1, D, c->st.dtype, s));
+                }
+            }
+            if (c->st.bits != 0) KV_HIP(launch_append_quant(c->st, new_k, new_v, 1, 0, new_slot, 1, s, rope));
+            else KV_HIP(launch_append_fp(c->st, new_k, new_v, 1, 0, new_slot, 1, s, rope));
         }
     }
     if (g_policy != 1 && attend_decode_supported(a)) {
@@ -1336,6 +1357,26 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
     RopeDev r;
     const int64_t offset = c->offset;
     KV_TRY(rope_dev(rope, Dk, Hkv, dtype, offset + (c->staging ? (int64_t)c->staged.size() : 0), batch_offsets, r));
+    // One new token without a mask: the decode kernels rotate its rows themselves, as they write the new one
+    // (kvhip_cache_update_attend), and the step is a launch less.
+    if (L == 1 && !c->staging && (dtype == KVHIP_F16 || dtype == KVHIP_BF16) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
+        c->has_geom && c->has_buffers && !c->padded() && c->B == B && c->Hkv == Hkv && c->st.Dk == Dk && c->st.Dv == Dv &&
+        c->st.dtype == dtype && (size_t)B * Hkv + (size_t)B * Hq <= 65535) {
+        int32_t slot = -1;
+        if (c->kind == KVHIP_KIND_ROTATING) {
+            KV_TRY(update_rotating(c, k, v, 1, S(c, stream), &slot));
+        } else {
+            KV_TRY(update_simple(c, k, v, 1, S(c, stream), false));
+            slot = (int32_t)c->offset - 1;
+        }
+        const kvhip_status st = attend_impl(c, q, B, Hq, L, Dk, scale, mask, out, stream, nullptr, 0, k, v, slot, &r);
+        if (st != KVHIP_OK) {  // the cache holds what its counters say
+            r.qx = nullptr;
+            if (c->st.bits != 0) (void)launch_append_quant(c->st, k, v, 1, 0, slot, 1, S(c, stream), &r);
+            else (void)launch_append_fp(c->st, k, v, 1, 0, slot, 1, S(c, stream), &r);
+        }
+        return st;
+    }
     if (!q_rotated) {
         KV_TRY(ensure_pad_buf(c, 4, (size_t)B * Hq * L * Dk * (dtype == KVHIP_F32 ? 4 : 2)));
         q_rotated = c->pad_buf[4];
@@ -1344,12 +1385,7 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
     // 3 to 5 us on the device and as much on the host).
     const size_t q_rows = (size_t)B * L;  // (at most so many grid rows of query workgroups: rope_ride_rows)
     if (r.vec && !c->staging && (size_t)B * Hkv + (q_rows >= 256 ? q_rows : q_rows * Hq) <= 65535) {
-        r.qx = static_cast<const char *>(q);
-        r.qo = static_cast<char *>(q_rotated);
-        r.qB = B;
-        r.qH = Hq;
-        r.qL = L;
-        r.qD = Dk;
+        queries_ride(r, q, q_rotated, B, Hq, L, Dk);
     }
     const bool ride = r.qx != nullptr;
     c->rope = &r;

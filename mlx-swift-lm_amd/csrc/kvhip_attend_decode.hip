@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "kvhip_mask.hpp"
+#include "kvhip_rope.hpp"
 
 // piece buffers of the full-precision decode kernel (at most the D / 32 pieces of one tile)
 #ifndef KVHIP_DECODE_FP_NBUF
@@ -205,9 +206,12 @@ template <int BITS, int D, int G> struct TileRegs {
 // NW = wavefronts per workgroup: 4 (two workgroups per CU), or 8 when that lets one
 // workgroup take the whole sequence of its (batch, kv-head) pair -- then the output rows are
 // normalised and written here and no partial goes through memory.
-template <int BITS, int D, int GS, int DT, int RG, int MM, int NW>
+// MODE 3: MM 0, with the step's rows still to be rotated.
+template <int BITS, int D, int GS, int DT, int RG, int MODE, int NW>
 __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
-decode_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
+decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_wg, int nsplit) {
+    constexpr int MM = MODE == 3 ? 0 : MODE;
+    constexpr bool rot = MODE == 3;
     using GEO = Geo<BITS>;
     constexpr int G = D / GS;      // quantization groups per row (1, 2 or 4)
     constexpr int NH = D / 64;     // 64-column halves of the output
@@ -239,7 +243,15 @@ decode_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
     const int r = a.Hq / a.Hkv;
     const int R = r * a.L;
 
-    __shared__ float cbuf[NW][RR][D + 2];
+    __shared__ __attribute__((aligned(16))) float cbuf[NW][RR][D + 2];
+    // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
+    // the end) for the wavefronts to fetch them.
+    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
+    if constexpr (rot) {
+        rope_stage_step<DT, D>(a.turn, bh, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
+                                static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R, rot_s);
+        __syncthreads();
+    }
 
     // ---- query operands: lane (blk, qi) holds row qi's 4 elements of step 16 x + blk ----
     // qsum[rg][g][i] = sum over group g of the (rounded, fp16-held) query row 4 rg + i, for
@@ -265,7 +277,10 @@ decode_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
             const int step = 16 * x + blk;
             const int w = step / GEO::WSTEPS, h = step % GEO::WSTEPS;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) raw[x][k] = Elem<DT>::load(a.q, qoff + w * GEO::EPW + GEO::elem(h, k));
+            for (int k = 0; k < 4; ++k) {
+                const int d = w * GEO::EPW + GEO::elem(h, k);
+                raw[x][k] = rot ? Elem<DT>::load(rot_s, rep * D + d) : Elem<DT>::load(a.q, qoff + d);
+            }
         }
         float part[G];
 #pragma unroll
@@ -388,7 +403,7 @@ decode_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
             if (tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % NW) == wave) {
                 const char *krow = static_cast<const char *>(a.new_k) + (size_t)bh * D * 2;
                 const char *vrow = static_cast<const char *>(a.new_v) + (size_t)bh * D * 2;
-                quantize_row_wave_from<DT, BITS>([&](int d) { return Elem<DT>::load(krow, d); }, D, GS, lane,
+                quantize_row_wave_from<DT, BITS>([&](int d) { return rot ? Elem<DT>::load(rot_s, R * D + d) : Elem<DT>::load(krow, d); }, D, GS, lane,
                                                  reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))),
                                                  [](int, uint32_t) {}, const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
                 char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
@@ -642,6 +657,7 @@ decode_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
     }
 
     // ---- wavefront partial -> LDS ---------------------------------------------------
+    if (rot) __syncthreads();  // (the rotated rows have been fetched)
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
 #pragma unroll
@@ -722,9 +738,11 @@ decode_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
 // The load of the next piece is issued as soon as a buffer has been consumed.
 // bf16 keeps P as a (hi, lo) pair of bf16 values so the PV product carries 16 bits of
 // probability; rows of a RotatingKVCache are found through the run table.
-template <int D, int DT, int RG, int MM, bool IDENT>
+template <int D, int DT, int RG, int MODE, bool IDENT>
 __global__ void __launch_bounds__(WAVES * 64, 2)
-decode_fp_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
+decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_wg, int nsplit) {
+    constexpr int MM = MODE == 3 ? 0 : MODE;
+    constexpr bool rot = MODE == 3;
     constexpr bool BF = DT == 1;
     constexpr int NP = D / 64;   // pieces per K row and per V tile column set
     constexpr int RR = 4 * RG;
@@ -738,7 +756,15 @@ decode_fp_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
     const int r = a.Hq / a.Hkv;
     const int R = r * a.L;
 
-    __shared__ float cbuf[WAVES][RR][D + 2];
+    __shared__ __attribute__((aligned(16))) float cbuf[WAVES][RR][D + 2];
+    // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
+    // the end) for the wavefronts to fetch them.
+    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
+    if constexpr (rot) {
+        rope_stage_step<DT, D>(a.turn, bh, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
+                                static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R, rot_s);
+        __syncthreads();
+    }
 
     // query operands: lane (blk, qi) holds row qi's elements 4*(16 x + blk) .. +3, unscaled
     // (fetched by the main loop after it has requested its first two pieces)
@@ -752,8 +778,10 @@ decode_fp_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
 #pragma unroll
             for (int x = 0; x < NP; ++x) {
                 uint2 w = make_uint2(0, 0);
-                if (i < R)
-                    w = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.q) + qoff + 4 * (16 * x + blk));
+                if (i < R) {
+                    if (rot) w = *reinterpret_cast<const uint2 *>(rot_s + rep * D + 4 * (16 * x + blk));
+                    else w = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.q) + qoff + 4 * (16 * x + blk));
+                }
                 qa[rg][x].u[0] = w.x;
                 qa[rg][x].u[1] = w.y;
             }
@@ -803,7 +831,8 @@ decode_fp_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
                 char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot));
                 char *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
                 if (lane < D / 8)  // one 16-byte chunk of the K row per lane
-                    *reinterpret_cast<uint4 *>(kc + kfp_off(st, slot, 8 * lane)) = *reinterpret_cast<const uint4 *>(krow + 8 * lane);
+                    *reinterpret_cast<uint4 *>(kc + kfp_off(st, slot, 8 * lane)) =
+                        rot ? *reinterpret_cast<const uint4 *>(rot_s + R * D + 8 * lane) : *reinterpret_cast<const uint4 *>(krow + 8 * lane);
                 for (int d = lane; d < D; d += 64)
                     *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, d)) = vrow[d];
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -981,6 +1010,7 @@ decode_fp_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
         }
     }
 
+    if (rot) __syncthreads();  // (the rotated rows have been fetched)
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
 #pragma unroll
@@ -1373,18 +1403,21 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
     const Plan p = plan_for(a);
     const Store &st = a.st;
     dim3 grid(p.nsplit, st.BH), block(WAVES * 64);  // the quantized kernel sets its own block size
-    const int mm = a.mask.mode == KVHIP_MASK_NONE ? 0 : (a.mask.mode == KVHIP_MASK_ARRAY ? 2 : 1);
+    const int mm = decode_mode(a);
 #define DEC_K(BITS, D, GS, DT, RG, MM, NW)                                                                \
-    hipLaunchKernelGGL((decode_kernel<BITS, D, GS, DT, RG, MM, NW>), grid, dim3(NW * 64), 0, s, a,        \
+    hipLaunchKernelGGL((decode_kernel<BITS, D, GS, DT, RG, MM, NW>), grid, dim3(NW * 64), 0, s, DecodeArgs<MM>::type(a), \
                        p.tiles_total, p.tiles_per_wg, p.nsplit)
 #define DEC(BITS, D, GS, DT, RG)                                                                          \
     do {                                                                                                  \
         profile_mark(s, true);                                                                            \
         if (p.nw == 2 * WAVES) {                                                                          \
             if (mm == 0) DEC_K(BITS, D, GS, DT, RG, 0, 2 * WAVES);                                        \
+            else if (mm == 3) DEC_K(BITS, D, GS, DT, RG, 3, 2 * WAVES);                                   \
             else DEC_K(BITS, D, GS, DT, RG, 1, 2 * WAVES);                                                \
         } else if (mm == 0) {                                                                             \
             DEC_K(BITS, D, GS, DT, RG, 0, WAVES);                                                         \
+        } else if (mm == 3) {                                                                             \
+            DEC_K(BITS, D, GS, DT, RG, 3, WAVES);                                                         \
         } else if (mm == 1) {                                                                             \
             DEC_K(BITS, D, GS, DT, RG, 1, WAVES);                                                         \
         } else {                                                                                          \
@@ -1422,7 +1455,7 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
 #define FP(D, DT, RG, M, I)                                                                               \
     do {                                                                                                  \
         profile_mark(s, true);                                                                            \
-        hipLaunchKernelGGL((decode_fp_kernel<D, DT, RG, M, I>), grid, block, 0, s, a, p.tiles_total,      \
+        hipLaunchKernelGGL((decode_fp_kernel<D, DT, RG, M, I>), grid, block, 0, s, DecodeArgs<M>::type(a), p.tiles_total, \
                            p.tiles_per_wg, p.nsplit);                                                     \
         profile_mark(s, false);                                                                           \
         if (p.nsplit > 1)                                                                                 \
@@ -1432,6 +1465,8 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
     do {                                                          \
         if (mm == 0 && ident) FP(D, DT, RG, 0, true);             \
         else if (mm == 0) FP(D, DT, RG, 0, false);                \
+        else if (mm == 3 && ident) FP(D, DT, RG, 3, true);        \
+        else if (mm == 3) FP(D, DT, RG, 3, false);                \
         else if (mm == 1 && ident) FP(D, DT, RG, 1, true);        \
         else if (mm == 1) FP(D, DT, RG, 1, false);                \
         else if (ident) FP(D, DT, RG, 2, true);                   \

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "kvhip_mask.hpp"
+#include "kvhip_rope.hpp"
 
 namespace kvhip {
 
@@ -141,9 +142,12 @@ template <int BITS> __device__ __forceinline__ constexpr bool hi_of(int p) { ret
 // (8-bit codes at D = 256 take more than 256 registers: one workgroup per CU)
 // DK / DV: head sizes of keys / queries and of values / outputs (192 and 128 for the multi-head latent attention
 // models, equal otherwise).
-template <int BITS, int DK, int DV, int GS, int DT, int MM>
+// MODE 3: MM 0, with the step's rows still to be rotated.
+template <int BITS, int DK, int DV, int GS, int DT, int MODE>
 __global__ void __launch_bounds__(WAVES * 64, (DK >= 256 && BITS == 8) ? 1 : 2)
-decode16_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
+decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_wg, int nsplit) {
+    constexpr int MM = MODE == 3 ? 0 : MODE;
+    constexpr bool rot = MODE == 3;
     constexpr bool GEN = BITS != 4 && BITS != 8;  // bit streams
     using SK = Seg<(GS / 4) * BITS, GS * BITS / 32>;  // a lane's segment of a K group
     using SV = Seg<16 * BITS, 2 * BITS>;              // a lane's 16 tokens of a V tile row
@@ -174,9 +178,17 @@ decode16_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
     const int R = r * a.L;
     size_t part_slot = (size_t)bh * nsplit + split;  // where this workgroup's partial goes
 
-    __shared__ float cbuf[WAVES][RR][DV + 2];
+    __shared__ __attribute__((aligned(16))) float cbuf[WAVES][RR][DV + 2];
     __shared__ __attribute__((aligned(16))) uint32_t sbuf[WAVES][2][2][SB_WORDS];  // [wavefront][tile parity][K, V][pairs]
 
+    // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
+    // the end) for the wavefronts to fetch them.
+    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
+    if constexpr (rot) {
+        rope_stage_step<DT, DK>(a.turn, bh, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * DK,
+                                static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK, R, rot_s);
+        __syncthreads();
+    }
     // ---- span of this workgroup (as in the 4-row kernel) -----------------------------------
     if constexpr (MM == 1) {
         // a ragged batch whose rows divide their own ranges over the same number of spans: long and short
@@ -226,7 +238,7 @@ decode16_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
             if (tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % WAVES) == wave) {
                 const char *krow = static_cast<const char *>(a.new_k) + (size_t)bh * DK * 2;
                 const char *vrow = static_cast<const char *>(a.new_v) + (size_t)bh * DV * 2;
-                quantize_row_wave_from<DT, BITS>([&](int d) { return Elem<DT>::load(krow, d); }, DK, GS, lane,
+                quantize_row_wave_from<DT, BITS>([&](int d) { return rot ? Elem<DT>::load(rot_s, R * DK + d) : Elem<DT>::load(krow, d); }, DK, GS, lane,
                                                  reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))),
                                                  [](int, uint32_t) {}, const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
                 char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
@@ -394,8 +406,10 @@ decode16_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
 #pragma unroll
         for (int g = 0; g < GK; ++g)
 #pragma unroll
-            for (int h = 0; h < SPG; ++h)
-                raw[g][h] = *reinterpret_cast<const u4 *>(qrow + GS * g + (GS / 4) * jj + 8 * h);
+            for (int h = 0; h < SPG; ++h) {
+                if (rot) raw[g][h] = *reinterpret_cast<const u4 *>(rot_s + rep * DK + GS * g + (GS / 4) * jj + 8 * h);
+                else raw[g][h] = *reinterpret_cast<const u4 *>(qrow + GS * g + (GS / 4) * jj + 8 * h);
+            }
 #pragma unroll
         for (int g = 0; g < GK; ++g) {
             float part = 0.f;
@@ -642,6 +656,7 @@ decode16_kernel(AttendArgs a, int tiles_total, int tiles_per_wg, int nsplit) {
         for (int g = 0; g < GK; ++g) qsum[g] = 0.f;
     }
 
+    if (rot) __syncthreads();  // (the rotated rows have been fetched)
     // ---- wavefront partial -> LDS: lane (n, jj) holds out^T[d = 16 db + 4 jj + i][row n] ---------
     if constexpr (SPLIT_HI) {
         l_part = __builtin_fmaf(l_hi, 16.f, l_part);
@@ -718,10 +733,11 @@ template <int BITS>
 hipError_t launch_decode16_bits(const AttendArgs &a, int tiles_total, int tiles_per_wg, int nsplit, hipStream_t s) {
     const Store &st = a.st;
     dim3 grid(nsplit, st.BH), block(WAVES * 64);
-    const int mm = a.mask.mode == KVHIP_MASK_NONE ? 0 : (a.mask.mode == KVHIP_MASK_ARRAY ? 2 : 1);
+    const int mm = decode_mode(a);
 #define D16_M(DK, DV, GS, DT)                                                                                   \
     do {                                                                                                        \
         if (mm == 0) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 0>), grid, block, 0, s, a, tiles_total, tiles_per_wg, nsplit); \
+        else if (mm == 3) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 3>), grid, block, 0, s, AttendStepArgs(a), tiles_total, tiles_per_wg, nsplit); \
         else if (mm == 1) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 1>), grid, block, 0, s, a, tiles_total, tiles_per_wg, nsplit); \
         else hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 2>), grid, block, 0, s, a, tiles_total, tiles_per_wg, nsplit); \
     } while (0)

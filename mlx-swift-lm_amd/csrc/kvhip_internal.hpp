@@ -302,10 +302,26 @@ struct AttendArgs {
     const void *new_k = nullptr;
     const void *new_v = nullptr;
     int new_slot = -1;
+    // With new_k: the rotation that the queries and the new key row still need, at the new row's position (host; NULL: none).
+    const RopeDev *rope = nullptr;
     // Upper bound on the scratch a launch may plan for (0: none).  The planners then split the sequence over
     // fewer spans or key-range parts, down to one, which needs no scratch at all.
     size_t workspace_cap = 0;
 };
+// What a decode kernel that rotates the step's rows itself is launched with (MODE 3 of the kernels; MODE 0 to 2: their
+// mask code).  A struct and instances of their own: a test of the arguments in the others cost the 16-row kernel 3 to 5 %
+// (B8, 64q/8kv, 8192 keys, 4 bits: 27.2 against 28.7 us).
+struct AttendStepArgs : AttendArgs {
+    RopeDev turn;
+    explicit AttendStepArgs(const AttendArgs &a) : AttendArgs(a), turn(a.rope ? *a.rope : RopeDev()) {}
+};
+template <int MODE> struct DecodeArgs { using type = AttendArgs; };
+template <> struct DecodeArgs<3> { using type = AttendStepArgs; };
+// 0: no mask, 1: index-only mask, 2: array mask, 3: no mask, rows still to be rotated
+inline int decode_mode(const AttendArgs &a) {
+    if (a.mask.mode == KVHIP_MASK_NONE) return a.new_k && a.rope ? 3 : 0;
+    return a.mask.mode == KVHIP_MASK_ARRAY ? 2 : 1;
+}
 // Whether launch_attend_decode writes a.new_k / a.new_v itself for these arguments.
 bool attend_decode_fuses_append(const AttendArgs &a);
 // Bytes of scratch each kernel family needs for these arguments.

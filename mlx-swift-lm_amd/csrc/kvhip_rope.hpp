@@ -136,6 +136,33 @@ __device__ __forceinline__ void rope_chunk(const RopeDev &r, const float *inv_s,
         w[j] = round_dt<DT>(r.traditional ? rope_turn(x[j], x[j ^ 1], (j & 1) == 0, sn[j], cs[j]) : rope_turn(x[j], y[j], first, sn[j], cs[j]));
 }
 
+// ---- one token's rows, for the decode kernels --------------------------------------------------------------------
+// The R query rows (adjacent, D elements) and the key row of one kv head, rotated and rounded to the dtype, into LDS
+// [R + 1][D]; the caller synchronises.  A thread owns one pair of columns and forms its sine and cosine once; all 256
+// (512) threads of the workgroup take part.  Every workgroup of the launch does this for itself: about 1 us behind
+// which no launch, no copy of the queries and no gap stand (a launch for it: 4 to 6.5 us).
+template <int DT, int D>
+__device__ __forceinline__ void rope_stage_step(const RopeDev &r, int bh, const uint16_t *q, const uint16_t *k, int R, uint16_t *dst) {
+    constexpr int P = D / 2;
+    const int p = threadIdx.x % P, ns = blockDim.x / P, half = r.dims >> 1;
+    const bool turn = p < half;
+    const int d0 = !turn ? r.dims + 2 * (p - half) : r.traditional ? 2 * p : p;
+    const int d1 = turn && !r.traditional ? d0 + half : d0 + 1;
+    float sn = 0.f, cs = 1.f;
+    if (turn) rope_sincos(rope_angle(r, rope_pos(r, bh, 0), rope_inv_freq(r, p)), sn, cs);
+    for (int i = threadIdx.x / P; i <= R && threadIdx.x < ns * P; i += ns) {
+        const uint16_t *row = i < R ? q + (size_t)i * D : k;
+        uint16_t x = row[d0], y = row[d1];
+        if (turn) {
+            const float a = Elem<DT>::load(&x, 0), b = Elem<DT>::load(&y, 0);
+            Elem<DT>::store(&x, 0, rope_turn(a, b, true, sn, cs));
+            Elem<DT>::store(&y, 0, rope_turn(b, a, false, sn, cs));
+        }
+        dst[i * D + d0] = x;
+        dst[i * D + d1] = y;
+    }
+}
+
 // ---- the queries of a forward ----------------------------------------------------------------------------------
 // One row position (batch row b, row l of L) of `x` [B, H, L, D] into `out` (which may be x) for heads [h0, h1): a
 // thread owns one chunk pair (chunk, when the pairs are adjacent), works out its sines and cosines once and turns

@@ -201,22 +201,23 @@ def _cache_of(kind):
     return kvhip.RotatingKVCache(150, keep=4) if kind == "ring" else kvhip.QuantizedKVCache(32, kind)
 
 
-@pytest.mark.parametrize("kind", ["simple", "ring", 4, 3])
+@pytest.mark.parametrize("kind", ["simple", "ring", 4, 3, 8])
 @pytest.mark.parametrize("dtype,Hq,Hkv,Dk,Dv,dims,traditional", [
     (torch.float16, 8, 2, 128, 128, 128, False), (torch.bfloat16, 40, 4, 64, 64, 64, False),
-    (torch.float16, 6, 2, 96, 96, 64, True), (torch.bfloat16, 4, 4, 192, 128, 64, False),
+    (torch.float16, 6, 2, 96, 96, 64, True), (torch.bfloat16, 8, 4, 256, 256, 256, False), (torch.float16, 4, 4, 128, 128, 32, True), (torch.bfloat16, 4, 4, 192, 128, 64, False),
     (torch.float16, 4, 2, 128, 128, 72, False),     # pairs cut through 16-byte chunks: a launch of its own
     (torch.bfloat16, 4, 1, 512, 512, 512, False), (torch.float32, 4, 2, 64, 64, 64, False)])
 def test_queries_in_the_appends_launch_equal_separate_calls(kind, dtype, Hq, Hkv, Dk, Dv, dims, traditional):
-    """Bit for bit: the one call runs the same rotation, append and attention as the three."""
+    """Bit for bit: the one call runs the same rotation, append and attention as the three (and a single token's decode
+    kernel, which rotates its rows itself, the same arithmetic)."""
     B = 3
     rope = kvhip.RoPE(dims, traditional=traditional, base=1e6)
     one, three = _cache_of(kind), _cache_of(kind)
     gen = torch.Generator(device="cuda").manual_seed(11)
     positions = torch.tensor([5, 0, 1000], dtype=torch.int32, device="cuda")
-    for step, Lq in enumerate((70, 1, 5, 131, 2, 1)):
+    for step, Lq in enumerate((70, 1, 5, 131, 2, 1, 1, 1)):
         q, k, v = (torch.randn(B, h, Lq, d, generator=gen, device="cuda").to(dtype) for h, d in ((Hq, Dk), (Hkv, Dk), (Hkv, Dv)))
-        at = positions if step == 2 else None
+        at = positions if step in (2, 6) else None
         mask = kvhip.create_attention_mask(Lq, one)
         got = kvhip.attention_with_rope_and_cache_update(rope, q, k, v, one, Dk ** -0.5, mask, at)
         turned = kvhip.apply_rotary_position(rope, q, at if at is not None else three.offset)
