@@ -1146,51 +1146,55 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
     }
 }
 
-// The same merge for the prefill tiles' key-range parts: many query rows, at most 8 parts.  One wavefront per
-// query row, four rows per workgroup; a lane takes four adjacent columns; no LDS and no barrier (the
-// per-row workgroups above spend their time being launched: 22 us for 16 384 rows of 256 columns).  Decode
-// launches keep the kernel above: with few rows and many parts it has the loads of a column in flight together
+// The same merge for the prefill tiles' key-range parts: many query rows, at most 8 parts.  D / 4 lanes per query row,
+// four adjacent columns each, as many rows per workgroup as fit 256 threads; no LDS and no barrier (the
+// per-row workgroups above spend their time being launched: 22 us for 16 384 rows of 256 columns).  Bound by the latency of
+// its loads: every part's columns, maximum and sum are requested before any of them is looked at (parts up to MAXP = 2, 4
+// or 8; the numbers beyond nsplit repeat the last one's loads and are left out of the sums).  With the maxima read first and a part's columns
+// behind a branch of their own it took 12.0 us where it takes 7.6 (16 384 rows of 128, 3 or 4 parts), 11.1 where 9.6 (256
+// columns).
+// Decode launches keep the kernel above: with few rows and many parts it has the loads of a column in flight together
 // (configs[3]'s ring decode, 2 rows of 16 parts: 29.1 us per step against 31.7 us with this one).
-template <int D, int DT>
+template <int D, int DT, int MAXP>
 __global__ void __launch_bounds__(256) combine_rows_kernel(AttendArgs a, int nsplit, int rr) {
-    const int lane = threadIdx.x & 63;
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), bh = blockIdx.y;
+    constexpr int LPR = D / 4, RPW = 256 / LPR;
+    const int in_wg = threadIdx.x / LPR, c = 4 * (threadIdx.x % LPR);
+    const int i = blockIdx.x * RPW + in_wg, bh = blockIdx.y;
     const int r = a.Hq / a.Hkv;
-    if (i >= r * a.L) return;  // (rr, the rows a part holds, may exceed the query rows there are)
+    if (in_wg >= RPW || i >= r * a.L) return;  // (rr, the rows a part holds, may exceed the query rows there are)
     const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
     const int rep = i / a.L, l = i - rep * a.L;
     const size_t sstride = (size_t)rr * (D + 2);
     const float *part = a.workspace + (size_t)bh * nsplit * sstride + (size_t)i * (D + 2);
-    constexpr int MAXP = 8;
-    float m[MAXP], w[MAXP];
+    float2 ml[MAXP], p[MAXP][2];  // (a row of partials is 8-byte aligned: D + 2 floats)
+#pragma unroll
+    for (int s = 0; s < MAXP; ++s) {
+        const float *row = part + min(s, nsplit - 1) * sstride;
+        ml[s] = *reinterpret_cast<const float2 *>(row + D);
+        p[s][0] = *reinterpret_cast<const float2 *>(row + c);
+        p[s][1] = *reinterpret_cast<const float2 *>(row + c + 2);
+    }
     float mx = -INFINITY;
 #pragma unroll
-    for (int s = 0; s < MAXP; ++s) {
-        m[s] = s < nsplit ? part[s * sstride + D] : -INFINITY;
-        mx = fmaxf(mx, m[s]);
-    }
-    float den = 0.f;
+    for (int s = 0; s < MAXP; ++s) mx = fmaxf(mx, ml[s].x);
+    float den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < MAXP; ++s) {
-        w[s] = (m[s] == -INFINITY) ? 0.f : fast_exp2((m[s] - mx) * LOG2E);
-        if (s < nsplit) den += w[s] * part[s * sstride + D + 1];
+        const float w = ml[s].x == -INFINITY ? 0.f : fast_exp2((ml[s].x - mx) * LOG2E);
+        const bool own = s < nsplit;
+        den = own ? den + w * ml[s].y : den;
+        num[0] = own ? num[0] + w * p[s][0].x : num[0];
+        num[1] = own ? num[1] + w * p[s][0].y : num[1];
+        num[2] = own ? num[2] + w * p[s][1].x : num[2];
+        num[3] = own ? num[3] + w * p[s][1].y : num[3];
     }
-    if (lane >= D / 4) return;
-    float num[4] = {0.f, 0.f, 0.f, 0.f};
+    const size_t ooff = ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D + c;
+    uint32_t *dst = reinterpret_cast<uint32_t *>(static_cast<char *>(a.out) + ooff * 2);
 #pragma unroll
-    for (int s = 0; s < MAXP; ++s)
-        if (s < nsplit) {
-            // (a row of partials is 8-byte aligned: D + 2 floats)
-            const float2 p0 = *reinterpret_cast<const float2 *>(part + s * sstride + 4 * lane);
-            const float2 p1 = *reinterpret_cast<const float2 *>(part + s * sstride + 4 * lane + 2);
-            num[0] += w[s] * p0.x;
-            num[1] += w[s] * p0.y;
-            num[2] += w[s] * p1.x;
-            num[3] += w[s] * p1.y;
-        }
-    const size_t ooff = ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D + 4 * lane;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) Elem<DT>::store(a.out, ooff + c, den > 0.f ? num[c] / den : 0.f);
+    for (int k = 0; k < 2; ++k) {
+        const float o0 = den > 0.f ? num[2 * k] / den : 0.f, o1 = den > 0.f ? num[2 * k + 1] / den : 0.f;
+        dst[k] = DT == 0 ? pk_h2(o0, o1) : pk_bf2(o0, o1);
+    }
 }
 
 struct Plan {
@@ -1323,11 +1327,13 @@ hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t
     const int R = (a.Hq / a.Hkv) * a.L;
     dim3 grid(R, a.st.BH);
     if (rows > 16 && nsplit <= 8 && rows == R) {  // the prefill tiles' parts
-        dim3 grid4((R + 3) / 4, a.st.BH);
+#define CMBR_P(D, DT, P) hipLaunchKernelGGL((combine_rows_kernel<D, DT, P>), dim3((R + 256 / (D / 4) - 1) / (256 / (D / 4)), a.st.BH), dim3(256), 0, s, a, nsplit, rows)
 #define CMBR(D)                                                                                      \
     do {                                                                                             \
-        if (a.st.dtype == KVHIP_F16) hipLaunchKernelGGL((combine_rows_kernel<D, 0>), grid4, dim3(256), 0, s, a, nsplit, rows); \
-        else hipLaunchKernelGGL((combine_rows_kernel<D, 1>), grid4, dim3(256), 0, s, a, nsplit, rows); \
+        const bool h = a.st.dtype == KVHIP_F16;                                                      \
+        if (nsplit <= 2) { if (h) CMBR_P(D, 0, 2); else CMBR_P(D, 1, 2); }                           \
+        else if (nsplit <= 4) { if (h) CMBR_P(D, 0, 4); else CMBR_P(D, 1, 4); }                      \
+        else { if (h) CMBR_P(D, 0, 8); else CMBR_P(D, 1, 8); }                                       \
     } while (0)
         if (a.st.Dv == 64) CMBR(64);
         else if (a.st.Dv == 80) CMBR(80);
@@ -1335,6 +1341,7 @@ hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t
         else if (a.st.Dv == 128) CMBR(128);
         else CMBR(256);
 #undef CMBR
+#undef CMBR_P
         return hipGetLastError();
     }
 #define CMB(D)                                                                                       \
