@@ -1355,8 +1355,8 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
     if (dtype != KVHIP_F16 && dtype != KVHIP_BF16 && dtype != KVHIP_F32)
         return fail(KVHIP_ERR_INVALID_ARG, "rope needs a floating-point dtype");
     RopeDev r;
-    const int64_t offset = c->offset;
-    KV_TRY(rope_dev(rope, Dk, Hkv, dtype, offset + (c->staging ? (int64_t)c->staged.size() : 0), batch_offsets, r));
+    const int64_t pos0 = c->offset + (c->staging ? (int64_t)c->staged.size() : 0);  // (before the write, as in kvhip_cache_update_rope)
+    KV_TRY(rope_dev(rope, Dk, Hkv, dtype, pos0, batch_offsets, r));
     // One new token without a mask: the decode kernels rotate its rows themselves, as they write the new one
     // (kvhip_cache_update_attend), and the step is a launch less.
     if (L == 1 && !c->staging && (dtype == KVHIP_F16 || dtype == KVHIP_BF16) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
@@ -1394,7 +1394,7 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
     if (st != KVHIP_OK) return st;
     if (!ride || r.qx != nullptr) {
         RopeDev own;
-        KV_TRY(rope_dev(rope, Dk, Hq, dtype, offset, batch_offsets, own));
+        KV_TRY(rope_dev(rope, Dk, Hq, dtype, pos0, batch_offsets, own));
         KV_HIP(launch_rope_apply(own, q, q_rotated, B, Hq, L, Dk, dtype, S(c, stream)));
     }
     return kvhip_cache_attend(c, q_rotated, B, Hq, L, Dk, scale, mask, out, stream);

@@ -225,3 +225,30 @@ def test_queries_in_the_appends_launch_equal_separate_calls(kind, dtype, Hq, Hkv
         assert torch.equal(got, three.attend(turned, Dk ** -0.5, mask)), f"step {step}"
     for a, b in zip(one.state, three.state):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("D,dims", [(64, 64), (40, 32), (128, 72)])
+def test_one_call_in_a_staged_round_counts_the_staged_rows(dtype, D, dims):
+    """Queries and keys turn at the offset plus the rows staged so far, as `ropeOffset` has it in an open round (40: a
+    head size stored zero-padded; 72: pairs that cut through 16-byte chunks)."""
+    B, Hq, Hkv = 2, 4, 2
+    rope = kvhip.RoPE(dims, base=1e4)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+
+    def rows(n):
+        return [torch.randn(B, h, n, D, generator=gen, device="cuda").to(dtype) for h in (Hq, Hkv, Hkv)]
+
+    rings = [kvhip.RotatingKVCache(48, keep=2) for _ in range(2)]
+    _, k, v = rows(30)
+    for ring in rings:
+        ring.update(k, v, fetch=False)
+    staged = [kvhip.RotatingStagedKVCache(ring) for ring in rings]
+    for Lq in (2, 1, 3):
+        q, k, v = rows(Lq)
+        turned = kvhip.apply_rotary_position(rope, q, staged[1].rope_offset)
+        staged[1].update_rope(rope, k, v)
+        want = staged[1].attend(turned, D ** -0.5, kvhip.MaskMode.causal())
+        got = rings[0].update_attend_rope(rope, q, k, v, D ** -0.5, kvhip.MaskMode.causal())
+        assert torch.equal(got, want), Lq
+    assert all(torch.equal(a, b) for a, b in zip(staged[0].staged_arrays, staged[1].staged_arrays))
