@@ -5,16 +5,8 @@
 
 namespace kvhip {
 
-// Sine and cosine of a float32 angle.  The angle is reduced by the nearest multiple of pi/2 in double (positions of
-// 10^5 leave an error below 10^-11), the remainder, at most pi/4, goes through the Taylor polynomials of degree 9 and
-// 10 (next terms below 2 10^-9 and 2 10^-10 there).  Some 30 instructions; the library's sincosf carries a
-// multi-word reduction for large angles that the appends spent most of their time in (512 rows of 8 heads x 128:
-// 22.7 us full precision and 18.8 us quantized with it and an exponential per element, 10.3 and 11.4 us so).
-__device__ __forceinline__ void rope_sincos(float theta, float &sn, float &cs) {
-    const double t = (double)theta;
-    const double k = rint(t * 0.63661977236758134308);
-    const float x = (float)fma(-k, 1.57079632679489661923, t);
-    const int quad = (int)(k - 4.0 * floor(k * 0.25));
+// Sine and cosine of a remainder of at most pi/4 and the quadrant it was taken from.
+__device__ __forceinline__ void rope_sincos_reduced(float x, int quad, float &sn, float &cs) {
     const float z = x * x;
     float s = __builtin_fmaf(z, 2.7557319223985893e-6f, -1.9841269841269841e-4f);
     s = __builtin_fmaf(z, s, 8.3333333333333332e-3f);
@@ -28,6 +20,71 @@ __device__ __forceinline__ void rope_sincos(float theta, float &sn, float &cs) {
     const float a = (quad & 1) ? c : s, b = (quad & 1) ? s : c;
     sn = (quad & 2) ? -a : a;
     cs = ((quad + 1) & 2) ? -b : b;
+}
+
+// The same for an angle of 2^24 and more, by Payne and Hanek's method: the angle is m 2^e with an integer m < 2^24, and of
+// 2/pi only the 64 bits from weight 2^(1 - e) on matter to the product modulo 4 (an error of the remainder below 2^-37).
+// A function of its own: positions times frequencies do not get there in ordinary use, and a copy of it beside each of the
+// sixteen short ones of a chunk kept the tile kernels' loops from being unrolled.
+static __device__ __attribute__((noinline)) float2 rope_sincos_large(float theta) {
+    const uint32_t u = __float_as_uint(theta);
+    const int at = (int)((u >> 23) & 255u) - 151;  // the first bit that matters: 0 .. 103 (104: infinite, NaN)
+    const uint64_t m = (u & 0x7fffffu) | 0x800000u;
+    constexpr uint64_t T0 = 0x517cc1b727220a94ull, T1 = 0xfe13abe8fa9a6ee0ull, T2 = 0x6db14acc9e21c820ull;  // 2/pi, the first bit has weight 1
+    const uint64_t hi = at < 64 ? T0 : T1, lo = at < 64 ? T1 : T2;
+    const uint64_t p = m * ((hi << (at & 63)) | ((lo >> 1) >> (63 - (at & 63))));  // times 2^62, modulo 4
+    const uint64_t k = (p + (1ull << 61)) >> 62;
+    const float x = at == 104 ? theta - theta : (float)((double)(int64_t)(p - (k << 62)) * 3.4061215800865545e-19);  // pi/2 2^-62
+    float2 sc;
+    rope_sincos_reduced(x, (int)k, sc.x, sc.y);
+    if (u >> 31) sc.x = -sc.x;
+    return sc;
+}
+
+// Sine and cosine of a float32 angle.  The angle is reduced by the nearest multiple of pi/2 in double (an error below
+// 10^-9 up to 2^24), the remainder goes through the Taylor polynomials of degree 9 and 10 (next terms below 2 10^-9 and
+// 2 10^-10 there): against float64, rotated float32 rows at positions up to 10^6 are off by 4.4 10^-8 (2-norm), by
+// 4.5 10^-8 with the library's sincosf.  Some 30 instructions; sincosf carries a multi-word reduction for large angles
+// that the appends spent most of their time in (512 rows of 8 heads x 128: 22.7 us full precision and 18.8 us quantized
+// with it and an exponential per element, 10.3 and 11.4 us so).
+__device__ __forceinline__ void rope_sincos_ordinary(float theta, float &sn, float &cs) {
+    const double t = (double)theta;
+    const double k = rint(t * 0.63661977236758134308);
+    rope_sincos_reduced((float)fma(-k, 1.57079632679489661923, t), (int)(k - 4.0 * floor(k * 0.25)), sn, cs);
+}
+constexpr float ROPE_LARGE = 16777216.f;
+__device__ __forceinline__ void rope_sincos(float theta, float &sn, float &cs) {
+    rope_sincos_ordinary(theta, sn, cs);
+    if (__builtin_expect(fabsf(theta) >= ROPE_LARGE, 0)) {
+        const float2 sc = rope_sincos_large(theta);
+        sn = sc.x;
+        cs = sc.y;
+    }
+}
+// The same for V angles, with one look at the largest (512 rows of 8 heads x 128 at 4 bits, the rotated append: 11.8 us;
+// 13.3 with a branch behind each angle, 11.0 with none).
+template <int V, class ANGLE>
+__device__ __forceinline__ void rope_sincos_many(ANGLE angle, float (&sn)[V], float (&cs)[V]) {
+    float largest = 0.f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const float theta = angle(j);
+        largest = fmaxf(largest, fabsf(theta));
+        rope_sincos_ordinary(theta, sn[j], cs[j]);
+    }
+    if (__builtin_expect(largest >= ROPE_LARGE, 0)) {
+#pragma unroll 1
+        for (int i = 0; i < V; ++i) {
+            const float theta = angle(i);
+            if (fabsf(theta) < ROPE_LARGE) continue;
+            const float2 sc = rope_sincos_large(theta);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                sn[j] = j == i ? sc.x : sn[j];
+                cs[j] = j == i ? sc.y : cs[j];
+            }
+        }
+    }
 }
 
 // The inverse frequency of pair i is formed in double and rounded once, so that it does not depend on
@@ -107,16 +164,16 @@ __device__ __forceinline__ void rope_chunk_sincos(const RopeDev &r, const float 
                                                   float (&sn)[rope_chunk_elems<DT>()], float (&cs)[rope_chunk_elems<DT>()]) {
     constexpr int V = rope_chunk_elems<DT>();
     if (r.traditional) {
+        float s[V / 2], c[V / 2];
+        rope_sincos_many<V / 2>([&](int j) { return rope_angle(r, pos, inv_s[d0 / 2 + j]); }, s, c);
 #pragma unroll
-        for (int j = 0; j < V / 2; ++j) {
-            rope_sincos(rope_angle(r, pos, inv_s[d0 / 2 + j]), sn[2 * j], cs[2 * j]);
-            sn[2 * j + 1] = sn[2 * j];
-            cs[2 * j + 1] = cs[2 * j];
+        for (int j = 0; j < V; ++j) {
+            sn[j] = s[j / 2];
+            cs[j] = c[j / 2];
         }
     } else {
         const int half = r.dims >> 1, i0 = d0 < half ? d0 : d0 - half;
-#pragma unroll
-        for (int j = 0; j < V; ++j) rope_sincos(rope_angle(r, pos, inv_s[i0 + j]), sn[j], cs[j]);
+        rope_sincos_many<V>([&](int j) { return rope_angle(r, pos, inv_s[i0 + j]); }, sn, cs);
     }
 }
 // The chunk at d0 < dims of a row, rotated and rounded to the dtype; `row` is the unrotated row.

@@ -252,3 +252,18 @@ def test_one_call_in_a_staged_round_counts_the_staged_rows(dtype, D, dims):
         got = rings[0].update_attend_rope(rope, q, k, v, D ** -0.5, kvhip.MaskMode.causal())
         assert torch.equal(got, want), Lq
     assert all(torch.equal(a, b) for a, b in zip(staged[0].staged_arrays, staged[1].staged_arrays))
+
+
+@pytest.mark.parametrize("traditional", [False, True])
+@pytest.mark.parametrize("dims", [64, 56])  # (56: pairs that cut through 16-byte chunks)
+def test_angles_of_any_size(dims, traditional):
+    """Frequencies and a scale that give angles from 10^-3 to 10^38 (all finite): float32 sines and cosines of the float32 angle."""
+    rng = np.random.default_rng(8)
+    x32, xd = randn(rng, (1, 2, 9, 64), torch.float32)
+    freqs = np.logspace(0., -34., dims // 2).astype(np.float32)
+    rope = kvhip.RoPE(dims, traditional=traditional, scale=0.5, freqs=freqs)
+    for offset in (0, 3, 4000):
+        got = np32(kvhip.apply_rotary_position(rope, xd, offset))
+        want = OR.rope(x32, dims, traditional, 10000.0, 0.5, offset, freqs=freqs, dtype="float32")
+        ok, mx = within_one_ulp(got, want, torch.float32, pair_norms(x32, dims, traditional))
+        assert ok, f"offset {offset}: max diff {mx:.3e}"
