@@ -12,7 +12,11 @@
 //                 QT = 1: every wavefront for all sixteen rows (no second barrier);
 //   out^T         V^T (128 columns x 32 tokens) . P^T, the probabilities as the sum of two 16-bit operands, high part
 //                 and remainder: 22 bits of a float32 probability in float16 (scaled by 2^10, so that the remainder
-//                 stays above the subnormals), 16 in bfloat16, where the output keeps 8.
+//                 stays above the subnormals), 16 in bfloat16, where the output keeps 8.  Against float64 over 1 to
+//                 512 rows and 333 to 8191 keys the outputs are off as with float32 probabilities (2.0 to 2.2 10^-4 and
+//                 1.6 to 1.7 10^-3, equal to within 10^-5 of that).  An infinite value would meet a remainder of zero or of the
+//                 other sign: where an output comes out NaN the workgroup goes over its keys again with the
+//                 remainder's product over finite values only.
 // Two rows of query tiles at most: the accumulators of four leave one wavefront per SIMD and are copied between the two
 // register files every tile (512 rows x 2048 keys, 8 query and 2 kv heads, bfloat16: 69 us the call, against 57 us).
 // Decode is bound by HBM where the batch fills the chip (B8, 4096 keys, one token: 26.5 us, 5.1 TB/s)
@@ -22,6 +26,7 @@
 // K rows are loaded in the token order that leaves lane group g of the scores with tokens 8 g .. 8 g + 7, which is the
 // order the probabilities are read in as an operand: they never cross lanes.
 #include <algorithm>
+#include <type_traits>
 
 #include "kvhip_mask.hpp"
 
@@ -51,6 +56,13 @@ template <int DT> __device__ __forceinline__ float low_of(uint32_t w) {
 template <int DT> __device__ __forceinline__ float high_of(uint32_t w) {
     return DT == 0 ? (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)) : __uint_as_float(w & 0xffff0000u);
 }
+// the elements of an operand that are finite, zeros for the others
+template <int DT> __device__ __forceinline__ kv_u4 finite_only(kv_u4 v) {
+    constexpr uint32_t E = DT == 0 ? 0x7c00u : 0x7f80u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = ((v[i] & E) == E ? 0u : v[i] & 0xffffu) | ((v[i] & (E << 16)) == (E << 16) ? 0u : v[i] & 0xffff0000u);
+    return v;
+}
 
 // grid (row blocks of 16 QT, BH, parts), four wavefronts.  Parts divide the key tiles the row block sees.
 template <int DT, int QT>
@@ -60,6 +72,7 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
     __shared__ f4 part_s[NB][WW][QT][2][64];      // partial scores of the wavefronts
     __shared__ kv_u4 prob_s[QT == 1 ? 1 : QT][2][64];
     __shared__ float stat_s[QT][16], sum_s[QT][16], max_s[QT][16];
+    __shared__ int nan_s[WW];
     const Store &st = a.st;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, g = lane >> 4;
@@ -116,19 +129,15 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
     };
 
     f4 acc[QT][NCT];
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-        for (int c = 0; c < NCT; ++c) acc[qt][c] = f4{0.f, 0.f, 0.f, 0.f};
     const int own = QT == 1 ? 0 : wave & 1;  // the query rows whose softmax this wavefront works out
     const int my = row0 + 16 * own + col;
     const int my_hq = h * r + min(my, R - 1) / a.L, my_l = min(my, R - 1) % a.L;
-    float m_run = -INFINITY, l_run = 0.f;
+    float m_run, l_run;
     constexpr float P_UP = DT == 0 ? 10.f : 0.f;  // (float16 probabilities are carried times 2^10)
 
     // the probabilities of row `my` for tokens 8 g .. 8 g + 7 of tile t, high parts and remainders, and the factor its
     // sums so far take
-    auto softmax = [&](int t, int buf, kv_u4 &ph, kv_u4 &pl, float &alpha) __attribute__((always_inline)) {
+    auto softmax = [&](auto careful, int t, int buf, kv_u4 &ph, kv_u4 &pl, float &alpha) __attribute__((always_inline)) {
         f4 sum[2];
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
@@ -172,71 +181,99 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             hi[j] = pack2<DT>(p[2 * j], p[2 * j + 1]);
+            if constexpr (DT == 0 && decltype(careful)::value) {  // no weight rounds to nothing (the remainder takes it off again)
+                if (p[2 * j] > 0.f && (hi[j] & 0xffffu) == 0u) hi[j] |= 1u;
+                if (p[2 * j + 1] > 0.f && (hi[j] >> 16) == 0u) hi[j] |= 0x10000u;
+            }
             lo[j] = pack2<DT>(p[2 * j] - low_of<DT>(hi[j]), p[2 * j + 1] - high_of<DT>(hi[j]));
         }
         ph = kv_u4{hi[0], hi[1], hi[2], hi[3]};
         pl = kv_u4{lo[0], lo[1], lo[2], lo[3]};
     };
 
-    if (tb < te) {  // workgroup-uniform
-        load_k(tb);
-        load_v(tb);
-    }
-    for (int t = tb; t < te; ++t) {
-        f4 sacc[QT][2];
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) sacc[qt][0] = sacc[qt][1] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-                for (int x = 0; x < 2; ++x) sacc[qt][x] = mfma<DT>(kreg[s][x], qop[qt][s], sacc[qt][x]);
-        load_k(min(t + 1, te - 1));
-        const int buf = NB == 1 ? 0 : (t & 1);
+    // All the keys; true if an output came out NaN (`careful`: infinite values are about).
+    auto walk = [&](auto careful) __attribute__((always_inline)) {
+        m_run = -INFINITY;
+        l_run = 0.f;
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-            for (int x = 0; x < 2; ++x) part_s[buf][wave][qt][x][lane] = sacc[qt][x];
-        __syncthreads();
-        kv_u4 ph, pl;
-        float alpha = 1.f;
-        if (QT == 1 || wave < QT) softmax(t, buf, ph, pl, alpha);  // wave-uniform
-        if constexpr (QT > 1) {
-            if (wave < QT) {
-                prob_s[own][0][lane] = ph;
-                prob_s[own][1][lane] = pl;
-                if (g == 0) stat_s[own][col] = alpha;
-            }
+            for (int c = 0; c < NCT; ++c) acc[qt][c] = f4{0.f, 0.f, 0.f, 0.f};
+        if (tb < te) {  // workgroup-uniform
+            load_k(tb);
+            load_v(tb);
+        }
+        for (int t = tb; t < te; ++t) {
+            f4 sacc[QT][2];
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) sacc[qt][0] = sacc[qt][1] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                    for (int x = 0; x < 2; ++x) sacc[qt][x] = mfma<DT>(kreg[s][x], qop[qt][s], sacc[qt][x]);
+            load_k(min(t + 1, te - 1));
+            const int buf = NB == 1 ? 0 : (t & 1);
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) part_s[buf][wave][qt][x][lane] = sacc[qt][x];
             __syncthreads();
-        }
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            const float al = QT == 1 ? alpha : stat_s[qt][col];
-            if (__any(al != 1.f)) {  // (a raised maximum: rare after the first tiles)
-#pragma unroll
-                for (int c = 0; c < NCT; ++c) acc[qt][c] *= al;
-            }
+            kv_u4 ph, pl;
+            float alpha = 1.f;
+            if (QT == 1 || wave < QT) softmax(careful, t, buf, ph, pl, alpha);  // wave-uniform
             if constexpr (QT > 1) {
-                ph = prob_s[qt][0][lane];
-                pl = prob_s[qt][1][lane];
+                if (wave < QT) {
+                    prob_s[own][0][lane] = ph;
+                    prob_s[own][1][lane] = pl;
+                    if (g == 0) stat_s[own][col] = alpha;
+                }
+                __syncthreads();
             }
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(vreg[c], ph, acc[qt][c]);
+            for (int qt = 0; qt < QT; ++qt) {
+                const float al = QT == 1 ? alpha : stat_s[qt][col];
+                if (__any(al != 1.f)) {  // (a raised maximum: rare after the first tiles)
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(vreg[c], pl, acc[qt][c]);
+                    for (int c = 0; c < NCT; ++c) acc[qt][c] *= al;
+                }
+                if constexpr (QT > 1) {
+                    ph = prob_s[qt][0][lane];
+                    pl = prob_s[qt][1][lane];
+                }
+#pragma unroll
+                for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(vreg[c], ph, acc[qt][c]);
+#pragma unroll
+                for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(decltype(careful)::value ? finite_only<DT>(vreg[c]) : vreg[c], pl, acc[qt][c]);
+            }
+            load_v(min(t + 1, te - 1));
         }
-        load_v(min(t + 1, te - 1));
+
+        // ---- the rows' maxima and sums to every wavefront ----------------------------------------------
+        l_run += __shfl_xor(l_run, 16);
+        l_run += __shfl_xor(l_run, 32);
+        bool nan = false;
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+            for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) nan = nan || acc[qt][c][i] != acc[qt][c][i];
+        nan = __any(nan);
+        if (lane == 0) nan_s[wave] = nan;
+        if (g == 0 && wave < QT) {
+            max_s[own][col] = m_run;
+            sum_s[own][col] = l_run;
+        }
+        __syncthreads();
+        return (nan_s[0] | nan_s[1] | nan_s[2] | nan_s[3]) != 0;  // workgroup-uniform
+    };
+    if (walk(std::false_type())) {
+        __syncthreads();
+        walk(std::true_type());
     }
 
-    // ---- the rows' maxima and sums to every wavefront, then the output ------------------------------
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
-    if (g == 0 && wave < QT) {
-        max_s[own][col] = m_run;
-        sum_s[own][col] = l_run;
-    }
-    __syncthreads();
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const int rr = row0 + 16 * qt + col;

@@ -1,0 +1,51 @@
+"""Infinite elements in the float32 and head-size-512 attention kernels (family 5): an infinite value reaches its output
+column with its sign.  The other columns against float64 at the dtype's own rounding."""
+import pytest
+import torch
+
+import kvhip
+
+pytestmark = pytest.mark.gpu
+
+INF, NAN = float("inf"), float("nan")
+KINDS = [(torch.float16, 512), (torch.bfloat16, 512), (torch.float32, 64), (torch.float32, 128), (torch.float32, 256)]
+# one rounding of the output, of values up to about 5 (float32: sums of D products and T probabilities)
+TOL = {torch.float16: 2.0 ** -8, torch.bfloat16: 2.0 ** -5, torch.float32: 1e-5}
+
+
+def tensors(dtype, D, T, n, seed=1):
+    gen = torch.Generator(device="cuda").manual_seed(seed + T + n + D)
+    return [torch.randn(2, h, m, D, generator=gen, device="cuda").to(dtype) for h, m in ((8, n), (2, T), (2, T))]
+
+
+def attend(q, k, v, mask, ring=False):
+    c = kvhip.RotatingKVCache(k.shape[2], keep=4) if ring else kvhip.KVCacheSimple()
+    c.update(k, v, fetch=False)
+    out = c.attend(q, q.shape[3] ** -0.5, mask)
+    assert kvhip.load().kvhip_last_attend_kernel() == 5
+    return out.double()
+
+
+def exact(q, k, v, keep, add=None):
+    """float64, infinite values left out (`keep`: keys that weigh something)."""
+    k, v = (torch.nan_to_num(x.double(), 0., 0., 0.).repeat_interleave(4, 1) for x in (k, v))
+    s = torch.matmul(torch.nan_to_num(q.double()), k.transpose(2, 3).contiguous()) * q.shape[3] ** -0.5
+    s = s if add is None else s + add.double()
+    p = torch.softmax(s.masked_fill(~keep, -INF), -1)
+    return torch.matmul(torch.nan_to_num(p), v)
+
+
+@pytest.mark.parametrize("dtype,D", KINDS)
+@pytest.mark.parametrize("T,n", [(40, 1), (40, 9), (3000, 1), (3000, 9)])
+def test_infinite_values_reach_the_output(dtype, D, T, n):
+    q, k, v = tensors(dtype, D, T, n)
+    add = torch.zeros(1, T, device="cuda")
+    add[0, 9] = -60.  # weights down to 2^-100: nothing beside the others, but not zero
+    v[:, :, 7, 3], v[:, :, 7, 6], v[:, :, 9, 5], v[:, :, 9, D - 1] = INF, -INF, INF, -INF
+    out = attend(q, k, v, kvhip.MaskMode.from_array(add.expand(n, T)))
+    for col, want in ((3, INF), (6, -INF), (5, INF), (D - 1, -INF)):
+        assert (out[..., col] == want).all(), col
+        out[..., col] = 0.
+    ref = exact(q, k, v, torch.ones(1, T, dtype=torch.bool, device="cuda"), add)
+    ref[..., [3, 5, 6, D - 1]] = 0.
+    assert (out - ref).abs().max() <= TOL[dtype]
