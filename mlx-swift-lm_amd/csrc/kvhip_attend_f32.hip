@@ -168,7 +168,10 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
 #pragma unroll
             for (int x = 0; x < TB; ++x)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[qt][x][j]);
+                for (int j = 0; j < 4; ++j) {
+                    s[qt][x][j] = fmaxf(s[qt][x][j], -INFINITY);  // (a score that is NaN weighs nothing)
+                    mx = fmaxf(mx, s[qt][x][j]);
+                }
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             // (the reference is raised only by more than 3, so that the accumulators are rarely touched after the first tiles)

@@ -159,9 +159,12 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
                 sc[j] = keep ? sc[j] + add : -INFINITY;
             }
         }
-        float mx = sc[0];
+        float mx = -INFINITY;
 #pragma unroll
-        for (int j = 1; j < 8; ++j) mx = fmaxf(mx, sc[j]);
+        for (int j = 0; j < 8; ++j) {
+            sc[j] = fmaxf(sc[j], -INFINITY);  // (a score that is NaN weighs nothing)
+            mx = fmaxf(mx, sc[j]);
+        }
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         // The reference of the exponentials is raised only when a score exceeds it by more than 2^5, so that the

@@ -1,5 +1,6 @@
-"""Infinite elements in the float32 and head-size-512 attention kernels (family 5): an infinite value reaches its output
-column with its sign.  The other columns against float64 at the dtype's own rounding."""
+"""Infinite and NaN elements in the float32 and head-size-512 attention kernels (family 5): an infinite value reaches its
+output column with its sign, a key whose score is NaN weighs nothing.  The other columns against float64 at the dtype's
+own rounding."""
 import pytest
 import torch
 
@@ -49,3 +50,19 @@ def test_infinite_values_reach_the_output(dtype, D, T, n):
     ref = exact(q, k, v, torch.ones(1, T, dtype=torch.bool, device="cuda"), add)
     ref[..., [3, 5, 6, D - 1]] = 0.
     assert (out - ref).abs().max() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,D", KINDS)
+@pytest.mark.parametrize("T,n", [(40, 1), (40, 9), (3000, 1), (3000, 9)])
+def test_keys_whose_score_is_nan_weigh_nothing(dtype, D, T, n):
+    q, k, v = tensors(dtype, D, T, n)
+    k[0, :, 7, 3] = NAN
+    k[0, 1, T - 2, D - 1] = NAN
+    q[1, 5, 0, 2] = NAN  # every score of one row: zeros, as where every key is excluded
+    out = attend(q, k, v, kvhip.MaskMode.none())
+    keep = torch.ones(2, 8, n, T, dtype=torch.bool, device="cuda")
+    keep[0, :, :, 7] = False
+    keep[0, 4:, :, T - 2] = False
+    keep[1, 5, 0] = False
+    assert (out - exact(q, k, v, keep)).abs().max() <= TOL[dtype]
+    assert (out[1, 5, 0] == 0).all()
