@@ -31,7 +31,13 @@ constexpr int token_blocks(int dk, int qt) { return dk <= 64 ? 4 / qt : dk <= 12
 constexpr int query_tiles(int dk) { return dk <= 128 ? 2 : 1; }
 
 // grid (row blocks of 16 QT, BH, parts).  Parts divide the key tiles the row block sees.
-template <int DK, int DV, int QT>
+// ARR 1 / 2: boolean and additive array masks.  Their elements are requested before the next tile's keys, whose arrival
+// they would otherwise wait for, and a wavefront steps over tiles that none of its rows sees under a boolean one, as
+// those of the vector-ALU kernel do.
+// One token, B8, 32q/8kv, D 128, 8192 keys: all seen under a boolean mask 107 us, a window of 512 31, an additive mask
+// 104; 119, 120 and 112 with the elements fetched one by one behind the keys and every tile read, 105, 43 and 100 on
+// the vector-ALU kernel; 256 rows of B4 over 4096 keys, the boolean window: 236, 893, 476.
+template <int DK, int DV, int QT, int ARR>
 __global__ void __launch_bounds__(256, 2)
 attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
     constexpr int TB = token_blocks(DK, QT), WT = 16 * TB;
@@ -112,12 +118,89 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
 #pragma unroll
         for (int c = 0; c < NCT; ++c) acc[qt][c] = f4{0.f, 0.f, 0.f, 0.f};
     }
-    if (first < te) {  // wave-uniform
-        load_k(first);
-        load_v(first);
+    // (ARR) the raw mask elements of a tile, and (1) which of the lane's keys its rows see, bit (qt TB + x) 4 + j
+    constexpr bool bools = ARR == 1;
+    uint32_t raw[QT][TB][bools ? 1 : 4];
+    auto mask_fetch = [&](int t) __attribute__((always_inline)) {
+        const int row = run_row(a.runs, t * WT, WT);
+        if (row < 0) return;
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+            for (int x = 0; x < TB; ++x) {
+                if constexpr (bools) mask_bool_words<1>(a.mask, b, my_hq[qt], my_l[qt], row + 16 * x + 4 * g, raw[qt][x]);
+                else if constexpr (ARR == 2) mask_add_words<4>(a.mask, b, my_hq[qt], my_l[qt], row + 16 * x + 4 * g, raw[qt][x]);
+            }
+    };
+    auto mask_bits = [&](int t) __attribute__((always_inline)) -> uint32_t {
+        const bool whole = run_row(a.runs, t * WT, WT) >= 0;
+        uint32_t bits = 0;
+#pragma unroll
+        for (int x = 0; x < TB; ++x)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int slot = t * WT + 16 * x + 4 * g + j;
+                const int row = whole ? 0 : slot < a.slots ? slot_to_row(a.runs, slot) : -1;
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    float add;
+                    const bool keep = whole ? ((raw[qt][x][0] >> (8 * j)) & 0xffu) != 0u
+                                            : row >= 0 && row < a.T && mask_keep(a.mask, b, my_hq[qt], my_l[qt], row, a.L, a.T, add);
+                    bits |= keep ? 1u << ((qt * TB + x) * 4 + j) : 0u;
+                }
+            }
+        return bits;
+    };
+    // the first of this wavefront's tiles from t on (its elements are there) that a row sees
+    auto seen_from = [&](int t, uint32_t &bits) __attribute__((always_inline)) -> int {
+        bits = t < te ? mask_bits(t) : 0u;
+        while (t < te && !__any(bits != 0u)) {
+            t += MW;
+            // (unseen tiles come in rows: as many as sixteen words hold are asked for at once)
+            constexpr int U = 16 / (QT * TB);
+            uint32_t w[U][QT][TB][1];
+            bool known[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int c = t + u * MW, row = c < te ? run_row(a.runs, c * WT, WT) : -1;
+                known[u] = row >= 0;
+                if (row < 0) continue;
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                    for (int x = 0; x < TB; ++x) mask_bool_words<1>(a.mask, b, my_hq[qt], my_l[qt], row + 16 * x + 4 * g, w[u][qt][x]);
+            }
+            int unseen = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                uint32_t any = 0;
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                    for (int x = 0; x < TB; ++x) any |= known[u] ? w[u][qt][x][0] : 0u;
+                if (unseen == u && known[u] && !__any(any != 0u)) unseen = u + 1;
+            }
+            t += unseen * MW;
+            if (t < te) {
+                mask_fetch(t);
+                bits = mask_bits(t);
+            }
+        }
+        return t;
+    };
+    int t = first;
+    uint32_t bits = 0, next_bits = 0;
+    if constexpr (bools) {
+        if (t < te) mask_fetch(t);
+        t = seen_from(t, bits);
     }
-    for (int t = first; t < te; t += MW) {
-        const int next = t + MW < te ? t + MW : t;
+    if (t < te) {  // wave-uniform
+        load_k(t);
+        if (ARR && t + (bools ? MW : 0) < te) mask_fetch(t + (bools ? MW : 0));
+        load_v(t);
+    }
+    while (t < te) {
+        int next = t + MW;
         f4 s[QT][TB];
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt)
@@ -145,14 +228,31 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
                     for (int qt = 0; qt < QT; ++qt) s[qt][x] = mfma4(kreg[x][e][j], q[qt][j], s[qt][x]);
             if constexpr (QL) __builtin_amdgcn_sched_barrier(0);  // (one step's queries ahead, not all of them: registers)
         }
-        load_k(next);
+        if constexpr (bools) next = seen_from(next, next_bits);
+        load_k(next < te ? next : t);
         const int slot0 = t * WT;
+        const bool whole = ARR == 2 && run_row(a.runs, slot0, WT) >= 0;  // wave-uniform
         const bool full = ident && slot0 >= keys.full_lo && slot0 + WT - 1 <= keys.full_hi;  // wave-uniform
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
 #pragma unroll
             for (int x = 0; x < TB; ++x) s[qt][x] *= a.scale;
-            if (!full) {
+            if constexpr (bools) {
+#pragma unroll
+                for (int x = 0; x < TB; ++x)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) s[qt][x][j] = (bits >> ((qt * TB + x) * 4 + j)) & 1u ? s[qt][x][j] : -INFINITY;
+            } else if (whole) {
+#pragma unroll
+                for (int x = 0; x < TB; ++x) {
+                    if constexpr (ARR == 2) {
+                        float add[4];
+                        mask_add_floats<4>(a.mask, raw[qt][x], add);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) s[qt][x][j] += add[j];
+                    }
+                }
+            } else if (!full) {
 #pragma unroll
                 for (int x = 0; x < TB; ++x)
 #pragma unroll
@@ -202,7 +302,10 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
                 for (int c = 0; c < NCT; ++c)
 #pragma unroll
                     for (int qt = 0; qt < QT; ++qt) acc[qt][c] = mfma4(vreg[x][c][j], s[qt][x][j], acc[qt][c]);
-        load_v(next);
+        if (ARR && next + (bools ? MW : 0) < te) mask_fetch(next + (bools ? MW : 0));
+        load_v(next < te ? next : t);
+        t = next;
+        bits = next_bits;
     }
 
     // ---- the four wavefronts' states: each scales its own to the common maximum, then adds up a quarter of the columns ----
@@ -278,8 +381,11 @@ PlanF32 plan_f32(const AttendArgs &a) {
 
 template <int DK, int DV, int QT>
 hipError_t launch_instance(const AttendArgs &a, const PlanF32 &p, hipStream_t s) {
-    hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT>), dim3(p.row_blocks, a.st.BH, p.nparts), dim3(256), MW * QT * (DV / 16) * 64 * sizeof(f4), s,
-                       a, p.tiles, p.nparts);
+    const dim3 grid(p.row_blocks, a.st.BH, p.nparts), block(256);
+    const size_t lds = MW * QT * (DV / 16) * 64 * sizeof(f4);
+    if (a.mask.mode != KVHIP_MASK_ARRAY) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, 0>), grid, block, lds, s, a, p.tiles, p.nparts);
+    else if (a.mask.dtype == KVHIP_BOOL) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, 1>), grid, block, lds, s, a, p.tiles, p.nparts);
+    else hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, 2>), grid, block, lds, s, a, p.tiles, p.nparts);
     return hipGetLastError();
 }
 

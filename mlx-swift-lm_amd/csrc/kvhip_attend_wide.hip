@@ -64,8 +64,16 @@ template <int DT> __device__ __forceinline__ kv_u4 finite_only(kv_u4 v) {
     return v;
 }
 
+constexpr int SEEN = 4096;     // tiles of a part that a boolean mask is looked through for (131072 keys; beyond: taken as seen)
+
 // grid (row blocks of 16 QT, BH, parts), four wavefronts.  Parts divide the key tiles the row block sees.
-template <int DT, int QT>
+// ARR 1 / 2: boolean and additive array masks.  A row's elements are requested before the next tile's keys, whose arrival
+// they would otherwise wait for; under a boolean mask the workgroup first looks which of its tiles any row sees and
+// steps over the others, as the vector-ALU kernel does.  (All four wavefronts go by one table in LDS: they meet in the
+// loop's barriers.)  One token, B8, 16q/8kv, 8192 keys: all seen under a boolean mask 212 us, a window of 512 47, an
+// additive mask 193; 275, 276 and 262 with the elements fetched one by one behind the keys and every tile read, 198, 66
+// and 193 on the vector-ALU kernel.
+template <int DT, int QT, int ARR>
 __global__ void __launch_bounds__(256, 2)
 attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
     constexpr int NB = QT == 1 ? 2 : 1;           // score buffers (QT = 1 has one barrier per tile)
@@ -73,6 +81,7 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
     __shared__ kv_u4 prob_s[QT == 1 ? 1 : QT][2][64];
     __shared__ float stat_s[QT][16], sum_s[QT][16], max_s[QT][16];
     __shared__ int nan_s[WW];
+    __shared__ uint8_t seen_s[ARR == 1 ? SEEN : 1];
     const Store &st = a.st;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, g = lane >> 4;
@@ -135,6 +144,62 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
     float m_run, l_run;
     constexpr float P_UP = DT == 0 ? 10.f : 0.f;  // (float16 probabilities are carried times 2^10)
 
+    // (1) the first tile from t on that a row sees
+    if constexpr (ARR == 1) {
+        constexpr int U = 4;  // tiles a wavefront asks for together
+        const int n = min(te - tb, SEEN);
+        for (int i0 = wave; i0 < n; i0 += U * WW) {
+            uint32_t w[U][QT][2];
+            bool seen[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int slot0 = (tb + min(i0 + u * WW, n - 1)) * WT, row = run_row(a.runs, slot0, WT);
+                seen[u] = false;
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    const int rr = min(row0 + 16 * qt + col, R - 1), hq = h * r + rr / a.L, l = rr % a.L;
+                    w[u][qt][0] = w[u][qt][1] = 0u;
+                    if (row >= 0) {
+                        mask_bool_words<2>(a.mask, b, hq, l, row + 8 * g, w[u][qt]);
+                    } else {
+                        for (int j = 0; j < 8; ++j) {
+                            const int slot = slot0 + 8 * g + j, key = slot < a.slots ? slot_to_row(a.runs, slot) : -1;
+                            float add;
+                            seen[u] = seen[u] || (key >= 0 && key < a.T && mask_keep(a.mask, b, hq, l, key, a.L, a.T, add));
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) seen[u] = seen[u] || (w[u][qt][0] | w[u][qt][1]) != 0u;
+                const bool any = __any(seen[u]);
+                if (lane == 0 && i0 + u * WW < n) seen_s[i0 + u * WW] = any;
+            }
+        }
+        __syncthreads();
+    }
+    auto seen_from = [&](int t) __attribute__((always_inline)) -> int {
+        if constexpr (ARR == 1) {
+            while (t < te && t - tb < SEEN) {
+                const int i = t - tb + lane;
+                const unsigned long long m = __ballot(t + lane < te && (i >= SEEN || seen_s[min(i, SEEN - 1)] != 0));
+                if (m != 0ull) return t + __ffsll(m) - 1;
+                t += 64;
+            }
+            return min(t, te);
+        }
+        return t;
+    };
+    uint32_t raw[ARR == 1 ? 2 : 8];  // (ARR) the mask elements of row `my` for tokens 8 g .. 8 g + 7 of a tile
+    auto mask_fetch = [&](int t) __attribute__((always_inline)) {
+        const int row = run_row(a.runs, t * WT, WT);
+        if (row < 0 || (QT > 1 && wave >= QT)) return;
+        if constexpr (ARR == 1) mask_bool_words<2>(a.mask, b, my_hq, my_l, row + 8 * g, raw);
+        if constexpr (ARR == 2) mask_add_words<8>(a.mask, b, my_hq, my_l, row + 8 * g, raw);
+    };
+
     // the probabilities of row `my` for tokens 8 g .. 8 g + 7 of tile t, high parts and remainders, and the factor its
     // sums so far take
     auto softmax = [&](auto careful, int t, int buf, kv_u4 &ph, kv_u4 &pl, float &alpha) __attribute__((always_inline)) {
@@ -149,7 +214,17 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) sc[j] = sum[j >> 2][j & 3] * a.scale;
         const int slot0 = t * WT;
-        if (!ident || slot0 < keys.full_lo || slot0 + WT - 1 > keys.full_hi) {  // workgroup-uniform
+        if (ARR != 0 && run_row(a.runs, slot0, WT) >= 0) {  // workgroup-uniform
+            if constexpr (ARR == 1) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) sc[j] = ((raw[j >> 2] >> (8 * (j & 3))) & 0xffu) != 0u ? sc[j] : -INFINITY;
+            } else if constexpr (ARR == 2) {
+                float add[8];
+                mask_add_floats<8>(a.mask, raw, add);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) sc[j] += add[j];
+            }
+        } else if (!ident || slot0 < keys.full_lo || slot0 + WT - 1 > keys.full_hi) {  // workgroup-uniform
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int slot = slot0 + 8 * g + j;
@@ -202,11 +277,14 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
         for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
             for (int c = 0; c < NCT; ++c) acc[qt][c] = f4{0.f, 0.f, 0.f, 0.f};
-        if (tb < te) {  // workgroup-uniform
-            load_k(tb);
-            load_v(tb);
+        int t = seen_from(tb), buf = 0;
+        if (t < te) {  // workgroup-uniform
+            load_k(t);
+            load_v(t);
         }
-        for (int t = tb; t < te; ++t) {
+        while (t < te) {
+            const int next = seen_from(t + 1), load = next < te ? next : t;
+            if constexpr (ARR != 0) mask_fetch(t);
             f4 sacc[QT][2];
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) sacc[qt][0] = sacc[qt][1] = f4{0.f, 0.f, 0.f, 0.f};
@@ -216,8 +294,7 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
                 for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
                     for (int x = 0; x < 2; ++x) sacc[qt][x] = mfma<DT>(kreg[s][x], qop[qt][s], sacc[qt][x]);
-            load_k(min(t + 1, te - 1));
-            const int buf = NB == 1 ? 0 : (t & 1);
+            load_k(load);
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
@@ -250,7 +327,9 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
 #pragma unroll
                 for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(decltype(careful)::value ? finite_only<DT>(vreg[c]) : vreg[c], pl, acc[qt][c]);
             }
-            load_v(min(t + 1, te - 1));
+            load_v(load);
+            t = next;
+            buf ^= NB - 1;
         }
 
         // ---- the rows' maxima and sums to every wavefront ----------------------------------------------
@@ -345,7 +424,14 @@ hipError_t launch_attend_wide(const AttendArgs &a, hipStream_t s) {
     const PlanWide p = plan_wide(a);
     const dim3 grid(p.row_blocks, a.st.BH, p.nparts), block(256);
     profile_mark(s, true);
-#define WIDE(DT, QT) hipLaunchKernelGGL((attend_wide_kernel<DT, QT>), grid, block, 0, s, a, p.tiles, p.nparts)
+    const int arr = a.mask.mode != KVHIP_MASK_ARRAY ? 0 : a.mask.dtype == KVHIP_BOOL ? 1 : 2;
+#define WIDE_A(DT, QT, ARR) hipLaunchKernelGGL((attend_wide_kernel<DT, QT, ARR>), grid, block, 0, s, a, p.tiles, p.nparts)
+#define WIDE(DT, QT)                       \
+    do {                                   \
+        if (arr == 0) WIDE_A(DT, QT, 0);   \
+        else if (arr == 1) WIDE_A(DT, QT, 1); \
+        else WIDE_A(DT, QT, 2);            \
+    } while (0)
     if (a.st.dtype == KVHIP_F16) {
         if (p.qt == 1) WIDE(0, 1);
         else WIDE(0, 2);
@@ -354,6 +440,7 @@ hipError_t launch_attend_wide(const AttendArgs &a, hipStream_t s) {
         else WIDE(1, 2);
     }
 #undef WIDE
+#undef WIDE_A
     profile_mark(s, false);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.nparts == 1) return e;

@@ -47,6 +47,44 @@ __device__ __forceinline__ void mask_bool_words(const MaskDev &m, int b, int hq,
     for (int i = 0; i < W; ++i) w[i] = raw.v[i];
 }
 
+// The presented row of `slot0` when the slots slot0 .. slot0 + n - 1 lie in one run (wave-uniform); -1 otherwise.
+__device__ __forceinline__ int run_row(const Runs &r, int slot0, int n) {
+    int row = -1;
+#pragma unroll
+    for (int i = 0; i < MAXRUNS; ++i)
+        if (i < r.n && slot0 >= r.phys0[i] && slot0 + n <= r.phys0[i] + r.len[i]) row = r.row0[i] + slot0 - r.phys0[i];
+    return row;
+}
+// Elements row .. row + N - 1 (all presented) of an additive array mask for query row l of (b, hq), as they lie in memory
+// (a wide load, which can be requested well before the scores that the elements belong to), and as floats.
+template <int N> __device__ __forceinline__ void mask_add_words(const MaskDev &m, int b, int hq, int l, int row, uint32_t (&w)[N]) {
+    struct __attribute__((packed, aligned(1))) Raw32 {
+        uint32_t v[N];
+    };
+    struct __attribute__((packed, aligned(1))) Raw16 {
+        uint32_t v[N / 2];
+    };
+    const size_t i = (size_t)(b * m.sb + hq * m.sh + l * m.sl) + row;
+    if (m.dtype == KVHIP_F32) {
+        const Raw32 x = *reinterpret_cast<const Raw32 *>(reinterpret_cast<const char *>(m.data) + 4 * i);
+#pragma unroll
+        for (int k = 0; k < N; ++k) w[k] = x.v[k];
+    } else {
+        const Raw16 x = *reinterpret_cast<const Raw16 *>(reinterpret_cast<const char *>(m.data) + 2 * i);
+#pragma unroll
+        for (int k = 0; k < N; ++k) w[k] = k < N / 2 ? x.v[k % (N / 2)] : 0u;
+    }
+}
+template <int N> __device__ __forceinline__ void mask_add_floats(const MaskDev &m, const uint32_t (&w)[N], float (&add)[N]) {
+    const bool f32 = m.dtype == KVHIP_F32, bf16 = m.dtype == KVHIP_BF16;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const uint32_t whole = w[j], half = w[j >> 1] >> (16 * (j & 1));
+        const float narrow = bf16 ? __uint_as_float(half << 16) : __half2float(__ushort_as_half((unsigned short)half));
+        add[j] = f32 ? __uint_as_float(whole) : narrow;
+    }
+}
+
 // Index-only masks (causal, window with optional per-batch bounds) with the per-batch
 // bounds already in registers: no memory access, so kernels can keep loads in flight.
 struct SymMask {

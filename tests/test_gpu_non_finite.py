@@ -1,6 +1,6 @@
 """Infinite and NaN elements in the float32 and head-size-512 attention kernels (family 5): an infinite value reaches its
-output column with its sign, a key whose score is NaN weighs nothing.  The other columns against float64 at the dtype's
-own rounding."""
+output column with its sign, a key whose score is NaN weighs nothing, and tiles that no row sees under a boolean array
+mask are not read.  The other columns against float64 at the dtype's own rounding."""
 import pytest
 import torch
 
@@ -66,3 +66,17 @@ def test_keys_whose_score_is_nan_weigh_nothing(dtype, D, T, n):
     keep[1, 5, 0] = False
     assert (out - exact(q, k, v, keep)).abs().max() <= TOL[dtype]
     assert (out[1, 5, 0] == 0).all()
+
+
+@pytest.mark.parametrize("dtype,D", KINDS)
+@pytest.mark.parametrize("T,n,seen", [(300, 1, 70), (3000, 1, 6), (3000, 9, 200), (700, 70, 64), (5000, 1, 4000)])
+@pytest.mark.parametrize("ring", [False, True])
+def test_tiles_nobody_sees_are_not_read(dtype, D, T, n, seen, ring):
+    """A boolean window over the last keys: values in front of the first tile with a visible key do not matter."""
+    q, k, v = tensors(dtype, D, T, n)
+    i, j = torch.arange(n, device="cuda")[:, None] + T - n, torch.arange(T, device="cuda")[None]
+    keep = (j <= i) & (j > i - seen)
+    hidden = (T - n - seen + 1) // 64 * 64  # whole tiles of 64 in front of every row's window
+    v[:, :, :hidden] = NAN
+    out = attend(q, k, v, kvhip.MaskMode.from_array(keep), ring)
+    assert (out - exact(q, k, v, keep)).abs().max() <= TOL[dtype]
