@@ -404,6 +404,20 @@ bool attend_f32_supported(const AttendArgs &a) {
     // loads are the better ones (B8, 8 kv heads, 8192 keys, one token: 185 us against 201; B4, 4 kv heads, 4096 keys: 36.2
     // against 37.0; but one sequence, 8 kv heads, 8192 keys: 40.6 against 31).
     if (s.Dk == 256 && s.BH >= 16 && (size_t)s.BH * a.T >= 65536 && (a.Hq / a.Hkv) * a.L <= 8) return false;
+    // So are one to four rows over many pairs of the smaller sizes, without a mask that leaves tiles out, in the ranges
+    // where they measured 3 to 25 % ahead (vector ALUs / here; outside them this kernel is equal or ahead).  One row: 67 MB
+    // of 128 pairs D 64 21.9 / 24.5 us, D 96 101 MB 25.7 / 28.4, D 128 134 MB 30.8 / 35.2 and 1074 MB 176 / 198, 256 pairs of
+    // 256 keys 20.1 / 26.2, but D 64 537 MB 112 / 101, 16 pairs 34 MB 16.5 / 15.3.  Four rows: D 128 134 MB 32.0 / 35.8, 1074 MB
+    // 182 / 199, but 32 pairs 537 MB 106 / 101, D 96 201 MB 42.0 / 42.0.
+    const int R = (a.Hq / a.Hkv) * a.L;
+    const size_t mb = (size_t)s.BH * a.T * (s.Dk + s.Dv) * 4 >> 20;
+    if (s.Dk == s.Dv && a.mask.mode <= KVHIP_MASK_CAUSAL) {
+        const bool many = s.BH >= 256;
+        if (R == 1 && s.Dk <= 128 && s.BH >= 16 && mb >= (many ? 32 : 64) && (s.Dk == 128 || mb < 256)) return false;
+        if (R <= 4 && s.Dk == 64 && s.BH >= 32 && mb >= (many ? 32 : 64) && mb < 256) return false;
+        if (R <= 4 && s.Dk == 128 && s.BH >= 32 && mb >= (many ? 64 : 128) && (s.BH >= 64 || mb < 256)) return false;
+        if (R == 1 && s.Dk == 256 && s.BH >= 128 && mb >= 64) return false;
+    }
     return (s.Dk == 192 && s.Dv == 128) || (s.Dk == s.Dv && (s.Dk == 64 || s.Dk == 96 || s.Dk == 128 || s.Dk == 256));
 }
 

@@ -224,3 +224,19 @@ def test_edges_of_the_matrix_core_tiles(Dk, Dv, T, n):
         s = torch.matmul(q.double(), kk.transpose(-1, -2).contiguous()) * Dk ** -0.5
         p = torch.nan_to_num(torch.softmax(s.masked_fill(hidden, float("-inf")), -1))  # (a row without keys gives zeros)
         close(out, torch.matmul(p, vv).cpu().numpy(), f"{mask.mode}")
+
+
+@pytest.mark.parametrize("D,pairs,r,T", [(64, 128, 1, 1050), (64, 128, 4, 1050), (96, 64, 1, 1400), (128, 256, 1, 300), (128, 256, 4, 300), (256, 128, 1, 300)])
+def test_few_rows_over_many_pairs(D, pairs, r, T):
+    """Single tokens that the vector ALUs take back from the matrix-core kernel, which takes the masked call beside each."""
+    gen = torch.Generator(device="cuda").manual_seed(D + pairs)
+    q, k, v = (torch.randn(2, h, m, D, generator=gen, device="cuda") for h, m in ((pairs // 2 * r, 1), (pairs // 2, T), (pairs // 2, T)))
+    c = kvhip.KVCacheSimple()
+    c.update(k, v, fetch=False)
+    kk, vv = (x.double().repeat_interleave(r, 1) for x in (k, v))
+    s = torch.matmul(q.double(), kk.transpose(-1, -2).contiguous()) * D ** -0.5
+    hidden = torch.arange(T, device="cuda") < T // 2
+    for mask, s_ in ((kvhip.MaskMode.none(), s), (kvhip.MaskMode.window_mask(T - 1, T - T // 2), s.masked_fill(hidden, float("-inf")))):
+        out = c.attend(q, D ** -0.5, mask)
+        assert family() == 5
+        close(out, torch.matmul(torch.softmax(s_, -1), vv).cpu().numpy(), f"{mask.mode}")
