@@ -881,18 +881,29 @@ hipError_t launch_append_quant_rows(const Store &st, const void *keys, const voi
 }
 }  // namespace
 
-// rows from which the whole-tile quantizer is the faster one
-constexpr int QUANT_TILE_ROWS = 9;
+// Rows in one tile from which the tile quantizer is the faster one.  The row kernel's wavefronts take their rows one
+// after the other, 64 columns at a time (128 with groups of 128); a tile takes its time whatever its rows.  Row kernel at
+// the count just below / tile kernel there, 4 bits: D 128 11 / 12.5 us with the rotation, 7 / 7.2 without; D 256 groups
+// of 64 19 / 23 and 12.5 / 12.3, groups of 128 20 / 22.5 and 12.4 / 12.5; keys of 192 with values of 128 15 / 18 and 11 / 12.
+int quant_tile_rows(const Store &st, bool rotated) {
+    const int D = std::max(st.Dk, st.Dv);
+    if (D <= 64 || (D <= 128 && !rotated)) return 9;
+    if (D <= 128) return D <= 96 ? 10 : 14;
+    if (st.gs == 128) return rotated ? 20 : 17;
+    return rotated ? 17 : 14;
+}
 
 hipError_t launch_append_quant(const Store &st, const void *keys, const void *values, int L, int src0,
                                int slot0, int n, hipStream_t s, RopeDev *rope) {
     if (n <= 0) return hipSuccess;
     const RopeDev r = take_rope(rope);
     const bool tiled = quant_tiles_one_launch(st) || quant_tiles_two_sided(st);
-    // The row kernel's wavefronts take their rows one after the other (about 2.6 us a row and wavefront: 33 us for 50
-    // rows of 128); one launch of the tile kernel takes every row of its tiles at once, 7 to 11 us whatever their number.
+    // One launch of the tile kernel takes every row of its tiles at once, 7 to 25 us whatever their number; the row kernel's
+    // wavefronts take theirs one after the other, each tile's in a workgroup of its own (33 us for 50 rows of 128).
     // A 501-row piece at an odd slot, rotated: 50 us as rows, whole tiles, rows (three launches), 11.5 us so.
-    if (!tiled || n < QUANT_TILE_ROWS) return launch_append_quant_rows(st, keys, values, L, src0, slot0, n, s, r);
+    const int head = std::min(n, TILE - (slot0 & (TILE - 1)));
+    const int most = std::max(head, std::min(n - head, TILE));
+    if (!tiled || most < quant_tile_rows(st, r.dims > 0)) return launch_append_quant_rows(st, keys, values, L, src0, slot0, n, s, r);
     if (st.bits == 4) return launch_quant_tiles_bits<4, true, false>(st, st, keys, values, L, src0, slot0, n, s, r);
     if (st.bits == 8) return launch_quant_tiles_bits<8, true, false>(st, st, keys, values, L, src0, slot0, n, s, r);
     return launch_quant_tiles_other(st, keys, values, L, src0, slot0, n, s, r);

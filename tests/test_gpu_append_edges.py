@@ -12,9 +12,10 @@ from tests.util import randn
 
 pytestmark = pytest.mark.gpu
 
-# a first piece inside one tile, one that ends on a tile's edge, one of a whole tile at an odd slot, one row more than
-# the row kernel takes, one that begins on an edge and crosses a 256-row page; 'trim' leaves older rows behind the end
-PIECES = [(9, 0), (55, 0), (5, 0), (64, 3), (9, 0), (63, 20), (10, 0), (130, 1), (61, 0)]
+# a first piece inside one tile, one that ends on a tile's edge, one of a whole tile at an odd slot, one that begins on an
+# edge and crosses a 256-row page; pieces on both sides of the counts from which the quantized tile kernel takes over (9 to
+# 20 by size and rotation), and one whose two halves lie below them; 'trim' leaves older rows behind the end
+PIECES = [(9, 0), (55, 0), (5, 0), (64, 3), (9, 0), (63, 20), (10, 0), (130, 1), (61, 0), (13, 0), (14, 0), (16, 0), (17, 0), (22, 0), (19, 0), (20, 0)]
 
 
 def _fill(cache, k, v, pieces, rope, quantized, one_by_one):
