@@ -24,7 +24,7 @@ __device__ __forceinline__ void unpack8(const u4v &raw, const char *row, int d0,
             rope_chunk<DT>(rope, inv_s, row, d0, pos, raw, w);
         } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] = rope_elem<DT>(rope, row, d0 + j, pos);
+            for (int j = 0; j < 8; ++j) w[j] = rope_elem<DT, true>(rope, row, d0 + j, pos);
         }
         return;
     }

@@ -22,11 +22,10 @@ __device__ __forceinline__ void rope_sincos_reduced(float x, int quad, float &sn
     cs = ((quad + 1) & 2) ? -b : b;
 }
 
-// The same for an angle of 2^24 and more, by Payne and Hanek's method: the angle is m 2^e with an integer m < 2^24, and of
-// 2/pi only the 64 bits from weight 2^(1 - e) on matter to the product modulo 4 (an error of the remainder below 2^-37).
-// A function of its own: positions times frequencies do not get there in ordinary use, and a copy of it beside each of the
-// sixteen short ones of a chunk kept the tile kernels' loops from being unrolled.
-static __device__ __attribute__((noinline)) float2 rope_sincos_large(float theta) {
+// The remainder and quadrant of an angle of 2^24 and more, by Payne and Hanek's method: the angle is m 2^e with an integer
+// m < 2^24, and of 2/pi only the 64 bits from weight 2^(1 - e) on matter to the product modulo 4 (an error of the
+// remainder below 2^-37).
+__device__ __forceinline__ void rope_reduce_large(float theta, float &x, int &quad) {
     const uint32_t u = __float_as_uint(theta);
     const int at = (int)((u >> 23) & 255u) - 151;  // the first bit that matters: 0 .. 103 (104: infinite, NaN)
     const uint64_t m = (u & 0x7fffffu) | 0x800000u;
@@ -34,10 +33,21 @@ static __device__ __attribute__((noinline)) float2 rope_sincos_large(float theta
     const uint64_t hi = at < 64 ? T0 : T1, lo = at < 64 ? T1 : T2;
     const uint64_t p = m * ((hi << (at & 63)) | ((lo >> 1) >> (63 - (at & 63))));  // times 2^62, modulo 4
     const uint64_t k = (p + (1ull << 61)) >> 62;
-    const float x = at == 104 ? theta - theta : (float)((double)(int64_t)(p - (k << 62)) * 3.4061215800865545e-19);  // pi/2 2^-62
+    x = at == 104 ? theta - theta : (float)((double)(int64_t)(p - (k << 62)) * 3.4061215800865545e-19);  // pi/2 2^-62
+    quad = (int)k;
+    if (u >> 31) {
+        x = -x;
+        quad = -quad;
+    }
+}
+// A function of its own: positions times frequencies do not get there in ordinary use, and a copy of it beside each of the
+// sixteen short ones of a chunk kept the tile kernels' loops from being unrolled.
+static __device__ __attribute__((noinline)) float2 rope_sincos_large(float theta) {
+    float x;
+    int quad;
+    rope_reduce_large(theta, x, quad);
     float2 sc;
-    rope_sincos_reduced(x, (int)k, sc.x, sc.y);
-    if (u >> 31) sc.x = -sc.x;
+    rope_sincos_reduced(x, quad, sc.x, sc.y);
     return sc;
 }
 
@@ -47,15 +57,22 @@ static __device__ __attribute__((noinline)) float2 rope_sincos_large(float theta
 // 4.5 10^-8 with the library's sincosf.  Some 30 instructions; sincosf carries a multi-word reduction for large angles
 // that the appends spent most of their time in (512 rows of 8 heads x 128: 22.7 us full precision and 18.8 us quantized
 // with it and an exponential per element, 10.3 and 11.4 us so).
-__device__ __forceinline__ void rope_sincos_ordinary(float theta, float &sn, float &cs) {
+constexpr float ROPE_LARGE = 16777216.f;
+__device__ __forceinline__ void rope_reduce(float theta, float &x, int &quad) {
     const double t = (double)theta;
     const double k = rint(t * 0.63661977236758134308);
-    rope_sincos_reduced((float)fma(-k, 1.57079632679489661923, t), (int)(k - 4.0 * floor(k * 0.25)), sn, cs);
+    x = (float)fma(-k, 1.57079632679489661923, t);
+    quad = (int)(k - 4.0 * floor(k * 0.25));
 }
-constexpr float ROPE_LARGE = 16777216.f;
+// (CALL: in code that is repeated for many elements)
+template <bool CALL>
 __device__ __forceinline__ void rope_sincos(float theta, float &sn, float &cs) {
-    rope_sincos_ordinary(theta, sn, cs);
-    if (__builtin_expect(fabsf(theta) >= ROPE_LARGE, 0)) {
+    float x;
+    int quad;
+    rope_reduce(theta, x, quad);
+    if (!CALL && __builtin_expect(fabsf(theta) >= ROPE_LARGE, 0)) rope_reduce_large(theta, x, quad);
+    rope_sincos_reduced(x, quad, sn, cs);
+    if (CALL && __builtin_expect(fabsf(theta) >= ROPE_LARGE, 0)) {
         const float2 sc = rope_sincos_large(theta);
         sn = sc.x;
         cs = sc.y;
@@ -70,7 +87,10 @@ __device__ __forceinline__ void rope_sincos_many(ANGLE angle, float (&sn)[V], fl
     for (int j = 0; j < V; ++j) {
         const float theta = angle(j);
         largest = fmaxf(largest, fabsf(theta));
-        rope_sincos_ordinary(theta, sn[j], cs[j]);
+        float x;
+        int quad;
+        rope_reduce(theta, x, quad);
+        rope_sincos_reduced(x, quad, sn[j], cs[j]);
     }
     if (__builtin_expect(largest >= ROPE_LARGE, 0)) {
 #pragma unroll 1
@@ -105,7 +125,7 @@ __device__ __forceinline__ float rope_turn(float x, float y, bool first, float s
 // (what the reference hands to the cache: `applyRotaryPosition` runs before `update`,
 // Llama.swift:58-62).  The angle is the float32 product of position * scale and the inverse
 // frequency exp(-i * log(base) / half), or 1 / freqs[i].
-template <int DT>
+template <int DT, bool CALL = false>
 __device__ __forceinline__ float rope_elem(const RopeDev &r, const void *row, int d, int pos) {
     const float x = Elem<DT>::load(row, d);
     if (d >= r.dims) return x;
@@ -122,7 +142,7 @@ __device__ __forceinline__ float rope_elem(const RopeDev &r, const void *row, in
         partner = first ? d + half : d - half;
     }
     float sn, cs;
-    rope_sincos(rope_angle(r, pos, rope_inv_freq(r, i)), sn, cs);
+    rope_sincos<CALL>(rope_angle(r, pos, rope_inv_freq(r, i)), sn, cs);
     return round_dt<DT>(rope_turn(x, Elem<DT>::load(row, partner), first, sn, cs));
 }
 
@@ -206,7 +226,7 @@ __device__ __forceinline__ void rope_stage_step(const RopeDev &r, int bh, const 
     const int d0 = !turn ? r.dims + 2 * (p - half) : r.traditional ? 2 * p : p;
     const int d1 = turn && !r.traditional ? d0 + half : d0 + 1;
     float sn = 0.f, cs = 1.f;
-    if (turn) rope_sincos(rope_angle(r, rope_pos(r, bh, 0), rope_inv_freq(r, p)), sn, cs);
+    if (turn) rope_sincos<false>(rope_angle(r, rope_pos(r, bh, 0), rope_inv_freq(r, p)), sn, cs);
     for (int i = threadIdx.x / P; i <= R && threadIdx.x < ns * P; i += ns) {
         const uint16_t *row = i < R ? q + (size_t)i * D : k;
         uint16_t x = row[d0], y = row[d1];
