@@ -1165,13 +1165,27 @@ void queries_ride(RopeDev &r, const void *q, void *q_rotated, int B, int Hq, int
     r.qD = D;
 }
 
+// whether a decode kernel takes a single-token step without a mask of this cache, its rows still to be written and rotated
+bool decode_takes_step(const kvhip_cache *c, int Hq) {
+    AttendArgs a;
+    a.st = c->st;
+    a.B = c->B;
+    a.Hq = Hq;
+    a.Hkv = c->Hkv;
+    a.L = 1;
+    a.runs.n = 1;  // (quantized caches are never in pieces, the full-precision kernel takes them)
+    a.runs.row0[0] = a.runs.phys0[0] = 0;
+    return g_policy != 1 && attend_decode_fuses_append(a);
+}
+
 // new_k / new_v: the rows of a single-token step whose bookkeeping is done but whose write into physical
 // slot `new_slot` is still owed; the decode kernel takes them along when it can, else they are
 // appended by a launch of their own first.  `rope`: the queries and the new key row are still to be rotated (its H:
-// kv heads), by whichever of the two launches takes the row.
+// kv heads), by whichever of the two launches takes the row; `q_rotated` takes the queries if it is not the decode kernel.
 kvhip_status attend_impl(kvhip_cache *c, const void *q, int32_t B, int32_t Hq, int32_t L, int32_t D, float scale,
                          const kvhip_mask *mask, void *out, void *stream, float *fixed, size_t fixed_bytes,
-                         const void *new_k = nullptr, const void *new_v = nullptr, int32_t new_slot = -1, RopeDev *rope = nullptr) {
+                         const void *new_k = nullptr, const void *new_v = nullptr, int32_t new_slot = -1, RopeDev *rope = nullptr,
+                         void *q_rotated = nullptr) {
     if (!c || !q || !out) return fail(KVHIP_ERR_INVALID_ARG, "null argument");
     const bool staged_view = c->staging && !c->stage_view.empty();
     if (!c->has_geom || (!c->has_buffers && !staged_view) || c->presented <= 0)
@@ -1247,13 +1261,13 @@ kvhip_status attend_impl(kvhip_cache *c, const void *q, int32_t B, int32_t Hq, i
             a.rope = rope;
         } else {
             if (rope) {
-                KV_TRY(ensure_pad_buf(c, 4, (size_t)B * Hq * D * c->st.es));
-                a.q = c->pad_buf[4];
-                if (rope->vec) queries_ride(*rope, q, c->pad_buf[4], B, Hq, 1, D);
+                if (!q_rotated) return fail(KVHIP_ERR_INTERNAL, "rotary step without room for its queries");
+                a.q = q_rotated;
+                if (rope->vec) queries_ride(*rope, q, q_rotated, B, Hq, 1, D);
                 else {
                     RopeDev own = *rope;
                     own.H = Hq;
-                    KV_HIP(launch_rope_apply(own, q, c->pad_buf[4], B, Hq, 1, D, c->st.dtype, s));
+                    KV_HIP(launch_rope_apply(own, q, q_rotated, B, Hq, 1, D, c->st.dtype, s));
                 }
             }
             if (c->st.bits != 0) KV_HIP(launch_append_quant(c->st, new_k, new_v, 1, 0, new_slot, 1, s, rope));
@@ -1359,9 +1373,20 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
     KV_TRY(rope_dev(rope, Dk, Hkv, dtype, pos0, batch_offsets, r));
     // One new token without a mask: the decode kernels rotate its rows themselves, as they write the new one
     // (kvhip_cache_update_attend), and the step is a launch less.
-    if (L == 1 && !c->staging && (dtype == KVHIP_F16 || dtype == KVHIP_BF16) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
-        c->has_geom && c->has_buffers && !c->padded() && c->B == B && c->Hkv == Hkv && c->st.Dk == Dk && c->st.Dv == Dv &&
-        c->st.dtype == dtype && (size_t)B * Hkv + (size_t)B * Hq <= 65535) {
+    const bool token = L == 1 && !c->staging && (dtype == KVHIP_F16 || dtype == KVHIP_BF16) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
+                       c->has_geom && c->has_buffers && !c->padded() && c->B == B && c->Hkv == Hkv && c->st.Dk == Dk && c->st.Dv == Dv &&
+                       c->st.dtype == dtype && (size_t)B * Hkv + (size_t)B * Hq <= 65535;
+    if (!q_rotated && !(token && decode_takes_step(c, Hq))) {
+        // (before anything is written: a stream that is being captured cannot have the memory, and its caller asks again)
+        const size_t need = (size_t)B * Hq * L * Dk * elem_size(dtype);
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (need > c->pad_bytes[4]) KV_HIP(hipStreamIsCapturing(S(stream), &capture));
+        if (capture != hipStreamCaptureStatusNone)
+            return fail(KVHIP_ERR_UNSUPPORTED, "a captured rotary step needs q_rotated: the cache's own buffer cannot grow here");
+        KV_TRY(ensure_pad_buf(c, 4, need));
+        q_rotated = c->pad_buf[4];
+    }
+    if (token) {
         int32_t slot = -1;
         if (c->kind == KVHIP_KIND_ROTATING) {
             KV_TRY(update_rotating(c, k, v, 1, S(c, stream), &slot));
@@ -1369,17 +1394,13 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
             KV_TRY(update_simple(c, k, v, 1, S(c, stream), false));
             slot = (int32_t)c->offset - 1;
         }
-        const kvhip_status st = attend_impl(c, q, B, Hq, L, Dk, scale, mask, out, stream, nullptr, 0, k, v, slot, &r);
+        const kvhip_status st = attend_impl(c, q, B, Hq, L, Dk, scale, mask, out, stream, nullptr, 0, k, v, slot, &r, q_rotated);
         if (st != KVHIP_OK) {  // the cache holds what its counters say
             r.qx = nullptr;
             if (c->st.bits != 0) (void)launch_append_quant(c->st, k, v, 1, 0, slot, 1, S(c, stream), &r);
             else (void)launch_append_fp(c->st, k, v, 1, 0, slot, 1, S(c, stream), &r);
         }
         return st;
-    }
-    if (!q_rotated) {
-        KV_TRY(ensure_pad_buf(c, 4, (size_t)B * Hq * L * Dk * (dtype == KVHIP_F32 ? 4 : 2)));
-        q_rotated = c->pad_buf[4];
     }
     // The queries turn in the append's launch when their rows are whole 16-byte chunks (a launch of their own costs
     // 3 to 5 us on the device and as much on the host).

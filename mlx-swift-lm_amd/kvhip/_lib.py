@@ -11,7 +11,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libkvhip.so")
 
-OK = 0
+OK, ERR_UNSUPPORTED = 0, -3
 KIND_SIMPLE, KIND_ROTATING, KIND_QUANTIZED = 0, 1, 2
 F16, BF16, F32, U32, BOOL = 0, 1, 2, 3, 4
 MASK_NONE, MASK_CAUSAL, MASK_ARRAY, MASK_WINDOW = 0, 1, 2, 3

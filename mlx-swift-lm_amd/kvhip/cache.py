@@ -270,9 +270,14 @@ class _Cache:
         m, keep = (mask or MaskMode.none()).to_c(B, Hq, Lq)
         r, freqs = rope.to_c()
         bo = None if batch_offsets is None else batch_offsets.to(device="cuda", dtype=torch.int32).contiguous()
-        L.check(self._lib.kvhip_cache_update_attend_rope(
-            self._h, C.byref(r), _ptr(bo) if bo is not None else None, _ptr(q), _ptr(k), _ptr(v), B, Hq, k.shape[1], Lq, D, Dv,
-            _DT[k.dtype], float(scale), C.byref(m), _ptr(q_rot) if q_rot is not None else None, _ptr(out), _stream()))
+        while True:
+            st = self._lib.kvhip_cache_update_attend_rope(
+                self._h, C.byref(r), _ptr(bo) if bo is not None else None, _ptr(q), _ptr(k), _ptr(v), B, Hq, k.shape[1], Lq, D, Dv,
+                _DT[k.dtype], float(scale), C.byref(m), _ptr(q_rot) if q_rot is not None else None, _ptr(out), _stream())
+            if st != L.ERR_UNSUPPORTED or q_rot is not None or not torch.cuda.is_current_stream_capturing():
+                break
+            q_rot = torch.empty_like(q)  # (the cache's own buffer cannot grow under capture)
+        L.check(st)
         self._note_shape(k, v)
         del keep, freqs
         return out

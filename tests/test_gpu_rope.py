@@ -267,3 +267,45 @@ def test_angles_of_any_size(dims, traditional):
         want = OR.rope(x32, dims, traditional, 10000.0, 0.5, offset, freqs=freqs, dtype="float32")
         ok, mx = within_one_ulp(got, want, torch.float32, pair_norms(x32, dims, traditional))
         assert ok, f"offset {offset}: max diff {mx:.3e}"
+
+
+@pytest.mark.parametrize("kind,dtype,D,Lq", [("simple", torch.float16, 128, 5), ("simple", torch.bfloat16, 512, 1), ("simple", torch.float32, 64, 1),
+                                             ("simple", torch.float16, 128, 1), (4, torch.float16, 128, 5), (4, torch.bfloat16, 128, 1)])
+def test_one_call_is_captured_where_the_separate_calls_are(kind, dtype, D, Lq):
+    """Pages reserved and attention scratch there from calls without the rotation: the one call allocates nothing of its
+    own, so it can be captured, and each replay equals the separate calls on the same rows."""
+    B, Hq, Hkv = 2, 8, 2
+    rope = kvhip.RoPE(D, base=1e4)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+
+    def rows(n):
+        return [torch.randn(B, h, n, D, generator=gen, device="cuda").to(dtype) for h in (Hq, Hkv, Hkv)]
+
+    cache = kvhip.KVCacheSimple() if kind == "simple" else kvhip.QuantizedKVCache(64, kind)
+    cache.reserve(B, Hkv, D, D, dtype, 600)
+    _, k, v = rows(300)
+    cache._update(k, v)
+    mask = kvhip.create_attention_mask(Lq, cache)
+    q, k, v = rows(Lq)
+
+    def separate():
+        turned = kvhip.apply_rotary_position(rope, q, cache.rope_offset)
+        cache.update_rope(rope, k, v)
+        out = cache.attend(turned, D ** -0.5, mask)
+        cache.trim(Lq)
+        return out
+
+    separate()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = kvhip.attention_with_rope_and_cache_update(rope, q, k, v, cache, D ** -0.5, mask)
+    cache.trim(Lq)
+    for _ in range(3):
+        for t, new in zip((q, k, v), rows(Lq)):
+            t.copy_(new)
+        graph.replay()
+        got = out.clone()
+        torch.cuda.synchronize()
+        assert torch.equal(got, separate())
+        torch.cuda.synchronize()
