@@ -46,9 +46,12 @@ def test_gathered_rows_are_the_rows_written(window, keep, dtype, Dk, Dv):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("D", [64, 80, 96, 128, 256])
-@pytest.mark.parametrize("keys", [200, 700, 1500, 3001])
-def test_parts_of_many_rows_merge(dtype, D, keys):
-    """Two to eight parts, rows that do not fill the last workgroup, parts that a row's mask leaves empty."""
+@pytest.mark.parametrize("keys,parts", [(200, 1), (700, 2), (900, 3), (1100, 4), (1500, 5), (2100, 8), (3001, 11)])
+def test_parts_of_many_rows_merge(dtype, D, keys, parts):
+    """One part (no merge), the two to eight of combine_rows_kernel, each of its instances at its last count and at one
+    below, and a count above (combine_kernel); rows that do not fill the last workgroup, parts that a row's mask leaves
+    empty.  These few workgroups get an eighth of the 32-key tiles each."""
+    assert (keys + 31) // 32 // 8 in (parts, parts - 1) and max(1, (keys + 31) // 32 // 8) == parts
     rng = np.random.default_rng(D + keys)
     B, Hq, Hkv, L = 2, 6, 2, 131
     cache = kvhip.KVCacheSimple()
