@@ -241,3 +241,43 @@ def test_inputs_at_odd_element_offsets(kind, Lq):
         states.append([a.clone() for a in c.state])
     assert torch.equal(outs[0], outs[1])
     assert len(states[0]) == len(states[1]) and all(torch.equal(a, b) for a, b in zip(*states))
+
+
+@pytest.mark.parametrize("kind,dtype,D", [("simple", torch.float16, 128), ("rotating", torch.bfloat16, 256), (4, torch.float16, 128), (6, torch.bfloat16, 64),
+                                          ("simple", torch.bfloat16, 512), (8, torch.float16, 512), ("simple", torch.float32, 64), ("rotating", torch.float32, 256)])
+@pytest.mark.parametrize("Lq", [1, 5, 70])
+def test_rotary_inputs_and_wide_heads_at_odd_element_offsets(kind, dtype, D, Lq):
+    """The same for the rotary calls (separate, in place and with the update), head size 512 and float32, outputs too."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    B, Hq, Hkv, T0 = 2, 8, 2, 90
+    es = 4 if dtype == torch.float32 else 2
+
+    def odd(*shape):
+        flat = torch.randn(int(np.prod(shape)) + 1, generator=g, device="cuda").to(dtype)
+        v = flat[1:].view(*shape)
+        assert v.data_ptr() % 16 == es and v.is_contiguous()
+        return v
+
+    rope = kvhip.RoPE(D, base=1e5)
+    first, new = ([odd(B, h, n, D) for h in (Hq, Hkv, Hkv)] for n in (T0, Lq))
+    results = []
+    for aligned in (False, True):
+        f = (lambda t: t.clone()) if aligned else (lambda t: t)
+        c = kvhip.KVCacheSimple() if kind == "simple" else kvhip.RotatingKVCache(130, keep=4) if kind == "rotating" else kvhip.QuantizedKVCache(64, kind)
+        outs = [c.update_attend_rope(rope, *map(f, first), D ** -0.5, kvhip.MaskMode.causal()),
+                c.update_attend_rope(rope, *map(f, new), D ** -0.5, kvhip.create_attention_mask(Lq, c))]
+        outs += [t.clone() for t in c.state] + [kvhip.apply_rotary_position(rope, f(new[0]), 7)]
+        turned, dst = (torch.empty(new[0].numel() + 1, dtype=dtype, device="cuda")[0 if aligned else 1:][:new[0].numel()].view_as(new[0]) for _ in range(2))
+        turned.copy_(new[0])
+        r, keep = rope.to_c()
+        L.check(kvhip.load().kvhip_rope_apply(r, turned.data_ptr(), turned.data_ptr(), B, Hq, Lq, D, c_dtype(dtype), 7, None, None))
+        torch.cuda.synchronize()
+        outs += [turned, c.attend(f(new[0]), D ** -0.5, kvhip.MaskMode.none(), out=dst)]
+        results.append(outs)
+    for i, (a, b) in enumerate(zip(*results)):
+        assert torch.equal(a, b), i
+    assert torch.equal(results[0][-2], results[0][-3])
+
+
+def c_dtype(dtype):
+    return {torch.float16: L.F16, torch.bfloat16: L.BF16, torch.float32: L.F32}[dtype]
