@@ -140,9 +140,9 @@ namespace {
 // replaced, the memory of a freed cache) cannot be freed on the spot: hipFree waits for the whole
 // device.  They are retired behind an event recorded on the stream of their last reader.  Once
 // that event has completed (hipEventQuery: no waiting) a buffer moves to a free list, from which
-// later allocations of a similar size are served instead of hipMalloc, so a loop that creates,
-// grows and frees caches without ever calling a blocking entry point neither waits nor keeps
-// growing the device's memory.  Buffers the free list holds beyond its limits, and everything on
+// later allocations of a similar size are served instead of hipMalloc (pages for work on that same stream at
+// once), so a loop that creates, grows and frees caches without ever calling a blocking entry point neither
+// waits nor keeps growing the device's memory.  Buffers the free list holds beyond its limits, and everything on
 // it when a blocking call runs (kvhip_sync, kvhip_cache_reserve, a hipMalloc that failed), are
 // released with hipFree there.  Only the stream a cache was last used on is tracked: a caller who
 // reads one cache on several streams orders them before kvhip_cache_free.
@@ -397,7 +397,9 @@ kvhip_status ensure_slots(kvhip_cache *c, int64_t slots, hipStream_t stream, boo
     const size_t bytes = part[0] + part[1] + part[2] + part[3];
     void *base = nullptr;
     size_t got = bytes;
-    hipError_t e = pool_alloc(&base, bytes, &got);
+    // The pages are cleared on `stream` before anything else touches them, so pages retired behind earlier work of that
+    // stream will do: a host that runs ahead of the device does not hold a cache's memory for each one in flight.
+    hipError_t e = pool_alloc(&base, bytes, &got, &stream);
     if (e != hipSuccess) {  // memory of freed caches may still be waiting for its release: wait for it and retry
         (void)hipGetLastError();
         (void)hipDeviceSynchronize();

@@ -194,6 +194,40 @@ def test_created_grown_and_freed_caches_reuse_their_memory_without_a_blocking_ca
     assert all(torch.equal(outs[0], o) for o in outs[1:])
 
 
+def test_caches_of_a_busy_stream_take_over_each_others_pages():
+    """The host far ahead of the device: caches are created, filled, read and dropped behind work that keeps the stream
+    busy, so none of their pages is finished with when the next cache asks.  It is served from those retired on its own
+    stream, behind whose readers it runs, and the answers are those of caches on their own."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    B, H, D = 4, 8, 128
+    k, v = (torch.randn(B, H, 16384, D, generator=g, device="cuda").half() for _ in range(2))
+    qs = torch.randn(12, B, 32, 1, D, generator=g, device="cuda").half()
+    per_cache = 2 * B * H * 16384 * D * 2  # (larger than what other tests leave on the free list)
+    heavy = torch.randn(8192, 8192, device="cuda").bfloat16()
+
+    def serve(i):
+        c = kvhip.KVCacheSimple()
+        c.update(k if i % 2 else v, v if i % 2 else k, fetch=False)
+        return c.attend(qs[i], D ** -0.5)
+
+    want = []
+    for i in range(12):
+        want.append(serve(i))
+        torch.cuda.synchronize()
+    torch.mm(heavy, heavy)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    for _ in range(40):
+        torch.mm(heavy, heavy)
+    got = [serve(i) for i in range(12)]
+    after = torch.cuda.mem_get_info()[0]
+    torch.cuda.synchronize()
+    # (torch's own allocator holds the products and outputs, which it keeps between the calls)
+    assert before - after < 3 * per_cache, (before - after, per_cache)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_dequantize_first_scratch_is_one_buffer_per_stream():
     """A large prompt chunk over a quantized cache runs over scratch pages the cache is dequantized into.  The scratch
     is taken from the pool at the call and retired behind it, and a call may take a buffer retired on its own stream
