@@ -154,6 +154,7 @@ struct Buf {
 struct Retired {
     hipEvent_t done;
     hipStream_t stream;  // where `done` was recorded: work enqueued there later runs after the buffers' last reader
+    bool captured;       // ... by a stream that was capturing: the graph's launches use the buffers whenever they run
     std::vector<Buf> bufs;
 };
 std::mutex g_retired_mu;
@@ -168,10 +169,18 @@ int current_device() {
     return d;
 }
 
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) == hipSuccess) return capture != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 void retire(std::vector<std::pair<void *, size_t>> &&ptrs, hipStream_t stream) {
     if (ptrs.empty()) return;
     Retired r;
     r.stream = stream;
+    r.captured = capturing(stream);
     const int dev = current_device();
     for (auto &q : ptrs) r.bufs.push_back(Buf{q.first, q.second, dev});
     if (hipEventCreateWithFlags(&r.done, hipEventDisableTiming) != hipSuccess || hipEventRecord(r.done, stream) != hipSuccess) {
@@ -210,10 +219,11 @@ hipError_t pool_alloc(void **out, size_t bytes, size_t *got, const hipStream_t *
         std::lock_guard<std::mutex> lock(g_retired_mu);
         harvest_locked();
         const int dev = current_device();
-        if (same_stream) {
+        if (same_stream && *same_stream != hipStreamPerThread) {  // (that handle is another stream in each thread)
+            const bool in_graph = capturing(*same_stream);
             for (size_t i = 0; i < g_retired.size(); ++i) {
                 Retired &r = g_retired[i];
-                if (r.stream != *same_stream) continue;
+                if (r.stream != *same_stream || (r.captured && !in_graph)) continue;
                 for (size_t j = 0; j < r.bufs.size(); ++j) {
                     const Buf &b = r.bufs[j];
                     if (b.dev != dev || b.bytes < bytes || b.bytes > bytes + bytes / 2) continue;
@@ -398,8 +408,9 @@ kvhip_status ensure_slots(kvhip_cache *c, int64_t slots, hipStream_t stream, boo
     void *base = nullptr;
     size_t got = bytes;
     // The pages are cleared on `stream` before anything else touches them, so pages retired behind earlier work of that
-    // stream will do: a host that runs ahead of the device does not hold a cache's memory for each one in flight.
-    hipError_t e = pool_alloc(&base, bytes, &got, &stream);
+    // stream will do: a host that runs ahead of the device does not hold a cache's memory for each one in flight.  (Not
+    // in a capture: the graph's launches would write them at any later time.)
+    hipError_t e = pool_alloc(&base, bytes, &got, capturing(stream) ? nullptr : &stream);
     if (e != hipSuccess) {  // memory of freed caches may still be waiting for its release: wait for it and retry
         (void)hipGetLastError();
         (void)hipDeviceSynchronize();

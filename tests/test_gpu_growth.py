@@ -4,6 +4,8 @@ further allocation and are entered into the cache's page table, so nothing that 
 Contents, offsets and capacities are compared with the oracle across page, allocation and page-table
 boundaries, and on a stream other than the default one."""
 
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 import torch
@@ -225,6 +227,41 @@ def test_caches_of_a_busy_stream_take_over_each_others_pages():
     torch.cuda.synchronize()
     # (torch's own allocator holds the products and outputs, which it keeps between the calls)
     assert before - after < 3 * per_cache, (before - after, per_cache)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_pages_of_a_threads_own_stream_stay_out_of_other_threads(monkeypatch):
+    """The per-thread default stream is one handle in every thread and a stream of its own in each.  A cache dropped
+    behind work in flight on one thread's must not give its pages to a cache of another thread, which would write them
+    while the first thread's kernels still wait to."""
+    PER_THREAD = 2  # hipStreamPerThread
+    monkeypatch.setattr("kvhip.cache._stream", lambda: PER_THREAD)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(2)
+    B, H, D, T = 4, 8, 128, 16384
+    k, v = (torch.randn(B, H, T, D, generator=g, device="cuda").half() for _ in range(2))
+    q = torch.randn(B, 32, 1, D, generator=g, device="cuda").half()
+    torch.cuda.synchronize()
+    kept = []  # (torch's allocator does not know of the stream: nothing goes back to it before the end)
+
+    def serve(swap, busy=0):
+        for _ in range(busy):
+            kept.append(big.attend(q, D ** -0.5))
+        c = kvhip.KVCacheSimple()
+        c.update(v if swap else k, k if swap else v, fetch=False)
+        kept.append(c.attend(q, D ** -0.5))
+        return kept[-1]
+
+    big = kvhip.KVCacheSimple()
+    big.update(k, v, fetch=False)
+    torch.cuda.synchronize()
+    with ThreadPoolExecutor(1) as one, ThreadPoolExecutor(1) as other:  # (both threads live until the device is done)
+        want = []
+        for thread, swap in ((one, False), (other, True)):
+            want.append(thread.submit(serve, swap).result())
+            torch.cuda.synchronize()
+        got = [one.submit(serve, False, 400).result(), other.submit(serve, True).result()]
+        torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
