@@ -10,7 +10,7 @@
 //   out^T = V^T P^T  lane (i, g) loads tokens 4 g .. 4 g + 3 of column i, and the scores leave the first product with
 //                  tokens 4 g .. 4 g + 3 of query i in lane (i, g): the probabilities are the operand as they are.
 // Measured against the vector-ALU kernel, whole calls: 512 x 4096, B4, 32q/8kv 1626 -> 654 us (D 64), 2644 -> 1215
-// (D 128: 106 TFLOP/s of the 157 that the instruction has), 6755 -> 2524 (D 256); one token of one sequence, 16q/4kv, 1500
+// (D 128: 106 TFLOP/s of the 157 that the instruction has), 6755 -> 2480 (D 256); one token of one sequence, 16q/4kv, 1500
 // keys 17.3 -> 12.4 us (D 64: one pass of loads and the merge); 8192 keys of B8, 8 kv heads, HBM: 102 -> 101 us (D 128).
 #include <algorithm>
 
@@ -45,7 +45,8 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
     extern __shared__ __align__(16) float smem[];
     f4 *acc_s = reinterpret_cast<f4 *>(smem);         // [MW][QT][NCT][64]
     constexpr bool QL = DK > 128;                     // query operands in LDS: no registers are left for them
-    __shared__ f4 q_s[QL ? QT * NS * 64 : 1];
+    f4 *q_s = reinterpret_cast<f4 *>(smem);           // [QT][NS][64], where the accumulators go after the loop: beside them
+                                                      // only one workgroup of head size 256 would fit a CU (that call: 2607)
     __shared__ float max_s[MW][QT][16], sum_s[MW][QT][16];
     const Store &st = a.st;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
