@@ -263,7 +263,11 @@ class _Cache:
         """Queries and keys rotated at this cache's `ropeOffset` (or at `batch_offsets`), update, attention."""
         q, k, v = queries.contiguous(), keys.contiguous(), values.contiguous()
         assert k.is_cuda and v.is_cuda and k.dtype == v.dtype
+        if q.dtype != k.dtype:
+            self._check_query_dtype(q, k)
         B, Hq, Lq, D = q.shape
+        if (B, Lq, D) != (k.shape[0], k.shape[2], k.shape[3]):
+            raise ValueError(f"queries {tuple(q.shape)} do not go with keys {tuple(k.shape)} row by row")
         Dv = v.shape[3]
         out = torch.empty((B, Hq, Lq, Dv), dtype=q.dtype, device=q.device)
         q_rot = torch.empty_like(q) if q.numel() * q.element_size() > _Q_ROTATED_KEPT else None

@@ -309,3 +309,18 @@ def test_one_call_is_captured_where_the_separate_calls_are(kind, dtype, D, Lq):
         torch.cuda.synchronize()
         assert torch.equal(got, separate())
         torch.cuda.synchronize()
+
+
+def test_one_call_refuses_queries_that_do_not_go_with_the_keys():
+    """The library reads the queries as the keys' dtype and row count; the method itself says so, before any write."""
+    rope = kvhip.RoPE(64, base=1e4)
+    cache = kvhip.KVCacheSimple()
+    k = torch.randn(1, 2, 3, 64, device="cuda").bfloat16()
+    with pytest.raises(TypeError):
+        cache.update_attend_rope(rope, torch.randn(1, 4, 3, 64, device="cuda"), k, k, 0.125)
+    for shape in [(1, 4, 5, 64), (2, 4, 3, 64), (1, 4, 3, 128)]:
+        with pytest.raises(ValueError):
+            cache.update_attend_rope(rope, torch.randn(shape, device="cuda").bfloat16(), k, k, 0.125)
+    assert cache.offset == 0
+    q = torch.randn(1, 4, 3, 64, device="cuda").bfloat16()
+    assert cache.update_attend_rope(rope, q, k, k, 0.125).shape == q.shape and cache.offset == 3
