@@ -259,7 +259,8 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     // one group (group sizes of 64 and more; with 32 the lane groups 0-7 and 8-15 feed two sums), so a lane sums its 4 elements, the 16
     // lane groups are added up by shuffles and the four rows are read out of their quad.
     // (Built by a lambda that the main loop calls after it has requested its first tile, so the
-    // first K/V loads are in flight while the queries are fetched and reduced.)
+    // first K/V loads are in flight while the queries are fetched and reduced.  MODE 3 has staged the
+    // rotated rows before that: its loads start behind the rotation.)
     Op qa[RG][NQA];
     float qsum[RG][G][4];
     auto load_queries = [&]() __attribute__((always_inline)) {
@@ -767,7 +768,7 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     }
 
     // query operands: lane (blk, qi) holds row qi's elements 4*(16 x + blk) .. +3, unscaled
-    // (fetched by the main loop after it has requested its first two pieces)
+    // (fetched by the main loop after it has requested its first two pieces; MODE 3's loads start behind the rotation)
     Op qa[RG][NP];
     auto load_queries = [&]() __attribute__((always_inline)) {
 #pragma unroll

@@ -1,5 +1,6 @@
-// Quantize-on-append of whole 64-token tiles: the element functions, the tile body and its two kernels,
-// and the launchers of one code width (instantiated per width in kvhip_io.hip and kvhip_quant_tile_other.hip).
+// Quantize-on-append of many rows by 64-token tiles, whole ones and the partial ones at either end (from 9 to 20 rows up:
+// `quant_tile_rows`): the element functions, the tile body and its two kernels, and the launchers of one code width
+// (instantiated per width in kvhip_io.hip and kvhip_quant_tile_other.hip).
 #pragma once
 #include "kvhip_rope.hpp"
 
@@ -7,9 +8,9 @@ namespace kvhip {
 
 namespace {
 
-// ---- whole 64-token tiles (prompt-sized appends) -----------------------------------------
+// ---- 64-token tiles (prompt-sized appends) -----------------------------------------------
 // The per-row kernels above fetch one element per lane and wait for every row in turn; for
-// many rows that is bound by load latency.  Here a workgroup takes one whole tile of one
+// many rows that is bound by load latency.  Here a workgroup takes one tile of one
 // (batch, kv-head): every thread first requests all of its 16-byte chunks of the 64 new K and
 // V rows, then quantizes / copies eight elements at a time.  Values, rounding and the
 // rotation are those of the per-row kernels (the same element functions).
