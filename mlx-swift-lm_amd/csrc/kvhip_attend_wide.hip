@@ -335,14 +335,11 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
         // ---- the rows' maxima and sums to every wavefront ----------------------------------------------
         l_run += __shfl_xor(l_run, 16);
         l_run += __shfl_xor(l_run, 32);
-        bool nan = false;
+        f4 probe = acc[0][0];  // (a sum: NaN where one of them is; infinities of both signs only cost the second walk)
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-            for (int c = 0; c < NCT; ++c)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) nan = nan || acc[qt][c][i] != acc[qt][c][i];
-        nan = __any(nan);
+        for (int i = 1; i < QT * NCT; ++i) probe += acc[i / NCT][i % NCT];
+        const float probed = (probe.x + probe.y) + (probe.z + probe.w);
+        const bool nan = __any(probed != probed);
         if (lane == 0) nan_s[wave] = nan;
         if (g == 0 && wave < QT) {
             max_s[own][col] = m_run;
@@ -351,7 +348,7 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
         __syncthreads();
         return (nan_s[0] | nan_s[1] | nan_s[2] | nan_s[3]) != 0;  // workgroup-uniform
     };
-    if (walk(std::false_type())) {
+    if (__builtin_expect(walk(std::false_type()), 0)) {
         __syncthreads();
         walk(std::true_type());
     }
