@@ -26,6 +26,7 @@
 //   q . (scale*code + bias)            = scale * 2^24 * mfma(q, masked K words) + bias * sum(q)
 //   sum_t p_t (scale_t*code_t + bias_t) = 2^24 * mfma(p*scale, masked V words) + sum_t p_t bias_t
 #include <cstdlib>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -247,20 +248,18 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
     // the end) for the wavefronts to fetch them.
     uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
-    if constexpr (rot) {
-        rope_stage_step<DT, D>(a.turn, bh, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
-                                static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R, rot_s);
-        __syncthreads();
-    }
+    [[maybe_unused]] RopeStep<DT, D, NW * 64, 4> step;
+    if constexpr (rot)
+        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
+                   static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R);
 
     // ---- query operands: lane (blk, qi) holds row qi's 4 elements of step 16 x + blk ----
     // qsum[rg][g][i] = sum over group g of the (rounded, fp16-held) query row 4 rg + i, for
     // the bias term; built from the same registers: the 16 steps of one operand pair lie in
     // one group (group sizes of 64 and more; with 32 the lane groups 0-7 and 8-15 feed two sums), so a lane sums its 4 elements, the 16
     // lane groups are added up by shuffles and the four rows are read out of their quad.
-    // (Built by a lambda that the main loop calls after it has requested its first tile, so the
-    // first K/V loads are in flight while the queries are fetched and reduced.  MODE 3 has staged the
-    // rotated rows before that: its loads start behind the rotation.)
+    // (Built by a lambda that is called after the first tile has been requested, so the first K/V loads are in flight
+    // while the queries are fetched and reduced, and in MODE 3 rotated.)
     Op qa[RG][NQA];
     float qsum[RG][G][4];
     auto load_queries = [&]() __attribute__((always_inline)) {
@@ -378,10 +377,15 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     const size_t v_off = (size_t)bh * st.v_cell + (size_t)tip * D * VROW;
     const size_t ksb_off = (size_t)bh * st.ksb_cell + (size_t)tip * TILE * st.ksb_row;
     const size_t vsb_off = (size_t)bh * st.vsb_cell + (size_t)tip * TILE * st.vsb_row;
-    gptr kp = as_global(st.pt[page_k].k) + k_off;
-    gptr vp = as_global(st.pt[page_k].v) + v_off;
-    gptr ksp = as_global(st.pt[page_k].ksb) + ksb_off;
-    gptr vsp = as_global(st.pt[page_k].vsb) + vsb_off;
+    // Four wavefronts: entries by scalar loads, and the offsets added where the tile's loads are formed, so that nothing
+    // waits for an entry before then.  Eight (the chip full of them) read 2 % faster where a half tile's loads arrive
+    // before the next are requested, which a page entry that is a vector load of its own sees to: 32768 keys of 256 pairs at
+    // 4 bits 196.9 us, 200.7 with scalar entries, 199 with a wait in the loop, 201.5 in workgroups of four.
+    constexpr bool LATE = NW == 4;
+    using Table = typename std::conditional<LATE, ptab, const PageEntry *>::type;
+    const Table pt = (Table) reinterpret_cast<uintptr_t>(st.pt);
+    gptr kp = as_global(pt[page_k].k) + (LATE ? 0 : k_off), ksp = as_global(pt[page_k].ksb) + (LATE ? 0 : ksb_off);
+    gptr vp = as_global(pt[page_v].v) + (LATE ? 0 : v_off), vsp = as_global(pt[page_v].vsb) + (LATE ? 0 : vsb_off);
     const uint32_t k_lane = lane * st.k_row, v_lane = lane * VROW;
     const uint32_t ksb_lane = lane * st.ksb_row, vsb_lane = lane * st.vsb_row;
     int slot_next = tile0 * TILE + lane;  // slot of this lane's token in the tile loaded next
@@ -394,42 +398,59 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     }
 
     // ---- the step's new row, when it is still to be written (unmasked single-token decode) -----
-    // Slot T - 1 lies in the last tile, which exactly one wavefront of one workgroup reads (spans
-    // are equal and cover every tile): that wavefront quantizes the row into the cache before it
-    // requests any tile, with the arithmetic of the append kernel, so its own later loads of the
-    // tile see it.  The V code goes into its column's packed word read-modify-write.
+    // Slot T - 1 lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one (spans
+    // are equal and cover every tile): that wavefront quantizes the row into the cache, with the arithmetic of the append
+    // kernel, after it has requested its first tile and before it requests another, so its own later loads of the
+    // row's tile see it; if its first tile is that tile, it requests it again.  The V code goes into its column's packed
+    // word read-modify-write; the row and the old words are requested in front of the tile.  (The row written first and
+    // the tiles requested behind it: the last wavefront of the launch to finish, by four round trips to memory.)
+    bool own = false;
+    uint16_t own_k[NH], own_v[NH];
+    uint32_t own_w[NH];
     if constexpr (MM == 0 && RG == 1) {
         if (a.new_k != nullptr) {  // wave-uniform
             const int slot = a.new_slot, tl = slot >> 6;
-            if (tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % NW) == wave) {
-                const char *krow = static_cast<const char *>(a.new_k) + (size_t)bh * D * 2;
-                const char *vrow = static_cast<const char *>(a.new_v) + (size_t)bh * D * 2;
-                quantize_row_wave_from<DT, BITS>([&](int d) { return rot ? Elem<DT>::load(rot_s, R * D + d) : Elem<DT>::load(krow, d); }, D, GS, lane,
-                                                 reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))),
-                                                 [](int, uint32_t) {}, const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
-                char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
-                const int bp = v_bitpos<BITS>(slot & (TILE - 1));
-                quantize_row_wave_from<DT, BITS>(
-                    [&](int d) { return Elem<DT>::load(vrow, d); }, D, GS, lane, nullptr,
-                    [&](int d, uint32_t code) {
-                        uint32_t *p = reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d)) + (bp >> 5);
-                        *p = (*p & ~(((1u << BITS) - 1u) << (bp & 31))) | (code << (bp & 31));
-                    },
-                    const_cast<char *>(vsb_row_ptr(st, bh, slot)), nullptr, nullptr);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            own = tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % NW) == wave;
+            if (own) {
+                const uint16_t *krow = static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D;
+                const uint16_t *vrow = static_cast<const uint16_t *>(a.new_v) + (size_t)bh * D;
+                const char *vcell = v_cell_ptr(st, bh, slot);
+#pragma unroll
+                for (int h = 0; h < NH; ++h) {
+                    if constexpr (!rot) own_k[h] = krow[64 * h + lane];
+                    own_v[h] = vrow[64 * h + lane];
+                    own_w[h] = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, 64 * h + lane))[v_bitpos<BITS>(slot & (TILE - 1)) >> 5];
+                }
             }
         }
     }
+    auto write_row = [&]() __attribute__((always_inline)) {
+        const int slot = a.new_slot;
+        quantize_row_wave_from<DT, BITS>(
+            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * D + d) : Elem<DT>::load(&own_k[(d - lane) >> 6], 0); }, D, GS, lane,
+            reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))), [](int, uint32_t) {},
+            const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
+        char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
+        const int bp = v_bitpos<BITS>(slot & (TILE - 1));
+        quantize_row_wave_from<DT, BITS>(
+            [&](int d) { return Elem<DT>::load(&own_v[(d - lane) >> 6], 0); }, D, GS, lane, nullptr,
+            [&](int d, uint32_t code) {
+                reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d))[bp >> 5] =
+                    (own_w[(d - lane) >> 6] & ~(((1u << BITS) - 1u) << (bp & 31))) | (code << (bp & 31));
+            },
+            const_cast<char *>(vsb_row_ptr(st, bh, slot)), nullptr, nullptr);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
 
     // The K half (codes, scales, row bookkeeping) and the V half of tile number k_loaded /
     // v_loaded of this wavefront (clamped to its last tile, so loads past the end stay
     // unconditional and in bounds).
     int k_loaded = 0, v_loaded = 0;
     auto load_k = [&](T &t) {
-        load_words<T::KW>(t.k, kp + k_lane);
+        load_words<T::KW>(t.k, kp + (LATE ? k_off : 0) + k_lane);
         uint32_t kraw[G];  // (scale, bias) pairs of a 16-bit dtype
-        load_words<G>(kraw, ksp + ksb_lane);
+        load_words<G>(kraw, ksp + (LATE ? ksb_off : 0) + ksb_lane);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             if (DT == 0) {
@@ -445,17 +466,17 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
         ++k_loaded;
         if (k_loaded < my_tiles) {  // wave-uniform: step to the same tile of the next page
             page_k += PSTEP;
-            kp = as_global(st.pt[page_k].k) + k_off;
-            ksp = as_global(st.pt[page_k].ksb) + ksb_off;
+            kp = as_global(pt[page_k].k) + (LATE ? 0 : k_off);
+            ksp = as_global(pt[page_k].ksb) + (LATE ? 0 : ksb_off);
             slot_next += PAGE * PSTEP;
             base_next += PAGE * PSTEP;
         }
     };
     auto load_v = [&](T &t) {
 #pragma unroll
-        for (int h = 0; h < NH; ++h) load_words<T::VW>(t.v[h], vp + v_lane + (size_t)h * 64 * VROW);
+        for (int h = 0; h < NH; ++h) load_words<T::VW>(t.v[h], vp + (LATE ? v_off : 0) + v_lane + (size_t)h * 64 * VROW);
         uint32_t vraw[G];
-        load_words<G>(vraw, vsp + vsb_lane);
+        load_words<G>(vraw, vsp + (LATE ? vsb_off : 0) + vsb_lane);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             if (DT == 0) {
@@ -469,8 +490,8 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
         ++v_loaded;
         if (v_loaded < my_tiles) {
             page_v += PSTEP;
-            vp = as_global(st.pt[page_v].v) + v_off;
-            vsp = as_global(st.pt[page_v].vsb) + vsb_off;
+            vp = as_global(pt[page_v].v) + (LATE ? 0 : v_off);
+            vsp = as_global(pt[page_v].vsb) + (LATE ? 0 : vsb_off);
         }
     };
     auto load_tile = [&](T &t) {
@@ -631,28 +652,43 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     // halves skewed: V of a tile is requested before its QK^T and softmax, K of the next
     // tile before its PV, so each half has the other half's arithmetic to arrive in.
     constexpr bool PREFETCH = (RG == 1 && !(BITS == 8 && D >= 128)) || (BITS == 4 && D <= 128 && (RG == 2 || D == 64));
+    T first;
+    auto request_first = [&]() __attribute__((always_inline)) {
+        if constexpr (PREFETCH) load_tile(first);
+        else load_k(first);
+    };
+    if (my_tiles > 0) request_first();
+    if constexpr (rot) {
+        step.turn(a.turn, bh, R, rot_s);
+        __syncthreads();
+    }
+    if constexpr (MM == 0 && RG == 1) {
+        if (own) {  // wave-uniform
+            write_row();
+            if (my_tiles == 1) {  // (then no pointer has moved on)
+                k_loaded = v_loaded = 0;
+                request_first();
+            }
+        }
+    }
     if (my_tiles > 0) {
+        load_queries();
         if constexpr (PREFETCH) {
-            T bufA, bufB;
-            load_tile(bufA);
-            load_queries();
+            T bufB;
             for (int done = 0;;) {
                 load_tile(bufB);
-                compute_tile(bufA);
+                compute_tile(first);
                 if (++done == my_tiles) break;
-                load_tile(bufA);
+                load_tile(first);
                 compute_tile(bufB);
                 if (++done == my_tiles) break;
             }
         } else {
-            T buf;
-            load_k(buf);
-            load_queries();
             for (int done = 0; done < my_tiles; ++done) {
-                load_v(buf);
-                compute_qk_softmax(buf);
-                load_k(buf);
-                compute_pv(buf);
+                load_v(first);
+                compute_qk_softmax(first);
+                load_k(first);
+                compute_pv(first);
             }
         }
     }
@@ -761,14 +797,12 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
     // the end) for the wavefronts to fetch them.
     uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
-    if constexpr (rot) {
-        rope_stage_step<DT, D>(a.turn, bh, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
-                                static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R, rot_s);
-        __syncthreads();
-    }
+    [[maybe_unused]] RopeStep<DT, D, WAVES * 64, RR> step;
+    if constexpr (rot)
+        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
+                   static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R);
 
     // query operands: lane (blk, qi) holds row qi's elements 4*(16 x + blk) .. +3, unscaled
-    // (fetched by the main loop after it has requested its first two pieces; MODE 3's loads start behind the rotation)
     Op qa[RG][NP];
     auto load_queries = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -819,48 +853,23 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     }
     const int tile0 = tile_begin + wave;
     const int my_tiles = tile0 < tile_end ? (tile_end - tile0 + WAVES - 1) / WAVES : 0;
-    // ---- the step's new row, when it is still to be written (unmasked single-token decode) -----
-    // Exactly one wavefront of one workgroup reads the tile of physical slot `new_slot` (spans are equal and
-    // cover every tile): it copies the row into the page before it requests any tile, so its own later
-    // loads of the tile see it.
-    if constexpr (MM == 0) {
-        if (a.new_k != nullptr) {  // wave-uniform
-            const int slot = a.new_slot, tl = slot >> 6;
-            if (tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % WAVES) == wave) {
-                const uint16_t *krow = static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D;
-                const uint16_t *vrow = static_cast<const uint16_t *>(a.new_v) + (size_t)bh * D;
-                char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot));
-                char *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
-                if (lane < D / 8)  // one 16-byte chunk of the K row per lane
-                    *reinterpret_cast<uint4 *>(kc + kfp_off(st, slot, 8 * lane)) =
-                        rot ? *reinterpret_cast<const uint4 *>(rot_s + R * D + 8 * lane) : *reinterpret_cast<const uint4 *>(krow + 8 * lane);
-                for (int d = lane; d < D; d += 64)
-                    *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, d)) = vrow[d];
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            }
-        }
-    }
     // a wavefront's tiles are a page apart: each is found through the page table (a scalar load)
     const int tip = tile0 & 3;
     int page_k = my_tiles > 0 ? tile0 >> 2 : 0, page_v = page_k;
     constexpr int VROW = TILE * 2;  // bytes of one V tile row
     const size_t k_off = (size_t)bh * st.k_cell + (size_t)tip * TILE * st.k_row;
     const size_t v_off = (size_t)bh * st.v_cell + (size_t)tip * D * VROW;
-    // (plain pointers, hence FLAT loads, on purpose: as GLOBAL loads with a scalar base the short launches
-    // of this kernel measured 0.4-1 us slower -- 19.1 against 18.7 us on a 4096-row ring at D = 256,
-    // 10.4-11.2 against 9.1-10.1 us at 1024 rows of D = 128 -- and the long ones the same)
-    const char *kp = st.pt[page_k].k + k_off;
-    const char *vp = st.pt[page_k].v + v_off;
+    const ptab pt = page_table(st);
+    gptr kp = as_global(pt[page_k].k), vp = as_global(pt[page_v].v);
     // chunk-interleaved tiles: chunk j of the lane's token (K) or column (V) sits 16 * lane bytes into
     // a 1 KB (K) / 16 D byte (V) row of chunks, so every load below is contiguous across the wavefront
     const uint32_t k_lane = lane * 16, v_lane = lane * 16;
     int slot_cur = tile0 * TILE + lane;
     int k_loaded = 0, v_loaded = 0;  // tiles whose K / V pieces have been requested
-    auto load_chunks = [&](uint32_t *buf, const char *p, size_t stride) __attribute__((always_inline)) {
+    auto load_chunks = [&](uint32_t *buf, gptr p, size_t stride) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < PW / 4; ++j) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(p + (size_t)j * stride);
+            const kv_u4 v = ld_global<kv_u4>(p + (size_t)j * stride);
             buf[4 * j] = v.x; buf[4 * j + 1] = v.y; buf[4 * j + 2] = v.z; buf[4 * j + 3] = v.w;
         }
     };
@@ -869,17 +878,17 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     // after the last piece the pointer steps to this wavefront's next tile (clamped, so
     // the prefetch past the end stays unconditional and in bounds)
     auto load_k = [&](uint32_t *buf, int x) {
-        load_chunks(buf, kp + k_lane + (size_t)x * (PW / 4) * (TILE * 16), TILE * 16);  // chunks 8x .. 8x+7 of the lane's token
+        load_chunks(buf, kp + k_off + k_lane + (size_t)x * (PW / 4) * (TILE * 16), TILE * 16);  // chunks 8x .. 8x+7 of the lane's token
         if (x == NP - 1) {
             ++k_loaded;
-            if (k_loaded < my_tiles) kp = st.pt[++page_k].k + k_off;
+            if (k_loaded < my_tiles) kp = as_global(pt[++page_k].k);
         }
     };
     auto load_v = [&](uint32_t *buf, int x) {
-        load_chunks(buf, vp + v_lane + (size_t)x * 64 * 16, (size_t)D * 16);  // the 8 token chunks of column 64x + lane
+        load_chunks(buf, vp + v_off + v_lane + (size_t)x * 64 * 16, (size_t)D * 16);  // the 8 token chunks of column 64x + lane
         if (x == NP - 1) {
             ++v_loaded;
-            if (v_loaded < my_tiles) vp = st.pt[++page_v].v + v_off;
+            if (v_loaded < my_tiles) vp = as_global(pt[++page_v].v);
         }
     };
 
@@ -897,12 +906,63 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
         else load_v(buf, n - NP);
     };
 
-    if (my_tiles > 0) {
-        // (the queries first: loads complete in order, and a wait for queries requested after the
-        // first pieces would be a wait for those pieces too -- in every iteration, the compiler
-        // placing one wait for all ways into the loop)
-        load_queries();
+    // ---- the step's new row, when it is still to be written (unmasked single-token decode) -----
+    // Exactly one wavefront of one workgroup reads the tile of physical slot `new_slot` (spans are equal and
+    // cover every tile): it copies the row into the page after it has requested its first pieces and before it requests
+    // others, so its own later loads of the tile see it; if its first tile is that tile, it requests them again.  The row
+    // is requested in front of the pieces.
+    bool own = false;
+    kv_u4 own_k;
+    uint16_t own_v[NP];
+    if constexpr (MM == 0) {
+        if (a.new_k != nullptr) {  // wave-uniform
+            const int tl = a.new_slot >> 6;
+            own = tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % WAVES) == wave;
+            if (own) {
+                if constexpr (!rot) {  // one 16-byte chunk of the K row per lane
+                    if (lane < D / 8) own_k = ld_global<kv_u4>(as_global(a.new_k) + ((size_t)bh * D + 8 * lane) * 2);
+                }
+#pragma unroll
+                for (int h = 0; h < NP; ++h) own_v[h] = ld_global<uint16_t>(as_global(a.new_v) + ((size_t)bh * D + 64 * h + lane) * 2);
+            }
+        }
+    }
+    // (the queries before the pieces: loads complete in order, and a wait for queries requested after the
+    // first pieces would be a wait for those pieces too -- in every iteration, the compiler
+    // placing one wait for all ways into the loop)
+    auto request_first = [&]() __attribute__((always_inline)) {
         static_for<NBUF>([&](auto N) { request(buf_of(decltype(N)::value), decltype(N)::value); });
+    };
+    if (my_tiles > 0) {
+        if constexpr (!rot) load_queries();
+        request_first();
+    }
+    if constexpr (rot) {
+        step.turn(a.turn, bh, R, rot_s);
+        __syncthreads();
+        if (my_tiles > 0) load_queries();
+    }
+    if constexpr (MM == 0) {
+        if (own) {  // wave-uniform
+            const int slot = a.new_slot;
+            char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot));
+            char *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
+            if (lane < D / 8)
+                *reinterpret_cast<kv_u4 *>(kc + kfp_off(st, slot, 8 * lane)) = rot ? *reinterpret_cast<const kv_u4 *>(rot_s + R * D + 8 * lane) : own_k;
+#pragma unroll
+            for (int h = 0; h < NP; ++h) *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, 64 * h + lane)) = own_v[h];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            if (tile0 == slot >> 6) {
+                k_loaded = v_loaded = 0;
+                page_k = page_v = tile0 >> 2;
+                kp = as_global(pt[page_k].k);
+                vp = as_global(pt[page_v].v);
+                request_first();
+            }
+        }
+    }
+    if (my_tiles > 0) {
         for (int done = 0; done < my_tiles; ++done) {
             int row;
             if (IDENT) row = slot_cur;

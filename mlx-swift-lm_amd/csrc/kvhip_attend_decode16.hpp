@@ -184,11 +184,10 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
     // the end) for the wavefronts to fetch them.
     uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
-    if constexpr (rot) {
-        rope_stage_step<DT, DK>(a.turn, bh, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * DK,
-                                static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK, R, rot_s);
-        __syncthreads();
-    }
+    [[maybe_unused]] RopeStep<DT, DK, WAVES * 64, RR> step;
+    if constexpr (rot)
+        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * DK,
+                   static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK, R);
     // ---- span of this workgroup (as in the 4-row kernel) -----------------------------------
     if constexpr (MM == 1) {
         // a ragged batch whose rows divide their own ranges over the same number of spans: long and short
@@ -227,36 +226,61 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     const bool row_ok = n < R;
 
     // ---- the step's new row, when it is still to be written (unmasked single-token step) --------
-    // Its slot lies in the last tile, which exactly one wavefront of one workgroup reads: that wavefront
-    // quantizes the row into the cache before it requests any tile, with the arithmetic of the append kernel,
-    // so its own later loads of the tile (and of the tile's scale / bias pairs) see it.  A lane owns the V
-    // columns it quantizes; their codes go into the columns' tile rows read-modify-write (a code of a bit
-    // stream may lie across two dwords).
+    // Its slot lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one: that wavefront
+    // quantizes the row into the cache, with the arithmetic of the append kernel, after it has requested its first tile and
+    // before it requests another, so its own later loads of the row's tile (and of the tile's scale / bias pairs) see it; if
+    // its first tile is that tile, it requests it again.  A lane owns the V columns it quantizes; their codes go into the
+    // columns' tile rows read-modify-write (a code of a bit stream may lie across two dwords).  The row and the old words
+    // are requested in front of the tile.
+    constexpr int NHK = (DK + 63) / 64, NHV = (DV + 63) / 64;
+    bool own = false;
+    uint16_t own_k[NHK], own_v[NHV];
+    uint32_t own_w[NHV][2];
     if constexpr (MM == 0) {
         if (a.new_k != nullptr) {  // wave-uniform
             const int slot = a.new_slot, tl = slot >> 6;
-            if (tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % WAVES) == wave) {
-                const char *krow = static_cast<const char *>(a.new_k) + (size_t)bh * DK * 2;
-                const char *vrow = static_cast<const char *>(a.new_v) + (size_t)bh * DV * 2;
-                quantize_row_wave_from<DT, BITS>([&](int d) { return rot ? Elem<DT>::load(rot_s, R * DK + d) : Elem<DT>::load(krow, d); }, DK, GS, lane,
-                                                 reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))),
-                                                 [](int, uint32_t) {}, const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
-                char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
-                const int bp = v_bitpos<BITS>(slot & (TILE - 1)), sh = bp & 31;
-                constexpr uint32_t M = (1u << BITS) - 1u;
-                quantize_row_wave_from<DT, BITS>(
-                    [&](int d) { return Elem<DT>::load(vrow, d); }, DV, GS, lane, nullptr,
-                    [&](int d, uint32_t code) {
-                        uint32_t *p = reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d)) + (bp >> 5);
-                        p[0] = (p[0] & ~(M << sh)) | (code << sh);
-                        if ((32 % BITS) != 0 && sh + BITS > 32) p[1] = (p[1] & ~(M >> (32 - sh))) | (code >> (32 - sh));
-                    },
-                    const_cast<char *>(vsb_row_ptr(st, bh, slot)), nullptr, nullptr);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            own = tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % WAVES) == wave;
+            if (own) {
+                const uint16_t *krow = static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK;
+                const uint16_t *vrow = static_cast<const uint16_t *>(a.new_v) + (size_t)bh * DV;
+                const char *vcell = v_cell_ptr(st, bh, slot);
+                const int bp = v_bitpos<BITS>(slot & (TILE - 1));
+                const bool second = (32 % BITS) != 0 && (bp & 31) + BITS > 32;
+#pragma unroll
+                for (int h = 0; h < NHK; ++h)
+                    if (!rot && 64 * h + lane < DK) own_k[h] = krow[64 * h + lane];
+#pragma unroll
+                for (int h = 0; h < NHV; ++h)
+                    if (64 * h + lane < DV) {
+                        const uint32_t *p = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, 64 * h + lane)) + (bp >> 5);
+                        own_v[h] = vrow[64 * h + lane];
+                        own_w[h][0] = p[0];
+                        if (second) own_w[h][1] = p[1];
+                    }
             }
         }
     }
+    auto write_row = [&]() __attribute__((always_inline)) {
+        const int slot = a.new_slot;
+        quantize_row_wave_from<DT, BITS>(
+            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * DK + d) : Elem<DT>::load(&own_k[(d - lane) >> 6], 0); }, DK, GS, lane,
+            reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))), [](int, uint32_t) {},
+            const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
+        char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
+        const int bp = v_bitpos<BITS>(slot & (TILE - 1)), sh = bp & 31;
+        constexpr uint32_t M = (1u << BITS) - 1u;
+        quantize_row_wave_from<DT, BITS>(
+            [&](int d) { return Elem<DT>::load(&own_v[(d - lane) >> 6], 0); }, DV, GS, lane, nullptr,
+            [&](int d, uint32_t code) {
+                uint32_t *p = reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d)) + (bp >> 5);
+                const uint32_t (&old)[2] = own_w[(d - lane) >> 6];
+                p[0] = (old[0] & ~(M << sh)) | (code << sh);
+                if ((32 % BITS) != 0 && sh + BITS > 32) p[1] = (old[1] & ~(M >> (32 - sh))) | (code >> (32 - sh));
+            },
+            const_cast<char *>(vsb_row_ptr(st, bh, slot)), nullptr, nullptr);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
 
     // ---- per-lane addresses inside a tile; tiles of one wavefront are a page apart -----------
     // K block tb, lane (n, jj): row of token tok(tb, n) = 16 (n / 4) + 4 tb + n % 4, segment jj
@@ -277,7 +301,8 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     // are issued and its latency passes behind the tile's arithmetic.  (Adding the lane's offset as soon
     // as the entry arrived put a wait for the scalar load into every tile: 44 -> 50 us on a ragged
     // batch of 16 rows.)
-    gptr kb = as_global(st.pt[page_k].k), vb = as_global(st.pt[page_k].v), ksb_b = as_global(st.pt[page_k].ksb), vsb_b = as_global(st.pt[page_k].vsb);
+    const ptab pt = page_table(st);
+    gptr kb = as_global(pt[page_k].k), vb = as_global(pt[page_k].v), ksb_b = as_global(pt[page_k].ksb), vsb_b = as_global(pt[page_k].vsb);
     int base_next = tile0 * TILE;
 
     struct Tile {
@@ -302,8 +327,8 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         ++sb_issued;
         if (sb_issued < my_tiles) {
             ++page_sb;
-            ksb_n = as_global(st.pt[page_sb].ksb);
-            vsb_n = as_global(st.pt[page_sb].vsb);
+            ksb_n = as_global(pt[page_sb].ksb);
+            vsb_n = as_global(pt[page_sb].vsb);
         }
     };
     // (SB_LDS) the pairs of tokens 4 tb .. 4 tb + 3 of the lane group, side 0 K (G = GK) / 1 V (G = GV): out[i * G + g]
@@ -357,8 +382,8 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         ++k_loaded;
         if (k_loaded < my_tiles) {  // wave-uniform: the same tile of the next page
             ++page_k;
-            kb = as_global(st.pt[page_k].k);
-            if constexpr (!SB_LDS) ksb_b = as_global(st.pt[page_k].ksb);
+            kb = as_global(pt[page_k].k);
+            if constexpr (!SB_LDS) ksb_b = as_global(pt[page_k].ksb);
             base_next += PAGE;
         }
     };
@@ -389,8 +414,8 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         ++v_loaded;
         if (v_loaded < my_tiles) {
             ++page_v;
-            vb = as_global(st.pt[page_v].v);
-            if constexpr (!SB_LDS) vsb_b = as_global(st.pt[page_v].vsb);
+            vb = as_global(pt[page_v].v);
+            if constexpr (!SB_LDS) vsb_b = as_global(pt[page_v].vsb);
         }
     };
 
@@ -632,10 +657,26 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
 
     // one buffer with the halves skewed: V of a tile is requested before its scores, K of the
     // next tile before its PV
-    if (my_tiles > 0) {
-        Tile buf;
+    Tile buf;
+    auto request_first = [&]() __attribute__((always_inline)) {
         if constexpr (SB_LDS) dma_sb();
         load_k(buf);
+    };
+    if (my_tiles > 0) request_first();
+    if constexpr (rot) {
+        step.turn(a.turn, bh, R, rot_s);
+        __syncthreads();
+    }
+    if constexpr (MM == 0) {
+        if (own) {  // wave-uniform
+            write_row();
+            if (my_tiles == 1) {  // (then no pointer has moved on)
+                k_loaded = v_loaded = sb_issued = 0;
+                request_first();
+            }
+        }
+    }
+    if (my_tiles > 0) {
         load_queries();
         for (int done = 0; done < my_tiles; ++done) {
             if constexpr (SB_LDS) {
@@ -651,9 +692,6 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
             load_k(buf);
             compute_pv(buf);
         }
-    } else {
-#pragma unroll
-        for (int g = 0; g < GK; ++g) qsum[g] = 0.f;
     }
 
     if (rot) __syncthreads();  // (the rotated rows have been fetched)

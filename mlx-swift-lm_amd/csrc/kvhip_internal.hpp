@@ -85,18 +85,24 @@ struct MaskDev {
 
 #if defined(__HIPCC__)
 // ---- device-side address helpers -------------------------------------------
-// A wave-uniform slot makes the table lookup a scalar load.
+// The page table as a kernel that walks a cache reads it: constant memory (address space 4), which no kernel that reads
+// it also writes.  A wave-uniform slot then makes the lookup a scalar load wherever it stands.  Through the plain pointer
+// it is one only as long as the kernel has not stored anything before it: in the decode kernels that write the step's new
+// row themselves every lookup came out as a vector load with a wait for all loads in flight, the next tile's among them.
+#define KV_CONST __attribute__((address_space(4)))
+typedef const KV_CONST PageEntry *ptab;
+__device__ __forceinline__ ptab page_table(const Store &st) { return (ptab) reinterpret_cast<uintptr_t>(st.pt); }
 __device__ __forceinline__ const char *k_row_ptr(const Store &st, int bh, int slot) {
-    return st.pt[slot >> PAGE_SHIFT].k + (size_t)bh * st.k_cell + (size_t)(slot & (PAGE - 1)) * st.k_row;
+    return page_table(st)[slot >> PAGE_SHIFT].k + (size_t)bh * st.k_cell + (size_t)(slot & (PAGE - 1)) * st.k_row;
 }
 __device__ __forceinline__ const char *ksb_row_ptr(const Store &st, int bh, int slot) {
-    return st.pt[slot >> PAGE_SHIFT].ksb + (size_t)bh * st.ksb_cell + (size_t)(slot & (PAGE - 1)) * st.ksb_row;
+    return page_table(st)[slot >> PAGE_SHIFT].ksb + (size_t)bh * st.ksb_cell + (size_t)(slot & (PAGE - 1)) * st.ksb_row;
 }
 __device__ __forceinline__ const char *vsb_row_ptr(const Store &st, int bh, int slot) {
-    return st.pt[slot >> PAGE_SHIFT].vsb + (size_t)bh * st.vsb_cell + (size_t)(slot & (PAGE - 1)) * st.vsb_row;
+    return page_table(st)[slot >> PAGE_SHIFT].vsb + (size_t)bh * st.vsb_cell + (size_t)(slot & (PAGE - 1)) * st.vsb_row;
 }
 __device__ __forceinline__ const char *v_cell_ptr(const Store &st, int bh, int slot) {
-    return st.pt[slot >> PAGE_SHIFT].v + (size_t)bh * st.v_cell;
+    return page_table(st)[slot >> PAGE_SHIFT].v + (size_t)bh * st.v_cell;
 }
 // Full-precision pages are interleaved in 16-byte chunks inside every 64-token tile, so that a
 // wavefront whose lanes are the 64 tokens (K) or 64 adjacent columns (V) reads 1 KB contiguous
@@ -113,7 +119,7 @@ __device__ __forceinline__ size_t vfp_off(const Store &st, int slot, int d) {
     return (size_t)(t >> 6) * ((size_t)TILE * st.Dv * st.es) + ((size_t)(tk / epc) * st.Dv + d) * 16 + (size_t)(tk % epc) * st.es;
 }
 __device__ __forceinline__ const char *k_cell_ptr(const Store &st, int bh, int slot) {
-    return st.pt[slot >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;
+    return page_table(st)[slot >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;
 }
 // A pointer taken from the page table is a plain `char *` to the compiler, which then emits FLAT loads
 // for it: those count on both the vector-memory and the LDS/scalar counter, and since they may
@@ -140,11 +146,11 @@ struct PageCursor {
     PageEntry e;
     __device__ __forceinline__ void fetch(const Store &st, int p) {
         page = p;
-        const PageEntry &src = st.pt[p];
-        e.k = wave_uniform(src.k);
-        e.ksb = wave_uniform(src.ksb);
-        e.v = wave_uniform(src.v);
-        e.vsb = wave_uniform(src.vsb);
+        const ptab src = page_table(st) + p;
+        e.k = wave_uniform(src->k);
+        e.ksb = wave_uniform(src->ksb);
+        e.v = wave_uniform(src->v);
+        e.vsb = wave_uniform(src->vsb);
     }
     // starts on the page of `slot` (any slot the kernel may read: the entry is valid from the start)
     __device__ __forceinline__ PageCursor(const Store &st, int slot) { fetch(st, __builtin_amdgcn_readfirstlane(slot >> PAGE_SHIFT)); }

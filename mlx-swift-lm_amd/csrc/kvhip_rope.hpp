@@ -215,31 +215,56 @@ __device__ __forceinline__ void rope_chunk(const RopeDev &r, const float *inv_s,
 
 // ---- one token's rows, for the decode kernels --------------------------------------------------------------------
 // The R query rows (adjacent, D elements) and the key row of one kv head, rotated and rounded to the dtype, into LDS
-// [R + 1][D]; the caller synchronises.  A thread owns one pair of columns and forms its sine and cosine once; all 256
-// (512) threads of the workgroup take part.  Every workgroup of the launch does this for itself, in front of its
-// first key loads: 0.9 to 1.4 us (4 bits, 32 query and 8 kv heads of 128: 7.5 -> 8.9 us over 6000 keys of one sequence,
-// 12.6 -> 13.5 over 30 000, 18.8 -> 19.7 over 8000 of batch 8), where a launch for it takes 4 to 6.5 us.
-template <int DT, int D>
-__device__ __forceinline__ void rope_stage_step(const RopeDev &r, int bh, const uint16_t *q, const uint16_t *k, int R, uint16_t *dst) {
-    constexpr int P = D / 2;
-    const int p = threadIdx.x % P, ns = blockDim.x / P, half = r.dims >> 1;
-    const bool turn = p < half;
-    const int d0 = !turn ? r.dims + 2 * (p - half) : r.traditional ? 2 * p : p;
-    const int d1 = turn && !r.traditional ? d0 + half : d0 + 1;
-    float sn = 0.f, cs = 1.f;
-    if (turn) rope_sincos<false>(rope_angle(r, rope_pos(r, bh, 0), rope_inv_freq(r, p)), sn, cs);
-    for (int i = threadIdx.x / P; i <= R && threadIdx.x < ns * P; i += ns) {
-        const uint16_t *row = i < R ? q + (size_t)i * D : k;
-        uint16_t x = row[d0], y = row[d1];
-        if (turn) {
-            const float a = Elem<DT>::load(&x, 0), b = Elem<DT>::load(&y, 0);
-            Elem<DT>::store(&x, 0, rope_turn(a, b, true, sn, cs));
-            Elem<DT>::store(&y, 0, rope_turn(b, a, false, sn, cs));
+// [R + 1][D]; the caller synchronises.  A thread owns one pair of columns and forms its sine and cosine once; all THREADS
+// threads of the workgroup take part.  Every workgroup of the launch does this for itself, where a launch for it takes 4 to
+// 6.5 us.  In two halves: `fetch` requests the elements (of at most RMAX query rows) in front of the workgroup's first key
+// loads -- loads complete in order --, `turn` works the angles out and turns the rows while those keys are on their way.
+template <int DT, int D, int THREADS, int RMAX> struct RopeStep {
+    static constexpr int P = D / 2, NS = THREADS / P, NR = (RMAX + 1 + NS - 1) / NS;  // pairs of a row; rows at once; rows of a thread
+    static_assert(NS >= 1, "a thread per pair of columns");
+    int d0, d1;
+    bool rotates;
+    float freq;
+    using E = typename Elem<DT>::type;
+    E x[NR], y[NR];
+    __device__ __forceinline__ void fetch(const RopeDev &r, const E *q, const E *k, int R) {
+        const int p = threadIdx.x % P, half = r.dims >> 1;
+        rotates = p < half;
+        d0 = !rotates ? r.dims + 2 * (p - half) : r.traditional ? 2 * p : p;
+        d1 = rotates && !r.traditional ? d0 + half : d0 + 1;
+        freq = 1.f;
+        if (r.freqs && rotates) freq = r.freqs[p];
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            const int i = threadIdx.x / P + j * NS;
+            if (i <= R && threadIdx.x < NS * P) {
+                const E *row = i < R ? q + (size_t)i * D : k;
+                x[j] = row[d0];
+                y[j] = row[d1];
+            }
         }
-        dst[i * D + d0] = x;
-        dst[i * D + d1] = y;
     }
-}
+    __device__ __forceinline__ void turn(const RopeDev &r, int bh, int R, E *dst) {
+        float sn = 0.f, cs = 1.f;
+        if (rotates) {
+            const float inv = r.freqs ? 1.0f / freq : (float)exp(-(double)(int)(threadIdx.x % P) * r.log_base_over_half);
+            rope_sincos<false>(rope_angle(r, rope_pos(r, bh, 0), inv), sn, cs);
+        }
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            const int i = threadIdx.x / P + j * NS;
+            if (i <= R && threadIdx.x < NS * P) {
+                if (rotates) {
+                    const float a = Elem<DT>::load(&x[j], 0), b = Elem<DT>::load(&y[j], 0);
+                    Elem<DT>::store(&x[j], 0, rope_turn(a, b, true, sn, cs));
+                    Elem<DT>::store(&y[j], 0, rope_turn(b, a, false, sn, cs));
+                }
+                dst[i * D + d0] = x[j];
+                dst[i * D + d1] = y[j];
+            }
+        }
+    }
+};
 
 // ---- the queries of a forward ----------------------------------------------------------------------------------
 // One row position (batch row b, row l of L) of `x` [B, H, L, D] into `out` (which may be x) for heads [h0, h1): a
