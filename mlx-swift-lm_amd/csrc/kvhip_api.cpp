@@ -420,15 +420,14 @@ kvhip_status ensure_slots(kvhip_cache *c, int64_t slots, hipStream_t stream, boo
     }
     if (e != hipSuccess)
         return fail(KVHIP_ERR_HIP, std::string("hipMalloc of ") + std::to_string(bytes) + " bytes of cache pages failed: " + hipGetErrorString(e));
-    // packed V words are merged read-modify-write: new pages start from zero
-    KV_HIP_OR(launch_fill_zero(base, bytes, stream), (void)hipFree(base));
     PageEntry first;
     char *p = static_cast<char *>(base);
     first.k = p;
     first.v = p + part[0];
     first.ksb = st.ksb_cell ? p + part[0] + part[1] : nullptr;
     first.vsb = st.vsb_cell ? p + part[0] + part[1] + part[2] : nullptr;
-    KV_HIP_OR(launch_set_pages(const_cast<PageEntry *>(st.pt), (int)c->cap_pages, (int)add, first, stride, stream), (void)hipFree(base));
+    // packed V words are merged read-modify-write: new pages start from zero
+    KV_HIP_OR(launch_set_pages(base, bytes, const_cast<PageEntry *>(st.pt), (int)c->cap_pages, (int)add, first, stride, stream), (void)hipFree(base));
     Slab sl;
     sl.base = base;
     sl.first_page = c->cap_pages;
@@ -1154,7 +1153,7 @@ kvhip_status attend_dequant_first(kvhip_cache *c, const AttendArgs &a, hipStream
     } else {  // float32 scales: the page table, then the element-wise pass over whole tiles (what lies past the
               // presented rows in the last tile is zeros or rows trimmed earlier: finite values the kernel weighs with 0)
         const size_t stride4[4] = {stride[0], stride[1], 0, 0};
-        e = launch_set_pages(const_cast<PageEntry *>(t.pt), 0, (int)pages, first, stride4, s);
+        e = launch_set_pages(nullptr, 0, const_cast<PageEntry *>(t.pt), 0, (int)pages, first, stride4, s);
         const int rows_up = (int)std::min<int64_t>(pages * PAGE, ((int64_t)a.T + TILE - 1) / TILE * TILE);
         if (e == hipSuccess) e = launch_dequant_pages(a.st, t, rows_up, s);
     }

@@ -278,14 +278,14 @@ hipError_t launch_affine_dequantize(const uint32_t *wq, const void *scales, cons
                                     int64_t rows, int D, int gs, int bits, int dtype, void *dst,
                                     hipStream_t s);
 hipError_t launch_mask_materialize(const kvhip_mask_plan_t &plan, uint8_t *dst, hipStream_t s);
-// Zero / copy `bytes` of device memory with a kernel (16-byte aligned pointers and sizes).
-hipError_t launch_fill_zero(void *dst, size_t bytes, hipStream_t s);
+// Copy `bytes` of device memory with a kernel (16-byte aligned pointers and sizes).
 hipError_t launch_copy_bytes(void *dst, const void *src, size_t bytes, hipStream_t s);
 // `rows` dense rows of src_pitch bytes into rows of dst_pitch bytes (both even): common prefix copied, rest zero-filled
 hipError_t launch_repitch_rows(void *dst, size_t dst_pitch, const void *src, size_t src_pitch, size_t rows, hipStream_t s);
 // Page-table entries [first, first + count): page first + i keeps its cells at base.x + i * stride.x
-// for each plane x (pages backed by one allocation lie at a regular stride).
-hipError_t launch_set_pages(PageEntry *pt, int first, int count, PageEntry base, const size_t stride[4], hipStream_t s);
+// for each plane x (pages backed by one allocation lie at a regular stride); `clear` not null: its `bytes` (multiples of 16)
+// are cleared by the same launch.
+hipError_t launch_set_pages(void *clear, size_t bytes, PageEntry *pt, int first, int count, PageEntry base, const size_t stride[4], hipStream_t s);
 // Every plane of pages [0, pages) of `src` into the same pages of `dst` (stores of one geometry).
 hipError_t launch_copy_pages(const Store &src, const Store &dst, int pages, hipStream_t s);
 

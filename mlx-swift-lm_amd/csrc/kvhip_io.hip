@@ -1086,25 +1086,25 @@ hipError_t launch_affine_dequantize(const uint32_t *wq, const void *scales, cons
 // Plain fills and copies of plane memory run as kernels: they see virtual addresses only, so a
 // range may span any number of separately mapped physical chunks, and no memset node ends up in
 // a stream capture.  16-byte aligned pointers and sizes.
-__global__ void __launch_bounds__(256) fill_zero_kernel(u4v *dst, size_t n16) {
-    const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) dst[i] = u4v{0u, 0u, 0u, 0u};
-}
 __global__ void __launch_bounds__(256) copy_bytes_kernel(u4v *dst, const u4v *src, size_t n16) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) dst[i] = src[i];
 }
 
-// one thread per new page-table entry
-__global__ void set_pages_kernel(PageEntry *pt, int first, int count, PageEntry base, size_t sk, size_t sv, size_t sksb, size_t svsb) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    PageEntry e;
-    e.k = base.k + (size_t)i * sk;
-    e.v = base.v + (size_t)i * sv;
-    e.ksb = base.ksb ? base.ksb + (size_t)i * sksb : nullptr;
-    e.vsb = base.vsb ? base.vsb + (size_t)i * svsb : nullptr;
-    pt[first + i] = e;
+// New pages: the memory behind them cleared and their entries put into the table, a thread to an entry, in one launch (a
+// launch of its own for the entries held the next kernel up by 3 us).  `dst` may be null: entries only.
+__global__ void __launch_bounds__(256) set_pages_kernel(u4v *dst, size_t n16, PageEntry *pt, int first, int count, PageEntry base, size_t sk, size_t sv,
+                                                        size_t sksb, size_t svsb) {
+    const size_t stride = (size_t)gridDim.x * 256, tid = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = tid; i < (size_t)count; i += stride) {
+        PageEntry e;
+        e.k = base.k + i * sk;
+        e.v = base.v + i * sv;
+        e.ksb = base.ksb ? base.ksb + i * sksb : nullptr;
+        e.vsb = base.vsb ? base.vsb + i * svsb : nullptr;
+        pt[first + i] = e;
+    }
+    for (size_t i = tid; i < n16; i += stride) dst[i] = u4v{0u, 0u, 0u, 0u};
 }
 
 // grid (pages, 4 planes): the [BH] cells of one plane of one page, 16 bytes per thread and step
@@ -1118,9 +1118,12 @@ __global__ void __launch_bounds__(256) copy_pages_kernel(Store src, Store dst) {
     for (size_t i = threadIdx.x; i < n16; i += 256) reinterpret_cast<u4v *>(to)[i] = reinterpret_cast<const u4v *>(from)[i];
 }
 
-hipError_t launch_set_pages(PageEntry *pt, int first, int count, PageEntry base, const size_t stride[4], hipStream_t s) {
+hipError_t launch_set_pages(void *clear, size_t bytes, PageEntry *pt, int first, int count, PageEntry base, const size_t stride[4], hipStream_t s) {
     if (count <= 0) return hipSuccess;
-    hipLaunchKernelGGL(set_pages_kernel, dim3((count + 63) / 64), dim3(64), 0, s, pt, first, count, base, stride[0], stride[1],
+    if (((uintptr_t)clear | bytes) & 15) return hipErrorInvalidValue;
+    const size_t n16 = clear ? bytes / 16 : 0;
+    const unsigned grid = (unsigned)std::min<size_t>((std::max(n16, (size_t)count) + 255) / 256, 256 * 16);
+    hipLaunchKernelGGL(set_pages_kernel, dim3(grid), dim3(256), 0, s, static_cast<u4v *>(clear), n16, pt, first, count, base, stride[0], stride[1],
                        stride[2], stride[3]);
     return hipGetLastError();
 }
@@ -1128,15 +1131,6 @@ hipError_t launch_set_pages(PageEntry *pt, int first, int count, PageEntry base,
 hipError_t launch_copy_pages(const Store &src, const Store &dst, int pages, hipStream_t s) {
     if (pages <= 0) return hipSuccess;
     hipLaunchKernelGGL(copy_pages_kernel, dim3(pages, src.bits ? 4 : 2), dim3(256), 0, s, src, dst);
-    return hipGetLastError();
-}
-
-hipError_t launch_fill_zero(void *dst, size_t bytes, hipStream_t s) {
-    if (bytes == 0) return hipSuccess;
-    if (((uintptr_t)dst | bytes) & 15) return hipErrorInvalidValue;
-    const size_t n16 = bytes / 16;
-    const unsigned grid = (unsigned)std::min<size_t>((n16 + 255) / 256, 256 * 16);
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(grid), dim3(256), 0, s, static_cast<u4v *>(dst), n16);
     return hipGetLastError();
 }
 
