@@ -417,14 +417,25 @@ __global__ void __launch_bounds__(256) dequant_units_kernel(Store q, Store dst, 
     }
 }
 
-// grid (tiles touched, BH), 256 threads: rows src0 .. src0 + n - 1 to slots slot0 .. slot0 + n - 1, which may start and
-// end inside a tile; 16-bit dtypes, Dk == 32 NCK, Dv == 32 NCV
+// grid (tiles touched x pieces of a tile, BH), 256 threads: rows src0 .. src0 + n - 1 to slots slot0 .. slot0 + n - 1, which
+// may start and end inside a tile; 16-bit dtypes, Dk == 32 NCK, Dv == 32 NCV.  A tile's K rows go in pieces of 8 to 32
+// tokens, a 16-byte chunk to a thread, its V rows in blocks of columns that are turned through LDS: many short workgroups,
+// whose loads are all in flight at once and whose threads form the sines of one chunk.  (A workgroup to a tile, as it was,
+// walked four to sixteen chunks a thread: 512 rows of 8 heads x 128 with the queries of 32, 11.3 us.)
+template <int NCK, int NCV> struct FpTile {
+    static constexpr int KT = NCK <= 2 ? 32 : NCK <= 4 ? 16 : 8;  // tokens of a K piece
+    static constexpr int KP = TILE / KT;
+    static constexpr int VC = NCV % 2 == 0 ? 64 : 32;             // columns of a V piece
+    static constexpr int VP = 32 * NCV / VC;
+    static constexpr int PIECES = KP + VP;
+};
 template <int NCK, int NCV>
 __global__ void __launch_bounds__(256)
 append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, int n, RopeDev rope) {
+    using P = FpTile<NCK, NCV>;
     constexpr int DK = 32 * NCK, D = 32 * NCV;
-    constexpr int TPRK = DK / 8, TPR = D / 8;
-    constexpr int VPW = D / 2 + 1;  // dword pitch of a token's V row in LDS (odd: column reads spread over banks)
+    constexpr int TPRK = DK / 8, TPR = P::VC / 8;  // chunks of a row, K and V (of the piece's columns)
+    constexpr int VPW = P::VC / 2 + 1;  // dword pitch of a token's V row in LDS (odd: column reads spread over banks)
     __shared__ uint32_t vt[TILE * VPW];
     __shared__ float inv_s[DK / 2];
     const int bh = blockIdx.y;
@@ -433,54 +444,51 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
         else rope_queries_ride<1>(rope, st.BH, inv_s);
         return;
     }
-    const int slot_t = (slot0 & ~(TILE - 1)) + blockIdx.x * TILE;
+    const int piece = blockIdx.x % P::PIECES;
+    const int slot_t = (slot0 & ~(TILE - 1)) + blockIdx.x / P::PIECES * TILE;
     const int l_t = src0 + slot_t - slot0;  // the row in the tile's first slot (before the first new row: t_lo > 0)
     // tokens [t_lo, t_hi) of the tile are new; the threads of the others repeat the nearest new row and write nothing
     const int t_lo = max(slot0 - slot_t, 0), t_hi = min(slot0 + n - slot_t, TILE);
-    const char *kbase = keys + ((ptrdiff_t)bh * L + l_t) * DK * 2;
-    const char *vbase = values + ((ptrdiff_t)bh * L + l_t) * D * 2;
     auto new_row = [&](int r) { return min(max(r, t_lo), t_hi - 1); };
-    char *kcell = st.pt[slot_t >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;  // a tile lies inside one page
-    u4v kraw[NCK], vraw[NCV];
-#pragma unroll
-    for (int e = 0; e < NCK; ++e) {
-        const int c = e * 256 + threadIdx.x, r = c / TPRK;
-        kraw[e] = *reinterpret_cast<const u4v *>(kbase + (ptrdiff_t)(c + (new_row(r) - r) * TPRK) * 16);
-    }
-#pragma unroll
-    for (int e = 0; e < NCV; ++e) {
-        const int c = e * 256 + threadIdx.x, r = c / TPR;
-        vraw[e] = *reinterpret_cast<const u4v *>(vbase + (ptrdiff_t)(c + (new_row(r) - r) * TPR) * 16);
-    }
-    if (rope.dims > 0) {
-        rope_inv_table(rope, inv_s);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int e = 0; e < NCK; ++e) {
-        const int c = e * 256 + threadIdx.x;
-        const int r = c / TPRK, d0 = (c - r * TPRK) * 8;
-        u4v k = kraw[e];
-        if (rope.dims > 0 && d0 < rope.dims) {
-            const int rn = new_row(r);
-            const int pos = rope_pos(rope, bh, l_t + rn);
-            const char *row = kbase + (ptrdiff_t)rn * DK * 2;
-            float w[8];
-            if (st.dtype == KVHIP_F16) {
-                unpack8<0>(k, row, d0, rope, inv_s, pos, w);
-                k = chunk_pack<0>(w);
-            } else {
-                unpack8<1>(k, row, d0, rope, inv_s, pos, w);
-                k = chunk_pack<1>(w);
+    if (piece < P::KP) {
+        if (piece * P::KT >= t_hi || (piece + 1) * P::KT <= t_lo) return;  // (workgroup-uniform)
+        const int r = piece * P::KT + threadIdx.x / TPRK, d0 = (threadIdx.x % TPRK) * 8, rn = new_row(r);
+        const bool live = threadIdx.x < P::KT * TPRK;
+        const char *row = keys + ((ptrdiff_t)bh * L + l_t + rn) * DK * 2;
+        u4v k{0u, 0u, 0u, 0u};
+        if (live) k = *reinterpret_cast<const u4v *>(row + 2 * d0);
+        if (rope.dims > 0) {
+            rope_inv_table(rope, inv_s);
+            __syncthreads();
+            if (live && d0 < rope.dims) {
+                const int pos = rope_pos(rope, bh, l_t + rn);
+                float w[8];
+                if (st.dtype == KVHIP_F16) {
+                    unpack8<0>(k, row, d0, rope, inv_s, pos, w);
+                    k = chunk_pack<0>(w);
+                } else {
+                    unpack8<1>(k, row, d0, rope, inv_s, pos, w);
+                    k = chunk_pack<1>(w);
+                }
             }
         }
-        if (r >= t_lo && r < t_hi) *reinterpret_cast<u4v *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
+        char *kcell = page_table(st)[slot_t >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;  // a tile lies inside one page
+        if (live && r >= t_lo && r < t_hi) *reinterpret_cast<u4v *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
+        return;
+    }
+    const int c0 = (piece - P::KP) * P::VC;  // first column
+    const char *vbase = values + ((ptrdiff_t)bh * L + l_t) * D * 2 + 2 * c0;
+    constexpr int NV = TILE * TPR / 256;  // chunks of a thread
+    u4v vraw[NV];
+#pragma unroll
+    for (int e = 0; e < NV; ++e) {
+        const int c = e * 256 + threadIdx.x, r = c / TPR;
+        vraw[e] = *reinterpret_cast<const u4v *>(vbase + (ptrdiff_t)new_row(r) * D * 2 + (c - r * TPR) * 16);
     }
 #pragma unroll
-    for (int e = 0; e < NCV; ++e) {
-        const int c = e * 256 + threadIdx.x;
-        const int r = c / TPR, d0 = (c - r * TPR) * 8;
-        uint32_t *vrow = &vt[r * VPW + d0 / 2];
+    for (int e = 0; e < NV; ++e) {
+        const int c = e * 256 + threadIdx.x, r = c / TPR;
+        uint32_t *vrow = &vt[r * VPW + (c - r * TPR) * 4];
         vrow[0] = vraw[e].x;
         vrow[1] = vraw[e].y;
         vrow[2] = vraw[e].z;
@@ -491,8 +499,8 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
     // consecutive threads take consecutive columns, so a chunk row is written contiguously
     char *cell = const_cast<char *>(v_cell_ptr(st, bh, slot_t));
     const uint16_t *vt16 = reinterpret_cast<const uint16_t *>(vt);
-    for (int c = threadIdx.x; c < D * 8; c += 256) {
-        const int c8 = c / D, d = c - c8 * D;
+    for (int c = threadIdx.x; c < P::VC * 8; c += 256) {
+        const int c8 = c / P::VC, d = c - c8 * P::VC;
         uint32_t out[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -500,7 +508,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
             const uint32_t hi = vt16[(8 * c8 + 2 * j + 1) * (2 * VPW) + d];
             out[j] = lo | (hi << 16);
         }
-        char *dst = cell + vfp_off(st, slot_t + 8 * c8, d);
+        char *dst = cell + vfp_off(st, slot_t + 8 * c8, c0 + d);
         if (8 * c8 >= t_lo && 8 * c8 + 8 <= t_hi) {
             *reinterpret_cast<u4v *>(dst) = u4v{out[0], out[1], out[2], out[3]};
         } else {
@@ -837,8 +845,12 @@ hipError_t launch_append_fp(const Store &st, const void *keys, const void *value
     // that takes 5 us whatever their number, less than a tile's workgroup behind its barriers.
     if (!tiled || n < TILE) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
     const int tiles = ((slot0 & (TILE - 1)) + n + TILE - 1) / TILE;
-    dim3 grid(tiles, st.BH + rope_ride_rows(r, tiles, st.es)), block(256);
-#define FP_TILE(NCK, NCV) hipLaunchKernelGGL((append_fp_tile_kernel<NCK, NCV>), grid, block, 0, s, st, (const char *)keys, (const char *)values, L, src0, slot0, n, r)
+#define FP_TILE(NCK, NCV)                                                                                                 \
+    do {                                                                                                                  \
+        const int gx = tiles * FpTile<NCK, NCV>::PIECES;                                                                  \
+        hipLaunchKernelGGL((append_fp_tile_kernel<NCK, NCV>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es)), dim3(256), 0, s, st, \
+                           (const char *)keys, (const char *)values, L, src0, slot0, n, r);                               \
+    } while (0)
     if (mla) FP_TILE(6, 4);
     else if (st.Dk == 64) FP_TILE(2, 2);
     else if (st.Dk == 96) FP_TILE(3, 3);
