@@ -32,6 +32,7 @@
 
 #include "kvhip_mask.hpp"
 #include "kvhip_rope.hpp"
+#include "kvhip_wave.hpp"
 
 // piece buffers of the full-precision decode kernel (at most the D / 32 pieces of one tile)
 #ifndef KVHIP_DECODE_FP_NBUF
@@ -52,7 +53,6 @@ union Op {  // one 4-element 16-bit operand
 };
 
 constexpr int WAVES = 4;
-constexpr float LOG2E = 1.4426950408889634f;
 constexpr float TWO24 = 16777216.0f;
 
 template <class F, int... I>
@@ -71,38 +71,6 @@ template <int ABID> __device__ __forceinline__ f4 mfma444_bf(const Op &a, const 
     return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(a.s, b.s, c, 4, ABID, 0);
 }
 
-// v_exp_f32 without the denormal-range fix-up (results below 2^-126 flush to zero)
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// Wavefront reductions on the data-parallel-primitive path (no LDS round trips): two quad
-// permutes and two row mirrors leave each row of 16 lanes reduced, two row broadcasts
-// carry the rows into lane 63, which is read out as a wave-uniform scalar.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_take(float v) {  // v of the lane CTRL names; own v outside ROWS
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v),
-                                                                 CTRL, ROWS, 0xF, false));
-}
-__device__ __forceinline__ float wave_max(float v) {
-    v = fmaxf(v, dpp_take<0xB1, 0xF>(v));   // quad_perm [1,0,3,2]
-    v = fmaxf(v, dpp_take<0x4E, 0xF>(v));   // quad_perm [2,3,0,1]
-    v = fmaxf(v, dpp_take<0x141, 0xF>(v));  // row_half_mirror
-    v = fmaxf(v, dpp_take<0x140, 0xF>(v));  // row_mirror
-    v = fmaxf(v, dpp_take<0x142, 0xA>(v));  // row_bcast15 into rows 1 and 3
-    v = fmaxf(v, dpp_take<0x143, 0xC>(v));  // row_bcast31 into rows 2 and 3
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
-__device__ __forceinline__ float wave_sum(float v) {
-    v += dpp_take<0xB1, 0xF>(v);
-    v += dpp_take<0x4E, 0xF>(v);
-    v += dpp_take<0x141, 0xF>(v);
-    v += dpp_take<0x140, 0xF>(v);
-    // the broadcast steps must add only into the rows they target
-    const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xA, 0xF, false));
-    v += r1;
-    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));
-    v += r2;
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
 __device__ __forceinline__ float uniform(float v) {  // v is the same in every lane
     return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
@@ -233,12 +201,23 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     const int split = blockIdx.x;
     int b = bh / a.Hkv;
     const int hk = bh - b * a.Hkv;
+    size_t part_slot = (size_t)bh * nsplit + split;  // where this workgroup's partial goes
+    [[maybe_unused]] RaggedSpan span;
+    [[maybe_unused]] int wid = 0;
     if constexpr (MM == 1) {
-        // a ragged batch whose rows divide their own ranges over the same number of spans: long and short
-        // rows are paired on the CUs (balanced_row); partials stay indexed by the batch row itself
-        if (tiles_per_wg == 0 && a.B <= 64 && a.B > 2) {
+        if (tiles_per_wg < 0) {  // a ragged batch that shares its spans out
+            const int wgs = nsplit * a.B;
+            wid = b * nsplit + split;
+            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, wgs, NW, wid, true);
+            if (span.count == 0) return;  // (workgroup-uniform)
+            part_slot = (size_t)hk * wgs + wid;
+            b = span.b;
+            bh = b * a.Hkv + hk;
+        } else if (tiles_per_wg == 0 && a.B <= 64 && a.B > 2) {
+            // rows of one span each: long and short ones are paired on the CUs; outputs stay the batch row's own
             b = __builtin_amdgcn_readfirstlane(balanced_row(a.mask, a.B, a.L, a.T, tiles_total, b));
             bh = b * a.Hkv + hk;
+            part_slot = (size_t)bh * nsplit + split;
         }
     }
     const int r = a.Hq / a.Hkv;
@@ -339,25 +318,21 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     if constexpr (MM == 1) {
         // length-aware partition: an index-only mask bounds the rows this (batch) can see
         // (left padding, lengths, causal/window reach); spans of equal size start at the first
-        // visible tile, so a ragged batch gets workgroups in proportion to each length
-        int vis_lo, vis_hi;
-        sym_mask_row_range(sym, vis_lo, vis_hi);
-        int t_lo = max(0, vis_lo) >> 6, t_hi = min(tiles_total, (min(vis_hi, a.T - 1) >> 6) + 1);
-        if (sym_mask_some_row_empty(sym)) {  // a fully masked row averages over every key
-            t_lo = 0;
-            t_hi = tiles_total;
-        }
+        // visible tile
+        const TileRange vis = visible_tiles(sym, tiles_total, true);
         // tiles_per_wg == 0: divide this batch row's own visible range over the spans
         const int per = tiles_per_wg > 0 ? tiles_per_wg
-                                         : (max(t_hi - t_lo, 1) + nsplit * NW - 1) / (nsplit * NW) * NW;
-        tile_begin = t_lo + split * per;  // spans past t_hi are empty
-        tile_end = min(t_hi, tile_begin + per);
+                                         : (max(vis.hi - vis.lo, 1) + nsplit * NW - 1) / (nsplit * NW) * NW;
+        tile_begin = tiles_per_wg < 0 ? span.t.lo : vis.lo + split * per;  // spans past the last tile are empty
+        tile_end = tiles_per_wg < 0 ? span.t.hi : min(vis.hi, tile_begin + per);
     }
-    int mrow_l[RG][4];  // query position l of each carried row
+    [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees
+    if constexpr (MM == 1) {
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg)
+        for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) mrow_l[rg][i] = (4 * rg + i) % a.L;
+            for (int i = 0; i < 4; ++i) seen[rg][i] = sym_mask_bounds(sym, (4 * rg + i) % a.L);
+    }
     // tokens whose V code sits in a high nibble carry 1/16 on the probability side
     const float vfac = (BITS == 4 && (lane & 2)) ? 0.0625f : 1.0f;
 
@@ -549,7 +524,7 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
                     float s_ = sc[i];
                     [[maybe_unused]] const int row_i = 4 * rg + i;
                     if constexpr (MM == 1) {
-                        if (!sym_mask_keep(sym, mrow_l[rg][i], t.row)) s_ = fill;
+                        if (!seen[rg][i].keep(t.row)) s_ = fill;
                     } else if constexpr (MM == 2) {
                         if (live && row_i < R) {
                             const int rep = row_i / a.L, l = row_i - rep * a.L;
@@ -743,7 +718,11 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
         }
         return;
     }
-    float *part = a.workspace + ((size_t)bh * nsplit + split) * RR * (D + 2);
+    float *part = a.workspace + part_slot * RR * (D + 2);
+    if constexpr (MM == 1) {
+        if (tiles_per_wg < 0 && wid == span.first && threadIdx.x == 0)  // (for the merge)
+            span_table(a.workspace, st.BH, nsplit, RR * (D + 2))[bh] = make_int2((int)part_slot, span.count);
+    }
     for (int idx = threadIdx.x; idx < RR * (D + 2); idx += NW * 64) {
         const int i = idx / (D + 2), c = idx - i * (D + 2);
         float mx = -INFINITY;
@@ -788,10 +767,26 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int blk = lane >> 2, qi = lane & 3;
-    const int bh = blockIdx.y, split = blockIdx.x;
-    const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
+    int bh = blockIdx.y;
+    const int split = blockIdx.x;
+    int b = bh / a.Hkv;
+    const int hk = bh - b * a.Hkv;
     const int r = a.Hq / a.Hkv;
     const int R = r * a.L;
+    size_t part_slot = (size_t)bh * nsplit + split;  // where this workgroup's partial goes
+    [[maybe_unused]] RaggedSpan span;
+    [[maybe_unused]] int wid = 0;
+    if constexpr (MM == 1 && IDENT) {
+        if (tiles_per_wg < 0) {  // a ragged batch that shares its spans out
+            const int wgs = nsplit * a.B;
+            wid = b * nsplit + split;
+            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, wgs, WAVES, wid, false);
+            if (span.count == 0) return;  // (workgroup-uniform)
+            part_slot = (size_t)hk * wgs + wid;
+            b = span.b;
+            bh = b * a.Hkv + hk;
+        }
+    }
 
     __shared__ __attribute__((aligned(16))) float cbuf[WAVES][RR][D + 2];
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
@@ -834,22 +829,22 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     }
 
     const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
-    int mrow_l[RG][4];
+    [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees
+    if constexpr (MM == 1) {
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg)
+        for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) mrow_l[rg][i] = (4 * rg + i) % a.L;
+            for (int i = 0; i < 4; ++i) seen[rg][i] = sym_mask_bounds(sym, (4 * rg + i) % a.L);
+    }
     int tile_begin = split * tiles_per_wg;
     int tile_end = min(tiles_total, tile_begin + tiles_per_wg);
     if constexpr (MM == 1 && IDENT) {
-        int vis_lo, vis_hi;
-        sym_mask_row_range(sym, vis_lo, vis_hi);
-        const int t_lo = max(0, vis_lo) >> 6, t_hi = min(tiles_total, (min(vis_hi, a.T - 1) >> 6) + 1);
+        const TileRange vis = visible_tiles(sym, tiles_total, false);
         // tiles_per_wg == 0: divide this batch row's own visible range over the spans
         const int per = tiles_per_wg > 0 ? tiles_per_wg
-                                         : (max(t_hi - t_lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
-        tile_begin = t_lo + split * per;  // spans past t_hi are empty
-        tile_end = min(t_hi, tile_begin + per);
+                                         : (max(vis.hi - vis.lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
+        tile_begin = tiles_per_wg < 0 ? span.t.lo : vis.lo + split * per;  // spans past the last tile are empty
+        tile_end = tiles_per_wg < 0 ? span.t.hi : min(vis.hi, tile_begin + per);
     }
     const int tile0 = tile_begin + wave;
     const int my_tiles = tile0 < tile_end ? (tile_end - tile0 + WAVES - 1) / WAVES : 0;
@@ -998,7 +993,7 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
                     float s_ = sacc[rg][i] * a.scale;
                     [[maybe_unused]] const int row_i = 4 * rg + i;
                     if constexpr (MM == 1) {
-                        if (!sym_mask_keep(sym, mrow_l[rg][i], row)) s_ = -INFINITY;
+                        if (!seen[rg][i].keep(row)) s_ = -INFINITY;
                     } else if constexpr (MM == 2) {
                         if (live && row_i < R) {
                             const int rep = row_i / a.L, l = row_i - rep * a.L;
@@ -1106,7 +1101,11 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
         }
         return;
     }
-    float *part = a.workspace + ((size_t)bh * nsplit + split) * RR * (D + 2);
+    float *part = a.workspace + part_slot * RR * (D + 2);
+    if constexpr (MM == 1 && IDENT) {
+        if (tiles_per_wg < 0 && wid == span.first && threadIdx.x == 0)  // (for the merge)
+            span_table(a.workspace, st.BH, nsplit, RR * (D + 2))[bh] = make_int2((int)part_slot, span.count);
+    }
     for (int idx = threadIdx.x; idx < RR * (D + 2); idx += WAVES * 64) {
         const int i = idx / (D + 2), c = idx - i * (D + 2);
         float mx = -INFINITY;
@@ -1125,136 +1124,6 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
             }
         }
         part[idx] = v;
-    }
-}
-
-// grid (R, BH), 256 threads: merge the span partials of one query row and write the output row.
-// A launch with few rows and many spans (a single sequence: 8 pairs, 32 to 512 spans each) lasts as long as its
-// chain of memory round trips, so everything is asked for at once: a thread is (column pair, span group) and
-// requests its first eight partial pairs before anything else, then the (max, sum) of up to two spans; the weights
-// are formed while the columns are in flight, go through LDS, and the span groups' sums meet there at the end.
-template <int D, int DT>
-__global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, int rr) {
-    constexpr int CP = D / 2;     // column pairs
-    constexpr int NG = 256 / CP;  // span groups: 8 (D 64), 6, 5, 4 (D 128), 2 (D 256)
-    constexpr int UN = 8;         // loads in flight per thread and round
-    __shared__ float w_s[512];    // weight of each span for this row (nsplit <= 512)
-    __shared__ float red_s[2][4];
-    __shared__ kv_f2 acc_s[NG][CP];
-    const int i = blockIdx.x, bh = blockIdx.y;
-    const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
-    const int r = a.Hq / a.Hkv;
-    const int rep = i / a.L, l = i - rep * a.L;
-    const size_t sstride = (size_t)rr * (D + 2);
-    const size_t first_slot = (size_t)bh * nsplit;
-    // (rows of D + 2 floats, D even: every pair below is 8-byte aligned)
-    const float *part = a.workspace + first_slot * sstride + (size_t)i * (D + 2);
-    const int t = threadIdx.x;
-    const int g = t / CP, cp = t - g * CP;
-    const bool col = g < NG;
-    auto pair_at = [&](int s, int c) { return *reinterpret_cast<const kv_f2 *>(part + (size_t)s * sstride + c); };
-    kv_f2 v[UN];
-#pragma unroll
-    for (int u = 0; u < UN; ++u) {
-        const int s = g + NG * u;
-        v[u] = (col && s < nsplit) ? pair_at(s, 2 * cp) : kv_f2{0.f, 0.f};
-    }
-    kv_f2 ml[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) ml[u] = t + 256 * u < nsplit ? pair_at(t + 256 * u, D) : kv_f2{-INFINITY, 0.f};
-    float mloc = wave_max(fmaxf(ml[0].x, ml[1].x));
-    if ((t & 63) == 0) red_s[0][t >> 6] = mloc;
-    __syncthreads();
-    const float mx = fmaxf(fmaxf(red_s[0][0], red_s[0][1]), fmaxf(red_s[0][2], red_s[0][3]));
-    float dloc = 0.f;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const float w = (ml[u].x == -INFINITY) ? 0.f : fast_exp2((ml[u].x - mx) * LOG2E);
-        if (t + 256 * u < nsplit) w_s[t + 256 * u] = w;
-        dloc += w * ml[u].y;
-    }
-    dloc = wave_sum(dloc);
-    if ((t & 63) == 0) red_s[1][t >> 6] = dloc;
-    __syncthreads();
-    const float den = (red_s[1][0] + red_s[1][1]) + (red_s[1][2] + red_s[1][3]);
-    kv_f2 num{0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < UN; ++u) {
-        const int s = g + NG * u;
-        if (col && s < nsplit) num += w_s[s] * v[u];
-    }
-    for (int s0 = g + NG * UN; col && s0 < nsplit; s0 += NG * UN) {  // more than 8 NG spans: further rounds
-#pragma unroll
-        for (int u = 0; u < UN; ++u) {
-            const int s = s0 + NG * u;
-            v[u] = s < nsplit ? pair_at(s, 2 * cp) : kv_f2{0.f, 0.f};
-        }
-#pragma unroll
-        for (int u = 0; u < UN; ++u) {
-            const int s = s0 + NG * u;
-            if (s < nsplit) num += w_s[s] * v[u];
-        }
-    }
-    if (col) acc_s[g][cp] = num;
-    __syncthreads();
-    if (t < CP) {
-        kv_f2 o = acc_s[0][t];
-#pragma unroll
-        for (int k = 1; k < NG; ++k) o += acc_s[k][t];
-        const float o0 = den > 0.f ? o.x / den : 0.f, o1 = den > 0.f ? o.y / den : 0.f;
-        uint32_t *dst = reinterpret_cast<uint32_t *>(static_cast<char *>(a.out) + (((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D + 2 * t) * 2);
-        *dst = DT == 0 ? pk_h2(o0, o1) : pk_bf2(o0, o1);
-    }
-}
-
-// The same merge for the prefill tiles' key-range parts: many query rows, at most 8 parts.  D / 4 lanes per query row,
-// four adjacent columns each, as many rows per workgroup as fit 256 threads; no LDS and no barrier (the
-// per-row workgroups above spend their time being launched: 22 us for 16 384 rows of 256 columns).  Bound by the latency of
-// its loads: every part's columns, maximum and sum are requested before any of them is looked at (parts up to MAXP = 2, 4
-// or 8; the numbers beyond nsplit repeat the last one's loads and are left out of the sums).  With the maxima read first and a part's columns
-// behind a branch of their own it took 12.0 us where it takes 7.6 (16 384 rows of 128, 3 or 4 parts), 11.1 where 9.6 (256
-// columns).
-// Decode launches keep the kernel above: with few rows and many parts it has the loads of a column in flight together
-// (configs[3]'s ring decode, 2 rows of 16 parts: 29.1 us per step against 31.7 us with this one).
-template <int D, int DT, int MAXP>
-__global__ void __launch_bounds__(256) combine_rows_kernel(AttendArgs a, int nsplit, int rr) {
-    constexpr int LPR = D / 4, RPW = 256 / LPR;
-    const int in_wg = threadIdx.x / LPR, c = 4 * (threadIdx.x % LPR);
-    const int i = blockIdx.x * RPW + in_wg, bh = blockIdx.y;
-    const int r = a.Hq / a.Hkv;
-    if (in_wg >= RPW || i >= r * a.L) return;  // (rr, the rows a part holds, may exceed the query rows there are)
-    const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
-    const int rep = i / a.L, l = i - rep * a.L;
-    const size_t sstride = (size_t)rr * (D + 2);
-    const float *part = a.workspace + (size_t)bh * nsplit * sstride + (size_t)i * (D + 2);
-    float2 ml[MAXP], p[MAXP][2];  // (a row of partials is 8-byte aligned: D + 2 floats)
-#pragma unroll
-    for (int s = 0; s < MAXP; ++s) {
-        const float *row = part + min(s, nsplit - 1) * sstride;
-        ml[s] = *reinterpret_cast<const float2 *>(row + D);
-        p[s][0] = *reinterpret_cast<const float2 *>(row + c);
-        p[s][1] = *reinterpret_cast<const float2 *>(row + c + 2);
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int s = 0; s < MAXP; ++s) mx = fmaxf(mx, ml[s].x);
-    float den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < MAXP; ++s) {
-        const float w = ml[s].x == -INFINITY ? 0.f : fast_exp2((ml[s].x - mx) * LOG2E);
-        const bool own = s < nsplit;
-        den = own ? den + w * ml[s].y : den;
-        num[0] = own ? num[0] + w * p[s][0].x : num[0];
-        num[1] = own ? num[1] + w * p[s][0].y : num[1];
-        num[2] = own ? num[2] + w * p[s][1].x : num[2];
-        num[3] = own ? num[3] + w * p[s][1].y : num[3];
-    }
-    const size_t ooff = ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D + c;
-    uint32_t *dst = reinterpret_cast<uint32_t *>(static_cast<char *>(a.out) + ooff * 2);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const float o0 = den > 0.f ? num[2 * k] / den : 0.f, o1 = den > 0.f ? num[2 * k + 1] / den : 0.f;
-        dst[k] = DT == 0 ? pk_h2(o0, o1) : pk_bf2(o0, o1);
     }
 }
 
@@ -1295,17 +1164,14 @@ Plan plan_for(const AttendArgs &a) {
     while ((p.tiles_total + per - 1) / per > 512) per *= 2;  // the merge kernel holds 512 span weights
     p.tiles_per_wg = per;
     p.nsplit = (p.tiles_total + per - 1) / per;
-    // ragged batches (per-batch bounds): the same number of spans for every batch row, each
-    // row's visible range divided among them in the kernel (all workgroups stay resident
-    // and none is empty; measured faster than equal-sized spans with more of them for the
-    // long rows, and than one span size for the whole batch with a row taking as many span slots
-    // as its length needs: 37.8 against 42.1 us for B16 U[1024, 16384] at 4 bits, 53.8 against
-    // 61.1 us with every row full).  The division needs slots in presented order: a ring
-    // presented through a row map keeps equal spans over all of its slots.
+    // ragged batches (per-batch bounds), marked by tiles_per_wg < 0: up to 64 rows share the launch's workgroups out by
+    // their lengths (ragged_span); 0: more rows, or one span each, where every row divides its own visible range
+    // over the same number of spans.  Both need slots in presented order: a
+    // ring presented through a row map keeps equal spans over all of its slots.
     p.nw = WAVES;
     const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
     if (a.mask.mode == KVHIP_MASK_WINDOW && (a.mask.left_pad || a.mask.lengths) && forced_tiles <= 0 && ident) {
-        p.tiles_per_wg = 0;
+        p.tiles_per_wg = a.B >= 2 && a.B <= 64 && p.nsplit >= 2 ? -1 : 0;
         // KVHIP_RAGGED_SPANS forces the number of spans per batch row (timing builds only: measure_knob)
         static const int forced_spans = measure_knob("KVHIP_RAGGED_SPANS", 0);
         if (forced_spans > 0) p.nsplit = std::min(forced_spans, 512);
@@ -1327,7 +1193,7 @@ Plan plan_for(const AttendArgs &a) {
     if (a.workspace_cap) {
         const size_t per_span = (size_t)BH * (a.st.bits != 0 && (p.rg >= 2 || only_decode16(a.st)) ? 16 : 4 * p.rg) *
                                 (a.st.Dv + 2) * sizeof(float);
-        while (p.nsplit > 1 && per_span * p.nsplit > a.workspace_cap) {
+        while (p.nsplit > 1 && per_span * p.nsplit + BH * sizeof(int2) > a.workspace_cap) {
             if (p.tiles_per_wg > 0) {
                 p.tiles_per_wg *= 2;
                 p.nsplit = (p.tiles_total + p.tiles_per_wg - 1) / p.tiles_per_wg;
@@ -1335,6 +1201,7 @@ Plan plan_for(const AttendArgs &a) {
                 p.nsplit /= 2;
             }
         }
+        if (p.nsplit == 1) p.tiles_per_wg = std::max(p.tiles_per_wg, 0);
     }
     return p;
 }
@@ -1384,42 +1251,6 @@ hipError_t profile_read(int *launches, double *total_ms) {
     return hipSuccess;
 }
 
-hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t s) {
-    const int R = (a.Hq / a.Hkv) * a.L;
-    dim3 grid(R, a.st.BH);
-    if (rows > 16 && nsplit <= 8 && rows == R) {  // the prefill tiles' parts
-#define CMBR_P(D, DT, P) hipLaunchKernelGGL((combine_rows_kernel<D, DT, P>), dim3((R + 256 / (D / 4) - 1) / (256 / (D / 4)), a.st.BH), dim3(256), 0, s, a, nsplit, rows)
-#define CMBR(D)                                                                                      \
-    do {                                                                                             \
-        const bool h = a.st.dtype == KVHIP_F16;                                                      \
-        if (nsplit <= 2) { if (h) CMBR_P(D, 0, 2); else CMBR_P(D, 1, 2); }                           \
-        else if (nsplit <= 4) { if (h) CMBR_P(D, 0, 4); else CMBR_P(D, 1, 4); }                      \
-        else { if (h) CMBR_P(D, 0, 8); else CMBR_P(D, 1, 8); }                                       \
-    } while (0)
-        if (a.st.Dv == 64) CMBR(64);
-        else if (a.st.Dv == 80) CMBR(80);
-        else if (a.st.Dv == 96) CMBR(96);
-        else if (a.st.Dv == 128) CMBR(128);
-        else CMBR(256);
-#undef CMBR
-#undef CMBR_P
-        return hipGetLastError();
-    }
-#define CMB(D)                                                                                       \
-    do {                                                                                             \
-        if (a.st.dtype == KVHIP_F16) hipLaunchKernelGGL((combine_kernel<D, 0>), grid, dim3(256), 0, s, a, nsplit, rows); \
-        else hipLaunchKernelGGL((combine_kernel<D, 1>), grid, dim3(256), 0, s, a, nsplit, rows);       \
-    } while (0)
-    // (the partials hold output columns: the head size of the values)
-    if (a.st.Dv == 64) CMB(64);
-    else if (a.st.Dv == 80) CMB(80);
-    else if (a.st.Dv == 96) CMB(96);
-    else if (a.st.Dv == 128) CMB(128);
-    else CMB(256);
-#undef CMB
-    return hipGetLastError();
-}
-
 bool attend_decode_supported(const AttendArgs &a) {
     const Store &s = a.st;
     if (s.dtype != KVHIP_F16 && s.dtype != KVHIP_BF16) return false;
@@ -1463,7 +1294,8 @@ size_t attend_decode_workspace(const AttendArgs &a) {
     const Plan p = plan_for(a);
     const int rows = use_decode16(a, p) ? 16 : 4 * p.rg;
     if (p.nsplit == 1) return 0;  // a single span writes the output rows itself: no partials
-    return (size_t)a.st.BH * p.nsplit * rows * (a.st.Dv + 2) * sizeof(float);  // (partials hold output columns)
+    return (size_t)a.st.BH * p.nsplit * rows * (a.st.Dv + 2) * sizeof(float)  // (partials hold output columns)
+           + (p.tiles_per_wg < 0 ? a.st.BH * sizeof(int2) : 0);
 }
 
 hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
@@ -1472,6 +1304,7 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
     const Store &st = a.st;
     dim3 grid(p.nsplit, st.BH), block(WAVES * 64);  // the quantized kernel sets its own block size
     const int mm = decode_mode(a);
+    auto spans_of = [&](int rows) { return p.tiles_per_wg < 0 ? span_table(a.workspace, st.BH, p.nsplit, rows * (st.Dv + 2)) : nullptr; };
 #define DEC_K(BITS, D, GS, DT, RG, MM, NW)                                                                \
     hipLaunchKernelGGL((decode_kernel<BITS, D, GS, DT, RG, MM, NW>), grid, dim3(NW * 64), 0, s, DecodeArgs<MM>::type(a), \
                        p.tiles_total, p.tiles_per_wg, p.nsplit)
@@ -1493,7 +1326,7 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
         }                                                                                                 \
         profile_mark(s, false);                                                                           \
         if (p.nsplit > 1)                                                                                 \
-            (void)launch_combine(a, p.nsplit, 4 * RG, s);                                                \
+            (void)launch_combine(a, p.nsplit, 4 * RG, s, spans_of(4 * RG));                              \
     } while (0)
 #define DEC_RG(BITS, D, GS, DT) DEC(BITS, D, GS, DT, 1) /* more rows: the 16-row kernel above */
     if (use_decode16(a_in, p)) {
@@ -1501,7 +1334,7 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
         hipError_t e = launch_attend_decode16(a_in, p.tiles_total, p.tiles_per_wg, p.nsplit, s);
         profile_mark(s, false);
         if (e != hipSuccess) return e;
-        if (p.nsplit > 1) return launch_combine(a_in, p.nsplit, 16, s);
+        if (p.nsplit > 1) return launch_combine(a_in, p.nsplit, 16, s, spans_of(16));
         return hipSuccess;
     }
 #define DEC_DT(BITS, D, GS)                                \
@@ -1527,7 +1360,7 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
                            p.tiles_per_wg, p.nsplit);                                                     \
         profile_mark(s, false);                                                                           \
         if (p.nsplit > 1)                                                                                 \
-            (void)launch_combine(a, p.nsplit, 4 * RG, s);                                                \
+            (void)launch_combine(a, p.nsplit, 4 * RG, s, spans_of(4 * RG));                              \
     } while (0)
 #define FP_MI(D, DT, RG)                                          \
     do {                                                          \

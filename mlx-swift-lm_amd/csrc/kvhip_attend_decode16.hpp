@@ -35,6 +35,7 @@
 
 #include "kvhip_mask.hpp"
 #include "kvhip_rope.hpp"
+#include "kvhip_wave.hpp"
 
 namespace kvhip {
 
@@ -50,10 +51,8 @@ union Op8 {
 };
 
 constexpr int WAVES = 4;
-constexpr float LOG2E = 1.4426950408889634f;
 constexpr float TWO24 = 16777216.0f;
 
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ uint32_t pack_h2(float lo, float hi) { return pk_h2(lo, hi); }
 // scale / bias of a raw (scale, bias) pair; for fp16 the widening folds into the consuming fma
 template <int DT> __device__ __forceinline__ float sb_scale(uint32_t raw) {
@@ -159,10 +158,12 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     constexpr int VWL = GEN ? SV::NWL : 16 * BITS / 32;      // words per lane and V row: its 16 tokens
     constexpr int VROW = 64 * BITS / 8;          // bytes of one V tile row
     constexpr int RR = 16;
-    // Three or four groups per row (group size 32 at D = 96 / 128, 64 at D = 256), and D = 256 with two: the (scale, bias) pairs of a tile -- 64 tokens
-    // x G pairs per side, 2 G registers per token of the lane group if held in registers -- go from global memory
-    // straight into LDS one tile ahead and are read from there four tokens at a time when they are used.
-    constexpr bool SB_LDS = GK >= 3 || GV >= 3 || DK >= 256;  // (D = 256: the accumulators alone take 64 registers)
+    // Two groups per row and more: the (scale, bias) pairs of a tile -- 64 tokens x G pairs per side -- go from global memory
+    // straight into LDS one tile ahead and are read from there four tokens at a time when they are used.  (Each lane
+    // group's sixteen tokens loaded into its lanes' registers, 2 G of them per token, are 1 KB a load returned for
+    // 64 bytes read: twice what the codes take, and the return path, busy 71 % of the kernel's time, held the rest up.  B16, 16
+    // query rows over 16384 keys of 8 kv heads x 128 at 4 bits: 70.3 us, 62.3 with the pairs in LDS.)
+    constexpr bool SB_LDS = GK >= 2 || GV >= 2;
     // words between the 64-word pieces the pairs arrive in (G = 2, 4: no lane group's pairs straddle two pieces;
     // the gap keeps the four lane groups' reads on different banks)
     constexpr int SB_PAD_K = (GK == 4 || GK == 2) ? 4 : 0, SB_PAD_V = (GV == 4 || GV == 2) ? 4 : 0;
@@ -189,10 +190,18 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * DK,
                    static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK, R);
     // ---- span of this workgroup (as in the 4-row kernel) -----------------------------------
+    [[maybe_unused]] RaggedSpan span;
+    [[maybe_unused]] int wid = 0;
     if constexpr (MM == 1) {
-        // a ragged batch whose rows divide their own ranges over the same number of spans: long and short
-        // rows are paired on the CUs (balanced_row)
-        if (tiles_per_wg == 0 && a.B <= 64 && a.B > 2) {
+        if (tiles_per_wg < 0) {
+            const int wgs = nsplit * a.B;
+            wid = b * nsplit + split;
+            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, wgs, WAVES, wid, true);
+            if (span.count == 0) return;  // (workgroup-uniform)
+            part_slot = (size_t)hk * wgs + wid;
+            b = span.b;
+            bh = b * a.Hkv + hk;
+        } else if (tiles_per_wg == 0 && a.B <= 64 && a.B > 2) {
             b = __builtin_amdgcn_readfirstlane(balanced_row(a.mask, a.B, a.L, a.T, tiles_total, b));
             bh = b * a.Hkv + hk;
             part_slot = (size_t)bh * nsplit + split;
@@ -202,17 +211,11 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     int tile_begin = split * tiles_per_wg;
     int tile_end = min(tiles_total, tile_begin + tiles_per_wg);
     if constexpr (MM == 1) {
-        int vis_lo, vis_hi;
-        sym_mask_row_range(sym, vis_lo, vis_hi);
-        int t_lo = max(0, vis_lo) >> 6, t_hi = min(tiles_total, (min(vis_hi, a.T - 1) >> 6) + 1);
-        if (sym_mask_some_row_empty(sym)) {  // a fully masked row averages over every key
-            t_lo = 0;
-            t_hi = tiles_total;
-        }
+        const TileRange vis = visible_tiles(sym, tiles_total, true);
         const int per = tiles_per_wg > 0 ? tiles_per_wg
-                                         : (max(t_hi - t_lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
-        tile_begin = t_lo + split * per;
-        tile_end = min(t_hi, tile_begin + per);
+                                         : (max(vis.hi - vis.lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
+        tile_begin = tiles_per_wg < 0 ? span.t.lo : vis.lo + split * per;
+        tile_end = tiles_per_wg < 0 ? span.t.hi : min(vis.hi, tile_begin + per);
     }
     // (wave-uniform by construction; saying so keeps the page walk in scalar registers and scalar loads)
     const int tile0 = __builtin_amdgcn_readfirstlane(tile_begin + wave);
@@ -224,6 +227,8 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     }
     const int row_l = n % a.L, row_rep = n / a.L;  // this lane's query row n = (head rep, position l)
     const bool row_ok = n < R;
+    [[maybe_unused]] KeyBounds seen{0, 0};
+    if constexpr (MM == 1) seen = sym_mask_bounds(sym, row_l);
 
     // ---- the step's new row, when it is still to be written (unmasked single-token step) --------
     // Its slot lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one: that wavefront
@@ -534,21 +539,17 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
             for (int tl = 0; tl < 16; ++tl) {
                 const int row = t.base + 16 * jj + tl;  // slots are presented rows
                 float s_ = (float)x[tl];
-                if (row < a.T) {
-                    if constexpr (MM == 1) {
-                        if (!sym_mask_keep(sym, row_l, row)) s_ = fill;
-                    } else if constexpr (MM == 2) {
-                        if (row_ok) {
-                            float add;
-                            const bool keep = mask_keep(a.mask, b, hk * r + row_rep, row_l, row, a.L, a.T, add);
-                            if (!keep) s_ = fill;
-                            else if (a.mask.dtype != KVHIP_BOOL) s_ = round_dt<DT>(s_ + add);
-                        }
+                if constexpr (MM == 1) {
+                    s_ = seen.keep(row) ? s_ : fill;
+                } else if constexpr (MM == 2) {
+                    if (row < a.T && row_ok) {
+                        float add;
+                        const bool keep = mask_keep(a.mask, b, hk * r + row_rep, row_l, row, a.L, a.T, add);
+                        if (!keep) s_ = fill;
+                        else if (a.mask.dtype != KVHIP_BOOL) s_ = round_dt<DT>(s_ + add);
                     }
-                } else {
-                    s_ = -INFINITY;
                 }
-                x[tl] = (XT)s_;
+                x[tl] = (XT)(row < a.T ? s_ : -INFINITY);
             }
         }
         // this lane's largest score: a tree of packed maxima (float16 scores sit two to a register) or of
@@ -749,6 +750,10 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         return;
     }
     float *part = a.workspace + part_slot * RR * (DV + 2);
+    if constexpr (MM == 1) {
+        if (tiles_per_wg < 0 && wid == span.first && threadIdx.x == 0)  // (for the merge)
+            span_table(a.workspace, st.BH, nsplit, RR * (DV + 2))[bh] = make_int2((int)part_slot, span.count);
+    }
     for (int idx = threadIdx.x; idx < RR * (DV + 2); idx += WAVES * 64) {
         const int i = idx / (DV + 2), c = idx - i * (DV + 2);
         float v;

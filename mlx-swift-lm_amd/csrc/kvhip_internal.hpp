@@ -368,7 +368,9 @@ bool mask_may_leave_rows_without_keys(const AttendArgs &a);
 hipError_t launch_rows_without_keys(const AttendArgs &a, hipStream_t s);
 // Merge `nsplit` partials per query row, laid out [bh][split][rows][D+2] in a.workspace
 // (out[D] unnormalised, running max, running sum), and write the normalised rows to a.out.
-hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t s);
+// `spans` not null: a pair's partials are spans[bh].x .. + spans[bh].y - 1 of one row of partials instead (span_table).
+hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t s, const int2 *spans = nullptr);
+bool combine_supported(const Store &s);  // whether it is built for the store's value head size
 hipError_t launch_attend_prefill(const AttendArgs &a, hipStream_t s);
 hipError_t launch_attend_decode16(const AttendArgs &a, int tiles_total, int tiles_per_wg, int nsplit, hipStream_t s);
 // (2- / 3-bit and 5- / 6-bit instances of the same kernel, and the shapes they are built for)

@@ -1,6 +1,7 @@
 // Mask evaluation shared by the attention kernels.
 #pragma once
 #include "kvhip_device.hpp"
+#include "kvhip_wave.hpp"
 
 namespace kvhip {
 
@@ -101,12 +102,17 @@ __device__ __forceinline__ SymMask sym_mask_init(const MaskDev &m, int b, int L,
     s.L = L;
     return s;
 }
-__device__ __forceinline__ bool sym_mask_keep(const SymMask &s, int l, int j) {
-    if (s.mode == KVHIP_MASK_CAUSAL) return j <= s.T - s.L + l;
-    const int li = s.offset + l;
-    bool keep = li >= j && j < s.len_b && j >= s.pad_b;
-    if (s.window > 0) keep = keep && (li < j + s.window);
-    return keep;
+// The key rows [lo, hi] that query position l sees (empty if lo > hi): two comparisons a key in the tiles at the edges.
+// (Evaluated condition by condition for every key, such a tile took the 16-row kernel as long as two others.)
+struct KeyBounds {
+    int lo, hi;
+    __device__ __forceinline__ bool keep(int j) const { return j >= lo && j <= hi; }
+};
+__device__ __forceinline__ KeyBounds sym_mask_bounds(const SymMask &s, int l) {
+    if (s.mode == KVHIP_MASK_CAUSAL) return KeyBounds{0, s.T - s.L + l};
+    KeyBounds k{s.pad_b, min(s.offset + l, s.len_b - 1)};
+    if (s.window > 0) k.lo = max(k.lo, s.offset + l - s.window + 1);
+    return k;
 }
 
 // Inclusive range of key rows any query position l in [0, L) may see under an index-only mask.
@@ -175,7 +181,68 @@ __device__ __forceinline__ KeyRange visible_keys(const MaskDev &m, int b, int L,
     return k;
 }
 
+// ---- the spans of a ragged batch -----------------------------------------------------------------------------------
+// The 64-token tiles batch row `b` sees, [lo, hi).  `all_if_empty`: a query position that sees no key averages over every
+// one of them (the quantized path), so no tile may be left out for its row.
+struct TileRange {
+    int lo, hi;
+};
+__device__ __forceinline__ TileRange visible_tiles(const SymMask &s, int tiles_total, bool all_if_empty) {
+    int vis_lo, vis_hi;
+    sym_mask_row_range(s, vis_lo, vis_hi);
+    TileRange t{max(0, vis_lo) >> 6, min(tiles_total, (min(vis_hi, s.T - 1) >> 6) + 1)};
+    if (all_if_empty && sym_mask_some_row_empty(s)) {
+        t.lo = 0;
+        t.hi = tiles_total;
+    }
+    return t;
+}
+
+// Workgroup `wid` of the `wgs` that share one kv head's batch rows (2 <= B <= 64, B <= wgs <= 512, `waves` wavefronts
+// each, which take every waves-th tile): all spans have the same length and a row gets as many as its keys need, so that
+// the launch lasts as long as the batch's keys do in all and not as its longest row does.  The length is the first from an
+// even share on -- the rows' last spans taken for half full -- with which the spans go round.  Every workgroup works the
+// partition out for itself, a lane to a batch row (about half a microsecond; the sums are of small whole numbers, exact in
+// float).  Spans of a row are adjacent: first .. first + count - 1; count 0: nothing is left for this workgroup.
+// (B16 of 1024 to 16384 keys, 4 new tokens, 8 kv heads of 128 at 4 bits, the kernel 42 us with every row over the same
+// number of spans, long rows and short ones paired on the CUs.)
+struct RaggedSpan {
+    int b, first, count;  // batch row; its spans
+    TileRange t;          // this workgroup's tiles
+};
+__device__ __forceinline__ RaggedSpan ragged_span(const MaskDev &m, int B, int L, int T, int tiles_total, int wgs, int waves, int wid, bool all_if_empty) {
+    const int lane = threadIdx.x & 63;
+    TileRange mine{0, 0};
+    if (lane < B) mine = visible_tiles(sym_mask_init(m, lane, L, T), tiles_total, all_if_empty);
+    const int tiles = max(mine.hi - mine.lo, 0), steps = (tiles + waves - 1) / waves;
+    const int total = (int)wave_sum((float)steps);
+    int len = max(1, (2 * total + 2 * wgs - B - 1) / (2 * wgs - B)), spans;
+    float upto;
+    for (;; ++len) {  // (ends: with `len` the longest row's steps every row has one span, and B <= wgs)
+        spans = lane < B ? max(1, (steps + len - 1) / len) : 0;
+        upto = wave_scan((float)spans);
+        if (__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, upto), 63)) <= (float)wgs) break;
+    }
+    const unsigned long long before = __ballot(lane < B && upto <= (float)wid);
+    RaggedSpan r;
+    r.b = min(__popcll(before), B - 1);
+    const bool some = __popcll(before) < B;
+    const int end = (int)__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, upto), r.b));
+    r.count = some ? __builtin_amdgcn_readlane(spans, r.b) : 0;
+    r.first = end - r.count;
+    const int lo = __builtin_amdgcn_readlane(mine.lo, r.b), hi = __builtin_amdgcn_readlane(mine.hi, r.b);
+    r.t.lo = lo + (wid - r.first) * len * waves;
+    r.t.hi = min(hi, r.t.lo + len * waves);
+    return r;
+}
+
+// Where such a launch notes, behind its partials, which of them are a pair's: first and count, per (batch row, kv head).
+__host__ __device__ __forceinline__ int2 *span_table(float *workspace, int BH, int nsplit, int floats_per_span) {
+    return reinterpret_cast<int2 *>(workspace + (size_t)BH * nsplit * floats_per_span);
+}
+
 // ---- which batch row a workgroup row takes, for ragged batches ------------------------------------
+// (Batches that ragged_span does not take: a single span to a row.)
 // Workgroups are started in id order, one per CU and then a second one per CU, so rows v and v + B/2 of a
 // launch of 512 workgroups share CUs.  Taking the batch rows in order of their visible length -- the first
 // half of the workgroup rows in descending order, the second half in ascending order -- pairs the longest
@@ -187,15 +254,8 @@ __device__ __forceinline__ int balanced_row(const MaskDev &m, int B, int L, int 
     const int lane = threadIdx.x & 63;
     int tiles = -1;
     if (lane < B) {
-        const SymMask s = sym_mask_init(m, lane, L, T);
-        int vis_lo, vis_hi;
-        sym_mask_row_range(s, vis_lo, vis_hi);
-        int t_lo = max(0, vis_lo) >> 6, t_hi = min(tiles_total, (min(vis_hi, T - 1) >> 6) + 1);
-        if (sym_mask_some_row_empty(s)) {
-            t_lo = 0;
-            t_hi = tiles_total;
-        }
-        tiles = max(t_hi - t_lo, 0);
+        const TileRange t = visible_tiles(sym_mask_init(m, lane, L, T), tiles_total, true);
+        tiles = max(t.hi - t.lo, 0);
     }
     int rank = 0;  // rows that come before this lane's: more tiles, or as many and a lower index
     for (int j = 0; j < B; ++j) {
