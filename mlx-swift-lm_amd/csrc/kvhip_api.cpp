@@ -1266,7 +1266,9 @@ kvhip_status attend_impl(kvhip_cache *c, const void *q, int32_t B, int32_t Hq, i
     hipStream_t s = S(c, stream);
     a.workspace_cap = fixed ? fixed_bytes : 0;
     if (new_k) {
-        if (g_policy != 1 && attend_decode_fuses_append(a)) {
+        const bool fuses = attend_decode_fuses_append(a) ||
+                           (!attend_decode_supported(a) && !attend_prefill_supported(a) && attend_valu_fuses_append(a));
+        if (g_policy != 1 && fuses) {
             a.new_k = new_k;
             a.new_v = new_v;
             a.new_slot = new_slot;
@@ -1350,12 +1352,12 @@ kvhip_status kvhip_cache_update_attend(kvhip_cache *c, const void *q, const void
         }
         return st;
     }
-    // One new token into a full-precision cache of a 16-bit dtype (KVCacheSimple, or the in-place step of a
-    // RotatingKVCache): the decode kernel copies the row into its slot itself.  The bookkeeping of `update`
+    // One new token into a full-precision cache (KVCacheSimple, or the in-place step of a
+    // RotatingKVCache): the attention kernel copies the row into its slot itself where it can.  The bookkeeping of `update`
     // runs here as usual; if the attention cannot be enqueued the row is written by the append kernel, so
     // the cache holds what its counters say.
     if (c && k && v && q && out && L == 1 && (c->kind == KVHIP_KIND_SIMPLE || c->kind == KVHIP_KIND_ROTATING) &&
-        !c->staging && !c->rope && (dtype == KVHIP_F16 || dtype == KVHIP_BF16) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
+        !c->staging && !c->rope && (dtype == KVHIP_F16 || dtype == KVHIP_BF16 || dtype == KVHIP_F32) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
         c->has_geom && c->has_buffers && !c->padded() && c->B == B && c->Hkv == Hkv && c->st.Dk == Dk && c->st.Dv == Dv && c->st.dtype == dtype) {
         int32_t slot = -1;
         if (c->kind == KVHIP_KIND_SIMPLE) {
@@ -1383,9 +1385,9 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
     RopeDev r;
     const int64_t pos0 = c->offset + (c->staging ? (int64_t)c->staged.size() : 0);  // (before the write, as in kvhip_cache_update_rope)
     KV_TRY(rope_dev(rope, Dk, Hkv, dtype, pos0, batch_offsets, r));
-    // One new token without a mask: the decode kernels rotate its rows themselves, as they write the new one
+    // One new token without a mask: the attention kernels rotate its rows themselves, as they write the new one
     // (kvhip_cache_update_attend), and the step is a launch less.
-    const bool token = L == 1 && !c->staging && (dtype == KVHIP_F16 || dtype == KVHIP_BF16) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
+    const bool token = L == 1 && !c->staging && (dtype != KVHIP_F32 || c->kind != KVHIP_KIND_QUANTIZED) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
                        c->has_geom && c->has_buffers && !c->padded() && c->B == B && c->Hkv == Hkv && c->st.Dk == Dk && c->st.Dv == Dv &&
                        c->st.dtype == dtype && (size_t)B * Hkv + (size_t)B * Hq <= 65535;
     if (!q_rotated && !(token && decode_takes_step(c, Hq))) {

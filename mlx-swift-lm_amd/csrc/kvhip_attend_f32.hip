@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include "kvhip_mask.hpp"
+#include "kvhip_rope.hpp"
 
 namespace kvhip {
 
@@ -37,10 +38,14 @@ constexpr int query_tiles(int dk) { return dk <= 128 ? 2 : 1; }
 // One token, B8, 32q/8kv, D 128, 8192 keys: all seen under a boolean mask 107 us, a window of 512 31, an additive mask
 // 104; 119, 120 and 112 with the elements fetched one by one behind the keys and every tile read, 105, 43 and 100 on
 // the vector-ALU kernel; 256 rows of B4 over 4096 keys, the boolean window: 236, 893, 476.
-template <int DK, int DV, int QT, int ARR>
+// A single-token step without a mask: the wavefront that reads the new row's tile writes the row after it has requested
+// its first tile -- and if that is the row's tile, puts the row into its registers too --, and ROT turns the query rows and
+// the new key row in LDS first, as the decode kernels do.  A launch that appends takes 4.2 us.
+// TB: token blocks of 16 per tile.
+template <int DK, int DV, int QT, int TB, int ARR, bool ROT>
 __global__ void __launch_bounds__(256, 2)
-attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
-    constexpr int TB = token_blocks(DK, QT), WT = 16 * TB;
+attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int nparts) {
+    constexpr int WT = 16 * TB;
     constexpr int NS = DK / 16, NCT = DV / 16;
     extern __shared__ __align__(16) float smem[];
     f4 *acc_s = reinterpret_cast<f4 *>(smem);         // [MW][QT][NCT][64]
@@ -71,6 +76,46 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
     const int per = (max(t_hi - t_lo, 1) + nparts - 1) / nparts;
     const int tb = min(t_lo + part * per, t_hi), te = min(tb + per, t_hi);
 
+    // ---- a step's rows ----------------------------------------------------------------------------------------
+    constexpr bool STEP = QT == 1 && ARR == 0;  // (up to 16 query rows: one row block)
+    float *rot_s = smem + (QL ? NS * 256 : 0);  // [R + 1][DK] behind the query operands, under what the accumulators take at the end
+    static_assert((QL ? NS * 256 : 0) + 17 * DK <= MW * NCT * 256, "room for sixteen query rows and the key row");
+    [[maybe_unused]] RopeStep<2, DK, 256, 16> step;
+    if constexpr (ROT)
+        step.fetch(a.turn, static_cast<const float *>(a.q) + (size_t)(b * a.Hq + h * r) * DK, static_cast<const float *>(a.new_k) + (size_t)bh * DK, R);
+    // (lane (col, g): the row's elements that its key operands of the row's token hold, and its values of columns 16 c + col)
+    bool own = false;  // wave-uniform
+    f4 own_k[NS];
+    float own_v[NCT];
+    if constexpr (STEP) {
+        const int tn = a.new_slot / WT;
+        own = a.new_k != nullptr && tn >= tb && tn < te && (tn - tb) % MW == wave;
+        if (own) {
+#pragma unroll
+            for (int s = 0; s < (ROT ? 0 : NS); ++s) own_k[s] = ld_global<f4>(as_global(a.new_k) + ((size_t)bh * DK + 16 * s + 4 * g) * 4);
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) own_v[c] = ld_global<float>(as_global(a.new_v) + ((size_t)bh * DV + 16 * c + col) * 4);
+        }
+    }
+    auto write_row = [&]() __attribute__((always_inline)) {
+        const int slot = a.new_slot;
+        char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot)), *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
+        if constexpr (ROT) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) own_k[s] = *reinterpret_cast<const f4 *>(rot_s + R * DK + 16 * s + 4 * g);
+        }
+        if (col == 0) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) *reinterpret_cast<f4 *>(kc + kfp_off(st, slot, 16 * s + 4 * g)) = own_k[s];
+        }
+        if (g == 0) {
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) *reinterpret_cast<float *>(vc + vfp_off(st, slot, 16 * c + col)) = own_v[c];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+
     // rows beyond the last: the last again, which nobody keeps
     f4 qop[QT][QL ? 1 : NS];
     int my_hq[QT], my_l[QT];
@@ -81,12 +126,12 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
         my_l[qt] = rr % a.L;
         gptr qp = as_global(a.q) + (((size_t)(b * a.Hq + my_hq[qt]) * a.L + my_l[qt]) * DK + 4 * g) * 4;
 #pragma unroll
-        for (int s = 0; s < (QL ? 0 : NS); ++s) qop[qt][s] = ld_global<f4>(qp + s * 64);
-        if constexpr (QL) {
+        for (int s = 0; s < (QL || ROT ? 0 : NS); ++s) qop[qt][s] = ld_global<f4>(qp + s * 64);
+        if constexpr (QL && !ROT) {
             for (int s = wave; s < NS; s += MW) q_s[(qt * NS + s) * 64 + lane] = ld_global<f4>(qp + s * 64);
         }
     }
-    if constexpr (QL) __syncthreads();
+    if constexpr (QL && !ROT) __syncthreads();
 
     f4 kreg[TB][NS], vreg[TB][NCT];
     const uint32_t k_lane = ((uint32_t)g * TILE + col) * 16, v_lane = ((uint32_t)g * DV + col) * 16;
@@ -199,6 +244,35 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
         load_k(t);
         if (ARR && t + (bools ? MW : 0) < te) mask_fetch(t + (bools ? MW : 0));
         load_v(t);
+    }
+    if constexpr (ROT) {
+        step.turn(a.turn, bh, R, rot_s);
+        __syncthreads();
+        const float *qr = rot_s + min(row0 + col, R - 1) * DK + 4 * g;
+        if constexpr (QL) {
+            for (int s = wave; s < NS; s += MW) q_s[s * 64 + lane] = *reinterpret_cast<const f4 *>(qr + 16 * s);
+            __syncthreads();
+        } else {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) qop[0][s] = *reinterpret_cast<const f4 *>(qr + 16 * s);
+        }
+    }
+    if constexpr (STEP) {
+        if (own) {
+            write_row();
+            if (a.new_slot / WT == first) {
+                const int tn = a.new_slot % WT;
+#pragma unroll
+                for (int x = 0; x < TB; ++x) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) kreg[x][s] = x == tn >> 4 && col == (tn & 15) ? own_k[s] : kreg[x][s];
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) vreg[x][c][j] = 16 * x + 4 * g + j == tn ? own_v[c] : vreg[x][c][j];
+                }
+            }
+        }
     }
     while (t < te) {
         int next = t + MW;
@@ -360,15 +434,20 @@ attend_f32_kernel(AttendArgs a, int tiles_total, int nparts) {
 }
 
 struct PlanF32 {
-    int qt, row_blocks, tiles, nparts;
+    int qt, tb, row_blocks, tiles, nparts;
 };
 
 PlanF32 plan_f32(const AttendArgs &a) {
     PlanF32 p;
     const int R = (a.Hq / a.Hkv) * a.L;
     p.qt = R <= 16 ? 1 : query_tiles(a.st.Dk);
-    const int wt = 16 * token_blocks(a.st.Dk, p.qt);
     p.row_blocks = (R + 16 * p.qt - 1) / (16 * p.qt);
+    // A few rows over so few keys that wide tiles would leave wavefronts of the resident workgroups (two per CU) without one:
+    // tiles of one token block (one sequence of 1500 keys, 4 kv heads of 64: the kernel 11.0 us with tiles of 64 tokens, of
+    // which each workgroup has one).
+    p.tb = token_blocks(a.st.Dk, p.qt);
+    if (p.qt == 1 && (long)((a.slots + 16 * p.tb - 1) / (16 * p.tb)) * a.st.BH < 512 * MW) p.tb = 1;
+    const int wt = 16 * p.tb;
     p.tiles = (a.slots + wt - 1) / wt;
     static const int target = measure_knob("KVHIP_F32_TARGET", 512), least = measure_knob("KVHIP_F32_LEAST", 2);  // (timing builds only)
     const long wgs = (long)p.row_blocks * a.st.BH;
@@ -380,20 +459,29 @@ PlanF32 plan_f32(const AttendArgs &a) {
     return p;
 }
 
-template <int DK, int DV, int QT>
+template <int DK, int DV, int QT, int TB>
 hipError_t launch_instance(const AttendArgs &a, const PlanF32 &p, hipStream_t s) {
     const dim3 grid(p.row_blocks, a.st.BH, p.nparts), block(256);
     const size_t lds = MW * QT * (DV / 16) * 64 * sizeof(f4);
-    if (a.mask.mode != KVHIP_MASK_ARRAY) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, 0>), grid, block, lds, s, a, p.tiles, p.nparts);
-    else if (a.mask.dtype == KVHIP_BOOL) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, 1>), grid, block, lds, s, a, p.tiles, p.nparts);
-    else hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, 2>), grid, block, lds, s, a, p.tiles, p.nparts);
+    if constexpr (QT == 1) {
+        if (a.new_k && a.rope) {
+            hipLaunchKernelGGL((attend_f32_kernel<DK, DV, 1, TB, 0, true>), grid, block, lds, s, AttendStepArgs(a), p.tiles, p.nparts);
+            return hipGetLastError();
+        }
+    }
+    if (a.mask.mode != KVHIP_MASK_ARRAY) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 0, false>), grid, block, lds, s, a, p.tiles, p.nparts);
+    else if (a.mask.dtype == KVHIP_BOOL) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 1, false>), grid, block, lds, s, a, p.tiles, p.nparts);
+    else hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 2, false>), grid, block, lds, s, a, p.tiles, p.nparts);
     return hipGetLastError();
 }
 
 template <int DK, int DV>
 hipError_t launch_sizes(const AttendArgs &a, const PlanF32 &p, hipStream_t s) {
-    if (p.qt == 1) return launch_instance<DK, DV, 1>(a, p, s);
-    return launch_instance<DK, DV, query_tiles(DK)>(a, p, s);
+    if constexpr (token_blocks(DK, 1) != 1) {
+        if (p.tb == 1 && p.qt == 1) return launch_instance<DK, DV, 1, 1>(a, p, s);
+    }
+    if (p.qt == 1) return launch_instance<DK, DV, 1, token_blocks(DK, 1)>(a, p, s);
+    return launch_instance<DK, DV, query_tiles(DK), token_blocks(DK, query_tiles(DK))>(a, p, s);
 }
 
 }  // namespace

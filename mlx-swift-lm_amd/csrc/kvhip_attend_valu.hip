@@ -375,6 +375,11 @@ bool attend_valu_supported(const AttendArgs &a) {
     return s.bits == 0 && s.Dk <= 1024 && s.Dv <= 512 && s.BH <= 65535 && plan_valu(a).lds <= 64 * 1024;
 }
 
+bool attend_valu_fuses_append(const AttendArgs &a) {
+    static const bool off = measure_knob("KVHIP_NO_FUSED_APPEND", 0) != 0;  // (timing builds only)
+    return !off && a.L == 1 && a.mask.mode == KVHIP_MASK_NONE && a.Hq / a.Hkv <= 16 && (attend_wide_supported(a) || attend_f32_supported(a));
+}
+
 bool attend_valu_dequant_first(const AttendArgs &a) {
     const Store &s = a.st;
     if (s.bits == 0) return false;
@@ -386,6 +391,7 @@ bool attend_valu_dequant_first(const AttendArgs &a) {
 }
 
 hipError_t launch_merge_valu(const AttendArgs &a, int nparts, hipStream_t s) {
+    if (combine_supported(a.st)) return launch_combine(a, nparts, (a.Hq / a.Hkv) * a.L, s);
     const dim3 grid((a.Hq / a.Hkv) * a.L, a.st.BH), block(FT);
     if (a.st.dtype == KVHIP_F16) hipLaunchKernelGGL(merge_valu_kernel<0>, grid, block, 0, s, a, nparts);
     else if (a.st.dtype == KVHIP_BF16) hipLaunchKernelGGL(merge_valu_kernel<1>, grid, block, 0, s, a, nparts);

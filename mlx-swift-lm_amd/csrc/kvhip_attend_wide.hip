@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "kvhip_mask.hpp"
+#include "kvhip_rope.hpp"
 
 namespace kvhip {
 
@@ -73,15 +74,21 @@ constexpr int SEEN = 4096;     // tiles of a part that a boolean mask is looked 
 // loop's barriers.)  One token, B8, 16q/8kv, 8192 keys: all seen under a boolean mask 212 us, a window of 512 47, an
 // additive mask 193; 275, 276 and 262 with the elements fetched one by one behind the keys and every tile read, 198, 66
 // and 193 on the vector-ALU kernel.
-template <int DT, int QT, int ARR>
+// A single-token step without a mask: the workgroup whose part holds the new row's tile writes the row, each wavefront
+// its quarter, after its first tile has been requested -- and if that is the row's tile, puts the row into its registers
+// too --, and ROT turns the query rows and the new key row in LDS first, as the decode kernels do.  A launch that appends
+// takes 5.2 us.
+template <int DT, int QT, int ARR, bool ROT>
 __global__ void __launch_bounds__(256, 2)
-attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
+attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int nparts) {
     constexpr int NB = QT == 1 ? 2 : 1;           // score buffers (QT = 1 has one barrier per tile)
     __shared__ f4 part_s[NB][WW][QT][2][64];      // partial scores of the wavefronts
     __shared__ kv_u4 prob_s[QT == 1 ? 1 : QT][2][64];
     __shared__ float stat_s[QT][16], sum_s[QT][16], max_s[QT][16];
     __shared__ int nan_s[WW];
     __shared__ uint8_t seen_s[ARR == 1 ? SEEN : 1];
+    constexpr bool STEP = QT == 1 && ARR == 0;  // (up to 16 query rows: one row block)
+    __shared__ __align__(16) uint16_t rot_s[ROT ? 17 * WD : 1];
     const Store &st = a.st;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, g = lane >> 4;
@@ -106,10 +113,47 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
     const int per = (max(t_hi - t_lo, 1) + nparts - 1) / nparts;
     const int tb = min(t_lo + part * per, t_hi), te = min(tb + per, t_hi);
 
+    // ---- a step's rows ----------------------------------------------------------------------------------------
+    [[maybe_unused]] RopeStep<DT, WD, 256, 16> step;
+    if constexpr (ROT)
+        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + h * r) * WD,
+                   static_cast<const uint16_t *>(a.new_k) + (size_t)bh * WD, R);
+    // (lane (col, g): the row's elements that its key operands of the row's token hold, and its values of columns 16 c + col)
+    bool owner = false;  // workgroup-uniform
+    kv_u4 own_k[NS];
+    uint16_t own_v[NCT];
+    if constexpr (STEP) {
+        owner = a.new_k != nullptr && a.new_slot / WT >= tb && a.new_slot / WT < te;
+        if (owner) {
+#pragma unroll
+            for (int s = 0; s < (ROT ? 0 : NS); ++s) own_k[s] = ld_global<kv_u4>(as_global(a.new_k) + ((size_t)bh * WD + wave * (WD / WW) + 8 * g + 32 * s) * 2);
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) own_v[c] = ld_global<uint16_t>(as_global(a.new_v) + ((size_t)bh * WD + wave * (WD / WW) + 16 * c + col) * 2);
+        }
+    }
+    auto write_row = [&]() __attribute__((always_inline)) {
+        const int slot = a.new_slot, c0 = wave * (WD / WW);
+        char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot)), *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
+        if constexpr (ROT) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) own_k[s] = *reinterpret_cast<const kv_u4 *>(rot_s + R * WD + c0 + 8 * g + 32 * s);
+        }
+        if (col == 0) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) *reinterpret_cast<kv_u4 *>(kc + kfp_off(st, slot, c0 + 8 * g + 32 * s)) = own_k[s];
+        }
+        if (g == 0) {
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, c0 + 16 * c + col)) = own_v[c];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+
     // ---- query operands: lane (col, g) holds elements 8 g .. 8 g + 7 of step s of row 16 qt + col ----
     kv_u4 qop[QT][NS];
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
+    for (int qt = 0; qt < (ROT ? 0 : QT); ++qt) {
         const int rr = min(row0 + 16 * qt + col, R - 1);  // rows beyond the last: the last again, which nobody keeps
         gptr qp = as_global(a.q) + (((size_t)(b * a.Hq + h * r + rr / a.L) * a.L + rr % a.L) * WD + wave * (WD / WW) + 8 * g) * 2;
 #pragma unroll
@@ -278,7 +322,7 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
 #pragma unroll
             for (int c = 0; c < NCT; ++c) acc[qt][c] = f4{0.f, 0.f, 0.f, 0.f};
         int t = seen_from(tb), buf = 0;
-        if (t < te) {  // workgroup-uniform
+        if (t < te && (decltype(careful)::value || !STEP)) {  // workgroup-uniform
             load_k(t);
             load_v(t);
         }
@@ -348,6 +392,38 @@ attend_wide_kernel(AttendArgs a, int tiles_total, int nparts) {
         __syncthreads();
         return (nan_s[0] | nan_s[1] | nan_s[2] | nan_s[3]) != 0;  // workgroup-uniform
     };
+    if constexpr (STEP) {  // (ahead of the first walk: the row is written, and the rows turned, meanwhile)
+        if (tb < te) {
+            load_k(tb);
+            load_v(tb);
+        }
+        if constexpr (ROT) {
+            step.turn(a.turn, bh, R, rot_s);
+            __syncthreads();
+            const uint16_t *qr = rot_s + min(row0 + col, R - 1) * WD + wave * (WD / WW) + 8 * g;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) qop[0][s] = *reinterpret_cast<const kv_u4 *>(qr + 32 * s);
+        }
+        if (owner) {
+            write_row();
+            if (a.new_slot / WT == tb) {
+                const int tn = a.new_slot & (WT - 1);  // token 8 (c / 4) + 4 x + c % 4 is operand row c of block x
+                const bool mine = col == 4 * (tn >> 3) + (tn & 3);
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+#pragma unroll
+                    for (int x = 0; x < 2; ++x) kreg[s][x] = mine && ((tn >> 2) & 1) == x ? own_k[s] : kreg[s][x];
+#pragma unroll
+                for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {  // value tn % 8 of the lane's eight, if they are token tn's
+                        const uint32_t old = vreg[c][w];
+                        const uint32_t both = (tn & 1) ? (old & 0xffffu) | ((uint32_t)own_v[c] << 16) : (old & 0xffff0000u) | own_v[c];
+                        vreg[c][w] = g == tn >> 3 && w == ((tn & 7) >> 1) ? both : old;
+                    }
+            }
+        }
+    }
     if (__builtin_expect(walk(std::false_type()), 0)) {
         __syncthreads();
         walk(std::true_type());
@@ -392,10 +468,10 @@ PlanWide plan_wide(const AttendArgs &a) {
     p.qt = R <= 16 ? 1 : 2;
     p.row_blocks = (R + 16 * p.qt - 1) / (16 * p.qt);
     p.tiles = (a.slots + WT - 1) / WT;
-    // One token: a workgroup per CU (two: B8 over 4096 keys 29.4 us against 26.8), parts of at least two tiles (one: 14.1 us
-    // against 12.1 for a sequence of 2048 keys, whose merge then reads twice the partials).  Chunks: two per CU (one: 76 us
-    // against 57 for 512 x 2048; three, which need a second round: 72 us).
-    static const int target = measure_knob("KVHIP_WIDE_TARGET", 256), target2 = measure_knob("KVHIP_WIDE_TARGET2", 512), least = measure_knob("KVHIP_WIDE_LEAST", 2);  // (timing builds only)
+    // One token: a workgroup per CU (two: B8 over 4096 keys 29.4 us against 26.8), parts of a tile and up (two: 11.2 us against
+    // 10.1 for a sequence of 2048 keys, the merge, which has every part's loads in flight at once, 3.5 us for either).
+    // Chunks: two per CU (one: 76 us against 57 for 512 x 2048; three, which need a second round: 72 us).
+    static const int target = measure_knob("KVHIP_WIDE_TARGET", 256), target2 = measure_knob("KVHIP_WIDE_TARGET2", 512), least = measure_knob("KVHIP_WIDE_LEAST", 1);  // (timing builds only)
     const long wgs = (long)p.row_blocks * a.st.BH;
     int n = (int)std::max(1L, std::min<long>((p.qt == 1 ? target : target2) / std::max(1L, wgs), p.tiles / (p.qt == 1 ? least : 4)));
     n = std::min(n, 64);
@@ -422,10 +498,12 @@ hipError_t launch_attend_wide(const AttendArgs &a, hipStream_t s) {
     const dim3 grid(p.row_blocks, a.st.BH, p.nparts), block(256);
     profile_mark(s, true);
     const int arr = a.mask.mode != KVHIP_MASK_ARRAY ? 0 : a.mask.dtype == KVHIP_BOOL ? 1 : 2;
-#define WIDE_A(DT, QT, ARR) hipLaunchKernelGGL((attend_wide_kernel<DT, QT, ARR>), grid, block, 0, s, a, p.tiles, p.nparts)
+#define WIDE_A(DT, QT, ARR) hipLaunchKernelGGL((attend_wide_kernel<DT, QT, ARR, false>), grid, block, 0, s, a, p.tiles, p.nparts)
 #define WIDE(DT, QT)                       \
     do {                                   \
-        if (arr == 0) WIDE_A(DT, QT, 0);   \
+        if (QT == 1 && a.new_k && a.rope)  \
+            hipLaunchKernelGGL((attend_wide_kernel<DT, 1, 0, true>), grid, block, 0, s, AttendStepArgs(a), p.tiles, p.nparts); \
+        else if (arr == 0) WIDE_A(DT, QT, 0); \
         else if (arr == 1) WIDE_A(DT, QT, 1); \
         else WIDE_A(DT, QT, 2);            \
     } while (0)

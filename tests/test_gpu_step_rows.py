@@ -41,7 +41,10 @@ def _compare(caches, q, k, v, rope):
     (8, 128, torch.bfloat16, 1, 4, 1, 256, 256), (4, 64, torch.float16, 70, 4, 2, 128, 128),
     (4, 64, torch.bfloat16, 2, 16, 2, 128, 128), (6, 64, torch.float16, 1, 8, 2, 128, 128), (3, 64, torch.bfloat16, 2, 4, 4, 256, 256),
     (4, 32, torch.float16, 1, 8, 8, 96, 96), (8, 64, torch.bfloat16, 1, 4, 4, 192, 128),
-    ("simple", 0, torch.float16, 1, 8, 2, 64, 64), ("simple", 0, torch.bfloat16, 2, 16, 2, 128, 128), ("simple", 0, torch.float16, 1, 4, 1, 256, 256)])
+    ("simple", 0, torch.float16, 1, 8, 2, 64, 64), ("simple", 0, torch.bfloat16, 2, 16, 2, 128, 128), ("simple", 0, torch.float16, 1, 4, 1, 256, 256),
+    ("simple", 0, torch.bfloat16, 1, 8, 2, 512, 512), ("simple", 0, torch.float16, 2, 16, 1, 512, 512),
+    ("simple", 0, torch.float32, 1, 16, 4, 64, 64), ("simple", 0, torch.float32, 1, 4, 4, 96, 96), ("simple", 0, torch.float32, 2, 16, 1, 128, 128),
+    ("simple", 0, torch.float32, 1, 8, 2, 256, 256), ("simple", 0, torch.float32, 1, 4, 2, 192, 128)])
 def test_a_step_equals_its_separate_calls(kind, gs, dtype, B, Hq, Hkv, Dk, Dv, rotary):
     gen = torch.Generator(device="cuda").manual_seed(17)
     rope = kvhip.RoPE(Dk, base=1e4) if rotary else None
@@ -57,17 +60,17 @@ def test_a_step_equals_its_separate_calls(kind, gs, dtype, B, Hq, Hkv, Dk, Dv, r
 
 
 @pytest.mark.parametrize("rotary", [False, True])
-@pytest.mark.parametrize("D", [64, 128, 256])
-def test_a_ring_step_equals_its_separate_calls(D, rotary):
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.bfloat16), (256, torch.bfloat16), (512, torch.bfloat16), (128, torch.float32), (256, torch.float32)])
+def test_a_ring_step_equals_its_separate_calls(D, dtype, rotary):
     """The ring's write cursor goes round: the new row lies in any tile of any wavefront."""
     gen = torch.Generator(device="cuda").manual_seed(18)
     rope = kvhip.RoPE(D, base=1e4) if rotary else None
     caches = [kvhip.RotatingKVCache(1400, keep=4) for _ in range(2)]
-    k, v = _rows(gen, 1, 2, 1300, D, torch.bfloat16), _rows(gen, 1, 2, 1300, D, torch.bfloat16)
+    k, v = _rows(gen, 1, 2, 1300, D, dtype), _rows(gen, 1, 2, 1300, D, dtype)
     for c in caches:
         c._update(k, v)
     for i in range(400):
-        q, k, v = (_rows(gen, 1, h, 1, D, torch.bfloat16) for h in (8, 2, 2))
+        q, k, v = (_rows(gen, 1, h, 1, D, dtype) for h in (8, 2, 2))
         _compare(caches, q, k, v, rope)
     for a, b in zip(caches[0].state, caches[1].state):
         assert torch.equal(a, b)
