@@ -425,7 +425,7 @@ __global__ void __launch_bounds__(256) dequant_units_kernel(Store q, Store dst, 
 template <int NCK, int NCV> struct FpTile {
     static constexpr int KT = NCK <= 2 ? 32 : NCK <= 4 ? 16 : 8;  // tokens of a K piece
     static constexpr int KP = TILE / KT;
-    static constexpr int VC = NCV % 2 == 0 ? 64 : 32;             // columns of a V piece
+    static constexpr int VC = NCV % 2 == 0 ? 64 : 32 * NCV;       // columns of a V piece
     static constexpr int VP = 32 * NCV / VC;
     static constexpr int PIECES = KP + VP;
 };

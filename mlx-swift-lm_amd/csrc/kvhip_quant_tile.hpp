@@ -86,82 +86,79 @@ template <int DT> __device__ __forceinline__ uint32_t pack_scale_bias(float scal
     return (uint32_t)Elem<1>::bits(scale) | ((uint32_t)Elem<1>::bits(bias) << 16);
 }
 
-// grid (tiles touched, BH), 256 threads: rows src0 .. src0 + n - 1 go to slots slot0 .. slot0 + n - 1, which may start
-// and end inside a tile; 16-bit dtypes, Dk == Dv == 32 NC;
+// One workgroup of NT threads: rows src0 .. src0 + n - 1 go to slots slot0 .. slot0 + n - 1, which may start
+// and end inside a tile; 16-bit dtypes.
 // GL = group size / 8 lanes share a quantization group; ROPE = false carries no rotation code.
-// A thread holds 16-byte chunks of K and of V rows (a "chunk-instance" each), up to eight at a
+// A thread holds 16-byte chunks of rows (a "chunk-instance" each), up to four at a
 // time.  The extrema of every chunk-instance are reduced over the lanes of its group; then the
 // affine parameters -- four exact divisions, the costly part -- are worked out once per group
 // instead of once per lane: lane j of a group takes chunk-instance j (and j + GL, ...), writes
 // that group's (scale, bias) pair, and the other lanes fetch bias and reciprocal from it.
+// (Keys and values of a whole tile in one workgroup: 512 rows of
+// 8 heads x 128 with the queries of 32, 13.3 us; the conversion of 5000 rows of 16 (batch, head) pairs 23.9 us.)
 // PAGED: the 64 rows are tile `l_t / 64` of the full-precision page store `src` (a cache being
 // converted) instead of rows of dense arrays: K chunks are read from the interleaved tile where
 // they lie, the V tile (stored by column) is turned back into rows through LDS.
-// SIDE: 0 keys and values of one head size 32 NC; 1 the keys alone, 2 the values alone (caches whose keys and
-// values differ in head size take one launch for each, NC being that side's).
-template <int DT, int BITS, int NC, int GL, bool ROPE, bool PAGED, int SIDE = 0>
+// SIDE: 1 the keys, 2 the values (NC being that side's head size by 32).  A workgroup takes TOK tokens of a tile, from
+// token tok0 on, and COLS columns from col0 on: keys, which no column order asks for whole tiles of, go in pieces of few
+// tokens, values in whole tiles of up to 128 columns.
+template <int DT, int BITS, int NC, int GL, bool ROPE, bool PAGED, int SIDE, int NT, int TOK, int COLS>
 __device__ __forceinline__ void append_quant_tile_body(const Store &st, const Store &src, const char *keys, const char *values,
-                                                       int L, int src0, int slot0, int n, const RopeDev &rope) {
+                                                       int L, int src0, int slot0, int n, const RopeDev &rope, int tile, int tok0, int col0) {
     constexpr int D = 32 * NC;
     constexpr int GS = 8 * GL;
-    constexpr int TPR = D / 8;   // threads per row
-    constexpr int VP = D + 8;    // byte pitch of a token's V codes in LDS
-    constexpr bool DO_K = SIDE != 2, DO_V = SIDE != 1;
-    // chunks per batch (a divisor of NC; one side alone: a count whose instances share out evenly over a group's lanes)
-    constexpr int EB = SIDE == 0 ? (NC < 4 ? NC : 4) : (NC % 4 == 0 ? 4 : 2);
-    static_assert(NC % EB == 0, "a batch holds a whole number of chunks");
-    // chunk-instances per batch: both sides (chunk e0 + i / 2, K or V by i & 1), or one side's chunks e0 + i
-    constexpr int NI = SIDE == 0 ? 2 * EB : EB;
-    auto chunk_of = [](int i) { return SIDE == 0 ? i / 2 : i; };
-    auto is_v = [](int i) { return SIDE == 0 ? (i & 1) != 0 : SIDE == 2; };
-    constexpr int SH = GL < NI ? GL : NI;  // lanes of a group that work out parameters
-    constexpr int PER = (NI + SH - 1) / SH;  // chunk-instances per such lane (D = 96: six over four lanes, two of them take two)
-    // a row's TPR threads: where 256 is a multiple of TPR the rows of a thread's chunks are 256 / TPR apart and
+    constexpr int TPR = COLS / 8;   // threads per row
+    constexpr int VP = COLS + 8;    // byte pitch of a token's V codes in LDS
+    constexpr bool DO_K = SIDE == 1, DO_V = SIDE == 2;
+    static_assert(COLS % GS == 0 && (DO_K ? COLS == D : TOK == TILE), "whole groups; whole rows of keys, whole tiles of values");
+    constexpr int NCH = TOK * TPR / NT;  // chunks of a thread
+    static_assert(NCH * NT == TOK * TPR, "every thread holds as many");
+    constexpr int EB = NCH % 4 == 0 ? 4 : NCH % 3 == 0 ? 3 : NCH % 2 == 0 ? 2 : 1;  // chunks per batch
+    constexpr int SH = EB == 3 ? 4 : EB;  // lanes of a group that work out parameters, one chunk-instance each
+    // a row's TPR threads: where NT is a multiple of TPR the rows of a thread's chunks are NT / TPR apart and
     // its columns the same; at D = 96 (12 threads per row) row and column are worked out per chunk
-    constexpr bool EVEN = 256 % TPR == 0;
+    constexpr bool EVEN = NT % TPR == 0;
     constexpr bool GEN = BITS != 4 && BITS != 8;  // 2, 3, 5, 6 bits: codes as a plain bit stream, K rows and V tile rows alike
-    __shared__ __attribute__((aligned(8))) uint8_t vcodes[DO_V ? TILE * VP : 8];
-    __shared__ __attribute__((aligned(16))) uint8_t kcodes[GEN && DO_K ? TILE * D * BITS / 8 : 16];  // the tile's K rows as stored
+    // the source V tile as stored and, once every thread has its chunks of it, the codes
+    __shared__ __attribute__((aligned(16))) uint8_t vcodes[!DO_V ? 16 : PAGED ? TILE * COLS * 2 : TILE * VP];
+    __shared__ __attribute__((aligned(16))) uint8_t kcodes[GEN && DO_K ? TOK * D * BITS / 8 : 16];  // the K rows as stored
     __shared__ float inv_s[ROPE ? D / 2 : 1];
-    __shared__ __attribute__((aligned(16))) uint8_t vstage[PAGED && DO_V ? TILE * D * 2 : 16];  // the source V tile as stored
     const int bh = blockIdx.y;
-    const int slot_t = (slot0 & ~(TILE - 1)) + blockIdx.x * TILE;
+    const int slot_t = (slot0 & ~(TILE - 1)) + tile * TILE;
     const int l_t = src0 + slot_t - slot0;  // the row in the tile's first slot (before the first new row: t_lo > 0)
     // tokens [t_lo, t_hi) of the tile are new.  The threads of the others repeat the nearest new row, which keeps their
     // loads inside the arrays, and write nothing.
-    const int t_lo = PAGED ? 0 : max(slot0 - slot_t, 0), t_hi = PAGED ? TILE : min(slot0 + n - slot_t, TILE);
-    const bool whole = t_lo == 0 && t_hi == TILE;
-    const char *kbase = PAGED ? nullptr : keys + ((ptrdiff_t)bh * L + l_t) * D * 2;
-    const char *vbase = PAGED ? nullptr : values + ((ptrdiff_t)bh * L + l_t) * D * 2;
-    u4v kraw[NC], vraw[NC];
+    const int t_lo = PAGED ? 0 : max(slot0 - slot_t, 0), t_hi = min(PAGED ? TILE : slot0 + n - slot_t, tok0 + TOK);
+    if (DO_K && (tok0 >= t_hi || tok0 + TOK <= t_lo)) return;  // (workgroup-uniform)
+    const bool whole = t_lo <= tok0 && t_hi == tok0 + TOK;
+    const char *base = PAGED ? nullptr : (DO_K ? keys : values) + (((ptrdiff_t)bh * L + l_t) * D + col0) * 2;
+    u4v raw[NCH];
     if constexpr (PAGED) {
         const char *kt = k_cell_ptr(src, bh, l_t) + kfp_off(src, l_t, 0);   // tile start: [chunk][token][16 B]
         const char *vt = v_cell_ptr(src, bh, l_t) + vfp_off(src, l_t, 0);   // tile start: [8-token chunk][column][16 B]
 #pragma unroll
-        for (int e = 0; e < NC; ++e) {
-            const int c = e * 256 + threadIdx.x;
-            const int r = c / TPR, ch = c - r * TPR;
-            if constexpr (DO_K) kraw[e] = *reinterpret_cast<const u4v *>(kt + ((size_t)ch * TILE + r) * 16);
-            if constexpr (DO_V) *reinterpret_cast<u4v *>(vstage + (size_t)c * 16) = *reinterpret_cast<const u4v *>(vt + (size_t)c * 16);
+        for (int e = 0; e < NCH; ++e) {
+            const int c = e * NT + threadIdx.x;
+            if constexpr (DO_K) raw[e] = *reinterpret_cast<const u4v *>(kt + ((size_t)(c % TPR) * TILE + tok0 + c / TPR) * 16);
+            if constexpr (DO_V) *reinterpret_cast<u4v *>(vcodes + (size_t)c * 16) = *reinterpret_cast<const u4v *>(vt + ((size_t)(c / COLS) * D + col0 + c % COLS) * 16);
         }
         if constexpr (DO_V) __syncthreads();
 #pragma unroll
-        for (int e = 0; e < (DO_V ? NC : 0); ++e) {
-            const int c = e * 256 + threadIdx.x;
+        for (int e = 0; e < (DO_V ? NCH : 0); ++e) {
+            const int c = e * NT + threadIdx.x;
             const int r = c / TPR, dd = (c - r * TPR) * 8;
-            const uint16_t *col = reinterpret_cast<const uint16_t *>(vstage) + ((size_t)(r >> 3) * D + dd) * 8 + (r & 7);
+            const uint16_t *col = reinterpret_cast<const uint16_t *>(vcodes) + ((size_t)(r >> 3) * COLS + dd) * 8 + (r & 7);
             uint32_t u[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) u[j] = (uint32_t)col[(2 * j) * 8] | ((uint32_t)col[(2 * j + 1) * 8] << 16);
-            vraw[e] = u4v{u[0], u[1], u[2], u[3]};
+            raw[e] = u4v{u[0], u[1], u[2], u[3]};
         }
+        if constexpr (DO_V) __syncthreads();
     } else {
 #pragma unroll
-        for (int e = 0; e < NC; ++e) {
-            const int c = e * 256 + threadIdx.x, r = c / TPR;
-            const int cc = c + (min(max(r, t_lo), t_hi - 1) - r) * TPR;
-            if constexpr (DO_K) kraw[e] = *reinterpret_cast<const u4v *>(kbase + (ptrdiff_t)cc * 16);
-            if constexpr (DO_V) vraw[e] = *reinterpret_cast<const u4v *>(vbase + (ptrdiff_t)cc * 16);
+        for (int e = 0; e < NCH; ++e) {
+            const int c = e * NT + threadIdx.x, r = tok0 + c / TPR;
+            raw[e] = *reinterpret_cast<const u4v *>(base + ((ptrdiff_t)min(max(r, t_lo), t_hi - 1) * D + (c % TPR) * 8) * 2);
         }
     }
     if constexpr (ROPE) {
@@ -173,25 +170,25 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
     const int pos = lane & (GL - 1);            // place in the group
     const int psel = pos & (SH - 1);
     const int gbase4 = (lane & ~(GL - 1)) * 4;  // byte address (lane number x 4) of the group's first lane
-    const int r_t = threadIdx.x / TPR;          // row of this thread's chunk 0; chunk e lies 256 / TPR rows further
-    const int d0_t = (threadIdx.x - r_t * TPR) * 8;
-    auto row_of = [&](int e) { return EVEN ? r_t + e * (256 / TPR) : (e * 256 + (int)threadIdx.x) / TPR; };
-    auto col_of = [&](int e) { return EVEN ? d0_t : ((e * 256 + (int)threadIdx.x) % TPR) * 8; };
+    const int r_t = tok0 + threadIdx.x / TPR;   // row of this thread's chunk 0; chunk e lies NT / TPR rows further
+    const int d0_t = (threadIdx.x % TPR) * 8;   // (columns count from col0)
+    auto row_of = [&](int e) { return EVEN ? r_t + e * (NT / TPR) : tok0 + (e * NT + (int)threadIdx.x) / TPR; };
+    auto col_of = [&](int e) { return EVEN ? d0_t : ((e * NT + (int)threadIdx.x) % TPR) * 8; };
     const int page_off = (slot_t & (PAGE - 1));
-    const PageEntry page = st.pt[slot_t >> PAGE_SHIFT];  // a tile lies inside one page
+    const ptab entry = page_table(st) + (slot_t >> PAGE_SHIFT);  // a tile lies inside one page
+    const PageEntry page{entry->k, entry->ksb, entry->v, entry->vsb};
 #pragma unroll
-    for (int e0 = 0; e0 < NC; e0 += EB) {
-        float w[NI][8], mn[NI], mx[NI];
+    for (int e0 = 0; e0 < NCH; e0 += EB) {
+        float w[EB][8], mn[EB], mx[EB];
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int e = e0 + chunk_of(i);
+        for (int i = 0; i < EB; ++i) {
+            const int e = e0 + i;
             const int d0 = col_of(e);
-            if (!is_v(i)) {
+            if constexpr (ROPE && DO_K) {
                 const int r = min(max(row_of(e), t_lo), t_hi - 1);
-                if constexpr (ROPE) unpack8<DT>(kraw[e], kbase + (size_t)r * D * 2, d0, rope, inv_s, rope_pos(rope, bh, l_t + r), w[i]);
-                else chunk_unpack<DT>(kraw[e], w[i]);
+                unpack8<DT>(raw[e], base + (size_t)r * D * 2, d0, rope, inv_s, rope_pos(rope, bh, l_t + r), w[i]);
             } else {
-                chunk_unpack<DT>(vraw[e], w[i]);
+                chunk_unpack<DT>(raw[e], w[i]);
             }
             float a = w[i][0], b = w[i][0];
 #pragma unroll
@@ -203,39 +200,35 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
             mn[i] = a;
             mx[i] = b;
         }
-        float sc[PER], bi[PER], iv[PER];
+        float sc, bi, iv;  // of chunk-instance psel (the fourth of three: the first again, which nobody asks for)
+        {
+            float a = mn[0], b = mx[0];
 #pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            float a = mn[k * SH], b = mx[k * SH];
-#pragma unroll
-            for (int j = 1; j < SH; ++j)
-                if (k * SH + j < NI) {
-                    a = psel == j ? mn[k * SH + j] : a;
-                    b = psel == j ? mx[k * SH + j] : b;
-                }
-            affine_params(a, b, nb, sc[k], bi[k]);
-            iv[k] = __builtin_amdgcn_rcpf(sc[k]);
-            const int t_sb = row_of(e0 + chunk_of(psel + k * SH));
-            if (pos < SH && psel + k * SH < NI && t_sb >= t_lo && t_sb < t_hi) {
-                const int i = psel + k * SH;  // this lane's chunk-instance
+            for (int j = 1; j < EB; ++j) {
+                a = psel == j ? mn[j] : a;
+                b = psel == j ? mx[j] : b;
+            }
+            affine_params(a, b, nb, sc, bi);
+            iv = __builtin_amdgcn_rcpf(sc);
+            const int e = e0 + psel, t_sb = row_of(e);
+            if (pos < SH && psel < EB && t_sb >= t_lo && t_sb < t_hi) {
                 const int row = page_off + t_sb;
-                const int d0 = col_of(e0 + chunk_of(i));
-                char *sb = is_v(i) ? page.vsb + (size_t)bh * st.vsb_cell + (size_t)row * st.vsb_row
-                                   : page.ksb + (size_t)bh * st.ksb_cell + (size_t)row * st.ksb_row;
-                reinterpret_cast<uint32_t *>(sb)[d0 / GS] = pack_scale_bias<DT>(sc[k], bi[k]);
+                char *sb = DO_V ? page.vsb + (size_t)bh * st.vsb_cell + (size_t)row * st.vsb_row
+                                : page.ksb + (size_t)bh * st.ksb_cell + (size_t)row * st.ksb_row;
+                reinterpret_cast<uint32_t *>(sb)[(col0 + col_of(e)) / GS] = pack_scale_bias<DT>(sc, bi);
             }
         }
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int e = e0 + chunk_of(i);
+        for (int i = 0; i < EB; ++i) {
+            const int e = e0 + i;
             const int r = row_of(e), d0 = col_of(e);
-            const int src = gbase4 + (i % SH) * 4;
-            const float scale = lane_value(src, sc[i / SH]);
-            const float bias = lane_value(src, bi[i / SH]);
-            const float inv = lane_value(src, iv[i / SH]);
+            const int src = gbase4 + i * 4;
+            const float scale = lane_value(src, sc);
+            const float bias = lane_value(src, bi);
+            const float inv = lane_value(src, iv);
             float q[8];
             codes8<BITS>(w[i], scale, bias, inv, q);
-            if (!is_v(i)) {
+            if constexpr (DO_K) {
                 // ---- K: packed words in natural order --------------------------------------------
                 uint32_t *kw = reinterpret_cast<uint32_t *>(page.k + (size_t)bh * st.k_cell + (size_t)(page_off + r) * st.k_row);
                 if (!GEN && (r < t_lo || r >= t_hi)) continue;
@@ -250,7 +243,7 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
                     uint64_t bits8 = 0;
 #pragma unroll
                     for (int j = 0; j < 8; ++j) bits8 |= (uint64_t)(uint32_t)q[j] << (j * BITS);
-                    uint8_t *kb = &kcodes[r * (D * BITS / 8) + (d0 / 8) * BITS];
+                    uint8_t *kb = &kcodes[(r - tok0) * (D * BITS / 8) + (d0 / 8) * BITS];
 #pragma unroll
                     for (int j = 0; j < BITS; ++j) kb[j] = (uint8_t)(bits8 >> (8 * j));
                 }
@@ -263,82 +256,136 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
     }
     if constexpr (GEN && DO_K) {
         __syncthreads();
-        char *kt = page.k + (size_t)bh * st.k_cell + (size_t)page_off * st.k_row;  // 64 rows of D BITS / 8 bytes, contiguous
+        char *kt = page.k + (size_t)bh * st.k_cell + (size_t)(page_off + tok0) * st.k_row;  // TOK rows of D BITS / 8 bytes, contiguous
         if (whole) {
-            for (int c = threadIdx.x; c < TILE * D * BITS / 8 / 16; c += 256)
+            for (int c = threadIdx.x; c < TOK * D * BITS / 8 / 16; c += NT)
                 *reinterpret_cast<u4v *>(kt + (size_t)c * 16) = *reinterpret_cast<const u4v *>(&kcodes[c * 16]);
         } else {  // (rows are whole words: D is a multiple of 32)
             constexpr int RW = D * BITS / 32;
-            for (int c = t_lo * RW + threadIdx.x; c < t_hi * RW; c += 256)
+            for (int c = max(t_lo - tok0, 0) * RW + threadIdx.x; c < min(t_hi - tok0, TOK) * RW; c += NT)
                 reinterpret_cast<uint32_t *>(kt)[c] = reinterpret_cast<const uint32_t *>(kcodes)[c];
         }
     }
     if constexpr (!DO_V) return;
-    if constexpr (!(GEN && DO_K)) __syncthreads();
-    char *cell = page.v + (size_t)bh * st.v_cell + v_row_off(st, slot_t, 0);
+    __syncthreads();
+    char *cell = page.v + (size_t)bh * st.v_cell + v_row_off(st, slot_t, col0);
     if constexpr (GEN) {
-        // a transposed row is the bit stream of its 64 tokens' codes, 2 BITS words: each thread assembles one word
-        // from the codes that have bits in it; consecutive threads write consecutive words
-        constexpr int WPR = 2 * BITS;
-        for (int c = threadIdx.x; c < D * WPR; c += 256) {
-            const int d = c / WPR, w = c - d * WPR;
-            const int t0 = (32 * w) / BITS;  // the first token with bits in word w
-            uint32_t word = 0, mine = 0;  // (mine: the bits of new tokens)
+        // a transposed row is the bit stream of its 64 tokens' codes: 32 tokens fill BITS words, which a thread
+        // assembles with every shift a constant; consecutive threads write consecutive words.  (A word to a thread, whose
+        // first token depends on the word: 3 bits, 2048 rows of 64 pairs x 128: 33.9 us for 24.0.)
+        for (int c = threadIdx.x; c < COLS * 2; c += NT) {
+            const int d = c >> 1, t0 = (c & 1) * 32;
+            uint32_t word[BITS] = {}, mine[BITS] = {};  // (mine: the bits of new tokens)
 #pragma unroll
-            for (int i = 0; i < 32 / BITS + 2; ++i) {
-                const int t = t0 + i;
-                if (t < TILE && t * BITS < 32 * w + 32 && t >= t_lo && t < t_hi) {
-                    word |= stream_bits(vcodes[t * VP + d], t * BITS, w);
-                    mine |= stream_bits((1u << BITS) - 1u, t * BITS, w);
+            for (int t = 0; t < 32; ++t) {
+                const uint32_t code = vcodes[(t0 + t) * VP + d];
+                const uint32_t ones = t0 + t >= t_lo && t0 + t < t_hi ? (1u << BITS) - 1u : 0u;
+                const int w = t * BITS / 32, sh = t * BITS % 32;
+                word[w] |= code << sh;
+                mine[w] |= ones << sh;
+                if (sh + BITS > 32) {
+                    word[w + 1] |= code >> (32 - sh);
+                    mine[w + 1] |= ones >> (32 - sh);
                 }
             }
-            uint32_t *p = reinterpret_cast<uint32_t *>(cell + (size_t)d * (TILE * BITS / 8)) + w;
-            if (mine == 0xffffffffu) *p = word;
-            else if (mine != 0) *p = (*p & ~mine) | word;
+            uint32_t *p = reinterpret_cast<uint32_t *>(cell + (size_t)d * (TILE * BITS / 8)) + (c & 1) * BITS;
+#pragma unroll
+            for (int w = 0; w < BITS; ++w) {
+                if (mine[w] == 0xffffffffu) p[w] = word[w];
+                else if (mine[w] != 0) p[w] = (p[w] & ~mine[w]) | (word[w] & mine[w]);
+            }
         }
         return;
     }
-    // each thread assembles 16 bytes (4 words) of one transposed row; consecutive threads
-    // continue the same row, so the tile rows are written contiguously
+    // Two words of the transposed rows of four columns to a thread: tokens are read four codes at a time, nibbles paired
+    // with the bytes still side by side and the bytes turned by permutes, in the order v_bitpos gives.  Consecutive threads
+    // continue the rows.  (A row's 16 bytes to a thread, code by code: 4 bits, 2048 rows of 64 pairs x 128, 19.5 us for
+    // 19.2; 8 bits 23.8 for 21.5.)
     constexpr int TPW = 32 / BITS;        // tokens per word
-    constexpr int CPR = TILE / TPW / 4;   // 16-byte chunks per row
-    for (int c = threadIdx.x; c < D * CPR; c += 256) {
-        const int d = c / CPR, q = c - d * CPR;
-        uint32_t out[4];
+    constexpr int CPR = TILE / TPW / 2;   // 8-byte chunks per row
+    for (int c = threadIdx.x; c < COLS / 4 * CPR; c += NT) {
+        const int d = c / CPR * 4, q = c % CPR;
+        uint32_t out[4][2];
 #pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            uint32_t word = 0;
+        for (int wi = 0; wi < 2; ++wi) {
+            uint32_t in[TPW];  // one token's codes of the four columns
 #pragma unroll
-            for (int tt = 0; tt < TPW; ++tt) {
-                const int t = (4 * q + wi) * TPW + tt;
-                word |= (uint32_t)vcodes[t * VP + d] << (v_bitpos<BITS>(t) & 31);
+            for (int t = 0; t < TPW; ++t) in[t] = *reinterpret_cast<const uint32_t *>(&vcodes[((2 * q + wi) * TPW + t) * VP + d]);
+            uint32_t byte[4];  // byte j of the four columns' words
+            if constexpr (BITS == 4) {
+                byte[0] = in[0] | (in[2] << 4), byte[1] = in[4] | (in[6] << 4);
+                byte[2] = in[1] | (in[3] << 4), byte[3] = in[5] | (in[7] << 4);
+            } else {
+                byte[0] = in[0], byte[1] = in[2], byte[2] = in[1], byte[3] = in[3];
             }
-            out[wi] = word;
+            const uint32_t a01 = __builtin_amdgcn_perm(byte[1], byte[0], 0x05010400), a23 = __builtin_amdgcn_perm(byte[1], byte[0], 0x07030602);
+            const uint32_t b01 = __builtin_amdgcn_perm(byte[3], byte[2], 0x05010400), b23 = __builtin_amdgcn_perm(byte[3], byte[2], 0x07030602);
+            out[0][wi] = __builtin_amdgcn_perm(b01, a01, 0x05040100);
+            out[1][wi] = __builtin_amdgcn_perm(b01, a01, 0x07060302);
+            out[2][wi] = __builtin_amdgcn_perm(b23, a23, 0x05040100);
+            out[3][wi] = __builtin_amdgcn_perm(b23, a23, 0x07060302);
         }
-        char *dst = cell + (size_t)d * (TILE * BITS / 8) + 16 * q;
+        uint32_t *dst = reinterpret_cast<uint32_t *>(cell + (size_t)d * (TILE * BITS / 8) + 8 * q);
+        constexpr int RW = TILE * BITS / 32;  // words from row to row
         if (whole) {
-            *reinterpret_cast<u4v *>(dst) = u4v{out[0], out[1], out[2], out[3]};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<uint2 *>(dst + j * RW) = make_uint2(out[j][0], out[j][1]);
         } else {
 #pragma unroll
-            for (int wi = 0; wi < 4; ++wi) {
+            for (int wi = 0; wi < 2; ++wi) {
                 uint32_t mine = 0;  // the bits of new tokens in this word
 #pragma unroll
                 for (int tt = 0; tt < TPW; ++tt) {
-                    const int t = (4 * q + wi) * TPW + tt;
+                    const int t = (2 * q + wi) * TPW + tt;
                     if (t >= t_lo && t < t_hi) mine |= ((1u << BITS) - 1u) << (v_bitpos<BITS>(t) & 31);
                 }
-                uint32_t *p = reinterpret_cast<uint32_t *>(dst) + wi;
-                if (mine == 0xffffffffu) *p = out[wi];
-                else if (mine != 0) *p = (*p & ~mine) | (out[wi] & mine);
+                if (mine == 0) continue;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    uint32_t *p = dst + j * RW + wi;
+                    *p = mine == 0xffffffffu ? out[j][wi] : (*p & ~mine) | (out[j][wi] & mine);
+                }
             }
         }
     }
 }
 
-// (Rotating 128 columns in bfloat16 it would take 169 registers, with the call for large angles in it, one more than
-// three wavefronts per SIMD allow: 512 rows of 64 (batch, head) pairs 24.2 us, a second round of workgroups, against 20.5.)
+// How a tile's work is cut: workgroups of NT threads, K in pieces of TOK tokens, V in blocks of COLS columns.  Rows that
+// turn: few chunks to a thread, each of eight angles (2048 rows of 64 (batch, head) pairs, 4 bits: x 128 38.7 us with keys
+// and values of a tile in one workgroup, 33.2 so; 32 pairs x 256 26.2 and 19.1).  Others: the chunks of a group share the
+// lanes that work out parameters, so up to four to a thread (x 128 20.5 and 19.2 us; 8 bits 23.1 and 21.5; 3 bits 30.3 and
+// 24.0).  With 128 threads and eight chunks it was 22.6.  PAGED in blocks of 64 columns, whose LDS -- the workgroups of K
+// are charged it too -- decides how many fit a CU (the conversion above: 15.5 us, 25.2 with blocks of 128 columns).
+// (NC = 3: 192 threads, of which every row takes twelve.)
+template <int NC, int GL, int SIDE, bool ROPE, bool PAGED> struct QuantTile {
+    static constexpr int NT = NC == 3 ? 192 : 256;
+    static constexpr int TOK = ROPE ? (NC == 2 ? 32 : NC <= 4 ? 16 : NC == 8 ? 8 : TILE) : NC >= 6 ? 32 : TILE;
+    static constexpr int COLS = NC == 3 ? 96 : PAGED ? (GL > 8 ? 128 : 64) : NC > 4 ? 128 : 32 * NC;
+    static constexpr int KP = SIDE == 2 ? 0 : TILE / TOK, VP = SIDE == 1 ? 0 : 32 * NC / COLS;
+    static constexpr int PIECES = KP + VP;
+};
+// piece `piece` of tile `tile`: the values first, whose workgroups take the longer
+template <int DT, int BITS, int NC, int GL, bool ROPE, bool PAGED, int SIDE>
+__device__ __forceinline__ void quant_tile_piece(const Store &st, const Store &src, const char *keys, const char *values, int L, int src0, int slot0,
+                                                 int n, const RopeDev &rope) {
+    using Q = QuantTile<NC, GL, SIDE, ROPE, PAGED>;
+    const int tile = blockIdx.x / Q::PIECES, piece = blockIdx.x - tile * Q::PIECES;
+    if constexpr (SIDE != 1) {
+        if (SIDE == 2 || piece < Q::VP) {
+            append_quant_tile_body<DT, BITS, NC, GL, false, PAGED, 2, Q::NT, TILE, Q::COLS>(st, src, keys, values, L, src0, slot0, n, rope, tile, 0,
+                                                                                            piece * Q::COLS);
+            return;
+        }
+    }
+    if constexpr (SIDE != 2)
+        append_quant_tile_body<DT, BITS, NC, GL, ROPE, PAGED, 1, Q::NT, Q::TOK, 32 * NC>(st, src, keys, values, L, src0, slot0, n, rope, tile,
+                                                                                         (piece - Q::VP) * Q::TOK, 0);
+}
+
+// SIDE: 0 keys and values of one head size 32 NC; 1 the keys alone, 2 the values alone (caches whose keys and
+// values differ in head size take one launch for each, NC being that side's).
 template <int DT, int BITS, int NC, int GL, bool ROPE, int SIDE = 0>
-__global__ void __launch_bounds__(256, ROPE && NC == 4 ? 3 : 1)
+__global__ void __launch_bounds__((QuantTile<NC, GL, SIDE, ROPE, false>::NT))
 append_quant_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, int n, RopeDev rope) {
     if constexpr (ROPE) {
         if ((int)blockIdx.y >= st.BH) {  // queries of the same forward
@@ -347,13 +394,13 @@ append_quant_tile_kernel(Store st, const char *keys, const char *values, int L, 
             return;
         }
     }
-    append_quant_tile_body<DT, BITS, NC, GL, ROPE, false, SIDE>(st, st, keys, values, L, src0, slot0, n, rope);
+    quant_tile_piece<DT, BITS, NC, GL, ROPE, false, SIDE>(st, st, keys, values, L, src0, slot0, n, rope);
 }
 
-// grid (tiles, BH): tiles [0, gridDim.x) of the full-precision store `src` into the same slots of `st`
+// grid (pieces of tiles, BH): the tiles of the full-precision store `src` into the same slots of `st`
 template <int DT, int BITS, int NC, int GL, int SIDE = 0>
-__global__ void __launch_bounds__(256) requant_tile_kernel(Store st, Store src) {
-    append_quant_tile_body<DT, BITS, NC, GL, false, true, SIDE>(st, src, nullptr, nullptr, 0, 0, 0, 0, RopeDev());
+__global__ void __launch_bounds__((QuantTile<NC, GL, SIDE, false, true>::NT)) requant_tile_kernel(Store st, Store src) {
+    quant_tile_piece<DT, BITS, NC, GL, false, true, SIDE>(st, src, nullptr, nullptr, 0, 0, 0, 0, RopeDev());
 }
 
 // Which stores the tile kernels take: 16-bit dtypes, group size 32 / 64 / 128 dividing the head size; keys and
@@ -373,17 +420,19 @@ inline bool quant_tiles_two_sided(const Store &st) {
 template <int DT, int BITS, int NC, int GL, int SIDE, bool PAGED>
 void launch_quant_tile_instance(const Store &st, const Store &src, const void *keys, const void *values, int L, int a0,
                                 int b0, int n, hipStream_t s, const RopeDev &r) {
-    dim3 grid((PAGED ? (n + TILE - 1) : ((b0 & (TILE - 1)) + n + TILE - 1)) / TILE, st.BH), block(256);
+    const int tiles = (PAGED ? (n + TILE - 1) : ((b0 & (TILE - 1)) + n + TILE - 1)) / TILE;
     if constexpr (PAGED) {
-        hipLaunchKernelGGL((requant_tile_kernel<DT, BITS, NC, GL, SIDE>), grid, block, 0, s, st, src);
+        using Q = QuantTile<NC, GL, SIDE, false, true>;
+        hipLaunchKernelGGL((requant_tile_kernel<DT, BITS, NC, GL, SIDE>), dim3(tiles * Q::PIECES, st.BH), dim3(Q::NT), 0, s, st, src);
+    } else if (r.dims > 0 && SIDE != 2) {
+        using Q = QuantTile<NC, GL, SIDE, true, false>;
+        const int gx = tiles * Q::PIECES;
+        hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, true, SIDE>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es)), dim3(Q::NT), 0, s, st,
+                           (const char *)keys, (const char *)values, L, a0, b0, n, r);
     } else {
-        if (SIDE != 2) grid.y += rope_ride_rows(r, grid.x, st.es);
-        if (r.dims > 0 && SIDE != 2)
-            hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, true, SIDE>), grid, block, 0, s, st,
-                               (const char *)keys, (const char *)values, L, a0, b0, n, r);
-        else
-            hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, false, SIDE>), grid, block, 0, s, st,
-                               (const char *)keys, (const char *)values, L, a0, b0, n, r);
+        using Q = QuantTile<NC, GL, SIDE, false, false>;
+        hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, false, SIDE>), dim3(tiles * Q::PIECES, st.BH), dim3(Q::NT), 0, s, st,
+                           (const char *)keys, (const char *)values, L, a0, b0, n, r);
     }
 }
 
@@ -398,7 +447,8 @@ hipError_t launch_quant_tiles_dt(const Store &st, const Store &src, const void *
         else KV_TILE(NC, 16, 0);              \
     } while (0)
     if (quant_tiles_one_launch(st)) {
-        if (st.Dk == 64) KV_TILE_GL(2);
+        if (st.Dk == 64 && st.gs == 32) KV_TILE(2, 4, 0);
+        else if (st.Dk == 64) KV_TILE(2, 8, 0);
         else if (st.Dk == 96) KV_TILE(3, 4, 0);
         else if (st.Dk == 128) KV_TILE_GL(4);
         else KV_TILE_GL(8);
