@@ -126,6 +126,27 @@ def load():
     return _lib
 
 
+_step = None
+
+
+def step():
+    """The extension that carries a layer's attention call from its tensors to the library (csrc/py/kvhip_step.cpp), and the
+    addresses of its two entry points: (module, update_attend, update_attend_rope).  Raises if it is not built."""
+    global _step
+    if _step is None:
+        import torch
+
+        from . import _step as module
+        from .rope import RoPE
+
+        module.bind(torch.Tensor, RoPE, (torch.float16, torch.bfloat16, torch.float32), torch._C._cuda_getDevice,
+                    torch._C._cuda_getCurrentRawStream)
+        lib = load()
+        at = [C.cast(getattr(lib, name), C.c_void_p).value for name in ("kvhip_cache_update_attend", "kvhip_cache_update_attend_rope")]
+        _step = (module, at[0], at[1])
+    return _step
+
+
 def check(status):
     if status < 0:
         msg = load().kvhip_last_error_message()

@@ -13,7 +13,7 @@ def attention_with_cache_update(queries, keys, values, cache, scale, mask=None):
     """
     if cache is None:
         raise ValueError("a kvhip cache is required; cache-less attention is outside this path")
-    return cache.update_attend(queries, keys, values, scale, mask or MaskMode.none())
+    return cache.update_attend(queries, keys, values, scale, mask)
 
 
 def quantized_scaled_dot_product_attention(queries, cache: QuantizedKVCache, scale, mask=None):

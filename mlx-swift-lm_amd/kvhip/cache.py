@@ -101,6 +101,7 @@ class MaskMode:
 
 # masks that are nothing but their mode, read by the library and never written
 _PLAIN = {L.MASK_NONE: L.Mask(mode=L.MASK_NONE), L.MASK_CAUSAL: L.Mask(mode=L.MASK_CAUSAL)}
+_PLAIN_AT = {mode: C.addressof(m) for mode, m in _PLAIN.items()}
 # rotated queries up to this size stay in a buffer of the cache's; larger ones are allocated for the call
 _Q_ROTATED_KEPT = 1 << 18
 
@@ -111,6 +112,7 @@ class _Cache:
     def __init__(self, handle=None, **cfg):
         L.init()
         self._lib = L.load()
+        self._step, self._step_at, self._step_rope_at = L.step()
         if handle is None:
             c = L.Config(kind=self.kind, step=cfg.get("step", 0), max_size=cfg.get("max_size", 0),
                          keep=cfg.get("keep", 0), group_size=cfg.get("group_size", 0), bits=cfg.get("bits", 0))
@@ -243,8 +245,27 @@ class _Cache:
         del keep
         return out
 
+    def _attend_natively(self, rope, queries, keys, values, scale, mask):
+        """The call as one native step, if it is of the ordinary form (contiguous arrays that go together and with what the
+        cache holds, no mask or the causal one): the output, or None with nothing done."""
+        at = _PLAIN_AT.get(mask.mode if type(mask) is MaskMode else None if mask else L.MASK_NONE)
+        if at is None:
+            return None
+        out = self._step.attend(self._step_at if rope is None else self._step_rope_at, self._h.value, self._shape, queries, keys, values,
+                                scale, at, rope, _Q_ROTATED_KEPT)
+        if type(out) is int:
+            # (a captured rotary step that needs room for its queries is refused before anything is written: the
+            # general path hands it some)
+            if out == L.ERR_UNSUPPORTED and rope is not None and torch.cuda.is_current_stream_capturing():
+                return None
+            L.check(out)
+        return out
+
     def update_attend(self, queries, keys, values, scale, mask=None):
         """`attentionWithCacheUpdate` for this cache (AttentionUtils.swift:37-95)."""
+        out = self._attend_natively(None, queries, keys, values, scale, mask)
+        if out is not None:
+            return out
         q, k, v = queries.contiguous(), keys.contiguous(), values.contiguous()
         self._check_query_dtype(q, k)
         B, Hq, Lq, D = q.shape
@@ -261,6 +282,9 @@ class _Cache:
 
     def update_attend_rope(self, rope, queries, keys, values, scale, mask=None, batch_offsets=None):
         """Queries and keys rotated at this cache's `ropeOffset` (or at `batch_offsets`), update, attention."""
+        out = self._attend_natively(rope, queries, keys, values, scale, mask) if batch_offsets is None else None
+        if out is not None:
+            return out
         q, k, v = queries.contiguous(), keys.contiguous(), values.contiguous()
         assert k.is_cuda and v.is_cuda and k.dtype == v.dtype
         if q.dtype != k.dtype:
