@@ -418,29 +418,48 @@ __global__ void __launch_bounds__(256) dequant_units_kernel(Store q, Store dst, 
 }
 
 // grid (tiles touched x pieces of a tile, BH), 256 threads: rows src0 .. src0 + n - 1 to slots slot0 .. slot0 + n - 1, which
-// may start and end inside a tile; 16-bit dtypes, Dk == 32 NCK, Dv == 32 NCV.  A tile's K rows go in pieces of 8 to 32
+// may start and end inside a tile; ES bytes an element, keys of DK and values of DV.  A tile's K rows go in pieces of 4 to 32
 // tokens, a 16-byte chunk to a thread, its V rows in blocks of columns that are turned through LDS: many short workgroups,
 // whose loads are all in flight at once and whose threads form the sines of one chunk.  (A workgroup to a tile, as it was,
 // walked four to sixteen chunks a thread: 512 rows of 8 heads x 128 with the queries of 32, 11.3 us.)
-template <int NCK, int NCV> struct FpTile {
-    static constexpr int KT = NCK <= 2 ? 32 : NCK <= 4 ? 16 : 8;  // tokens of a K piece
+// HBM-bound from a few thousand rows on: 2048 rows of 64 (batch, head) pairs x 128, 16-bit 20.8 us, float32 40.1 (6.7
+// TB/s); a row to a workgroup, whose values leave an element at a time, takes 113 us for the float32 rows, 70 for the
+// 14.4 of 2048 rows of 64 pairs x 80 and 88 for the 22.4 of 2048 rows of 16 pairs x 512.
+template <int ES, int DK, int DV> struct FpTile {
+    static constexpr int E = 16 / ES;     // elements of a chunk
+    static constexpr int TPRK = DK / E;   // chunks of a K row
+    static constexpr int KT = TPRK <= 8 ? 32 : TPRK <= 16 ? 16 : TPRK <= 32 ? 8 : 4;        // tokens of a K piece
     static constexpr int KP = TILE / KT;
-    static constexpr int VC = NCV % 2 == 0 ? 64 : 32 * NCV;       // columns of a V piece
-    static constexpr int VP = 32 * NCV / VC;
+    static constexpr int VC = ES == 4 ? 32 : DV % 64 == 0 ? 64 : DV;                        // columns of a V piece
+    static constexpr int VP = DV / VC;
     static constexpr int PIECES = KP + VP;
 };
-template <int NCK, int NCV>
+// the chunk `k` of `row` at d0, rotated
+template <int DT>
+__device__ __forceinline__ kv_u4 turned_chunk(const kv_u4 &k, const char *row, int d0, const RopeDev &rope, const float *inv_s, int pos) {
+    float w[rope_chunk_elems<DT>()];
+    if (rope.vec) {
+        rope_chunk<DT>(rope, inv_s, row, d0, pos, k, w);
+    } else {
+#pragma unroll
+        for (int j = 0; j < rope_chunk_elems<DT>(); ++j) w[j] = rope_elem<DT, true>(rope, row, d0 + j, pos);
+    }
+    return chunk_pack<DT>(w);
+}
+template <int ES, int DK, int DV>
 __global__ void __launch_bounds__(256)
 append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int src0, int slot0, int n, RopeDev rope) {
-    using P = FpTile<NCK, NCV>;
-    constexpr int DK = 32 * NCK, D = 32 * NCV;
-    constexpr int TPRK = DK / 8, TPR = P::VC / 8;  // chunks of a row, K and V (of the piece's columns)
-    constexpr int VPW = P::VC / 2 + 1;  // dword pitch of a token's V row in LDS (odd: column reads spread over banks)
+    using P = FpTile<ES, DK, DV>;
+    using T = typename std::conditional<ES == 2, uint16_t, uint32_t>::type;
+    constexpr int E = P::E, TPRK = P::TPRK, TPR = P::VC / E;  // chunks of a row, K and V (of the piece's columns)
+    constexpr int VPW = P::VC * ES / 4 + 1;  // dword pitch of a token's V row in LDS (odd: column reads spread over banks)
+    static_assert(DK % E == 0 && DV % P::VC == 0 && P::VC % E == 0 && P::KT * TPRK <= 256, "whole chunks, one to a thread");
     __shared__ uint32_t vt[TILE * VPW];
     __shared__ float inv_s[DK / 2];
     const int bh = blockIdx.y;
     if (bh >= st.BH) {  // queries of the same forward
-        if (st.dtype == KVHIP_F16) rope_queries_ride<0>(rope, st.BH, inv_s);
+        if constexpr (ES == 4) rope_queries_ride<2>(rope, st.BH, inv_s);
+        else if (st.dtype == KVHIP_F16) rope_queries_ride<0>(rope, st.BH, inv_s);
         else rope_queries_ride<1>(rope, st.BH, inv_s);
         return;
     }
@@ -452,42 +471,38 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
     auto new_row = [&](int r) { return min(max(r, t_lo), t_hi - 1); };
     if (piece < P::KP) {
         if (piece * P::KT >= t_hi || (piece + 1) * P::KT <= t_lo) return;  // (workgroup-uniform)
-        const int r = piece * P::KT + threadIdx.x / TPRK, d0 = (threadIdx.x % TPRK) * 8, rn = new_row(r);
+        const int r = piece * P::KT + threadIdx.x / TPRK, d0 = (threadIdx.x % TPRK) * E, rn = new_row(r);
         const bool live = threadIdx.x < P::KT * TPRK;
-        const char *row = keys + ((ptrdiff_t)bh * L + l_t + rn) * DK * 2;
-        u4v k{0u, 0u, 0u, 0u};
-        if (live) k = *reinterpret_cast<const u4v *>(row + 2 * d0);
+        const char *row = keys + ((ptrdiff_t)bh * L + l_t + rn) * DK * ES;
+        kv_u4 k{0u, 0u, 0u, 0u};
+        if (live) k = *reinterpret_cast<const kv_u4 *>(row + ES * d0);
         if (rope.dims > 0) {
             rope_inv_table(rope, inv_s);
             __syncthreads();
             if (live && d0 < rope.dims) {
                 const int pos = rope_pos(rope, bh, l_t + rn);
-                float w[8];
-                if (st.dtype == KVHIP_F16) {
-                    unpack8<0>(k, row, d0, rope, inv_s, pos, w);
-                    k = chunk_pack<0>(w);
-                } else {
-                    unpack8<1>(k, row, d0, rope, inv_s, pos, w);
-                    k = chunk_pack<1>(w);
-                }
+                if constexpr (ES == 4) k = turned_chunk<2>(k, row, d0, rope, inv_s, pos);
+                else if (st.dtype == KVHIP_F16) k = turned_chunk<0>(k, row, d0, rope, inv_s, pos);
+                else k = turned_chunk<1>(k, row, d0, rope, inv_s, pos);
             }
         }
         char *kcell = page_table(st)[slot_t >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;  // a tile lies inside one page
-        if (live && r >= t_lo && r < t_hi) *reinterpret_cast<u4v *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
+        if (live && r >= t_lo && r < t_hi) *reinterpret_cast<kv_u4 *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
         return;
     }
     const int c0 = (piece - P::KP) * P::VC;  // first column
-    const char *vbase = values + ((ptrdiff_t)bh * L + l_t) * D * 2 + 2 * c0;
-    constexpr int NV = TILE * TPR / 256;  // chunks of a thread
-    u4v vraw[NV];
+    const char *vbase = values + (((ptrdiff_t)bh * L + l_t) * DV + c0) * ES;
+    constexpr int CHUNKS = TILE * TPR, NV = (CHUNKS + 255) / 256;  // chunks of the piece, of a thread
+    kv_u4 vraw[NV];
 #pragma unroll
     for (int e = 0; e < NV; ++e) {
-        const int c = e * 256 + threadIdx.x, r = c / TPR;
-        vraw[e] = *reinterpret_cast<const u4v *>(vbase + (ptrdiff_t)new_row(r) * D * 2 + (c - r * TPR) * 16);
+        const int c = min(e * 256 + (int)threadIdx.x, CHUNKS - 1), r = c / TPR;
+        vraw[e] = *reinterpret_cast<const kv_u4 *>(vbase + (ptrdiff_t)new_row(r) * DV * ES + (c - r * TPR) * 16);
     }
 #pragma unroll
     for (int e = 0; e < NV; ++e) {
         const int c = e * 256 + threadIdx.x, r = c / TPR;
+        if (CHUNKS % 256 != 0 && c >= CHUNKS) break;
         uint32_t *vrow = &vt[r * VPW + (c - r * TPR) * 4];
         vrow[0] = vraw[e].x;
         vrow[1] = vraw[e].y;
@@ -495,26 +510,26 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
         vrow[3] = vraw[e].w;
     }
     __syncthreads();
-    // 8-token chunks of every column: thread (c8, d) gathers tokens 8 c8 .. 8 c8 + 7 of column d;
+    // chunks of E tokens of every column: a thread gathers tokens E ce .. E ce + E - 1 of column d;
     // consecutive threads take consecutive columns, so a chunk row is written contiguously
     char *cell = const_cast<char *>(v_cell_ptr(st, bh, slot_t));
-    const uint16_t *vt16 = reinterpret_cast<const uint16_t *>(vt);
-    for (int c = threadIdx.x; c < P::VC * 8; c += 256) {
-        const int c8 = c / P::VC, d = c - c8 * P::VC;
+    const T *vte = reinterpret_cast<const T *>(vt);
+    constexpr int VPE = VPW * 4 / ES;
+    for (int c = threadIdx.x; c < P::VC * (TILE / E); c += 256) {
+        const int t0 = c / P::VC * E, d = c % P::VC;
         uint32_t out[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const uint32_t lo = vt16[(8 * c8 + 2 * j) * (2 * VPW) + d];
-            const uint32_t hi = vt16[(8 * c8 + 2 * j + 1) * (2 * VPW) + d];
-            out[j] = lo | (hi << 16);
+            if constexpr (ES == 4) out[j] = vte[(t0 + j) * VPE + d];
+            else out[j] = (uint32_t)vte[(t0 + 2 * j) * VPE + d] | ((uint32_t)vte[(t0 + 2 * j + 1) * VPE + d] << 16);
         }
-        char *dst = cell + vfp_off(st, slot_t + 8 * c8, c0 + d);
-        if (8 * c8 >= t_lo && 8 * c8 + 8 <= t_hi) {
-            *reinterpret_cast<u4v *>(dst) = u4v{out[0], out[1], out[2], out[3]};
+        char *dst = cell + vfp_off(st, slot_t + t0, c0 + d);
+        if (t0 >= t_lo && t0 + E <= t_hi) {
+            *reinterpret_cast<kv_u4 *>(dst) = kv_u4{out[0], out[1], out[2], out[3]};
         } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (8 * c8 + j >= t_lo && 8 * c8 + j < t_hi) reinterpret_cast<uint16_t *>(dst)[j] = (uint16_t)(out[j >> 1] >> (16 * (j & 1)));
+            for (int j = 0; j < E; ++j)
+                if (t0 + j >= t_lo && t0 + j < t_hi) reinterpret_cast<T *>(dst)[j] = (T)(ES == 4 ? out[j] : out[j / 2] >> (16 * (j & 1)));
         }
     }
 }
@@ -839,25 +854,35 @@ hipError_t launch_append_fp(const Store &st, const void *keys, const void *value
                             int slot0, int n, hipStream_t s, RopeDev *rope) {
     if (n <= 0) return hipSuccess;
     const RopeDev r = take_rope(rope);
-    const bool mla = st.Dk == 192 && st.Dv == 128;  // keys of 192 with values of 128
-    const bool tiled = st.es == 2 && ((st.Dk == st.Dv && (st.Dk == 64 || st.Dk == 96 || st.Dk == 128 || st.Dk == 256)) || mla);
     // One launch for whole tiles and the pieces of tiles at either end.  Fewer rows than a tile go one to a workgroup:
     // that takes 5 us whatever their number, less than a tile's workgroup behind its barriers.
-    if (!tiled || n < TILE) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
+    if (n < TILE) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
     const int tiles = ((slot0 & (TILE - 1)) + n + TILE - 1) / TILE;
-#define FP_TILE(NCK, NCV)                                                                                                 \
+#define FP_TILE(ES, DK, DV)                                                                                               \
     do {                                                                                                                  \
-        const int gx = tiles * FpTile<NCK, NCV>::PIECES;                                                                  \
-        hipLaunchKernelGGL((append_fp_tile_kernel<NCK, NCV>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es)), dim3(256), 0, s, st, \
+        const int gx = tiles * FpTile<ES, DK, DV>::PIECES;                                                                \
+        hipLaunchKernelGGL((append_fp_tile_kernel<ES, DK, DV>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es)), dim3(256), 0, s, st, \
                            (const char *)keys, (const char *)values, L, src0, slot0, n, r);                               \
+        return hipGetLastError();                                                                                         \
     } while (0)
-    if (mla) FP_TILE(6, 4);
-    else if (st.Dk == 64) FP_TILE(2, 2);
-    else if (st.Dk == 96) FP_TILE(3, 3);
-    else if (st.Dk == 128) FP_TILE(4, 4);
-    else FP_TILE(8, 8);
+    if (st.es == 2) {
+        if (st.Dk == 192 && st.Dv == 128) FP_TILE(2, 192, 128);
+        if (st.Dk == st.Dv) {
+            if (st.Dk == 64) FP_TILE(2, 64, 64);
+            if (st.Dk == 80) FP_TILE(2, 80, 80);
+            if (st.Dk == 96) FP_TILE(2, 96, 96);
+            if (st.Dk == 128) FP_TILE(2, 128, 128);
+            if (st.Dk == 256) FP_TILE(2, 256, 256);
+            if (st.Dk == 512) FP_TILE(2, 512, 512);
+        }
+    } else if (st.Dk == st.Dv) {
+        if (st.Dk == 64) FP_TILE(4, 64, 64);
+        if (st.Dk == 96) FP_TILE(4, 96, 96);
+        if (st.Dk == 128) FP_TILE(4, 128, 128);
+        if (st.Dk == 256) FP_TILE(4, 256, 256);
+    }
 #undef FP_TILE
-    return hipGetLastError();
+    return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);  // other head sizes
 }
 
 hipError_t launch_rope_apply(const RopeDev &rope, const void *x, void *out, int B, int H, int L, int D,

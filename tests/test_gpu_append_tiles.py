@@ -1,0 +1,44 @@
+"""Full-precision appends of a tile and more at the head sizes and types that share the tile kernel: pieces that begin and
+end inside tiles, and rows whose memory begins at an odd element, give the bits that single rows give (moved, not computed;
+the rotation is the same elementwise function of position and pair)."""
+import pytest
+import torch
+
+import kvhip
+
+pytestmark = pytest.mark.gpu
+
+PIECES = [64, 5, 65, 130, 64, 200]  # a whole tile, then starts and ends inside tiles and pages
+
+
+def _shifted(x):
+    """`x` in memory that begins one element behind a 16-byte boundary."""
+    flat = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:].view(x.shape)
+    return flat.copy_(x)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 80), (torch.bfloat16, 80), (torch.float16, 512), (torch.bfloat16, 512),
+                                     (torch.float32, 64), (torch.float32, 96), (torch.float32, 128), (torch.float32, 256)])
+@pytest.mark.parametrize("rotary", ["none", "halves", "pairs", "part", "odd", "queries"])
+def test_tiles_equal_single_rows(dtype, D, rotary):
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    rope = {"none": None, "halves": kvhip.RoPE(D, base=5e5), "pairs": kvhip.RoPE(D, traditional=True), "part": kvhip.RoPE(D // 2),
+            "odd": kvhip.RoPE(20), "queries": kvhip.RoPE(D)}[rotary]
+    tiled, single = kvhip.KVCacheSimple(), kvhip.KVCacheSimple()
+    for piece, n in enumerate(PIECES):
+        q, k, v = (torch.randn(2, h, n, D, generator=gen, device="cuda").to(dtype) for h in (6, 3, 3))
+        kk, vv = (k, v) if piece % 2 == 0 else (_shifted(k), _shifted(v))
+        if rotary == "queries":
+            tiled.update_attend_rope(rope, q, kk, vv, D ** -0.5)
+        elif rope is not None:
+            tiled.update_rope(rope, kk, vv)
+        else:
+            tiled.update(kk, vv, fetch=False)
+        for i in range(n):
+            row = k[:, :, i:i + 1].contiguous(), v[:, :, i:i + 1].contiguous()
+            if rope is not None:
+                single.update_rope(rope, *row)
+            else:
+                single.update(*row, fetch=False)
+    for a, b in zip(tiled.state, single.state):
+        assert a.shape == b.shape and torch.equal(a, b)
