@@ -854,9 +854,13 @@ hipError_t launch_append_fp(const Store &st, const void *keys, const void *value
                             int slot0, int n, hipStream_t s, RopeDev *rope) {
     if (n <= 0) return hipSuccess;
     const RopeDev r = take_rope(rope);
-    // One launch for whole tiles and the pieces of tiles at either end.  Fewer rows than a tile go one to a workgroup:
-    // that takes 5 us whatever their number, less than a tile's workgroup behind its barriers.
-    if (n < TILE) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
+    // One launch for whole tiles and the pieces of tiles at either end.  Few rows go one to a workgroup, which takes 3 us
+    // until there are more of them than run at once.  Row / tile kernel, us: 16-bit rows x 128, of 128 (batch, head) pairs,
+    // 8 each 3.1 / 3.5, 16 4.3 / 3.5, 63 9.0 / 4.0; of 8 pairs, 63 each 2.8 / 3.1; x 256, 32 pairs, 16 each 3.5 / 3.5, 24
+    // 3.8 / 3.4; x 64, 128 pairs, 16 each 3.3 / 3.2, 32 4.6 / 3.2; float32 x 128, 32 pairs, 16 each 3.1 / 3.0, 48 4.3 / 3.1.
+    // (Queries that ride are the longer part of whichever launch takes them.)
+    const bool many = n >= 16 && (size_t)n * st.BH * (st.Dk + st.Dv) * st.es > (512u << 10);
+    if (!many && (n < TILE || !r.qx)) return launch_append_fp_rows(st, keys, values, L, src0, slot0, n, s, r);
     const int tiles = ((slot0 & (TILE - 1)) + n + TILE - 1) / TILE;
 #define FP_TILE(ES, DK, DV)                                                                                               \
     do {                                                                                                                  \
@@ -928,15 +932,14 @@ hipError_t launch_append_quant_rows(const Store &st, const void *keys, const voi
 }  // namespace
 
 // Rows in one tile from which the tile quantizer is the faster one.  The row kernel's wavefronts take their rows one
-// after the other, 64 columns at a time (128 with groups of 128); a tile takes its time whatever its rows.  Row kernel at
-// the count just below / tile kernel there, 4 bits: D 128 11 / 12.5 us with the rotation, 7 / 7.2 without; D 256 groups
-// of 64 19 / 23 and 12.5 / 12.3, groups of 128 20 / 22.5 and 12.4 / 12.5; keys of 192 with values of 128 15 / 18 and 11 / 12.
+// after the other, 64 columns at a time (128 with groups of 128); a tile takes its time whatever its rows.  Row / tile
+// kernel, us, 4 bits, 128 (batch, head) pairs: x 128 rotated 5.5 / 5.2 for 2 rows, 6.0 / 5.3 for 4, 11.2 / 5.6 for 11;
+// as they are 4.6 / 5.0 for 4, 5.8 / 5.2 for 5; x 256, groups of 128, 7.4 / 5.9 rotated for 3 and 5.5 / 6.0, 7.1 / 6.0 for
+// 4 and 5; x 64 5.0 / 4.8 rotated for 4, 4.0 / 4.0 and 4.7 / 4.0 for 4 and 6.  Keys of 192 with values of 128 take two
+// launches: 9.4 / 9.6 for 9 and 10.8 / 9.6 for 12, rotated 13.6 / 12.6 and 15.2 / 12.3.
 int quant_tile_rows(const Store &st, bool rotated) {
-    const int D = std::max(st.Dk, st.Dv);
-    if (D <= 64 || (D <= 128 && !rotated)) return 9;
-    if (D <= 128) return D <= 96 ? 10 : 14;
-    if (st.gs == 128) return rotated ? 20 : 17;
-    return rotated ? 17 : 14;
+    if (quant_tiles_two_sided(st)) return 12;
+    return rotated ? 3 : 5;
 }
 
 hipError_t launch_append_quant(const Store &st, const void *keys, const void *values, int L, int src0,
@@ -944,9 +947,9 @@ hipError_t launch_append_quant(const Store &st, const void *keys, const void *va
     if (n <= 0) return hipSuccess;
     const RopeDev r = take_rope(rope);
     const bool tiled = quant_tiles_one_launch(st) || quant_tiles_two_sided(st);
-    // One launch of the tile kernel takes every row of its tiles at once, 7 to 25 us whatever their number; the row kernel's
+    // One launch of the tile kernel takes every row of its tiles at once, 4 to 12 us whatever their number; the row kernel's
     // wavefronts take theirs one after the other, each tile's in a workgroup of its own (33 us for 50 rows of 128).
-    // A 501-row piece at an odd slot, rotated: 50 us as rows, whole tiles, rows (three launches), 11.5 us so.
+    // A 501-row piece at an odd slot, rotated: 50 us as rows, whole tiles, rows (three launches), 7 us so.
     const int head = std::min(n, TILE - (slot0 & (TILE - 1)));
     const int most = std::max(head, std::min(n - head, TILE));
     if (!tiled || most < quant_tile_rows(st, r.dims > 0)) return launch_append_quant_rows(st, keys, values, L, src0, slot0, n, s, r);

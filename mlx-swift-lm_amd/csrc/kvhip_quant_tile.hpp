@@ -1,4 +1,4 @@
-// Quantize-on-append of many rows by 64-token tiles, whole ones and the partial ones at either end (from 9 to 20 rows up:
+// Quantize-on-append of many rows by 64-token tiles, whole ones and the partial ones at either end (from 3 to 12 rows up:
 // `quant_tile_rows`): the element functions, the tile body and its two kernels, and the launchers of one code width
 // (instantiated per width in kvhip_io.hip and kvhip_quant_tile_other.hip).
 #pragma once
@@ -356,10 +356,10 @@ __device__ __forceinline__ void append_quant_tile_body(const Store &st, const St
 // lanes that work out parameters, so up to four to a thread (x 128 20.5 and 19.2 us; 8 bits 23.1 and 21.5; 3 bits 30.3 and
 // 24.0).  With 128 threads and eight chunks it was 22.6.  PAGED in blocks of 64 columns, whose LDS -- the workgroups of K
 // are charged it too -- decides how many fit a CU (the conversion above: 15.5 us, 25.2 with blocks of 128 columns).
-// (NC = 3: 192 threads, of which every row takes twelve.)
+// (NC = 3, 6: 192 threads, of which every row takes twelve or twenty-four.)
 template <int NC, int GL, int SIDE, bool ROPE, bool PAGED> struct QuantTile {
-    static constexpr int NT = NC == 3 ? 192 : 256;
-    static constexpr int TOK = ROPE ? (NC == 2 ? 32 : NC <= 4 ? 16 : NC == 8 ? 8 : TILE) : NC >= 6 ? 32 : TILE;
+    static constexpr int NT = NC % 3 == 0 ? 192 : 256;
+    static constexpr int TOK = ROPE ? (NC == 2 ? 32 : NC <= 6 ? 16 : 8) : NC >= 6 ? 32 : TILE;
     static constexpr int COLS = NC == 3 ? 96 : PAGED ? (GL > 8 ? 128 : 64) : NC > 4 ? 128 : 32 * NC;
     static constexpr int KP = SIDE == 2 ? 0 : TILE / TOK, VP = SIDE == 1 ? 0 : 32 * NC / COLS;
     static constexpr int PIECES = KP + VP;

@@ -42,3 +42,25 @@ def test_tiles_equal_single_rows(dtype, D, rotary):
                 single.update(*row, fetch=False)
     for a, b in zip(tiled.state, single.state):
         assert a.shape == b.shape and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("bits,gs,dtype,Dk,Dv", [(4, 64, torch.float16, 128, 128), (8, 32, torch.bfloat16, 64, 64), (4, 128, torch.float16, 256, 256),
+                                                 (3, 32, torch.float16, 96, 96), (4, 64, torch.bfloat16, 192, 128), (0, 0, torch.float16, 128, 128),
+                                                 (0, 0, torch.bfloat16, 64, 64), (0, 0, torch.float32, 128, 128)])
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 12, 15, 16, 33, 63])
+def test_few_rows_equal_single_rows(bits, gs, dtype, Dk, Dv, n):
+    """Either side of the row counts from which tiles take over, in many (batch, head) pairs, from slots that leave the
+    rows in one tile, in two, and in two pages."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    for rope in (None, kvhip.RoPE(Dk)):
+        for at in (3, 256 - n // 2):
+            caches = [kvhip.QuantizedKVCache(gs, bits) if bits else kvhip.KVCacheSimple() for _ in range(2)]
+            k0, v0, k, v = (torch.randn(5, 16, m, d, generator=gen, device="cuda").to(dtype) for m in (at, n) for d in (Dk, Dv))
+            for c in caches:
+                c._update(k0, v0)
+            rows = [(k, v)], [(k[:, :, i:i + 1].contiguous(), v[:, :, i:i + 1].contiguous()) for i in range(n)]
+            for c, parts in zip(caches, rows):
+                for part in parts:
+                    c.update_rope(rope, *part) if rope is not None else c._update(*part)
+            for a, b in zip(caches[0].state, caches[1].state):
+                assert a.shape == b.shape and torch.equal(a, b)
