@@ -13,7 +13,7 @@ namespace {
 template <int DT>
 __global__ void __launch_bounds__(256) rope_rows_kernel(RopeDev r, const char *x, char *out, int H, int L, int D) {
     __shared__ float inv_s[512];
-    const int hg = rope_heads_per_group(gridDim.x * gridDim.y, H, D, DT == 2 ? 4 : 2), h0 = blockIdx.z * hg;
+    const int hg = rope_heads_per_group(gridDim.x * gridDim.y, H, D, DT == 2 ? 4 : 2, 256), h0 = blockIdx.z * hg;
     rope_rows_body<DT>(r, x, out, H, L, D, blockIdx.y, blockIdx.x, h0, min(H, h0 + hg), inv_s);
 }
 
@@ -834,7 +834,7 @@ RopeDev take_rope(RopeDev *rope) {
 hipError_t launch_append_fp_rows(const Store &st, const void *keys, const void *values, int L, int src0,
                                  int slot0, int n, hipStream_t s, const RopeDev &r) {
     if (n <= 0) return hipSuccess;
-    dim3 grid(n, st.BH + rope_ride_rows(r, n, st.es)), block(r.qx ? 256 : 128);
+    const dim3 block(r.qx ? 256 : 128), grid(n, st.BH + rope_ride_rows(r, n, st.es, block.x));
     // (without queries an instance of its own: their LDS table cost the plain append of 512 rows of 64 (batch, head) pairs x 80
     // 25 us instead of 21)
 #define FP_ROWS(ES, RIDE) hipLaunchKernelGGL((append_fp_kernel<ES, RIDE>), grid, block, 0, s, st, (const char *)keys, (const char *)values, L, src0, slot0, r)
@@ -865,7 +865,7 @@ hipError_t launch_append_fp(const Store &st, const void *keys, const void *value
 #define FP_TILE(ES, DK, DV)                                                                                               \
     do {                                                                                                                  \
         const int gx = tiles * FpTile<ES, DK, DV>::PIECES;                                                                \
-        hipLaunchKernelGGL((append_fp_tile_kernel<ES, DK, DV>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es)), dim3(256), 0, s, st, \
+        hipLaunchKernelGGL((append_fp_tile_kernel<ES, DK, DV>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es, 256)), dim3(256), 0, s, st, \
                            (const char *)keys, (const char *)values, L, src0, slot0, n, r);                               \
         return hipGetLastError();                                                                                         \
     } while (0)
@@ -893,7 +893,7 @@ hipError_t launch_rope_apply(const RopeDev &rope, const void *x, void *out, int 
                              int dtype, hipStream_t s) {
     if ((size_t)B * H * L == 0) return hipSuccess;
     if (rope.vec) {
-        const int hg = rope_heads_per_group(L * B, H, D, dtype == KVHIP_F32 ? 4 : 2);
+        const int hg = rope_heads_per_group(L * B, H, D, dtype == KVHIP_F32 ? 4 : 2, 256);
 #define ROPE_ROWS(DT) hipLaunchKernelGGL(rope_rows_kernel<DT>, dim3(L, B, (H + hg - 1) / hg), dim3(256), 0, s, rope, (const char *)x, (char *)out, H, L, D)
         if (dtype == KVHIP_F16) ROPE_ROWS(0);
         else if (dtype == KVHIP_BF16) ROPE_ROWS(1);
@@ -914,7 +914,7 @@ hipError_t launch_append_quant_rows(const Store &st, const void *keys, const voi
     if (n <= 0) return hipSuccess;
     const int ntile = ((slot0 + n - 1) >> 6) - (slot0 >> 6) + 1;
     // (a speculative-verify step appends 4 rows: 8 (row, K or V) items, one per wavefront)
-    dim3 grid(ntile, st.BH + rope_ride_rows(r, ntile, st.es)), block(n >= 3 ? 512 : 256);
+    const dim3 block(n >= 3 ? 512 : 256), grid(ntile, st.BH + rope_ride_rows(r, ntile, st.es, block.x));
     const size_t lds = (size_t)TILE * st.Dv;
 #define CALL(DT, BITS)                                                                                      \
     do {                                                                                                    \

@@ -427,7 +427,7 @@ void launch_quant_tile_instance(const Store &st, const Store &src, const void *k
     } else if (r.dims > 0 && SIDE != 2) {
         using Q = QuantTile<NC, GL, SIDE, true, false>;
         const int gx = tiles * Q::PIECES;
-        hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, true, SIDE>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es)), dim3(Q::NT), 0, s, st,
+        hipLaunchKernelGGL((append_quant_tile_kernel<DT, BITS, NC, GL, true, SIDE>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es, Q::NT)), dim3(Q::NT), 0, s, st,
                            (const char *)keys, (const char *)values, L, a0, b0, n, r);
     } else {
         using Q = QuantTile<NC, GL, SIDE, false, false>;

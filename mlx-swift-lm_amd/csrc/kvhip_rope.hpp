@@ -267,9 +267,12 @@ template <int DT, int D, int THREADS, int RMAX> struct RopeStep {
 };
 
 // ---- the queries of a forward ----------------------------------------------------------------------------------
+// Threads of a workgroup that turn queries.
+__host__ __device__ __forceinline__ int rope_ride_threads(int block) { return block < 256 ? block : 256; }
 // One row position (batch row b, row l of L) of `x` [B, H, L, D] into `out` (which may be x) for heads [h0, h1): a
 // thread owns one chunk pair (chunk, when the pairs are adjacent), works out its sines and cosines once and turns
-// that chunk pair of every head it takes.  `inv_s`: dims / 2 floats of LDS.  blockDim.x >= 256.
+// that chunk pair of every head it takes.  `inv_s`: dims / 2 floats of LDS.  Workgroups of any width that holds a head's
+// items (the appends' are 192, 256 and 512 wide; of 512 threads the first 256 work).
 // Bound by the read and the write of the queries: 512 rows of 32 heads x 128 in bfloat16, 8.4 MB, see
 // rope_rows_kernel.
 template <int DT>
@@ -279,7 +282,7 @@ __device__ __forceinline__ void rope_rows_body(const RopeDev &r, const char *x, 
     const int half = r.dims >> 1;
     const int np = r.traditional ? r.dims / V : half / V;  // rotating items of a head, then the chunks that pass through
     const int items = np + (D - r.dims) / V;
-    const int item = threadIdx.x % items, slot = threadIdx.x / items, ns = 256 / items;  // (wider workgroups: the rest idle)
+    const int item = threadIdx.x % items, slot = threadIdx.x / items, ns = rope_ride_threads((int)blockDim.x) / items;
     const bool live = slot < ns;
     const bool turn = item < np;
     const int d0 = turn ? item * V : r.dims + (item - np) * V;
@@ -330,11 +333,11 @@ __device__ __forceinline__ void rope_rows_body(const RopeDev &r, const char *x, 
 }
 
 // Heads one workgroup of the query pass takes: all of them where the row positions fill the chip, and otherwise as many
-// as its 256 threads turn at once, so that none of them walks heads one after the other behind its exponentials.
+// as its threads turn at once, so that none of them walks heads one after the other behind its exponentials.
 // (64 heads x 128, one token, batch 8, with a workgroup per batch row: 4.75 us, against 4.2 us in workgroups of 32 heads.)
-__host__ __device__ __forceinline__ int rope_heads_per_group(int rows, int H, int D, int es) {
+__host__ __device__ __forceinline__ int rope_heads_per_group(int rows, int H, int D, int es, int block) {
     if (rows >= 256) return H;
-    const int at_once = 256 / max(1, D * es / 32);  // 32 bytes, a chunk pair, per thread
+    const int at_once = rope_ride_threads(block) / max(1, D * es / 32);  // 32 bytes, a chunk pair, per thread
     return min(H, max(1, at_once));
 }
 // The query workgroups behind the `bh` rows of an append's grid (blockIdx.y >= bh): workgroup number i of them takes
@@ -342,15 +345,15 @@ __host__ __device__ __forceinline__ int rope_heads_per_group(int rows, int H, in
 template <int DT>
 __device__ __forceinline__ void rope_queries_ride(const RopeDev &r, int bh, float *inv_s) {
     const int i = (blockIdx.y - bh) * gridDim.x + blockIdx.x, rows = r.qB * r.qL;
-    const int hg = rope_heads_per_group(rows, r.qH, r.qD, DT == 2 ? 4 : 2), groups = (r.qH + hg - 1) / hg;
+    const int hg = rope_heads_per_group(rows, r.qH, r.qD, DT == 2 ? 4 : 2, (int)blockDim.x), groups = (r.qH + hg - 1) / hg;
     const int row = i / groups, h0 = (i - row * groups) * hg;
     if (row >= rows) return;
     rope_rows_body<DT>(r, r.qx, r.qo, r.qH, r.qL, r.qD, row / r.qL, row % r.qL, h0, min(r.qH, h0 + hg), inv_s);
 }
-// Rows those workgroups add to the grid of an append whose rows are `gx` workgroups wide; 0: none ride.
-inline int rope_ride_rows(const RopeDev &r, int gx, int es) {
+// Rows those workgroups add to the grid of an append whose rows are `gx` workgroups of `block` threads wide; 0: none ride.
+inline int rope_ride_rows(const RopeDev &r, int gx, int es, int block) {
     if (r.qx == nullptr) return 0;
-    const int rows = r.qB * r.qL, hg = rope_heads_per_group(rows, r.qH, r.qD, es);
+    const int rows = r.qB * r.qL, hg = rope_heads_per_group(rows, r.qH, r.qD, es, block);
     return (int)(((long)rows * ((r.qH + hg - 1) / hg) + gx - 1) / gx);
 }
 

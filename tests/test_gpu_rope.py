@@ -227,6 +227,26 @@ def test_queries_in_the_appends_launch_equal_separate_calls(kind, dtype, Hq, Hkv
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("bits,gs", [(4, 32), (8, 32), (3, 32)])
+@pytest.mark.parametrize("Hq,Hkv,Dk,Dv,dims,traditional", [
+    (40, 8, 96, 96, 96, False), (32, 32, 96, 96, 64, False), (32, 8, 96, 96, 96, True), (24, 24, 192, 128, 192, False),
+    (128, 16, 192, 128, 192, False), (16, 16, 192, 128, 64, False), (16, 8, 192, 128, 192, True)])
+def test_every_query_head_turns_in_the_quantizers_launch(bits, gs, Hq, Hkv, Dk, Dv, dims, traditional):
+    """Head counts that the query workgroups beside rows of 96 and 192 elements (three quarters of the usual width) pass
+    over more than once, below and above the number of row positions from which one workgroup takes every head.  Each row
+    position has its own values, so that a head left as an earlier call had it shows."""
+    B, dtype = 3, torch.bfloat16
+    rope = kvhip.RoPE(dims, traditional=traditional, base=1e6)
+    one, three = kvhip.QuantizedKVCache(gs, bits), kvhip.QuantizedKVCache(gs, bits)
+    gen = torch.Generator(device="cuda").manual_seed(13)
+    for Lq in (90, 12, 13, 5, 91):
+        q, k, v = (torch.randn(B, h, Lq, d, generator=gen, device="cuda").to(dtype) for h, d in ((Hq, Dk), (Hkv, Dk), (Hkv, Dv)))
+        got = kvhip.attention_with_rope_and_cache_update(rope, q, k, v, one, Dk ** -0.5, kvhip.MaskMode.causal())
+        turned = kvhip.apply_rotary_position(rope, q, three.offset)
+        three.update_rope(rope, k, v)
+        assert torch.equal(got, three.attend(turned, Dk ** -0.5, kvhip.MaskMode.causal())), Lq
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("D,dims", [(64, 64), (40, 32), (128, 72)])
 def test_one_call_in_a_staged_round_counts_the_staged_rows(dtype, D, dims):
