@@ -391,7 +391,8 @@ bool attend_valu_dequant_first(const AttendArgs &a) {
 }
 
 hipError_t launch_merge_valu(const AttendArgs &a, int nparts, hipStream_t s) {
-    if (combine_supported(a.st)) return launch_combine(a, nparts, (a.Hq / a.Hkv) * a.L, s);
+    // (16-bit partials of other sizes: the library's exponential here, the hardware's there)
+    if ((a.st.dtype == KVHIP_F32 && combine_supported(a.st)) || a.st.Dv == 512) return launch_combine(a, nparts, (a.Hq / a.Hkv) * a.L, s);
     const dim3 grid((a.Hq / a.Hkv) * a.L, a.st.BH), block(FT);
     if (a.st.dtype == KVHIP_F16) hipLaunchKernelGGL(merge_valu_kernel<0>, grid, block, 0, s, a, nparts);
     else if (a.st.dtype == KVHIP_BF16) hipLaunchKernelGGL(merge_valu_kernel<1>, grid, block, 0, s, a, nparts);

@@ -7,11 +7,17 @@ namespace kvhip {
 
 namespace {
 
-// the weight of a partial with maximum m beside the row's maximum mx (float32 outputs: the library's exponential, which
-// takes the difference without rounding it to base two first)
-template <int DT> __device__ __forceinline__ float part_weight(float m, float mx) {
+// Partials of the float32 and the head-size-512 kernels: weights by the library's exponential, which takes the difference
+// without rounding it to base two first and has no smallest weight above 2^-149 (an infinite value reaches the output from
+// a span whose weight is denormal, as it does within a span), and sums by fused multiply-adds.
+template <int D, int DT> constexpr bool exact_merge() { return DT == 2 || D == 512; }
+// the weight of a partial with maximum m beside the row's maximum mx
+template <bool EXACT> __device__ __forceinline__ float part_weight(float m, float mx) {
     if (m == -INFINITY) return 0.f;
-    return DT == 2 ? expf(m - mx) : fast_exp2((m - mx) * LOG2E);
+    return EXACT ? expf(m - mx) : fast_exp2((m - mx) * LOG2E);
+}
+template <bool EXACT> __device__ __forceinline__ float add_weighed(float sum, float w, float v) {
+    return EXACT ? __builtin_fmaf(w, v, sum) : sum + w * v;
 }
 template <int DT> __device__ __forceinline__ void store_pair(void *out, size_t i, float o0, float o1) {
     if constexpr (DT == 2) *reinterpret_cast<kv_f2 *>(static_cast<float *>(out) + i) = kv_f2{o0, o1};
@@ -30,6 +36,7 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
     constexpr int CP = CB / 2;    // column pairs
     constexpr int NG = 256 / CP;  // span groups: 8 (64 columns), 6, 5, 4 (128)
     constexpr int UN = 8;         // loads in flight per thread and round
+    constexpr bool EXACT = exact_merge<D, DT>();
     __shared__ float w_s[512];    // weight of each span for this row (nsplit <= 512)
     __shared__ float red_s[2][4];
     __shared__ kv_f2 acc_s[NG][CP];
@@ -66,7 +73,7 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
     float dloc = 0.f;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        const float w = part_weight<DT>(ml[u].x, mx);
+        const float w = part_weight<EXACT>(ml[u].x, mx);
         if (t + 256 * u < nsplit) w_s[t + 256 * u] = w;
         dloc += w * ml[u].y;
     }
@@ -78,7 +85,7 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
         const int s = g + NG * u;
-        if (col && s < nsplit) num += w_s[s] * v[u];
+        if (col && s < nsplit) num = kv_f2{add_weighed<EXACT>(num.x, w_s[s], v[u].x), add_weighed<EXACT>(num.y, w_s[s], v[u].y)};
     }
     for (int s0 = g + NG * UN; col && s0 < nsplit; s0 += NG * UN) {  // more than 8 NG spans: further rounds
 #pragma unroll
@@ -89,7 +96,7 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const int s = s0 + NG * u;
-            if (s < nsplit) num += w_s[s] * v[u];
+            if (s < nsplit) num = kv_f2{add_weighed<EXACT>(num.x, w_s[s], v[u].x), add_weighed<EXACT>(num.y, w_s[s], v[u].y)};
         }
     }
     if (col) acc_s[g][cp] = num;
@@ -114,6 +121,7 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
 template <int D, int DT, int MAXP>
 __global__ void __launch_bounds__(256) combine_rows_kernel(AttendArgs a, int nsplit, int rr) {
     constexpr int LPR = D / 4, RPW = 256 / LPR;
+    constexpr bool EXACT = exact_merge<D, DT>();
     const int in_wg = threadIdx.x / LPR, c = 4 * (threadIdx.x % LPR);
     const int i = blockIdx.x * RPW + in_wg, bh = blockIdx.y;
     const int r = a.Hq / a.Hkv;
@@ -136,13 +144,13 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(AttendArgs a, int nsp
     float den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < MAXP; ++s) {
-        const float w = part_weight<DT>(ml[s].x, mx);
+        const float w = part_weight<EXACT>(ml[s].x, mx);
         const bool own = s < nsplit;
-        den = own ? den + w * ml[s].y : den;
-        num[0] = own ? num[0] + w * p[s][0].x : num[0];
-        num[1] = own ? num[1] + w * p[s][0].y : num[1];
-        num[2] = own ? num[2] + w * p[s][1].x : num[2];
-        num[3] = own ? num[3] + w * p[s][1].y : num[3];
+        den = own ? add_weighed<EXACT>(den, w, ml[s].y) : den;
+        num[0] = own ? add_weighed<EXACT>(num[0], w, p[s][0].x) : num[0];
+        num[1] = own ? add_weighed<EXACT>(num[1], w, p[s][0].y) : num[1];
+        num[2] = own ? add_weighed<EXACT>(num[2], w, p[s][1].x) : num[2];
+        num[3] = own ? add_weighed<EXACT>(num[3], w, p[s][1].y) : num[3];
     }
     const size_t ooff = ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D + c;
 #pragma unroll

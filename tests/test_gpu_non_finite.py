@@ -80,3 +80,24 @@ def test_tiles_nobody_sees_are_not_read(dtype, D, T, n, seen, ring):
     v[:, :, :hidden] = NAN
     out = attend(q, k, v, kvhip.MaskMode.from_array(keep), ring)
     assert (out - exact(q, k, v, keep)).abs().max() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Dk,Dv", [(512, 512), (576, 512), (320, 64), (320, 96), (1024, 128), (320, 256)])
+@pytest.mark.parametrize("n", [1, 5, 40])
+def test_infinite_values_of_a_range_with_a_denormal_weight_reach_the_output(dtype, Dk, Dv, n):
+    """The merge of key ranges: one range's maximum lies 90 above another's, which leaves that a weight of 2^-130 -- not
+    zero in float32, so its infinite value stays infinite."""
+    T = 2048
+    q, k, v = torch.zeros(1, 2, n, Dk), torch.zeros(1, 1, T, Dk), torch.ones(1, 1, T, Dv)
+    q[..., 0] = 1.
+    k[0, 0, :, 0] = -90.
+    k[0, 0, 5, 0] = 0.
+    v[0, 0, 1500, 3], v[0, 0, 1500, Dv - 1] = INF, -INF
+    c = kvhip.KVCacheSimple()
+    c.update(k.to(dtype).cuda(), v.to(dtype).cuda(), fetch=False)
+    out = c.attend(q.to(dtype).cuda(), 1.0, kvhip.MaskMode.none())
+    assert kvhip.load().kvhip_last_attend_kernel() == 5
+    assert (out[..., 3] == INF).all() and (out[..., Dv - 1] == -INF).all()
+    out[..., 3] = out[..., Dv - 1] = 1.
+    assert (out.double() - 1.).abs().max() <= TOL[dtype]
