@@ -232,10 +232,10 @@ kvhip_status kvhip_cache_update_rope(kvhip_cache *cache, const kvhip_rope *rope,
 
 /* An attention layer's call sequence (Llama.swift:58-70) in one: kvhip_rope_apply on the queries and
  * kvhip_cache_update_rope at the cache's `ropeOffset` (or at batch_offsets), then kvhip_cache_attend.  The queries
- * turn in the append's launch where their rows are whole 16-byte chunks; a single token's may turn inside the decode
- * kernel.  `q_rotated`: device scratch of the queries' size that may hold them in between (it may be `queries`), of no
- * defined content afterwards; NULL: a buffer the cache keeps for it, which grows with hipMalloc (on a stream that is
- * being captured the call then returns KVHIP_ERR_UNSUPPORTED and has done nothing). */
+ * turn in the append's launch where their rows are whole 16-byte chunks; a single token's turn inside the attention
+ * kernel where that writes the row too (kvhip_cache_update_attend).  `q_rotated`: device scratch of the queries' size that may hold them in between (it may be `queries`), of no
+ * defined content afterwards; NULL: a buffer the cache keeps for it where there is need of one, which grows with
+ * hipMalloc (on a stream that is being captured the call then returns KVHIP_ERR_UNSUPPORTED and has done nothing). */
 kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *cache, const kvhip_rope *rope, const int32_t *batch_offsets,
                                             const void *queries, const void *keys, const void *values, int32_t B,
                                             int32_t Hq, int32_t Hkv, int32_t L, int32_t Dk, int32_t Dv, int32_t dtype,

@@ -1177,23 +1177,36 @@ void queries_ride(RopeDev &r, const void *q, void *q_rotated, int B, int Hq, int
     r.qD = D;
 }
 
-// whether a decode kernel takes a single-token step without a mask of this cache, its rows still to be written and rotated
-bool decode_takes_step(const kvhip_cache *c, int Hq) {
+// Whether the kernel that attends writes (and rotates) the rows of a step itself.
+bool attention_writes_step(const AttendArgs &a) {
+    return g_policy != 1 && (attend_decode_fuses_append(a) ||
+                             (!attend_decode_supported(a) && !attend_prefill_supported(a) && attend_valu_fuses_append(a)));
+}
+
+// The same for a single-token step without a mask that has yet to be entered into this cache's bookkeeping.
+bool attention_will_write_step(const kvhip_cache *c, int Hq) {
     AttendArgs a;
     a.st = c->st;
     a.B = c->B;
     a.Hq = Hq;
     a.Hkv = c->Hkv;
     a.L = 1;
-    a.runs.n = 1;  // (quantized caches are never in pieces, the full-precision kernel takes them)
+    int64_t rows = c->offset + 1;
+    if (c->kind == KVHIP_KIND_ROTATING && rows >= c->max_size) {  // (what update_rotating presents)
+        rows = (int64_t)c->rows.size();
+        if (c->offset >= c->ref_len && c->ref_len < c->max_size) rows += std::max<int64_t>(0, std::min<int64_t>(c->step, c->max_size - c->offset));
+        rows = std::min<int64_t>(rows, c->max_size);
+    }
+    a.T = a.slots = (int)rows;
+    a.runs.n = 1;  // (quantized caches are never in pieces, the full-precision kernels take them)
     a.runs.row0[0] = a.runs.phys0[0] = 0;
-    return g_policy != 1 && attend_decode_fuses_append(a);
+    return attention_writes_step(a);
 }
 
 // new_k / new_v: the rows of a single-token step whose bookkeeping is done but whose write into physical
-// slot `new_slot` is still owed; the decode kernel takes them along when it can, else they are
+// slot `new_slot` is still owed; the attention kernel takes them along when it can, else they are
 // appended by a launch of their own first.  `rope`: the queries and the new key row are still to be rotated (its H:
-// kv heads), by whichever of the two launches takes the row; `q_rotated` takes the queries if it is not the decode kernel.
+// kv heads), by whichever of the two launches takes the row; `q_rotated` takes the queries if it is the append.
 kvhip_status attend_impl(kvhip_cache *c, const void *q, int32_t B, int32_t Hq, int32_t L, int32_t D, float scale,
                          const kvhip_mask *mask, void *out, void *stream, float *fixed, size_t fixed_bytes,
                          const void *new_k = nullptr, const void *new_v = nullptr, int32_t new_slot = -1, RopeDev *rope = nullptr,
@@ -1266,9 +1279,7 @@ kvhip_status attend_impl(kvhip_cache *c, const void *q, int32_t B, int32_t Hq, i
     hipStream_t s = S(c, stream);
     a.workspace_cap = fixed ? fixed_bytes : 0;
     if (new_k) {
-        const bool fuses = attend_decode_fuses_append(a) ||
-                           (!attend_decode_supported(a) && !attend_prefill_supported(a) && attend_valu_fuses_append(a));
-        if (g_policy != 1 && fuses) {
+        if (attention_writes_step(a)) {
             a.new_k = new_k;
             a.new_v = new_v;
             a.new_slot = new_slot;
@@ -1390,7 +1401,7 @@ kvhip_status kvhip_cache_update_attend_rope(kvhip_cache *c, const kvhip_rope *ro
     const bool token = L == 1 && !c->staging && (dtype != KVHIP_F32 || c->kind != KVHIP_KIND_QUANTIZED) && (!mask || mask->mode == KVHIP_MASK_NONE) &&
                        c->has_geom && c->has_buffers && !c->padded() && c->B == B && c->Hkv == Hkv && c->st.Dk == Dk && c->st.Dv == Dv &&
                        c->st.dtype == dtype && (size_t)B * Hkv + (size_t)B * Hq <= 65535;
-    if (!q_rotated && !(token && decode_takes_step(c, Hq))) {
+    if (!q_rotated && !(token && attention_will_write_step(c, Hq))) {
         // (before anything is written: a stream that is being captured cannot have the memory, and its caller asks again)
         const size_t need = (size_t)B * Hq * L * Dk * elem_size(dtype);
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;

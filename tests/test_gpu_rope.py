@@ -6,11 +6,14 @@ float32 products, the restatement works in float64: which intermediate roundings
 CPU path makes is parity unpinned).  The fused rotate-and-append must equal rotate-then-append
 on the device bit for bit, for every cache kind, since both run the same element function.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 import kvhip
+from kvhip.cache import _DT as DT
 from oracle import kv_oracle as O
 from oracle import rope as OR
 from tests.util import NAME, dev, err_stats, np32, randn
@@ -329,6 +332,73 @@ def test_one_call_is_captured_where_the_separate_calls_are(kind, dtype, D, Lq):
         torch.cuda.synchronize()
         assert torch.equal(got, separate())
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 512), (torch.float16, 512), (torch.float32, 64), (torch.float32, 128), (torch.float16, 128)])
+@pytest.mark.parametrize("ring", [False, True])
+def test_a_captured_token_that_turns_in_the_attention_kernel_needs_no_scratch(dtype, D, ring):
+    """The first rotary call of a cache, captured, through the C entry without `q_rotated`: the kernel that attends turns
+    the queries itself, so there is nothing to refuse."""
+    B, Hq, Hkv = 2, 8, 2
+    rope = kvhip.RoPE(D, base=1e4)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+
+    def rows(n):
+        return [torch.randn(B, h, n, D, generator=gen, device="cuda").to(dtype) for h in (Hq, Hkv, Hkv)]
+
+    _, k, v = rows(300)
+    warm = [rows(1) for _ in range(2)]  # (the ring at its size, the attention scratch there)
+    caches = [kvhip.RotatingKVCache(256, keep=4) if ring else kvhip.KVCacheSimple() for _ in range(4)]
+    for c in caches:
+        c.update(k, v, fetch=False)
+        for row in warm:
+            c.update_attend(*row, D ** -0.5)
+        if not ring:
+            c.trim(2)
+    one, others = caches[0], caches[1:]
+    q, k, v = rows(1)
+    out = torch.empty_like(q)
+    r, keep = rope.to_c()
+    lib, mask = kvhip.load(), kvhip.MaskMode.none().to_c(B, Hq, 1)[0]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        status = lib.kvhip_cache_update_attend_rope(one._h, C.byref(r), None, q.data_ptr(), k.data_ptr(), v.data_ptr(), B, Hq, Hkv, 1, D, D, DT[dtype],
+                                                    D ** -0.5, C.byref(mask), None, out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert status == 0, lib.kvhip_last_error_message()
+    for other in others:
+        for t, new in zip((q, k, v), rows(1)):
+            t.copy_(new)
+        graph.replay()
+        got = out.clone()
+        torch.cuda.synchronize()
+        turned = kvhip.apply_rotary_position(rope, q, other.rope_offset)
+        other.update_rope(rope, k, v)
+        assert torch.equal(got, other.attend(turned, D ** -0.5))
+        torch.cuda.synchronize()
+
+
+def test_one_call_across_the_lengths_at_which_the_float32_kernel_changes():
+    """One token of 128 pairs of 128 columns in float32: from 512 rows on the vector-ALU kernel, which neither writes nor
+    turns rows, takes the step, and the call sees that before it decides whether the queries need room."""
+    B, Hq, Hkv, D = 16, 8, 8, 128
+    rope = kvhip.RoPE(D, base=1e4)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+
+    def rows(n):
+        return [torch.randn(B, h, n, D, generator=gen, device="cuda") for h in (Hq, Hkv, Hkv)]
+
+    for ring in (False, True):
+        one, three = (kvhip.RotatingKVCache(514, keep=4) if ring else kvhip.KVCacheSimple() for _ in range(2))
+        _, k, v = rows(507)
+        for c in (one, three):
+            c.update(k, v, fetch=False)
+        for _ in range(10):
+            q, k, v = rows(1)
+            got = one.update_attend_rope(rope, q, k, v, D ** -0.5)
+            turned = kvhip.apply_rotary_position(rope, q, three.rope_offset)
+            three.update_rope(rope, k, v)
+            assert torch.equal(got, three.attend(turned, D ** -0.5)), one.offset
 
 
 def test_one_call_refuses_queries_that_do_not_go_with_the_keys():
