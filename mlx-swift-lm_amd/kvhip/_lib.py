@@ -131,12 +131,19 @@ _step = None
 
 def step():
     """The extension that carries a layer's attention call from its tensors to the library (csrc/py/kvhip_step.cpp), and the
-    addresses of its two entry points: (module, update_attend, update_attend_rope).  Raises if it is not built."""
+    addresses of its two entry points: (module, update_attend, update_attend_rope).  (None, None, None) where it is not built
+    (a library made without this interpreter's headers): the Python methods take every call."""
     global _step
     if _step is None:
+        import importlib
+
         import torch
 
-        from . import _step as module
+        try:
+            module = importlib.import_module("._step", __package__)
+        except ModuleNotFoundError:
+            _step = (None, None, None)
+            return _step
         from .rope import RoPE
 
         module.bind(torch.Tensor, RoPE, (torch.float16, torch.bfloat16, torch.float32), torch._C._cuda_getDevice,

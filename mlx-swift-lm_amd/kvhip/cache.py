@@ -249,7 +249,7 @@ class _Cache:
         """The call as one native step, if it is of the ordinary form (contiguous arrays that go together and with what the
         cache holds, no mask or the causal one): the output, or None with nothing done."""
         at = _PLAIN_AT.get(mask.mode if type(mask) is MaskMode else None if mask else L.MASK_NONE)
-        if at is None:
+        if at is None or self._step is None:
             return None
         out = self._step.attend(self._step_at if rope is None else self._step_rope_at, self._h.value, self._shape, queries, keys, values,
                                 scale, at, rope, _Q_ROTATED_KEPT)

@@ -1,5 +1,7 @@
 """The attention call carried from its tensors to the library in one native step: the same bits as the Python methods give
 on a second cache, and the same errors; what is not of the ordinary form is left to those methods with nothing done."""
+import sys
+
 import pytest
 import torch
 
@@ -120,3 +122,26 @@ def test_host_tensors_and_wrong_arguments_are_not_taken():
     assert step.attend(1, 1, None, None, x, x, 1.0, 1, None, 0) is None
     with pytest.raises(TypeError):
         step.attend(1, 1)
+
+
+def test_the_package_does_without_the_extension(monkeypatch):
+    monkeypatch.setitem(sys.modules, "kvhip._step", None)
+    monkeypatch.setattr(L, "_step", None)
+    assert L.step() == (None, None, None)
+
+
+@pytest.mark.gpu
+def test_caches_without_the_extension_give_the_same(monkeypatch):
+    caches, outcomes, gen = _pair("q4", torch.float16)
+    with monkeypatch.context() as m:
+        m.setitem(sys.modules, "kvhip._step", None)
+        m.setattr(L, "_step", None)
+        other = kvhip.QuantizedKVCache(64, 4)
+    other.state = caches[0].state
+    other.offset = caches[0].offset
+    rope = kvhip.RoPE(D)
+    for n in (1, 3):
+        q, k, v = (_rand(gen, B, h, n, D, dtype=torch.float16) for h in (HQ, HKV, HKV))
+        _same([caches[0], other], lambda c: kvhip.attention_with_rope_and_cache_update(rope, q, k, v, c, 0.125))
+        _same([caches[0], other], lambda c: kvhip.attention_with_cache_update(q, k, v, c, 0.125))
+    assert outcomes and all(o is not None for o in outcomes)
