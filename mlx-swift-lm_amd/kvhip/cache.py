@@ -283,8 +283,10 @@ class _Cache:
     def update_attend_rope(self, rope, queries, keys, values, scale, mask=None, batch_offsets=None):
         """Queries and keys rotated at this cache's `ropeOffset` (or at `batch_offsets`), update, attention."""
         out = self._attend_natively(rope, queries, keys, values, scale, mask) if batch_offsets is None else None
-        if out is not None:
-            return out
+        return out if out is not None else self._update_attend_rope(rope, queries, keys, values, scale, mask, batch_offsets)
+
+    def _update_attend_rope(self, rope, queries, keys, values, scale, mask, batch_offsets):
+        """`update_attend_rope` of any form."""
         q, k, v = queries.contiguous(), keys.contiguous(), values.contiguous()
         assert k.is_cuda and v.is_cuda and k.dtype == v.dtype
         if q.dtype != k.dtype:

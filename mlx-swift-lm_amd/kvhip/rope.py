@@ -61,14 +61,16 @@ def attention_with_rope_and_cache_update(rope, queries, keys, values, cache, sca
     (Llama.swift:58-70 + AttentionUtils.swift:37-95): one launch rotates the queries and rotates and appends
     (or rotates, quantizes and appends) the keys and values, then attention.  Queries that do not go with the
     keys row by row are taken in separate calls."""
-    if batch_offsets is None and getattr(type(cache), "update_attend_rope", None) is _Cache.update_attend_rope:
+    own = getattr(type(cache), "update_attend_rope", None) is _Cache.update_attend_rope
+    if own and batch_offsets is None:
         out = cache._attend_natively(rope, queries, keys, values, scale, mask)
         if out is not None:
             return out
     if (isinstance(cache, _Cache) and queries.dtype == keys.dtype and queries.dim() == 4 and keys.dim() == 4
             and (cache._shape is None or cache._shape[4] == keys.dtype)
             and queries.shape[0] == keys.shape[0] and queries.shape[2:] == keys.shape[2:]):
-        return cache.update_attend_rope(rope, queries, keys, values, scale, mask, batch_offsets)
+        general = cache._update_attend_rope if own else cache.update_attend_rope
+        return general(rope, queries, keys, values, scale, mask, batch_offsets)
     offset = batch_offsets if batch_offsets is not None else cache.rope_offset
     q = apply_rotary_position(rope, queries, offset)
     cache.update_rope(rope, keys, values, batch_offsets)

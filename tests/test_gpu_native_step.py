@@ -145,3 +145,17 @@ def test_caches_without_the_extension_give_the_same(monkeypatch):
         _same([caches[0], other], lambda c: kvhip.attention_with_rope_and_cache_update(rope, q, k, v, c, 0.125))
         _same([caches[0], other], lambda c: kvhip.attention_with_cache_update(q, k, v, c, 0.125))
     assert outcomes and all(o is not None for o in outcomes)
+
+
+@pytest.mark.gpu
+def test_a_call_that_is_not_taken_is_tried_once():
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    cache, tried = kvhip.KVCacheSimple(), []
+    native = cache._attend_natively
+    cache._attend_natively = lambda *a: tried.append(a) or native(*a)
+    rope = kvhip.RoPE(D)
+    for n, mask in ((CTX, None), (700, kvhip.MaskMode.causal()), (2, kvhip.MaskMode.window_mask(CTX + 700, 16))):
+        q, k, v = (_rand(gen, B, h, n, D, dtype=torch.float16) for h in (HQ, HKV, HKV))
+        kvhip.attention_with_rope_and_cache_update(rope, q, k, v, cache, 0.125, mask)
+        assert len(tried) == 1, n
+        tried.clear()
