@@ -50,8 +50,11 @@ bool take(PyObject *t, Array &a) {
     Py_XDECREF(ptr);
     return a.p != nullptr;
 }
-PyObject *none() {
-    PyErr_Clear();
+PyObject *none() {  // (an interrupt or an exit is not a form of the call)
+    if (PyErr_Occurred()) {
+        if (!PyErr_ExceptionMatches(PyExc_Exception)) return nullptr;
+        PyErr_Clear();
+    }
     Py_RETURN_NONE;
 }
 

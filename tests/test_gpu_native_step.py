@@ -159,3 +159,23 @@ def test_a_call_that_is_not_taken_is_tried_once():
         kvhip.attention_with_rope_and_cache_update(rope, q, k, v, cache, 0.125, mask)
         assert len(tried) == 1, n
         tried.clear()
+
+
+@pytest.mark.gpu
+def test_an_interrupt_is_not_swallowed():
+    class Scale:
+        interrupted = False
+
+        def __float__(self):
+            if not self.interrupted:
+                self.interrupted = True
+                raise KeyboardInterrupt
+            return 0.125
+
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    cache = kvhip.KVCacheSimple()
+    q, k, v = (_rand(gen, B, h, 4, D, dtype=torch.float16) for h in (HQ, HKV, HKV))
+    kvhip.attention_with_cache_update(q, k, v, cache, 0.125)
+    with pytest.raises(KeyboardInterrupt):
+        kvhip.attention_with_cache_update(q, k, v, cache, Scale())
+    assert cache.offset == 4
