@@ -30,7 +30,7 @@ template <int DT> __device__ __forceinline__ void store_pair(void *out, size_t i
 // requests its first eight partial pairs before anything else, then the (max, sum) of up to two spans; the weights
 // are formed while the columns are in flight, go through LDS, and the span groups' sums meet there at the end.  Wide rows
 // are cut into blocks of columns so that one round of requests holds every span of the usual plans.
-template <int D, int DT, int CB>
+template <int D, int DT, int CB, bool SPANS>
 __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, int rr, const int2 *spans) {
     static_assert(D % CB == 0, "whole blocks of columns");
     constexpr int CP = CB / 2;    // column pairs
@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
     const int rep = i / a.L, l = i - rep * a.L;
     const size_t sstride = (size_t)rr * (D + 2);
     size_t first_slot = (size_t)bh * nsplit;
-    if (spans != nullptr) {  // (a ragged batch's rows have spans in proportion to their keys: kvhip_mask.hpp)
+    if constexpr (SPANS) {  // (a ragged batch's rows have spans in proportion to their keys: kvhip_mask.hpp)
         const int2 own = spans[bh];
         first_slot = own.x;
         nsplit = own.y;
@@ -166,7 +166,14 @@ template <int D, int DT, int CB> hipError_t merge(const AttendArgs &a, int nspli
         else if (nsplit <= 4) hipLaunchKernelGGL((combine_rows_kernel<D, DT, 4>), grid, block, 0, s, a, nsplit, rows);
         else hipLaunchKernelGGL((combine_rows_kernel<D, DT, 8>), grid, block, 0, s, a, nsplit, rows);
     } else {
-        hipLaunchKernelGGL((combine_kernel<D, DT, CB>), dim3(R, a.st.BH, D / CB), dim3(256), 0, s, a, nsplit, rows, spans);
+        const dim3 grid(R, a.st.BH, D / CB), block(256);
+        if constexpr (DT != 2 && D <= 256) {
+            if (spans != nullptr) {
+                hipLaunchKernelGGL((combine_kernel<D, DT, CB, true>), grid, block, 0, s, a, nsplit, rows, spans);
+                return hipGetLastError();
+            }
+        }
+        hipLaunchKernelGGL((combine_kernel<D, DT, CB, false>), grid, block, 0, s, a, nsplit, rows, spans);
     }
     return hipGetLastError();
 }
