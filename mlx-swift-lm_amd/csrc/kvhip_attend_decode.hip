@@ -376,9 +376,11 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     // Slot T - 1 lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one (spans
     // are equal and cover every tile): that wavefront quantizes the row into the cache, with the arithmetic of the append
     // kernel, after it has requested its first tile and before it requests another, so its own later loads of the
-    // row's tile see it; if its first tile is that tile, it requests it again.  The V code goes into its column's packed
+    // row's tile see it; if its first tile is that tile, it requests it only then.  The V code goes into its column's packed
     // word read-modify-write; the row and the old words are requested in front of the tile.  (The row written first and
-    // the tiles requested behind it: the last wavefront of the launch to finish, by four round trips to memory.)
+    // the tiles requested behind it: the last wavefront of the launch to finish, by four round trips to memory.  The row's
+    // own tile requested in front as well and once more behind the row: 8 bits, one sequence of 2000 keys x 64, the step
+    // 10.6 us for 10.2; 60 keys x 128 9.5 for 9.2.)
     bool own = false;
     uint16_t own_k[NH], own_v[NH];
     uint32_t own_w[NH];
@@ -632,19 +634,15 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
         if constexpr (PREFETCH) load_tile(first);
         else load_k(first);
     };
-    if (my_tiles > 0) request_first();
+    const bool row_first = own && my_tiles == 1;  // wave-uniform: the first tile is the new row's
+    if (my_tiles > 0 && !row_first) request_first();
     if constexpr (rot) {
         step.turn(a.turn, bh, R, rot_s);
         __syncthreads();
     }
     if constexpr (MM == 0 && RG == 1) {
-        if (own) {  // wave-uniform
-            write_row();
-            if (my_tiles == 1) {  // (then no pointer has moved on)
-                k_loaded = v_loaded = 0;
-                request_first();
-            }
-        }
+        if (own) write_row();
+        if (row_first) request_first();
     }
     if (my_tiles > 0) {
         load_queries();
@@ -904,8 +902,8 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     // ---- the step's new row, when it is still to be written (unmasked single-token decode) -----
     // Exactly one wavefront of one workgroup reads the tile of physical slot `new_slot` (spans are equal and
     // cover every tile): it copies the row into the page after it has requested its first pieces and before it requests
-    // others, so its own later loads of the tile see it; if its first tile is that tile, it requests them again.  The row
-    // is requested in front of the pieces.
+    // others, so its own later loads of the tile see it; if its first tile is that tile, it requests them only then.  The
+    // row is requested in front of the pieces.
     bool own = false;
     kv_u4 own_k;
     uint16_t own_v[NP];
@@ -928,9 +926,10 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     auto request_first = [&]() __attribute__((always_inline)) {
         static_for<NBUF>([&](auto N) { request(buf_of(decltype(N)::value), decltype(N)::value); });
     };
+    const bool row_first = own && tile0 == a.new_slot >> 6;  // wave-uniform
     if (my_tiles > 0) {
         if constexpr (!rot) load_queries();
-        request_first();
+        if (!row_first) request_first();
     }
     if constexpr (rot) {
         step.turn(a.turn, bh, R, rot_s);
@@ -948,13 +947,7 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
             for (int h = 0; h < NP; ++h) *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, 64 * h + lane)) = own_v[h];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            if (tile0 == slot >> 6) {
-                k_loaded = v_loaded = 0;
-                page_k = page_v = tile0 >> 2;
-                kp = as_global(pt[page_k].k);
-                vp = as_global(pt[page_v].v);
-                request_first();
-            }
+            if (row_first) request_first();
         }
     }
     if (my_tiles > 0) {

@@ -234,7 +234,7 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     // Its slot lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one: that wavefront
     // quantizes the row into the cache, with the arithmetic of the append kernel, after it has requested its first tile and
     // before it requests another, so its own later loads of the row's tile (and of the tile's scale / bias pairs) see it; if
-    // its first tile is that tile, it requests it again.  A lane owns the V columns it quantizes; their codes go into the
+    // its first tile is that tile, it requests it only then.  A lane owns the V columns it quantizes; their codes go into the
     // columns' tile rows read-modify-write (a code of a bit stream may lie across two dwords).  The row and the old words
     // are requested in front of the tile.
     constexpr int NHK = (DK + 63) / 64, NHV = (DV + 63) / 64;
@@ -663,19 +663,15 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         if constexpr (SB_LDS) dma_sb();
         load_k(buf);
     };
-    if (my_tiles > 0) request_first();
+    const bool row_first = own && my_tiles == 1;  // wave-uniform: the first tile is the new row's
+    if (my_tiles > 0 && !row_first) request_first();
     if constexpr (rot) {
         step.turn(a.turn, bh, R, rot_s);
         __syncthreads();
     }
     if constexpr (MM == 0) {
-        if (own) {  // wave-uniform
-            write_row();
-            if (my_tiles == 1) {  // (then no pointer has moved on)
-                k_loaded = v_loaded = sb_issued = 0;
-                request_first();
-            }
-        }
+        if (own) write_row();
+        if (row_first) request_first();
     }
     if (my_tiles > 0) {
         load_queries();
