@@ -205,12 +205,11 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     [[maybe_unused]] RaggedSpan span;
     [[maybe_unused]] int wid = 0;
     if constexpr (MM == 1) {
-        if (tiles_per_wg < 0) {  // a ragged batch that shares its spans out
-            const int wgs = nsplit * a.B;
+        if (__builtin_expect(tiles_per_wg < 0, 0)) {  // a ragged batch that shares its spans out (behind the rest of the kernel)
             wid = b * nsplit + split;
-            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, wgs, NW, wid, true);
+            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, nsplit, NW, wid, true);
             if (span.count == 0) return;  // (workgroup-uniform)
-            part_slot = (size_t)hk * wgs + wid;
+            part_slot = (size_t)hk * nsplit * a.B + wid;
             b = span.b;
             bh = b * a.Hkv + hk;
         } else if (tiles_per_wg == 0 && a.B <= 64 && a.B > 2) {
@@ -312,19 +311,26 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     }
 
     const float fill = finfo_min_dt(DT);
-    const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
+    [[maybe_unused]] SymMask sym{};
     int tile_begin = split * tiles_per_wg;
     int tile_end = min(tiles_total, tile_begin + tiles_per_wg);
     if constexpr (MM == 1) {
         // length-aware partition: an index-only mask bounds the rows this (batch) can see
         // (left padding, lengths, causal/window reach); spans of equal size start at the first
         // visible tile
-        const TileRange vis = visible_tiles(sym, tiles_total, true);
-        // tiles_per_wg == 0: divide this batch row's own visible range over the spans
-        const int per = tiles_per_wg > 0 ? tiles_per_wg
-                                         : (max(vis.hi - vis.lo, 1) + nsplit * NW - 1) / (nsplit * NW) * NW;
-        tile_begin = tiles_per_wg < 0 ? span.t.lo : vis.lo + split * per;  // spans past the last tile are empty
-        tile_end = tiles_per_wg < 0 ? span.t.hi : min(vis.hi, tile_begin + per);
+        if (__builtin_expect(tiles_per_wg < 0, 0)) {
+            sym = span.sym;
+            tile_begin = span.t.lo;
+            tile_end = span.t.hi;
+        } else {
+            sym = sym_mask_init(a.mask, b, a.L, a.T);
+            const TileRange vis = visible_tiles(sym, tiles_total, true);
+            // tiles_per_wg == 0: divide this batch row's own visible range over the spans
+            const int per = tiles_per_wg > 0 ? tiles_per_wg
+                                             : (max(vis.hi - vis.lo, 1) + nsplit * NW - 1) / (nsplit * NW) * NW;
+            tile_begin = vis.lo + split * per;  // spans past the last tile are empty
+            tile_end = min(vis.hi, tile_begin + per);
+        }
     }
     [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees
     if constexpr (MM == 1) {
@@ -775,12 +781,11 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     [[maybe_unused]] RaggedSpan span;
     [[maybe_unused]] int wid = 0;
     if constexpr (MM == 1 && IDENT) {
-        if (tiles_per_wg < 0) {  // a ragged batch that shares its spans out
-            const int wgs = nsplit * a.B;
+        if (__builtin_expect(tiles_per_wg < 0, 0)) {  // a ragged batch that shares its spans out (behind the rest of the kernel)
             wid = b * nsplit + split;
-            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, wgs, WAVES, wid, false);
+            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, nsplit, WAVES, wid, false);
             if (span.count == 0) return;  // (workgroup-uniform)
-            part_slot = (size_t)hk * wgs + wid;
+            part_slot = (size_t)hk * nsplit * a.B + wid;
             b = span.b;
             bh = b * a.Hkv + hk;
         }
@@ -826,23 +831,32 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
         for (int h = 0; h < NP; ++h) oacc[rg][h] = f4{0.f, 0.f, 0.f, 0.f};
     }
 
-    const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
+    [[maybe_unused]] SymMask sym{};
+    int tile_begin = split * tiles_per_wg;
+    int tile_end = min(tiles_total, tile_begin + tiles_per_wg);
+    if constexpr (MM == 1 && IDENT) {
+        if (__builtin_expect(tiles_per_wg < 0, 0)) {
+            sym = span.sym;
+            tile_begin = span.t.lo;
+            tile_end = span.t.hi;
+        } else {
+            sym = sym_mask_init(a.mask, b, a.L, a.T);
+            const TileRange vis = visible_tiles(sym, tiles_total, false);
+            // tiles_per_wg == 0: divide this batch row's own visible range over the spans
+            const int per = tiles_per_wg > 0 ? tiles_per_wg
+                                             : (max(vis.hi - vis.lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
+            tile_begin = vis.lo + split * per;  // spans past the last tile are empty
+            tile_end = min(vis.hi, tile_begin + per);
+        }
+    } else if constexpr (MM == 1) {
+        sym = sym_mask_init(a.mask, b, a.L, a.T);
+    }
     [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees
     if constexpr (MM == 1) {
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
             for (int i = 0; i < 4; ++i) seen[rg][i] = sym_mask_bounds(sym, (4 * rg + i) % a.L);
-    }
-    int tile_begin = split * tiles_per_wg;
-    int tile_end = min(tiles_total, tile_begin + tiles_per_wg);
-    if constexpr (MM == 1 && IDENT) {
-        const TileRange vis = visible_tiles(sym, tiles_total, false);
-        // tiles_per_wg == 0: divide this batch row's own visible range over the spans
-        const int per = tiles_per_wg > 0 ? tiles_per_wg
-                                         : (max(vis.hi - vis.lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
-        tile_begin = tiles_per_wg < 0 ? span.t.lo : vis.lo + split * per;  // spans past the last tile are empty
-        tile_end = tiles_per_wg < 0 ? span.t.hi : min(vis.hi, tile_begin + per);
     }
     const int tile0 = tile_begin + wave;
     const int my_tiles = tile0 < tile_end ? (tile_end - tile0 + WAVES - 1) / WAVES : 0;
@@ -1164,7 +1178,8 @@ Plan plan_for(const AttendArgs &a) {
     p.nw = WAVES;
     const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
     if (a.mask.mode == KVHIP_MASK_WINDOW && (a.mask.left_pad || a.mask.lengths) && forced_tiles <= 0 && ident) {
-        p.tiles_per_wg = a.B >= 2 && a.B <= 64 && p.nsplit >= 2 ? -1 : 0;
+        const bool paired = a.st.bits != 0 && a.B > 2;  // (balanced_row, in the quantized kernels)
+        p.tiles_per_wg = a.B >= 2 && a.B <= 64 && p.nsplit >= (paired ? 3 : 2) && p.tiles_total > p.nsplit * WAVES ? -1 : 0;
         // KVHIP_RAGGED_SPANS forces the number of spans per batch row (timing builds only: measure_knob)
         static const int forced_spans = measure_knob("KVHIP_RAGGED_SPANS", 0);
         if (forced_spans > 0) p.nsplit = std::min(forced_spans, 512);

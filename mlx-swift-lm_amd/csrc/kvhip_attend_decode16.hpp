@@ -193,12 +193,11 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     [[maybe_unused]] RaggedSpan span;
     [[maybe_unused]] int wid = 0;
     if constexpr (MM == 1) {
-        if (tiles_per_wg < 0) {
-            const int wgs = nsplit * a.B;
+        if (__builtin_expect(tiles_per_wg < 0, 0)) {
             wid = b * nsplit + split;
-            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, wgs, WAVES, wid, true);
+            span = ragged_span(a.mask, a.B, a.L, a.T, tiles_total, nsplit, WAVES, wid, true);
             if (span.count == 0) return;  // (workgroup-uniform)
-            part_slot = (size_t)hk * wgs + wid;
+            part_slot = (size_t)hk * nsplit * a.B + wid;
             b = span.b;
             bh = b * a.Hkv + hk;
         } else if (tiles_per_wg == 0 && a.B <= 64 && a.B > 2) {
@@ -207,15 +206,22 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
             part_slot = (size_t)bh * nsplit + split;
         }
     }
-    const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
+    [[maybe_unused]] SymMask sym{};
     int tile_begin = split * tiles_per_wg;
     int tile_end = min(tiles_total, tile_begin + tiles_per_wg);
     if constexpr (MM == 1) {
-        const TileRange vis = visible_tiles(sym, tiles_total, true);
-        const int per = tiles_per_wg > 0 ? tiles_per_wg
-                                         : (max(vis.hi - vis.lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
-        tile_begin = tiles_per_wg < 0 ? span.t.lo : vis.lo + split * per;
-        tile_end = tiles_per_wg < 0 ? span.t.hi : min(vis.hi, tile_begin + per);
+        if (__builtin_expect(tiles_per_wg < 0, 0)) {
+            sym = span.sym;
+            tile_begin = span.t.lo;
+            tile_end = span.t.hi;
+        } else {
+            sym = sym_mask_init(a.mask, b, a.L, a.T);
+            const TileRange vis = visible_tiles(sym, tiles_total, true);
+            const int per = tiles_per_wg > 0 ? tiles_per_wg
+                                             : (max(vis.hi - vis.lo, 1) + nsplit * WAVES - 1) / (nsplit * WAVES) * WAVES;
+            tile_begin = vis.lo + split * per;
+            tile_end = min(vis.hi, tile_begin + per);
+        }
     }
     // (wave-uniform by construction; saying so keeps the page walk in scalar registers and scalar loads)
     const int tile0 = __builtin_amdgcn_readfirstlane(tile_begin + wave);

@@ -198,41 +198,61 @@ __device__ __forceinline__ TileRange visible_tiles(const SymMask &s, int tiles_t
     return t;
 }
 
-// Workgroup `wid` of the `wgs` that share one kv head's batch rows (2 <= B <= 64, B <= wgs <= 512, `waves` wavefronts
-// each, which take every waves-th tile): all spans have the same length and a row gets as many as its keys need, so that
-// the launch lasts as long as the batch's keys do in all and not as its longest row does.  The length is the first from an
-// even share on -- the rows' last spans taken for half full -- with which the spans go round.  Every workgroup works the
-// partition out for itself, a lane to a batch row (about half a microsecond; the sums are of small whole numbers, exact in
-// float).  Spans of a row are adjacent: first .. first + count - 1; count 0: nothing is left for this workgroup.
+// ceil(x / d) for small whole numbers, r = 1 / d (a quotient in float, put right by its remainder)
+__device__ __forceinline__ int quotient_up(int x, int d, float r) {
+    x += d - 1;
+    const int q = (int)((float)x * r), rem = x - q * d;
+    return q + (rem >= d ? 1 : rem < 0 ? -1 : 0);
+}
+// Workgroup `wid` of the nsplit * B that share one kv head's batch rows (2 <= B <= 64, 2 <= nsplit, at most 512 workgroups,
+// of `waves` wavefronts each, which take every waves-th tile): all spans have the same length and a row gets as many as its
+// keys need, so that the launch lasts as long as the batch's keys do in all and not as its longest row does.  The length is
+// the first from an even share on with which the spans go round -- unless the longest row over nsplit spans of its own is
+// done as soon, and then every row goes by its own length over up to nsplit spans.  Workgroups without a span are the last.
+// Every workgroup works the partition out for itself, a lane to a batch row, and hands on the row's bounds, which are in
+// the lanes already (the sums are of small whole numbers, exact in float).  Spans of a row are adjacent:
+// first .. first + count - 1; count 0: nothing is left for this workgroup.
 // (B16 of 1024 to 16384 keys, 4 new tokens, 8 kv heads of 128 at 4 bits, the kernel 42 us with every row over the same
 // number of spans, long rows and short ones paired on the CUs.)
 struct RaggedSpan {
     int b, first, count;  // batch row; its spans
     TileRange t;          // this workgroup's tiles
+    SymMask sym;          // what the row sees
 };
-__device__ __forceinline__ RaggedSpan ragged_span(const MaskDev &m, int B, int L, int T, int tiles_total, int wgs, int waves, int wid, bool all_if_empty) {
-    const int lane = threadIdx.x & 63;
-    TileRange mine{0, 0};
-    if (lane < B) mine = visible_tiles(sym_mask_init(m, lane, L, T), tiles_total, all_if_empty);
-    const int tiles = max(mine.hi - mine.lo, 0), steps = (tiles + waves - 1) / waves;
-    const int total = (int)wave_sum((float)steps);
-    int len = max(1, (2 * total + 2 * wgs - B - 1) / (2 * wgs - B)), spans;
+__device__ __forceinline__ RaggedSpan ragged_span(const MaskDev &m, int B, int L, int T, int tiles_total, int nsplit, int waves, int wid, bool all_if_empty) {
+    const int lane = threadIdx.x & 63, wgs = nsplit * B;
+    const SymMask row = sym_mask_init(m, min(lane, B - 1), L, T);
+    const TileRange mine = visible_tiles(row, tiles_total, all_if_empty);
+    const int tiles = lane < B ? max(mine.hi - mine.lo, 0) : 0, steps = (tiles + waves - 1) / waves;
+    auto lane_of = [](int v, int l) { return __builtin_amdgcn_readlane(v, l); };
+    auto end_of = [&](float upto, int l) { return (int)__builtin_bit_cast(float, lane_of(__builtin_bit_cast(int, upto), l)); };
+    int len = max(1, quotient_up(steps, nsplit, __builtin_amdgcn_rcpf((float)nsplit)));  // a row's own
+    const int most = (int)wave_max((float)len);
+    int spans;
     float upto;
-    for (;; ++len) {  // (ends: with `len` the longest row's steps every row has one span, and B <= wgs)
-        spans = lane < B ? max(1, (steps + len - 1) / len) : 0;
+    auto share = [&]() {
+        spans = lane < B ? max(1, quotient_up(steps, len, __builtin_amdgcn_rcpf((float)len))) : 0;
         upto = wave_scan((float)spans);
-        if (__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, upto), 63)) <= (float)wgs) break;
+        return end_of(upto, 63);
+    };
+    const int own = len;
+    len = max(1, quotient_up((int)wave_sum((float)steps), wgs, __builtin_amdgcn_rcpf((float)wgs)));
+    while (len < most && share() > wgs) ++len;
+    if (len >= most) {  // wave-uniform
+        len = own;
+        share();
     }
-    const unsigned long long before = __ballot(lane < B && upto <= (float)wid);
+    const int before = __popcll(__ballot(lane < B && upto <= (float)wid));
     RaggedSpan r;
-    r.b = min(__popcll(before), B - 1);
-    const bool some = __popcll(before) < B;
-    const int end = (int)__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, upto), r.b));
-    r.count = some ? __builtin_amdgcn_readlane(spans, r.b) : 0;
-    r.first = end - r.count;
-    const int lo = __builtin_amdgcn_readlane(mine.lo, r.b), hi = __builtin_amdgcn_readlane(mine.hi, r.b);
-    r.t.lo = lo + (wid - r.first) * len * waves;
-    r.t.hi = min(hi, r.t.lo + len * waves);
+    r.b = min(before, B - 1);
+    r.count = before < B ? lane_of(spans, r.b) : 0;
+    r.first = end_of(upto, r.b) - r.count;
+    len = lane_of(len, r.b);
+    r.t.lo = lane_of(mine.lo, r.b) + (wid - r.first) * len * waves;
+    r.t.hi = min(lane_of(mine.hi, r.b), r.t.lo + len * waves);
+    r.sym = row;
+    r.sym.len_b = lane_of(row.len_b, r.b);
+    r.sym.pad_b = lane_of(row.pad_b, r.b);
     return r;
 }
 

@@ -1,5 +1,6 @@
-"""Batches of rows of very different lengths: the decode kernels share their spans out by length (2 to 64 rows) or give
-every row the same number (more rows).  Against the plain kernel, which knows nothing of spans, over the same cache."""
+"""Batches of rows of very different lengths: the decode kernels share their spans out by length (2 to 64 rows, where a
+workgroup has more than one step over the longest) or give every row the same number.  Against the plain kernel, which
+knows nothing of spans, over the same cache."""
 import pytest
 import torch
 
@@ -26,13 +27,16 @@ def _pads(how, B, gen):
 
 @pytest.mark.parametrize("how", ["one long", "equal", "steps", "random"])
 @pytest.mark.parametrize("B", [2, 3, 16, 64, 65])
+@pytest.mark.parametrize("many", [False, True])  # (batch, kv head) pairs: few, a step to a workgroup; 120 and more, several
 @pytest.mark.parametrize("kind,Hq,L", [(4, 8, 1), (8, 4, 2), (4, 8, 4), (5, 4, 1), ("bf16", 8, 1), ("f16", 4, 4)])
-def test_ragged_rows_equal_the_plain_kernel(kind, Hq, L, B, how):
+def test_ragged_rows_equal_the_plain_kernel(kind, Hq, L, many, B, how):
+    hkv = {2: 64, 3: 40, 16: 8}.get(B, HKV) if many else HKV
+    Hq = Hq // HKV * hkv
     gen = torch.Generator(device="cuda").manual_seed(3)
     dtype = torch.bfloat16 if kind == "bf16" else torch.float16
     cache = kvhip.KVCacheSimple() if isinstance(kind, str) else kvhip.QuantizedKVCache(64, kind)
     rows = lambda h, n: torch.randn(B, h, n, D, generator=gen, device="cuda").to(dtype)
-    cache._update(rows(HKV, T), rows(HKV, T))
+    cache._update(rows(hkv, T), rows(hkv, T))
     pad = _pads(how, B, torch.Generator().manual_seed(4))
     for lengths in (None, torch.clamp(pad + 700, max=T)):
         mask = kvhip.MaskMode.window_mask(T - L, 0, left_pad=pad, lengths=lengths)
