@@ -155,6 +155,14 @@ template <> struct Geo<8> {
     }
 };
 
+// scale / bias of a (scale, bias) pair of a 16-bit dtype; the first also: the one element in the low half
+template <int DT> __device__ __forceinline__ float pair_scale(uint32_t raw) {
+    return DT == 0 ? (float)__builtin_bit_cast(_Float16, (uint16_t)raw) : __uint_as_float(raw << 16);
+}
+template <int DT> __device__ __forceinline__ float pair_bias(uint32_t raw) {
+    return DT == 0 ? (float)__builtin_bit_cast(_Float16, (uint16_t)(raw >> 16)) : __uint_as_float(raw & 0xffff0000u);
+}
+
 // One tile (64 slots) of raw operand data in registers; lane l owns token l of the tile
 // for K and head-dim column l (+64h) for V.
 template <int BITS, int D, int G> struct TileRegs {
@@ -162,7 +170,7 @@ template <int BITS, int D, int G> struct TileRegs {
     static constexpr int VW = 64 * BITS / 32;  // dwords of one V tile row
     uint32_t k[KW];
     uint32_t v[D / 64][VW];
-    float ks[G], kb[G], vs[G], vb[G];
+    uint32_t ksb[G], vsb[G];  // (scale, bias) pairs as stored: turned into floats where they are used, so that nothing waits for them before
     int row;    // presented row of this lane's token, -1 if none
     bool edge;  // wave-uniform: some token of the tile is dead or masked for some query row
 };
@@ -332,13 +340,7 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
             tile_end = min(vis.hi, tile_begin + per);
         }
     }
-    [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees
-    if constexpr (MM == 1) {
-#pragma unroll
-        for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) seen[rg][i] = sym_mask_bounds(sym, (4 * rg + i) % a.L);
-    }
+    [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees (formed behind the first requests)
     // tokens whose V code sits in a high nibble carry 1/16 on the probability side
     const float vfac = (BITS == 4 && (lane & 2)) ? 0.0625f : 1.0f;
 
@@ -388,7 +390,7 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     // own tile requested in front as well and once more behind the row: 8 bits, one sequence of 2000 keys x 64, the step
     // 10.6 us for 10.2; 60 keys x 128 9.5 for 9.2.)
     bool own = false;
-    uint16_t own_k[NH], own_v[NH];
+    uint32_t own_k[NH], own_v[NH];  // (an element each)
     uint32_t own_w[NH];
     if constexpr (MM == 0 && RG == 1) {
         if (a.new_k != nullptr) {  // wave-uniform
@@ -409,14 +411,21 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     }
     auto write_row = [&]() __attribute__((always_inline)) {
         const int slot = a.new_slot;
+        // (the elements' first use, and so the wait for them: turned into floats as soon as they were loaded, they were
+        // waited for in front of the first tile's request)
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            if constexpr (!rot) asm("" : "+v"(own_k[h]));
+            asm("" : "+v"(own_v[h]));
+        }
         quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * D + d) : Elem<DT>::load(&own_k[(d - lane) >> 6], 0); }, D, GS, lane,
+            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * D + d) : pair_scale<DT>(own_k[(d - lane) >> 6]); }, D, GS, lane,
             reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))), [](int, uint32_t) {},
             const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
         char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
         const int bp = v_bitpos<BITS>(slot & (TILE - 1));
         quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return Elem<DT>::load(&own_v[(d - lane) >> 6], 0); }, D, GS, lane, nullptr,
+            [&](int d) { return pair_scale<DT>(own_v[(d - lane) >> 6]); }, D, GS, lane, nullptr,
             [&](int d, uint32_t code) {
                 reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d))[bp >> 5] =
                     (own_w[(d - lane) >> 6] & ~(((1u << BITS) - 1u) << (bp & 31))) | (code << (bp & 31));
@@ -432,18 +441,7 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     int k_loaded = 0, v_loaded = 0;
     auto load_k = [&](T &t) {
         load_words<T::KW>(t.k, kp + (LATE ? k_off : 0) + k_lane);
-        uint32_t kraw[G];  // (scale, bias) pairs of a 16-bit dtype
-        load_words<G>(kraw, ksp + (LATE ? ksb_off : 0) + ksb_lane);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            if (DT == 0) {
-                t.ks[g] = (float)__builtin_bit_cast(_Float16, (uint16_t)kraw[g]);
-                t.kb[g] = (float)__builtin_bit_cast(_Float16, (uint16_t)(kraw[g] >> 16));
-            } else {
-                t.ks[g] = __uint_as_float(kraw[g] << 16);
-                t.kb[g] = __uint_as_float(kraw[g] & 0xffff0000u);
-            }
-        }
+        load_words<G>(t.ksb, ksp + (LATE ? ksb_off : 0) + ksb_lane);
         t.row = slot_next < a.T ? slot_next : -1;
         t.edge = base_next < full_lo || base_next + (TILE - 1) > full_hi;
         ++k_loaded;
@@ -458,18 +456,7 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     auto load_v = [&](T &t) {
 #pragma unroll
         for (int h = 0; h < NH; ++h) load_words<T::VW>(t.v[h], vp + (LATE ? v_off : 0) + v_lane + (size_t)h * 64 * VROW);
-        uint32_t vraw[G];
-        load_words<G>(vraw, vsp + (LATE ? vsb_off : 0) + vsb_lane);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            if (DT == 0) {
-                t.vs[g] = (float)__builtin_bit_cast(_Float16, (uint16_t)vraw[g]);
-                t.vb[g] = (float)__builtin_bit_cast(_Float16, (uint16_t)(vraw[g] >> 16));
-            } else {
-                t.vs[g] = __uint_as_float(vraw[g] << 16);
-                t.vb[g] = __uint_as_float(vraw[g] & 0xffff0000u);
-            }
-        }
+        load_words<G>(t.vsb, vsp + (LATE ? vsb_off : 0) + vsb_lane);
         ++v_loaded;
         if (v_loaded < my_tiles) {
             page_v += PSTEP;
@@ -511,17 +498,17 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
         float ks24[G], vsf[G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            ks24[g] = t.ks[g] * TWO24;
-            vsf[g] = t.vs[g] * vfac;
+            ks24[g] = pair_scale<DT>(t.ksb[g]) * TWO24;
+            vsf[g] = pair_scale<DT>(t.vsb[g]) * vfac;
         }
         auto softmax_rg = [&](auto RGC) {
             constexpr int rg = decltype(RGC)::value;
             float sc[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float s_ = t.kb[0] * qsum[rg][0][i];
+                float s_ = pair_bias<DT>(t.ksb[0]) * qsum[rg][0][i];
 #pragma unroll
-                for (int g = 1; g < G; ++g) s_ = __builtin_fmaf(t.kb[g], qsum[rg][g][i], s_);
+                for (int g = 1; g < G; ++g) s_ = __builtin_fmaf(pair_bias<DT>(t.ksb[g]), qsum[rg][g][i], s_);
 #pragma unroll
                 for (int g = 0; g < G; ++g) s_ = __builtin_fmaf(ks24[g], sacc[rg][g][i], s_);
                 sc[i] = round_dt<DT>(s_);
@@ -582,7 +569,7 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
                 pv[2 * GP - 1] = 0.f;
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
-                    bacc[rg][g][i] = __builtin_fmaf(p, t.vb[g], bacc[rg][g][i]);
+                    bacc[rg][g][i] = __builtin_fmaf(p, pair_bias<DT>(t.vsb[g]), bacc[rg][g][i]);
                     pv[g] = p * vsf[g];
                 }
 #pragma unroll
@@ -642,6 +629,12 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     };
     const bool row_first = own && my_tiles == 1;  // wave-uniform: the first tile is the new row's
     if (my_tiles > 0 && !row_first) request_first();
+    if constexpr (MM == 1) {
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) seen[rg][i] = sym_mask_bounds(sym, (4 * rg + i) % a.L);
+    }
     if constexpr (rot) {
         step.turn(a.turn, bh, R, rot_s);
         __syncthreads();
@@ -851,13 +844,7 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     } else if constexpr (MM == 1) {
         sym = sym_mask_init(a.mask, b, a.L, a.T);
     }
-    [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees
-    if constexpr (MM == 1) {
-#pragma unroll
-        for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) seen[rg][i] = sym_mask_bounds(sym, (4 * rg + i) % a.L);
-    }
+    [[maybe_unused]] KeyBounds seen[RG][4];  // what each carried row sees (formed behind the first requests)
     const int tile0 = tile_begin + wave;
     const int my_tiles = tile0 < tile_end ? (tile_end - tile0 + WAVES - 1) / WAVES : 0;
     // a wavefront's tiles are a page apart: each is found through the page table (a scalar load)
@@ -920,7 +907,7 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
     // row is requested in front of the pieces.
     bool own = false;
     kv_u4 own_k;
-    uint16_t own_v[NP];
+    uint32_t own_v[NP];
     if constexpr (MM == 0) {
         if (a.new_k != nullptr) {  // wave-uniform
             const int tl = a.new_slot >> 6;
@@ -945,6 +932,12 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
         if constexpr (!rot) load_queries();
         if (!row_first) request_first();
     }
+    if constexpr (MM == 1) {
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) seen[rg][i] = sym_mask_bounds(sym, (4 * rg + i) % a.L);
+    }
     if constexpr (rot) {
         step.turn(a.turn, bh, R, rot_s);
         __syncthreads();
@@ -958,7 +951,7 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
             if (lane < D / 8)
                 *reinterpret_cast<kv_u4 *>(kc + kfp_off(st, slot, 8 * lane)) = rot ? *reinterpret_cast<const kv_u4 *>(rot_s + R * D + 8 * lane) : own_k;
 #pragma unroll
-            for (int h = 0; h < NP; ++h) *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, 64 * h + lane)) = own_v[h];
+            for (int h = 0; h < NP; ++h) *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, 64 * h + lane)) = (uint16_t)own_v[h];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
             if (row_first) request_first();

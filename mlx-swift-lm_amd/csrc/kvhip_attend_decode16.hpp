@@ -245,7 +245,7 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     // are requested in front of the tile.
     constexpr int NHK = (DK + 63) / 64, NHV = (DV + 63) / 64;
     bool own = false;
-    uint16_t own_k[NHK], own_v[NHV];
+    uint32_t own_k[NHK], own_v[NHV];  // (an element each)
     uint32_t own_w[NHV][2];
     if constexpr (MM == 0) {
         if (a.new_k != nullptr) {  // wave-uniform
@@ -273,15 +273,21 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     }
     auto write_row = [&]() __attribute__((always_inline)) {
         const int slot = a.new_slot;
+        // (the elements' first use, and so the wait for them: as in the 4-row kernel)
+#pragma unroll
+        for (int h = 0; h < NHK; ++h)
+            if constexpr (!rot) asm("" : "+v"(own_k[h]));
+#pragma unroll
+        for (int h = 0; h < NHV; ++h) asm("" : "+v"(own_v[h]));
         quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * DK + d) : Elem<DT>::load(&own_k[(d - lane) >> 6], 0); }, DK, GS, lane,
+            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * DK + d) : sb_scale<DT>(own_k[(d - lane) >> 6]); }, DK, GS, lane,
             reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))), [](int, uint32_t) {},
             const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
         char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
         const int bp = v_bitpos<BITS>(slot & (TILE - 1)), sh = bp & 31;
         constexpr uint32_t M = (1u << BITS) - 1u;
         quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return Elem<DT>::load(&own_v[(d - lane) >> 6], 0); }, DV, GS, lane, nullptr,
+            [&](int d) { return sb_scale<DT>(own_v[(d - lane) >> 6]); }, DV, GS, lane, nullptr,
             [&](int d, uint32_t code) {
                 uint32_t *p = reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d)) + (bp >> 5);
                 const uint32_t (&old)[2] = own_w[(d - lane) >> 6];

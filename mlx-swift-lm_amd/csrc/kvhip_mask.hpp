@@ -108,11 +108,11 @@ struct KeyBounds {
     int lo, hi;
     __device__ __forceinline__ bool keep(int j) const { return j >= lo && j <= hi; }
 };
+// (No branches: a wavefront forms those of four rows and more per group at its start.)
 __device__ __forceinline__ KeyBounds sym_mask_bounds(const SymMask &s, int l) {
-    if (s.mode == KVHIP_MASK_CAUSAL) return KeyBounds{0, s.T - s.L + l};
-    KeyBounds k{s.pad_b, min(s.offset + l, s.len_b - 1)};
-    if (s.window > 0) k.lo = max(k.lo, s.offset + l - s.window + 1);
-    return k;
+    const bool causal = s.mode == KVHIP_MASK_CAUSAL;
+    const int from = !causal && s.window > 0 ? s.offset - s.window + 1 : -0x40000000, upto = causal ? s.T - s.L : s.offset;
+    return KeyBounds{max(causal ? 0 : s.pad_b, from + l), min(causal ? 0x7fffffff : s.len_b - 1, upto + l)};
 }
 
 // Inclusive range of key rows any query position l in [0, L) may see under an index-only mask.
