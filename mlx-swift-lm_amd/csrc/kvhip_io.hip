@@ -937,9 +937,17 @@ hipError_t launch_append_quant_rows(const Store &st, const void *keys, const voi
 // as they are 4.6 / 5.0 for 4, 5.8 / 5.2 for 5; x 256, groups of 128, 7.4 / 5.9 rotated for 3 and 5.5 / 6.0, 7.1 / 6.0 for
 // 4 and 5; x 64 5.0 / 4.8 rotated for 4, 4.0 / 4.0 and 4.7 / 4.0 for 4 and 6.  Keys of 192 with values of 128 take two
 // launches: 9.4 / 9.6 for 9 and 10.8 / 9.6 for 12, rotated 13.6 / 12.6 and 15.2 / 12.3.
+// Where the tile kernel's pieces no longer run at once and the row kernel's workgroups still do, the line lies higher.  Tile
+// less row kernel, us, 256 and 512 pairs: rotated, 4 rows, 4 bits x 128 +0.1 and +0.8, 8 bits +0.8 and +1.0 (128 pairs -0.6,
+// -0.2; 1024 pairs -1.0, -0.9), 5 rows -1.7 and -1.8, -1.2 and -1.3, but 3 bits -1.4 and -2.4 for 4; as they are, 5 rows, 4
+// bits +0.2 and +0.8, 8 bits +1.6 and +0.9, x 64 +0.3 and +0.5, 3 bits -0.6 and -0.4, 6 bits x 64 +0.4 and +0.6; x 256 in
+// groups of 128 +0.1 and +1.9 for 8 rows, -3.4 and -2.4 for 12; keys of 192 rotated, 512 pairs, +0.9 for 12, -5.0 for 16.
 int quant_tile_rows(const Store &st, bool rotated) {
-    if (quant_tiles_two_sided(st)) return 12;
-    return rotated ? 3 : 5;
+    const bool between = st.BH > 128 && st.BH < 1024, stream = st.bits != 4 && st.bits != 8;
+    if (quant_tiles_two_sided(st)) return rotated && between && st.BH > 256 ? 14 : 12;
+    if (rotated) return between && !stream ? 5 : 3;
+    if (!between || (stream && st.Dk > 64)) return 5;
+    return st.Dk == 256 && st.gs == 128 ? 12 : 8;
 }
 
 hipError_t launch_append_quant(const Store &st, const void *keys, const void *values, int L, int src0,
