@@ -469,11 +469,12 @@ PlanWide plan_wide(const AttendArgs &a) {
     p.row_blocks = (R + 16 * p.qt - 1) / (16 * p.qt);
     p.tiles = (a.slots + WT - 1) / WT;
     // One token: a workgroup per CU (two: B8 over 4096 keys 29.4 us against 26.8), parts of a tile and up (two: 11.2 us against
-    // 10.1 for a sequence of 2048 keys, the merge, which has every part's loads in flight at once, 3.5 us for either).
+    // 10.1 for a sequence of 2048 keys, the merge, which has every part's loads in flight at once, 3.5 us for either), but
+    // up to three tiles one part, without a merge (a step of 60 keys 12.6 us against 14.4, of 90 13.7 against 14.5).
     // Chunks: two per CU (one: 76 us against 57 for 512 x 2048; three, which need a second round: 72 us).
     static const int target = measure_knob("KVHIP_WIDE_TARGET", 256), target2 = measure_knob("KVHIP_WIDE_TARGET2", 512), least = measure_knob("KVHIP_WIDE_LEAST", 1);  // (timing builds only)
     const long wgs = (long)p.row_blocks * a.st.BH;
-    int n = (int)std::max(1L, std::min<long>((p.qt == 1 ? target : target2) / std::max(1L, wgs), p.tiles / (p.qt == 1 ? least : 4)));
+    int n = p.qt == 1 && p.tiles <= 3 ? 1 : (int)std::max(1L, std::min<long>((p.qt == 1 ? target : target2) / std::max(1L, wgs), p.tiles / (p.qt == 1 ? least : 4)));
     n = std::min(n, 64);
     const size_t per_part = (size_t)a.st.BH * R * (a.st.Dv + 2) * sizeof(float);
     while (n > 1 && a.workspace_cap && per_part * n > a.workspace_cap) --n;
