@@ -123,7 +123,8 @@ kvhip_status kvhip_sync(void *stream);
 /* 0 = choose the fastest kernel for the shape (default); 1 = always the generic kernel; 2 and 3 = as 0, but a
  * prompt chunk over a quantized cache never (2) or whenever the shape allows (3) runs dequantize-first -- the
  * cached rows converted once into scratch pages, then the full-precision tile -- instead of by row count.
- * The setting, kvhip_last_attend_kernel and the profile record below belong to the calling thread. */
+ * The setting, kvhip_last_attend_kernel, kvhip_last_append_kernel and the profile record below belong to the calling
+ * thread. */
 void kvhip_set_kernel_policy(int32_t policy);
 /*
  * Measurement hooks (no counterpart in the reference, which times whole
@@ -141,6 +142,9 @@ void kvhip_set_kernel_policy(int32_t policy);
  * quantized cache of such head sizes, or one with float32 scales, was dequantized into first; -1 before the first
  * call.  For tests and reports. */
 int32_t kvhip_last_attend_kernel(void);
+/* Which kernel the last append launch of this thread used: 0 rows (a workgroup to a row, or to a tile's few quantized rows),
+ * 1 64-token tiles; -1 before the first.  Rows that the attention kernel writes itself do not count.  For tests. */
+int32_t kvhip_last_append_kernel(void);
 void kvhip_profile_enable(int32_t every);
 kvhip_status kvhip_profile_read(int32_t *out_launches, double *out_total_ms);
 

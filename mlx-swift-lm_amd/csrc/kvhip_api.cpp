@@ -877,6 +877,7 @@ kvhip_status kvhip_sync(void *stream) {
 void kvhip_set_kernel_policy(int32_t policy) { g_policy = policy; }
 
 int32_t kvhip_last_attend_kernel(void) { return g_last_kernel; }
+int32_t kvhip_last_append_kernel(void) { return last_append_kernel(); }
 
 void kvhip_profile_enable(int32_t every) { profile_enable(every); }
 

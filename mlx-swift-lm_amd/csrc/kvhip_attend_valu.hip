@@ -12,7 +12,8 @@
 // A workgroup takes RB query rows of one kv head (row = query head of the group * L + position) and one range of
 // key tiles; its four wavefronts walk alternate tiles with their own running maximum / sum / accumulators and are
 // merged through LDS at the end.  With more than one key range per (kv head, row block) the workgroup writes an
-// unnormalised partial and `merge_valu_kernel` finishes the rows.
+// unnormalised partial, and `combine_kernel` (float32 values of 64 / 80 / 96 / 128 / 256 / 512, any of 512) or
+// `merge_valu_kernel` (the rest) finishes the rows.
 #include <algorithm>
 
 #include "kvhip_mask.hpp"

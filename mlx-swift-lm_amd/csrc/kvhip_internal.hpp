@@ -237,6 +237,7 @@ struct RopeDev {
 // ---- kernel launchers (defined in the .hip files) ---------------------------
 // New rows src[l] for l in [src0, src0+n) go to physical slots [slot0, slot0+n); with `rope`
 // the K rows are rotated (and rounded to the cache dtype) on the way in.
+int last_append_kernel();  // kvhip_last_append_kernel: set by the two below
 hipError_t launch_append_fp(const Store &st, const void *keys, const void *values, int L, int src0,
                             int slot0, int n, hipStream_t s, RopeDev *rope = nullptr);
 hipError_t launch_append_quant(const Store &st, const void *keys, const void *values, int L, int src0,
@@ -303,8 +304,8 @@ struct AttendArgs {
     size_t workspace_bytes = 0;
     // Single-token decode (`attentionWithCacheUpdate` with L = 1): the new row [BH, 1, D] of keys and
     // values, still to be written (quantized caches: quantized) into physical slot `new_slot`.  The decode
-    // kernel does it itself -- the wavefront that reads the slot's tile writes the row first -- so a
-    // step needs no launch for the append.  NULL: the row is already in the cache.
+    // kernel does it itself -- the wavefront that reads the slot's tile writes the row behind its first requests and in
+    // front of that tile's -- so a step needs no launch for the append.  NULL: the row is already in the cache.
     const void *new_k = nullptr;
     const void *new_v = nullptr;
     int new_slot = -1;

@@ -823,6 +823,7 @@ __global__ void mask_materialize_kernel(kvhip_mask_plan_t p, uint8_t *dst) {
     } while (0)
 
 namespace {
+thread_local int g_last_append = -1;
 // The caller's rotation as this launch takes it: queries that ride along ride once.
 RopeDev take_rope(RopeDev *rope) {
     if (!rope) return RopeDev();
@@ -834,6 +835,7 @@ RopeDev take_rope(RopeDev *rope) {
 hipError_t launch_append_fp_rows(const Store &st, const void *keys, const void *values, int L, int src0,
                                  int slot0, int n, hipStream_t s, const RopeDev &r) {
     if (n <= 0) return hipSuccess;
+    g_last_append = 0;
     const dim3 block(r.qx ? 256 : 128), grid(n, st.BH + rope_ride_rows(r, n, st.es, block.x));
     // (without queries an instance of its own: their LDS table cost the plain append of 512 rows of 64 (batch, head) pairs x 80
     // 25 us instead of 21)
@@ -850,6 +852,8 @@ hipError_t launch_append_fp_rows(const Store &st, const void *keys, const void *
 }
 }  // namespace
 
+int last_append_kernel() { return g_last_append; }
+
 hipError_t launch_append_fp(const Store &st, const void *keys, const void *values, int L, int src0,
                             int slot0, int n, hipStream_t s, RopeDev *rope) {
     if (n <= 0) return hipSuccess;
@@ -865,6 +869,7 @@ hipError_t launch_append_fp(const Store &st, const void *keys, const void *value
 #define FP_TILE(ES, DK, DV)                                                                                               \
     do {                                                                                                                  \
         const int gx = tiles * FpTile<ES, DK, DV>::PIECES;                                                                \
+        g_last_append = 1;                                                                                                \
         hipLaunchKernelGGL((append_fp_tile_kernel<ES, DK, DV>), dim3(gx, st.BH + rope_ride_rows(r, gx, st.es, 256)), dim3(256), 0, s, st, \
                            (const char *)keys, (const char *)values, L, src0, slot0, n, r);                               \
         return hipGetLastError();                                                                                         \
@@ -912,6 +917,7 @@ namespace {
 hipError_t launch_append_quant_rows(const Store &st, const void *keys, const void *values, int L, int src0,
                                     int slot0, int n, hipStream_t s, const RopeDev &r) {
     if (n <= 0) return hipSuccess;
+    g_last_append = 0;
     const int ntile = ((slot0 + n - 1) >> 6) - (slot0 >> 6) + 1;
     // (a speculative-verify step appends 4 rows: 8 (row, K or V) items, one per wavefront)
     const dim3 block(n >= 3 ? 512 : 256), grid(ntile, st.BH + rope_ride_rows(r, ntile, st.es, block.x));
@@ -961,6 +967,7 @@ hipError_t launch_append_quant(const Store &st, const void *keys, const void *va
     const int head = std::min(n, TILE - (slot0 & (TILE - 1)));
     const int most = std::max(head, std::min(n - head, TILE));
     if (!tiled || most < quant_tile_rows(st, r.dims > 0)) return launch_append_quant_rows(st, keys, values, L, src0, slot0, n, s, r);
+    g_last_append = 1;
     if (st.bits == 4) return launch_quant_tiles_bits<4, true, false>(st, st, keys, values, L, src0, slot0, n, s, r);
     if (st.bits == 8) return launch_quant_tiles_bits<8, true, false>(st, st, keys, values, L, src0, slot0, n, s, r);
     return launch_quant_tiles_other(st, keys, values, L, src0, slot0, n, s, r);

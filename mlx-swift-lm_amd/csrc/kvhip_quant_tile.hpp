@@ -1,4 +1,4 @@
-// Quantize-on-append of many rows by 64-token tiles, whole ones and the partial ones at either end (from 3 to 12 rows up:
+// Quantize-on-append of many rows by 64-token tiles, whole ones and the partial ones at either end (from 3 to 14 rows up:
 // `quant_tile_rows`): the element functions, the tile body and its two kernels, and the launchers of one code width
 // (instantiated per width in kvhip_io.hip and kvhip_quant_tile_other.hip).
 #pragma once

@@ -9,6 +9,7 @@ import kvhip
 pytestmark = pytest.mark.gpu
 
 PIECES = [64, 5, 65, 130, 64, 200]  # a whole tile, then starts and ends inside tiles and pages
+BATCH, HEADS = 4, 8  # (pieces of a tile and more are past the 512 KB of rows from which tiles take them, at every size)
 
 
 def _shifted(x):
@@ -26,7 +27,7 @@ def test_tiles_equal_single_rows(dtype, D, rotary):
             "odd": kvhip.RoPE(20), "queries": kvhip.RoPE(D)}[rotary]
     tiled, single = kvhip.KVCacheSimple(), kvhip.KVCacheSimple()
     for piece, n in enumerate(PIECES):
-        q, k, v = (torch.randn(2, h, n, D, generator=gen, device="cuda").to(dtype) for h in (6, 3, 3))
+        q, k, v = (torch.randn(BATCH, h, n, D, generator=gen, device="cuda").to(dtype) for h in (2 * HEADS, HEADS, HEADS))
         kk, vv = (k, v) if piece % 2 == 0 else (_shifted(k), _shifted(v))
         if rotary == "queries":
             tiled.update_attend_rope(rope, q, kk, vv, D ** -0.5)
@@ -34,12 +35,14 @@ def test_tiles_equal_single_rows(dtype, D, rotary):
             tiled.update_rope(rope, kk, vv)
         else:
             tiled.update(kk, vv, fetch=False)
+        assert kvhip.load().kvhip_last_append_kernel() == (n >= 64)
         for i in range(n):
             row = k[:, :, i:i + 1].contiguous(), v[:, :, i:i + 1].contiguous()
             if rope is not None:
                 single.update_rope(rope, *row)
             else:
                 single.update(*row, fetch=False)
+        assert kvhip.load().kvhip_last_append_kernel() == 0
     for a, b in zip(tiled.state, single.state):
         assert a.shape == b.shape and torch.equal(a, b)
 
