@@ -163,7 +163,16 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     // group's sixteen tokens loaded into its lanes' registers, 2 G of them per token, are 1 KB a load returned for
     // 64 bytes read: twice what the codes take, and the return path, busy 71 % of the kernel's time, held the rest up.  B16, 16
     // query rows over 16384 keys of 8 kv heads x 128 at 4 bits: 70.3 us, 62.3 with the pairs in LDS.)
-    constexpr bool SB_LDS = GK >= 2 || GV >= 2;
+    // Three groups and more, or rows of 256 elements, leave no registers for them.  With two groups the one wait that opens a
+    // tile costs as much as the loads did where cutting the codes out of bit streams hides those, in launches without a mask
+    // (registers / LDS, us): one token of 6 bits, 32 query and 8 kv heads x 128, 4000 keys of 32 sequences 47.4 / 49.1, 1000 of
+    // 8 13.1 / 13.5 (but four tokens over 8000 keys of 8, masked, 36.4 / 35.7); x 64 in groups of 32, 64 query heads, 1000 keys of
+    // one sequence 3 bits 9.9 / 10.5, 5 bits 10.0 / 10.5, 6 bits 9.9 / 10.3, 8000 of 8 17.7 / 17.5, 18.3 / 18.2, 18.2 / 18.2, but
+    // 2 bits 21.7 / 19.4.  The rest is ahead or level with LDS: 8000 keys x 128 of 8 sequences, one token, 2 / 3 / 5 bits
+    // 25.6 / 23.6, 23.2 / 23.2, 29.5 / 28.2, 4 bits with 64 query heads 25.5 / 23.9; 8 bits 34.9 / 35.3, two and four tokens of
+    // one sequence 16.0 / 15.5 and 17.1 / 16.6.  Behind it stay single tokens of one sequence of 3 and 5 bits x 128, by 0.3 us.
+    constexpr bool SB_REGS = GEN && MM == 0 && (BITS == 6 || (DK == 64 && BITS != 2));
+    constexpr bool SB_LDS = GK >= 3 || GV >= 3 || DK >= 256 || (GK == 2 && !SB_REGS);
     // words between the 64-word pieces the pairs arrive in (G = 2, 4: no lane group's pairs straddle two pieces;
     // the gap keeps the four lane groups' reads on different banks)
     constexpr int SB_PAD_K = (GK == 4 || GK == 2) ? 4 : 0, SB_PAD_V = (GV == 4 || GV == 2) ? 4 : 0;
