@@ -275,8 +275,11 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
                         const uint32_t *p = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, 64 * h + lane)) + (bp >> 5);
                         own_v[h] = vrow[64 * h + lane];
                         own_w[h][0] = p[0];
-                        if (second) own_w[h][1] = p[1];
                     }
+                if (second)  // (apart: an element widened in another block than its load's is waited for there)
+#pragma unroll
+                    for (int h = 0; h < NHV; ++h)
+                        if (64 * h + lane < DV) own_w[h][1] = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, 64 * h + lane))[(bp >> 5) + 1];
             }
         }
     }

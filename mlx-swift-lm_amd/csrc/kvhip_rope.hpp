@@ -250,6 +250,9 @@ template <int DT, int D, int THREADS, int RMAX> struct RopeStep {
             const float inv = r.freqs ? 1.0f / freq : (float)exp(-(double)(int)(threadIdx.x % P) * r.log_base_over_half);
             rope_sincos<false>(rope_angle(r, rope_pos(r, bh, 0), inv), sn, cs);
         }
+        // (`freq` lives to here: its register holds what may be a load in flight, and the angle, formed in it, would wait for
+        // every load requested since, the first tile's with them)
+        asm volatile("" ::"v"(freq));
 #pragma unroll
         for (int j = 0; j < NR; ++j) {
             const int i = threadIdx.x / P + j * NS;
