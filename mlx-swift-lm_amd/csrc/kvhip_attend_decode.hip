@@ -32,6 +32,7 @@
 
 #include "kvhip_mask.hpp"
 #include "kvhip_rope.hpp"
+#include "kvhip_span_merge.hpp"
 #include "kvhip_wave.hpp"
 
 // piece buffers of the full-precision decode kernel (at most the D / 32 pieces of one tile)
@@ -186,7 +187,8 @@ template <int BITS, int D, int G> struct TileRegs {
 // MODE 3: MM 0, with the step's rows still to be rotated.
 template <int BITS, int D, int GS, int DT, int RG, int MODE, int NW>
 __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
-decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_wg, int nsplit) {
+decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs<MODE>::type a) {
+    fetch_arguments(a, tiles_total, tiles_per_wg, nsplit);
     constexpr int MM = MODE == 3 ? 0 : MODE;
     constexpr bool rot = MODE == 3;
     using GEO = Geo<BITS>;
@@ -230,10 +232,10 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     const int r = a.Hq / a.Hkv;
     const int R = r * a.L;
 
-    __shared__ __attribute__((aligned(16))) float cbuf[NW][RR][D + 2];
+    __shared__ __attribute__((aligned(16))) WaveParts<D, NW, RR> parts;
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
     // the end) for the wavefronts to fetch them.
-    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
+    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&parts.rows[0][0][0]);
     [[maybe_unused]] RopeStep<DT, D, NW * 64, 4> step;
     if constexpr (rot)
         step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
@@ -369,6 +371,9 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
     const Table pt = (Table) reinterpret_cast<uintptr_t>(st.pt);
     gptr kp = as_global(pt[page_k].k) + (LATE ? 0 : k_off), ksp = as_global(pt[page_k].ksb) + (LATE ? 0 : ksb_off);
     gptr vp = as_global(pt[page_v].v) + (LATE ? 0 : v_off), vsp = as_global(pt[page_v].vsb) + (LATE ? 0 : vsb_off);
+    // (the new row's page, if there is one to write: looked up with the first tile's, for one wait)
+    const char *own_page = page_table(st)[max(a.new_slot, 0) >> PAGE_SHIFT].v;
+    if constexpr (LATE && MM == 0) asm volatile("" ::"s"(own_page), "s"(kp), "s"(ksp), "s"(vp), "s"(vsp));
     const uint32_t k_lane = lane * st.k_row, v_lane = lane * VROW;
     const uint32_t ksb_lane = lane * st.ksb_row, vsb_lane = lane * st.vsb_row;
     int slot_next = tile0 * TILE + lane;  // slot of this lane's token in the tile loaded next
@@ -399,7 +404,7 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
             if (own) {
                 const uint16_t *krow = static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D;
                 const uint16_t *vrow = static_cast<const uint16_t *>(a.new_v) + (size_t)bh * D;
-                const char *vcell = v_cell_ptr(st, bh, slot);
+                const char *vcell = own_page + (size_t)bh * st.v_cell;
 #pragma unroll
                 for (int h = 0; h < NH; ++h) {
                     if constexpr (!rot) own_k[h] = krow[64 * h + lane];
@@ -538,12 +543,13 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
 #pragma unroll
             for (int i = 0; i < 4; ++i) need = need || (sc[i] > m_run[rg][i]);
             if (__any(need)) {
+                float top[4] = {sc[0], sc[1], sc[2], sc[3]};
+                asm volatile("" : "+v"(top[0]));
+                wave_max4(top);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    float x_ = sc[i];
-                    asm volatile("" : "+v"(x_));
                     // wave-uniform values, kept in scalar registers
-                    const float mn = uniform(fmaxf(m_run[rg][i], wave_max(x_)));
+                    const float mn = uniform(fmaxf(m_run[rg][i], top[i]));
                     const float alpha = (mn == -INFINITY) ? 1.f : fast_exp2((m_run[rg][i] - mn) * LOG2E);
                     m_run[rg][i] = mn;
                     m_use[rg][i] = uniform((mn == -INFINITY) ? 0.f : mn);
@@ -665,16 +671,23 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
         }
     }
 
-    // ---- wavefront partial -> LDS ---------------------------------------------------
-    if (rot) __syncthreads();  // (the rotated rows have been fetched)
+    // ---- the wavefronts' parts -> LDS ---------------------------------------------------
+    if (lane == 0)
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg) *reinterpret_cast<f4 *>(&parts.m[wave][4 * rg]) = f4{m_run[rg][0], m_run[rg][1], m_run[rg][2], m_run[rg][3]};
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
+        wave_sum4(l_part[rg]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            l_part[rg][i] = wave_sum(l_part[rg][i]);
+        for (int g = 0; g < G; ++g) wave_sum4(bacc[rg][g]);
+    }
+    __syncthreads();  // (the rotated rows have been fetched, too)
 #pragma unroll
-            for (int g = 0; g < G; ++g) bacc[rg][g][i] = wave_sum(bacc[rg][g][i]);
-        }
+    for (int rg = 0; rg < RG; ++rg) {
+        float wgt[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wgt[i] = wave_weight(parts, 4 * rg + i, m_run[rg][i]);
+        if (lane == 0) *reinterpret_cast<f4 *>(&parts.l[wave][4 * rg]) = f4{wgt[0] * l_part[rg][0], wgt[1] * l_part[rg][1], wgt[2] * l_part[rg][2], wgt[3] * l_part[rg][3]};
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
 #pragma unroll
@@ -686,59 +699,17 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
                         b_ = bacc[rg][2 * h + 1][i];
                     }
                 }
-                cbuf[wave][4 * rg + i][64 * h + lane] = o_ * TWO24 + b_;
+                parts.rows[wave][4 * rg + i][64 * h + lane] = wgt[i] * (o_ * TWO24 + b_);
             }
-        }
-        if (lane < 4) {
-            cbuf[wave][4 * rg + lane][D] = m_run[rg][lane];
-            cbuf[wave][4 * rg + lane][D + 1] = l_part[rg][lane];
         }
     }
     __syncthreads();
-    // ---- merge the wavefronts; a single span writes the output rows, several leave partials
-    if (nsplit == 1) {
-        for (int idx = threadIdx.x; idx < R * D; idx += NW * 64) {
-            const int i = idx / D, c = idx - i * D;
-            float mx = -INFINITY;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) mx = fmaxf(mx, cbuf[w][i][D]);
-            float v = 0.f, l = 0.f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const float mw = cbuf[w][i][D];
-                const float wgt = (mw == -INFINITY) ? 0.f : fast_exp2((mw - mx) * LOG2E);
-                v += wgt * cbuf[w][i][c];
-                l += wgt * cbuf[w][i][D + 1];
-            }
-            const int rep = i / a.L, lq = i - rep * a.L;
-            Elem<DT>::store(a.out, ((size_t)(b * a.Hq + hk * r + rep) * a.L + lq) * D + c, l > 0.f ? v / l : 0.f);
-        }
-        return;
-    }
-    float *part = a.workspace + part_slot * RR * (D + 2);
     if constexpr (MM == 1) {
-        if (tiles_per_wg < 0 && wid == span.first && threadIdx.x == 0)  // (for the merge)
+        if (tiles_per_wg < 0 && nsplit > 1 && wid == span.first && threadIdx.x == 0)  // (for the merge)
             span_table(a.workspace, st.BH, nsplit, RR * (D + 2))[bh] = make_int2((int)part_slot, span.count);
     }
-    for (int idx = threadIdx.x; idx < RR * (D + 2); idx += NW * 64) {
-        const int i = idx / (D + 2), c = idx - i * (D + 2);
-        float mx = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) mx = fmaxf(mx, cbuf[w][i][D]);
-        float v;
-        if (c == D) {
-            v = mx;
-        } else {
-            v = 0.f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const float mw = cbuf[w][i][D];
-                const float wgt = (mw == -INFINITY) ? 0.f : fast_exp2((mw - mx) * LOG2E);
-                v += wgt * cbuf[w][i][c];
-            }
-        }
-        part[idx] = v;
-    }
+    // a single span writes the output rows, several leave partials
+    leave_rows<D, DT>(a, parts, R, nsplit == 1, (size_t)(b * a.Hq + hk * r) * a.L, part_slot);
 }
 
 // ---------------------------------------------------------------------------------
@@ -753,7 +724,8 @@ decode_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_
 // probability; rows of a RotatingKVCache are found through the run table.
 template <int D, int DT, int RG, int MODE, bool IDENT>
 __global__ void __launch_bounds__(WAVES * 64, 2)
-decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_wg, int nsplit) {
+decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs<MODE>::type a) {
+    fetch_arguments(a, tiles_total, tiles_per_wg, nsplit);
     constexpr int MM = MODE == 3 ? 0 : MODE;
     constexpr bool rot = MODE == 3;
     constexpr bool BF = DT == 1;
@@ -784,10 +756,10 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
         }
     }
 
-    __shared__ __attribute__((aligned(16))) float cbuf[WAVES][RR][D + 2];
+    __shared__ __attribute__((aligned(16))) WaveParts<D, WAVES, RR> parts;
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
     // the end) for the wavefronts to fetch them.
-    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
+    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&parts.rows[0][0][0]);
     [[maybe_unused]] RopeStep<DT, D, WAVES * 64, RR> step;
     if constexpr (rot)
         step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
@@ -1008,11 +980,12 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
 #pragma unroll
                 for (int i = 0; i < 4; ++i) need = need || (sc[i] > m_run[rg][i]);
                 if (__any(need)) {
+                    float top[4] = {sc[0], sc[1], sc[2], sc[3]};
+                    asm volatile("" : "+v"(top[0]));  // keeps the reductions inside the branch
+                    wave_max4(top);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float x_ = sc[i];
-                        asm volatile("" : "+v"(x_));  // keeps the reduction inside the branch
-                        const float mn = fmaxf(m_run[rg][i], wave_max(x_));
+                        const float mn = fmaxf(m_run[rg][i], top[i]);
                         const float alpha = (mn == -INFINITY) ? 1.f : fast_exp2((m_run[rg][i] - mn) * LOG2E);
                         m_run[rg][i] = mn;
                         l_part[rg][i] *= alpha;
@@ -1066,65 +1039,30 @@ decode_fp_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_p
         }
     }
 
-    if (rot) __syncthreads();  // (the rotated rows have been fetched)
+    if (lane == 0)
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg) *reinterpret_cast<f4 *>(&parts.m[wave][4 * rg]) = f4{m_run[rg][0], m_run[rg][1], m_run[rg][2], m_run[rg][3]};
+#pragma unroll
+    for (int rg = 0; rg < RG; ++rg) wave_sum4(l_part[rg]);
+    __syncthreads();  // (the rotated rows have been fetched, too)
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
+        float wgt[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) l_part[rg][i] = wave_sum(l_part[rg][i]);
+        for (int i = 0; i < 4; ++i) wgt[i] = wave_weight(parts, 4 * rg + i, m_run[rg][i]);
+        if (lane == 0) *reinterpret_cast<f4 *>(&parts.l[wave][4 * rg]) = f4{wgt[0] * l_part[rg][0], wgt[1] * l_part[rg][1], wgt[2] * l_part[rg][2], wgt[3] * l_part[rg][3]};
 #pragma unroll
         for (int h = 0; h < NP; ++h)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) cbuf[wave][4 * rg + i][64 * h + lane] = oacc[rg][h][i];
-        if (lane < 4) {
-            cbuf[wave][4 * rg + lane][D] = m_run[rg][lane];
-            cbuf[wave][4 * rg + lane][D + 1] = l_part[rg][lane];
-        }
+            for (int i = 0; i < 4; ++i) parts.rows[wave][4 * rg + i][64 * h + lane] = wgt[i] * oacc[rg][h][i];
     }
     __syncthreads();
-    // a single span writes the output rows itself, several leave partials for the merge kernel
-    if (nsplit == 1) {
-        for (int idx = threadIdx.x; idx < R * D; idx += WAVES * 64) {
-            const int i = idx / D, c = idx - i * D;
-            float mx = -INFINITY;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) mx = fmaxf(mx, cbuf[w][i][D]);
-            float v = 0.f, l = 0.f;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) {
-                const float mw = cbuf[w][i][D];
-                const float wgt = (mw == -INFINITY) ? 0.f : fast_exp2((mw - mx) * LOG2E);
-                v += wgt * cbuf[w][i][c];
-                l += wgt * cbuf[w][i][D + 1];
-            }
-            const int rep = i / a.L, lq = i - rep * a.L;
-            Elem<DT>::store(a.out, ((size_t)(b * a.Hq + hk * r + rep) * a.L + lq) * D + c, l > 0.f ? v / l : 0.f);
-        }
-        return;
-    }
-    float *part = a.workspace + part_slot * RR * (D + 2);
     if constexpr (MM == 1 && IDENT) {
-        if (tiles_per_wg < 0 && wid == span.first && threadIdx.x == 0)  // (for the merge)
+        if (tiles_per_wg < 0 && nsplit > 1 && wid == span.first && threadIdx.x == 0)  // (for the merge)
             span_table(a.workspace, st.BH, nsplit, RR * (D + 2))[bh] = make_int2((int)part_slot, span.count);
     }
-    for (int idx = threadIdx.x; idx < RR * (D + 2); idx += WAVES * 64) {
-        const int i = idx / (D + 2), c = idx - i * (D + 2);
-        float mx = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) mx = fmaxf(mx, cbuf[w][i][D]);
-        float v;
-        if (c == D) {
-            v = mx;
-        } else {
-            v = 0.f;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) {
-                const float mw = cbuf[w][i][D];
-                const float wgt = (mw == -INFINITY) ? 0.f : fast_exp2((mw - mx) * LOG2E);
-                v += wgt * cbuf[w][i][c];
-            }
-        }
-        part[idx] = v;
-    }
+    // a single span writes the output rows itself, several leave partials for the merge kernel
+    leave_rows<D, DT>(a, parts, R, nsplit == 1, (size_t)(b * a.Hq + hk * r) * a.L, part_slot);
 }
 
 struct Plan {
@@ -1307,8 +1245,8 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
     const int mm = decode_mode(a);
     auto spans_of = [&](int rows) { return p.tiles_per_wg < 0 ? span_table(a.workspace, st.BH, p.nsplit, rows * (st.Dv + 2)) : nullptr; };
 #define DEC_K(BITS, D, GS, DT, RG, MM, NW)                                                                \
-    hipLaunchKernelGGL((decode_kernel<BITS, D, GS, DT, RG, MM, NW>), grid, dim3(NW * 64), 0, s, DecodeArgs<MM>::type(a), \
-                       p.tiles_total, p.tiles_per_wg, p.nsplit)
+    hipLaunchKernelGGL((decode_kernel<BITS, D, GS, DT, RG, MM, NW>), grid, dim3(NW * 64), 0, s, p.tiles_total, p.tiles_per_wg, \
+                       p.nsplit, DecodeArgs<MM>::type(a))
 #define DEC(BITS, D, GS, DT, RG)                                                                          \
     do {                                                                                                  \
         profile_mark(s, true);                                                                            \
@@ -1357,8 +1295,8 @@ hipError_t launch_attend_decode(const AttendArgs &a_in, hipStream_t s) {
 #define FP(D, DT, RG, M, I)                                                                               \
     do {                                                                                                  \
         profile_mark(s, true);                                                                            \
-        hipLaunchKernelGGL((decode_fp_kernel<D, DT, RG, M, I>), grid, block, 0, s, DecodeArgs<M>::type(a), p.tiles_total, \
-                           p.tiles_per_wg, p.nsplit);                                                     \
+        hipLaunchKernelGGL((decode_fp_kernel<D, DT, RG, M, I>), grid, block, 0, s, p.tiles_total, p.tiles_per_wg, \
+                           p.nsplit, DecodeArgs<M>::type(a));                                                     \
         profile_mark(s, false);                                                                           \
         if (p.nsplit > 1)                                                                                 \
             (void)launch_combine(a, p.nsplit, 4 * RG, s, spans_of(4 * RG));                              \

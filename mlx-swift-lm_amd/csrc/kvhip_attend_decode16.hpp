@@ -35,6 +35,7 @@
 
 #include "kvhip_mask.hpp"
 #include "kvhip_rope.hpp"
+#include "kvhip_span_merge.hpp"
 #include "kvhip_wave.hpp"
 
 namespace kvhip {
@@ -144,7 +145,8 @@ template <int BITS> __device__ __forceinline__ constexpr bool hi_of(int p) { ret
 // MODE 3: MM 0, with the step's rows still to be rotated.
 template <int BITS, int DK, int DV, int GS, int DT, int MODE>
 __global__ void __launch_bounds__(WAVES * 64, (DK >= 256 && BITS == 8) ? 1 : 2)
-decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_per_wg, int nsplit) {
+decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs<MODE>::type a) {
+    fetch_arguments(a, tiles_total, tiles_per_wg, nsplit);
     constexpr int MM = MODE == 3 ? 0 : MODE;
     constexpr bool rot = MODE == 3;
     constexpr bool GEN = BITS != 4 && BITS != 8;  // bit streams
@@ -188,12 +190,12 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     const int R = r * a.L;
     size_t part_slot = (size_t)bh * nsplit + split;  // where this workgroup's partial goes
 
-    __shared__ __attribute__((aligned(16))) float cbuf[WAVES][RR][DV + 2];
+    __shared__ __attribute__((aligned(16))) WaveParts<DV, WAVES, RR> parts;
     __shared__ __attribute__((aligned(16))) uint32_t sbuf[WAVES][2][2][SB_WORDS];  // [wavefront][tile parity][K, V][pairs]
 
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
     // the end) for the wavefronts to fetch them.
-    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&cbuf[0][0][0]);
+    uint16_t *rot_s = reinterpret_cast<uint16_t *>(&parts.rows[0][0][0]);
     [[maybe_unused]] RopeStep<DT, DK, WAVES * 64, RR> step;
     if constexpr (rot)
         step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * DK,
@@ -245,6 +247,19 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     [[maybe_unused]] KeyBounds seen{0, 0};
     if constexpr (MM == 1) seen = sym_mask_bounds(sym, row_l);
 
+    const int tip = tile0 & 3;
+    int page_k = my_tiles > 0 ? tile0 >> 2 : 0, page_v = page_k;
+    // The plane bases of the wavefront's next tile stay wave-uniform (scalar registers) until the loads
+    // that use them are formed: the entry of the following page is asked for right after a tile's loads
+    // are issued and its latency passes behind the tile's arithmetic.  (Adding the lane's offset as soon
+    // as the entry arrived put a wait for the scalar load into every tile: 44 -> 50 us on a ragged
+    // batch of 16 rows.)
+    const ptab pt = page_table(st);
+    gptr kb = as_global(pt[page_k].k), vb = as_global(pt[page_k].v), ksb_b = as_global(pt[page_k].ksb), vsb_b = as_global(pt[page_k].vsb);
+    // (the new row's page, if there is one to write: looked up with the first tile's, for one wait)
+    const char *own_page = pt[max(a.new_slot, 0) >> PAGE_SHIFT].v;
+    if constexpr (MM == 0) asm volatile("" ::"s"(own_page), "s"(kb), "s"(ksb_b), "s"(vb), "s"(vsb_b));
+
     // ---- the step's new row, when it is still to be written (unmasked single-token step) --------
     // Its slot lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one: that wavefront
     // quantizes the row into the cache, with the arithmetic of the append kernel, after it has requested its first tile and
@@ -263,7 +278,7 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
             if (own) {
                 const uint16_t *krow = static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK;
                 const uint16_t *vrow = static_cast<const uint16_t *>(a.new_v) + (size_t)bh * DV;
-                const char *vcell = v_cell_ptr(st, bh, slot);
+                const char *vcell = own_page + (size_t)bh * st.v_cell;
                 const int bp = v_bitpos<BITS>(slot & (TILE - 1));
                 const bool second = (32 % BITS) != 0 && (bp & 31) + BITS > 32;
 #pragma unroll
@@ -315,8 +330,6 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     // K block tb, lane (n, jj): row of token tok(tb, n) = 16 (n / 4) + 4 tb + n % 4, segment jj
     // each page is found through the page table (a scalar load per plane pair); the offsets below are
     // the same in every page
-    const int tip = tile0 & 3;
-    int page_k = my_tiles > 0 ? tile0 >> 2 : 0, page_v = page_k;
     const size_t k_off = (size_t)bh * st.k_cell + (size_t)tip * TILE * st.k_row
                          + (size_t)(16 * (n >> 2) + (n & 3)) * st.k_row + (GEN ? SK::lane_w0(jj) * 4 : jj * (KWL * 4));
     const size_t v_off = (size_t)bh * st.v_cell + (size_t)tip * DV * VROW + (size_t)n * VROW + (GEN ? SV::lane_w0(jj) * 4 : jj * (VWL * 4));
@@ -325,13 +338,6 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
     // (scale, bias) pairs of this lane group's 16 tokens, 16 jj .. 16 jj + 15
     const size_t ksb_off = (size_t)bh * st.ksb_cell + (size_t)(tip * TILE + 16 * jj) * st.ksb_row;
     const size_t vsb_off = (size_t)bh * st.vsb_cell + (size_t)(tip * TILE + 16 * jj) * st.vsb_row;
-    // The plane bases of the wavefront's next tile stay wave-uniform (scalar registers) until the loads
-    // that use them are formed: the entry of the following page is asked for right after a tile's loads
-    // are issued and its latency passes behind the tile's arithmetic.  (Adding the lane's offset as soon
-    // as the entry arrived put a wait for the scalar load into every tile: 44 -> 50 us on a ragged
-    // batch of 16 rows.)
-    const ptab pt = page_table(st);
-    gptr kb = as_global(pt[page_k].k), vb = as_global(pt[page_k].v), ksb_b = as_global(pt[page_k].ksb), vsb_b = as_global(pt[page_k].vsb);
     int base_next = tile0 * TILE;
 
     struct Tile {
@@ -715,8 +721,8 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         }
     }
 
-    if (rot) __syncthreads();  // (the rotated rows have been fetched)
-    // ---- wavefront partial -> LDS: lane (n, jj) holds out^T[d = 16 db + 4 jj + i][row n] ---------
+    // ---- the wavefronts' parts -> LDS: lane (n, jj) holds out^T[d = 16 db + 4 jj + i][row n] ---------
+    if (jj == 0) parts.m[wave][n] = m_run;
     if constexpr (SPLIT_HI) {
         l_part = __builtin_fmaf(l_hi, 16.f, l_part);
 #pragma unroll
@@ -729,63 +735,21 @@ decode16_kernel(typename DecodeArgs<MODE>::type a, int tiles_total, int tiles_pe
         bacc[g] += __shfl_xor(bacc[g], 16);
         bacc[g] += __shfl_xor(bacc[g], 32);
     }
+    __syncthreads();  // (the rotated rows have been fetched, too)
+    const float wgt = wave_weight(parts, n, m_run);
+    if (jj == 0) parts.l[wave][n] = wgt * l_part;
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         const int g = (16 * db) / GS;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            cbuf[wave][n][16 * db + 4 * jj + i] = oacc[db][i] * TWO24 + bacc[g];
-    }
-    if (jj == 0) {
-        cbuf[wave][n][DV] = m_run;
-        cbuf[wave][n][DV + 1] = l_part;
+        *reinterpret_cast<f4 *>(&parts.rows[wave][n][16 * db + 4 * jj]) = wgt * (oacc[db] * TWO24 + bacc[g]);
     }
     __syncthreads();
-    // ---- merge the 4 wavefronts; a single span writes the output rows, several leave partials ---
-    // the weights of a row's four parts once per row (not once per column: an exponential each)
-    __shared__ float wrow[WAVES][RR], mrow[RR];
-    if (threadIdx.x < WAVES * RR) {
-        const int i = threadIdx.x / WAVES, w = threadIdx.x - i * WAVES;
-        float mx = -INFINITY;
-#pragma unroll
-        for (int w2 = 0; w2 < WAVES; ++w2) mx = fmaxf(mx, cbuf[w2][i][DV]);
-        const float mw = cbuf[w][i][DV];
-        wrow[w][i] = (mw == -INFINITY) ? 0.f : fast_exp2((mw - mx) * LOG2E);
-        if (w == 0) mrow[i] = mx;
-    }
-    __syncthreads();
-    if (nsplit == 1) {
-        for (int idx = threadIdx.x; idx < R * DV; idx += WAVES * 64) {
-            const int i = idx / DV, c = idx - i * DV;
-            float v = 0.f, l = 0.f;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) {
-                const float wgt = wrow[w][i];
-                v += wgt * cbuf[w][i][c];
-                l += wgt * cbuf[w][i][DV + 1];
-            }
-            const int rep = i / a.L, lq = i - rep * a.L;
-            Elem<DT>::store(a.out, ((size_t)(b * a.Hq + hk * r + rep) * a.L + lq) * DV + c, l > 0.f ? v / l : 0.f);
-        }
-        return;
-    }
-    float *part = a.workspace + part_slot * RR * (DV + 2);
     if constexpr (MM == 1) {
-        if (tiles_per_wg < 0 && wid == span.first && threadIdx.x == 0)  // (for the merge)
+        if (tiles_per_wg < 0 && nsplit > 1 && wid == span.first && threadIdx.x == 0)  // (for the merge)
             span_table(a.workspace, st.BH, nsplit, RR * (DV + 2))[bh] = make_int2((int)part_slot, span.count);
     }
-    for (int idx = threadIdx.x; idx < RR * (DV + 2); idx += WAVES * 64) {
-        const int i = idx / (DV + 2), c = idx - i * (DV + 2);
-        float v;
-        if (c == DV) {
-            v = mrow[i];
-        } else {
-            v = 0.f;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) v += wrow[w][i] * cbuf[w][i][c];
-        }
-        part[idx] = v;
-    }
+    // a single span writes the output rows, several leave partials
+    leave_rows<DV, DT>(a, parts, R, nsplit == 1, (size_t)(b * a.Hq + hk * r) * a.L, part_slot);
 }
 
 }  // namespace
@@ -799,10 +763,10 @@ hipError_t launch_decode16_bits(const AttendArgs &a, int tiles_total, int tiles_
     const int mm = decode_mode(a);
 #define D16_M(DK, DV, GS, DT)                                                                                   \
     do {                                                                                                        \
-        if (mm == 0) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 0>), grid, block, 0, s, a, tiles_total, tiles_per_wg, nsplit); \
-        else if (mm == 3) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 3>), grid, block, 0, s, AttendStepArgs(a), tiles_total, tiles_per_wg, nsplit); \
-        else if (mm == 1) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 1>), grid, block, 0, s, a, tiles_total, tiles_per_wg, nsplit); \
-        else hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 2>), grid, block, 0, s, a, tiles_total, tiles_per_wg, nsplit); \
+        if (mm == 0) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 0>), grid, block, 0, s, tiles_total, tiles_per_wg, nsplit, a); \
+        else if (mm == 3) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 3>), grid, block, 0, s, tiles_total, tiles_per_wg, nsplit, AttendStepArgs(a)); \
+        else if (mm == 1) hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 1>), grid, block, 0, s, tiles_total, tiles_per_wg, nsplit, a); \
+        else hipLaunchKernelGGL((decode16_kernel<BITS, DK, DV, GS, DT, 2>), grid, block, 0, s, tiles_total, tiles_per_wg, nsplit, a); \
     } while (0)
 #define D16_DT(DK, DV, GS)                             \
     do {                                               \

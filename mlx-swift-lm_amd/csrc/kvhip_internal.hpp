@@ -290,25 +290,26 @@ hipError_t launch_set_pages(void *clear, size_t bytes, PageEntry *pt, int first,
 // Every plane of pages [0, pages) of `src` into the same pages of `dst` (stores of one geometry).
 hipError_t launch_copy_pages(const Store &src, const Store &dst, int pages, hipStream_t s);
 
+// (What every decode kernel starts from stands first, in whole cache lines of the argument segment: fetch_arguments.)
 struct AttendArgs {
     Store st;
-    Runs runs;
     const void *q = nullptr;  // [B, Hq, L, Dk]
     void *out = nullptr;      // [B, Hq, L, Dv]
-    int32_t B = 0, Hq = 0, Hkv = 0, L = 0;
-    int32_t T = 0;            // presented length
-    int32_t slots = 0;        // physical slots in use span [0, slots)
-    float scale = 1.f;
-    MaskDev mask;
-    float *workspace = nullptr;
-    size_t workspace_bytes = 0;
     // Single-token decode (`attentionWithCacheUpdate` with L = 1): the new row [BH, 1, D] of keys and
     // values, still to be written (quantized caches: quantized) into physical slot `new_slot`.  The decode
     // kernel does it itself -- the wavefront that reads the slot's tile writes the row behind its first requests and in
     // front of that tile's -- so a step needs no launch for the append.  NULL: the row is already in the cache.
     const void *new_k = nullptr;
     const void *new_v = nullptr;
-    int new_slot = -1;
+    float *workspace = nullptr;
+    int32_t new_slot = -1;
+    int32_t B = 0, Hq = 0, Hkv = 0, L = 0;
+    int32_t T = 0;            // presented length
+    int32_t slots = 0;        // physical slots in use span [0, slots)
+    float scale = 1.f;
+    MaskDev mask;
+    Runs runs;
+    size_t workspace_bytes = 0;
     // With new_k: the rotation that the queries and the new key row still need, at the new row's position (host; NULL: none).
     const RopeDev *rope = nullptr;
     // Upper bound on the scratch a launch may plan for (0: none).  The planners then split the sequence over
@@ -324,6 +325,23 @@ struct AttendStepArgs : AttendArgs {
 };
 template <int MODE> struct DecodeArgs { using type = AttendArgs; };
 template <> struct DecodeArgs<3> { using type = AttendStepArgs; };
+#if defined(__HIPCC__)
+// A decode kernel's arguments, requested together and waited for once.  Left alone the compiler loads each in front of its
+// first use, wait behind wait before the first tile is requested.  The first wait is the long one (the arguments are new
+// memory in every launch), so that this alone is level in time; three more arguments looked up apart cost 0.5 us a launch.
+__device__ __forceinline__ void fetch_arguments(const AttendArgs &a, int tiles_total, int tiles_per_wg, int nsplit) {
+    asm volatile("" ::"s"(a.st.pt), "s"(a.st.BH), "s"(a.st.k_cell), "s"(a.st.v_cell), "s"(a.st.ksb_cell), "s"(a.st.vsb_cell), "s"(a.st.k_row),
+                 "s"(a.st.ksb_row), "s"(a.st.vsb_row), "s"(a.q), "s"(a.out), "s"(a.new_k), "s"(a.new_v), "s"(a.workspace), "s"(a.new_slot), "s"(a.Hq),
+                 "s"(a.Hkv), "s"(a.L), "s"(a.T), "s"(a.scale), "s"(tiles_total), "s"(tiles_per_wg), "s"(nsplit));
+}
+__device__ __forceinline__ void fetch_arguments(const AttendStepArgs &a, int tiles_total, int tiles_per_wg, int nsplit) {
+    const RopeDev &r = a.turn;
+    asm volatile("" ::"s"(a.st.pt), "s"(a.st.BH), "s"(a.st.k_cell), "s"(a.st.v_cell), "s"(a.st.ksb_cell), "s"(a.st.vsb_cell), "s"(a.st.k_row),
+                 "s"(a.st.ksb_row), "s"(a.st.vsb_row), "s"(a.q), "s"(a.new_k), "s"(a.new_v), "s"(a.new_slot), "s"(a.Hq), "s"(a.Hkv), "s"(a.T), "s"(a.scale),
+                 "s"(tiles_total), "s"(tiles_per_wg), "s"(nsplit), "s"(r.dims), "s"(r.traditional), "s"(r.freqs), "s"(r.batch_pos), "s"(r.pos0), "s"(r.H),
+                 "s"(r.scale), "s"(r.log_base_over_half));
+}
+#endif
 // 0: no mask, 1: index-only mask, 2: array mask, 3: no mask, rows still to be rotated
 inline int decode_mode(const AttendArgs &a) {
     if (a.mask.mode == KVHIP_MASK_NONE) return a.new_k && a.rope ? 3 : 0;

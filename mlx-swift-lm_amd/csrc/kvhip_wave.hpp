@@ -11,32 +11,35 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 
 // Wavefront reductions on the data-parallel-primitive path (no LDS round trips): two quad
 // permutes and two row mirrors leave each row of 16 lanes reduced, two row broadcasts
-// carry the rows into lane 63, which is read out as a wave-uniform scalar.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_take(float v) {  // v of the lane CTRL names; own v outside ROWS
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v),
-                                                                 CTRL, ROWS, 0xF, false));
-}
+// carry the rows into lane 63, which is read out as a wave-uniform scalar.  Written as assembly, an instruction a step:
+// through the permuting-move builtin a step is a copy, a wait, the move and the sum or (quieting) maximum.  A step waits two
+// instructions for the one before it: N values are reduced in turn, one value waits.
+#define KV_DPP_STEP(OP, V, CTRL) #OP "_dpp " V ", " V ", " V " " CTRL "\n\t"
+#define KV_DPP_1(OP, CTRL) KV_DPP_STEP(OP, "%0", CTRL) "s_nop 1\n\t"
+#define KV_DPP_4(OP, CTRL) KV_DPP_STEP(OP, "%0", CTRL) KV_DPP_STEP(OP, "%1", CTRL) KV_DPP_STEP(OP, "%2", CTRL) KV_DPP_STEP(OP, "%3", CTRL)
+#define KV_DPP_REDUCE(STEP, OP)                                                                            \
+    "s_nop 1\n\t" STEP(OP, "quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf")                              \
+    STEP(OP, "quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf") STEP(OP, "row_half_mirror row_mask:0xf bank_mask:0xf") \
+    STEP(OP, "row_mirror row_mask:0xf bank_mask:0xf") STEP(OP, "row_bcast:15 row_mask:0xa bank_mask:0xf")   \
+    STEP(OP, "row_bcast:31 row_mask:0xc bank_mask:0xf") "s_nop 1"
+__device__ __forceinline__ float lane_63(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63)); }
 __device__ __forceinline__ float wave_max(float v) {
-    v = fmaxf(v, dpp_take<0xB1, 0xF>(v));   // quad_perm [1,0,3,2]
-    v = fmaxf(v, dpp_take<0x4E, 0xF>(v));   // quad_perm [2,3,0,1]
-    v = fmaxf(v, dpp_take<0x141, 0xF>(v));  // row_half_mirror
-    v = fmaxf(v, dpp_take<0x140, 0xF>(v));  // row_mirror
-    v = fmaxf(v, dpp_take<0x142, 0xA>(v));  // row_bcast15 into rows 1 and 3
-    v = fmaxf(v, dpp_take<0x143, 0xC>(v));  // row_bcast31 into rows 2 and 3
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+    asm(KV_DPP_REDUCE(KV_DPP_1, v_max_f32) : "+v"(v));
+    return lane_63(v);
 }
 __device__ __forceinline__ float wave_sum(float v) {
-    v += dpp_take<0xB1, 0xF>(v);
-    v += dpp_take<0x4E, 0xF>(v);
-    v += dpp_take<0x141, 0xF>(v);
-    v += dpp_take<0x140, 0xF>(v);
-    // the broadcast steps must add only into the rows they target
-    const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xA, 0xF, false));
-    v += r1;
-    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));
-    v += r2;
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+    asm(KV_DPP_REDUCE(KV_DPP_1, v_add_f32) : "+v"(v));
+    return lane_63(v);
+}
+__device__ __forceinline__ void wave_max4(float (&v)[4]) {
+    asm(KV_DPP_REDUCE(KV_DPP_4, v_max_f32) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = lane_63(v[i]);
+}
+__device__ __forceinline__ void wave_sum4(float (&v)[4]) {
+    asm(KV_DPP_REDUCE(KV_DPP_4, v_add_f32) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = lane_63(v[i]);
 }
 
 // inclusive prefix sums over the lanes
