@@ -372,8 +372,9 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
     gptr kp = as_global(pt[page_k].k) + (LATE ? 0 : k_off), ksp = as_global(pt[page_k].ksb) + (LATE ? 0 : ksb_off);
     gptr vp = as_global(pt[page_v].v) + (LATE ? 0 : v_off), vsp = as_global(pt[page_v].vsb) + (LATE ? 0 : vsb_off);
     // (the new row's page, if there is one to write: looked up with the first tile's, for one wait)
-    const char *own_page = page_table(st)[max(a.new_slot, 0) >> PAGE_SHIFT].v;
-    if constexpr (LATE && MM == 0) asm volatile("" ::"s"(own_page), "s"(kp), "s"(ksp), "s"(vp), "s"(vsp));
+    const ptab own_page = page_table(st) + (max(a.new_slot, 0) >> PAGE_SHIFT);
+    char *const own_pk = own_page->k, *const own_pks = own_page->ksb, *const own_pv = own_page->v, *const own_pvs = own_page->vsb;
+    if constexpr (LATE && MM == 0) asm volatile("" ::"s"(own_pk), "s"(own_pks), "s"(own_pv), "s"(own_pvs), "s"(kp), "s"(ksp), "s"(vp), "s"(vsp));
     const uint32_t k_lane = lane * st.k_row, v_lane = lane * VROW;
     const uint32_t ksb_lane = lane * st.ksb_row, vsb_lane = lane * st.vsb_row;
     int slot_next = tile0 * TILE + lane;  // slot of this lane's token in the tile loaded next
@@ -387,57 +388,76 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
 
     // ---- the step's new row, when it is still to be written (unmasked single-token decode) -----
     // Slot T - 1 lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one (spans
-    // are equal and cover every tile): that wavefront quantizes the row into the cache, with the arithmetic of the append
-    // kernel, after it has requested its first tile and before it requests another, so its own later loads of the
-    // row's tile see it; if its first tile is that tile, it requests it only then.  The V code goes into its column's packed
-    // word read-modify-write; the row and the old words are requested in front of the tile.  (The row written first and
-    // the tiles requested behind it: the last wavefront of the launch to finish, by four round trips to memory.  The row's
+    // are equal and cover every tile).  The wavefronts of that workgroup quantize the row into the cache, with the arithmetic
+    // of the append kernel, behind their first tile's request and in front of any other: the row's keys and values go in units
+    // of UC columns (whole groups), shared out from the wavefront behind the tile's reader on, which has the most tiles.  A
+    // barrier stands between the row and later loads of the row's tile; if that is its reader's first, it is requested only then.
+    // V codes go into their columns' packed words read-modify-write; the row and the old words are requested in front of the tile.
+    // (The whole row quantized by the tile's reader, the last wavefront of the launch to finish: 16 layers of 512 keys x 64 at 8 bits
+    // 109.6 us for 107.6, four of 30 000 x 128 at 4 bits 65.8 for 64.5.  The row written first
+    // and the tiles requested behind it: by four round trips to memory later.  The row's
     // own tile requested in front as well and once more behind the row: 8 bits, one sequence of 2000 keys x 64, the step
     // 10.6 us for 10.2; 60 keys x 128 9.5 for 9.2.)
-    bool own = false;
-    uint32_t own_k[NH], own_v[NH];  // (an element each)
-    uint32_t own_w[NH];
+    constexpr int UC = GS > 64 ? GS : 64, EU = UC / 64, NU = D / UC, UPW = (2 * NU + NW - 1) / NW;  // columns and elements of a lane in a unit; units of a side and of a wavefront
+    bool row_here = false, own = false;  // workgroup-uniform; wave-uniform: reads the row's tile
+    int unit0 = 2 * NU;                  // this wavefront's first unit: 0 .. NU - 1 keys, NU .. 2 NU - 1 values
+    uint32_t row_e[UPW][EU], row_w[UPW][EU];
     if constexpr (MM == 0 && RG == 1) {
         if (a.new_k != nullptr) {  // wave-uniform
             const int slot = a.new_slot, tl = slot >> 6;
-            own = tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % NW) == wave;
-            if (own) {
+            row_here = tl >= tile_begin && tl < tile_end;
+            if (row_here) {
+                const int reader = (tl - tile_begin) % NW;
+                own = wave == reader;
+                unit0 = (wave - reader - 1 + 2 * NW) % NW;
                 const uint16_t *krow = static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D;
                 const uint16_t *vrow = static_cast<const uint16_t *>(a.new_v) + (size_t)bh * D;
-                const char *vcell = own_page + (size_t)bh * st.v_cell;
+                const char *vcell = own_pv + (size_t)bh * st.v_cell;
 #pragma unroll
-                for (int h = 0; h < NH; ++h) {
-                    if constexpr (!rot) own_k[h] = krow[64 * h + lane];
-                    own_v[h] = vrow[64 * h + lane];
-                    own_w[h] = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, 64 * h + lane))[v_bitpos<BITS>(slot & (TILE - 1)) >> 5];
+                for (int j = 0; j < UPW; ++j) {
+                    const int u = unit0 + j * NW;
+                    if (u < 2 * NU && !(rot && u < NU)) {
+#pragma unroll
+                        for (int e = 0; e < EU; ++e) {
+                            const int d = (u < NU ? u : u - NU) * UC + 64 * e + lane;
+                            if (u < NU) {
+                                row_e[j][e] = krow[d];
+                            } else {
+                                row_e[j][e] = vrow[d];
+                                row_w[j][e] = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, d))[v_bitpos<BITS>(slot & (TILE - 1)) >> 5];
+                            }
+                        }
+                    }
                 }
             }
         }
     }
     auto write_row = [&]() __attribute__((always_inline)) {
-        const int slot = a.new_slot;
-        // (the elements' first use, and so the wait for them: turned into floats as soon as they were loaded, they were
-        // waited for in front of the first tile's request)
+        const int slot = a.new_slot, bp = v_bitpos<BITS>(slot & (TILE - 1));
+        const size_t in_page = slot & (PAGE - 1);
 #pragma unroll
-        for (int h = 0; h < NH; ++h) {
-            if constexpr (!rot) asm("" : "+v"(own_k[h]));
-            asm("" : "+v"(own_v[h]));
+        for (int j = 0; j < UPW; ++j) {
+            // (the elements' first use, and so the wait for them: turned into floats as soon as they were loaded, they were
+            // waited for in front of the first tile's request)
+#pragma unroll
+            for (int e = 0; e < EU; ++e) asm("" : "+v"(row_e[j][e]));
+            const int u = unit0 + j * NW, from = (u < NU ? u : u - NU) * UC;
+            if (u < NU) {
+                quantize_row_wave_from<DT, BITS>(
+                    [&](int d) { return rot ? Elem<DT>::load(rot_s, R * D + d) : pair_scale<DT>(row_e[j][EU == 1 ? 0 : (d - lane - from) >> 6]); }, from + UC, GS, lane,
+                    reinterpret_cast<uint32_t *>(own_pk + (size_t)bh * st.k_cell + in_page * st.k_row), [](int, uint32_t) {},
+                    own_pks + (size_t)bh * st.ksb_cell + in_page * st.ksb_row, nullptr, nullptr, from);
+            } else if (u < 2 * NU) {
+                char *vcell = own_pv + (size_t)bh * st.v_cell;
+                quantize_row_wave_from<DT, BITS>(
+                    [&](int d) { return pair_scale<DT>(row_e[j][EU == 1 ? 0 : (d - lane - from) >> 6]); }, from + UC, GS, lane, nullptr,
+                    [&](int d, uint32_t code) {
+                        reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d))[bp >> 5] =
+                            (row_w[j][EU == 1 ? 0 : (d - lane - from) >> 6] & ~(((1u << BITS) - 1u) << (bp & 31))) | (code << (bp & 31));
+                    },
+                    own_pvs + (size_t)bh * st.vsb_cell + in_page * st.vsb_row, nullptr, nullptr, from);
+            }
         }
-        quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * D + d) : pair_scale<DT>(own_k[(d - lane) >> 6]); }, D, GS, lane,
-            reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))), [](int, uint32_t) {},
-            const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
-        char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
-        const int bp = v_bitpos<BITS>(slot & (TILE - 1));
-        quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return pair_scale<DT>(own_v[(d - lane) >> 6]); }, D, GS, lane, nullptr,
-            [&](int d, uint32_t code) {
-                reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d))[bp >> 5] =
-                    (own_w[(d - lane) >> 6] & ~(((1u << BITS) - 1u) << (bp & 31))) | (code << (bp & 31));
-            },
-            const_cast<char *>(vsb_row_ptr(st, bh, slot)), nullptr, nullptr);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
 
     // The K half (codes, scales, row bookkeeping) and the V half of tile number k_loaded /
@@ -646,8 +666,11 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
         __syncthreads();
     }
     if constexpr (MM == 0 && RG == 1) {
-        if (own) write_row();
-        if (row_first) request_first();
+        if (row_here) {  // workgroup-uniform
+            write_row();
+            __syncthreads();
+            if (row_first) request_first();
+        }
     }
     if (my_tiles > 0) {
         load_queries();

@@ -257,73 +257,88 @@ decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeAr
     const ptab pt = page_table(st);
     gptr kb = as_global(pt[page_k].k), vb = as_global(pt[page_k].v), ksb_b = as_global(pt[page_k].ksb), vsb_b = as_global(pt[page_k].vsb);
     // (the new row's page, if there is one to write: looked up with the first tile's, for one wait)
-    const char *own_page = pt[max(a.new_slot, 0) >> PAGE_SHIFT].v;
-    if constexpr (MM == 0) asm volatile("" ::"s"(own_page), "s"(kb), "s"(ksb_b), "s"(vb), "s"(vsb_b));
+    const ptab own_page = pt + (max(a.new_slot, 0) >> PAGE_SHIFT);
+    char *const own_pk = own_page->k, *const own_pks = own_page->ksb, *const own_pv = own_page->v, *const own_pvs = own_page->vsb;
+    if constexpr (MM == 0) asm volatile("" ::"s"(own_pk), "s"(own_pks), "s"(own_pv), "s"(own_pvs), "s"(kb), "s"(ksb_b), "s"(vb), "s"(vsb_b));
 
     // ---- the step's new row, when it is still to be written (unmasked single-token step) --------
-    // Its slot lies in the last tile, which exactly one wavefront of one workgroup reads, as its last one: that wavefront
-    // quantizes the row into the cache, with the arithmetic of the append kernel, after it has requested its first tile and
-    // before it requests another, so its own later loads of the row's tile (and of the tile's scale / bias pairs) see it; if
-    // its first tile is that tile, it requests it only then.  A lane owns the V columns it quantizes; their codes go into the
-    // columns' tile rows read-modify-write (a code of a bit stream may lie across two dwords).  The row and the old words
+    // As in the 4-row kernel: the wavefronts of the workgroup whose span holds the row's slot (in the last tile) quantize it
+    // into the cache between them, in units of UC columns, behind their first tile's request, and a barrier stands in front of
+    // later loads of the row's tile (and of the tile's scale / bias pairs).  The V codes go into the columns' tile rows
+    // read-modify-write (a code of a bit stream may lie across two dwords).  The row and the old words
     // are requested in front of the tile.
-    constexpr int NHK = (DK + 63) / 64, NHV = (DV + 63) / 64;
-    bool own = false;
-    uint32_t own_k[NHK], own_v[NHV];  // (an element each)
-    uint32_t own_w[NHV][2];
+    constexpr int UC = GS > 64 ? GS : 64, EU = UC / 64, NUK = (DK + UC - 1) / UC, NUV = (DV + UC - 1) / UC, UPW = (NUK + NUV + WAVES - 1) / WAVES;
+    bool row_here = false, own = false;  // workgroup-uniform; wave-uniform: reads the row's tile
+    int unit0 = NUK + NUV;               // this wavefront's first unit: keys, then values
+    uint32_t row_e[UPW][EU], row_w[UPW][EU][2];
     if constexpr (MM == 0) {
         if (a.new_k != nullptr) {  // wave-uniform
             const int slot = a.new_slot, tl = slot >> 6;
-            own = tl >= tile_begin && tl < tile_end && ((tl - tile_begin) % WAVES) == wave;
-            if (own) {
+            row_here = tl >= tile_begin && tl < tile_end;
+            if (row_here) {
+                const int reader = (tl - tile_begin) % WAVES;
+                own = wave == reader;
+                unit0 = (wave - reader - 1 + 2 * WAVES) % WAVES;
                 const uint16_t *krow = static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK;
                 const uint16_t *vrow = static_cast<const uint16_t *>(a.new_v) + (size_t)bh * DV;
-                const char *vcell = own_page + (size_t)bh * st.v_cell;
+                const char *vcell = own_pv + (size_t)bh * st.v_cell;
                 const int bp = v_bitpos<BITS>(slot & (TILE - 1));
                 const bool second = (32 % BITS) != 0 && (bp & 31) + BITS > 32;
 #pragma unroll
-                for (int h = 0; h < NHK; ++h)
-                    if (!rot && 64 * h + lane < DK) own_k[h] = krow[64 * h + lane];
+                for (int j = 0; j < UPW; ++j) {
+                    const int u = unit0 + j * WAVES;
 #pragma unroll
-                for (int h = 0; h < NHV; ++h)
-                    if (64 * h + lane < DV) {
-                        const uint32_t *p = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, 64 * h + lane)) + (bp >> 5);
-                        own_v[h] = vrow[64 * h + lane];
-                        own_w[h][0] = p[0];
+                    for (int e = 0; e < EU; ++e) {
+                        const int d = (u < NUK ? u : u - NUK) * UC + 64 * e + lane;
+                        if (u < NUK) {
+                            if (!rot && d < DK) row_e[j][e] = krow[d];
+                        } else if (u < NUK + NUV && d < DV) {
+                            row_e[j][e] = vrow[d];
+                            row_w[j][e][0] = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, d))[bp >> 5];
+                        }
                     }
+                }
                 if (second)  // (apart: an element widened in another block than its load's is waited for there)
 #pragma unroll
-                    for (int h = 0; h < NHV; ++h)
-                        if (64 * h + lane < DV) own_w[h][1] = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, 64 * h + lane))[(bp >> 5) + 1];
+                    for (int j = 0; j < UPW; ++j) {
+                        const int u = unit0 + j * WAVES;
+#pragma unroll
+                        for (int e = 0; e < EU; ++e) {
+                            const int d = (u - NUK) * UC + 64 * e + lane;
+                            if (u >= NUK && u < NUK + NUV && d < DV) row_w[j][e][1] = reinterpret_cast<const uint32_t *>(vcell + v_row_off(st, slot, d))[(bp >> 5) + 1];
+                        }
+                    }
             }
         }
     }
     auto write_row = [&]() __attribute__((always_inline)) {
-        const int slot = a.new_slot;
-        // (the elements' first use, and so the wait for them: as in the 4-row kernel)
-#pragma unroll
-        for (int h = 0; h < NHK; ++h)
-            if constexpr (!rot) asm("" : "+v"(own_k[h]));
-#pragma unroll
-        for (int h = 0; h < NHV; ++h) asm("" : "+v"(own_v[h]));
-        quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return rot ? Elem<DT>::load(rot_s, R * DK + d) : sb_scale<DT>(own_k[(d - lane) >> 6]); }, DK, GS, lane,
-            reinterpret_cast<uint32_t *>(const_cast<char *>(k_row_ptr(st, bh, slot))), [](int, uint32_t) {},
-            const_cast<char *>(ksb_row_ptr(st, bh, slot)), nullptr, nullptr);
-        char *vcell = const_cast<char *>(v_cell_ptr(st, bh, slot));
-        const int bp = v_bitpos<BITS>(slot & (TILE - 1)), sh = bp & 31;
+        const int slot = a.new_slot, bp = v_bitpos<BITS>(slot & (TILE - 1)), sh = bp & 31;
+        const size_t in_page = slot & (PAGE - 1);
         constexpr uint32_t M = (1u << BITS) - 1u;
-        quantize_row_wave_from<DT, BITS>(
-            [&](int d) { return sb_scale<DT>(own_v[(d - lane) >> 6]); }, DV, GS, lane, nullptr,
-            [&](int d, uint32_t code) {
-                uint32_t *p = reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d)) + (bp >> 5);
-                const uint32_t (&old)[2] = own_w[(d - lane) >> 6];
-                p[0] = (old[0] & ~(M << sh)) | (code << sh);
-                if ((32 % BITS) != 0 && sh + BITS > 32) p[1] = (old[1] & ~(M >> (32 - sh))) | (code >> (32 - sh));
-            },
-            const_cast<char *>(vsb_row_ptr(st, bh, slot)), nullptr, nullptr);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+#pragma unroll
+        for (int j = 0; j < UPW; ++j) {
+            // (the elements' first use, and so the wait for them: as in the 4-row kernel)
+#pragma unroll
+            for (int e = 0; e < EU; ++e) asm("" : "+v"(row_e[j][e]));
+            const int u = unit0 + j * WAVES, from = (u < NUK ? u : u - NUK) * UC;
+            if (u < NUK) {
+                quantize_row_wave_from<DT, BITS>(
+                    [&](int d) { return rot ? Elem<DT>::load(rot_s, R * DK + d) : sb_scale<DT>(row_e[j][EU == 1 ? 0 : (d - lane - from) >> 6]); }, min(from + UC, DK), GS, lane,
+                    reinterpret_cast<uint32_t *>(own_pk + (size_t)bh * st.k_cell + in_page * st.k_row), [](int, uint32_t) {},
+                    own_pks + (size_t)bh * st.ksb_cell + in_page * st.ksb_row, nullptr, nullptr, from);
+            } else if (u < NUK + NUV) {
+                char *vcell = own_pv + (size_t)bh * st.v_cell;
+                quantize_row_wave_from<DT, BITS>(
+                    [&](int d) { return sb_scale<DT>(row_e[j][EU == 1 ? 0 : (d - lane - from) >> 6]); }, min(from + UC, DV), GS, lane, nullptr,
+                    [&](int d, uint32_t code) {
+                        uint32_t *p = reinterpret_cast<uint32_t *>(vcell + v_row_off(st, slot, d)) + (bp >> 5);
+                        const uint32_t (&old)[2] = row_w[j][EU == 1 ? 0 : (d - lane - from) >> 6];
+                        p[0] = (old[0] & ~(M << sh)) | (code << sh);
+                        if ((32 % BITS) != 0 && sh + BITS > 32) p[1] = (old[1] & ~(M >> (32 - sh))) | (code >> (32 - sh));
+                    },
+                    own_pvs + (size_t)bh * st.vsb_cell + in_page * st.vsb_row, nullptr, nullptr, from);
+            }
+        }
     };
 
     // ---- per-lane addresses inside a tile; tiles of one wavefront are a page apart -----------
@@ -700,8 +715,11 @@ decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeAr
         __syncthreads();
     }
     if constexpr (MM == 0) {
-        if (own) write_row();
-        if (row_first) request_first();
+        if (row_here) {  // workgroup-uniform
+            write_row();
+            __syncthreads();
+            if (row_first) request_first();
+        }
     }
     if (my_tiles > 0) {
         load_queries();

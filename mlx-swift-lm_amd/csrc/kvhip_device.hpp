@@ -152,7 +152,8 @@ __device__ __forceinline__ uint32_t group_or(uint32_t v, int width) {
     return v;
 }
 
-// One wavefront quantizes one row of D elements (groupwise affine, MLX's CPU algorithm).
+// One wavefront quantizes elements `from` (a multiple of 64 and of the group size) to D of one row (groupwise affine, MLX's
+// CPU algorithm).
 // `load(d)` hands element d of the row as float; `code_sink(d, code)` receives every code.
 // Optional outputs:
 //   k_words   packed codes in MLX order (D*BITS/32 words)
@@ -161,12 +162,12 @@ __device__ __forceinline__ uint32_t group_or(uint32_t v, int width) {
 template <int DT, int BITS, class LOAD, class SINK>
 __device__ __forceinline__ void quantize_row_wave_from(LOAD load, int D, int gs, int lane,
                                                        uint32_t *k_words, SINK code_sink, void *sb_row,
-                                                       void *scales, void *biases) {
+                                                       void *scales, void *biases, int from = 0) {
     const float nb = (float)((1 << BITS) - 1);
     const int K = gs > 64 ? gs / 64 : 1;
     const int width = gs < 64 ? gs : 64;
     constexpr int per = 32 / BITS;
-    for (int base = 0; base < D; base += 64 * K) {
+    for (int base = from; base < D; base += 64 * K) {
         float w[2] = {0.f, 0.f};
         float mn = INFINITY, mx = -INFINITY;
         for (int k = 0; k < K; ++k) {

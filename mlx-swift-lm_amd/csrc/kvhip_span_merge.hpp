@@ -6,8 +6,6 @@
 
 namespace kvhip {
 
-typedef float kv_f4 __attribute__((ext_vector_type(4)));
-
 // The wavefronts' maxima, and behind a barrier their rows and sums, weighed by exp2(own maximum - row's maximum) as they
 // are written: what is left to do is to add them up.  (The weights formed by every thread that adds, an exponential per
 // wavefront and column, cost the last wavefront 1100 cycles behind its last tile at four rows of 64; now 600.)
@@ -23,41 +21,57 @@ template <int D, int NW, int RR> __device__ __forceinline__ float wave_weight(co
     return m == -INFINITY ? 0.f : fast_exp2((m - mx) * LOG2E);
 }
 // v / l, a thread's columns by one division and a correction each
-__device__ __forceinline__ kv_f4 normalised(kv_f4 v, float l) {
-    if (!(l > 0.f)) return kv_f4{0.f, 0.f, 0.f, 0.f};
+template <int N> __device__ __forceinline__ void normalise(float (&v)[N], float l) {
     const float r = 1.f / l;
-    kv_f4 q;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < N; ++k) {
         const float x = v[k] * r, y = __builtin_fmaf(__builtin_fmaf(-x, l, v[k]), r, x);
-        q[k] = __builtin_isfinite(x) ? y : x;
+        v[k] = !(l > 0.f) ? 0.f : __builtin_isfinite(x) ? y : x;
     }
-    return q;
 }
-// R rows, a thread to four columns of one: output rows row0 .. (`whole`), or partial `slot` of the workspace (RR rows of D
-// columns, maximum, sum).
+// N adjacent elements of an output row
+template <int DT, int N> __device__ __forceinline__ void store_columns(void *out, size_t i, const float (&v)[N]) {
+    uint16_t *p = static_cast<uint16_t *>(out) + i;
+    if constexpr (N == 1) {
+        Elem<DT>::store(p, 0, v[0]);
+    } else {
+        uint32_t w[N / 2];
+#pragma unroll
+        for (int k = 0; k < N / 2; ++k) w[k] = DT == 0 ? pk_h2(v[2 * k], v[2 * k + 1]) : pk_bf2(v[2 * k], v[2 * k + 1]);
+        if constexpr (N == 2) *reinterpret_cast<uint32_t *>(p) = w[0];
+        else *reinterpret_cast<kv_u2 *>(p) = kv_u2{w[0], w[1]};
+    }
+}
+template <int N> __device__ __forceinline__ void store_floats(float *p, const float (&v)[N]) {  // (8-byte aligned where N > 1)
+    if constexpr (N == 1) p[0] = v[0];
+#pragma unroll
+    for (int k = 0; k + 1 < N; k += 2) *reinterpret_cast<kv_f2 *>(p + k) = kv_f2{v[k], v[k + 1]};
+}
+// R rows, a thread to CPT columns of one (as few as leave no thread of a full workgroup without any): output rows row0 ..
+// (`whole`), or partial `slot` of the workspace (RR rows of D columns, maximum, sum).
 template <int D, int DT, int NW, int RR>
 __device__ __forceinline__ void leave_rows(const AttendArgs &a, const WaveParts<D, NW, RR> &parts, int R, bool whole, size_t row0, size_t slot) {
-    constexpr int LPR = D / 4, RPB = NW * 64 / LPR;
-    const int c = 4 * (threadIdx.x % LPR);
+    constexpr int EACH = RR * D / (NW * 64), CPT = EACH >= 4 ? 4 : EACH >= 2 ? 2 : 1;
+    constexpr int LPR = D / CPT, RPB = NW * 64 / LPR;
+    const int c = CPT * (threadIdx.x % LPR);
     if (RPB * LPR < NW * 64 && threadIdx.x >= RPB * LPR) return;  // (96 columns: lanes left over)
 #pragma unroll 1
     for (int i = threadIdx.x / LPR; i < R; i += RPB) {
-        kv_f4 v{0.f, 0.f, 0.f, 0.f};
-        float l = 0.f;
+        float v[CPT], l = 0.f;
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) v[k] = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            v += *reinterpret_cast<const kv_f4 *>(&parts.rows[w][i][c]);
+#pragma unroll
+            for (int k = 0; k < CPT; ++k) v[k] += parts.rows[w][i][c + k];
             l += parts.l[w][i];
         }
         if (whole) {
-            const kv_f4 o = normalised(v, l);
-            *reinterpret_cast<kv_u2 *>(static_cast<uint16_t *>(a.out) + (row0 + i) * D + c) =
-                DT == 0 ? kv_u2{pk_h2(o.x, o.y), pk_h2(o.z, o.w)} : kv_u2{pk_bf2(o.x, o.y), pk_bf2(o.z, o.w)};
+            normalise(v, l);
+            store_columns<DT>(a.out, (row0 + i) * D + c, v);
         } else {
             float *part = a.workspace + (slot * RR + i) * (D + 2);
-            *reinterpret_cast<kv_f2 *>(part + c) = kv_f2{v.x, v.y};
-            *reinterpret_cast<kv_f2 *>(part + c + 2) = kv_f2{v.z, v.w};
+            store_floats(part + c, v);
             if (c == 0) {
                 float mx = parts.m[0][i];
 #pragma unroll
