@@ -88,11 +88,16 @@ static int prefill_block_rows(const AttendArgs &a) {
     return prefill_wide(a) ? 128 : 64;
 }
 
+// Query rows per workgroup, key-range parts per query block, and whether a workgroup takes two parts at once.
+struct PrefillPlan {
+    int rows, parts;
+    bool halves;
+};
+
 // Key-range parts per query block: only when the grid would leave most CUs without a
 // second workgroup, and only while the partials stay small.
-static int prefill_splits(const AttendArgs &a) {
+static int prefill_splits(const AttendArgs &a, int bm) {
     const int R = (a.Hq / a.Hkv) * a.L;
-    const int bm = prefill_block_rows(a);
     if (a.st.bits != 0 && bm > 64) return 1;  // (chosen only when the grid fills the chip)
     const size_t wgs = (size_t)((R + bm - 1) / bm) * a.st.BH;
     // (few keys and a workgroup per CU: see prefill_wide; the quantized tile likewise -- a single sequence's 512 x 512
@@ -110,17 +115,30 @@ static int prefill_splits(const AttendArgs &a) {
     // single sequence, 32q/8kv, 5 new tokens: over 8192 keys 43 -> 18 us at 4 bits and 31 -> 15 us in float16, over
     // 32768 keys 152 -> 31 us and 97 -> 28 us; 32 new tokens over 32768 keys 154 -> 50 us and 97 -> 39 us)
     const int cap = (size_t)R * a.st.BH <= 4096 ? 64 : 8;  // (the many-part merge takes a workgroup per query row)
-    if (n > cap) n = cap;
-    if (n < 2) return 1;
-    const size_t per_part = (size_t)a.st.BH * R * (a.st.Dv + 2) * sizeof(float);
-    if (per_part * n > ((size_t)256 << 20)) return 1;
+    return n > cap ? cap : n;
+}
+
+static PrefillPlan prefill_plan(const AttendArgs &a) {
+    PrefillPlan p;
+    p.rows = prefill_block_rows(a);
+    int n = prefill_splits(a, p.rows);
+    // An even number of parts of 128-row workgroups: a workgroup of eight wavefronts takes two of them and adds them up in
+    // LDS, which halves the partials in memory and the merge that reads them.  The kernel itself gives nothing or 1 us
+    // (bfloat16 D 128 32q/8kv, 512 new rows: over 8192 keys 73.0 us in four parts of four wavefronts, 72.9 in two of
+    // eight; 4096 keys 41.8 / 41.2; 2048 keys 26.5 / 25.5), the merge behind it 3.5 us of 7.  Without parts it costs
+    // (2048 x 8192 239 -> 255 us: eight wavefronts wait for each other at a barrier), and an odd number would leave CUs idle.
+    p.halves = a.st.bits == 0 && p.rows == 128 && n > 1 && n % 2 == 0;
+    if (p.halves) n /= 2;
+    const size_t R = (size_t)(a.Hq / a.Hkv) * a.L, per_part = a.st.BH * R * (a.st.Dv + 2) * sizeof(float);
+    if (n < 2 || per_part * n > ((size_t)256 << 20)) n = 1;
     // a caller with a fixed amount of scratch: fewer parts until they fit (one part has no partials)
     while (a.workspace_cap && n > 1 && per_part * n > a.workspace_cap) --n;
-    return n;
+    p.parts = n;
+    return p;
 }
 
 size_t attend_prefill_workspace(const AttendArgs &a) {
-    const int n = prefill_splits(a);
+    const int n = prefill_plan(a).parts;
     if (n <= 1) return 0;
     return (size_t)a.st.BH * n * (a.Hq / a.Hkv) * a.L * (a.st.Dv + 2) * sizeof(float);
 }
@@ -128,20 +146,16 @@ size_t attend_prefill_workspace(const AttendArgs &a) {
 hipError_t launch_attend_prefill(const AttendArgs &a, hipStream_t s) {
     const Store &st = a.st;
     const int R = (a.Hq / a.Hkv) * a.L;
-    // 128 query rows per workgroup reuse each staged tile twice as often; 64 rows are used
-    // when that would leave the grid too small to fill 256 CUs twice over
-    const int bm = prefill_block_rows(a);
-    const bool wide = bm == 128;
-    const int nsplit = prefill_splits(a);
+    const PrefillPlan plan = prefill_plan(a);
+    const int nsplit = plan.parts;
     if (st.bits != 0) {
         profile_mark(s, true);
-        hipError_t e = launch_attend_prefill_q(a, nsplit, bm, s);
+        hipError_t e = launch_attend_prefill_q(a, nsplit, plan.rows, s);
         profile_mark(s, false);
         if (e != hipSuccess) return e;
     } else {
-        // full-precision caches have their own double-buffered kernel
         profile_mark(s, true);
-        hipError_t e = launch_attend_prefill_fp(a, nsplit, wide, s);
+        hipError_t e = plan.rows == 128 ? launch_attend_prefill_rows32(a, nsplit, plan.halves, s) : launch_attend_prefill_fp(a, nsplit, s);
         profile_mark(s, false);
         if (e != hipSuccess) return e;
     }

@@ -1,8 +1,8 @@
 // Chunked-prefill attention for full-precision caches (fp16 / bf16) on the matrix cores
 // (gfx950, v_mfma_f32_16x16x32_f16 / _bf16).
 //
-// One workgroup (4 wavefronts) owns 64 (QT = 1) or 128 (QT = 2) query rows of one
-// (batch, kv-head) pair and walks the cached keys in tiles of 32 slots:
+// One workgroup (4 wavefronts) owns 64 query rows of one (batch, kv-head) pair (grids of few rows, head size 256, keys of
+// 192 with values of 128; more rows of head sizes up to 128: kvhip_attend_prefill_rows32.hip) and walks the cached keys in tiles of 32 slots:
 //   S^T   = K . Q^T      A = K rows from LDS in the cache's own dtype (no conversion),
 //                        B = query rows held in registers
 //   out^T += V^T . P^T   A = V^T rows from LDS as fp16 (bf16 is converted while staging),
@@ -15,7 +15,7 @@
 // are padded so that both the writes and the operand reads are bank-conflict free.
 // The online softmax rescales the accumulators only when a row maximum rises, and key tiles
 // that every query row of the workgroup sees completely skip all mask tests.
-#include "kvhip_mask.hpp"
+#include "kvhip_prefill_fp.hpp"
 
 #ifndef KVHIP_PREFILL_LM
 #define KVHIP_PREFILL_LM 1
@@ -23,25 +23,15 @@
 #ifndef KVHIP_PREFILL_BF16_P
 #define KVHIP_PREFILL_BF16_P 1
 #endif
-// how far ahead of their use the matrix-core operands are read from LDS (registers permitting):
-// per query-block count (1: 16 query rows per wavefront, 2: 32)
-#ifndef KVHIP_PF_VG1
-#define KVHIP_PF_VG1 2
+// how far ahead of their use the matrix-core operands are read from LDS
+#ifndef KVHIP_PF_VG
+#define KVHIP_PF_VG 2
 #endif
-#ifndef KVHIP_PF_VG2
-#define KVHIP_PF_VG2 2
+#ifndef KVHIP_PF_NVB
+#define KVHIP_PF_NVB 2
 #endif
-#ifndef KVHIP_PF_NVB1
-#define KVHIP_PF_NVB1 2
-#endif
-#ifndef KVHIP_PF_NVB2
-#define KVHIP_PF_NVB2 2
-#endif
-#ifndef KVHIP_PF_AHEAD1
-#define KVHIP_PF_AHEAD1 2
-#endif
-#ifndef KVHIP_PF_AHEAD2
-#define KVHIP_PF_AHEAD2 1
+#ifndef KVHIP_PF_AHEAD
+#define KVHIP_PF_AHEAD 2
 #endif
 
 #ifndef KV_SB
@@ -51,47 +41,9 @@ namespace kvhip {
 
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) uint32_t LDS_U32;
+using namespace prefill_fp;
 
-// 16 bytes per lane from global memory straight into LDS: lane i's land at `lds_wave_base` + 16 i
-// (the base is the same for the whole wavefront).  Written as assembly, with the waits for it placed
-// by hand (s_waitcnt vmcnt): the compiler's own bookkeeping of such loads makes every LDS read that
-// follows one wait for all vector-memory operations in flight, register loads included, wherever it
-// cannot prove on every path which buffer the load fills.  Its waits for its own loads stay correct:
-// vector-memory operations complete in order, so an operation it does not count only makes a wait
-// stricter.
-// INVARIANT for anyone who edits this kernel: (1) an iteration ends with vmcnt(0) and a barrier before
-// any wavefront reads the buffer the loads fill, and every wavefront of the workgroup runs the same
-// iterations with the same requests (which variant of an iteration it runs may differ); (2)
-// vector-memory operations of one wavefront complete in order on this hardware -- the compiler's own
-// waits for register loads rely on that when an uncounted LDS load sits between them.
-// (address = wave-uniform 64-bit `base` in scalar registers + the lane's unsigned 32-bit byte offset)
-__device__ __forceinline__ void load_to_lds(const char *base, uint32_t lane_off, const void *lds_wave_base) {
-    // (the low half of a flat address inside the LDS aperture is the LDS address itself)
-    const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds_wave_base);
-    const uint64_t b = reinterpret_cast<uint64_t>(base);
-    // (readfirstlane returns a signed int: without the casts the low half would be sign-extended over the high one)
-    const uint32_t b_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    const uint32_t b_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-    const uint64_t sb = ((uint64_t)b_hi << 32) | (uint64_t)b_lo;
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(sb), "s"(lds) : "memory", "m0");
-}
-union Op8 {
-    h8 h;
-    b8 b;
-    u4 v;
-};
 
-constexpr int BN = 32;  // key slots per tile
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr float RAISE = 8.f;  // log2 units
-
-__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ uint32_t rn_h2(float lo, float hi) { return pk_h2(lo, hi); }    // round to nearest even
 __device__ __forceinline__ uint32_t rn_bf2(float lo, float hi) { return pk_bf2(lo, hi); }
 // the probabilities of one lane as the PV operand: fp16, or bf16 for bf16 caches on the direct path
@@ -103,8 +55,6 @@ template <bool BF> __device__ __forceinline__ u4 pack_p(const float (&p)[2][4]) 
 __device__ __forceinline__ uint32_t bf2_to_h2(uint32_t w) {
     return rn_h2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
 }
-
-__device__ __forceinline__ int st_BH(const AttendArgs &a) { return a.st.BH; }
 
 // c += a . b and c = a . b on the matrix cores.  DT: 0 fp16 operands, 1 bf16 operands.
 template <int DT> __device__ __forceinline__ void mfma_acc(f4 &c, const Op8 &a, const Op8 &b) {
@@ -129,9 +79,10 @@ template <int DT> __device__ __forceinline__ void mfma_new(f4 &c, const Op8 &a, 
 // into the buffer of its tile's parity; one barrier per iteration.
 // DK and DV are the head sizes of keys / queries and of values / outputs (192 and 128 for the multi-head
 // latent attention models, equal otherwise).
-template <int DK, int DV, int DT, bool IDENT, int QT, int MM>
+template <int DK, int DV, int DT, bool IDENT, int MM>
 __global__ void __launch_bounds__(256, 2)
 prefill_fp_kernel(AttendArgs a, int nsplit) {
+    constexpr int QT = 1;  // blocks of 16 query rows per wavefront
     constexpr int BM = 64 * QT;
     constexpr int S = (DK + 31) / 32;  // contraction steps over the head dim (the last one partly zero at D = 80)
     constexpr int NDT = DV / 16;   // 16-row tiles of out^T
@@ -157,44 +108,16 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     auto Vs = [&](int par) __attribute__((always_inline)) -> uint16_t * { return (par == 0 ? KV0 : KV1) + KSZ; };
     __shared__ int rows_s[2][BN];
     __shared__ int full_s[2];
-    __shared__ int seg_lo_s[MAXRUNS], seg_hi_s[MAXRUNS], nseg_s;  // tile segments to visit (ring presentations)
+    __shared__ VisitShared visit_s;
 
     const Store &st = a.st;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, jj = lane >> 4;
-    // Workgroups go to the 8 XCDs round-robin by linear id, and each XCD has its own L2.  All
-    // query blocks of one (batch, kv-head) pair re-read that pair's K and V, so they are given
-    // ids of the same residue: a pair's tiles then stay hot in one L2 instead of missing in all.
     const int r = a.Hq / a.Hkv;
     const int R = r * a.L;
-    const int nblk = (R + BM - 1) / BM;
-    int blk_x, bh, split;
-    {
-        const int id = blockIdx.x;
-        const int BH = st_BH(a);
-        if ((BH & 7) == 0) {
-            const int xcd = id & 7;
-            int j = id >> 3;
-            // A grid of exactly two workgroups per CU is resident all at once and gets no balancing from the
-            // order of the ids.  Under a causal or window mask the two workgroups of a CU -- 32 apart among the
-            // 64 of their XCD -- then take a long and a short query block: the second 32 count backwards.
-            if (MM == 1 && gridDim.x == 512 && (j & 32)) j = 95 - j;
-            const int per_pair = nblk * nsplit;
-            const int h_local = j / per_pair, rem = j - h_local * per_pair;
-            bh = h_local * 8 + xcd;
-            split = rem / nblk;
-            blk_x = rem - split * nblk;
-        } else {
-            blk_x = id % nblk;
-            const int t = id / nblk;
-            bh = t % BH;
-            split = t / BH;
-        }
-    }
-    // Under a causal or window mask the later query blocks see more keys: they are given the lower
-    // workgroup ids, which the hardware starts first, so that the launch does not end on its longest blocks.
-    if (MM == 1) blk_x = nblk - 1 - blk_x;
+    const WorkItem item = work_item<MM>(a, (R + BM - 1) / BM, nsplit);
+    const int blk_x = item.block, bh = item.bh;
     const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
     const int row0 = blk_x * BM + wave * 16 * QT;  // first query row of this wavefront
     const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
@@ -247,126 +170,10 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     }
 
     // ---- key tiles this workgroup has to visit, and the rows all of its queries keep ---------
-    int tile_lo = 0, tile_hi = (a.slots + BN - 1) / BN;
-    int keep_lo = 0, keep_hi = -1;
-    {
-        const int i_first = blk_x * BM, i_last = min(R, i_first + BM) - 1;
-        const bool spans = (i_first / a.L) != (i_last / a.L);
-        const int l_min = spans ? 0 : i_first % a.L, l_max = spans ? a.L - 1 : i_last % a.L;
-        if (MM != 2) {
-            keep_hi = a.T - 1;
-            if (MM == 1) {
-                if (sym.mode == KVHIP_MASK_CAUSAL) {
-                    keep_hi = a.T - a.L + l_min;
-                } else {
-                    keep_lo = sym.pad_b;
-                    keep_hi = min(sym.offset + l_min, sym.len_b - 1);
-                    if (sym.window > 0) keep_lo = max(keep_lo, sym.offset + l_max - sym.window + 1);
-                }
-                keep_hi = min(keep_hi, a.T - 1);
-            }
-        }
-        if (IDENT) {  // slots are presented rows: tiles outside a symbolic mask are skipped
-            if (a.mask.mode == KVHIP_MASK_CAUSAL) {
-                tile_hi = min(tile_hi, (a.T - a.L + l_max) / BN + 1);
-            } else if (a.mask.mode == KVHIP_MASK_WINDOW) {
-                tile_hi = min(tile_hi, (a.mask.offset + l_max) / BN + 1);
-                if (a.mask.window > 0) tile_lo = max(0, (a.mask.offset + l_min - a.mask.window + 1) / BN);
-            }
-            tile_hi = min(tile_hi, (a.T + BN - 1) / BN);
-        }
-    }
-    // The tiles to visit, in slot order, as up to NSEG segments; position v of the visiting order is tile
-    // vt_of(v).  With slots in presented order that is the one range found above.  A ring presented
-    // through a run table keeps its rows in rotated order, so the rows no query of this block can see
-    // (older than the window, newer than the block) lie somewhere inside the slot range: thread 0 maps
-    // the visible row range through every run to slot tiles, sorts and merges them (a few dozen scalar
-    // steps, once per workgroup), and whole tiles of invisible rows are never requested -- 14 of 144
-    // tiles for a 512-row chunk over a 4096-row window.
-    constexpr int NSEG = 4;
-    int seg_start[NSEG], seg_cnt[NSEG];
-#pragma unroll
-    for (int k = 0; k < NSEG; ++k) seg_start[k] = seg_cnt[k] = 0;
-    seg_start[0] = tile_lo;
-    seg_cnt[0] = max(tile_hi - tile_lo, 0);
-    if constexpr (!IDENT && MM == 1) {
-        if (tid == 0) {
-            const int i_first = blk_x * BM, i_last = min(R, i_first + BM) - 1;
-            const bool spans = (i_first / a.L) != (i_last / a.L);
-            const int l_min = spans ? 0 : i_first % a.L, l_max = spans ? a.L - 1 : i_last % a.L;
-            int vis_lo = 0, vis_hi = a.T - a.L + l_max;  // rows some query of the block may see
-            if (sym.mode != KVHIP_MASK_CAUSAL) {
-                vis_lo = sym.pad_b;
-                vis_hi = min(sym.offset + l_max, sym.len_b - 1);
-                if (sym.window > 0) vis_lo = max(vis_lo, sym.offset + l_min - sym.window + 1);
-            }
-            vis_lo = max(vis_lo, 0);
-            vis_hi = min(vis_hi, a.T - 1);
-            int ns = 0;
-#pragma unroll
-            for (int i = 0; i < MAXRUNS; ++i) {
-                if (i < a.runs.n) {
-                    const int r_lo = max(vis_lo, a.runs.row0[i]), r_hi = min(vis_hi, a.runs.row0[i] + a.runs.len[i] - 1);
-                    if (r_lo <= r_hi) {
-                        const int t_lo = (a.runs.phys0[i] + r_lo - a.runs.row0[i]) / BN;
-                        const int t_hi = (a.runs.phys0[i] + r_hi - a.runs.row0[i]) / BN;
-                        int pos = ns;  // insertion by first tile
-                        while (pos > 0 && seg_lo_s[pos - 1] > t_lo) {
-                            seg_lo_s[pos] = seg_lo_s[pos - 1];
-                            seg_hi_s[pos] = seg_hi_s[pos - 1];
-                            --pos;
-                        }
-                        seg_lo_s[pos] = t_lo;
-                        seg_hi_s[pos] = t_hi;
-                        ++ns;
-                    }
-                }
-            }
-            int m = 0;  // merge what overlaps or touches
-            for (int i = 0; i < ns; ++i) {
-                if (m > 0 && seg_lo_s[i] <= seg_hi_s[m - 1] + 1) {
-                    seg_hi_s[m - 1] = max(seg_hi_s[m - 1], seg_hi_s[i]);
-                } else {
-                    seg_lo_s[m] = seg_lo_s[i];
-                    seg_hi_s[m] = seg_hi_s[i];
-                    ++m;
-                }
-            }
-            if (m > NSEG) {  // more pieces than are kept: one range over all of them (nothing wrong, nothing skipped)
-                seg_hi_s[0] = seg_hi_s[m - 1];
-                m = 1;
-            }
-            nseg_s = m;
-        }
-        __syncthreads();
-        const int m = __builtin_amdgcn_readfirstlane(nseg_s);
-#pragma unroll
-        for (int k = 0; k < NSEG; ++k) {
-            const int lo = k < m ? __builtin_amdgcn_readfirstlane(seg_lo_s[k]) : 0;
-            const int hi = k < m ? __builtin_amdgcn_readfirstlane(seg_hi_s[k]) : -1;
-            seg_start[k] = lo;
-            seg_cnt[k] = hi - lo + 1;
-        }
-    }
-    auto vt_of = [&](int v) __attribute__((always_inline)) -> int {
-        int t = seg_start[0] + v, rem = v - seg_cnt[0];
-#pragma unroll
-        for (int k = 1; k < NSEG; ++k) {
-            if (rem >= 0) t = seg_start[k] + rem;
-            rem -= seg_cnt[k];
-        }
-        return t;
-    };
-    int v_lo = 0, v_hi = 0;
-#pragma unroll
-    for (int k = 0; k < NSEG; ++k) v_hi += seg_cnt[k];
-    // optional split of the visiting order (small grids): each part leaves an
-    // unnormalised partial per query row, merged by the decode path's combine kernel
-    if (nsplit > 1) {
-        const int span = (v_hi + nsplit - 1) / nsplit;
-        v_lo = split * span;
-        v_hi = min(v_hi, v_lo + span);
-    }
+    const Visit visit = visit_plan<BM, MM, IDENT>(a, sym, blk_x, R, item.split, nsplit, visit_s);
+    const int keep_lo = visit.keep_lo, keep_hi = visit.keep_hi;
+    auto vt_of = [&](int v) __attribute__((always_inline)) -> int { return visit.tile(v); };
+    const int v_lo = visit.lo, v_hi = visit.hi;
 
     // ---- requests -------------------------------------------------------------------------
     // direct global -> LDS: lane i of a wavefront's load lands at the wavefront's LDS base + 16 i, so
@@ -619,8 +426,8 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
             if (idx == NP - 1) round_pair(idx);
         };
         // V operands (16 columns each) are read in groups of VG, NVB - 1 groups ahead of their use
-        constexpr int VG = QT == 1 ? KVHIP_PF_VG1 : KVHIP_PF_VG2;
-        constexpr int NVB = QT == 1 ? KVHIP_PF_NVB1 : KVHIP_PF_NVB2;
+        constexpr int VG = KVHIP_PF_VG;
+        constexpr int NVB = KVHIP_PF_NVB;
         constexpr int NG = (NDT + VG - 1) / VG;
         Op8 va[NVB][VG];
         auto read_v = [&](int g, Op8 (&dst)[VG]) __attribute__((always_inline)) {
@@ -632,7 +439,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         if constexpr (HAS_NEXT) {
             constexpr int NM = 2 * S * QT;  // matrix-core instructions of the next tile's scores
             // K operands are asked for AHEAD contraction steps ahead, V's first group near the end
-            constexpr int AHEAD = QT == 1 ? KVHIP_PF_AHEAD1 : KVHIP_PF_AHEAD2;
+            constexpr int AHEAD = KVHIP_PF_AHEAD;
             constexpr int KA = S < AHEAD + 1 ? S : AHEAD + 1;
             Op8 ka[KA][2];
 #pragma unroll
@@ -786,7 +593,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         if (!q_ok[qt]) continue;
         if (nsplit > 1) {
             const int i = row0 + 16 * qt + n;
-            float *part = a.workspace + (((size_t)bh * nsplit + split) * R + i) * (DV + 2);
+            float *part = a.workspace + (((size_t)bh * nsplit + item.split) * R + i) * (DV + 2);
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f4 *>(part + 16 * dt + 4 * jj) = oacc[qt][dt];
             if (jj == 0) {
@@ -816,49 +623,37 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
 
 }  // namespace
 
-hipError_t launch_attend_prefill_fp(const AttendArgs &a, int nsplit, bool wide, hipStream_t s) {
+hipError_t launch_attend_prefill_fp(const AttendArgs &a, int nsplit, hipStream_t s) {
     const Store &st = a.st;
     const int R = (a.Hq / a.Hkv) * a.L;
-    const int bm = wide ? 128 : 64;
+    const int bm = 64;
     dim3 grid((unsigned)((R + bm - 1) / bm) * st.BH * nsplit), block(256);  // linear: the kernel maps ids to tiles
     const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
     const int mm = a.mask.mode == KVHIP_MASK_NONE ? 0 : (a.mask.mode == KVHIP_MASK_ARRAY ? 2 : 1);
-#define PF_M(DK, DV, DT, QT, MM)                                                                                   \
-    do {                                                                                                      \
-        if (ident) hipLaunchKernelGGL((prefill_fp_kernel<DK, DV, DT, true, QT, MM>), grid, block, 0, s, a, nsplit);  \
-        else hipLaunchKernelGGL((prefill_fp_kernel<DK, DV, DT, false, QT, MM>), grid, block, 0, s, a, nsplit);       \
+#define PF_M(DK, DV, DT, MM)                                                                                              \
+    do {                                                                                                                  \
+        if (ident) hipLaunchKernelGGL((prefill_fp_kernel<DK, DV, DT, true, MM>), grid, block, 0, s, a, nsplit);          \
+        else hipLaunchKernelGGL((prefill_fp_kernel<DK, DV, DT, false, MM>), grid, block, 0, s, a, nsplit);               \
     } while (0)
-#define PF2(DK, DV, DT, QT)                        \
-    do {                                     \
-        if (mm == 0) PF_M(DK, DV, DT, QT, 0);     \
-        else if (mm == 1) PF_M(DK, DV, DT, QT, 1); \
-        else PF_M(DK, DV, DT, QT, 2);             \
+#define PF(DK, DV, DT)                        \
+    do {                                      \
+        if (mm == 0) PF_M(DK, DV, DT, 0);     \
+        else if (mm == 1) PF_M(DK, DV, DT, 1); \
+        else PF_M(DK, DV, DT, 2);             \
     } while (0)
-#define PF(D, DT, QT) PF2(D, D, DT, QT)
-#define PF_QT(D, DT)                 \
-    do {                             \
-        if (wide) PF(D, DT, 2);      \
-        else PF(D, DT, 1);           \
+#define PF_DT(DK, DV)                              \
+    do {                                           \
+        if (st.dtype == KVHIP_F16) PF(DK, DV, 0);  \
+        else PF(DK, DV, 1);                        \
     } while (0)
-#define PF_DT(D)                                  \
-    do {                                          \
-        if (st.dtype == KVHIP_F16) PF_QT(D, 0);   \
-        else PF_QT(D, 1);                         \
-    } while (0)
-    // keys of 192 with values of 128 (multi-head latent attention): 64 query rows per workgroup
-    if (st.Dk == 192 && st.Dv == 128) {
-        if (st.dtype == KVHIP_F16) PF2(192, 128, 0, 1);
-        else PF2(192, 128, 1, 1);
-    } else if (st.Dk == 64) PF_DT(64);
-    else if (st.Dk == 80) PF_DT(80);
-    else if (st.Dk == 96) PF_DT(96);
-    else if (st.Dk == 128) PF_DT(128);
-    else if (st.dtype == KVHIP_F16) PF(256, 0, 1);
-    else PF(256, 1, 1);
+    if (st.Dk == 192 && st.Dv == 128) PF_DT(192, 128);  // (multi-head latent attention)
+    else if (st.Dk == 64) PF_DT(64, 64);
+    else if (st.Dk == 80) PF_DT(80, 80);
+    else if (st.Dk == 96) PF_DT(96, 96);
+    else if (st.Dk == 128) PF_DT(128, 128);
+    else PF_DT(256, 256);
 #undef PF_DT
-#undef PF_QT
 #undef PF
-#undef PF2
 #undef PF_M
     return hipGetLastError();
 }

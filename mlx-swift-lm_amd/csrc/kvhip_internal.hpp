@@ -398,7 +398,8 @@ hipError_t launch_attend_decode16(const AttendArgs &a, int tiles_total, int tile
 hipError_t launch_attend_decode16_low(const AttendArgs &a, int tiles_total, int tiles_per_wg, int nsplit, hipStream_t s);
 hipError_t launch_attend_decode16_high(const AttendArgs &a, int tiles_total, int tiles_per_wg, int nsplit, hipStream_t s);
 bool decode16_stream_shape(const Store &s);
-hipError_t launch_attend_prefill_fp(const AttendArgs &a, int nsplit, bool wide, hipStream_t s);
+hipError_t launch_attend_prefill_rows32(const AttendArgs &a, int nsplit, bool halves, hipStream_t s);
+hipError_t launch_attend_prefill_fp(const AttendArgs &a, int nsplit, hipStream_t s);
 // The pipelined tile for quantized caches (head sizes 64 / 128 / 256, slots in presented order).
 bool attend_prefill_q_supported(const AttendArgs &a);
 // rows: query rows per workgroup, 64 (4 wavefronts) or 256 (8 wavefronts; head size 128)
