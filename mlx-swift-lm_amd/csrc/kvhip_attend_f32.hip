@@ -44,7 +44,7 @@ constexpr int query_tiles(int dk) { return dk <= 128 ? 2 : 1; }
 // TB: token blocks of 16 per tile.
 template <int DK, int DV, int QT, int TB, int ARR, bool ROT>
 __global__ void __launch_bounds__(256, 2)
-attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int nparts) {
+attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_total, int nparts) {
     constexpr int WT = 16 * TB;
     constexpr int NS = DK / 16, NCT = DV / 16;
     extern __shared__ __align__(16) float smem[];
@@ -56,17 +56,13 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
     const Store &st = a.st;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, g = lane >> 4;
-    // (the row blocks of one kv head and part run on one XCD and share its L2: see attend_valu_kernel)
-    int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int total = gridDim.x * gridDim.y * gridDim.z;
-    if (gridDim.x > 1 && (total & 7) == 0) lin = (lin & 7) * (total >> 3) + (lin >> 3);
-    const int bh = (lin / gridDim.x) % gridDim.y, part = lin / (gridDim.x * gridDim.y);
-    const int b = bh / a.Hkv, h = bh % a.Hkv;
-    const int r = a.Hq / a.Hkv, R = r * a.L;
-    const int row0 = (lin % gridDim.x) * 16 * QT, row1 = min(row0 + 16 * QT, R) - 1;
+    const RowBlock rb(a);
+    const int bh = rb.bh, part = rb.part, b = rb.b, h = rb.h;
+    const int R = r * a.L;
+    const int row0 = rb.block * 16 * QT, row1 = min(row0 + 16 * QT, R) - 1;
 
-    const bool one_head = row0 / a.L == row1 / a.L;
-    const KeyRange keys = visible_keys(a.mask, b, a.L, a.T, one_head ? row0 % a.L : 0, one_head ? row1 % a.L : a.L - 1);
+    const bool one_head = rb.head(row0) == rb.head(row1);
+    const KeyRange keys = visible_keys(a.mask, b, a.L, a.T, one_head ? rb.pos(row0) : 0, one_head ? rb.pos(row1) : a.L - 1);
     const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
     int t_lo = 0, t_hi = tiles_total;
     if (ident) {
@@ -78,6 +74,9 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
 
     // ---- a step's rows ----------------------------------------------------------------------------------------
     constexpr bool STEP = QT == 1 && ARR == 0;  // (up to 16 query rows: one row block)
+    // (behind a wavefront's last tile, often a step's only one, the tile is not requested again; long loops keep their requests
+    // in front of no branch)
+    constexpr bool BRANCH = STEP && !QL;
     float *rot_s = smem + (QL ? NS * 256 : 0);  // [R + 1][DK] behind the query operands, under what the accumulators take at the end
     static_assert((QL ? NS * 256 : 0) + 17 * DK <= MW * NCT * 256, "room for sixteen query rows and the key row");
     [[maybe_unused]] RopeStep<2, DK, 256, 16> step;
@@ -97,23 +96,23 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
             for (int c = 0; c < NCT; ++c) own_v[c] = ld_global<float>(as_global(a.new_v) + ((size_t)bh * DV + 16 * c + col) * 4);
         }
     }
-    auto write_row = [&]() __attribute__((always_inline)) {
-        const int slot = a.new_slot;
-        char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot)), *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
+    auto write_row = [&](const PageEntry &page) __attribute__((always_inline)) {
         if constexpr (ROT) {
 #pragma unroll
             for (int s = 0; s < NS; ++s) own_k[s] = *reinterpret_cast<const f4 *>(rot_s + R * DK + 16 * s + 4 * g);
         }
+        // (global stores, and offsets as kfp_off and vfp_off give them for four-byte elements: see attend_wide_kernel)
+        const int t = a.new_slot & (PAGE - 1), tk = t & (TILE - 1);
+        KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell) + (t >> 6) * (TILE * DK * 4) + (g * TILE + tk) * 16;
+        KV_GLOBAL char *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell) + (t >> 6) * (TILE * DV * 4) + ((tk >> 2) * DV + col) * 16 + (tk & 3) * 4;
         if (col == 0) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) *reinterpret_cast<f4 *>(kc + kfp_off(st, slot, 16 * s + 4 * g)) = own_k[s];
+            for (int s = 0; s < NS; ++s) *reinterpret_cast<KV_GLOBAL f4 *>(kc + s * (4 * TILE * 16)) = own_k[s];
         }
         if (g == 0) {
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) *reinterpret_cast<float *>(vc + vfp_off(st, slot, 16 * c + col)) = own_v[c];
+            for (int c = 0; c < NCT; ++c) *reinterpret_cast<KV_GLOBAL float *>(vc + c * (16 * 16)) = own_v[c];
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
 
     // rows beyond the last: the last again, which nobody keeps
@@ -122,8 +121,8 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const int rr = min(row0 + 16 * qt + col, R - 1);
-        my_hq[qt] = h * r + rr / a.L;
-        my_l[qt] = rr % a.L;
+        my_hq[qt] = h * r + rb.head(rr);
+        my_l[qt] = rb.pos(rr);
         gptr qp = as_global(a.q) + (((size_t)(b * a.Hq + my_hq[qt]) * a.L + my_l[qt]) * DK + 4 * g) * 4;
 #pragma unroll
         for (int s = 0; s < (QL || ROT ? 0 : NS); ++s) qop[qt][s] = ld_global<f4>(qp + s * 64);
@@ -259,8 +258,12 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
     }
     if constexpr (STEP) {
         if (own) {
-            write_row();
-            if (a.new_slot / WT == first) {
+            PageCursor page = kpage;
+            write_row(page.at(st, a.new_slot));
+            if (a.new_slot / WT != first) {  // the row's tile is still to be read
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            } else {
                 const int tn = a.new_slot % WT;
 #pragma unroll
                 for (int x = 0; x < TB; ++x) {
@@ -304,7 +307,7 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
             if constexpr (QL) __builtin_amdgcn_sched_barrier(0);  // (one step's queries ahead, not all of them: registers)
         }
         if constexpr (bools) next = seen_from(next, next_bits);
-        load_k(next < te ? next : t);
+        if (!BRANCH || next < te) load_k(next < te ? next : t);
         const int slot0 = t * WT;
         const bool whole = ARR == 2 && run_row(a.runs, slot0, WT) >= 0;  // wave-uniform
         const bool full = ident && slot0 >= keys.full_lo && slot0 + WT - 1 <= keys.full_hi;  // wave-uniform
@@ -326,6 +329,16 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
 #pragma unroll
                         for (int j = 0; j < 4; ++j) s[qt][x][j] += add[j];
                     }
+                }
+            } else if (ARR == 0 && rb.one && ident) {  // one token: every row sees keys.lo to keys.hi
+                if (!full) {
+#pragma unroll
+                    for (int x = 0; x < TB; ++x)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int row = slot0 + 16 * x + 4 * g + j;
+                            s[qt][x][j] = row >= keys.lo && row <= keys.hi ? s[qt][x][j] : -INFINITY;
+                        }
                 }
             } else if (!full) {
 #pragma unroll
@@ -378,7 +391,7 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int
 #pragma unroll
                     for (int qt = 0; qt < QT; ++qt) acc[qt][c] = mfma4(vreg[x][c][j], s[qt][x][j], acc[qt][c]);
         if (ARR && next + (bools ? MW : 0) < te) mask_fetch(next + (bools ? MW : 0));
-        load_v(next < te ? next : t);
+        if (!BRANCH || next < te) load_v(next < te ? next : t);
         t = next;
         bits = next_bits;
     }
@@ -465,13 +478,13 @@ hipError_t launch_instance(const AttendArgs &a, const PlanF32 &p, hipStream_t s)
     const size_t lds = MW * QT * (DV / 16) * 64 * sizeof(f4);
     if constexpr (QT == 1) {
         if (a.new_k && a.rope) {
-            hipLaunchKernelGGL((attend_f32_kernel<DK, DV, 1, TB, 0, true>), grid, block, lds, s, AttendStepArgs(a), p.tiles, p.nparts);
+            hipLaunchKernelGGL((attend_f32_kernel<DK, DV, 1, TB, 0, true>), grid, block, lds, s, AttendStepArgs(a), a.Hq / a.Hkv, p.tiles, p.nparts);
             return hipGetLastError();
         }
     }
-    if (a.mask.mode != KVHIP_MASK_ARRAY) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 0, false>), grid, block, lds, s, a, p.tiles, p.nparts);
-    else if (a.mask.dtype == KVHIP_BOOL) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 1, false>), grid, block, lds, s, a, p.tiles, p.nparts);
-    else hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 2, false>), grid, block, lds, s, a, p.tiles, p.nparts);
+    if (a.mask.mode != KVHIP_MASK_ARRAY) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 0, false>), grid, block, lds, s, a, a.Hq / a.Hkv, p.tiles, p.nparts);
+    else if (a.mask.dtype == KVHIP_BOOL) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 1, false>), grid, block, lds, s, a, a.Hq / a.Hkv, p.tiles, p.nparts);
+    else hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 2, false>), grid, block, lds, s, a, a.Hq / a.Hkv, p.tiles, p.nparts);
     return hipGetLastError();
 }
 

@@ -20,7 +20,7 @@
 // Two rows of query tiles at most: the accumulators of four leave one wavefront per SIMD and are copied between the two
 // register files every tile (512 rows x 2048 keys, 8 query and 2 kv heads, bfloat16: 69 us the call, against 57 us).
 // Decode is bound by HBM where the batch fills the chip (B8, 4096 keys, one token: 26.5 us, 5.1 TB/s)
-// and by launch, one pass of loads and the merge below that (one sequence of 2048 keys, the kernel 10.4 us with the rotation
+// and by launch, one pass of loads and the merge below that (one sequence of 2064 keys, the kernel 8.2 us with the rotation
 // and the row's write, the merge 3.7; 63 us on the vector ALUs); a prompt chunk by the latency of the two barriers per tile
 // (512 x 2048, 33 us on average over a prompt's chunks and 7.4 us for the merge; 263 us).
 // K rows are loaded in the token order that leaves lane group g of the scores with tokens 8 g .. 8 g + 7, which is the
@@ -75,12 +75,11 @@ constexpr int SEEN = 4096;     // tiles of a part that a boolean mask is looked 
 // additive mask 193; 275, 276 and 262 with the elements fetched one by one behind the keys and every tile read, 198, 66
 // and 193 on the vector-ALU kernel.
 // A single-token step without a mask: the workgroup whose part holds the new row's tile writes the row, each wavefront
-// its quarter, after its first tile has been requested -- and if that is the row's tile, puts the row into its registers
-// too --, and ROT turns the query rows and the new key row in LDS first, as the decode kernels do.  A launch that appends
-// takes 5.2 us.
+// its quarter.  If that tile is its first, as in the steps of a single sequence, the row goes into the tile's registers too.  ROT
+// turns the query rows and the new key row in LDS first, as the decode kernels do.  A launch that appends takes 5.2 us.
 template <int DT, int QT, int ARR, bool ROT>
 __global__ void __launch_bounds__(256, 2)
-attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, int nparts) {
+attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_total, int nparts) {
     constexpr int NB = QT == 1 ? 2 : 1;           // score buffers (QT = 1 has one barrier per tile)
     __shared__ f4 part_s[NB][WW][QT][2][64];      // partial scores of the wavefronts
     __shared__ kv_u4 prob_s[QT == 1 ? 1 : QT][2][64];
@@ -92,18 +91,14 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
     const Store &st = a.st;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, g = lane >> 4;
-    // (the row blocks of one kv head and part run on one XCD and share its L2: see attend_valu_kernel)
-    int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int total = gridDim.x * gridDim.y * gridDim.z;
-    if (gridDim.x > 1 && (total & 7) == 0) lin = (lin & 7) * (total >> 3) + (lin >> 3);
-    const int bh = (lin / gridDim.x) % gridDim.y, part = lin / (gridDim.x * gridDim.y);
-    const int b = bh / a.Hkv, h = bh % a.Hkv;
-    const int r = a.Hq / a.Hkv, R = r * a.L;
-    const int row0 = (lin % gridDim.x) * 16 * QT, row1 = min(row0 + 16 * QT, R) - 1;
+    const RowBlock rb(a);
+    const int bh = rb.bh, part = rb.part, b = rb.b, h = rb.h;
+    const int R = r * a.L;
+    const int row0 = rb.block * 16 * QT, row1 = min(row0 + 16 * QT, R) - 1;
 
     // ---- the keys this row block sees ---------------------------------------------------------------
-    const bool one_head = row0 / a.L == row1 / a.L;
-    const KeyRange keys = visible_keys(a.mask, b, a.L, a.T, one_head ? row0 % a.L : 0, one_head ? row1 % a.L : a.L - 1);
+    const bool one_head = rb.head(row0) == rb.head(row1);
+    const KeyRange keys = visible_keys(a.mask, b, a.L, a.T, one_head ? rb.pos(row0) : 0, one_head ? rb.pos(row1) : a.L - 1);
     const bool ident = a.runs.n == 1 && a.runs.row0[0] == 0 && a.runs.phys0[0] == 0;
     int t_lo = 0, t_hi = tiles_total;
     if (ident) {
@@ -131,21 +126,22 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
             for (int c = 0; c < NCT; ++c) own_v[c] = ld_global<uint16_t>(as_global(a.new_v) + ((size_t)bh * WD + wave * (WD / WW) + 16 * c + col) * 2);
         }
     }
-    auto write_row = [&]() __attribute__((always_inline)) {
-        const int slot = a.new_slot, c0 = wave * (WD / WW);
-        char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot)), *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
-        if constexpr (ROT) {
-#pragma unroll
-            for (int s = 0; s < NS; ++s) own_k[s] = *reinterpret_cast<const kv_u4 *>(rot_s + R * WD + c0 + 8 * g + 32 * s);
-        }
+    auto write_row = [&](const PageEntry &page) __attribute__((always_inline)) {
+        // (global stores: behind one to a plain pointer every load in flight is waited for.  Offsets as kfp_off and vfp_off
+        // give them for two-byte elements, whose divisions by the element size take a microsecond here)
+        const int t = a.new_slot & (PAGE - 1), tk = t & (TILE - 1), c0 = wave * (WD / WW);
+        KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell) + (t >> 6) * (TILE * WD * 2) + ((c0 / 8 + g) * TILE + tk) * 16;
+        KV_GLOBAL char *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell) + (t >> 6) * (TILE * WD * 2) + ((tk >> 3) * WD + c0 + col) * 16 + (tk & 7) * 2;
         if (col == 0) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) *reinterpret_cast<kv_u4 *>(kc + kfp_off(st, slot, c0 + 8 * g + 32 * s)) = own_k[s];
+            for (int s = 0; s < NS; ++s) *reinterpret_cast<KV_GLOBAL kv_u4 *>(kc + s * (4 * TILE * 16)) = own_k[s];
         }
         if (g == 0) {
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, c0 + 16 * c + col)) = own_v[c];
+            for (int c = 0; c < NCT; ++c) *reinterpret_cast<KV_GLOBAL uint16_t *>(vc + c * (16 * 16)) = own_v[c];
         }
+    };
+    auto row_written = []() __attribute__((always_inline)) {  // (a wavefront reads the quarter that it wrote)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
@@ -155,7 +151,7 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
 #pragma unroll
     for (int qt = 0; qt < (ROT ? 0 : QT); ++qt) {
         const int rr = min(row0 + 16 * qt + col, R - 1);  // rows beyond the last: the last again, which nobody keeps
-        gptr qp = as_global(a.q) + (((size_t)(b * a.Hq + h * r + rr / a.L) * a.L + rr % a.L) * WD + wave * (WD / WW) + 8 * g) * 2;
+        gptr qp = as_global(a.q) + (((size_t)(b * a.Hq + h * r + rb.head(rr)) * a.L + rb.pos(rr)) * WD + wave * (WD / WW) + 8 * g) * 2;
 #pragma unroll
         for (int s = 0; s < NS; ++s) qop[qt][s] = ld_global<kv_u4>(qp + s * 64);
     }
@@ -184,7 +180,7 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
     f4 acc[QT][NCT];
     const int own = QT == 1 ? 0 : wave & 1;  // the query rows whose softmax this wavefront works out
     const int my = row0 + 16 * own + col;
-    const int my_hq = h * r + min(my, R - 1) / a.L, my_l = min(my, R - 1) % a.L;
+    const int my_hq = h * r + rb.head(min(my, R - 1)), my_l = rb.pos(min(my, R - 1));
     float m_run, l_run;
     constexpr float P_UP = DT == 0 ? 10.f : 0.f;  // (float16 probabilities are carried times 2^10)
 
@@ -268,6 +264,15 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
 #pragma unroll
                 for (int j = 0; j < 8; ++j) sc[j] += add[j];
             }
+        } else if (ARR == 0 && rb.one && ident) {  // one token: every row sees keys.lo to keys.hi
+            // (evaluated key by key as below, the tile at the edge, a step's last, took 2.5 us longer than the others)
+            if (slot0 < keys.lo || slot0 + WT - 1 > keys.hi) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int row = slot0 + 8 * g + j;
+                    sc[j] = row >= keys.lo && row <= keys.hi ? sc[j] : -INFINITY;
+                }
+            }
         } else if (!ident || slot0 < keys.full_lo || slot0 + WT - 1 > keys.full_hi) {  // workgroup-uniform
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -327,7 +332,7 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
             load_v(t);
         }
         while (t < te) {
-            const int next = seen_from(t + 1), load = next < te ? next : t;
+            const int next = seen_from(t + 1);
             if constexpr (ARR != 0) mask_fetch(t);
             f4 sacc[QT][2];
 #pragma unroll
@@ -338,7 +343,7 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
                 for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
                     for (int x = 0; x < 2; ++x) sacc[qt][x] = mfma<DT>(kreg[s][x], qop[qt][s], sacc[qt][x]);
-            load_k(load);
+            if (next < te) load_k(next);  // (behind the last tile, often a step's only one, nothing)
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
@@ -371,7 +376,7 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
 #pragma unroll
                 for (int c = 0; c < NCT; ++c) acc[qt][c] = mfma<DT>(decltype(careful)::value ? finite_only<DT>(vreg[c]) : vreg[c], pl, acc[qt][c]);
             }
-            load_v(load);
+            if (next < te) load_v(next);
             t = next;
             buf ^= NB - 1;
         }
@@ -405,8 +410,17 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
             for (int s = 0; s < NS; ++s) qop[0][s] = *reinterpret_cast<const kv_u4 *>(qr + 32 * s);
         }
         if (owner) {
-            write_row();
-            if (a.new_slot / WT == tb) {
+            if constexpr (ROT) {
+#pragma unroll
+                for (int s = 0; s < NS; ++s) own_k[s] = *reinterpret_cast<const kv_u4 *>(rot_s + R * WD + wave * (WD / WW) + 8 * g + 32 * s);
+            }
+            PageCursor page = kpage;
+            write_row(page.at(st, a.new_slot));
+            // (only a tile that is still to be read has to wait for the row: behind a fence and with the page looked up again
+            // a step's last workgroup ended 3 us behind the others)
+            if (a.new_slot / WT != tb) {
+                row_written();
+            } else {
                 const int tn = a.new_slot & (WT - 1);  // token 8 (c / 4) + 4 x + c % 4 is operand row c of block x
                 const bool mine = col == 4 * (tn >> 3) + (tn & 3);
 #pragma unroll
@@ -424,7 +438,9 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
             }
         }
     }
-    if (__builtin_expect(walk(std::false_type()), 0)) {
+    const bool again = walk(std::false_type());
+    if (__builtin_expect(again, 0)) {
+        if (owner) row_written();
         __syncthreads();
         walk(std::true_type());
     }
@@ -436,7 +452,7 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int tiles_total, in
         const float l = sum_s[qt][col];
         if (nparts == 1) {
             const float inv = l > 0.f ? 1.f / l : 0.f;
-            uint16_t *dst = reinterpret_cast<uint16_t *>(a.out) + ((size_t)(b * a.Hq + h * r + rr / a.L) * a.L + rr % a.L) * WD + wave * (WD / WW) + 4 * g;
+            uint16_t *dst = reinterpret_cast<uint16_t *>(a.out) + ((size_t)(b * a.Hq + h * r + rb.head(rr)) * a.L + rb.pos(rr)) * WD + wave * (WD / WW) + 4 * g;
 #pragma unroll
             for (int c = 0; c < NCT; ++c) {
                 const f4 v = acc[qt][c] * inv;
@@ -475,7 +491,7 @@ PlanWide plan_wide(const AttendArgs &a) {
     static const int target = measure_knob("KVHIP_WIDE_TARGET", 256), target2 = measure_knob("KVHIP_WIDE_TARGET2", 512), least = measure_knob("KVHIP_WIDE_LEAST", 1);  // (timing builds only)
     const long wgs = (long)p.row_blocks * a.st.BH;
     int n = p.qt == 1 && p.tiles <= 3 ? 1 : (int)std::max(1L, std::min<long>((p.qt == 1 ? target : target2) / std::max(1L, wgs), p.tiles / (p.qt == 1 ? least : 4)));
-    n = std::min(n, 64);
+    n = std::min(n, p.qt == 1 ? 128 : 64);
     const size_t per_part = (size_t)a.st.BH * R * (a.st.Dv + 2) * sizeof(float);
     while (n > 1 && a.workspace_cap && per_part * n > a.workspace_cap) --n;
     p.nparts = n;
@@ -499,11 +515,11 @@ hipError_t launch_attend_wide(const AttendArgs &a, hipStream_t s) {
     const dim3 grid(p.row_blocks, a.st.BH, p.nparts), block(256);
     profile_mark(s, true);
     const int arr = a.mask.mode != KVHIP_MASK_ARRAY ? 0 : a.mask.dtype == KVHIP_BOOL ? 1 : 2;
-#define WIDE_A(DT, QT, ARR) hipLaunchKernelGGL((attend_wide_kernel<DT, QT, ARR, false>), grid, block, 0, s, a, p.tiles, p.nparts)
+#define WIDE_A(DT, QT, ARR) hipLaunchKernelGGL((attend_wide_kernel<DT, QT, ARR, false>), grid, block, 0, s, a, a.Hq / a.Hkv, p.tiles, p.nparts)
 #define WIDE(DT, QT)                       \
     do {                                   \
         if (QT == 1 && a.new_k && a.rope)  \
-            hipLaunchKernelGGL((attend_wide_kernel<DT, 1, 0, true>), grid, block, 0, s, AttendStepArgs(a), p.tiles, p.nparts); \
+            hipLaunchKernelGGL((attend_wide_kernel<DT, 1, 0, true>), grid, block, 0, s, AttendStepArgs(a), a.Hq / a.Hkv, p.tiles, p.nparts); \
         else if (arr == 0) WIDE_A(DT, QT, 0); \
         else if (arr == 1) WIDE_A(DT, QT, 1); \
         else WIDE_A(DT, QT, 2);            \

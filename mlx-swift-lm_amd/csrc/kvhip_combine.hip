@@ -196,7 +196,7 @@ hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t
     if (a.st.Dv == 96) return merge_dtype<96, 96>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 128) return merge_dtype<128, 128>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 256) return merge_dtype<256, 128>(a, nsplit, rows, spans, s);
-    if (a.st.Dv == 512) return merge_dtype<512, 64>(a, nsplit, rows, spans, s);
+    if (a.st.Dv == 512) return merge_dtype<512, 32>(a, nsplit, rows, spans, s);
     return hipErrorInvalidValue;
 }
 

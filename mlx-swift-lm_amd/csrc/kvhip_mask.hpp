@@ -181,6 +181,31 @@ __device__ __forceinline__ KeyRange visible_keys(const MaskDev &m, int b, int L,
     return k;
 }
 
+// The workgroup of a grid (row blocks, BH, parts): its row block, pair and part, and which head and position a query row is.
+// No division where a step needs none: a dozen of them stood between a step's start and its first request (1.5 us of the
+// 2.7 of a step of head size 512).
+struct RowBlock {
+    int block, bh, part, b, h;
+    int L;
+    bool one;  // one new token: a row is a head
+    __device__ __forceinline__ RowBlock(const AttendArgs &a) : block(0), bh(blockIdx.y), part(blockIdx.z), L(a.L), one(a.L == 1) {
+        if (gridDim.x > 1) {
+            // (the row blocks of one kv head and part run on one XCD and share its L2: see attend_valu_kernel)
+            int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+            const int total = gridDim.x * gridDim.y * gridDim.z;
+            if ((total & 7) == 0) lin = (lin & 7) * (total >> 3) + (lin >> 3);
+            const int rest = lin / gridDim.x;
+            block = lin - rest * gridDim.x;
+            part = rest / gridDim.y;
+            bh = rest - part * gridDim.y;
+        }
+        b = a.B == 1 ? 0 : bh / a.Hkv;
+        h = bh - b * a.Hkv;
+    }
+    __device__ __forceinline__ int head(int row) const { return one ? row : row / L; }
+    __device__ __forceinline__ int pos(int row) const { return one ? 0 : row % L; }
+};
+
 // ---- the spans of a ragged batch -----------------------------------------------------------------------------------
 // The 64-token tiles batch row `b` sees, [lo, hi).  `all_if_empty`: a query position that sees no key averages over every
 // one of them (the quantized path), so no tile may be left out for its row.

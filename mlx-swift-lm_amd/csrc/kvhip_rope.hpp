@@ -227,6 +227,36 @@ template <int DT, int D, int THREADS, int RMAX> struct RopeStep {
     float freq;
     using E = typename Elem<DT>::type;
     E x[NR], y[NR];
+    // Row J * NS and on of a thread.  (One row at a time: a uniform number, and a wavefront does not run through the code of
+    // rows that there are not.)
+    template <int J> __device__ __forceinline__ void fetch_rows(const E *q, const E *k, int R) {
+        if constexpr (J < NR) {
+            const int i = (NS == 1 ? 0 : threadIdx.x / P) + J * NS;
+            if (NS == 1 && i > R) return;
+            if (i <= R && (NS * P == THREADS || threadIdx.x < NS * P)) {
+                const E *row = i < R ? q + (size_t)i * D : k;
+                x[J] = row[d0];
+                y[J] = row[d1];
+            }
+            fetch_rows<J + 1>(q, k, R);
+        }
+    }
+    template <int J> __device__ __forceinline__ void turn_rows(float sn, float cs, int R, E *dst) {
+        if constexpr (J < NR) {
+            const int i = (NS == 1 ? 0 : threadIdx.x / P) + J * NS;
+            if (NS == 1 && i > R) return;
+            if (i <= R && (NS * P == THREADS || threadIdx.x < NS * P)) {
+                if (rotates) {
+                    const float a = Elem<DT>::load(&x[J], 0), b = Elem<DT>::load(&y[J], 0);
+                    Elem<DT>::store(&x[J], 0, rope_turn(a, b, true, sn, cs));
+                    Elem<DT>::store(&y[J], 0, rope_turn(b, a, false, sn, cs));
+                }
+                dst[i * D + d0] = x[J];
+                dst[i * D + d1] = y[J];
+            }
+            turn_rows<J + 1>(sn, cs, R, dst);
+        }
+    }
     __device__ __forceinline__ void fetch(const RopeDev &r, const E *q, const E *k, int R) {
         const int p = threadIdx.x % P, half = r.dims >> 1;
         rotates = p < half;
@@ -234,15 +264,7 @@ template <int DT, int D, int THREADS, int RMAX> struct RopeStep {
         d1 = rotates && !r.traditional ? d0 + half : d0 + 1;
         freq = 1.f;
         if (r.freqs && rotates) freq = r.freqs[p];
-#pragma unroll
-        for (int j = 0; j < NR; ++j) {
-            const int i = threadIdx.x / P + j * NS;
-            if (i <= R && threadIdx.x < NS * P) {
-                const E *row = i < R ? q + (size_t)i * D : k;
-                x[j] = row[d0];
-                y[j] = row[d1];
-            }
-        }
+        fetch_rows<0>(q, k, R);
     }
     __device__ __forceinline__ void turn(const RopeDev &r, int bh, int R, E *dst) {
         float sn = 0.f, cs = 1.f;
@@ -253,19 +275,7 @@ template <int DT, int D, int THREADS, int RMAX> struct RopeStep {
         // (`freq` lives to here: its register holds what may be a load in flight, and the angle, formed in it, would wait for
         // every load requested since, the first tile's with them)
         asm volatile("" ::"v"(freq));
-#pragma unroll
-        for (int j = 0; j < NR; ++j) {
-            const int i = threadIdx.x / P + j * NS;
-            if (i <= R && threadIdx.x < NS * P) {
-                if (rotates) {
-                    const float a = Elem<DT>::load(&x[j], 0), b = Elem<DT>::load(&y[j], 0);
-                    Elem<DT>::store(&x[j], 0, rope_turn(a, b, true, sn, cs));
-                    Elem<DT>::store(&y[j], 0, rope_turn(b, a, false, sn, cs));
-                }
-                dst[i * D + d0] = x[j];
-                dst[i * D + d1] = y[j];
-            }
-        }
+        turn_rows<0>(sn, cs, R, dst);
     }
 };
 
