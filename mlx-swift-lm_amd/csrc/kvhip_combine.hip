@@ -41,9 +41,6 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
     __shared__ float red_s[2][4];
     __shared__ kv_f2 acc_s[NG][CP];
     const int i = blockIdx.x, bh = blockIdx.y;
-    const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
-    const int r = a.Hq / a.Hkv;
-    const int rep = i / a.L, l = i - rep * a.L;
     const size_t sstride = (size_t)rr * (D + 2);
     size_t first_slot = (size_t)bh * nsplit;
     if constexpr (SPANS) {  // (a ragged batch's rows have spans in proportion to their keys: kvhip_mask.hpp)
@@ -105,7 +102,8 @@ __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, 
         kv_f2 o = acc_s[0][t];
 #pragma unroll
         for (int k = 1; k < NG; ++k) o += acc_s[k][t];
-        store_pair<DT>(a.out, ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D + c0 + 2 * t, den > 0.f ? o.x / den : 0.f, den > 0.f ? o.y / den : 0.f);
+        // (a pair's query rows lie one behind the other: Hq / Hkv heads of L rows)
+        store_pair<DT>(a.out, ((size_t)bh * gridDim.x + i) * D + c0 + 2 * t, den > 0.f ? o.x / den : 0.f, den > 0.f ? o.y / den : 0.f);
     }
 }
 
@@ -124,10 +122,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(AttendArgs a, int nsp
     constexpr bool EXACT = exact_merge<D, DT>();
     const int in_wg = threadIdx.x / LPR, c = 4 * (threadIdx.x % LPR);
     const int i = blockIdx.x * RPW + in_wg, bh = blockIdx.y;
-    const int r = a.Hq / a.Hkv;
-    if (in_wg >= RPW || i >= r * a.L) return;  // (rr, the rows a part holds, may exceed the query rows there are)
-    const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
-    const int rep = i / a.L, l = i - rep * a.L;
+    if (in_wg >= RPW || i >= rr) return;
     const size_t sstride = (size_t)rr * (D + 2);
     const float *part = a.workspace + (size_t)bh * nsplit * sstride + (size_t)i * (D + 2);
     kv_f2 ml[MAXP], p[MAXP][2];  // (a row of partials is 8-byte aligned: D + 2 floats)
@@ -152,7 +147,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(AttendArgs a, int nsp
         num[2] = own ? add_weighed<EXACT>(num[2], w, p[s][1].x) : num[2];
         num[3] = own ? add_weighed<EXACT>(num[3], w, p[s][1].y) : num[3];
     }
-    const size_t ooff = ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D + c;
+    const size_t ooff = ((size_t)bh * rr + i) * D + c;  // (a pair's query rows lie one behind the other)
 #pragma unroll
     for (int k = 0; k < 2; ++k) store_pair<DT>(a.out, ooff + 2 * k, den > 0.f ? num[2 * k] / den : 0.f, den > 0.f ? num[2 * k + 1] / den : 0.f);
 }
@@ -194,9 +189,13 @@ hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t
     if (a.st.Dv == 64) return merge_dtype<64, 64>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 80) return merge_dtype<80, 80>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 96) return merge_dtype<96, 96>(a, nsplit, rows, spans, s);
-    if (a.st.Dv == 128) return merge_dtype<128, 128>(a, nsplit, rows, spans, s);
+    // Blocks of fewer columns shorten a workgroup's chain where the launch has few rows (a sequence's 32 rows of 64 spans: 3.4
+    // us of 128 columns, 3.2 of 64; 8 rows of 65 spans at head size 512: 3.8 of 64, 3.3 of 32), and are workgroups more where
+    // it has many (2048 rows: 1 us).
+    const size_t all = (size_t)(a.Hq / a.Hkv) * a.L * a.st.BH;
+    if (a.st.Dv == 128) return all <= 1024 ? merge_dtype<128, 64>(a, nsplit, rows, spans, s) : merge_dtype<128, 128>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 256) return merge_dtype<256, 128>(a, nsplit, rows, spans, s);
-    if (a.st.Dv == 512) return merge_dtype<512, 32>(a, nsplit, rows, spans, s);
+    if (a.st.Dv == 512) return all <= 128 ? merge_dtype<512, 32>(a, nsplit, rows, spans, s) : merge_dtype<512, 64>(a, nsplit, rows, spans, s);
     return hipErrorInvalidValue;
 }
 
