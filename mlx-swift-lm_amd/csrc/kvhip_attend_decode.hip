@@ -176,6 +176,15 @@ template <int BITS, int D, int G> struct TileRegs {
     bool edge;  // wave-uniform: some token of the tile is dead or masked for some query row
 };
 
+// Hq / Hkv for at most MAX query heads to a kv head: comparisons in place of a division, which a step's first request would
+// wait for (with those of the batch row and of the query rows' heads: 0.2 us of a launch).
+template <int MAX> __device__ __forceinline__ int heads_of_a_kv_head(int Hq, int Hkv) {
+    int r = 1;
+#pragma unroll
+    for (int i = 2; i <= MAX; ++i) r += Hq >= i * Hkv ? 1 : 0;
+    return r;
+}
+
 // RG = groups of 4 query rows handled per pass (R <= 4 RG).  MM selects the mask code:
 // 0 none (the tile loop is branch free), 1 index-only masks (causal / window, per-batch
 // bounds preloaded: no memory access in the loop), 2 array masks (loads in the loop, which
@@ -209,8 +218,8 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
     const int blk = lane >> 2, qi = lane & 3;  // lane group (MFMA block) and position in it
     int bh = blockIdx.y;
     const int split = blockIdx.x;
-    int b = bh / a.Hkv;
-    const int hk = bh - b * a.Hkv;
+    int b = MM == 0 ? 0 : bh / a.Hkv;  // (without a mask nothing asks for it)
+    [[maybe_unused]] const int hk = bh - b * a.Hkv;
     size_t part_slot = (size_t)bh * nsplit + split;  // where this workgroup's partial goes
     [[maybe_unused]] RaggedSpan span;
     [[maybe_unused]] int wid = 0;
@@ -229,8 +238,8 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
             part_slot = (size_t)bh * nsplit + split;
         }
     }
-    const int r = a.Hq / a.Hkv;
-    const int R = r * a.L;
+    const int r = heads_of_a_kv_head<RR>(a.Hq, a.Hkv);
+    const int R = r * a.L;  // (a pair's query rows lie one behind the other)
 
     __shared__ __attribute__((aligned(16))) WaveParts<D, NW, RR> parts;
     // A step with rotary positions: the query rows and the new key row, rotated, wait in LDS (where the partials go at
@@ -238,7 +247,7 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
     uint16_t *rot_s = reinterpret_cast<uint16_t *>(&parts.rows[0][0][0]);
     [[maybe_unused]] RopeStep<DT, D, NW * 64, 4> step;
     if constexpr (rot)
-        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
+        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)bh * R * D,
                    static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R);
 
     // ---- query operands: lane (blk, qi) holds row qi's 4 elements of step 16 x + blk ----
@@ -257,8 +266,8 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
         // rows past R read row 0 (in bounds) and count as zero: no branch around the loads, which
         // are then all in flight together instead of one after the other
         const bool ok = i < R;
-        const int rep = ok ? i / a.L : 0, l = ok ? i - rep * a.L : 0;
-        const size_t qoff = ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D;
+        const int row = ok ? i : 0;
+        const size_t qoff = ((size_t)bh * R + row) * D;
         float raw[NQA][4];
 #pragma unroll
         for (int x = 0; x < NQA; ++x) {
@@ -267,7 +276,7 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int d = w * GEO::EPW + GEO::elem(h, k);
-                raw[x][k] = rot ? Elem<DT>::load(rot_s, rep * D + d) : Elem<DT>::load(a.q, qoff + d);
+                raw[x][k] = rot ? Elem<DT>::load(rot_s, row * D + d) : Elem<DT>::load(a.q, qoff + d);
             }
         }
         float part[G];
@@ -732,7 +741,7 @@ decode_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeArgs
             span_table(a.workspace, st.BH, nsplit, RR * (D + 2))[bh] = make_int2((int)part_slot, span.count);
     }
     // a single span writes the output rows, several leave partials
-    leave_rows<D, DT>(a, parts, R, nsplit == 1, (size_t)(b * a.Hq + hk * r) * a.L, part_slot);
+    leave_rows<D, DT>(a, parts, R, nsplit == 1, (size_t)bh * R, part_slot);
 }
 
 // ---------------------------------------------------------------------------------
@@ -761,10 +770,10 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
     const int blk = lane >> 2, qi = lane & 3;
     int bh = blockIdx.y;
     const int split = blockIdx.x;
-    int b = bh / a.Hkv;
-    const int hk = bh - b * a.Hkv;
-    const int r = a.Hq / a.Hkv;
-    const int R = r * a.L;
+    int b = MM == 0 ? 0 : bh / a.Hkv;  // (without a mask nothing asks for it)
+    [[maybe_unused]] const int hk = bh - b * a.Hkv;
+    const int r = heads_of_a_kv_head<RR>(a.Hq, a.Hkv);
+    const int R = r * a.L;  // (a pair's query rows lie one behind the other)
     size_t part_slot = (size_t)bh * nsplit + split;  // where this workgroup's partial goes
     [[maybe_unused]] RaggedSpan span;
     [[maybe_unused]] int wid = 0;
@@ -785,7 +794,7 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
     uint16_t *rot_s = reinterpret_cast<uint16_t *>(&parts.rows[0][0][0]);
     [[maybe_unused]] RopeStep<DT, D, WAVES * 64, RR> step;
     if constexpr (rot)
-        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * D,
+        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)bh * R * D,
                    static_cast<const uint16_t *>(a.new_k) + (size_t)bh * D, R);
 
     // query operands: lane (blk, qi) holds row qi's elements 4*(16 x + blk) .. +3, unscaled
@@ -794,13 +803,12 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg) {
             const int i = 4 * rg + qi;
-            const int rep = i / a.L, l = i - rep * a.L;
-            const size_t qoff = ((size_t)(b * a.Hq + hk * r + rep) * a.L + l) * D;
+            const size_t qoff = ((size_t)bh * R + i) * D;
 #pragma unroll
             for (int x = 0; x < NP; ++x) {
                 uint2 w = make_uint2(0, 0);
                 if (i < R) {
-                    if (rot) w = *reinterpret_cast<const uint2 *>(rot_s + rep * D + 4 * (16 * x + blk));
+                    if (rot) w = *reinterpret_cast<const uint2 *>(rot_s + i * D + 4 * (16 * x + blk));
                     else w = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.q) + qoff + 4 * (16 * x + blk));
                 }
                 qa[rg][x].u[0] = w.x;
@@ -898,8 +906,10 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
     // ---- the step's new row, when it is still to be written (unmasked single-token decode) -----
     // Exactly one wavefront of one workgroup reads the tile of physical slot `new_slot` (spans are equal and
     // cover every tile): it copies the row into the page after it has requested its first pieces and before it requests
-    // others, so its own later loads of the tile see it; if its first tile is that tile, it requests them only then.  The
-    // row is requested in front of the pieces.
+    // others, so its own later loads of the tile see it; if its first tile is that tile, of the first pieces the K ones are
+    // requested ahead all the same and their lane of the row's token is given the row from LDS.  (All of them requested behind
+    // the row, with a wait for its stores, that wavefront ended the kernel.)  The row is
+    // requested in front of the pieces.
     bool own = false;
     kv_u4 own_k;
     uint32_t own_v[NP];
@@ -919,13 +929,18 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
     // (the queries before the pieces: loads complete in order, and a wait for queries requested after the
     // first pieces would be a wait for those pieces too -- in every iteration, the compiler
     // placing one wait for all ways into the loop)
-    auto request_first = [&]() __attribute__((always_inline)) {
-        static_for<NBUF>([&](auto N) { request(buf_of(decltype(N)::value), decltype(N)::value); });
+    constexpr int NK = NBUF < NP ? NBUF : NP;  // K pieces among the first
+    auto request_first_k = [&]() __attribute__((always_inline)) {
+        static_for<NK>([&](auto N) { request(buf_of(decltype(N)::value), decltype(N)::value); });
+    };
+    auto request_first_v = [&]() __attribute__((always_inline)) {
+        static_for<NBUF - NK>([&](auto N) { request(buf_of(NK + decltype(N)::value), NK + decltype(N)::value); });
     };
     const bool row_first = own && tile0 == a.new_slot >> 6;  // wave-uniform
     if (my_tiles > 0) {
         if constexpr (!rot) load_queries();
-        if (!row_first) request_first();
+        request_first_k();
+        if (!row_first) request_first_v();
     }
     if constexpr (MM == 1) {
 #pragma unroll
@@ -940,16 +955,37 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
     }
     if constexpr (MM == 0) {
         if (own) {  // wave-uniform
-            const int slot = a.new_slot;
-            char *kc = const_cast<char *>(k_cell_ptr(st, bh, slot));
-            char *vc = const_cast<char *>(v_cell_ptr(st, bh, slot));
-            if (lane < D / 8)
-                *reinterpret_cast<kv_u4 *>(kc + kfp_off(st, slot, 8 * lane)) = rot ? *reinterpret_cast<const kv_u4 *>(rot_s + R * D + 8 * lane) : own_k;
+            // (global stores, and offsets as kfp_off and vfp_off give them for two-byte elements: behind a store to a plain
+            // pointer every load in flight is waited for, and divisions by the element size cost a microsecond here.  What a
+            // wavefront loads behind its own stores it loads as stored: the fence holds the compiler)
+            const int t = a.new_slot & (PAGE - 1), tk = t & (TILE - 1);
+            const PageEntry page{const_cast<char *>(pt[a.new_slot >> PAGE_SHIFT].k), nullptr, const_cast<char *>(pt[a.new_slot >> PAGE_SHIFT].v), nullptr};
+            KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell) + (t >> 6) * (TILE * D * 2) + tk * 16;
+            KV_GLOBAL char *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell) + (t >> 6) * (TILE * D * 2) + (tk >> 3) * (D * 16) + (tk & 7) * 2;
+            uint16_t *row_s = rot ? rot_s + R * D : reinterpret_cast<uint16_t *>(&parts.rows[wave][0][0]);
+            if (lane < D / 8) {
+                if constexpr (rot) own_k = *reinterpret_cast<const kv_u4 *>(row_s + 8 * lane);
+                else *reinterpret_cast<kv_u4 *>(row_s + 8 * lane) = own_k;
+                *reinterpret_cast<KV_GLOBAL kv_u4 *>(kc + lane * (TILE * 16)) = own_k;
+            }
 #pragma unroll
-            for (int h = 0; h < NP; ++h) *reinterpret_cast<uint16_t *>(vc + vfp_off(st, slot, 64 * h + lane)) = (uint16_t)own_v[h];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            if (row_first) request_first();
+            for (int h = 0; h < NP; ++h) *reinterpret_cast<KV_GLOBAL uint16_t *>(vc + (64 * h + lane) * 16) = (uint16_t)own_v[h];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (row_first) {
+                request_first_v();
+                if (lane == tk) {
+                    static_for<NK>([&](auto X) {
+                        constexpr int x = decltype(X)::value;
+                        uint32_t *buf = buf_of(x);
+#pragma unroll
+                        for (int j = 0; j < PW / 4; ++j) {
+                            const kv_u4 v = *reinterpret_cast<const kv_u4 *>(row_s + 64 * x + 8 * j);
+                            buf[4 * j] = v.x; buf[4 * j + 1] = v.y; buf[4 * j + 2] = v.z; buf[4 * j + 3] = v.w;
+                        }
+                    });
+                }
+            }
         }
     }
     if (my_tiles > 0) {
@@ -1085,7 +1121,7 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
             span_table(a.workspace, st.BH, nsplit, RR * (D + 2))[bh] = make_int2((int)part_slot, span.count);
     }
     // a single span writes the output rows itself, several leave partials for the merge kernel
-    leave_rows<D, DT>(a, parts, R, nsplit == 1, (size_t)(b * a.Hq + hk * r) * a.L, part_slot);
+    leave_rows<D, DT>(a, parts, R, nsplit == 1, (size_t)bh * R, part_slot);
 }
 
 struct Plan {

@@ -185,7 +185,8 @@ decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeAr
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, jj = lane >> 4;
     int bh = blockIdx.y, split = blockIdx.x;
-    int b = bh / a.Hkv, hk = bh - b * a.Hkv;
+    int b = MM == 0 ? 0 : bh / a.Hkv;  // (without a mask nothing asks for it: see decode_kernel)
+    [[maybe_unused]] int hk = bh - b * a.Hkv;
     const int r = a.Hq / a.Hkv;
     const int R = r * a.L;
     size_t part_slot = (size_t)bh * nsplit + split;  // where this workgroup's partial goes
@@ -198,7 +199,7 @@ decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeAr
     uint16_t *rot_s = reinterpret_cast<uint16_t *>(&parts.rows[0][0][0]);
     [[maybe_unused]] RopeStep<DT, DK, WAVES * 64, RR> step;
     if constexpr (rot)
-        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)(b * a.Hq + hk * r) * DK,
+        step.fetch(a.turn, reinterpret_cast<const uint16_t *>(a.q) + (size_t)bh * R * DK,
                    static_cast<const uint16_t *>(a.new_k) + (size_t)bh * DK, R);
     // ---- span of this workgroup (as in the 4-row kernel) -----------------------------------
     [[maybe_unused]] RaggedSpan span;
@@ -242,7 +243,7 @@ decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeAr
         sym_mask_full_range(sym, full_lo, full_hi);
         full_hi = min(full_hi, a.T - 1);
     }
-    const int row_l = n % a.L, row_rep = n / a.L;  // this lane's query row n = (head rep, position l)
+    [[maybe_unused]] const int row_l = n % a.L, row_rep = n / a.L;  // this lane's query row n = (head rep, position l)
     const bool row_ok = n < R;
     [[maybe_unused]] KeyBounds seen{0, 0};
     if constexpr (MM == 1) seen = sym_mask_bounds(sym, row_l);
@@ -475,14 +476,14 @@ decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeAr
     auto load_queries = [&]() __attribute__((always_inline)) {
         // rows past R read row 0 (in bounds) and are zeroed: no branch around the loads, which
         // are one 16-byte piece per contraction step
-        const int rep = row_ok ? row_rep : 0, lq = row_ok ? row_l : 0;
-        const uint16_t *qrow = reinterpret_cast<const uint16_t *>(a.q) + ((size_t)(b * a.Hq + hk * r + rep) * a.L + lq) * DK;
+        const int row = row_ok ? n : 0;
+        const uint16_t *qrow = reinterpret_cast<const uint16_t *>(a.q) + ((size_t)bh * R + row) * DK;
         u4 raw[GK][SPG];
 #pragma unroll
         for (int g = 0; g < GK; ++g)
 #pragma unroll
             for (int h = 0; h < SPG; ++h) {
-                if (rot) raw[g][h] = *reinterpret_cast<const u4 *>(rot_s + rep * DK + GS * g + (GS / 4) * jj + 8 * h);
+                if (rot) raw[g][h] = *reinterpret_cast<const u4 *>(rot_s + row * DK + GS * g + (GS / 4) * jj + 8 * h);
                 else raw[g][h] = *reinterpret_cast<const u4 *>(qrow + GS * g + (GS / 4) * jj + 8 * h);
             }
 #pragma unroll
@@ -767,7 +768,7 @@ decode16_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeAr
             span_table(a.workspace, st.BH, nsplit, RR * (DV + 2))[bh] = make_int2((int)part_slot, span.count);
     }
     // a single span writes the output rows, several leave partials
-    leave_rows<DV, DT>(a, parts, R, nsplit == 1, (size_t)(b * a.Hq + hk * r) * a.L, part_slot);
+    leave_rows<DV, DT>(a, parts, R, nsplit == 1, (size_t)bh * R, part_slot);
 }
 
 }  // namespace
