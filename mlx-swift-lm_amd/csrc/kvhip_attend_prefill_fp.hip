@@ -118,7 +118,8 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     const int R = r * a.L;
     const WorkItem item = work_item<MM>(a, (R + BM - 1) / BM, nsplit);
     const int blk_x = item.block, bh = item.bh;
-    const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
+    const int b = MM == 0 ? 0 : bh / a.Hkv;  // (without a mask nothing asks for it)
+    [[maybe_unused]] const int hk = bh - b * a.Hkv;
     const int row0 = blk_x * BM + wave * 16 * QT;  // first query row of this wavefront
     const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
     // Scores enter the softmax as exp2(s * ef - m) with ef = |scale| log2 e > 0 -- a negative scale
@@ -136,17 +137,14 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
 
     // ---- query operands: B of S^T = K . Q^T; lane (n, jj) holds q[row][32 s + 8 jj ..] raw ----
     Op8 qop[QT][S];
-    int q_l[QT], q_h[QT];
+    int q_l[QT] = {}, q_h[QT] = {};
     bool q_ok[QT];
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const int i = row0 + 16 * qt + n;
         q_ok[qt] = i < R;
-        const int rep = q_ok[qt] ? i / a.L : 0;
-        q_l[qt] = q_ok[qt] ? i - rep * a.L : 0;
-        q_h[qt] = hk * r + rep;
-        const u4 *qp = reinterpret_cast<const u4 *>(
-            reinterpret_cast<const uint16_t *>(a.q) + ((size_t)(b * a.Hq + q_h[qt]) * a.L + q_l[qt]) * DK + 8 * jj);
+        // (a pair's query rows lie one behind the other; which positions they are is worked out behind the first requests)
+        const u4 *qp = reinterpret_cast<const u4 *>(reinterpret_cast<const uint16_t *>(a.q) + ((size_t)bh * R + i) * DK + 8 * jj);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             u4 w = (q_ok[qt] && (DK % 32 == 0 || 32 * s + 8 * jj < DK)) ? qp[4 * s] : u4{0, 0, 0, 0};
@@ -247,27 +245,6 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     // past the end), tested with one unsigned comparison per key.
     [[maybe_unused]] int q_lo[QT];
     [[maybe_unused]] uint32_t q_span[QT];
-    if constexpr (MM == 1) {
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            int lo, hi;
-            if (sym.mode == KVHIP_MASK_CAUSAL) {
-                lo = 0;
-                hi = a.T - a.L + q_l[qt];
-            } else {
-                const int li = sym.offset + q_l[qt];
-                lo = sym.pad_b;
-                hi = min(li, sym.len_b - 1);
-                if (sym.window > 0) lo = max(lo, li - sym.window + 1);
-            }
-            lo = max(lo, 0);
-            hi = min(hi, a.T - 1);
-            const bool any = q_ok[qt] && hi >= lo;
-            q_lo[qt] = any ? lo : 0;
-            q_span[qt] = any ? (uint32_t)(hi - lo) : 0u;
-            if (!any) q_lo[qt] = 0x40000000;  // no row reaches it: row - q_lo wraps to a huge unsigned value
-        }
-    }
     auto apply_mask = [&](int par, f4 (&sc)[QT][2]) __attribute__((always_inline)) {
         int trow[2][4];
 #pragma unroll
@@ -504,6 +481,35 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         dma_v(vt_of(v_lo), 0);
         if (v_lo + 1 < v_hi) dma_k(vt_of(v_lo + 1), 1);
     }
+    if constexpr (MM != 0) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            const int i = row0 + 16 * qt + n, rep = q_ok[qt] ? i / a.L : 0;
+            q_l[qt] = q_ok[qt] ? i - rep * a.L : 0;
+            q_h[qt] = hk * r + rep;
+        }
+    }
+    if constexpr (MM == 1) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            int lo, hi;
+            if (sym.mode == KVHIP_MASK_CAUSAL) {
+                lo = 0;
+                hi = a.T - a.L + q_l[qt];
+            } else {
+                const int li = sym.offset + q_l[qt];
+                lo = sym.pad_b;
+                hi = min(li, sym.len_b - 1);
+                if (sym.window > 0) lo = max(lo, li - sym.window + 1);
+            }
+            lo = max(lo, 0);
+            hi = min(hi, a.T - 1);
+            const bool any = q_ok[qt] && hi >= lo;
+            q_lo[qt] = any ? lo : 0;
+            q_span[qt] = any ? (uint32_t)(hi - lo) : 0u;
+            if (!any) q_lo[qt] = 0x40000000;  // no row reaches it: row - q_lo wraps to a huge unsigned value
+        }
+    }
     wait_all_loads();
     // (the same wait once more in a form the compiler's bookkeeping sees: it then knows that the
     // query operands have arrived, and does not wait for them -- and with them for every load just
@@ -603,7 +609,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
             continue;
         }
         const float inv = l > 0.f ? 1.0f / l : 0.f;
-        const size_t ooff = ((size_t)(b * a.Hq + q_h[qt]) * a.L + q_l[qt]) * DV;
+        const size_t ooff = ((size_t)bh * R + row0 + 16 * qt + n) * DV;
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
             const float o0 = oacc[qt][dt][0] * inv, o1 = oacc[qt][dt][1] * inv;

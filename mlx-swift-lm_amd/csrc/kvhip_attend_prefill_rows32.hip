@@ -15,10 +15,11 @@
 //
 // What bounds it: the matrix cores at the clock that the chip's power leaves (1000 TFLOP/s of the 1190 that a large matrix
 // product reaches; without exponentials 1050, without requests 1140), and for short chunks what stands around the loop: of
-// 512 new rows over 2048 keys (25.5 us) 10 are launch, first tile and partials.
+// 512 new rows over 2048 keys (25.0 us) 3.8 to the first scores, 3 for the partials and up to 3 for the blocks that see fewer
+// keys than the last.
 // Measured against 32 rows on 16x16x32 instructions, which this replaces (D 128, 32q/8kv, causal, TFLOP/s): bfloat16 2048 x
-// 8192 946 -> 1002, 512 x 8192 893 -> 915 and a merge of half the bytes; float16 2048 x 8192 924 -> 964, 512 x 8192 883
-// -> 873 and the same.
+// 8192 946 -> 1027, 512 x 8192 893 -> 939 and a merge of half the bytes; float16 2048 x 8192 924 -> 964, 512 x 8192 883
+// -> 885 and the same.
 #include "kvhip_prefill_fp.hpp"
 
 #ifndef KV_SB
@@ -63,28 +64,25 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
     const int R = r * a.L;
     const WorkItem item = work_item<MM>(a, (R + BM - 1) / BM, nsplit);
     const int blk_x = item.block, bh = item.bh;
-    const int b = bh / a.Hkv, hk = bh - b * a.Hkv;
+    const int b = MM == 0 ? 0 : bh / a.Hkv;  // (without a mask nothing asks for it)
+    [[maybe_unused]] const int hk = bh - b * a.Hkv;
     const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
     constexpr bool LM = DT == 0;
     const bool flip = a.scale < 0.f;
     const float sl2 = fmaxf(fabsf(a.scale) * LOG2E, 1e-30f);
     const float ef = MM == 2 ? 1.f : sl2;
 
-    // ---- query operands: B of S^T = K . Q^T; lane (n, hh) holds q[row][16 s + 8 hh ..] raw ----
+    // Query operands, B of S^T = K . Q^T: lane (n, hh) holds q[row][16 s + 8 hh ..] raw.  (A pair's query rows lie one behind
+    // the other.  Requested first, they arrive last: 64 rows a load.  Which positions they are is worked out behind the first
+    // requests for keys.)
     const int row = blk_x * BM + wave * 32 + n;
     const bool q_ok = row < R;
-    const int rep = q_ok ? row / a.L : 0;
-    const int q_l = q_ok ? row - rep * a.L : 0, q_h = hk * r + rep;
+    int q_l = 0, q_h = 0;
     Op8 qop[KS];
     {
-        const u4 *qp = reinterpret_cast<const u4 *>(
-            reinterpret_cast<const uint16_t *>(a.q) + ((size_t)(b * a.Hq + q_h) * a.L + q_l) * D + 8 * hh);
+        const u4 *qp = reinterpret_cast<const u4 *>(reinterpret_cast<const uint16_t *>(a.q) + ((size_t)bh * R + row) * D + 8 * hh);
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            u4 w = q_ok ? qp[2 * s] : u4{0, 0, 0, 0};
-            if (flip) w ^= u4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
-            qop[s].v = w;
-        }
+        for (int s = 0; s < KS; ++s) qop[s].v = q_ok ? qp[2 * s] : u4{0, 0, 0, 0};
     }
     // float16: the denominators ride on the matrix cores, which sum the rounded probabilities that the numerator uses.
     // Read as the operand of a 16x16x32 instruction the probabilities' lanes are 16 queries by four groups of eight
@@ -154,23 +152,6 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
     // ---- masks ----
     [[maybe_unused]] int q_lo = 0;
     [[maybe_unused]] uint32_t q_span = 0;
-    if constexpr (MM == 1) {
-        int lo, hi;
-        if (sym.mode == KVHIP_MASK_CAUSAL) {
-            lo = 0;
-            hi = a.T - a.L + q_l;
-        } else {
-            const int li = sym.offset + q_l;
-            lo = sym.pad_b;
-            hi = min(li, sym.len_b - 1);
-            if (sym.window > 0) lo = max(lo, li - sym.window + 1);
-        }
-        lo = max(lo, 0);
-        hi = min(hi, a.T - 1);
-        const bool any = q_ok && hi >= lo;
-        q_lo = any ? lo : 0x40000000;
-        q_span = any ? (uint32_t)(hi - lo) : 0u;
-    }
     auto masked_block = [&](int k, int slot) __attribute__((always_inline)) -> bool {
         if constexpr (MM == 2) return true;
         if constexpr (IDENT) {
@@ -322,6 +303,32 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
         request_k(2, 1);
         request_v(1, 1);
     }
+    if (flip) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) qop[s].v ^= u4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+    }
+    if constexpr (MM != 0) {
+        const int rep = q_ok ? row / a.L : 0;
+        q_l = q_ok ? row - rep * a.L : 0;
+        q_h = hk * r + rep;
+    }
+    if constexpr (MM == 1) {
+        int lo, hi;
+        if (sym.mode == KVHIP_MASK_CAUSAL) {
+            lo = 0;
+            hi = a.T - a.L + q_l;
+        } else {
+            const int li = sym.offset + q_l;
+            lo = sym.pad_b;
+            hi = min(li, sym.len_b - 1);
+            if (sym.window > 0) lo = max(lo, li - sym.window + 1);
+        }
+        lo = max(lo, 0);
+        hi = min(hi, a.T - 1);
+        const bool any = q_ok && hi >= lo;
+        q_lo = any ? lo : 0x40000000;
+        q_span = any ? (uint32_t)(hi - lo) : 0u;
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0x0f70);  // (in a form the compiler's bookkeeping sees)
     __syncthreads();
@@ -455,7 +462,7 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
         return;
     }
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + ((size_t)(b * a.Hq + q_h) * a.L + q_l) * D;
+    uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + ((size_t)bh * R + row) * D;
 #pragma unroll
     for (int c = 0; c < NCB; ++c)
 #pragma unroll
