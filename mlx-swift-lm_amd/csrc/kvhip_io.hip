@@ -487,7 +487,9 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
             }
         }
         char *kcell = page_table(st)[slot_t >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;  // a tile lies inside one page
-        if (live && r >= t_lo && r < t_hi) *reinterpret_cast<kv_u4 *>(kcell + kfp_off(st, slot_t + r, d0)) = k;
+        // (kfp_off and vfp_off, whose divisions by the element size run on every thread, with it known)
+        if (live && r >= t_lo && r < t_hi)
+            *reinterpret_cast<kv_u4 *>(kcell + (size_t)((slot_t & (PAGE - 1)) >> 6) * (TILE * DK * ES) + ((d0 / E) * TILE + r) * 16) = k;
         return;
     }
     const int c0 = (piece - P::KP) * P::VC;  // first column
@@ -512,7 +514,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
     __syncthreads();
     // chunks of E tokens of every column: a thread gathers tokens E ce .. E ce + E - 1 of column d;
     // consecutive threads take consecutive columns, so a chunk row is written contiguously
-    char *cell = const_cast<char *>(v_cell_ptr(st, bh, slot_t));
+    char *cell = const_cast<char *>(v_cell_ptr(st, bh, slot_t)) + (size_t)((slot_t & (PAGE - 1)) >> 6) * (TILE * DV * ES);
     const T *vte = reinterpret_cast<const T *>(vt);
     constexpr int VPE = VPW * 4 / ES;
     for (int c = threadIdx.x; c < P::VC * (TILE / E); c += 256) {
@@ -523,7 +525,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
             if constexpr (ES == 4) out[j] = vte[(t0 + j) * VPE + d];
             else out[j] = (uint32_t)vte[(t0 + 2 * j) * VPE + d] | ((uint32_t)vte[(t0 + 2 * j + 1) * VPE + d] << 16);
         }
-        char *dst = cell + vfp_off(st, slot_t + t0, c0 + d);
+        char *dst = cell + ((t0 / E) * DV + c0 + d) * 16;
         if (t0 >= t_lo && t0 + E <= t_hi) {
             *reinterpret_cast<kv_u4 *>(dst) = kv_u4{out[0], out[1], out[2], out[3]};
         } else {

@@ -295,7 +295,16 @@ __device__ __forceinline__ void rope_rows_body(const RopeDev &r, const char *x, 
     const int half = r.dims >> 1;
     const int np = r.traditional ? r.dims / V : half / V;  // rotating items of a head, then the chunks that pass through
     const int items = np + (D - r.dims) / V;
-    const int item = threadIdx.x % items, slot = threadIdx.x / items, ns = rope_ride_threads((int)blockDim.x) / items;
+    int slot, ns;  // (the usual numbers of items without a division: the first loads wait for these)
+    if (__builtin_expect((items & (items - 1)) == 0, 1)) {
+        const int sh = 31 - __clz(items);
+        slot = threadIdx.x >> sh;
+        ns = rope_ride_threads((int)blockDim.x) >> sh;
+    } else {
+        slot = threadIdx.x / items;
+        ns = rope_ride_threads((int)blockDim.x) / items;
+    }
+    const int item = threadIdx.x - slot * items;
     const bool live = slot < ns;
     const bool turn = item < np;
     const int d0 = turn ? item * V : r.dims + (item - np) * V;
@@ -358,10 +367,16 @@ __host__ __device__ __forceinline__ int rope_heads_per_group(int rows, int H, in
 template <int DT>
 __device__ __forceinline__ void rope_queries_ride(const RopeDev &r, int bh, float *inv_s) {
     const int i = (blockIdx.y - bh) * gridDim.x + blockIdx.x, rows = r.qB * r.qL;
-    const int hg = rope_heads_per_group(rows, r.qH, r.qD, DT == 2 ? 4 : 2, (int)blockDim.x), groups = (r.qH + hg - 1) / hg;
-    const int row = i / groups, h0 = (i - row * groups) * hg;
+    const int hg = rope_heads_per_group(rows, r.qH, r.qD, DT == 2 ? 4 : 2, (int)blockDim.x);
+    int row = i, h0 = 0, b = 0;
+    if (hg < r.qH) {
+        const int groups = (r.qH + hg - 1) / hg;
+        row = i / groups;
+        h0 = (i - row * groups) * hg;
+    }
     if (row >= rows) return;
-    rope_rows_body<DT>(r, r.qx, r.qo, r.qH, r.qL, r.qD, row / r.qL, row % r.qL, h0, min(r.qH, h0 + hg), inv_s);
+    if (r.qB > 1) b = row / r.qL;
+    rope_rows_body<DT>(r, r.qx, r.qo, r.qH, r.qL, r.qD, b, row - b * r.qL, h0, min(r.qH, h0 + hg), inv_s);
 }
 // Rows those workgroups add to the grid of an append whose rows are `gx` workgroups of `block` threads wide; 0: none ride.
 inline int rope_ride_rows(const RopeDev &r, int gx, int es, int block) {
