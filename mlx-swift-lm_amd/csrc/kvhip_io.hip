@@ -569,11 +569,24 @@ __global__ void import_fp_kernel(Store st, const char *src_k, const char *src_v,
     for (int d = threadIdx.x; d < st.Dv; d += blockDim.x) *reinterpret_cast<E *>(vc + vfp_off(st, slot, d)) = vs[d];
 }
 
+// kfp_off and vfp_off with the element size known
+template <int ES> __device__ __forceinline__ size_t kfp_at(const Store &st, int slot, int d) {
+    constexpr int EPC = 16 / ES;
+    const int t = slot & (PAGE - 1);
+    return (size_t)(t >> 6) * ((size_t)TILE * st.k_row) + (size_t)(((d / EPC) * TILE + (t & 63)) * 16 + (d % EPC) * ES);
+}
+template <int ES> __device__ __forceinline__ size_t vfp_at(const Store &st, int slot, int d) {
+    constexpr int EPC = 16 / ES;
+    const int t = slot & (PAGE - 1), tk = t & 63;
+    return (size_t)(t >> 6) * ((size_t)TILE * st.Dv * ES) + (size_t)(((tk / EPC) * st.Dv + d) * 16 + (tk % EPC) * ES);
+}
+
 // Rows in presented order into slots 0, 1, ... of another store (a ring that is laid out again, a copy).  grid (chunks of
 // 16 / ES rows, BH), 256 threads: the rows' 16-byte K chunks move whole, lanes along the rows; a thread puts a column's V
 // chunk together from the two that hold its tokens, shifted by where the run starts.  Chunks that a run begins or ends
-// inside (and rows of another launch's runs) go element by element.  HBM-bound: a ring
-// of 4096 rows of 16 (batch, head) pairs x 256, 16-bit (134 MB in and out) 42 us; element by element 155 us.
+// inside (and rows of another launch's runs) go element by element.  A ring of 4096 rows of 16 (batch, head) pairs x 256,
+// 16-bit (134 MB in and out): 34.7 us; 43 with offsets that divide by the element size, three divisions to a chunk and side;
+// element by element 155 us.
 template <int ES>
 __global__ void __launch_bounds__(256) compact_fp_kernel(Store src, Runs runs, Store dst, int nrows) {
     using E = typename std::conditional<ES == 2, uint16_t, uint32_t>::type;
@@ -592,17 +605,17 @@ __global__ void __launch_bounds__(256) compact_fp_kernel(Store src, Runs runs, S
         char *kd = const_cast<char *>(k_cell_ptr(dst, bh, row));
         const int chunks = src.Dk / EPC;
         for (int c = tid / EPC; c < chunks; c += 256 / EPC)
-            *reinterpret_cast<kv_u4 *>(kd + kfp_off(dst, row, c * EPC)) = *reinterpret_cast<const kv_u4 *>(ks + kfp_off(src, from, c * EPC));
+            *reinterpret_cast<kv_u4 *>(kd + kfp_at<ES>(dst, row, c * EPC)) = *reinterpret_cast<const kv_u4 *>(ks + kfp_at<ES>(src, from, c * EPC));
         for (int d = chunks * EPC + tid / EPC; d < src.Dk; d += 256 / EPC)
-            *reinterpret_cast<E *>(kd + kfp_off(dst, row, d)) = *reinterpret_cast<const E *>(ks + kfp_off(src, from, d));
+            *reinterpret_cast<E *>(kd + kfp_at<ES>(dst, row, d)) = *reinterpret_cast<const E *>(ks + kfp_at<ES>(src, from, d));
     }
     if (run) {
         const int sh = slot[0] % EPC, last = slot[0] + EPC - 1;
         const char *v0 = v_cell_ptr(src, bh, slot[0]), *v1 = v_cell_ptr(src, bh, last);
         char *vd = const_cast<char *>(v_cell_ptr(dst, bh, i0));
         for (int d = tid; d < src.Dv; d += 256) {
-            const kv_u4 x = *reinterpret_cast<const kv_u4 *>(v0 + vfp_off(src, slot[0] - sh, d));
-            const kv_u4 y = *reinterpret_cast<const kv_u4 *>(v1 + vfp_off(src, last - last % EPC, d));
+            const kv_u4 x = *reinterpret_cast<const kv_u4 *>(v0 + vfp_at<ES>(src, slot[0] - sh, d));
+            const kv_u4 y = *reinterpret_cast<const kv_u4 *>(v1 + vfp_at<ES>(src, last - last % EPC, d));
             uint32_t w[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
             const int words = sh * ES / 4;  // whole words to drop in front
             if (words & 2) {
@@ -617,7 +630,7 @@ __global__ void __launch_bounds__(256) compact_fp_kernel(Store src, Runs runs, S
 #pragma unroll
                 for (int k = 0; k < 4; ++k) w[k] = (w[k] >> 16) | (w[k + 1] << 16);
             }
-            *reinterpret_cast<kv_u4 *>(vd + vfp_off(dst, i0, d)) = kv_u4{w[0], w[1], w[2], w[3]};
+            *reinterpret_cast<kv_u4 *>(vd + vfp_at<ES>(dst, i0, d)) = kv_u4{w[0], w[1], w[2], w[3]};
         }
         return;
     }
@@ -627,7 +640,7 @@ __global__ void __launch_bounds__(256) compact_fp_kernel(Store src, Runs runs, S
         const char *vs = v_cell_ptr(src, bh, at);
         char *vd = const_cast<char *>(v_cell_ptr(dst, bh, i0 + j));
         for (int d = tid; d < src.Dv; d += 256)
-            *reinterpret_cast<E *>(vd + vfp_off(dst, i0 + j, d)) = *reinterpret_cast<const E *>(vs + vfp_off(src, at, d));
+            *reinterpret_cast<E *>(vd + vfp_at<ES>(dst, i0 + j, d)) = *reinterpret_cast<const E *>(vs + vfp_at<ES>(src, at, d));
     }
 }
 
