@@ -11,7 +11,7 @@
 //                  tokens 4 g .. 4 g + 3 of query i in lane (i, g): the probabilities are the operand as they are.
 // Measured against the vector-ALU kernel, whole calls: 512 x 4096, B4, 32q/8kv 1626 -> 654 us (D 64), 2644 -> 1215
 // (D 128: 106 TFLOP/s of the 157 that the instruction has), 6755 -> 2480 (D 256); one token of one sequence, 16q/4kv, 1500
-// keys 17.3 -> 12.4 us (D 64: one pass of loads and the merge); 8192 keys of B8, 8 kv heads, HBM: 102 -> 101 us (D 128).
+// keys 17.3 -> 9.9 us (D 64: one pass of loads, 6.4, and the merge, 3.5); 8192 keys of B8, 8 kv heads, HBM: 102 -> 101 us (D 128).
 #include <algorithm>
 
 #include "kvhip_mask.hpp"

@@ -20,8 +20,8 @@
 // Two rows of query tiles at most: the accumulators of four leave one wavefront per SIMD and are copied between the two
 // register files every tile (512 rows x 2048 keys, 8 query and 2 kv heads, bfloat16: 69 us the call, against 57 us).
 // Decode is bound by HBM where the batch fills the chip (B8, 4096 keys, one token: 26.5 us, 5.1 TB/s)
-// and by launch, one pass of loads and the merge below that (one sequence of 2064 keys, the kernel 8.2 us with the rotation
-// and the row's write, the merge 3.7; 63 us on the vector ALUs); a prompt chunk by the latency of the two barriers per tile
+// and by launch, one pass of loads and the merge below that (one sequence of 2064 keys, the kernel 7.7 us with the rotation
+// and the row's write, 10.4 before what its last workgroup and its first request waited for went, the merge 3.1; 63 us on the vector ALUs); a prompt chunk by the latency of the two barriers per tile
 // (512 x 2048, 33 us on average over a prompt's chunks and 7.4 us for the merge; 263 us).
 // K rows are loaded in the token order that leaves lane group g of the scores with tokens 8 g .. 8 g + 7, which is the
 // order the probabilities are read in as an operand: they never cross lanes.
