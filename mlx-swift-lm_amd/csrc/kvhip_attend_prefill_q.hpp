@@ -762,7 +762,7 @@ prefill_q_kernel(AttendArgs a, int nsplit) {
             const int i = row0 + 16 * qt + n;
             float *part = a.workspace + (((size_t)bh * nsplit + split) * R + i) * (DV + 2);
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f4 *>(part + 16 * dt + 4 * jj) = oacc[qt][dt];
+            for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<kv_part4 *>(part + 16 * dt + 4 * jj) = oacc[qt][dt];
             if (jj == 0) {
                 part[DV] = m_run[qt] * 0.6931471805599453f;  // back from the log2 domain
                 part[DV + 1] = l;

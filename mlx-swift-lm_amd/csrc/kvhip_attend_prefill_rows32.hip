@@ -454,7 +454,7 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
         for (int c = 0; c < NCB; ++c)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (32 * c + 8 * i < D && c >= c_lo && c < c_hi) *reinterpret_cast<f4 *>(part + 32 * c + 8 * i + 4 * hh) = f4{oacc[c][4 * i], oacc[c][4 * i + 1], oacc[c][4 * i + 2], oacc[c][4 * i + 3]};
+                if (32 * c + 8 * i < D && c >= c_lo && c < c_hi) *reinterpret_cast<kv_part4 *>(part + 32 * c + 8 * i + 4 * hh) = kv_part4{oacc[c][4 * i], oacc[c][4 * i + 1], oacc[c][4 * i + 2], oacc[c][4 * i + 3]};
         if (hh == 0 && half == 0) {
             part[D] = m_run * 0.6931471805599453f;  // back from the log2 domain
             part[D + 1] = l;

@@ -128,6 +128,8 @@ __device__ __forceinline__ const char *k_cell_ptr(const Store &st, int bh, int s
 // memory (address space 1): the loads become GLOBAL loads with counted, in-order waits.
 typedef uint32_t kv_u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t kv_u2 __attribute__((ext_vector_type(2)));
+// four floats of a row of partials: rows are D + 2 floats, every other one 8 bytes off a 16-byte boundary
+typedef float kv_part4 __attribute__((ext_vector_type(4), aligned(8)));
 #define KV_GLOBAL __attribute__((address_space(1)))
 typedef const KV_GLOBAL char *gptr;
 __device__ __forceinline__ gptr as_global(const void *p) { return (gptr) reinterpret_cast<const char *>(p); }
