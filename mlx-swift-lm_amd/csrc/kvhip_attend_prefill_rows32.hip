@@ -31,6 +31,7 @@ namespace {
 
 using namespace prefill_fp;
 typedef float f16v __attribute__((ext_vector_type(16)));
+typedef uint32_t out16 __attribute__((ext_vector_type(4), aligned(2)));  // 16 bytes of a caller's array, aligned as its elements are
 
 template <int DT> __device__ __forceinline__ void mfma32(f16v &c, const Op8 &a, const Op8 &b) {
     if constexpr (DT == 0) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, b.h, c, 0, 0, 0);
@@ -406,10 +407,10 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
 
     // ---- the two halves' sums: each group ends with the whole of half of the columns ----
     constexpr int C0 = (NCB + 1) / 2;  // column blocks of the first group
+    [[maybe_unused]] constexpr int WSZ = (C0 * 16 + 2) * 64;  // floats that a wavefront gives
     if constexpr (HV == 2) {
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the rings have been read
         float *const ex = reinterpret_cast<float *>(ring_s);
-        constexpr int WSZ = (C0 * 16 + 2) * 64;
         float *mine = ex + wave8 * WSZ + lane, *other = ex + (wave8 ^ 4) * WSZ + lane;
         const float l_mine = LM ? (upper ? lacc[1] : lacc[0]) : l_run;
         mine[0] = m_run;
@@ -440,15 +441,15 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
         if (half) take(C(), E(), mw, ow);
         else take(Z(), C(), mw, ow);
     }
-    // the column blocks that this wavefront stores
-    const int c_lo = HV == 2 && half ? C0 : 0, c_hi = HV == 2 && !half ? C0 : NCB;
 
     // ---- normalise and store: lane (n, hh) holds out[q = n][d = 32 c + 8 i + 4 hh + j] ----
     float l = l_run;
     if (LM && HV == 1) l = upper ? lacc[1] : lacc[0];
     if (!LM) l += __shfl_xor(l, 32);
-    if (!q_ok) return;
     if (nsplit > 1) {
+        if (!q_ok) return;
+        // the column blocks that this wavefront stores
+        const int c_lo = HV == 2 && half ? C0 : 0, c_hi = HV == 2 && !half ? C0 : NCB;
         float *part = a.workspace + (((size_t)bh * nsplit + item.split) * R + row) * (D + 2);
 #pragma unroll
         for (int c = 0; c < NCB; ++c)
@@ -461,19 +462,46 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
         }
         return;
     }
+    // Output rows go through LDS and leave it 16 bytes a lane, whole rows one behind the other.  (8 bytes a lane from the registers
+    // are 32 rows an instruction, of 16 bytes each: where keys are few the launch was one of such stores -- 16 prompts of 128,
+    // 32q/8kv x 128, bfloat16, the call 14.9 us for 12.3.)
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + ((size_t)bh * R + row) * D;
+    auto leave = [&](auto C_, auto N_, uint16_t *stage) __attribute__((always_inline)) {  // column blocks C .. C + N - 1
+        constexpr int C = decltype(C_)::value, N = decltype(N_)::value, W = 32 * (C + N) < D ? 32 * N : D - 32 * C;
+        constexpr int PITCH = W + 8, CPR = W / 8;  // 16-byte chunks of a row
 #pragma unroll
-    for (int c = 0; c < NCB; ++c)
+        for (int c = 0; c < N; ++c)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (32 * c + 8 * i < D && c >= c_lo && c < c_hi) {
-                const float o0 = oacc[c][4 * i] * inv, o1 = oacc[c][4 * i + 1] * inv, o2 = oacc[c][4 * i + 2] * inv, o3 = oacc[c][4 * i + 3] * inv;
-                uint2 w;
-                w.x = DT == 1 ? pk_bf2(o0, o1) : pk_h2(o0, o1);
-                w.y = DT == 1 ? pk_bf2(o2, o3) : pk_h2(o2, o3);
-                *reinterpret_cast<uint2 *>(op + 32 * c + 8 * i + 4 * hh) = w;
-            }
+            for (int i = 0; i < 4; ++i)
+                if (32 * c + 8 * i < W) {
+                    const f16v &o = oacc[C + c];
+                    const float o0 = o[4 * i] * inv, o1 = o[4 * i + 1] * inv, o2 = o[4 * i + 2] * inv, o3 = o[4 * i + 3] * inv;
+                    *reinterpret_cast<kv_u2 *>(stage + n * PITCH + 32 * c + 8 * i + 4 * hh) =
+                        DT == 1 ? kv_u2{pk_bf2(o0, o1), pk_bf2(o2, o3)} : kv_u2{pk_h2(o0, o1), pk_h2(o2, o3)};
+                }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (other lanes' columns: the order of the instructions is enough)
+        const int row0 = row - n;
+        uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + ((size_t)bh * R + row0) * D + 32 * C;
+#pragma unroll
+        for (int k = 0; k < (32 * CPR + 63) / 64; ++k) {
+            const int x = 64 * k + lane, rw = x / CPR, ch = x - rw * CPR;
+            if (((32 * CPR) % 64 == 0 || x < 32 * CPR) && row0 + rw < R)
+                *reinterpret_cast<out16 *>(op + rw * D + 8 * ch) = *reinterpret_cast<const kv_u4 *>(stage + rw * PITCH + 8 * ch);
+        }
+    };
+    using Z = std::integral_constant<int, 0>;
+    if constexpr (HV == 1) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the rings have been read
+        static_assert(4 * 32 * (D + 8) <= KSZ + VSZ, "room for every wavefront's rows");
+        leave(Z(), std::integral_constant<int, NCB>(), ring_s + wave * (32 * (D + 8)));
+    } else {
+        // (what the other group gave was for this wavefront alone, and it has read it)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        uint16_t *stage = reinterpret_cast<uint16_t *>(reinterpret_cast<float *>(ring_s) + (wave8 ^ 4) * WSZ);
+        static_assert(32 * (32 * C0 + 8) <= 2 * WSZ, "room for a wavefront's rows");
+        if (half) leave(std::integral_constant<int, C0>(), std::integral_constant<int, NCB - C0>(), stage);
+        else leave(Z(), std::integral_constant<int, C0>(), stage);
+    }
 }
 
 }  // namespace
