@@ -446,27 +446,53 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
     float l = l_run;
     if (LM && HV == 1) l = upper ? lacc[1] : lacc[0];
     if (!LM) l += __shfl_xor(l, 32);
+    // Both go through LDS, a wavefront's own part of it, and leave it 16 bytes a lane along the rows.
+    using Z = std::integral_constant<int, 0>;
+    using C = std::integral_constant<int, C0>;
+    using A = std::integral_constant<int, NCB>;
+    using E = std::integral_constant<int, NCB - C0>;
+    const int row0 = row - n;
+    uint16_t *stage;
+    if constexpr (HV == 1) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the rings have been read
+        static_assert(4 * 32 * (D + 8) <= KSZ + VSZ && 4 * 32 * 36 * 2 <= KSZ + VSZ, "room for every wavefront's rows");
+        stage = ring_s + wave * (32 * (D + 8 > 72 ? D + 8 : 72));
+    } else {
+        // (what the other group gave was for this wavefront alone, and it has read it)
+        static_assert(32 * (32 * C0 + 8) <= 2 * WSZ && 32 * 36 <= WSZ, "room for a wavefront's rows");
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        stage = reinterpret_cast<uint16_t *>(reinterpret_cast<float *>(ring_s) + (wave8 ^ 4) * WSZ);
+    }
     if (nsplit > 1) {
-        if (!q_ok) return;
-        // the column blocks that this wavefront stores
-        const int c_lo = HV == 2 && half ? C0 : 0, c_hi = HV == 2 && !half ? C0 : NCB;
-        float *part = a.workspace + (((size_t)bh * nsplit + item.split) * R + row) * (D + 2);
+        // (from the registers 32 rows an instruction, of 32 bytes each: one sequence's 1024 new rows over 2000 keys in seven parts,
+        // 8q/2kv x 128, 26.3 us the call for 24.2, and 25.8 on the tile before this one)
+        float *part = a.workspace + (((size_t)bh * nsplit + item.split) * R + row0) * (D + 2), *fs = reinterpret_cast<float *>(stage);
+        auto leave = [&](auto C_, auto N_) __attribute__((always_inline)) {  // column blocks C .. C + N - 1, one after the other
 #pragma unroll
-        for (int c = 0; c < NCB; ++c)
+            for (int c = decltype(C_)::value; c < decltype(C_)::value + decltype(N_)::value; ++c) {
+                const int W = 32 * c + 32 <= D ? 32 : 16, CPR = W / 4;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (32 * c + 8 * i < D && c >= c_lo && c < c_hi) *reinterpret_cast<kv_part4 *>(part + 32 * c + 8 * i + 4 * hh) = kv_part4{oacc[c][4 * i], oacc[c][4 * i + 1], oacc[c][4 * i + 2], oacc[c][4 * i + 3]};
-        if (hh == 0 && half == 0) {
-            part[D] = m_run * 0.6931471805599453f;  // back from the log2 domain
-            part[D + 1] = l;
-        }
+                for (int i = 0; i < W / 8; ++i)
+                    *reinterpret_cast<f4 *>(fs + n * 36 + 8 * i + 4 * hh) = f4{oacc[c][4 * i], oacc[c][4 * i + 1], oacc[c][4 * i + 2], oacc[c][4 * i + 3]};
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (other lanes' columns: the order of the instructions is enough)
+#pragma unroll
+                for (int k = 0; k < CPR / 2; ++k) {
+                    const int x = 64 * k + lane, rw = x / CPR, ch = x - rw * CPR;
+                    if (row0 + rw < R) *reinterpret_cast<kv_part4 *>(part + rw * (D + 2) + 32 * c + 4 * ch) = *reinterpret_cast<const f4 *>(fs + rw * 36 + 4 * ch);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+        };
+        if constexpr (HV == 1) leave(Z(), A());
+        else if (half) leave(C(), E());
+        else leave(Z(), C());
+        if (hh == 0 && half == 0 && q_ok) *reinterpret_cast<kv_f2 *>(part + n * (D + 2) + D) = kv_f2{m_run * 0.6931471805599453f, l};  // (the maximum back from the log2 domain)
         return;
     }
-    // Output rows go through LDS and leave it 16 bytes a lane, whole rows one behind the other.  (8 bytes a lane from the registers
-    // are 32 rows an instruction, of 16 bytes each: where keys are few the launch was one of such stores -- 16 prompts of 128,
-    // 32q/8kv x 128, bfloat16, the call 14.9 us for 12.3.)
+    // (8 bytes a lane from the registers are 32 rows an instruction, of 16 bytes each: where keys are few the launch was one of
+    // such stores -- 16 prompts of 128, 32q/8kv x 128, bfloat16, the call 14.9 us for 12.3)
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    auto leave = [&](auto C_, auto N_, uint16_t *stage) __attribute__((always_inline)) {  // column blocks C .. C + N - 1
+    auto leave = [&](auto C_, auto N_) __attribute__((always_inline)) {
         constexpr int C = decltype(C_)::value, N = decltype(N_)::value, W = 32 * (C + N) < D ? 32 * N : D - 32 * C;
         constexpr int PITCH = W + 8, CPR = W / 8;  // 16-byte chunks of a row
 #pragma unroll
@@ -479,8 +505,7 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
                     *reinterpret_cast<kv_u2 *>(stage + n * PITCH + 32 * c + 8 * i + 4 * hh) =
                         DT == 1 ? kv_u2{pk_bf2(o0, o1), pk_bf2(o2, o3)} : kv_u2{pk_h2(o0, o1), pk_h2(o2, o3)};
                 }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (other lanes' columns: the order of the instructions is enough)
-        const int row0 = row - n;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + ((size_t)bh * R + row0) * D + 32 * C;
 #pragma unroll
         for (int k = 0; k < (32 * CPR + 63) / 64; ++k) {
@@ -489,19 +514,9 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
                 *reinterpret_cast<out16 *>(op + rw * D + 8 * ch) = *reinterpret_cast<const kv_u4 *>(stage + rw * PITCH + 8 * ch);
         }
     };
-    using Z = std::integral_constant<int, 0>;
-    if constexpr (HV == 1) {
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the rings have been read
-        static_assert(4 * 32 * (D + 8) <= KSZ + VSZ, "room for every wavefront's rows");
-        leave(Z(), std::integral_constant<int, NCB>(), ring_s + wave * (32 * (D + 8)));
-    } else {
-        // (what the other group gave was for this wavefront alone, and it has read it)
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        uint16_t *stage = reinterpret_cast<uint16_t *>(reinterpret_cast<float *>(ring_s) + (wave8 ^ 4) * WSZ);
-        static_assert(32 * (32 * C0 + 8) <= 2 * WSZ, "room for a wavefront's rows");
-        if (half) leave(std::integral_constant<int, C0>(), std::integral_constant<int, NCB - C0>(), stage);
-        else leave(Z(), std::integral_constant<int, C0>(), stage);
-    }
+    if constexpr (HV == 1) leave(Z(), A());
+    else if (half) leave(C(), E());
+    else leave(Z(), C());
 }
 
 }  // namespace
