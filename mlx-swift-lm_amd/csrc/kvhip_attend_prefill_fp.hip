@@ -5,23 +5,17 @@
 // 192 with values of 128; more rows of head sizes up to 128: kvhip_attend_prefill_rows32.hip) and walks the cached keys in tiles of 32 slots:
 //   S^T   = K . Q^T      A = K rows from LDS in the cache's own dtype (no conversion),
 //                        B = query rows held in registers
-//   out^T += V^T . P^T   A = V^T rows from LDS as fp16 (bf16 is converted while staging),
-//                        B = the fp16 probabilities exactly where the S^T accumulators left
-//                        them, so P never moves between lanes
-// K/V tiles are double-buffered in LDS: while a tile is contracted, the next one (already in
-// registers) is written to the other buffer and the one after that is requested from global
-// memory, with a single barrier per tile.  Global reads and LDS writes of a tile are
-// chunk-interleaved over the 256 threads (consecutive lanes, consecutive 16 bytes), LDS rows
-// are padded so that both the writes and the operand reads are bank-conflict free.
+//   out^T += V^T . P^T   A = V^T rows from LDS in the cache's own dtype, B = the probabilities, rounded
+//                        to it, exactly where the S^T accumulators left them, so P never moves between lanes
+// K/V tiles are double-buffered in LDS and arrive there straight from global memory, K two tiles ahead of its use
+// and V one, with a single barrier per tile.  The interleaved page is made of the 16-byte chunks that the operands
+// want, so a buffer is the tile's chunks in page order, and its operand reads are bank-conflict free.
 // The online softmax rescales the accumulators only when a row maximum rises, and key tiles
 // that every query row of the workgroup sees completely skip all mask tests.
 #include "kvhip_prefill_fp.hpp"
 
 #ifndef KVHIP_PREFILL_LM
 #define KVHIP_PREFILL_LM 1
-#endif
-#ifndef KVHIP_PREFILL_BF16_P
-#define KVHIP_PREFILL_BF16_P 1
 #endif
 // how far ahead of their use the matrix-core operands are read from LDS
 #ifndef KVHIP_PF_VG
@@ -43,19 +37,8 @@ namespace {
 
 using namespace prefill_fp;
 
-
 __device__ __forceinline__ uint32_t rn_h2(float lo, float hi) { return pk_h2(lo, hi); }    // round to nearest even
 __device__ __forceinline__ uint32_t rn_bf2(float lo, float hi) { return pk_bf2(lo, hi); }
-// the probabilities of one lane as the PV operand: fp16, or bf16 for bf16 caches on the direct path
-template <bool BF> __device__ __forceinline__ u4 pack_p(const float (&p)[2][4]) {
-    if constexpr (BF) return u4{rn_bf2(p[0][0], p[0][1]), rn_bf2(p[0][2], p[0][3]), rn_bf2(p[1][0], p[1][1]), rn_bf2(p[1][2], p[1][3])};
-    else return u4{rn_h2(p[0][0], p[0][1]), rn_h2(p[0][2], p[0][3]), rn_h2(p[1][0], p[1][1]), rn_h2(p[1][2], p[1][3])};
-}
-// two bf16 (one dword) -> two fp16, exact for every bf16 inside the fp16 range
-__device__ __forceinline__ uint32_t bf2_to_h2(uint32_t w) {
-    return rn_h2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
-}
-
 // c += a . b and c = a . b on the matrix cores.  DT: 0 fp16 operands, 1 bf16 operands.
 template <int DT> __device__ __forceinline__ void mfma_acc(f4 &c, const Op8 &a, const Op8 &b) {
     if constexpr (DT == 0) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.h, b.h, c, 0, 0, 0);
@@ -65,9 +48,9 @@ template <int DT> __device__ __forceinline__ void mfma_new(f4 &c, const Op8 &a, 
     c = f4{0.f, 0.f, 0.f, 0.f};
     mfma_acc<DT>(c, a, b);
 }
-// D = 256 runs 64 query rows per workgroup only: 128 rows need the accumulator registers of
-// a whole SIMD lane (one wavefront per SIMD), which measured slower (0.34 ms against 0.29 ms
-// for a 512 x 4607 chunk at B4, 8 query heads).
+// 16 query rows per wavefront.  (32 at D = 256 need the accumulator registers of
+// a whole SIMD lane, one wavefront per SIMD, which measured slower: 0.34 ms against 0.29 ms
+// for a 512 x 4607 chunk at B4, 8 query heads.)
 //
 // The loop is software-pipelined over the key tiles: iteration t issues S^T(t+1) = K(t+1) Q^T on
 // the matrix cores and, between those instructions, the vector-ALU half of the softmax of tile t
@@ -82,8 +65,7 @@ template <int DT> __device__ __forceinline__ void mfma_new(f4 &c, const Op8 &a, 
 template <int DK, int DV, int DT, bool IDENT, int MM>
 __global__ void __launch_bounds__(256, 2)
 prefill_fp_kernel(AttendArgs a, int nsplit) {
-    constexpr int QT = 1;  // blocks of 16 query rows per wavefront
-    constexpr int BM = 64 * QT;
+    constexpr int BM = 64;
     constexpr int S = (DK + 31) / 32;  // contraction steps over the head dim (the last one partly zero at D = 80)
     constexpr int NDT = DV / 16;   // 16-row tiles of out^T
     constexpr int NCK = (DK + 63) / 64, NCV = (DV + 63) / 64;  // rounds of 256 16-byte chunks, for K and for V
@@ -120,7 +102,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     const int blk_x = item.block, bh = item.bh;
     const int b = MM == 0 ? 0 : bh / a.Hkv;  // (without a mask nothing asks for it)
     [[maybe_unused]] const int hk = bh - b * a.Hkv;
-    const int row0 = blk_x * BM + wave * 16 * QT;  // first query row of this wavefront
+    const int row = blk_x * BM + wave * 16 + n;  // this lane's query row
     const SymMask sym = sym_mask_init(a.mask, b, a.L, a.T);
     // Scores enter the softmax as exp2(s * ef - m) with ef = |scale| log2 e > 0 -- a negative scale
     // flips the sign of the query operands instead (exact), a zero one becomes a vanishing positive
@@ -136,36 +118,27 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     const float ef = MM == 2 ? 1.f : sl2;
 
     // ---- query operands: B of S^T = K . Q^T; lane (n, jj) holds q[row][32 s + 8 jj ..] raw ----
-    Op8 qop[QT][S];
-    int q_l[QT] = {}, q_h[QT] = {};
-    bool q_ok[QT];
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-        const int i = row0 + 16 * qt + n;
-        q_ok[qt] = i < R;
+    Op8 qop[S];
+    const bool q_ok = row < R;
+    int q_l = 0, q_h = 0;
+    {
         // (a pair's query rows lie one behind the other; which positions they are is worked out behind the first requests)
-        const u4 *qp = reinterpret_cast<const u4 *>(reinterpret_cast<const uint16_t *>(a.q) + ((size_t)bh * R + i) * DK + 8 * jj);
+        const u4 *qp = reinterpret_cast<const u4 *>(reinterpret_cast<const uint16_t *>(a.q) + ((size_t)bh * R + row) * DK + 8 * jj);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            u4 w = (q_ok[qt] && (DK % 32 == 0 || 32 * s + 8 * jj < DK)) ? qp[4 * s] : u4{0, 0, 0, 0};
+            u4 w = (q_ok && (DK % 32 == 0 || 32 * s + 8 * jj < DK)) ? qp[4 * s] : u4{0, 0, 0, 0};
             if (flip) w ^= u4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
-            qop[qt][s].v = w;
+            qop[s].v = w;
         }
     }
 
-    f4 oacc[QT][NDT];
-    float m_run[QT], l_run[QT];
-    f4 lacc[LM ? QT : 1];
+    f4 oacc[NDT];
+    float m_run = -INFINITY, l_run = 0.f;
+    [[maybe_unused]] f4 lacc = f4{0.f, 0.f, 0.f, 0.f};
     Op8 ones;
     ones.v = u4{0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u};
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-        m_run[qt] = -INFINITY;
-        l_run[qt] = 0.f;
-        if (LM) lacc[LM ? qt : 0] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) oacc[qt][dt] = f4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int dt = 0; dt < NDT; ++dt) oacc[dt] = f4{0.f, 0.f, 0.f, 0.f};
 
     // ---- key tiles this workgroup has to visit, and the rows all of its queries keep ---------
     const Visit visit = visit_plan<BM, MM, IDENT>(a, sym, blk_x, R, item.split, nsplit, visit_s);
@@ -200,12 +173,12 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         if (wave == (tile & 3) && lane < BN) {  // the wavefronts take this in turn
             const int pos = lane;
             const int slot = slot0 + 8 * ((pos & 15) >> 2) + 4 * (pos >> 4) + (pos & 3);
-            int row;
-            if (IDENT) row = slot;
-            else row = slot < a.slots ? slot_to_row(a.runs, slot) : -1;
-            row = (row >= 0 && row < a.T) ? row : -1;
-            rows_s[par][pos] = row;  // the row of the token in K slot `pos`
-            const bool full = __all(row >= keep_lo && row <= keep_hi);  // (the 32 active lanes)
+            int key;
+            if (IDENT) key = slot;
+            else key = slot < a.slots ? slot_to_row(a.runs, slot) : -1;
+            key = (key >= 0 && key < a.T) ? key : -1;
+            rows_s[par][pos] = key;  // the row of the token in K slot `pos`
+            const bool full = __all(key >= keep_lo && key <= keep_hi);  // (the 32 active lanes)
             if (lane == 0) full_s[par] = full;
         }
         const int t = slot0 & (PAGE - 1);
@@ -230,7 +203,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     };
     auto wait_all_loads = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
-    // ---- S^T = K . Q^T of one tile: acc[qt][mt] rows = tokens 16 mt + 4 jj + i, column = query n -----
+    // ---- S^T = K . Q^T of one tile: acc[mt] rows = tokens 16 mt + 4 jj + i, column = query n -----
     // operand reads: K slot (chunk 4 s + jj, position 16 mt + n)
     auto read_k = [&](int par, int s, Op8 (&ka)[2]) __attribute__((always_inline)) {
 #pragma unroll
@@ -241,11 +214,11 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     // ---- mask of a tile whose scores are in `sc` (raw): excluded keys become -inf; under an array
     // mask the scores are scaled here and additive terms added -----------------------------------
     // An index-only mask (causal, window, per-batch lengths and left padding) keeps, for one query, an
-    // interval of key rows: [q_lo, q_lo + q_span] per query block of this lane (empty for a query row
+    // interval of key rows: [q_lo, q_lo + q_span] for the query of this lane (empty for a query row
     // past the end), tested with one unsigned comparison per key.
-    [[maybe_unused]] int q_lo[QT];
-    [[maybe_unused]] uint32_t q_span[QT];
-    auto apply_mask = [&](int par, f4 (&sc)[QT][2]) __attribute__((always_inline)) {
+    [[maybe_unused]] int q_lo = 0;
+    [[maybe_unused]] uint32_t q_span = 0;
+    auto apply_mask = [&](int par, f4 (&sc)[2]) __attribute__((always_inline)) {
         int trow[2][4];
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
@@ -253,57 +226,46 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
             for (int i = 0; i < 4; ++i) trow[mt][i] = rows_s[par][16 * mt + 4 * jj + i];  // by K slot; -1: no row
         if constexpr (MM != 2) {
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
+            for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        bool keep;
-                        if constexpr (MM == 1) keep = (uint32_t)(trow[mt][i] - q_lo[qt]) <= q_span[qt];
-                        else keep = trow[mt][i] >= 0 && q_ok[qt];
-                        sc[qt][mt][i] = keep ? sc[qt][mt][i] : -INFINITY;
-                    }
-            return;
-        }
-        // a boolean array mask is read four keys at a time where this lane's four rows are consecutive
-        [[maybe_unused]] bool vec_ok[2] = {false, false};
-        if constexpr (MM == 2) {
+                for (int i = 0; i < 4; ++i) {
+                    bool keep;
+                    if constexpr (MM == 1) keep = (uint32_t)(trow[mt][i] - q_lo) <= q_span;
+                    else keep = trow[mt][i] >= 0 && q_ok;
+                    sc[mt][i] = keep ? sc[mt][i] : -INFINITY;
+                }
+        } else {
+            // a boolean array mask is read four keys at a time where this lane's four rows are consecutive
+            bool vec_ok[2];
+            uint32_t mword[2] = {0u, 0u};
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt)
                 vec_ok[mt] = a.mask.dtype == KVHIP_BOOL && trow[mt][0] >= 0 && trow[mt][3] == trow[mt][0] + 3 &&
                              trow[mt][1] == trow[mt][0] + 1 && trow[mt][2] == trow[mt][0] + 2;
-        }
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            [[maybe_unused]] uint32_t mword[2] = {0u, 0u};
-            if constexpr (MM == 2) {
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-                    if (vec_ok[mt] && q_ok[qt]) {
-                        uint32_t w[1];
-                        mask_bool_words<1>(a.mask, b, q_h[qt], q_l[qt], trow[mt][0], w);
-                        mword[mt] = w[0];
-                    }
-            }
+            for (int mt = 0; mt < 2; ++mt)
+                if (vec_ok[mt] && q_ok) {
+                    uint32_t w[1];
+                    mask_bool_words<1>(a.mask, b, q_h, q_l, trow[mt][0], w);
+                    mword[mt] = w[0];
+                }
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    float x_ = sc[qt][mt][i] * sl2;
-                    const int row = trow[mt][i];
-                    bool keep = row >= 0 && q_ok[qt];
-                    if constexpr (MM == 2) {
-                        if (keep) {
-                            if (vec_ok[mt]) {
-                                keep = ((mword[mt] >> (8 * i)) & 0xffu) != 0u;
-                            } else {
-                                float add;
-                                keep = mask_keep(a.mask, b, q_h[qt], q_l[qt], row, a.L, a.T, add);
-                                x_ += add * LOG2E;
-                            }
+                    float x_ = sc[mt][i] * sl2;
+                    const int key = trow[mt][i];
+                    bool keep = key >= 0 && q_ok;
+                    if (keep) {
+                        if (vec_ok[mt]) {
+                            keep = ((mword[mt] >> (8 * i)) & 0xffu) != 0u;
+                        } else {
+                            float add;
+                            keep = mask_keep(a.mask, b, q_h, q_l, key, a.L, a.T, add);
+                            x_ += add * LOG2E;
                         }
                     }
-                    sc[qt][mt][i] = keep ? x_ : -INFINITY;
+                    sc[mt][i] = keep ? x_ : -INFINITY;
                 }
         }
     };
@@ -314,26 +276,26 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     // the maximum seen) only when a score exceeds it by more than RAISE, so p stays below 2^RAISE
     // (exact in fp16, whose relative precision does not depend on magnitude) and the accumulators are
     // rescaled a handful of times per query, not on every tile that happens to hold a new maximum.
-    auto raise = [&](int qt, float tmax) __attribute__((always_inline)) {
+    auto raise = [&](float tmax) __attribute__((always_inline)) {
         tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float mn = fmaxf(m_run[qt], tmax);
-        const float alpha = (mn == -INFINITY) ? 1.f : exp2_fast(m_run[qt] - mn);
-        m_run[qt] = mn;
+        const float mn = fmaxf(m_run, tmax);
+        const float alpha = (mn == -INFINITY) ? 1.f : exp2_fast(m_run - mn);
+        m_run = mn;
         if constexpr (LM) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) lacc[LM ? qt : 0][i] *= alpha;
+            for (int i = 0; i < 4; ++i) lacc[i] *= alpha;
         } else {
-            l_run[qt] *= alpha;
+            l_run *= alpha;
         }
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) oacc[qt][dt][i] *= alpha;
+            for (int i = 0; i < 4; ++i) oacc[dt][i] *= alpha;
     };
-    auto tile_max = [&](const f4 (&sc)[QT][2], int qt) __attribute__((always_inline)) -> float {
-        return ef * fmaxf(fmaxf(fmaxf(sc[qt][0][0], sc[qt][0][1]), fmaxf(sc[qt][0][2], sc[qt][0][3])),
-                          fmaxf(fmaxf(sc[qt][1][0], sc[qt][1][1]), fmaxf(sc[qt][1][2], sc[qt][1][3])));
+    auto tile_max = [&](const f4 (&sc)[2]) __attribute__((always_inline)) -> float {
+        return ef * fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
+                          fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
     };
     // The same maximum in four instructions, for the end of an iteration.  `fmaxf` on values the compiler has not
     // seen an arithmetic instruction produce (matrix-core results, selects) first quiets each operand with a
@@ -341,28 +303,22 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     // barrier.  Written as assembly, which the compiler's hazard handling does not look into: the caller keeps it
     // behind a scheduling barrier that follows the out^T matrix-core instructions, so the score registers, written
     // by matrix-core instructions a whole block earlier (or by the mask's selects), are long complete.
-    auto tile_max_raw = [&](const f4 (&sc)[QT][2], int qt) __attribute__((always_inline)) -> float {
+    auto tile_max_raw = [&](const f4 (&sc)[2]) __attribute__((always_inline)) -> float {
         float m;  // (one statement per instruction: the result may then share a register with a finished operand)
-        asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(sc[qt][0][0]), "v"(sc[qt][0][1]), "v"(sc[qt][0][2]));
-        asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(m), "v"(sc[qt][0][3]), "v"(sc[qt][1][0]));
-        asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(m), "v"(sc[qt][1][1]), "v"(sc[qt][1][2]));
-        asm volatile("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m), "v"(sc[qt][1][3]));
+        asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(sc[0][0]), "v"(sc[0][1]), "v"(sc[0][2]));
+        asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(m), "v"(sc[0][3]), "v"(sc[1][0]));
+        asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(m), "v"(sc[1][1]), "v"(sc[1][2]));
+        asm volatile("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m), "v"(sc[1][3]));
         return ef * m;
     };
     // whether the tile whose scores are in `sc` exceeds some query's reference maximum by more than
     // RAISE (wavefront-uniform; a handful of times per query)
-    auto needs_raise = [&](const f4 (&sc)[QT][2]) __attribute__((always_inline)) -> bool {
-        bool need = false;
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) need = need || tile_max_raw(sc, qt) > m_run[qt] + RAISE;
-        return __any(need);
+    auto needs_raise = [&](const f4 (&sc)[2]) __attribute__((always_inline)) -> bool {
+        return __any(tile_max_raw(sc) > m_run + RAISE);
     };
-    auto do_raise = [&](const f4 (&sc)[QT][2]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            const float tmax = tile_max(sc, qt);
-            if (__any(tmax > m_run[qt] + RAISE)) raise(qt, tmax);
-        }
+    auto do_raise = [&](const f4 (&sc)[2]) __attribute__((always_inline)) {
+        const float tmax = tile_max(sc);
+        if (__any(tmax > m_run + RAISE)) raise(tmax);
     };
 
     // ---- one iteration: tile `tile` (parity PAR) has its scores in `sc`; `sn` receives tile + 1's ---
@@ -372,9 +328,9 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     // The iteration itself never touches the reference maxima or rescales the accumulators: it only
     // reports (`need`) that tile + 1 calls for it, and the loop below leaves its fast part to do so.
     // With the rescaling inside the fast loop the compiler joined the rescaled and the untouched
-    // accumulators through register copies on the path that does not rescale: 36 moves per query block
-    // and tile, and spills.
-    auto body = [&](auto HAS_NEXT_, auto PAR_, auto MASKED_, int tile, f4 (&sc)[QT][2], f4 (&sn)[QT][2], bool &need) __attribute__((always_inline)) {
+    // accumulators through register copies on the path that does not rescale: 36 moves per tile at two
+    // blocks of 16 query rows, and spills.
+    auto body = [&](auto HAS_NEXT_, auto PAR_, auto MASKED_, int tile, f4 (&sc)[2], f4 (&sn)[2], bool &need) __attribute__((always_inline)) {
         constexpr bool HAS_NEXT = decltype(HAS_NEXT_)::value;
         constexpr int PAR = decltype(PAR_)::value;
         constexpr bool MASKED = decltype(MASKED_)::value;
@@ -382,23 +338,22 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         if (tile + 2 < v_hi) dma_k(vt_of(tile + 2), PAR);  // (`tile`: the position in the visiting order)
         if constexpr (HAS_NEXT) dma_v(vt_of(tile + 1), PAR ^ 1);
 
-        float negmu[QT], pr[QT][2][4];
-        Op8 pb[QT];
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) negmu[qt] = (m_run[qt] == -INFINITY) ? 0.f : -m_run[qt];
-        // probability `idx` of this lane: query block idx / 8, accumulator idx % 8
+        float pr[2][4];
+        Op8 pb;
+        const float negmu = (m_run == -INFINITY) ? 0.f : -m_run;
+        // probability `idx` of this lane: accumulator idx
         // (the rounding of a pair of probabilities to 16 bits trails their exp2 by two probabilities, so
         // that it does not wait for a result just asked for)
         auto round_pair = [&](int idx) __attribute__((always_inline)) {  // idx: the odd member of the pair
-            const int qt = idx >> 3, mt = (idx >> 2) & 1, i = idx & 3;
-            const float p0 = pr[qt][mt][i - 1], p1 = pr[qt][mt][i];
-            if constexpr (!LM) l_run[qt] += p0 + p1;
-            pb[qt].v[2 * mt + (i >> 1)] = DT == 1 ? rn_bf2(p0, p1) : rn_h2(p0, p1);
+            const int mt = idx >> 2, i = idx & 3;
+            const float p0 = pr[mt][i - 1], p1 = pr[mt][i];
+            if constexpr (!LM) l_run += p0 + p1;
+            pb.v[2 * mt + (i >> 1)] = DT == 1 ? rn_bf2(p0, p1) : rn_h2(p0, p1);
         };
-        constexpr int NP = 8 * QT;      // probabilities per lane and tile
+        constexpr int NP = 8;  // probabilities per lane and tile
         auto softmax_slice = [&](int idx) __attribute__((always_inline)) {
-            const int qt = idx >> 3, mt = (idx >> 2) & 1, i = idx & 3;
-            pr[qt][mt][i] = exp2_fast(__builtin_fmaf(sc[qt][mt][i], ef, negmu[qt]));  // exp2(-inf) = 0 for excluded keys
+            const int mt = idx >> 2, i = idx & 3;
+            pr[mt][i] = exp2_fast(__builtin_fmaf(sc[mt][i], ef, negmu));  // exp2(-inf) = 0 for excluded keys
             if ((idx & 1) && idx >= 3) round_pair(idx - 2);
             if (idx == NP - 1) round_pair(idx);
         };
@@ -414,7 +369,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
                     dst[x].v = *reinterpret_cast<const u4 *>(&Vs(PAR)[(jj * DV + 16 * (VG * g + x) + n) * 8]);
         };
         if constexpr (HAS_NEXT) {
-            constexpr int NM = 2 * S * QT;  // matrix-core instructions of the next tile's scores
+            constexpr int NM = 2 * S;  // matrix-core instructions of the next tile's scores
             // K operands are asked for AHEAD contraction steps ahead, V's first group near the end
             constexpr int AHEAD = KVHIP_PF_AHEAD;
             constexpr int KA = S < AHEAD + 1 ? S : AHEAD + 1;
@@ -424,15 +379,15 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
             KV_SB;
 #pragma unroll
             for (int k = 0; k < NM; ++k) {
-                // 2 QT independent accumulator chains, taken in turn
-                const int s = k / (2 * QT), mt = (k / QT) & 1, qt = k % QT;
-                if (k % (2 * QT) == 0 && s + AHEAD < S) read_k(PAR ^ 1, s + AHEAD, ka[(s + AHEAD) % KA]);
-                if (k == (NM > 2 * QT ? NM - 2 * QT : 0)) {
+                // two independent accumulator chains, taken in turn
+                const int s = k / 2, mt = k & 1;
+                if (mt == 0 && s + AHEAD < S) read_k(PAR ^ 1, s + AHEAD, ka[(s + AHEAD) % KA]);
+                if (k == NM - 2) {
 #pragma unroll
                     for (int g = 0; g < NVB - 1 && g < NG; ++g) read_v(g, va[g]);
                 }
-                if (s == 0) mfma_new<DT>(sn[qt][mt], ka[s % KA][mt], qop[qt][s]);
-                else mfma_acc<DT>(sn[qt][mt], ka[s % KA][mt], qop[qt][s]);
+                if (s == 0) mfma_new<DT>(sn[mt], ka[s % KA][mt], qop[s]);
+                else mfma_acc<DT>(sn[mt], ka[s % KA][mt], qop[s]);
 #pragma unroll
                 for (int idx = k * NP / NM; idx < (k + 1) * NP / NM; ++idx) softmax_slice(idx);
                 KV_SB;
@@ -445,21 +400,13 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         }
 
         // ---- out^T += V^T . P^T: A = V^T chunks from LDS, B = the probabilities where they are ----
-        if constexpr (LM) {
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
-                mfma_acc<0>(lacc[LM ? qt : 0], ones, pb[qt]);
-        }
+        if constexpr (LM) mfma_acc<0>(lacc, ones, pb);
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
             if (g + NVB - 1 < NG) read_v(g + NVB - 1, va[(g + NVB - 1) % NVB]);
 #pragma unroll
             for (int x = 0; x < VG; ++x)
-                if (VG * g + x < NDT) {
-#pragma unroll
-                    for (int qt = 0; qt < QT; ++qt)
-                        mfma_acc<DT>(oacc[qt][VG * g + x], va[g % NVB][x], pb[qt]);
-                }
+                if (VG * g + x < NDT) mfma_acc<DT>(oacc[VG * g + x], va[g % NVB][x], pb);
         }
 
         need = false;
@@ -482,33 +429,26 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         if (v_lo + 1 < v_hi) dma_k(vt_of(v_lo + 1), 1);
     }
     if constexpr (MM != 0) {
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            const int i = row0 + 16 * qt + n, rep = q_ok[qt] ? i / a.L : 0;
-            q_l[qt] = q_ok[qt] ? i - rep * a.L : 0;
-            q_h[qt] = hk * r + rep;
-        }
+        const int rep = q_ok ? row / a.L : 0;
+        q_l = q_ok ? row - rep * a.L : 0;
+        q_h = hk * r + rep;
     }
     if constexpr (MM == 1) {
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            int lo, hi;
-            if (sym.mode == KVHIP_MASK_CAUSAL) {
-                lo = 0;
-                hi = a.T - a.L + q_l[qt];
-            } else {
-                const int li = sym.offset + q_l[qt];
-                lo = sym.pad_b;
-                hi = min(li, sym.len_b - 1);
-                if (sym.window > 0) lo = max(lo, li - sym.window + 1);
-            }
-            lo = max(lo, 0);
-            hi = min(hi, a.T - 1);
-            const bool any = q_ok[qt] && hi >= lo;
-            q_lo[qt] = any ? lo : 0;
-            q_span[qt] = any ? (uint32_t)(hi - lo) : 0u;
-            if (!any) q_lo[qt] = 0x40000000;  // no row reaches it: row - q_lo wraps to a huge unsigned value
+        int lo, hi;
+        if (sym.mode == KVHIP_MASK_CAUSAL) {
+            lo = 0;
+            hi = a.T - a.L + q_l;
+        } else {
+            const int li = sym.offset + q_l;
+            lo = sym.pad_b;
+            hi = min(li, sym.len_b - 1);
+            if (sym.window > 0) lo = max(lo, li - sym.window + 1);
         }
+        lo = max(lo, 0);
+        hi = min(hi, a.T - 1);
+        const bool any = q_ok && hi >= lo;
+        q_lo = any ? lo : 0x40000000;  // (none: no row reaches it, row - q_lo wraps to a huge unsigned value)
+        q_span = any ? (uint32_t)(hi - lo) : 0u;
     }
     wait_all_loads();
     // (the same wait once more in a form the compiler's bookkeeping sees: it then knows that the
@@ -517,19 +457,17 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), others untouched
     __syncthreads();
     if (v_lo < v_hi) {
-        f4 sa[QT][2], sb[QT][2];
+        f4 sa[2], sb[2];
         {  // scores of the first tile
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 Op8 ka[2];
                 read_k(0, s, ka);
 #pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                    for (int qt = 0; qt < QT; ++qt) {
-                        if (s == 0) mfma_new<DT>(sa[qt][mt], ka[mt], qop[qt][s]);
-                        else mfma_acc<DT>(sa[qt][mt], ka[mt], qop[qt][s]);
-                    }
+                for (int mt = 0; mt < 2; ++mt) {
+                    if (s == 0) mfma_new<DT>(sa[mt], ka[mt], qop[s]);
+                    else mfma_acc<DT>(sa[mt], ka[mt], qop[s]);
+                }
             }
             if (MM == 2 || full_s[0] == 0) apply_mask(0, sa);
             do_raise(sa);
@@ -541,7 +479,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         using P1 = std::integral_constant<int, 1>;
         int tile = v_lo;  // position in the visiting order
         // one iteration with the variant chosen at run time; false after the last tile
-        auto iterate = [&](auto PAR_, f4 (&sc)[QT][2], f4 (&sn)[QT][2], bool &need) __attribute__((always_inline)) -> bool {
+        auto iterate = [&](auto PAR_, f4 (&sc)[2], f4 (&sn)[2], bool &need) __attribute__((always_inline)) -> bool {
             constexpr int PAR = decltype(PAR_)::value;
             const bool has_next = tile + 1 < v_hi;
             // whether tile + 1 needs its mask evaluated (workgroup-uniform): with slots in presented
@@ -587,43 +525,39 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     }
 
     // ---- normalise and store: lane (n, jj) holds out[q = n][d = 16 dt + 4 jj + i] ------------
+    float l = l_run;
+    if constexpr (LM) {
+        l = lacc[0];
+    } else {
+        l += __shfl_xor(l, 16);
+        l += __shfl_xor(l, 32);
+    }
+    if (!q_ok) return;
+    if (nsplit > 1) {
+        float *part = a.workspace + (((size_t)bh * nsplit + item.split) * R + row) * (DV + 2);
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-        float l = l_run[qt];
-        if constexpr (LM) {
-            l = lacc[LM ? qt : 0][0];
+        for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<kv_part4 *>(part + 16 * dt + 4 * jj) = oacc[dt];
+        if (jj == 0) {
+            part[DV] = m_run * 0.6931471805599453f;  // back from the log2 domain
+            part[DV + 1] = l;
+        }
+        return;
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + ((size_t)bh * R + row) * DV;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+        const float o0 = oacc[dt][0] * inv, o1 = oacc[dt][1] * inv;
+        const float o2 = oacc[dt][2] * inv, o3 = oacc[dt][3] * inv;
+        uint2 w;
+        if (DT == 0) {
+            w.x = rn_h2(o0, o1);
+            w.y = rn_h2(o2, o3);
         } else {
-            l += __shfl_xor(l, 16);
-            l += __shfl_xor(l, 32);
+            w.x = rn_bf2(o0, o1);
+            w.y = rn_bf2(o2, o3);
         }
-        if (!q_ok[qt]) continue;
-        if (nsplit > 1) {
-            const int i = row0 + 16 * qt + n;
-            float *part = a.workspace + (((size_t)bh * nsplit + item.split) * R + i) * (DV + 2);
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<kv_part4 *>(part + 16 * dt + 4 * jj) = oacc[qt][dt];
-            if (jj == 0) {
-                part[DV] = m_run[qt] * 0.6931471805599453f;  // back from the log2 domain
-                part[DV + 1] = l;
-            }
-            continue;
-        }
-        const float inv = l > 0.f ? 1.0f / l : 0.f;
-        const size_t ooff = ((size_t)bh * R + row0 + 16 * qt + n) * DV;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-            const float o0 = oacc[qt][dt][0] * inv, o1 = oacc[qt][dt][1] * inv;
-            const float o2 = oacc[qt][dt][2] * inv, o3 = oacc[qt][dt][3] * inv;
-            uint2 w;
-            if (DT == 0) {
-                w.x = rn_h2(o0, o1);
-                w.y = rn_h2(o2, o3);
-            } else {
-                w.x = rn_bf2(o0, o1);
-                w.y = rn_bf2(o2, o3);
-            }
-            *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(a.out) + ooff + 16 * dt + 4 * jj) = w;
-        }
+        *reinterpret_cast<uint2 *>(op + 16 * dt + 4 * jj) = w;
     }
 }
 
