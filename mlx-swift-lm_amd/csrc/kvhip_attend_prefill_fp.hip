@@ -126,9 +126,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         const u4 *qp = reinterpret_cast<const u4 *>(reinterpret_cast<const uint16_t *>(a.q) + ((size_t)bh * R + row) * DK + 8 * jj);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            u4 w = (q_ok && (DK % 32 == 0 || 32 * s + 8 * jj < DK)) ? qp[4 * s] : u4{0, 0, 0, 0};
-            if (flip) w ^= u4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
-            qop[s].v = w;
+            qop[s].v = (q_ok && (DK % 32 == 0 || 32 * s + 8 * jj < DK)) ? qp[4 * s] : u4{0, 0, 0, 0};
         }
     }
 
@@ -427,6 +425,11 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
         dma_k(vt_of(v_lo), 0);
         dma_v(vt_of(v_lo), 0);
         if (v_lo + 1 < v_hi) dma_k(vt_of(v_lo + 1), 1);
+    }
+    // (behind the requests: a sign flipped as the queries are loaded put a wait for them in front of the first keys' request)
+    if (flip) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) qop[s].v ^= u4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
     }
     if constexpr (MM != 0) {
         const int rep = q_ok ? row / a.L : 0;
