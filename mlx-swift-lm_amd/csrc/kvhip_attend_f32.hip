@@ -41,8 +41,10 @@ constexpr int query_tiles(int dk) { return dk <= 128 ? 2 : 1; }
 // A single-token step without a mask: the wavefront that reads the new row's tile writes the row after it has requested
 // its first tile -- and if that is the row's tile, puts the row into its registers too --, and ROT turns the query rows and
 // the new key row in LDS first, as the decode kernels do.  A launch that appends takes 4.2 us.
-// TB: token blocks of 16 per tile.
-template <int DK, int DV, int QT, int TB, int ARR, bool ROT>
+// TB: token blocks of 16 per tile.  ONE: it may be a single token (head sizes above 128, where prompt chunks take one query tile
+// too, have an instance of its own for it): what only a token needs is not in the loop of prompt chunks, where it cost them 1 to
+// 2 % (16q/4kv x 64, 512 rows over 2048 keys 52.5 us for 51.5, over 6000 133.9 for 132.2; 192 / 128 103.8 for 102.2).
+template <int DK, int DV, int QT, int TB, int ARR, bool ROT, bool ONE>
 __global__ void __launch_bounds__(256, 2)
 attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_total, int nparts) {
     constexpr int WT = 16 * TB;
@@ -73,7 +75,7 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_tot
     const int tb = min(t_lo + part * per, t_hi), te = min(tb + per, t_hi);
 
     // ---- a step's rows ----------------------------------------------------------------------------------------
-    constexpr bool STEP = QT == 1 && ARR == 0;  // (up to 16 query rows: one row block)
+    constexpr bool STEP = QT == 1 && ARR == 0 && ONE;  // (up to 16 query rows: one row block)
     // (behind a wavefront's last tile, often a step's only one, the tile is not requested again; long loops keep their requests
     // in front of no branch)
     constexpr bool BRANCH = STEP && !QL;
@@ -330,7 +332,7 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_tot
                         for (int j = 0; j < 4; ++j) s[qt][x][j] += add[j];
                     }
                 }
-            } else if (ARR == 0 && rb.one && ident) {  // one token: every row sees keys.lo to keys.hi
+            } else if (ARR == 0 && ONE && rb.one && ident) {  // one token: every row sees keys.lo to keys.hi
                 if (!full) {
 #pragma unroll
                     for (int x = 0; x < TB; ++x)
@@ -476,15 +478,23 @@ template <int DK, int DV, int QT, int TB>
 hipError_t launch_instance(const AttendArgs &a, const PlanF32 &p, hipStream_t s) {
     const dim3 grid(p.row_blocks, a.st.BH, p.nparts), block(256);
     const size_t lds = MW * QT * (DV / 16) * 64 * sizeof(f4);
+    const int r = a.Hq / a.Hkv;
     if constexpr (QT == 1) {
         if (a.new_k && a.rope) {
-            hipLaunchKernelGGL((attend_f32_kernel<DK, DV, 1, TB, 0, true>), grid, block, lds, s, AttendStepArgs(a), a.Hq / a.Hkv, p.tiles, p.nparts);
+            hipLaunchKernelGGL((attend_f32_kernel<DK, DV, 1, TB, 0, true, true>), grid, block, lds, s, AttendStepArgs(a), r, p.tiles, p.nparts);
+            return hipGetLastError();
+        }
+        if ((DK <= 128 || a.L == 1) && a.mask.mode != KVHIP_MASK_ARRAY) {
+            hipLaunchKernelGGL((attend_f32_kernel<DK, DV, 1, TB, 0, false, true>), grid, block, lds, s, a, r, p.tiles, p.nparts);
             return hipGetLastError();
         }
     }
-    if (a.mask.mode != KVHIP_MASK_ARRAY) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 0, false>), grid, block, lds, s, a, a.Hq / a.Hkv, p.tiles, p.nparts);
-    else if (a.mask.dtype == KVHIP_BOOL) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 1, false>), grid, block, lds, s, a, a.Hq / a.Hkv, p.tiles, p.nparts);
-    else hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 2, false>), grid, block, lds, s, a, a.Hq / a.Hkv, p.tiles, p.nparts);
+    if (a.mask.mode == KVHIP_MASK_ARRAY) {
+        if (a.mask.dtype == KVHIP_BOOL) hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 1, false, false>), grid, block, lds, s, a, r, p.tiles, p.nparts);
+        else hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 2, false, false>), grid, block, lds, s, a, r, p.tiles, p.nparts);
+    } else if constexpr (QT > 1 || DK > 128) {
+        hipLaunchKernelGGL((attend_f32_kernel<DK, DV, QT, TB, 0, false, false>), grid, block, lds, s, a, r, p.tiles, p.nparts);
+    }
     return hipGetLastError();
 }
 
