@@ -101,3 +101,35 @@ def test_infinite_values_of_a_range_with_a_denormal_weight_reach_the_output(dtyp
     assert (out[..., 3] == INF).all() and (out[..., Dv - 1] == -INF).all()
     out[..., 3] = out[..., Dv - 1] = 1.
     assert (out.double() - 1.).abs().max() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,T", [(1, 40), (1, 64), (1, 3000), (70, 300)])  # (the new row in its part's only tile, or in the tenth)
+@pytest.mark.parametrize("rotary", [False, True])
+def test_a_step_that_reads_its_own_row_again(dtype, B, T, rotary):
+    """One token at head size 512 whose kernel writes the new row: an infinite value, in the new row or behind it, sends the
+    workgroup through its tiles once more, and there the row is read from the page.  Against separate calls."""
+    D = 512
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    rand = lambda h, n: torch.randn(B, h, n, D, generator=gen, device="cuda").to(dtype)
+    rope = kvhip.RoPE(D, base=1e4) if rotary else None
+    k, v = rand(4, T), rand(4, T)
+    v[:, :, T - 1, 3] = INF
+    one, two = kvhip.KVCacheSimple(), kvhip.KVCacheSimple()
+    for c in (one, two):
+        c.update(k, v, fetch=False)
+    for i in range(2):
+        q, nk, nv = rand(8, 1), rand(4, 1), rand(4, 1)
+        nv[..., 5], nv[..., D - 1] = -INF, INF
+        if rotary:
+            got = kvhip.attention_with_rope_and_cache_update(rope, q, nk, nv, one, D ** -0.5)
+            q = kvhip.apply_rotary_position(rope, q, two.rope_offset)
+            two.update_rope(rope, nk, nv)
+        else:
+            got = kvhip.attention_with_cache_update(q, nk, nv, one, D ** -0.5)
+            two._update(nk, nv)
+        assert kvhip.load().kvhip_last_attend_kernel() == 5
+        assert (got[..., 3] == INF).all() and (got[..., 5] == -INF).all() and (got[..., D - 1] == INF).all()
+        assert torch.equal(got, two.attend(q, D ** -0.5))
+    for a, b in zip(one.state, two.state):
+        assert torch.equal(a, b)
