@@ -34,7 +34,7 @@ template <int D, int DT, int CB, bool SPANS>
 __global__ void __launch_bounds__(256) combine_kernel(AttendArgs a, int nsplit, int rr, const int2 *spans) {
     static_assert(D % CB == 0, "whole blocks of columns");
     constexpr int CP = CB / 2;    // column pairs
-    constexpr int NG = 256 / CP;  // span groups: 8 (64 columns), 6, 5, 4 (128)
+    constexpr int NG = 256 / CP;  // span groups: 16 (32 columns), 8 (64), 6, 5, 4 (128)
     constexpr int UN = 8;         // loads in flight per thread and round
     constexpr bool EXACT = exact_merge<D, DT>();
     __shared__ float w_s[512];    // weight of each span for this row (nsplit <= 512)
@@ -189,13 +189,15 @@ hipError_t launch_combine(const AttendArgs &a, int nsplit, int rows, hipStream_t
     if (a.st.Dv == 64) return merge_dtype<64, 64>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 80) return merge_dtype<80, 80>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 96) return merge_dtype<96, 96>(a, nsplit, rows, spans, s);
-    // Blocks of fewer columns shorten a workgroup's chain where the launch has few rows (a sequence's 32 rows of 64 spans: 3.4
-    // us of 128 columns, 3.2 of 64; 8 rows of 65 spans at head size 512: 3.8 of 64, 3.3 of 32), and are workgroups more where
-    // it has many (2048 rows: 1 us).
+    // Blocks of fewer columns shorten a workgroup's chain, which is what a launch of few rows and many spans lasts, and are
+    // workgroups more.  Whole steps, us, 64 / 128 columns at head size 128: 32 rows over 16 000 keys of 4 bits 9.2 / 10.4, 64 rows
+    // 11.0 / 12.0, 128 rows over 2000 keys 7.3 / 7.5, 512 rows 10.6 / 10.8 (64q/8kv) and 13.3 / 13.1 (32q), 1024 rows 14.2 / 13.8, 2048
+    // 19.2 / 17.6.  32 / 64 columns at 512, bfloat16: 8 rows over 4000 keys 8.3 / 9.2, 16 rows 11.4 / 11.9, 32 rows 12.4 / 12.9 and 12.6 /
+    // 13.0, 64 rows 13.8 / 13.7, 128 rows 19.0 / 18.6 and 25.7 / 24.9.
     const size_t all = (size_t)(a.Hq / a.Hkv) * a.L * a.st.BH;
-    if (a.st.Dv == 128) return all <= 1024 ? merge_dtype<128, 64>(a, nsplit, rows, spans, s) : merge_dtype<128, 128>(a, nsplit, rows, spans, s);
+    if (a.st.Dv == 128) return all <= 512 ? merge_dtype<128, 64>(a, nsplit, rows, spans, s) : merge_dtype<128, 128>(a, nsplit, rows, spans, s);
     if (a.st.Dv == 256) return merge_dtype<256, 128>(a, nsplit, rows, spans, s);
-    if (a.st.Dv == 512) return all <= 128 ? merge_dtype<512, 32>(a, nsplit, rows, spans, s) : merge_dtype<512, 64>(a, nsplit, rows, spans, s);
+    if (a.st.Dv == 512) return all <= 32 ? merge_dtype<512, 32>(a, nsplit, rows, spans, s) : merge_dtype<512, 64>(a, nsplit, rows, spans, s);
     return hipErrorInvalidValue;
 }
 
