@@ -268,6 +268,7 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
             KV_SB;
         }
         float mx = 0.f;
+        static_assert(NCB >= 2, "three of out^T's instructions stand between the scores' last and their maximum");
         // (assembly: fmaxf quiets every matrix-core result first.  The compiler's hazard handling does not look into it: the
         // scores' last matrix-core instruction is two or more of out^T's behind, which issue one after the other)
         auto max_step = [&](int i) __attribute__((always_inline)) {
