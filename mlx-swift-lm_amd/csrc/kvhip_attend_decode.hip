@@ -955,21 +955,20 @@ decode_fp_kernel(int tiles_total, int tiles_per_wg, int nsplit, typename DecodeA
     }
     if constexpr (MM == 0) {
         if (own) {  // wave-uniform
-            // (global stores, and offsets as kfp_off and vfp_off give them for two-byte elements: behind a store to a plain
-            // pointer every load in flight is waited for, and divisions by the element size cost a microsecond here.  What a
+            // (global stores: behind a store to a plain pointer every load in flight is waited for.  What a
             // wavefront loads behind its own stores it loads as stored: the fence holds the compiler)
-            const int t = a.new_slot & (PAGE - 1), tk = t & (TILE - 1);
+            const int slot = a.new_slot, tk = slot & (TILE - 1);
             const PageEntry page{const_cast<char *>(pt[a.new_slot >> PAGE_SHIFT].k), nullptr, const_cast<char *>(pt[a.new_slot >> PAGE_SHIFT].v), nullptr};
-            KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell) + (t >> 6) * (TILE * D * 2) + tk * 16;
-            KV_GLOBAL char *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell) + (t >> 6) * (TILE * D * 2) + (tk >> 3) * (D * 16) + (tk & 7) * 2;
+            KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell);
+            KV_GLOBAL char *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell);
             uint16_t *row_s = rot ? rot_s + R * D : reinterpret_cast<uint16_t *>(&parts.rows[wave][0][0]);
             if (lane < D / 8) {
                 if constexpr (rot) own_k = *reinterpret_cast<const kv_u4 *>(row_s + 8 * lane);
                 else *reinterpret_cast<kv_u4 *>(row_s + 8 * lane) = own_k;
-                *reinterpret_cast<KV_GLOBAL kv_u4 *>(kc + lane * (TILE * 16)) = own_k;
+                *reinterpret_cast<KV_GLOBAL kv_u4 *>(kc + kfp_at<2>(2 * D, slot, 8 * lane)) = own_k;
             }
 #pragma unroll
-            for (int h = 0; h < NP; ++h) *reinterpret_cast<KV_GLOBAL uint16_t *>(vc + (64 * h + lane) * 16) = (uint16_t)own_v[h];
+            for (int h = 0; h < NP; ++h) *reinterpret_cast<KV_GLOBAL uint16_t *>(vc + vfp_at<2>(D, slot, 64 * h + lane)) = (uint16_t)own_v[h];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             if (row_first) {

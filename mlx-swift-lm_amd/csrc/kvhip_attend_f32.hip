@@ -103,17 +103,16 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_tot
 #pragma unroll
             for (int s = 0; s < NS; ++s) own_k[s] = *reinterpret_cast<const f4 *>(rot_s + R * DK + 16 * s + 4 * g);
         }
-        // (global stores, and offsets as kfp_off and vfp_off give them for four-byte elements: see attend_wide_kernel)
-        const int t = a.new_slot & (PAGE - 1), tk = t & (TILE - 1);
-        KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell) + (t >> 6) * (TILE * DK * 4) + (g * TILE + tk) * 16;
-        KV_GLOBAL char *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell) + (t >> 6) * (TILE * DV * 4) + ((tk >> 2) * DV + col) * 16 + (tk & 3) * 4;
+        // (global stores: see attend_wide_kernel)
+        const int slot = a.new_slot;
+        KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell), *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell);
         if (col == 0) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) *reinterpret_cast<KV_GLOBAL f4 *>(kc + s * (4 * TILE * 16)) = own_k[s];
+            for (int s = 0; s < NS; ++s) *reinterpret_cast<KV_GLOBAL f4 *>(kc + kfp_at<4>(4 * DK, slot, 16 * s + 4 * g)) = own_k[s];
         }
         if (g == 0) {
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) *reinterpret_cast<KV_GLOBAL float *>(vc + c * (16 * 16)) = own_v[c];
+            for (int c = 0; c < NCT; ++c) *reinterpret_cast<KV_GLOBAL float *>(vc + vfp_at<4>(DV, slot, 16 * c + col)) = own_v[c];
         }
     };
 

@@ -127,18 +127,16 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_to
         }
     }
     auto write_row = [&](const PageEntry &page) __attribute__((always_inline)) {
-        // (global stores: behind one to a plain pointer every load in flight is waited for.  Offsets as kfp_off and vfp_off
-        // give them for two-byte elements, whose divisions by the element size take a microsecond here)
-        const int t = a.new_slot & (PAGE - 1), tk = t & (TILE - 1), c0 = wave * (WD / WW);
-        KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell) + (t >> 6) * (TILE * WD * 2) + ((c0 / 8 + g) * TILE + tk) * 16;
-        KV_GLOBAL char *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell) + (t >> 6) * (TILE * WD * 2) + ((tk >> 3) * WD + c0 + col) * 16 + (tk & 7) * 2;
+        // (global stores: behind one to a plain pointer every load in flight is waited for)
+        const int slot = a.new_slot, c0 = wave * (WD / WW);
+        KV_GLOBAL char *kc = (KV_GLOBAL char *)as_global(page.k + (size_t)bh * st.k_cell), *vc = (KV_GLOBAL char *)as_global(page.v + (size_t)bh * st.v_cell);
         if (col == 0) {
 #pragma unroll
-            for (int s = 0; s < NS; ++s) *reinterpret_cast<KV_GLOBAL kv_u4 *>(kc + s * (4 * TILE * 16)) = own_k[s];
+            for (int s = 0; s < NS; ++s) *reinterpret_cast<KV_GLOBAL kv_u4 *>(kc + kfp_at<2>(2 * WD, slot, c0 + 8 * g + 32 * s)) = own_k[s];
         }
         if (g == 0) {
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) *reinterpret_cast<KV_GLOBAL uint16_t *>(vc + c * (16 * 16)) = own_v[c];
+            for (int c = 0; c < NCT; ++c) *reinterpret_cast<KV_GLOBAL uint16_t *>(vc + vfp_at<2>(WD, slot, c0 + 16 * c + col)) = own_v[c];
         }
     };
     auto row_written = []() __attribute__((always_inline)) {  // (a wavefront reads the quarter that it wrote)

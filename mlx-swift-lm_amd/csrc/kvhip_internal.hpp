@@ -118,6 +118,18 @@ __device__ __forceinline__ size_t vfp_off(const Store &st, int slot, int d) {
     const int t = slot & (PAGE - 1), epc = 16 / st.es, tk = t & 63;
     return (size_t)(t >> 6) * ((size_t)TILE * st.Dv * st.es) + ((size_t)(tk / epc) * st.Dv + d) * 16 + (size_t)(tk % epc) * st.es;
 }
+// The same with the element size known, and the bytes of a K row (the columns of V) where the caller knows them: kfp_off and
+// vfp_off divide by the element size three times, which in a kernel's few lanes takes a microsecond.
+template <int ES> __device__ __forceinline__ uint32_t kfp_at(uint32_t k_row, uint32_t slot, uint32_t d) {
+    constexpr uint32_t EPC = 16 / ES;
+    const uint32_t t = slot & (PAGE - 1);
+    return (t >> 6) * (TILE * k_row) + ((d / EPC) * TILE + (t & 63)) * 16 + (d % EPC) * ES;
+}
+template <int ES> __device__ __forceinline__ uint32_t vfp_at(uint32_t dv, uint32_t slot, uint32_t d) {
+    constexpr uint32_t EPC = 16 / ES;
+    const uint32_t t = slot & (PAGE - 1), tk = t & 63;
+    return (t >> 6) * (TILE * dv * ES) + ((tk / EPC) * dv + d) * 16 + (tk % EPC) * ES;
+}
 __device__ __forceinline__ const char *k_cell_ptr(const Store &st, int bh, int slot) {
     return page_table(st)[slot >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;
 }

@@ -487,9 +487,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
             }
         }
         char *kcell = page_table(st)[slot_t >> PAGE_SHIFT].k + (size_t)bh * st.k_cell;  // a tile lies inside one page
-        // (kfp_off and vfp_off, whose divisions by the element size run on every thread, with it known)
-        if (live && r >= t_lo && r < t_hi)
-            *reinterpret_cast<kv_u4 *>(kcell + (size_t)((slot_t & (PAGE - 1)) >> 6) * (TILE * DK * ES) + ((d0 / E) * TILE + r) * 16) = k;
+        if (live && r >= t_lo && r < t_hi) *reinterpret_cast<kv_u4 *>(kcell + kfp_at<ES>(DK * ES, slot_t, 0) + kfp_at<ES>(DK * ES, r, d0)) = k;
         return;
     }
     const int c0 = (piece - P::KP) * P::VC;  // first column
@@ -514,7 +512,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
     __syncthreads();
     // chunks of E tokens of every column: a thread gathers tokens E ce .. E ce + E - 1 of column d;
     // consecutive threads take consecutive columns, so a chunk row is written contiguously
-    char *cell = const_cast<char *>(v_cell_ptr(st, bh, slot_t)) + (size_t)((slot_t & (PAGE - 1)) >> 6) * (TILE * DV * ES);
+    char *cell = const_cast<char *>(v_cell_ptr(st, bh, slot_t)) + vfp_at<ES>(DV, slot_t, 0);
     const T *vte = reinterpret_cast<const T *>(vt);
     constexpr int VPE = VPW * 4 / ES;
     for (int c = threadIdx.x; c < P::VC * (TILE / E); c += 256) {
@@ -525,7 +523,7 @@ append_fp_tile_kernel(Store st, const char *keys, const char *values, int L, int
             if constexpr (ES == 4) out[j] = vte[(t0 + j) * VPE + d];
             else out[j] = (uint32_t)vte[(t0 + 2 * j) * VPE + d] | ((uint32_t)vte[(t0 + 2 * j + 1) * VPE + d] << 16);
         }
-        char *dst = cell + ((t0 / E) * DV + c0 + d) * 16;
+        char *dst = cell + vfp_at<ES>(DV, t0, c0 + d);
         if (t0 >= t_lo && t0 + E <= t_hi) {
             *reinterpret_cast<kv_u4 *>(dst) = kv_u4{out[0], out[1], out[2], out[3]};
         } else {
@@ -569,18 +567,6 @@ __global__ void import_fp_kernel(Store st, const char *src_k, const char *src_v,
     for (int d = threadIdx.x; d < st.Dv; d += blockDim.x) *reinterpret_cast<E *>(vc + vfp_off(st, slot, d)) = vs[d];
 }
 
-// kfp_off and vfp_off with the element size known
-template <int ES> __device__ __forceinline__ size_t kfp_at(const Store &st, int slot, int d) {
-    constexpr int EPC = 16 / ES;
-    const int t = slot & (PAGE - 1);
-    return (size_t)(t >> 6) * ((size_t)TILE * st.k_row) + (size_t)(((d / EPC) * TILE + (t & 63)) * 16 + (d % EPC) * ES);
-}
-template <int ES> __device__ __forceinline__ size_t vfp_at(const Store &st, int slot, int d) {
-    constexpr int EPC = 16 / ES;
-    const int t = slot & (PAGE - 1), tk = t & 63;
-    return (size_t)(t >> 6) * ((size_t)TILE * st.Dv * ES) + (size_t)(((tk / EPC) * st.Dv + d) * 16 + (tk % EPC) * ES);
-}
-
 // Rows in presented order into slots 0, 1, ... of another store (a ring that is laid out again, a copy).  grid (chunks of
 // 16 / ES rows, BH), 256 threads: the rows' 16-byte K chunks move whole, lanes along the rows; a thread puts a column's V
 // chunk together from the two that hold its tokens, shifted by where the run starts.  Chunks that a run begins or ends
@@ -605,17 +591,17 @@ __global__ void __launch_bounds__(256) compact_fp_kernel(Store src, Runs runs, S
         char *kd = const_cast<char *>(k_cell_ptr(dst, bh, row));
         const int chunks = src.Dk / EPC;
         for (int c = tid / EPC; c < chunks; c += 256 / EPC)
-            *reinterpret_cast<kv_u4 *>(kd + kfp_at<ES>(dst, row, c * EPC)) = *reinterpret_cast<const kv_u4 *>(ks + kfp_at<ES>(src, from, c * EPC));
+            *reinterpret_cast<kv_u4 *>(kd + kfp_at<ES>(dst.k_row, row, c * EPC)) = *reinterpret_cast<const kv_u4 *>(ks + kfp_at<ES>(src.k_row, from, c * EPC));
         for (int d = chunks * EPC + tid / EPC; d < src.Dk; d += 256 / EPC)
-            *reinterpret_cast<E *>(kd + kfp_at<ES>(dst, row, d)) = *reinterpret_cast<const E *>(ks + kfp_at<ES>(src, from, d));
+            *reinterpret_cast<E *>(kd + kfp_at<ES>(dst.k_row, row, d)) = *reinterpret_cast<const E *>(ks + kfp_at<ES>(src.k_row, from, d));
     }
     if (run) {
         const int sh = slot[0] % EPC, last = slot[0] + EPC - 1;
         const char *v0 = v_cell_ptr(src, bh, slot[0]), *v1 = v_cell_ptr(src, bh, last);
         char *vd = const_cast<char *>(v_cell_ptr(dst, bh, i0));
         for (int d = tid; d < src.Dv; d += 256) {
-            const kv_u4 x = *reinterpret_cast<const kv_u4 *>(v0 + vfp_at<ES>(src, slot[0] - sh, d));
-            const kv_u4 y = *reinterpret_cast<const kv_u4 *>(v1 + vfp_at<ES>(src, last - last % EPC, d));
+            const kv_u4 x = *reinterpret_cast<const kv_u4 *>(v0 + vfp_at<ES>(src.Dv, slot[0] - sh, d));
+            const kv_u4 y = *reinterpret_cast<const kv_u4 *>(v1 + vfp_at<ES>(src.Dv, last - last % EPC, d));
             uint32_t w[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
             const int words = sh * ES / 4;  // whole words to drop in front
             if (words & 2) {
@@ -630,7 +616,7 @@ __global__ void __launch_bounds__(256) compact_fp_kernel(Store src, Runs runs, S
 #pragma unroll
                 for (int k = 0; k < 4; ++k) w[k] = (w[k] >> 16) | (w[k + 1] << 16);
             }
-            *reinterpret_cast<kv_u4 *>(vd + vfp_at<ES>(dst, i0, d)) = kv_u4{w[0], w[1], w[2], w[3]};
+            *reinterpret_cast<kv_u4 *>(vd + vfp_at<ES>(dst.Dv, i0, d)) = kv_u4{w[0], w[1], w[2], w[3]};
         }
         return;
     }
@@ -640,7 +626,7 @@ __global__ void __launch_bounds__(256) compact_fp_kernel(Store src, Runs runs, S
         const char *vs = v_cell_ptr(src, bh, at);
         char *vd = const_cast<char *>(v_cell_ptr(dst, bh, i0 + j));
         for (int d = tid; d < src.Dv; d += 256)
-            *reinterpret_cast<E *>(vd + vfp_at<ES>(dst, i0 + j, d)) = *reinterpret_cast<const E *>(vs + vfp_at<ES>(src, at, d));
+            *reinterpret_cast<E *>(vd + vfp_at<ES>(dst.Dv, i0 + j, d)) = *reinterpret_cast<const E *>(vs + vfp_at<ES>(src.Dv, at, d));
     }
 }
 
