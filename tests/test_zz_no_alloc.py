@@ -131,11 +131,13 @@ def test_static_scratch_takes_large_batches_and_plans_fewer_parts_when_the_array
     got, want, family = both(big, q, 256 ** -0.5, kvhip.MaskMode.causal())
     assert family == 1 and torch.equal(got, want)
     del big
-    # a prompt chunk whose two key-range parts would need 25.5 MB of partials: the allocating entry point splits the
+    # a prompt chunk whose two key-range parts would need 25.5 MB of partials, were they not taken at once by workgroups that
+    # need none, and one that is left with two parts of 17 MB: the allocating entry point splits the
     # keys, the allocation-free one plans a single part (another summation order: compared within the tolerance)
-    c, g = filled(kvhip.KVCacheSimple, 1, 8, 1024, 128, torch.float16, 7)
-    q = torch.randn(1, 32, 768, 128, generator=g, device="cuda").half()
-    got, want, family = both(c, q, 128 ** -0.5, kvhip.MaskMode.causal())
-    assert family == 3
-    d = (got.float() - want.float()).abs()
-    assert float(d.max()) <= 2e-3 and float(d.mean()) <= 1e-4
+    for T, n in ((1024, 768), (2048, 512)):
+        c, g = filled(kvhip.KVCacheSimple, 1, 8, T, 128, torch.float16, 7)
+        q = torch.randn(1, 32, n, 128, generator=g, device="cuda").half()
+        got, want, family = both(c, q, 128 ** -0.5, kvhip.MaskMode.causal())
+        assert family == 3
+        d = (got.float() - want.float()).abs()
+        assert float(d.max()) <= 2e-3 and float(d.mean()) <= 1e-4
