@@ -1,6 +1,7 @@
 // Which prefill tile serves a call, how it is planned (query rows per workgroup, key-range parts, scratch) and
 // its launch.  Many query rows per kv head (r = Hq / Hkv heads times L new tokens): quantized caches take the
-// pipelined tile of kvhip_attend_prefill_q.hpp, full-precision caches the kernel of kvhip_attend_prefill_fp.hip.
+// pipelined tile of kvhip_attend_prefill_q.hpp, full-precision caches the kernels of kvhip_attend_prefill_fp.hip (64 rows a
+// workgroup) and kvhip_attend_prefill_rows32.hip (128).
 #include <cstdlib>
 
 #include "kvhip_mask.hpp"
@@ -35,30 +36,32 @@ bool attend_prefill_dequant_first(const AttendArgs &a, bool always) {
     if (always) return true;
     // The conversion pass is a launch more and 2 (Dk + Dv) bytes per cached row and kv head written and read again,
     // the same for any number of query rows: what it buys grows with the rows per kv head that share a converted
-    // key.  Per kv head both costs scale alike with batch and heads, so the bound is one on rows x keys x head
-    // sizes: measured ahead by 5-40 % from 512 rows and rows x keys = 4 M at D 128 (2048 x 2048, 1024 x 4096,
-    // 512 x 8192; B1 to B16) over 2048 keys and more, equal or behind below that (1024 x 2048: 44 against 40 us,
-    // 2048 x 1024: 44 against 42, 4096 x 1024: 50 against 41,
-    // B16 512 x 4096, where 256-row workgroups of the quantized tile fill the chip: 231 against 197) and with
-    // fewer rows whatever the keys (B8, 256 x 8192: 185 against 141 us).
+    // key.  Per kv head both costs scale alike with batch and heads, so the bound is one on rows x keys x head sizes.
+    // Calls, us, quantized tile / dequantized first (float16, 4 bits, 32q/8kv x 128, causal).  Inside the bound: 512 new rows over 2048 keys
+    // 47 / 42, over 4096 76 / 56, over 8192 133 / 91, 2048 over 2048 103 / 58, 256 over 4096 49 / 41, 128 over 8192 51 / 44, B8 128 over
+    // 8192 307 / 205, B16 512 over 4096 895 / 574; 8 bits x 64 512 over 8192 100 / 64; bfloat16 x 256 B4 256 over 4608 94 / 77.
+    // Outside, behind: B8 64 over 8192 (256 rows a kv head) 134 / 153, B16 128 over 4096 195 / 204, x 64 512 over 1024 27.5 / 28.3, over 512
+    // 15.8 / 19.0, x 256 (8q/4kv) 512 over 1024 28 / 30; level: 512 over 512 21.1 / 21.0, 256 over 2048 34.9 / 34.7.  Outside and ahead, since the
+    // 32-row tile: 512 over 1024 37 / 32, over 1536 41 / 38, 1024 over 1024 39 / 32, B4 512 over 1024 58 / 48, B32 128 over 4096 482 / 415,
+    // and x 64 over 2048 35 / 31 -- the line was drawn beside the tile before it and could go lower at head size 128.
     const int R = (a.Hq / a.Hkv) * a.L;
     static const int min_rows = measure_knob("KVHIP_DEQUANT_FIRST_ROWS", 512);  // (timing builds only)
     return R >= min_rows && a.T >= 2048 && (double)R * a.T * (s.Dk + s.Dv) >= 1073741824.0;
 }
 
-// 128 query rows per workgroup reuse each staged tile twice as often as 64, and measured ahead of 64 rows on every
-// grid from two such blocks per kv head up -- also where they leave the grid small, which key-range parts then fill
-// (TFLOP/s of the call, 64 / 128 rows, fp16 D 128 32q/8kv causal: B1 512 x 8192 542 / 598, 512 x 32768 709 / 855,
-// 1024 x 8192 590 / 714, 256 x 32768 643 / 754, B2 512 x 8192 603 / 712, B7 256 x 4096 547 / 695, B3 512 x 8192
-// 693 / 708; D 64 B1 2048 x 8192 334 / 446; equal at 128 rows of 4 heads).
+// 128 query rows per workgroup, on the 32-row tile, measured ahead of 64 rows on every grid from two such blocks per kv
+// head up -- also where they leave the grid small, which key-range parts then fill (us a call, 64 / 128 rows, bfloat16 x 128
+// 32q/8kv causal: B1 512 x 8192 93 / 76, 512 x 32768 336 / 264, 1024 x 8192 173 / 130, 256 x 32768 174 / 139, B2 512 x 8192 175 / 131, B7 256 x
+// 4096 181 / 122, 64 x 8192 (256 rows a kv head) 25.7 / 23.6, B4 256 x 512 16.9 / 15.8; x 64 512 x 2048 28 / 23).  At 160 rows a
+// kv head they are level (40 x 8192 21.5 / 20.8), at 124 behind (31 x 8192 19.1 / 20.0).
 static bool prefill_wide(const AttendArgs &a) {
     const int R = (a.Hq / a.Hkv) * a.L;
     static const int forced = measure_knob("KVHIP_PREFILL_WIDE", -1);  // (timing builds only)
     if (forced >= 0) return forced != 0 && a.st.Dk <= 128;
     if (R < 256 || a.st.Dk > 128) return false;
     // Few keys (a prompt's first chunks): where 128-row workgroups would need key-range parts to fill the chip and
-    // 64-row ones fill it without, the merge launch costs more than the wider tile gains (a single sequence's
-    // 512 x 512: 22 against 35 us; 512 x 1024: 33 against 43; equal from 2048 keys).
+    // 64-row ones fill it without, the merge launch costs more than the wider tile gains (a single sequence's, 64 / 128 rows: 512 x 512
+    // 13.2 / 14.1 us, 512 x 768 18.0 / 26.0, 512 x 1024 22.4 / 25.9; 512 x 1500 30.3 / 29.1; x 64 512 x 1024 18.7 / 18.3).
     const size_t wide_wgs = (size_t)((R + 127) / 128) * a.st.BH, narrow_wgs = (size_t)((R + 63) / 64) * a.st.BH;
     if (a.T <= 1024 && wide_wgs < 512 && narrow_wgs >= 256) return false;
     return true;
@@ -123,9 +126,11 @@ static PrefillPlan prefill_plan(const AttendArgs &a) {
     p.rows = prefill_block_rows(a);
     int n = prefill_splits(a, p.rows);
     // An even number of parts of 128-row workgroups: a workgroup of eight wavefronts takes two of them and adds them up in
-    // LDS, which halves the partials in memory and the merge that reads them.  The kernel itself gives nothing or 1 us
-    // (bfloat16 D 128 32q/8kv, 512 new rows: over 8192 keys 73.0 us in four parts of four wavefronts, 72.9 in two of
-    // eight; 4096 keys 41.8 / 41.2; 2048 keys 26.5 / 25.5), the merge behind it 3.5 us of 7.  Without parts it costs
+    // LDS, which halves the partials in memory and the merge that reads them, or saves both (us a call, bfloat16 x 128 causal, four
+    // wavefronts / eight: 32q/8kv 512 new rows over 2048 keys 35.6 / 33.5, over 8192 77.9 / 76.0, 1024 over 1100 33.2 / 24.0, over 4096 75.0 / 67.4, a
+    // window of 1024 39.2 / 27.2; 16q/16kv 2048 over 2048 39.1 / 35.1).  A CU then holds one workgroup, where two of four wavefronts were a long
+    // and a short query block (work_item): chunks of 3000 new rows and more over few other keys pay for that with up to 5 % (8q/8kv 3000
+    // over 3000 43.1 / 45.4, 4096 over 4096 58.9 / 60.0, over 8192 120.1 / 121.3; 3500 over 3500 53.7 / 51.7).  Without parts it costs
     // (2048 x 8192 239 -> 255 us: eight wavefronts wait for each other at a barrier), and an odd number would leave CUs idle.
     p.halves = a.st.bits == 0 && p.rows == 128 && n > 1 && n % 2 == 0;
     if (p.halves) n /= 2;

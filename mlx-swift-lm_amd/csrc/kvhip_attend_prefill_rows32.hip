@@ -10,16 +10,16 @@
 // set of requests.
 //
 // Pipeline: step k issues the scores of block k + 1 and spreads the softmax of block k, whose scores step k - 1 left in
-// registers, over those instructions and the first half of out^T's (over the scores' alone: 984 TFLOP/s for 1000).  K and V
-// move from global memory straight into two LDS rings of four blocks, an iteration ahead.
+// registers, over those instructions and the first half of out^T's (over the scores' alone: 2 % slower).  K and V
+// move from global memory straight into two LDS rings of four blocks, an iteration ahead.  Outputs and partials leave through LDS.
 //
-// What bounds it: the matrix cores at the clock that the chip's power leaves (1000 TFLOP/s of the 1190 that a large matrix
-// product reaches; without exponentials 1050, without requests 1140), and for short chunks what stands around the loop: of
-// 512 new rows over 2048 keys (25.0 us) 3.8 to the first scores, 3 for the partials and up to 3 for the blocks that see fewer
-// keys than the last.
-// Measured against 32 rows on 16x16x32 instructions, which this replaces (D 128, 32q/8kv, causal, TFLOP/s): bfloat16 2048 x
-// 8192 946 -> 1027, 512 x 8192 893 -> 939 and a merge of half the bytes; float16 2048 x 8192 924 -> 964, 512 x 8192 883
-// -> 885 and the same.
+// What bounds it: the matrix cores at the clock that the chip's power leaves (timed in turn with parts taken out, 2048 x 8192 is 7 %
+// faster without exponentials and 16 % without requests; a large matrix product reaches 1190 TFLOP/s), and for short chunks what
+// stands around the loop: of 512 new rows over 2048 keys 3.8 us to the first scores, 2 for the partials and up to 3 for
+// the blocks that see fewer keys than the last, of 25.
+// Events around the launch (bench.py --workload prefill, D 128, 32q/8kv, causal, TFLOP/s of two runs; before it 32 rows on 16x16x32
+// instructions, in turn on one box): bfloat16 2048 x 8192 853-866 -> 952-954, 512 x 8192 717-730 -> 732-745, 4096 x 4096 648-655 -> 773;
+// float16 2048 x 8192 857-872 -> 926-931, 512 x 8192 701-708 -> 721-738, and for 512 rows a merge of half the bytes.
 #include "kvhip_prefill_fp.hpp"
 
 #ifndef KV_SB
