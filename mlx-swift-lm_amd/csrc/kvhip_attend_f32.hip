@@ -436,9 +436,9 @@ attend_f32_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_tot
 #pragma unroll
             for (int w = 1; w < MW; ++w) v += acc_s[((w * QT + qt) * NCT + c) * 64 + lane];
             if (nparts == 1) v = L[qt] > 0.f ? v / L[qt] : f4{0.f, 0.f, 0.f, 0.f};
-            float *d = dst + 16 * c + 4 * g;  // (partials: rows of DV + 2 floats, 8-byte aligned)
-            *reinterpret_cast<kv_f2 *>(d) = kv_f2{v.x, v.y};
-            *reinterpret_cast<kv_f2 *>(d + 2) = kv_f2{v.z, v.w};
+            float *d = dst + 16 * c + 4 * g;  // (partials: rows of DV + 2 floats, 8-byte aligned; outputs: as their elements are)
+            *reinterpret_cast<kv_out2f *>(d) = kv_out2f{v.x, v.y};
+            *reinterpret_cast<kv_out2f *>(d + 2) = kv_out2f{v.z, v.w};
         }
         if (nparts > 1 && wave == 0 && g == 0) {
             dst[DV] = M[qt];

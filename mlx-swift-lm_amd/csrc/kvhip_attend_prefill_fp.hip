@@ -552,15 +552,7 @@ prefill_fp_kernel(AttendArgs a, int nsplit) {
     for (int dt = 0; dt < NDT; ++dt) {
         const float o0 = oacc[dt][0] * inv, o1 = oacc[dt][1] * inv;
         const float o2 = oacc[dt][2] * inv, o3 = oacc[dt][3] * inv;
-        uint2 w;
-        if (DT == 0) {
-            w.x = rn_h2(o0, o1);
-            w.y = rn_h2(o2, o3);
-        } else {
-            w.x = rn_bf2(o0, o1);
-            w.y = rn_bf2(o2, o3);
-        }
-        *reinterpret_cast<uint2 *>(op + 16 * dt + 4 * jj) = w;
+        *reinterpret_cast<kv_out4 *>(op + 16 * dt + 4 * jj) = DT == 0 ? kv_out4{rn_h2(o0, o1), rn_h2(o2, o3)} : kv_out4{rn_bf2(o0, o1), rn_bf2(o2, o3)};
     }
 }
 

@@ -775,15 +775,8 @@ prefill_q_kernel(AttendArgs a, int nsplit) {
         for (int dt = 0; dt < NDT; ++dt) {
             const float o0 = oacc[qt][dt][0] * inv, o1 = oacc[qt][dt][1] * inv;
             const float o2 = oacc[qt][dt][2] * inv, o3 = oacc[qt][dt][3] * inv;
-            uint2 w;
-            if (DT == 0) {
-                w.x = pk_h2(o0, o1);
-                w.y = pk_h2(o2, o3);
-            } else {
-                w.x = pk_bf2(o0, o1);
-                w.y = pk_bf2(o2, o3);
-            }
-            *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(a.out) + ooff + 16 * dt + 4 * jj) = w;
+            *reinterpret_cast<kv_out4 *>(reinterpret_cast<uint16_t *>(a.out) + ooff + 16 * dt + 4 * jj) =
+                DT == 0 ? kv_out4{pk_h2(o0, o1), pk_h2(o2, o3)} : kv_out4{pk_bf2(o0, o1), pk_bf2(o2, o3)};
         }
     }
 }

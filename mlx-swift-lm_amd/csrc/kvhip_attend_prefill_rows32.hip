@@ -31,7 +31,6 @@ namespace {
 
 using namespace prefill_fp;
 typedef float f16v __attribute__((ext_vector_type(16)));
-typedef uint32_t out16 __attribute__((ext_vector_type(4), aligned(2)));  // 16 bytes of a caller's array, aligned as its elements are
 
 template <int DT> __device__ __forceinline__ void mfma32(f16v &c, const Op8 &a, const Op8 &b) {
     if constexpr (DT == 0) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, b.h, c, 0, 0, 0);
@@ -512,7 +511,7 @@ prefill_rows32_kernel(AttendArgs a, int nsplit) {
         for (int k = 0; k < (32 * CPR + 63) / 64; ++k) {
             const int x = 64 * k + lane, rw = x / CPR, ch = x - rw * CPR;
             if (((32 * CPR) % 64 == 0 || x < 32 * CPR) && row0 + rw < R)
-                *reinterpret_cast<out16 *>(op + rw * D + 8 * ch) = *reinterpret_cast<const kv_u4 *>(stage + rw * PITCH + 8 * ch);
+                *reinterpret_cast<kv_out8 *>(op + rw * D + 8 * ch) = *reinterpret_cast<const kv_u4 *>(stage + rw * PITCH + 8 * ch);
         }
     };
     if constexpr (HV == 1) leave(Z(), A());

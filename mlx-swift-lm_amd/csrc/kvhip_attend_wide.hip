@@ -457,7 +457,7 @@ attend_wide_kernel(typename DecodeArgs<ROT ? 3 : 0>::type a, int r, int tiles_to
 #pragma unroll
             for (int c = 0; c < NCT; ++c) {
                 const f4 v = acc[qt][c] * inv;
-                *reinterpret_cast<kv_u2 *>(dst + 16 * c) = kv_u2{pack2<DT>(v.x, v.y), pack2<DT>(v.z, v.w)};
+                *reinterpret_cast<kv_out4 *>(dst + 16 * c) = kv_out4{pack2<DT>(v.x, v.y), pack2<DT>(v.z, v.w)};
             }
         } else {
             float *dst = a.workspace + ((size_t)(bh * nparts + part) * R + rr) * (WD + 2);

@@ -20,8 +20,8 @@ template <bool EXACT> __device__ __forceinline__ float add_weighed(float sum, fl
     return EXACT ? __builtin_fmaf(w, v, sum) : sum + w * v;
 }
 template <int DT> __device__ __forceinline__ void store_pair(void *out, size_t i, float o0, float o1) {
-    if constexpr (DT == 2) *reinterpret_cast<kv_f2 *>(static_cast<float *>(out) + i) = kv_f2{o0, o1};
-    else *reinterpret_cast<uint32_t *>(static_cast<uint16_t *>(out) + i) = DT == 0 ? pk_h2(o0, o1) : pk_bf2(o0, o1);
+    if constexpr (DT == 2) *reinterpret_cast<kv_out2f *>(static_cast<float *>(out) + i) = kv_out2f{o0, o1};
+    else *reinterpret_cast<kv_out2 *>(static_cast<uint16_t *>(out) + i) = DT == 0 ? pk_h2(o0, o1) : pk_bf2(o0, o1);
 }
 
 // grid (R, BH, D / CB), 256 threads: merge the span partials of CB columns of one query row and write them.

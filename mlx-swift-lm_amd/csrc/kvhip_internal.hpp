@@ -142,6 +142,11 @@ typedef uint32_t kv_u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t kv_u2 __attribute__((ext_vector_type(2)));
 // four floats of a row of partials: rows are D + 2 floats, every other one 8 bytes off a 16-byte boundary
 typedef float kv_part4 __attribute__((ext_vector_type(4), aligned(8)));
+// two, four and eight 16-bit elements, and two floats, of a caller's output array, which is aligned as its elements are
+typedef uint32_t kv_out2 __attribute__((aligned(2)));
+typedef uint32_t kv_out4 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t kv_out8 __attribute__((ext_vector_type(4), aligned(2)));
+typedef float kv_out2f __attribute__((ext_vector_type(2), aligned(4)));
 #define KV_GLOBAL __attribute__((address_space(1)))
 typedef const KV_GLOBAL char *gptr;
 __device__ __forceinline__ gptr as_global(const void *p) { return (gptr) reinterpret_cast<const char *>(p); }

@@ -38,8 +38,8 @@ template <int DT, int N> __device__ __forceinline__ void store_columns(void *out
         uint32_t w[N / 2];
 #pragma unroll
         for (int k = 0; k < N / 2; ++k) w[k] = DT == 0 ? pk_h2(v[2 * k], v[2 * k + 1]) : pk_bf2(v[2 * k], v[2 * k + 1]);
-        if constexpr (N == 2) *reinterpret_cast<uint32_t *>(p) = w[0];
-        else *reinterpret_cast<kv_u2 *>(p) = kv_u2{w[0], w[1]};
+        if constexpr (N == 2) *reinterpret_cast<kv_out2 *>(p) = w[0];
+        else *reinterpret_cast<kv_out4 *>(p) = kv_out4{w[0], w[1]};
     }
 }
 template <int N> __device__ __forceinline__ void store_floats(float *p, const float (&v)[N]) {  // (8-byte aligned where N > 1)

@@ -279,5 +279,25 @@ def test_rotary_inputs_and_wide_heads_at_odd_element_offsets(kind, dtype, D, Lq)
     assert torch.equal(results[0][-2], results[0][-3])
 
 
+@pytest.mark.parametrize("kind,dtype,D", [("simple", torch.float16, 64), ("simple", torch.bfloat16, 128), ("simple", torch.float16, 256), ("simple", torch.bfloat16, 512),
+                                          (4, torch.float16, 128), (8, torch.bfloat16, 64), (6, torch.float16, 128), (4, torch.float16, 256),
+                                          ("simple", torch.float32, 64), ("simple", torch.float32, 256)])
+@pytest.mark.parametrize("B,T", [(1, 5000), (130, 300)])  # spans that are merged; one span to a pair
+@pytest.mark.parametrize("Lq", [1, 4, 40])
+def test_outputs_at_odd_element_offsets(kind, dtype, D, B, T, Lq):
+    """Attention into arrays that start one and three elements into an allocation: the same rows, and nothing beside them."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda h, n: torch.randn(B, h, n, D, generator=g, device="cuda").to(dtype)
+    c = kvhip.KVCacheSimple() if kind == "simple" else kvhip.QuantizedKVCache(64, kind)
+    c._update(rand(2, T), rand(2, T))
+    q, mask = rand(8, Lq), kvhip.MaskMode.causal()
+    want = c.attend(q, D ** -0.5, mask)
+    for ahead in (1, 3):
+        room = torch.full((want.numel() + 8,), 7., dtype=dtype, device="cuda")
+        c.attend(q, D ** -0.5, mask, out=room[ahead:ahead + want.numel()].view_as(want))
+        assert torch.equal(room[ahead:ahead + want.numel()].view_as(want), want)
+        assert (room[:ahead] == 7).all() and (room[ahead + want.numel():] == 7).all()
+
+
 def c_dtype(dtype):
     return {torch.float16: L.F16, torch.bfloat16: L.BF16, torch.float32: L.F32}[dtype]
